@@ -18,7 +18,7 @@
 
 #include "../../include/lg_hip.h"
 #include "lg_kernels.h"
-#include "lg_mfma.h"
+#include "lg_wide.h"
 #include "lg_fused.h"
 #include "lg_xcd.h"
 #include "lg_xffn.h"
@@ -151,6 +151,8 @@ struct Layer {
     float *winp_f = nullptr, *wproj_f = nullptr;   // inp_gate / proj when the file keeps them in a float type (then winp / wproj are null)
     uint8_t *wdn_m = nullptr;                      // ffn_down again as the per-workgroup streams of lg_k_down_m
     uint8_t *wo_ch = nullptr;                      // attn_output again as matrix-core chains [row block][segment]: lg_k_attn_tail
+    // the matrices once more in the form of the prompt kernels (lg_wide.h)
+    uint8_t *wqkv_w = nullptr, *wo_w = nullptr, *wgu_w = nullptr, *wdown_w = nullptr, *winp_w = nullptr, *wproj_w = nullptr;
     uint8_t *wo_rb = nullptr;                      // attn_output again as row-block tiles: the chains of lg_k_merge_o
     uint8_t *xgu = nullptr, *xdn = nullptr;        // gate/up and ffn_down again as per-workgroup streams of the XCD-partitioned kernel (lg_xffn.h)
     float *attn_norm = nullptr, *q_norm = nullptr, *k_norm = nullptr, *post_attn = nullptr, *ffn_norm = nullptr,
@@ -189,6 +191,7 @@ struct lg_hip_model {
     // weights
     std::vector<Layer> L;
     uint8_t *emb = nullptr, *pmp = nullptr, *pte = nullptr;
+    uint8_t *pmp_w = nullptr;                      // per_layer_model_proj in the form of the prompt kernels
     float *pmp_f = nullptr;                        // per_layer_model_proj kept in a float type (then pmp is null)
     float *pgf = nullptr;                          // [rows][ple] f32 gate output, input of a float-typed proj
     uint8_t *emb_rb = nullptr;                     // token_embd again as row-block tiles: the lm_head of 4..8-row blocks (lg_k_head_m)
@@ -247,7 +250,9 @@ struct lg_hip_model {
 
 struct lg_hip_kv {
     lg_hip_model *m = nullptr;
-    int max_seq = 0, tiles_max = 0, wide_rows = 0;      // wide_rows: the widest prompt block (sliding rings and partials are sized for it)
+    int max_seq = 0, tiles_max = 0, wide_rows = 0;      // wide_rows: the block the partials are sized for
+    int prompt_rows = 0;                                // widest prompt block: what the rings' spare rows and the partials' memory (as the scratch of lg_k_wide_attn) allow
+    size_t scratch_bytes = 0;
     std::vector<int> seq, kv_dim;
     std::vector<uint16_t *> k, v, px_k, px_v;
     float *pm = nullptr, *pl = nullptr, *pacc = nullptr;
@@ -376,6 +381,15 @@ static int upload_tiled(lg_hip_model *m, const std::vector<const uint8_t *> &row
     if (dev_alloc(m, out, bytes)) return -7;
     HIP_TRY(hipMemcpy(*out, stage.data(), bytes, hipMemcpyHostToDevice));
     m->weight_bytes += bytes;
+    return 0;
+}
+// the wide form of an uploaded matrix (prompt blocks; a draft head takes none): not counted into weight_bytes
+static int wide_form(lg_hip_model *m, const uint8_t *tiles, int k, int rows, bool rowblocks, uint8_t **out) {
+    if (m->target) return 0;
+    if (dev_alloc(m, out, lg_wide_bytes(k, rows))) return -7;
+    const size_t n = (size_t)((rows + LG_WT - 1) / LG_WT * LG_WT) * (size_t)(k >> 5);
+    hipLaunchKernelGGL(lg_k_wide_pack, dim3((unsigned)((n + LG_WG - 1) / LG_WG)), dim3(LG_WG), 0, nullptr, tiles, k, rows, rowblocks ? 1 : 0, *out);
+    HIP_TRY(hipGetLastError());
     return 0;
 }
 static void push_rows(std::vector<const uint8_t *> &rows, const HostTensor *t, uint64_t r0, uint64_t n) {
@@ -572,6 +586,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
             std::vector<const uint8_t *> rows;
             push_rows(rows, p, 0, total);
             if ((rc = upload_tiled(m, rows, E, &m->pmp, stage))) return rc;
+            if ((rc = wide_form(m, m->pmp, E, (int)total, false, &m->pmp_w))) return rc;
         }
         if ((rc = upload_vec(m, "per_layer_proj_norm.weight", m->ple, true, &m->proj_norm))) return rc;
     } else m->ple = 0;
@@ -619,11 +634,13 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
             }
         }
         if ((rc = upload_tiled(m, rows, E, &y.wqkv, stage))) return rc;
+        if ((rc = wide_form(m, y.wqkv, E, y.qkv_m, false, &y.wqkv_w))) return rc;
         rows.clear();
         const HostTensor *o = find(m, lname(L, "attn_output.weight"));
         if ((rc = check_mat(o, lname(L, "attn_output.weight"), y.qd, E))) return rc;
         push_rows(rows, o, 0, E);
         if ((rc = upload_tiled(m, rows, y.qd, &y.wo, stage))) return rc;
+        if ((rc = wide_form(m, y.wo, y.qd, E, false, &y.wo_w))) return rc;
         // (8 query heads: the K segments of this projection are the heads, and the merge can run their chains itself)
         if (getenv("LG_HIP_XCD_ATTN_TAIL") && atoi(getenv("LG_HIP_XCD_ATTN_TAIL")) > 0 && !m->target && attn_tail_shape(y.qd, E, nullptr, nullptr) &&
             cu_count() == LG_XCDS * LG_XCD_WGS) {
@@ -643,9 +660,11 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         if ((rc = check_mat(d, lname(L, "ffn_down.weight"), y.nff, E))) return rc;
         for (int t = 0; t < y.nff / 32; ++t) { push_rows(rows, g, (uint64_t)t * 32, 32); push_rows(rows, u, (uint64_t)t * 32, 32); }
         if ((rc = upload_tiled(m, rows, E, &y.wgu, stage, true))) return rc;    // row-block tiles (lg_k_geglu_t)
+        if ((rc = wide_form(m, y.wgu, E, 2 * y.nff, true, &y.wgu_w))) return rc;
         rows.clear();
         push_rows(rows, d, 0, E);
         if ((rc = upload_tiled(m, rows, y.nff, &y.wdown, stage))) return rc;
+        if ((rc = wide_form(m, y.wdown, y.nff, E, false, &y.wdown_w))) return rc;
         rows.clear();
         if (!(getenv("LG_HIP_DOWN_M") && atoi(getenv("LG_HIP_DOWN_M")) <= 0) && !m->target && max_rows >= 4 && cu_count() == LG_XCDS * LG_XCD_WGS) {
             const DownMGeo dg = lg_down_m_geo(E, y.nff);
@@ -682,9 +701,11 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
             if ((rc = check_mat(pj, lname(L, "proj.weight"), m->ple, E))) return rc;
             push_rows(rows, ig, 0, m->ple);
             if ((rc = upload_tiled(m, rows, E, &y.winp, stage))) return rc;
+            if ((rc = wide_form(m, y.winp, E, m->ple, false, &y.winp_w))) return rc;
             rows.clear();
             push_rows(rows, pj, 0, E);
             if ((rc = upload_tiled(m, rows, m->ple, &y.wproj, stage))) return rc;
+            if ((rc = wide_form(m, y.wproj, m->ple, E, false, &y.wproj_w))) return rc;
             }
             if ((rc = upload_vec(m, lname(L, "post_norm.weight"), E, true, &y.post_norm))) return rc;
         }
@@ -723,13 +744,15 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
     // draft head (it is never prefilled).  What only the head touches (final-norm rows, per-workgroup maxima, logits)
     // holds max_rows: a prompt block has no head.
     const size_t R = (size_t)(m->target || max_rows > LG_WIDE_ROWS ? max_rows : LG_WIDE_ROWS), HR = (size_t)max_rows;
+    // a q8 row is 5/4 bytes per value in a verify block and 13/8 as the digits of a prompt block (tiles of 64 rows)
+    auto qb = [&](int k) { return m->target ? R * k * 5 / 4 : lg_wide_q8_bytes((int)R, k) + 256; };
     if (dev_alloc(m, &m->x[0], R * E) || dev_alloc(m, &m->x[1], R * E) || dev_alloc(m, &m->qkv, R * max_qkv) ||
         dev_alloc(m, &m->dout, 4 * R * E) || dev_alloc(m, &m->q_rot, R * max_qd) || dev_alloc(m, &m->hidden_rows, HR * E) || dev_alloc(m, &m->g_hidden, (size_t)E) ||
-        dev_alloc(m, &m->aq, R * max_qd * 5 / 4) || dev_alloc(m, &m->gq, R * max_ff * 5 / 4) || dev_alloc(m, &m->hq, R * E * 5 / 4 + (size_t)12 * E) ||
+        dev_alloc(m, &m->aq, qb(max_qd)) || dev_alloc(m, &m->gq, qb(max_ff)) || dev_alloc(m, &m->hq, qb(E) + (size_t)12 * E) ||
         dev_alloc(m, &m->pval, HR * (m->n_vocab / 32)) || dev_alloc(m, &m->pidx, HR * (m->n_vocab / 32)) ||
         dev_alloc(m, &m->logits, HR * m->n_vocab) || dev_alloc(m, &m->ctl, (size_t)1))
         return -7;
-    if (m->ple && dev_alloc(m, &m->eq, R * E * 5 / 4 + (size_t)12 * E)) return -7;
+    if (m->ple && dev_alloc(m, &m->eq, qb(E) + (size_t)12 * E)) return -7;
     if (!m->target) {                        // hand-over state of the one-XCD kernels (lg_xtail.h)
         if (dev_alloc(m, &m->tsync, (size_t)1) || dev_alloc(m, &m->tstamps, (size_t)2 * LG_XTAIL_UNITS * 8) ||
             dev_alloc(m, &m->tgf, (size_t)LG_HIP_MAX_ROWS * (m->ple > 0 ? m->ple : 1))) return -7;
@@ -737,14 +760,14 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         HIP_TRY(hipMemset(m->tsync, 0, sizeof(XtailSync)));
         if (dev_alloc(m, &m->rgsync, (size_t)1)) return -7;
         HIP_TRY(hipMemset(m->rgsync, 0, sizeof(RgSync)));
-        HIP_TRY(hipMemset(m->aq, 0, R * max_qd * 5 / 4));       // (row slots past the block are read as operand rows of the matrix cores)
+        HIP_TRY(hipMemset(m->aq, 0, qb(max_qd)));       // (row slots past the block are read as operand rows of the matrix cores)
         if (getenv("LG_HIP_XCD_TAIL")) m->xcd_tail = atoi(getenv("LG_HIP_XCD_TAIL"));
     }
     if (getenv("LG_HIP_XCD_ATTN_TAIL")) m->xcd_attn_tail = atoi(getenv("LG_HIP_XCD_ATTN_TAIL"));
     if (getenv("LG_HIP_DOWN_M")) m->down_m = atoi(getenv("LG_HIP_DOWN_M"));
     if (getenv("LG_HIP_MERGE_O")) m->merge_o = atoi(getenv("LG_HIP_MERGE_O"));
     if (getenv("LG_HIP_MERGE_O_SLICES")) m->merge_o_slices = atoi(getenv("LG_HIP_MERGE_O_SLICES"));
-    if (m->ple && (dev_alloc(m, &m->pmp_raw, R * m->ple * nl) || dev_alloc(m, &m->pq, R * m->ple * 5 / 4) || dev_alloc(m, &m->pgf, R * m->ple)))
+    if (m->ple && (dev_alloc(m, &m->pmp_raw, R * m->ple * nl) || dev_alloc(m, &m->pq, qb(m->ple)) || dev_alloc(m, &m->pgf, R * m->ple)))
         return -7;
     if (xffn) {
         if (dev_alloc(m, &m->slabs, (size_t)LG_XCDS * max_rows * E) || dev_alloc(m, &m->xact, (size_t)LG_XCDS * max_rows * xg.C) ||
@@ -758,11 +781,11 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
     HIP_TRY(hipMemset(m->ctl, 0, sizeof(StepCtl)));
     HIP_TRY(hipMemset(m->g_hidden, 0, (size_t)E * 4));
     m->sched_cap = 4096;
-    if (dev_alloc(m, &m->sched, (size_t)m->sched_cap * LG_HIP_MAX_ROWS + LG_WIDE_ROWS) || dev_alloc(m, &m->out, (size_t)m->sched_cap * LG_HIP_MAX_ROWS) ||
+    if (dev_alloc(m, &m->sched, (size_t)m->sched_cap * LG_HIP_MAX_ROWS) || dev_alloc(m, &m->out, (size_t)m->sched_cap * LG_HIP_MAX_ROWS) ||
         dev_alloc(m, &m->adv, (size_t)m->sched_cap))
         return -7;
-    // pinned staging: step state at 0, a verify block's successors at 32 and accept count at 48, a block's tokens from 64
-    HIP_TRY(hipHostMalloc((void **)&m->pin, (64 + LG_WIDE_ROWS) * sizeof(int32_t), hipHostMallocDefault));
+    // pinned staging: step state at 0, a verify block's successors at 32 and accept count at 48, a block's or a prompt's tokens from 64
+    HIP_TRY(hipHostMalloc((void **)&m->pin, (64 + (size_t)m->sched_cap * LG_HIP_MAX_ROWS) * sizeof(int32_t), hipHostMallocDefault));
     HIP_TRY(hipDeviceSynchronize());
     m->committed = true;
     return 0;
@@ -786,6 +809,19 @@ extern "C" void lg_hip_model_destroy(lg_hip_model *m) {
     if (m->ev_join) (void)hipEventDestroy(m->ev_join);
     for (lg_hip_model *d : m->drafts) { d->target = nullptr; d->stream = nullptr; }        // orphaned heads refuse to run
     delete m;
+}
+
+// Key tiles that the attention of a prompt block can touch per group of rows, and the scratch it keeps their weights in
+// when they are too many for LDS.
+static int wide_attn_tiles(const lg_hip_model *m, const Layer &y, int rows, int pos) {
+    const int rg = lg_wide_attn_rows(m->H / y.nkv), all = ((pos + rows - 1) >> 5) + 1;
+    if (!(y.is_local && m->window > 0)) return all;
+    const int t = (m->window + rg - 1 + 31) / 32 + 1;
+    return t < all ? t : all;
+}
+static size_t wide_attn_scratch(const lg_hip_model *m, const Layer &y, int rows, int pos) {
+    const int rg = lg_wide_attn_rows(m->H / y.nkv), tiles = wide_attn_tiles(m, y, rows, pos);
+    return tiles <= LG_WA_TILES ? 0 : (size_t)((rows + rg - 1) / rg) * y.nkv * tiles * (16 * 34 * 4);
 }
 
 // ---- KV cache ---------------------------------------------------------------------------------
@@ -817,6 +853,15 @@ extern "C" int lg_hip_kv_create(lg_hip_model *m, int max_seq, lg_hip_kv **out) {
         (void)hipMemset(kv->k[L], 0, bytes); (void)hipMemset(kv->v[L], 0, bytes);
     }
     const size_t slots = pbytes / ((size_t)max_hd * 4 + 8);
+    kv->scratch_bytes = slots * max_hd * 4;
+    for (kv->prompt_rows = wide_rows_for(max_seq); kv->prompt_rows > LG_WIDE; kv->prompt_rows -= LG_WIDE) {
+        size_t most = 0;
+        for (int L = 0; L < nl; ++L) {
+            const size_t n = wide_attn_scratch(m, m->L[L], kv->prompt_rows, max_seq - kv->prompt_rows > 0 ? max_seq - kv->prompt_rows : 0);
+            most = n > most ? n : most;
+        }
+        if (most <= kv->scratch_bytes) break;
+    }
     if (hipMalloc((void **)&kv->pm, slots * 4) != hipSuccess || hipMalloc((void **)&kv->pl, slots * 4) != hipSuccess ||
         hipMalloc((void **)&kv->pacc, slots * max_hd * 4) != hipSuccess) { lg_hip_kv_destroy(kv); return fail(-7, "kv_create: out of device memory for attention partials"); }
     HIP_TRY(hipDeviceSynchronize());
@@ -907,6 +952,8 @@ extern "C" int lg_hip_kv_restore_prefix(lg_hip_kv *kv, int n) {
     return 0;
 }
 
+__global__ void lg_k_set_ctl(StepCtl *ctl, int pos) { ctl->pos = pos; ctl->step = 0; ctl->err = 0; ctl->pad = 0; }
+
 // ---- launching --------------------------------------------------------------------------------
 static size_t lds_mm(int M, int k) { return (size_t)M * k + (size_t)M * (k / 32) * 8; }
 // lg_k_attn: queries of the G heads, K and V tiles, exponentials; with the q/k/v preparation fused in, a head
@@ -990,14 +1037,6 @@ template <int M, bool DUMP>
 static int launch_mm(Launcher &lx, int cls, const MmArgs &a_in, bool slabs_ok = false) {
     MmArgs a = a_in;                                      // (+ the workgroup size of the launch, set below)
     const int S = lg_segments(a.k), rw = 64 / S, ngroups = a.m / rw;
-    if constexpr (M > LG_HIP_MAX_ROWS) {                 // wide (prefill) block: matrix-core kernels, 32 weight rows per workgroup
-        if (a.m % 32) { lx.rc = fail(-2, "wide matmul: %d rows is not a multiple of 32", a.m); return 1; }
-        // S = 32: four workgroups per row block, each a quarter of the K segments, writing its own slab of a.out
-        const dim3 grid(a.m / 32, (M + LG_WIDE - 1) / LG_WIDE, S == 32 ? 4 : 1);
-        if (S == 32) LAUNCH(cls, (lg_k_mm_wide<M, 32, DUMP>), grid, dim3(LG_WIDE_WG), MfmaGeo::lds_bytes, a, M);
-        else         LAUNCH(cls, (lg_k_mm_wide<M, 8, DUMP>), grid, dim3(LG_WIDE_WG), MfmaGeo::lds_bytes, a, M);
-        return S == 32 ? 4 : 1;
-    } else {
     const size_t lds = lds_mm(M, a.k);
     if (S == 32 && M >= 4 && slabs_ok && !DUMP) {
         // blocks of four and more rows whose consumer adds four slabs: cut by K quarter (a quarter of the activations
@@ -1041,8 +1080,6 @@ static int launch_mm(Launcher &lx, int cls, const MmArgs &a_in, bool slabs_ok = 
         a.nthreads = 64 * W;
         LAUNCH(cls, (lg_k_mm<M, 8, 1, DUMP>), dim3((ngroups + W - 1) / W), dim3(64 * W), lds, LG_MM_FIELDS(LG_XA, a) 0);
     }
-    }
-    (void)rw; (void)ngroups;
     return 1;
 }
 
@@ -1062,32 +1099,6 @@ static bool attention_rows_shared(int rows, int tiles, int nkv, int hd, int seq)
 static int attention_rows_tp(int tiles, int nkv) {
     const int tp = (tiles * nkv + 3 * 256 - 1) / (3 * 256);
     return tp < 1 ? 1 : tp > 4 ? 4 : tp;
-}
-
-// lg_k_attn_u (prompt blocks, queries in registers, a wavefront per (row, head) unit, 8 units per workgroup): rows of
-// the block per workgroup, 0 when the shape does not fit
-static int attention_u_rows(int rows, int G, int hd, int seq) {
-    if (rows <= LG_HIP_MAX_ROWS || seq < 32 || (hd != 64 && hd != 128 && hd != 256 && hd != 512)) return 0;
-    if (G < 1 || G > 8 || 8 % G) return 0;
-    const int rw = 8 / G;
-    return rows % rw == 0 ? rw : 0;
-}
-// launch geometry: tiles a row group can touch, tiles per workgroup (so that the grid has about two workgroups per CU)
-template <typename L>
-static int attention_u_launch(L &&launch, int rows, int rw, int nkv, int hd, int window, int block_tiles) {
-    int nt = block_tiles;
-    if (window > 0) { const int t = (window + rw - 1 + 31) / 32 + 1; if (t < nt) nt = t; }
-    const int groups = rows / rw;
-    int tp = (int)(((long long)nt * nkv * groups + 511) / 512);
-    if (tp < 1) tp = 1;
-    if (tp > nt) tp = nt;
-    const dim3 grid((nt + tp - 1) / tp, nkv, groups);
-    switch (hd) {
-        case 512: return launch(lg_k_attn_u<512>, grid, AttnUGeo<512>::bytes(8), tp);
-        case 256: return launch(lg_k_attn_u<256>, grid, AttnUGeo<256>::bytes(8), tp);
-        case 128: return launch(lg_k_attn_u<128>, grid, AttnUGeo<128>::bytes(8), tp);
-        default:  return launch(lg_k_attn_u<64>, grid, AttnUGeo<64>::bytes(8), tp);
-    }
 }
 
 // the XCD-partitioned feed-forward launch: 256 workgroups of 512 threads, the instantiation of the shape's class
@@ -1266,7 +1277,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
     // rows kernel: fold the pending sub-layer output into the residual, norm with w_pre, quantize
     auto rows = [&](const float *w_pre, float *h_out, int units = 0, int8_t *q_out = nullptr) {
         RowArgs s{};
-        s.q_units = M <= LG_HIP_MAX_ROWS ? units : 0;
+        s.q_units = units;
         s.E = E; s.eps = m->eps; s.toks = m->sched; s.q = q_out ? q_out : m->hq;
         if (!have_x) {
             s.emb = m->emb; s.emb_seg = lg_segments(E); s.emb_nit = E / 32 / s.emb_seg; s.emb_scale = sqrtf((float)E);
@@ -1276,7 +1287,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         s.w_pre = w_pre; s.h_out = h_out;
         if (pend_dout || !have_x) s.x_out = m->x[cur ^ 1];
         // verify blocks: the tail of the row work (store, norm weight, q8) cut over one workgroup per float4 of a lane
-        const int slices = M <= LG_HIP_MAX_ROWS ? (E + 1023) / 1024 : 1;
+        const int slices = (E + 1023) / 1024;
         s.slices = slices;
         LAUNCH(KC_ROWS, (lg_k_rows<M>), dim3(M, slices), dim3(LG_WG), 0, m->ctl, LG_ROW_FIELDS(LG_XA, s) 0);
         if (s.x_out) cur ^= 1;
@@ -1372,7 +1383,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             else if (can_fuse()) rows_mm(y.attn_norm, a, KC_QKV);
             else { rows(y.attn_norm, nullptr); launch_mm<M, false>(lx, KC_QKV, a); }
             // blocks of the model itself, up to LG_HIP_MAX_ROWS rows: the attention kernel does this part as well
-            fused_post = M <= LG_HIP_MAX_ROWS && (pos_off == 0 || !y.owns);    // (a draft head's layers own no cache: queries only)
+            fused_post = pos_off == 0 || !y.owns;    // (a draft head's layers own no cache: queries only)
             // ... unless the layer has so many (tile, kv head) pairs that one workgroup per pair can serve all rows of
             // the block against one staged tile (long global contexts, wide windows): the rows then arrive prepared
             // (that kernel prepares them itself while it has few workgroups: each of them repeats the preparation of its kv
@@ -1400,15 +1411,6 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             const int tiles = layer_tiles(L);
             a.gx = tiles; a.gz = M;
             const bool shared = rows_shared(L);
-            // prompt blocks (the queries arrive prepared: lg_k_qkv_post ran): eight (row, head) units per workgroup with the
-            // queries in registers
-            const int urows = (!fused_post && pos_off == 0 && m->attn_rows) ? attention_u_rows(M, G, y.hd, kv->seq[y.src]) : 0;
-            if (urows) {
-                attention_u_launch([&](auto kernel, dim3 grid, size_t lds, int tp) {
-                    LAUNCH(KC_ATTN, kernel, grid, dim3(512), lds, a, m->ctl, urows, tp);
-                    return 0;
-                }, M, urows, y.nkv, y.hd, window, tiles);
-            } else
             if (shared) {
                 if constexpr (M > 1 && M <= LG_HIP_MAX_ROWS) {
                     const size_t lds = y.hd == 256 ? AttnRowsGeo<256>::bytes(M * G, fused_post) : y.hd == 128 ? AttnRowsGeo<128>::bytes(M * G, fused_post) : AttnRowsGeo<64>::bytes(M * G, fused_post);
@@ -1467,7 +1469,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         {   // feed-forward: gate/up + GeGLU, then down
             // verify blocks: 1..3 rows through v_dot4 with scalar operands, 4..8 rows through the matrix cores
             // (its float work per tile does not grow with the row count); each has its own activation order
-            constexpr bool mfma = M >= 4 && M <= LG_HIP_MAX_ROWS;
+            constexpr bool mfma = M >= 4;
             if (mfma && m->xffn_built && m->xcd_ffn && y.xgu && have_x && pend_dout && pend_parts == 1 && !pend_os) {
                 // the whole half as one launch partitioned by XCD: row work, gate/up + GeGLU and the XCD's K share of
                 // ffn_down; the consumer adds the 8 slabs (the top of the segment tree)
@@ -1501,9 +1503,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             if (rows_in_geglu) {
             } else {
             if (!ffn_rows_done) rows(y.ffn_norm, nullptr, mfma ? 2 : 1);
-            if constexpr (M > LG_HIP_MAX_ROWS)
-                LAUNCH(KC_GATEUP, (lg_k_mm_geglu_wide<M>), dim3(y.nff / 32, (M + LG_WIDE - 1) / LG_WIDE), dim3(LG_WIDE_WG), MfmaGeo::lds_bytes, a, M);
-            else if constexpr (mfma)
+            if constexpr (mfma)
                 LAUNCH(KC_GATEUP, (lg_k_geglu_m<M>), dim3(y.nff / 32), dim3(512), (size_t)(E / 32) * LG_MU_DWORDS * 4, LG_GEGLU_FIELDS(LG_XA, a) 0);
             else
                 LAUNCH(KC_GATEUP, (lg_k_geglu_t<M>), dim3(y.nff / 32), dim3(512), 0, LG_GEGLU_FIELDS(LG_XA, a) 0);
@@ -1531,10 +1531,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         } else
         if (m->ple) {   // per-layer embedding block
             PleGateArgs a{ y.winp, E, m->ple, m->hq, m->pmp_raw, L, nl, m->pq };
-            if constexpr (M > LG_HIP_MAX_ROWS) {
-                rows(nullptr, nullptr);
-                LAUNCH(KC_PLEGATE, (lg_k_mm_plegate_wide<M>), dim3(m->ple / 32, (M + LG_WIDE - 1) / LG_WIDE), dim3(LG_WIDE_WG), MfmaGeo::lds_bytes, a, M);
-            } else if (tail && (L + 1 < nl || with_head) && pend_dout && have_x && !pend_os) {
+            if (tail && (L + 1 < nl || with_head) && pend_dout && have_x && !pend_os) {
                 // the whole block and the row work that follows it (the next layer's, or the head's) in one launch on one XCD
                 const bool last = L + 1 == nl;
                 const bool head_m = M >= 4 && m->emb_rb && m->head_mfma;
@@ -1564,11 +1561,6 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         }
     }
     join();
-    if constexpr (M > LG_HIP_MAX_ROWS) {
-        if (with_head) return fail(-2, "a wide block has no head: verify blocks hold at most %d rows", LG_HIP_MAX_ROWS);
-        if (!lx.rc && !dry) hipLaunchKernelGGL(lg_k_advance, dim3(1), dim3(1), 0, m->stream, m->ctl, M);
-        return lx.rc;
-    } else
     if (with_head && !lx.rc) {
         const bool head_m = M >= 4 && m->emb_rb && m->head_mfma;
         if (!rows_done) rows(m->output_norm, m->hidden_rows, head_m ? 2 : 0);
@@ -1590,6 +1582,125 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
     return lx.rc;
 }
 
+// ---- prompt blocks ------------------------------------------------------------------------------
+// A matmul of a prompt block (lg_wide.h).  The workgroup's shape: 64 weight rows x 64 activation rows by four wavefronts
+// of two K segments each; 32 activation rows when the block has no more; and where 64 x 32 tiles would leave some CU
+// without a workgroup, eight wavefronts of one segment on such a tile (3072 x 2560, 32 rows, 48 workgroups: 8.8 -> 7.1 us).
+struct WideShape { int tb, wv; };
+static WideShape wide_shape(int m, int rows, int parts) {
+    if (((m + LG_WT - 1) / LG_WT) * ((rows + 31) / 32) * parts <= 256) return { 1, 8 };
+    return { rows <= 32 ? 1 : 2, 4 };
+}
+template <bool DUMP>
+static int launch_wide_mm(Launcher &lx, int cls, const uint8_t *w, const int8_t *q, int k, int m, int rows, float *out, int32_t *dots) {
+    const int parts = lg_segments(k) / 8;
+    const WideShape c = wide_shape(m, rows, parts);
+    const WideMm a{ w, (const uint8_t *)q, k, m, rows, (rows + 32 * c.tb - 1) / (32 * c.tb), parts };
+    const dim3 grid(lg_wide_grid(m, a.nb_tiles, parts)), block(64 * c.wv);
+    const size_t lds = (size_t)c.wv * 2 * c.tb * 4096;
+    if (c.wv == 8)      LAUNCH(cls, (lg_k_wide_mm<1, 8, DUMP>), grid, block, lds, a, out, dots);
+    else if (c.tb == 1) LAUNCH(cls, (lg_k_wide_mm<1, 4, DUMP>), grid, block, lds, a, out, dots);
+    else                LAUNCH(cls, (lg_k_wide_mm<2, 4, DUMP>), grid, block, lds, a, out, dots);
+    return parts;
+}
+template <int HD>
+static void launch_wide_attn(Launcher &lx, const WideAttn &a, int groups) {
+    const dim3 grid(groups, a.nkv);
+    if (a.tiles <= LG_WA_TILES) LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, true>), grid, dim3(LG_WG), lg_wide_attn_lds(a.tiles), a, lx.m->ctl);
+    else                        LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false>), grid, dim3(LG_WG), 0, a, lx.m->ctl);
+}
+
+// One block of `rows` prompt positions from pos on (tokens in device memory): the launch sequence of a verify step with
+// the kernels of lg_wide.h.  Launched as it is, not captured: a prompt's blocks differ in width and tile counts, and the
+// host stays ahead of launches of this size.
+static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int rows, int pos) {
+    Launcher lx{ m, false };
+    const int E = m->E, H = m->H, nl = m->n_layer;
+    int cur = 0;
+    bool have_x = false;
+    const float *pend_dout = nullptr, *pend_w = nullptr, *pend_os = nullptr;
+    int pend_parts = 1;
+    hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, m->stream, m->ctl, pos);
+    auto row_work = [&](const float *w_pre, int8_t *q) {
+        RowArgs s{};
+        s.E = E; s.eps = m->eps; s.toks = toks; s.q = q;
+        if (!have_x) { s.emb = m->emb; s.emb_seg = lg_segments(E); s.emb_nit = E / 32 / s.emb_seg; s.emb_scale = sqrtf((float)E); }
+        else s.x = m->x[cur];
+        s.dout = pend_dout; s.w_post = pend_w; s.os = pend_os; s.dparts = pend_parts;
+        s.w_pre = w_pre;
+        if (pend_dout || !have_x) s.x_out = m->x[cur ^ 1];
+        LAUNCH(KC_ROWS, lg_k_wide_rows, dim3(rows), dim3(LG_WG), 0, s, rows);
+        if (s.x_out) cur ^= 1;
+        have_x = true; pend_dout = pend_w = pend_os = nullptr; pend_parts = 1;
+    };
+    if (m->ple) {
+        row_work(nullptr, m->eq);
+        if (m->pmp_f) {
+            MmfArgs f{ m->pmp_f, E, m->ple * nl, m->x[cur], E, rows, m->pmp_raw, m->ple * nl, nullptr, 0 };
+            launch_mmf<LG_HIP_MAX_ROWS>(lx, KC_PMP, f);
+        } else launch_wide_mm<false>(lx, KC_PMP, m->pmp_w, m->eq, E, m->ple * nl, rows, m->pmp_raw, nullptr);
+        IplArgs i{ m->pmp_raw, m->ple, nl, rows, m->proj_norm, m->pte, toks,
+                   1.0f / sqrtf((float)E), sqrtf((float)m->ple), 1.0f / sqrtf(2.0f), m->eps };
+        LAUNCH(KC_PMP, lg_k_ipl, dim3(nl, rows), dim3(64), 0, i, m->ctl);
+    }
+    for (int L = 0; L < nl && !lx.rc; ++L) {
+        const Layer &y = m->L[L];
+        const int window = (y.is_local && m->window > 0) ? m->window : 0;
+        row_work(y.attn_norm, m->hq);
+        launch_wide_mm<false>(lx, KC_QKV, y.wqkv_w, m->hq, E, y.qkv_m, rows, m->qkv, nullptr);
+        QkvPostArgs p{};
+        p.qkv = m->qkv; p.ld = y.qkv_m; p.k_off = y.k_off; p.v_off = y.v_off;
+        p.H = H; p.nkv = y.nkv; p.hd = y.hd;
+        p.q_norm = y.q_norm; p.k_norm = y.k_norm; p.rope_tab = y.rope_tab; p.rope_ff = y.rope_ff;
+        p.q_rot = m->q_rot;
+        p.kc = y.owns ? kv->k[L] : nullptr; p.vc = y.owns ? kv->v[L] : nullptr;
+        p.seq = kv->seq[y.src]; p.kv_dim = y.kd; p.eps = m->eps;
+        LAUNCH(KC_QKVPOST, lg_k_qkv_post, dim3(H + (y.owns ? 2 * y.nkv : 0), rows), dim3(64), 0, p, m->ctl);
+        const int rg = lg_wide_attn_rows(H / y.nkv), groups = (rows + rg - 1) / rg;
+        const WideAttn a{ m->q_rot, kv->k[y.src], kv->v[y.src], H, y.nkv, kv->seq[y.src], y.kd, window, rows, kv->pacc,
+                          wide_attn_tiles(m, y, rows, pos), (uint8_t *)m->aq };
+        switch (y.hd) {
+            case 512: launch_wide_attn<512>(lx, a, groups); break;
+            case 256: launch_wide_attn<256>(lx, a, groups); break;
+            case 128: launch_wide_attn<128>(lx, a, groups); break;
+            default:  launch_wide_attn<64>(lx, a, groups);
+        }
+        pend_parts = launch_wide_mm<false>(lx, KC_O, y.wo_w, m->aq, y.qd, E, rows, m->dout, nullptr);
+        pend_dout = m->dout; pend_w = y.post_attn;
+        row_work(y.ffn_norm, m->hq);
+        {
+            const WideShape c = wide_shape(2 * y.nff, rows, 1);
+            const WideMm g{ y.wgu_w, (const uint8_t *)m->hq, E, 2 * y.nff, rows, (rows + 32 * c.tb - 1) / (32 * c.tb), 1 };
+            const dim3 grid(lg_wide_grid(g.m, g.nb_tiles, 1)), block(64 * c.wv);
+            const size_t lds = (size_t)c.wv * 2 * c.tb * 4096;
+            if (c.wv == 8)      LAUNCH(KC_GATEUP, (lg_k_wide_geglu<1, 8>), grid, block, lds, g, (uint8_t *)m->gq);
+            else if (c.tb == 1) LAUNCH(KC_GATEUP, (lg_k_wide_geglu<1, 4>), grid, block, lds, g, (uint8_t *)m->gq);
+            else                LAUNCH(KC_GATEUP, (lg_k_wide_geglu<2, 4>), grid, block, lds, g, (uint8_t *)m->gq);
+        }
+        pend_parts = launch_wide_mm<false>(lx, KC_DOWN, y.wdown_w, m->gq, y.nff, E, rows, m->dout, nullptr);
+        pend_dout = m->dout; pend_w = y.post_ffw; pend_os = m->ple ? nullptr : y.out_scale;
+        if (!m->ple) continue;
+        row_work(nullptr, y.winp_f ? nullptr : m->hq);
+        if (y.winp_f) {
+            MmfArgs g{ y.winp_f, E, m->ple, m->x[cur], E, rows, m->pgf, m->ple, m->pmp_raw + (size_t)L * m->ple, m->ple * nl };
+            launch_mmf<LG_HIP_MAX_ROWS>(lx, KC_PLEGATE, g);
+            MmfArgs pr{ y.wproj_f, m->ple, E, m->pgf, m->ple, rows, m->dout, E, nullptr, 0 };
+            launch_mmf<LG_HIP_MAX_ROWS>(lx, KC_PLEPROJ, pr);
+            pend_parts = 1;
+        } else {
+            const WideShape c = wide_shape(m->ple, rows, 1);
+            const WideMm g{ y.winp_w, (const uint8_t *)m->hq, E, m->ple, rows, (rows + 32 * c.tb - 1) / (32 * c.tb), 1 };
+            const dim3 grid(lg_wide_grid(g.m, g.nb_tiles, 1)), block(64 * c.wv);
+            const size_t lds = (size_t)c.wv * 2 * c.tb * 4096;
+            if (c.wv == 8) LAUNCH(KC_PLEGATE, (lg_k_wide_plegate<1, 8>), grid, block, lds, g, m->pmp_raw, L, nl, (uint8_t *)m->pq);
+            else           LAUNCH(KC_PLEGATE, (lg_k_wide_plegate<2, 4>), grid, block, lds, g, m->pmp_raw, L, nl, (uint8_t *)m->pq);
+            pend_parts = launch_wide_mm<false>(lx, KC_PLEPROJ, y.wproj_w, m->pq, m->ple, E, rows, m->dout, nullptr);
+        }
+        pend_dout = m->dout; pend_w = y.post_norm; pend_os = y.out_scale;
+    }
+    return lx.rc;
+}
+
 static int enqueue_step_rows(lg_hip_model *m, lg_hip_kv *kv, int rows, bool with_head, bool dry = false) {
     switch (rows) {
         case 1: return enqueue_step<1>(m, kv, with_head, dry);
@@ -1600,9 +1711,6 @@ static int enqueue_step_rows(lg_hip_model *m, lg_hip_kv *kv, int rows, bool with
         case 6: return enqueue_step<6>(m, kv, with_head, dry);
         case 7: return enqueue_step<7>(m, kv, with_head, dry);
         case 8: return enqueue_step<8>(m, kv, with_head, dry);
-        case LG_WIDE: return enqueue_step<LG_WIDE>(m, kv, with_head, dry);
-        case LG_WIDE_MID: return enqueue_step<LG_WIDE_MID>(m, kv, with_head, dry);
-        case LG_WIDE_ROWS: return enqueue_step<LG_WIDE_ROWS>(m, kv, with_head, dry);
     }
     return fail(-2, "rows %d outside 1..%d", rows, LG_HIP_MAX_ROWS);
 }
@@ -1631,9 +1739,9 @@ static int launch_step(lg_hip_model *m, lg_hip_kv *kv, int rows, bool with_head)
     return 0;
 }
 
-static int check_block(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int n, int rows, int pos, bool wide = false) {
+static int check_block(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int n, int rows, int pos) {
     if (!m || !kv || !toks || kv->m != m) return fail(-1, "bad model / cache / token pointer");
-    if (rows < 1 || (rows > m->max_rows && !(wide && (rows == LG_WIDE || rows == LG_WIDE_MID || rows == LG_WIDE_ROWS)))) return fail(-2, "block of %d rows; the model was committed for 1..%d", rows, m->max_rows);
+    if (rows < 1 || rows > m->max_rows) return fail(-2, "block of %d rows; the model was committed for 1..%d", rows, m->max_rows);
     if (pos < 0 || pos + rows > kv->max_seq) return fail(-2, "positions %d..%d do not fit a cache of %d", pos, pos + rows - 1, kv->max_seq);
     for (int i = 0; i < n; ++i) if (toks[i] < 0 || toks[i] >= m->n_vocab) return fail(-2, "token id %d outside the vocabulary of %d", toks[i], m->n_vocab);
     return 0;
@@ -1821,23 +1929,32 @@ extern "C" int lg_hip_mtp_rounds(lg_hip_model *d, lg_hip_kv *kv, int token, int 
 extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int n, int pos0) {
     if (n <= 0) return 0;
     if (!m) return fail(-1, "prefill: null model");
+    if (!kv || !toks || kv->m != m) return fail(-1, "bad model / cache / token pointer");
+    if (pos0 < 0 || n > kv->max_seq - pos0) return fail(-2, "positions %d..%lld do not fit a cache of %d", pos0, (long long)pos0 + n - 1, kv->max_seq);
+    for (int i = 0; i < n; ++i) if (toks[i] < 0 || toks[i] >= m->n_vocab) return fail(-2, "token id %d outside the vocabulary of %d", toks[i], m->n_vocab);
     HIP_TRY(hipSetDevice(m->device));
-    bool wide_ok = !m->target && m->wide_prefill;
-    for (int L = 0; L < m->n_layer && wide_ok; ++L) {
-        const Layer &y = m->L[L];
-        wide_ok = y.qkv_m % 32 == 0 && y.nff % 32 == 0;
-    }
-    for (int done = 0; done < n;) {
-        int rows = n - done < m->max_rows ? n - done : m->max_rows;
-        if (wide_ok && n - done >= LG_WIDE_ROWS && kv->wide_rows >= LG_WIDE_ROWS) rows = LG_WIDE_ROWS;     // matrix-core blocks while the prompt lasts,
-        else if (wide_ok && n - done >= LG_WIDE_MID && kv->wide_rows >= LG_WIDE_MID) rows = LG_WIDE_MID;
-        else if (wide_ok && n - done >= LG_WIDE && kv->wide_rows >= LG_WIDE) rows = LG_WIDE;        // a single row tile, then verify-width blocks for the tail
-        int rc = check_block(m, kv, toks + done, rows, rows, pos0 + done, true);
-        if (rc) return rc;
-        if ((rc = load_block(m, toks + done, rows, pos0 + done))) return rc;
-        if ((rc = launch_step(m, kv, rows, false))) return rc;
-        HIP_TRY(hipStreamSynchronize(m->stream));       // the pinned staging is reused by the next block
-        done += rows;
+    const bool wide_ok = !m->target && m->wide_prefill;
+    const int cap = m->sched_cap * LG_HIP_MAX_ROWS;        // tokens the staging holds
+    for (int at = 0; at < n;) {
+        // the tokens go over once, the blocks follow each other on the stream and the host waits at the end
+        const int part = n - at < cap ? n - at : cap;
+        memcpy(m->pin + 64, toks + at, (size_t)part * 4);
+        HIP_TRY(hipMemcpyAsync(m->sched, m->pin + 64, (size_t)part * 4, hipMemcpyHostToDevice, m->stream));
+        for (int done = 0; done < part;) {
+            const int left = part - done;
+            int rows = left < kv->prompt_rows ? left : kv->prompt_rows, rc;
+            if (wide_ok && left > m->max_rows) rc = enqueue_prompt(m, kv, m->sched + done, rows, pos0 + at + done);
+            else {                                           // a remainder that fits a verify block
+                rows = left < m->max_rows ? left : m->max_rows;
+                if (done) HIP_TRY(hipMemcpyAsync(m->sched, m->pin + 64 + done, (size_t)rows * 4, hipMemcpyHostToDevice, m->stream));   // (its kernels read the schedule from its start)
+                hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, m->stream, m->ctl, pos0 + at + done);
+                rc = wide_ok ? enqueue_step_rows(m, kv, rows, false) : launch_step(m, kv, rows, false);    // (a single one: not worth a capture)
+            }
+            if (rc) return rc;
+            done += rows;
+        }
+        at += part;
+        HIP_TRY(hipStreamSynchronize(m->stream));
     }
     return 0;
 }
@@ -2035,83 +2152,6 @@ static int matmul_rows(hipStream_t st, const uint8_t *dw, int k, int mrows, cons
     return rc;
 }
 
-extern "C" int lg_hip_matmul_f32w(const float *w, int k, int mrows, const float *x, int rows, float *out) {
-    if (!w || !x || !out) return fail(-1, "matmul_f32w: null argument");
-    if (k < 256 || k % 256 || mrows < 1 || rows < 1) return fail(-2, "matmul_f32w: k %d (a multiple of 256), m %d, rows %d", k, mrows, rows);
-    if (lg_hip_device_count() < 1) return fail(-3, "matmul_f32w: no HIP device");
-    Scratch sc;
-    float *dw, *dx, *dout;
-    if (sc.get(&dw, (size_t)mrows * k) || sc.get(&dx, (size_t)rows * k) || sc.get(&dout, (size_t)rows * mrows)) return -7;
-    HIP_TRY(hipMemcpy(dw, w, (size_t)mrows * k * 4, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(dx, x, (size_t)rows * k * 4, hipMemcpyHostToDevice));
-    MmfArgs a{ dw, k, mrows, dx, k, rows, dout, mrows, nullptr, 0 };
-    hipLaunchKernelGGL((lg_k_mmf<8>), dim3((mrows + LG_WG / 64 - 1) / (LG_WG / 64), (rows + 7) / 8), dim3(LG_WG), 0, nullptr, a);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipDeviceSynchronize());
-    HIP_TRY(hipMemcpy(out, dout, (size_t)rows * mrows * 4, hipMemcpyDeviceToHost));
-    return 0;
-}
-
-extern "C" int lg_hip_matmul_q4q8(const void *w, int k, int mrows, const float *x, int rows, float *out, int32_t *dots,
-                                  int8_t *xq, float *xd, int32_t *xsum, int repeats, float *kernel_ms) {
-    if (!w || !x) return fail(-1, "matmul: null input");
-    const bool wide = rows == LG_WIDE;                   // one full row tile through the matrix-core kernel
-    if (rows < 1 || (rows > LG_HIP_MAX_ROWS && !wide) || !lg_hip_repacked_bytes(k, mrows) || (!wide && lds_mm(rows, k) > 160 * 1024) || (wide && mrows % 32))
-        return fail(-2, "matmul: rows %d (1..%d, or %d with m %% 32 == 0), k %d (multiple of 256, rows*k*1.25 <= 160 KiB), m %d (multiple of 8)", rows, LG_HIP_MAX_ROWS, LG_WIDE, k, mrows);
-    if (lg_hip_device_count() < 1) return fail(-3, "matmul: no HIP device");
-    const int nb = k / 32;
-    std::vector<uint8_t> tiled(lg_hip_repacked_bytes(k, mrows));
-    int rc = lg_hip_repack_q4_0(w, k, mrows, tiled.data());
-    if (rc) return rc;
-    Scratch sc;
-    uint8_t *dw; float *dx, *dout; int32_t *ddots = nullptr; int8_t *dq;
-    if (sc.get(&dw, tiled.size()) || sc.get(&dx, (size_t)rows * k) || sc.get(&dout, (size_t)rows * mrows * 4) ||
-        sc.get(&dq, (size_t)rows * k * 5 / 4)) return -7;
-    if (dots && sc.get(&ddots, (size_t)rows * mrows * nb)) return -7;
-    HIP_TRY(hipMemcpy(dw, tiled.data(), tiled.size(), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(dx, x, (size_t)rows * k * 4, hipMemcpyHostToDevice));
-    hipStream_t st;
-    HIP_TRY(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-    switch (rows) {
-#define CASE(M) case M: rc = matmul_rows<M>(st, dw, k, mrows, dx, dout, ddots, dq, repeats, kernel_ms); break;
-        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(LG_WIDE)
-#undef CASE
-    }
-    (void)hipStreamDestroy(st);
-    if (rc) return rc;
-    if (out && wide && lg_segments(k) == 32) {             // four slabs of partial sums: the top of the segment tree is added here
-        std::vector<float> parts((size_t)4 * rows * mrows);
-        HIP_TRY(hipMemcpy(parts.data(), dout, parts.size() * 4, hipMemcpyDeviceToHost));
-        const size_t n = (size_t)rows * mrows;
-        for (size_t i = 0; i < n; ++i) out[i] = (parts[i] + parts[n + i]) + (parts[2 * n + i] + parts[3 * n + i]);
-    } else if (out) HIP_TRY(hipMemcpy(out, dout, (size_t)rows * mrows * 4, hipMemcpyDeviceToHost));
-    if (dots) HIP_TRY(hipMemcpy(dots, ddots, (size_t)rows * mrows * nb * 4, hipMemcpyDeviceToHost));
-    // the device keeps activation rows in the matmul's own order (lg_act_layout); hand them back in natural order
-    const ActLayout lay = lg_act_layout(k);
-    if (xq) {
-        std::vector<int8_t> dev((size_t)rows * k);
-        HIP_TRY(hipMemcpy(dev.data(), dq, dev.size(), hipMemcpyDeviceToHost));
-        for (int j = 0; j < rows; ++j)
-            for (int w = 0; w < k / 16; ++w) {
-                const int u = lg_act_unit(lay, w);
-                if (!wide) { memcpy(xq + (size_t)j * k + (size_t)w * 16, dev.data() + (size_t)j * k + (size_t)u * 16, 16); continue; }
-                for (int hh = 0; hh < 2; ++hh)           // wide layout: halves of a unit of all 32 rows side by side
-                    memcpy(xq + (size_t)j * k + (size_t)w * 16 + hh * 8, dev.data() + ((size_t)(u * 2 + hh) * 32 + j) * 8, 8);
-            }
-    }
-    if (xd || xsum) {
-        std::vector<float2> ds((size_t)rows * nb);
-        HIP_TRY(hipMemcpy(ds.data(), dq + (size_t)rows * k, ds.size() * 8, hipMemcpyDeviceToHost));
-        for (int j = 0; j < rows; ++j)
-            for (int b = 0; b < nb; ++b) {
-                const float2 v = wide ? ds[(size_t)lg_act_block(lay, b) * 32 + j] : ds[(size_t)j * nb + lg_act_block(lay, b)];
-                if (xd) xd[(size_t)j * nb + b] = v.x;
-                if (xsum) memcpy(&xsum[(size_t)j * nb + b], &v.y, 4);
-            }
-    }
-    return 0;
-}
-
 // q8 rows of a verify-width block from the device's activation order back to natural order
 static int read_back_q8(const int8_t *dq, int rows, int k, int8_t *xq, float *xd, int32_t *xsum) {
     const ActLayout lay = lg_act_layout(k);
@@ -2134,6 +2174,127 @@ static int read_back_q8(const int8_t *dq, int rows, int k, int8_t *xq, float *xd
             }
     }
     return 0;
+}
+
+// the same for a wide block: values from their two digits, sums from the values (the kernels need none)
+static int read_back_wide(const uint8_t *dq, int rows, int k, int8_t *xq, float *xd, int32_t *xsum) {
+    const int nb = k / 32;
+    std::vector<uint8_t> dev(lg_wide_q8_bytes(rows, k));
+    HIP_TRY(hipMemcpy(dev.data(), dq, dev.size(), hipMemcpyDeviceToHost));
+    static const int mag[9] = { 0, 12, 16, 18, 20, 21, 22, 23, 24 };          // 6-bit codes of 0..8
+    for (int j = 0; j < rows; ++j)
+        for (int b = 0; b < nb; ++b) {
+            const uint8_t *t = dev.data() + ((size_t)(j >> 6) * nb + b) * LG_QTILE;
+            int v[2][32], sum = 0;
+            for (int half = 0; half < 2; ++half) {
+                const int lane = half * 32 + (j & 31), base = ((j >> 5) & 1) * 1536;
+                uint8_t bytes[25] = { 0 };
+                memcpy(bytes, t + base + lane * 16, 16);
+                memcpy(bytes + 16, t + base + 1024 + lane * 8, 8);
+                for (int e = 0; e < 32; ++e) {
+                    const int code = ((bytes[6 * e / 8] | (bytes[6 * e / 8 + 1] << 8)) >> (6 * e % 8)) & 63;
+                    int x = 0;
+                    for (int i = 0; i < 9; ++i) if (mag[i] == (code & 31)) x = i;
+                    v[half][e] = (code & 32) ? -x : x;
+                }
+            }
+            for (int e = 0; e < 32; ++e) {
+                const int q = 16 * v[0][e] + v[1][e];
+                sum += q;
+                if (xq) xq[(size_t)j * k + b * 32 + e] = (int8_t)q;
+            }
+            if (xd) memcpy(&xd[(size_t)j * nb + b], t + 3072 + (j & 63) * 4, 4);
+            if (xsum) xsum[(size_t)j * nb + b] = sum;
+        }
+    return 0;
+}
+static int matmul_wide(hipStream_t st, const uint8_t *dw, uint8_t *dwide, int k, int mrows, int rows, const float *dx, float *dout, int32_t *ddots,
+                       int8_t *dq, int repeats, float *kernel_ms) {
+    const size_t np = (size_t)((mrows + LG_WT - 1) / LG_WT * LG_WT) * (k / 32);
+    hipLaunchKernelGGL(lg_k_wide_pack, dim3((unsigned)((np + LG_WG - 1) / LG_WG)), dim3(LG_WG), 0, st, dw, k, mrows, 0, dwide);
+    hipLaunchKernelGGL(lg_k_wide_quant, dim3((rows * (k / 32) * 8 + LG_WG - 1) / LG_WG), dim3(LG_WG), 0, st, dx, rows, k, (uint8_t *)dq);
+    lg_hip_model shim;
+    shim.stream = st;
+    Launcher lx{ &shim, false };
+    if (ddots) launch_wide_mm<true>(lx, 0, dwide, dq, k, mrows, rows, dout, ddots);
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    auto body = [&]() -> int {
+        HIP_TRY(hipEventCreate(&e0)); HIP_TRY(hipEventCreate(&e1));
+        launch_wide_mm<false>(lx, 0, dwide, dq, k, mrows, rows, dout, nullptr);
+        HIP_TRY(hipEventRecord(e0, st));
+        for (int r = 0; r < repeats; ++r) launch_wide_mm<false>(lx, 0, dwide, dq, k, mrows, rows, dout, nullptr);
+        if (lx.rc) return lx.rc;
+        HIP_TRY(hipEventRecord(e1, st));
+        HIP_TRY(hipStreamSynchronize(st));
+        HIP_TRY(hipGetLastError());
+        float t = 0;
+        if (repeats > 0) HIP_TRY(hipEventElapsedTime(&t, e0, e1));
+        if (kernel_ms) *kernel_ms = repeats > 0 ? t / repeats : 0.0f;
+        return 0;
+    };
+    const int rc = body();
+    if (e0) (void)hipEventDestroy(e0);
+    if (e1) (void)hipEventDestroy(e1);
+    return rc;
+}
+
+extern "C" int lg_hip_matmul_f32w(const float *w, int k, int mrows, const float *x, int rows, float *out) {
+    if (!w || !x || !out) return fail(-1, "matmul_f32w: null argument");
+    if (k < 256 || k % 256 || mrows < 1 || rows < 1) return fail(-2, "matmul_f32w: k %d (a multiple of 256), m %d, rows %d", k, mrows, rows);
+    if (lg_hip_device_count() < 1) return fail(-3, "matmul_f32w: no HIP device");
+    Scratch sc;
+    float *dw, *dx, *dout;
+    if (sc.get(&dw, (size_t)mrows * k) || sc.get(&dx, (size_t)rows * k) || sc.get(&dout, (size_t)rows * mrows)) return -7;
+    HIP_TRY(hipMemcpy(dw, w, (size_t)mrows * k * 4, hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(dx, x, (size_t)rows * k * 4, hipMemcpyHostToDevice));
+    MmfArgs a{ dw, k, mrows, dx, k, rows, dout, mrows, nullptr, 0 };
+    hipLaunchKernelGGL((lg_k_mmf<8>), dim3((mrows + LG_WG / 64 - 1) / (LG_WG / 64), (rows + 7) / 8), dim3(LG_WG), 0, nullptr, a);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipDeviceSynchronize());
+    HIP_TRY(hipMemcpy(out, dout, (size_t)rows * mrows * 4, hipMemcpyDeviceToHost));
+    return 0;
+}
+
+extern "C" int lg_hip_matmul_q4q8(const void *w, int k, int mrows, const float *x, int rows, float *out, int32_t *dots,
+                                  int8_t *xq, float *xd, int32_t *xsum, int repeats, float *kernel_ms) {
+    if (!w || !x) return fail(-1, "matmul: null input");
+    const bool wide = rows > LG_HIP_MAX_ROWS && rows % LG_WIDE == 0 && rows <= LG_WIDE_ROWS;     // row tiles through the kernels of prompt blocks
+    if (rows < 1 || (rows > LG_HIP_MAX_ROWS && !wide) || !lg_hip_repacked_bytes(k, mrows) || (!wide && lds_mm(rows, k) > 160 * 1024) || (rows > LG_HIP_MAX_ROWS && !wide))
+        return fail(-2, "matmul: rows %d (1..%d, or a multiple of %d), k %d (multiple of 256, rows*k*1.25 <= 160 KiB), m %d (multiple of 8)", rows, LG_HIP_MAX_ROWS, LG_WIDE, k, mrows);
+    if (lg_hip_device_count() < 1) return fail(-3, "matmul: no HIP device");
+    const int nb = k / 32;
+    std::vector<uint8_t> tiled(lg_hip_repacked_bytes(k, mrows));
+    int rc = lg_hip_repack_q4_0(w, k, mrows, tiled.data());
+    if (rc) return rc;
+    Scratch sc;
+    uint8_t *dw; float *dx, *dout; int32_t *ddots = nullptr; int8_t *dq;
+    if (sc.get(&dw, tiled.size()) || sc.get(&dx, (size_t)rows * k) || sc.get(&dout, (size_t)rows * mrows * 4) ||
+        sc.get(&dq, wide ? lg_wide_q8_bytes(rows, k) : (size_t)rows * k * 5 / 4)) return -7;
+    if (dots && sc.get(&ddots, (size_t)rows * mrows * nb)) return -7;
+    HIP_TRY(hipMemcpy(dw, tiled.data(), tiled.size(), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(dx, x, (size_t)rows * k * 4, hipMemcpyHostToDevice));
+    hipStream_t st;
+    HIP_TRY(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+    if (wide) {
+        uint8_t *dwide;
+        if (sc.get(&dwide, lg_wide_bytes(k, mrows))) rc = -7;
+        else rc = matmul_wide(st, dw, dwide, k, mrows, rows, dx, dout, ddots, dq, repeats, kernel_ms);
+    } else switch (rows) {
+#define CASE(M) case M: rc = matmul_rows<M>(st, dw, k, mrows, dx, dout, ddots, dq, repeats, kernel_ms); break;
+        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
+#undef CASE
+    }
+    (void)hipStreamDestroy(st);
+    if (rc) return rc;
+    if (out && wide && lg_segments(k) == 32) {             // four slabs of partial sums: the top of the segment tree is added here
+        std::vector<float> parts((size_t)4 * rows * mrows);
+        HIP_TRY(hipMemcpy(parts.data(), dout, parts.size() * 4, hipMemcpyDeviceToHost));
+        const size_t n = (size_t)rows * mrows;
+        for (size_t i = 0; i < n; ++i) out[i] = (parts[i] + parts[n + i]) + (parts[2 * n + i] + parts[3 * n + i]);
+    } else if (out) HIP_TRY(hipMemcpy(out, dout, (size_t)rows * mrows * 4, hipMemcpyDeviceToHost));
+    if (dots) HIP_TRY(hipMemcpy(dots, ddots, (size_t)rows * mrows * nb * 4, hipMemcpyDeviceToHost));
+    // the device keeps activation rows in the matmul's own order; hand them back in natural order
+    return wide ? read_back_wide((const uint8_t *)dq, rows, k, xq, xd, xsum) : read_back_q8(dq, rows, k, xq, xd, xsum);
 }
 
 template <int M>
@@ -2322,7 +2483,7 @@ extern "C" int lg_hip_attention(const float *q, const uint16_t *kc, const uint16
     int rc = 0;
     switch (rows) {
 #define CASE(M) case M: rc = attention_rows<M>(st, a, g, ctl, tiles, repeats, kernel_ms); break;
-        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(LG_WIDE)
+        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
 #undef CASE
     }
     (void)hipStreamDestroy(st);
@@ -2341,8 +2502,6 @@ extern "C" int lg_hip_attention(const float *q, const uint16_t *kc, const uint16
 static __device__ __align__(256) unsigned char lg_noalloc_scratch[LG_NOALLOC_BYTES];
 // the array's device address, asked once per device (each device holds its own copy at its own address)
 static unsigned char *g_noalloc_ptr[LG_NOALLOC_DEVICES];
-
-__global__ void lg_k_set_ctl(StepCtl *ctl, int pos) { ctl->pos = pos; ctl->step = 0; ctl->err = 0; ctl->pad = 0; }
 
 static size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
 

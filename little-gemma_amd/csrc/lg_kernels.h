@@ -75,23 +75,12 @@ template <int M>
 __device__ __forceinline__ const float2 *lg_q8_ds(const int8_t *q, int k) { return (const float2 *)(q + (size_t)M * k); }
 template <int M>
 __device__ __forceinline__ float2 *lg_q8_ds(int8_t *q, int k) { return (float2 *)(q + (size_t)M * k); }
-// Where row j keeps byte `byte` of its natural 16-byte unit w, and the {scale, sum} pair of block b.
-// Blocks of up to LG_HIP_MAX_ROWS_DEV rows: row-major rows in the order of lg_act_layout (what the
-// wavefront-dot kernels stage in LDS).  Wider blocks (the matrix-core kernels): tiles of 32 rows, and
-// inside a tile the 8-byte halves of a unit of all 32 rows side by side, so that the 64 lanes of an
-// operand load (row n = lane % 32, half = lane / 32) read 512 consecutive bytes.
+// Where row j keeps byte `byte` of its natural 16-byte unit w, and the {scale, sum} pair of block b: row-major rows in
+// the order of lg_act_layout (what the wavefront-dot kernels stage in LDS).
 template <int M>
-__device__ __forceinline__ size_t lg_q8_off(int k, int j, int w, int byte) {
-    const int u = lg_act_unit(lg_act_layout(k), w);
-    if (M <= LG_HIP_MAX_ROWS_DEV) return (size_t)j * k + (size_t)u * 16 + byte;
-    return (size_t)(j >> 5) * 32 * k + ((size_t)(u * 2 + (byte >> 3)) * 32 + (j & 31)) * 8 + (byte & 7);
-}
+__device__ __forceinline__ size_t lg_q8_off(int k, int j, int w, int byte) { return (size_t)j * k + (size_t)lg_act_unit(lg_act_layout(k), w) * 16 + byte; }
 template <int M>
-__device__ __forceinline__ size_t lg_q8_ds_idx(int k, int j, int b) {
-    const int u = lg_act_block(lg_act_layout(k), b);
-    if (M <= LG_HIP_MAX_ROWS_DEV) return (size_t)j * (k >> 5) + u;
-    return (size_t)(j >> 5) * 32 * (k >> 5) + (size_t)u * 32 + (j & 31);
-}
+__device__ __forceinline__ size_t lg_q8_ds_idx(int k, int j, int b) { return (size_t)j * (k >> 5) + lg_act_block(lg_act_layout(k), b); }
 #define LG_MU_DWORDS 80                     // dwords per block of the lg_k_geglu_m activation order
 #define LG_ROWV ((LG_MAXV + 3) / 4)        // float4 per thread of a residual row, 256 threads per row
 template <int M>
@@ -196,13 +185,13 @@ __global__ __launch_bounds__(LG_WG) void lg_k_rows(const StepCtl *ctl, LG_ROW_FI
         float d; int sum;
         const uint32_t packed = lg_quant4_8lanes(xv[v], &d, &sum);
         const int quad = t + 256 * v;                        // 4 values = a quarter of a 16-byte unit
-        if (M <= LG_HIP_MAX_ROWS_DEV && s.q_units == 1) {     // units of 32 dwords per (block, 3 rows): see lg_k_geglu_t
+        if (s.q_units == 1) {     // units of 32 dwords per (block, 3 rows): see lg_k_geglu_t
             uint32_t *unit = (uint32_t *)s.q + ((size_t)(quad >> 3) * ((M + 2) / 3) + j / 3) * 32;
             unit[(j % 3) * 8 + (quad & 7)] = packed;
             if ((t & 7) == 0) *(float2 *)(unit + 24 + 2 * (j % 3)) = make_float2(d, __int_as_float(sum));
             continue;
         }
-        if (M <= LG_HIP_MAX_ROWS_DEV && s.q_units == 2) {     // 80 dwords per block, 8 row slots: see lg_k_geglu_m
+        if (s.q_units == 2) {     // 80 dwords per block, 8 row slots: see lg_k_geglu_m
             uint32_t *blk = (uint32_t *)s.q + (size_t)(quad >> 3) * LG_MU_DWORDS;
             const int dw = quad & 7;
             blk[j * 8 + ((dw & 1) | ((dw & 2) << 1) | ((dw & 4) >> 1))] = packed;
@@ -225,11 +214,6 @@ __global__ __launch_bounds__(LG_WG) void lg_k_quant_flat(const float *x, int row
     const uint32_t packed = lg_quant4_8lanes(h, &d, &sum);
     if (!live) return;
     const int j = g / nb, b = g - j * nb;
-    if (rows > LG_HIP_MAX_ROWS_DEV) {                        // a wide block: the matrix-core kernels' layout
-        *(uint32_t *)(q + lg_q8_off<LG_HIP_MAX_ROWS_DEV + 1>(k, j, b * 2 + (l >> 2), (l & 3) * 4)) = packed;
-        if (l == 0) ds[lg_q8_ds_idx<LG_HIP_MAX_ROWS_DEV + 1>(k, j, b)] = make_float2(d, __int_as_float(sum));
-        return;
-    }
     const ActLayout lay = lg_act_layout(k);
     ((uint32_t *)(q + (size_t)j * k))[lg_act_unit(lay, b * 2 + (l >> 2)) * 4 + (l & 3)] = packed;
     if (l == 0) ds[(size_t)j * nb + lg_act_block(lay, b)] = make_float2(d, __int_as_float(sum));
@@ -445,7 +429,7 @@ __global__ __launch_bounds__(S == 32 ? 320 : LG_WG, 2) void lg_k_mm(LG_MM_FIELDS
 struct GegluArgs {
     const uint8_t *w;        // row-block tiles of [2*n_ff][k], virtual row order: 32 gate, 32 up, 32 gate, ...
     int            k, n_ff;
-    const int8_t  *q_in;     // verify blocks: unit order (below); wide blocks: lg_q8_off
+    const int8_t  *q_in;     // unit order (below)
     int8_t        *gq;       // q8 activation buffer of the result, width n_ff
     int            gq_units; // lg_k_geglu_m only: 2 = write the 80-dword blocks of the matrix-core kernels (what lg_k_down_m reads) instead of rows
 };
@@ -724,7 +708,7 @@ struct PleGateArgs {
     int            layer, n_layer;
     int8_t        *pq;       // q8 activation buffer of the result, width ple
 };
-// Verify blocks (wide blocks: lg_k_mm_plegate_wide): the row work that precedes the matmul is folded in,
+// The row work that precedes the matmul is folded in,
 // i.e. the residual update x += rmsnorm(dout) * w_post and the q8 of the new x (what lg_k_rows does
 // between two other matmuls).  One workgroup per (block of 32 gate rows, draft row): it updates and quantizes
 // its one row (lane assignment and summation order of lg_k_rows; the quantized row goes straight to LDS, the

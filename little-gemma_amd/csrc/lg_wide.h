@@ -1,0 +1,593 @@
+// lg_wide.h — the q4_0 x q8 matmuls of wide row blocks (prompts), on the matrix cores.
+//
+// Same arithmetic and the same float order as the wavefront-dot kernels of lg_kernels.h (so a prompt leaves
+// bit-identical cache rows): per 32-weight block an exact dot, p = fma(xd*dw, (float)dot, p) along each of the S
+// contiguous K segments, then the adjacent-pair tree over the segments.  What is left to the vector units is the one
+// fma per output and block that this order needs; everything else of a block runs on the matrix cores:
+//
+//  * the dot, as v_mfma_scale_f32_32x32x64_f8f6f4 on 6-bit floats (e3m2, which holds every integer -8..8 exactly).
+//    A weight is one such value (its nibble - 8).  A q8 value q is two, q = 16*hi + lo with hi = (q+8) >> 4 in -8..8
+//    and lo in -8..7: the instruction's K = 64 is the block's 32 weights twice against its 32 hi and its 32 lo digits,
+//    and the factor 16 is the E8M0 scale of the first half.  Products and sums are integers below 2^15, so the result
+//    is the exact dot, already a float.  On int8 (v_mfma_i32_32x32x32_i8, the same 32 cycles) every output needs a
+//    subtraction to become (float)(dot - 8*sum).
+//  * the products xd*dw, as the outer product v_mfma_f32_32x32x1_2b_f32 with a zero accumulator: fma(x, y, 0) is the
+//    correctly rounded product (subnormals included).  One instruction serves the two 32-row halves of a weight tile,
+//    and a lane loads one scale per block where the vector form loads the 16 scales of its outputs through LDS.
+//
+// Measured issue bound per 32x32x32 block and SIMD: 60 cycles of vector work, 66 of matrix work, two wavefronts
+// overlapping them (int8 with sub, mul and fma: 163 cycles).
+//
+// A workgroup is 4 wavefronts and owns 64 weight rows x 32*TB activation rows; wavefront w runs the K segments 2w and
+// 2w+1, so the wavefronts share no operands, the main loop has no barrier and the operands come straight from L2; LDS
+// only carries the partial sums (the first segment's while the second runs, and the tree over the wavefronts).
+#pragma once
+#include "lg_kernels.h"
+
+typedef int lg_v8i __attribute__((ext_vector_type(8)));
+typedef float lg_v16f __attribute__((ext_vector_type(16)));
+typedef float lg_v32f __attribute__((ext_vector_type(32)));
+
+#define LG_WT      64                      // weight rows of a tile
+#define LG_WTILE   1664                    // bytes of (64 weight rows, one block): [64][16] + [64][8] bytes of 6-bit values, [64] f16 scales
+#define LG_QTILE   3328                    // bytes of (64 activation rows, one block): 2 x ([64][16] + [64][8]) bytes of digits, [64] f32 scales
+#define LG_WIDE      32                    // activation rows of one matrix-core operand
+#define LG_WIDE_ROWS 512                   // rows of the widest block
+#define LG_WIDE_MID  128                   // the widest block of a short cache
+
+// 6-bit float code (sign, 3 exponent bits of bias 3, 2 mantissa bits) of an integer -8..8 given as a float
+__device__ __forceinline__ uint32_t lg_e3m2(float v) {
+    const uint32_t u = __float_as_uint(v);
+    const int e = (int)((u & 0x7FFFFFFFu) >> 21) - (124 << 2);
+    return (uint32_t)(e > 0 ? e : 0) | ((u >> 26) & 0x20u);
+}
+// Where the digits of (row j, block b) of a wide activation buffer of nb blocks per row live: dword d (0..5) of the hi
+// (half = 0) or lo (half = 1) digits, and the row's scale.
+__device__ __forceinline__ size_t lg_qtile(int nb, int j, int b) { return ((size_t)(j >> 6) * nb + b) * LG_QTILE; }
+__device__ __forceinline__ int lg_qdigit(int j, int half, int d) {
+    const int lane = half * 32 + (j & 31), t = ((j >> 5) & 1) * 1536;
+    return d < 4 ? t + lane * 16 + d * 4 : t + 1024 + lane * 8 + (d - 4) * 4;
+}
+__device__ __forceinline__ int lg_qscale(int j) { return 3072 + (j & 63) * 4; }
+// bytes of a wide activation buffer
+__host__ __device__ static inline size_t lg_wide_q8_bytes(int rows, int k) { return (size_t)((rows + 63) / 64) * (size_t)(k >> 5) * LG_QTILE; }
+
+// q8 of 32 values held as one float4 in each of 8 adjacent lanes (lane % 8 = i holds elements 4i..4i+3 of block b of row
+// j), written as digits: the arithmetic of lg_quant4_8lanes.
+__device__ __forceinline__ void lg_wide_quant4(float4 h, uint8_t *q, int nb, int j, int b) {
+    float amax = fmaxf(fmaxf(fabsf(h.x), fabsf(h.y)), fmaxf(fabsf(h.z), fabsf(h.w)));
+    amax = lg_max_n(amax, 8);
+    const float d = lg_div127(amax);
+    const float id = d > 0.0f ? 1.0f / d : 0.0f;
+    const float v[4] = { lg_rintf(h.x * id), lg_rintf(h.y * id), lg_rintf(h.z * id), lg_rintf(h.w * id) };
+    uint32_t hi = 0, lo = 0;
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float fh = floorf((v[i] + 8.0f) * 0.0625f), fl = lg_fmaf(-16.0f, fh, v[i]);
+        hi |= lg_e3m2(fh) << (6 * i);
+        lo |= lg_e3m2(fl) << (6 * i);
+    }
+    // 24 bits per lane, four lanes make three dwords: lane k (k = 0..2 of the four) completes its bits with its neighbour's
+    const int i = (int)threadIdx.x & 7, k = i & 3, dw = 3 * (i >> 2) + k;
+    const uint32_t nh = (uint32_t)lg_dpp_i<0xF9>((int)hi), nl = (uint32_t)lg_dpp_i<0xF9>((int)lo);   // quad_perm [1,2,3,3]
+    uint8_t *t = q + lg_qtile(nb, j, b);
+    if (k < 3) {
+        *(uint32_t *)(t + lg_qdigit(j, 0, dw)) = (hi >> (8 * k)) | (nh << (24 - 8 * k));
+        *(uint32_t *)(t + lg_qdigit(j, 1, dw)) = (lo >> (8 * k)) | (nl << (24 - 8 * k));
+    }
+    if (i == 0) *(float *)(t + lg_qscale(j)) = d;
+}
+
+// Wide form of a tiled matrix (segment tiles, or row-block tiles when RB), built on the device when a model is
+// committed: one thread per (row, block).  Rows past m (a row count that is no multiple of 64) are zero.
+__global__ __launch_bounds__(LG_WG) void lg_k_wide_pack(const uint8_t *w, int k, int m, int rb, uint8_t *dst) {
+    const int nb = k >> 5, mp = (m + LG_WT - 1) / LG_WT * LG_WT;
+    const size_t id = (size_t)blockIdx.x * LG_WG + threadIdx.x;
+    if (id >= (size_t)mp * nb) return;
+    const int row = (int)(id % (size_t)mp), b = (int)(id / (size_t)mp);
+    uint32_t out[6] = { 0, 0, 0, 0, 0, 0 };
+    uint16_t sc = 0;
+    if (row < m) {
+        const uint8_t *tile; int slot;
+        if (rb) { tile = w + ((size_t)(row >> 6) * nb + b) * LG_TILE; slot = row & 63; }
+        else {
+            const int S = lg_segments(k), nit = nb / S, rw = 64 / S, c = b / nit;
+            tile = w + ((size_t)(row / rw) * nit + (b - c * nit)) * LG_TILE; slot = (row % rw) * S + c;
+        }
+        const uint8_t *qs = tile + slot * 16;
+        sc = *(const uint16_t *)(tile + 1024 + slot * 2);
+        #pragma unroll
+        for (int e = 0; e < 32; ++e) {
+            const int nib = e < 16 ? (qs[e] & 15) : (qs[e - 16] >> 4);
+            const uint64_t c = (uint64_t)lg_e3m2((float)(nib - 8)) << ((6 * e) & 31);
+            out[(6 * e) >> 5] |= (uint32_t)c;
+            if (((6 * e) & 31) > 26) out[((6 * e) >> 5) + 1] |= (uint32_t)(c >> 32);
+        }
+    }
+    uint8_t *t = dst + ((size_t)(row >> 6) * nb + b) * LG_WTILE;
+    const int n = row & 63;
+    *(uint4 *)(t + n * 16) = make_uint4(out[0], out[1], out[2], out[3]);
+    *(uint2 *)(t + 1024 + n * 8) = make_uint2(out[4], out[5]);
+    *(uint16_t *)(t + 1536 + n * 2) = sc;
+}
+static inline size_t lg_wide_bytes(int k, int m) { return (size_t)((m + LG_WT - 1) / LG_WT) * (size_t)(k >> 5) * LG_WTILE; }
+
+struct WideMm {
+    const uint8_t *w;        // wide form of the weights
+    const uint8_t *q;        // wide activation buffer
+    int k, m, rows;          // row length, weight rows, activation rows of the block
+    int nb_tiles;            // activation tiles of 32*TB rows
+    int parts;               // 1: 8 K segments; 4: 32 segments, cut by quarter
+};
+// Workgroup -> (weight tile, activation tile, K quarter).  Consecutive workgroups are dealt to the 8 XCDs in turn; an
+// XCD walks the activation tiles of one weight tile before the next, so a weight tile is fetched from HBM by one XCD
+// once and the activations (2 MB of digits per 512 rows and 2560 inputs) stay in its 4 MB L2; with four K quarters an
+// XCD keeps to one quarter's activations.
+__device__ __forceinline__ bool lg_wide_map(const WideMm &a, int id, int &at, int &bt, int &part) {
+    const int x = id & 7, s = id >> 3, per = 8 / a.parts, an = s / a.nb_tiles;
+    bt = s - an * a.nb_tiles;
+    part = x % a.parts;
+    at = x / a.parts + per * an;
+    return at * LG_WT < a.m;
+}
+static inline int lg_wide_grid(int m, int nb_tiles, int parts) {
+    const int nt = (m + LG_WT - 1) / LG_WT, per = 8 / parts;
+    return 8 * ((nt + per - 1) / per) * nb_tiles;
+}
+
+// The tile's sums.  WV wavefronts: wavefront w runs the 8/WV segments from 8*part + w*8/WV of the K range and leaves their
+// sum in lds[w][(ta*TB + tb)*4 + g][lane] as float4 (weight rows 32*ta + 8*g + 4*h + 0..3 of the tile, activation row
+// 32*tb + n, lane = 32*h + n).  Synchronised on return.
+template <int TB, int WV, bool DUMP>
+__device__ __forceinline__ void lg_wide_tile(const WideMm &a, int at, int bt, int part, float4 *lds, int32_t *dots) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31;
+    const int nb = a.k >> 5, nit = nb / (8 * a.parts);
+    const int kb0 = (8 * part + 8 / WV * __builtin_amdgcn_readfirstlane(wave)) * nit;
+    const __amdgpu_buffer_rsrc_t rw = lg_buffer_rsrc(a.w + ((size_t)at * nb + kb0) * LG_WTILE);
+    const int sub = TB == 1 ? (bt & 1) : 0;
+    const __amdgpu_buffer_rsrc_t rq = lg_buffer_rsrc(a.q + ((size_t)(TB == 1 ? bt >> 1 : bt) * nb + kb0) * LG_QTILE);
+    const int vq16 = sub * 1536 + lane * 16, vq8 = sub * 1536 + 1024 + lane * 8, vxs = 3072 + (TB == 1 ? sub * 32 + n : lane) * 4;
+    // The operands of a block, as loaded (a lane holds weight row `lane` of the tile and its digits of each activation tile).
+    struct Ops { lg_v8i b[TB]; uint32_t a[6]; float xs; uint32_t ws; };
+    auto fetch = [&](Ops &o, int kb_) {
+        const int kb = __builtin_amdgcn_readfirstlane(kb_), wo = kb * LG_WTILE, qo = kb * LG_QTILE;
+        const auto a16 = __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16, wo, 0);
+        const auto a8 = __builtin_amdgcn_raw_buffer_load_b64(rw, 1024 + lane * 8, wo, 0);
+        o.a[0] = a16[0]; o.a[1] = a16[1]; o.a[2] = a16[2]; o.a[3] = a16[3]; o.a[4] = a8[0]; o.a[5] = a8[1];
+        o.ws = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rw, 1536 + lane * 2, wo, 0);
+        #pragma unroll
+        for (int t = 0; t < TB; ++t) {
+            const auto b16 = __builtin_amdgcn_raw_buffer_load_b128(rq, vq16 + t * 1536, qo, 0);
+            const auto b8 = __builtin_amdgcn_raw_buffer_load_b64(rq, vq8 + t * 1536, qo, 0);
+            o.b[t] = (lg_v8i){ (int)b16[0], (int)b16[1], (int)b16[2], (int)b16[3], (int)b8[0], (int)b8[1], 0, 0 };
+        }
+        o.xs = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rq, vxs, qo, 0));
+    };
+    const int sb = lane < 32 ? 131 : 127;                     // E8M0 scales of the K halves: 2^4 for the hi digits, 1 for the lo digits
+    const lg_v16f z16 = {};
+    const lg_v32f z32 = {};
+    float p[2][TB][16];
+    auto clear = [&]() {
+        #pragma unroll
+        for (int t = 0; t < 2 * TB; ++t)
+            #pragma unroll
+            for (int i = 0; i < 16; ++i) p[t & 1][t >> 1][i] = 0.0f;
+    };
+    float4 *mine = lds + (size_t)wave * (2 * TB * 4 * 64);
+    auto segment_end = [&]() {                                // the first segment's sums wait in LDS
+        #pragma unroll
+        for (int t = 0; t < 2 * TB; ++t)
+            #pragma unroll
+            for (int g = 0; g < 4; ++g)
+                mine[(t * 4 + g) * 64 + lane] = make_float4(p[t / TB][t % TB][4 * g], p[t / TB][t % TB][4 * g + 1], p[t / TB][t % TB][4 * g + 2], p[t / TB][t % TB][4 * g + 3]);
+        clear();
+    };
+    // A step is (block, activation tile): its scale products S, its two dots D0 and D1, and the 32 fma that use them.
+    // The matrix instructions of step q+1 are issued between the fma of step q (S ahead of the first 16, D0 ahead of
+    // the second, D1 behind them: each into registers that have just been read), so that neither pipe waits for the
+    // other; left to the compiler a wavefront issues one matrix instruction, waits it out and then does its fma
+    // (gate/up of 512 rows at the E4B shape: 91 us that way).
+    constexpr int NS = TB == 1 ? 4 : 2;                       // blocks in flight (even: a step's S alternates)
+    Ops o[NS];
+    lg_v32f S[2];
+    lg_v16f D0, D1;
+    lg_v8i a0, a1;
+    float dw, xd[2];
+    const int nblk = 8 / WV * nit, last = nblk - 1;
+    auto take = [&](const Ops &q) {                           // a block's weight operands: each 32-row half in both K halves
+        #pragma unroll
+        for (int i = 0; i < 6; ++i) { const lg_u2 r = lg_pair32(q.a[i]); a0[i] = (int)r.x; a1[i] = (int)r.y; }
+        a0[6] = a0[7] = a1[6] = a1[7] = 0;
+        dw = lg_h2f((uint16_t)q.ws);
+        if (TB == 1) xd[0] = q.xs;
+        else { const lg_u2 r = lg_pair32(__float_as_uint(q.xs)); xd[0] = __uint_as_float(r.x); xd[1] = __uint_as_float(r.y); }
+    };
+    #pragma unroll
+    for (int i = 0; i < NS; ++i) fetch(o[i], i < last ? i : last);
+    clear();
+    take(o[0]);
+    S[0] = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, xd[0], z32, 0, 0, 0);
+    D0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a0, o[0].b[0], z16, 3, 3, 0, 127, 0, sb);
+    D1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a1, o[0].b[0], z16, 3, 3, 0, 127, 0, sb);
+    for (int it = 0; it < nblk; it += NS) {
+        #pragma unroll
+        for (int u = 0; u < NS; ++u) {
+            if ((NS > 2 || WV == 8) && it + u >= nblk) break;   // (two segments: an even count)
+            if (WV == 4 && it + u == nit) segment_end();
+            #pragma unroll
+            for (int t = 0; t < TB; ++t) {
+                const int cur = TB == 2 ? t : (u & 1), nxt = cur ^ 1;
+                const Ops &on = t + 1 < TB ? o[u] : o[(u + 1) % NS];
+                const int tn = t + 1 < TB ? t + 1 : 0;
+                if (tn == 0) take(on);
+                S[nxt] = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, xd[tn], z32, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (DUMP) {
+                    const int an = (bt * TB + t) * 32 + n;
+                    if (an < a.rows)
+                        for (int i = 0; i < 16; ++i) {
+                            const int row = at * LG_WT + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+                            if (row < a.m) dots[((size_t)an * a.m + row) * nb + kb0 + it + u] = (int)D0[i];
+                            if (row + 32 < a.m) dots[((size_t)an * a.m + row + 32) * nb + kb0 + it + u] = (int)D1[i];
+                        }
+                }
+                #pragma unroll
+                for (int i = 0; i < 16; ++i) p[0][t][i] = lg_fmaf(S[cur][i], D0[i], p[0][t][i]);
+                __builtin_amdgcn_sched_barrier(0);
+                D0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a0, on.b[tn], z16, 3, 3, 0, 127, 0, sb);
+                __builtin_amdgcn_sched_barrier(0);
+                #pragma unroll
+                for (int i = 0; i < 16; ++i) p[1][t][i] = lg_fmaf(S[cur][16 + i], D1[i], p[1][t][i]);
+                __builtin_amdgcn_sched_barrier(0);
+                D1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a1, on.b[tn], z16, 3, 3, 0, 127, 0, sb);
+                if (t == (TB == 2 ? 0 : TB - 1)) { const int nx = it + u + NS; fetch(o[u], nx < last ? nx : last); }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+    #pragma unroll
+    for (int t = 0; t < 2 * TB; ++t)
+        #pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            float4 *s = &mine[(t * 4 + g) * 64 + lane];
+            const float4 v = WV == 4 ? *s : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            *s = make_float4(v.x + p[t / TB][t % TB][4 * g], v.y + p[t / TB][t % TB][4 * g + 1], v.z + p[t / TB][t % TB][4 * g + 2], v.w + p[t / TB][t % TB][4 * g + 3]);
+        }
+    __syncthreads();
+}
+// finished sums of float4 `u` (= (ta*TB + tb)*4 + g) of this lane: the tree over the wavefronts
+template <int TB, int WV>
+__device__ __forceinline__ float4 lg_wide_sum(const float4 *lds, int u) {
+    const int lane = threadIdx.x & 63, st = 2 * TB * 4 * 64;
+    auto quad = [&](int w) {
+        const float4 *l = lds + (size_t)w * st + u * 64 + lane;
+        const float4 a = l[0], b = l[st], c = l[2 * st], d = l[3 * st];
+        return make_float4((a.x + b.x) + (c.x + d.x), (a.y + b.y) + (c.y + d.y), (a.z + b.z) + (c.z + d.z), (a.w + b.w) + (c.w + d.w));
+    };
+    const float4 r = quad(0);
+    if (WV == 4) return r;
+    const float4 s = quad(4);
+    return make_float4(r.x + s.x, r.y + s.y, r.z + s.z, r.w + s.w);
+}
+
+// Plain matmul: out[part][row][m] f32 (four slabs when the K range is cut by quarter: the consumer adds them as
+// (p0 + p1) + (p2 + p3), the top of the segment tree).
+template <int TB, int WV, bool DUMP>
+__global__ __launch_bounds__(64 * WV, 2) void lg_k_wide_mm(WideMm a, float *out, int32_t *dots) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    float4 *lds = (float4 *)smem;
+    int at, bt, part;
+    if (!lg_wide_map(a, (int)blockIdx.x, at, bt, part)) return;
+    lg_wide_tile<TB, WV, DUMP>(a, at, bt, part, lds, dots);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
+    #pragma unroll
+    for (int v = 0; v < 8 * TB / WV; ++v) {
+        const int u = wave * (8 * TB / WV) + v, t = u >> 2, ta = t / TB, tb = t % TB, g = u & 3;
+        const float4 r = lg_wide_sum<TB, WV>(lds, u);
+        const int an = (bt * TB + tb) * 32 + n, col = at * LG_WT + 32 * ta + 8 * g + 4 * h;
+        if (an < a.rows && col < a.m) *(float4 *)(out + ((size_t)part * a.rows + an) * a.m + col) = r;
+    }
+}
+
+// Gate/up with the GeGLU and the q8 of its result: a weight tile is the 32 gate rows and the 32 up rows of 32 FFN columns.
+template <int TB, int WV>
+__global__ __launch_bounds__(64 * WV, 2) void lg_k_wide_geglu(WideMm a, uint8_t *gq) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ __align__(16) float vbuf[32 * TB * 36];
+    float4 *lds = (float4 *)smem;
+    int at, bt, part;
+    if (!lg_wide_map(a, (int)blockIdx.x, at, bt, part)) return;
+    lg_wide_tile<TB, WV, false>(a, at, bt, part, lds, nullptr);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
+    for (int u = wave; u < 4 * TB; u += WV) {
+        const int tb = u >> 2, g = u & 3;
+        const float4 gv = lg_wide_sum<TB, WV>(lds, tb * 4 + g), uv = lg_wide_sum<TB, WV>(lds, (TB + tb) * 4 + g);
+        *(float4 *)(vbuf + (32 * tb + n) * 36 + 8 * g + 4 * h) =
+            make_float4(lg_gelu(gv.x) * uv.x, lg_gelu(gv.y) * uv.y, lg_gelu(gv.z) * uv.z, lg_gelu(gv.w) * uv.w);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 32 * TB * 8; i += 64 * WV) {
+        const int row = i >> 3;
+        lg_wide_quant4(*(const float4 *)(vbuf + row * 36 + (i & 7) * 4), gq, a.m >> 6, bt * 32 * TB + row, at);
+    }
+}
+
+// Per-layer gate: gelu(inp_gate . x) * ipl of this layer, and the q8 of it.
+template <int TB, int WV>
+__global__ __launch_bounds__(64 * WV, 2) void lg_k_wide_plegate(WideMm a, const float *ipl, int layer, int n_layer, uint8_t *pq) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ __align__(16) float vbuf[2 * 32 * TB * 36];
+    float4 *lds = (float4 *)smem;
+    int at, bt, part;
+    if (!lg_wide_map(a, (int)blockIdx.x, at, bt, part)) return;
+    lg_wide_tile<TB, WV, false>(a, at, bt, part, lds, nullptr);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
+    for (int u = wave; u < 8 * TB; u += WV) {
+        const int t = u >> 2, g = u & 3, ta = t / TB, tb = t % TB, an = (bt * TB + tb) * 32 + n;
+        const float4 v = lg_wide_sum<TB, WV>(lds, u);
+        const int col = at * LG_WT + 32 * ta + 8 * g + 4 * h;
+        const float4 p = *(const float4 *)(ipl + ((size_t)(an < a.rows ? an : a.rows - 1) * n_layer + layer) * a.m + col);
+        *(float4 *)(vbuf + (ta * 32 * TB + 32 * tb + n) * 36 + 8 * g + 4 * h) =
+            make_float4(lg_gelu(v.x) * p.x, lg_gelu(v.y) * p.y, lg_gelu(v.z) * p.z, lg_gelu(v.w) * p.w);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 2 * 32 * TB * 8; i += 64 * WV) {
+        const int row = i >> 3, ta = row / (32 * TB);
+        lg_wide_quant4(*(const float4 *)(vbuf + row * 36 + (i & 7) * 4), pq, a.m >> 5, bt * 32 * TB + row - ta * 32 * TB, at * 2 + ta);
+    }
+}
+
+// Row kernel of a wide block (lg_k_rows of verify blocks, one workgroup per row, the result as wide digits): residual
+// update, norm, q8.  dparts = 4: dout is four [rows][E] slabs.
+__global__ __launch_bounds__(LG_WG) void lg_k_wide_rows(RowArgs s, int rows) {
+    __shared__ float red[2][4];
+    const int t = threadIdx.x, j = blockIdx.x, E = s.E, nq = E >> 2;
+    float4 xv[LG_ROWV], dv[LG_ROWV], wpost[LG_ROWV], wpre[LG_ROWV];
+    if (!s.x) {
+        const int tok = s.toks[j];
+        #pragma unroll
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) {
+            const float4 e = lg_tiled_deq4(s.emb, s.emb_nit, s.emb_seg, tok, 4 * (t + 256 * v));
+            xv[v] = make_float4(e.x * s.emb_scale, e.y * s.emb_scale, e.z * s.emb_scale, e.w * s.emb_scale);
+        }
+    } else {
+        const float4 *xr = (const float4 *)(s.x + (size_t)j * E);
+        #pragma unroll
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) xv[v] = xr[t + 256 * v];
+    }
+    const bool has_os = s.dout != nullptr && s.os != nullptr;
+    const float osv = has_os ? s.os[0] : 1.0f;
+    if (s.dout) {
+        const float4 *dr = (const float4 *)(s.dout + (size_t)j * E), *wr = (const float4 *)s.w_post;
+        #pragma unroll
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) { dv[v] = dr[t + 256 * v]; wpost[v] = wr[t + 256 * v]; }
+        if (s.dparts == 4) {
+            const size_t slab = (size_t)rows * nq;
+            #pragma unroll
+            for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) {
+                const float4 p1 = dr[slab + t + 256 * v], p2 = dr[2 * slab + t + 256 * v], p3 = dr[3 * slab + t + 256 * v], p0 = dv[v];
+                dv[v] = make_float4((p0.x + p1.x) + (p2.x + p3.x), (p0.y + p1.y) + (p2.y + p3.y), (p0.z + p1.z) + (p2.z + p3.z), (p0.w + p1.w) + (p2.w + p3.w));
+            }
+        }
+    }
+    if (s.w_pre) {
+        const float4 *wr = (const float4 *)s.w_pre;
+        #pragma unroll
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) wpre[v] = wr[t + 256 * v];
+    }
+    if (s.dout) {
+        float ss = 0.0f;
+        #pragma unroll
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) ss = lg_sumsq4(dv[v], ss);
+        ss = lg_block_sum256(ss, red[0]);
+        const float sc = 1.0f / sqrtf(ss / (float)E + s.eps);
+        #pragma unroll
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) {
+            const float4 w = wpost[v];
+            float4 r;
+            r.x = xv[v].x + dv[v].x * sc * w.x;  r.y = xv[v].y + dv[v].y * sc * w.y;
+            r.z = xv[v].z + dv[v].z * sc * w.z;  r.w = xv[v].w + dv[v].w * sc * w.w;
+            if (has_os) { r.x = r.x * osv; r.y = r.y * osv; r.z = r.z * osv; r.w = r.w * osv; }
+            xv[v] = r;
+        }
+    }
+    if (s.x_out) {
+        float4 *xo = (float4 *)(s.x_out + (size_t)j * E);
+        #pragma unroll
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) xo[t + 256 * v] = xv[v];
+    }
+    if (s.w_pre) {
+        float ss = 0.0f;
+        #pragma unroll
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) ss = lg_sumsq4(xv[v], ss);
+        ss = lg_block_sum256(ss, red[1]);
+        const float sc = 1.0f / sqrtf(ss / (float)E + s.eps);
+        #pragma unroll
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) {
+            const float4 w = wpre[v];
+            xv[v] = make_float4(xv[v].x * sc * w.x, xv[v].y * sc * w.y, xv[v].z * sc * w.z, xv[v].w * sc * w.w);
+        }
+    }
+    if (!s.q) return;
+    #pragma unroll
+    for (int v = 0; v < LG_ROWV; ++v) {
+        if (t + 256 * v >= nq) break;                        // nq is a multiple of 64: whole wavefronts
+        lg_wide_quant4(xv[v], (uint8_t *)s.q, E >> 5, j, (t + 256 * v) >> 3);
+    }
+}
+
+// Plain q8 of rows x k floats as wide digits (isolated matmul).
+__global__ __launch_bounds__(LG_WG) void lg_k_wide_quant(const float *x, int rows, int k, uint8_t *q) {
+    const int g = (blockIdx.x * LG_WG + threadIdx.x) >> 3, l = threadIdx.x & 7, nb = k >> 5;
+    if (g >= rows * nb) return;                              // (groups of 8 lanes leave together)
+    lg_wide_quant4(((const float4 *)x)[(size_t)g * 8 + l], q, nb, g / nb, g - g / nb * nb);
+}
+
+// ---------------------------------------------------------------------------------------------------------
+// Attention of a wide block.  A workgroup is 4 wavefronts on 16 units = (rows, query heads) of one kv head.  Both products
+// run on v_mfma_f32_16x16x1_4b_f32, whose every step is one fma per output (K = 1), so the defined chains are exactly its
+// accumulation order:
+//  * scores: the instruction's four blocks are the four chains c of a score (dims 4g + c, g ascending), a step per g; a
+//    lane ends up with all four chains of its outputs and adds (a0+a1)+(a2+a3).  The wavefronts take key tiles in turn.
+//    Queries stay in registers; K rows come straight from the cache, 64 bytes of a row by four lanes, and are dealt to the
+//    chains by a 4 x 4 exchange over the four 16-lane rows.
+//  * values: the four blocks are 16 dims each, a step per key slot (masked slots have weight 0); a wavefront takes 64 dims
+//    and walks the tiles in order, adding each tile's result to the running sum with the weight exp(m_tile - M).
+// The weights e of a row's tiles, their maxima and sums wait in LDS between the two (EL: up to LG_WA_TILES tiles; more: in
+// the cache's scratch).  On vector units the same block took a kernel per phase, and the tiles' results (1 KiB per tile
+// and head) went through memory: 56 + 15 us per layer and 512 rows at the E4B shape.
+#define LG_WA_TILES 36
+struct WideAttn {
+    const float *q;              // [rows][H*hd] normed + rotated
+    const uint16_t *kc, *vc;     // cache of the layer this one reads
+    int H, nkv, seq, kv_dim, window, rows;
+    float *scratch;              // !EL: per group tiles * 16 * 34 floats
+    int tiles;                   // tiles a group can touch
+    uint8_t *xq;                 // wide digits of the result, width H*hd
+};
+static inline int lg_wide_attn_rows(int G) { return 16 / G; }
+__device__ __forceinline__ float lg_max16(float v) {
+    v = lg_max8(v);
+    return fmaxf(v, lg_dpp_f<LG_DPP_MIRROR16>(v));
+}
+template <int HD, bool EL>
+__global__ __launch_bounds__(LG_WG, HD > 256 ? 1 : 2) void lg_k_wide_attn(WideAttn a, const StepCtl *ctl) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int NS = HD / 32;                               // 64-byte pieces of a K row
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), n = lane & 15, c = lane >> 4;
+    const int G = a.H / a.nkv, RG = 16 / G, U = RG * G, kvh = blockIdx.y, row0 = blockIdx.x * RG;
+    const int pos = ctl->pos;
+    int rlast = row0 + RG - 1;
+    if (rlast >= a.rows) rlast = a.rows - 1;
+    const int tfirst = lg_win_start(pos + row0, a.window) >> 5, tlast = (pos + rlast) >> 5, nt = tlast - tfirst + 1;
+    // e: [tile][16 units][36] (a 16-byte multiple off the 128-byte bank period), m and l: [tile][16]
+    constexpr int ES = EL ? 36 : 32;
+    float *eb = EL ? (float *)smem : a.scratch + ((size_t)blockIdx.x * a.nkv + kvh) * a.tiles * (16 * 34);
+    float *mb = eb + (size_t)(EL ? nt : a.tiles) * 16 * ES, *lb = mb + (size_t)(EL ? nt : a.tiles) * 16;
+    __shared__ float mx[16][17];
+    __shared__ __align__(16) float ob[16][HD + 4];
+    {
+        // this lane's query elements: unit n, chain c
+        const int ur = n / G, uh = n - ur * G;
+        int qr = row0 + ur;
+        if (n >= U || qr > rlast) qr = rlast;
+        const float *qp = a.q + (size_t)qr * a.H * HD + (size_t)(kvh * G + (n < U ? uh : 0)) * HD + c;
+        float qv[HD / 4];
+        #pragma unroll
+        for (int g = 0; g < HD / 4; ++g) qv[g] = qp[4 * g];
+        // validity of this lane's outputs: units 4c + i
+        int us[4], up[4];
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int u = 4 * c + i, r = row0 + u / G;
+            const bool on = u < U && r <= rlast;
+            up[i] = on ? pos + r : -1;
+            us[i] = on ? lg_win_start(pos + r, a.window) : 0;
+        }
+        for (int t = tfirst + wave; t <= tlast; t += 4) {
+            const int t0 = t << 5, ring0 = t0 % a.seq;
+            int r0 = ring0 + n, r1 = ring0 + 16 + n;          // ring rows of this lane's two keys
+            if (r0 >= a.seq) r0 -= a.seq;
+            if (r1 >= a.seq) r1 -= a.seq;
+            if (a.seq < 32) { r0 %= a.seq; r1 %= a.seq; }
+            const uint16_t *k0 = a.kc + (size_t)r0 * a.kv_dim + (size_t)kvh * HD + c * 8, *k1 = a.kc + (size_t)r1 * a.kv_dim + (size_t)kvh * HD + c * 8;
+            uint4 w0[NS], w1[NS];
+            #pragma unroll
+            for (int s = 0; s < NS; ++s) { w0[s] = *(const uint4 *)(k0 + s * 32); w1[s] = *(const uint4 *)(k1 + s * 32); }
+            lg_v16f d0 = {}, d1 = {};
+            #pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                // dims 32s + 8c + 0..7 of a key -> the same key's dims 32s + 4g + c, g = 0..7, as f16 pairs in g order
+                auto deal = [](uint4 w, uint32_t (&o)[4]) {
+                    uint32_t a0 = __builtin_amdgcn_perm(w.z, w.x, 0x05040100u), a1 = __builtin_amdgcn_perm(w.z, w.x, 0x07060302u);
+                    uint32_t a2 = __builtin_amdgcn_perm(w.w, w.y, 0x05040100u), a3 = __builtin_amdgcn_perm(w.w, w.y, 0x07060302u);
+                    const lg_u2 p = __builtin_amdgcn_permlane32_swap(a0, a2, false, false), q = __builtin_amdgcn_permlane32_swap(a1, a3, false, false);
+                    const lg_u2 x = __builtin_amdgcn_permlane16_swap(p.x, q.x, false, false), y = __builtin_amdgcn_permlane16_swap(p.y, q.y, false, false);
+                    o[0] = x.x; o[1] = x.y; o[2] = y.x; o[3] = y.y;
+                };
+                uint32_t o0[4], o1[4];
+                deal(w0[s], o0); deal(w1[s], o1);
+                #pragma unroll
+                for (int g = 0; g < 8; ++g) {
+                    const float b0 = lg_h2f((uint16_t)(o0[g >> 1] >> (16 * (g & 1)))), b1 = lg_h2f((uint16_t)(o1[g >> 1] >> (16 * (g & 1))));
+                    d0 = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[8 * s + g], b0, d0, 0, 0, 0);
+                    d1 = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[8 * s + g], b1, d1, 0, 0, 0);
+                }
+            }
+            float *et = eb + (size_t)(t - tfirst) * 16 * ES, *mt = mb + (t - tfirst) * 16, *lt = lb + (t - tfirst) * 16;
+            const int p0 = t0 + n, p1 = p0 + 16;
+            #pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bool v0 = p0 >= us[i] && p0 <= up[i], v1 = p1 >= us[i] && p1 <= up[i];
+                const float s0 = (d0[i] + d0[4 + i]) + (d0[8 + i] + d0[12 + i]), s1 = (d1[i] + d1[4 + i]) + (d1[8 + i] + d1[12 + i]);
+                const float m = lg_max16(fmaxf(v0 ? s0 : -INFINITY, v1 ? s1 : -INFINITY));
+                const float e0 = v0 ? lg_expf(s0 - m) : 0.0f, e1 = v1 ? lg_expf(s1 - m) : 0.0f;
+                const float l = lg_sum16(e0) + lg_sum16(e1);
+                et[(4 * c + i) * ES + n] = e0;
+                et[(4 * c + i) * ES + 16 + n] = e1;
+                if (n == 0) { mt[4 * c + i] = m; lt[4 * c + i] = l; }
+            }
+        }
+    }
+    __syncthreads();
+    {   // the units' maxima over their tiles, then m -> the tile's weight exp(m - M)
+        const int u = threadIdx.x & 15, k = threadIdx.x >> 4;
+        float m = -INFINITY;
+        for (int t = k; t < nt; t += 16) m = fmaxf(m, mb[t * 16 + u]);
+        mx[u][k] = m;
+        __syncthreads();
+        #pragma unroll
+        for (int i = 0; i < 16; ++i) m = fmaxf(m, mx[u][i]);
+        for (int t = k; t < nt; t += 16) { const float v = mb[t * 16 + u]; mb[t * 16 + u] = v == -INFINITY ? 0.0f : lg_expf(v - m); }
+    }
+    __syncthreads();
+    for (int dg = wave; dg < HD / 64; dg += 4) {
+        float o[16], L[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+        #pragma unroll
+        for (int i = 0; i < 16; ++i) o[i] = 0.0f;
+        const __amdgpu_buffer_rsrc_t rv = lg_buffer_rsrc(a.vc + (size_t)kvh * HD + dg * 64);
+        const int vstep = a.kv_dim * 2;
+        uint16_t vb[2][16];
+        auto fetch = [&](uint16_t (&v)[16], int t, int hf) {  // value rows 16*hf .. +15 of a tile, dim dg*64 + lane
+            int r = ((t << 5) + 16 * hf) % a.seq;
+            #pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                v[k] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rv, lane * 2, __builtin_amdgcn_readfirstlane(r) * vstep, 0);
+                if (++r == a.seq) r = 0;
+            }
+        };
+        fetch(vb[0], tfirst, 0);
+        for (int t = tfirst; t <= tlast; ++t) {
+            const float *et = eb + (size_t)(t - tfirst) * 16 * ES + n * ES;
+            const float4 w = *(const float4 *)(mb + (t - tfirst) * 16 + 4 * c), l = *(const float4 *)(lb + (t - tfirst) * 16 + 4 * c);
+            float4 e[8];
+            #pragma unroll
+            for (int i = 0; i < 8; ++i) e[i] = *(const float4 *)(et + 4 * i);
+            fetch(vb[1], t, 1);
+            lg_v16f acc = {};
+            #pragma unroll
+            for (int k = 0; k < 16; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x1f32(((const float *)&e[k >> 2])[k & 3], lg_h2f(vb[0][k]), acc, 0, 0, 0);
+            if (t < tlast) fetch(vb[0], t + 1, 0);
+            #pragma unroll
+            for (int k = 0; k < 16; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x1f32(((const float *)&e[4 + (k >> 2)])[k & 3], lg_h2f(vb[1][k]), acc, 0, 0, 0);
+            const float wv[4] = { w.x, w.y, w.z, w.w }, lv[4] = { l.x, l.y, l.z, l.w };
+            #pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                L[i] = lg_fmaf(lv[i], wv[i], L[i]);
+                #pragma unroll
+                for (int b = 0; b < 4; ++b) o[4 * b + i] = lg_fmaf(acc[4 * b + i], wv[i], o[4 * b + i]);
+            }
+        }
+        #pragma unroll
+        for (int i = 0; i < 4; ++i)
+            #pragma unroll
+            for (int b = 0; b < 4; ++b) ob[4 * c + i][dg * 64 + 16 * b + n] = o[4 * b + i] / L[i];
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 16 * (HD / 4); i += LG_WG) {
+        const int u = i / (HD / 4), qd = i - u * (HD / 4), r = row0 + u / G;
+        if (u >= U || r > rlast) continue;                   // (whole groups of 8 lanes)
+        lg_wide_quant4(*(const float4 *)(&ob[u][qd * 4]), a.xq, a.H * HD >> 5, r, (kvh * G + u - u / G * G) * (HD / 32) + (qd >> 3));
+    }
+}
+static inline size_t lg_wide_attn_lds(int tiles) { return (size_t)tiles * 16 * 38 * 4; }

@@ -1,0 +1,36 @@
+"""The kernels of prompt blocks (lg_wide.h) at the sizes where they can go wrong: every workgroup shape of the matmul, weight
+rows that are no multiple of its 64-row tile, ragged activation rows, and prompts of every remainder through blocks of
+their own width, against the oracle bit for bit."""
+import numpy as np
+import pytest
+
+from conftest import random_q4_0
+from test_gpu_kernels import oracle_matmul
+from test_gpu_prefill import check_wide_prefill
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,k,rows", [(20480, 256, 32), (20480, 512, 64), (8200, 3840, 96), (264, 2560, 512), (2560, 5120, 160), (4160, 256, 480)])
+def test_wide_matmul_shapes(lg, ob, gpu_required, m, k, rows):
+    """64 x 32 tiles by four and by eight wavefronts, 64 x 64 tiles, a last weight tile of 8 rows, 32 K segments."""
+    rng = np.random.default_rng(m + k + rows)
+    w = random_q4_0(rng, m, k)
+    x = rng.normal(0, 1, (rows, k)).astype(np.float32)
+    x[1, :64] = 0.0
+    x[2] = np.sign(x[2])                                  # every value at the end of the q8 range
+    print(f"wide matmul m={m} k={k} rows={rows}", flush=True)
+    r = lg.hiplib.matmul_q4q8(w, k, m, x)
+    xq, xd, xs, out, _ = oracle_matmul(ob, w, k, m, x)
+    assert np.array_equal(r["xq"], xq) and np.array_equal(r["xsum"], xs) and np.array_equal(r["xd"].view(np.uint32), xd.view(np.uint32))
+    assert np.array_equal(r["out"].view(np.uint32), out.view(np.uint32))
+
+
+@pytest.mark.parametrize("name,n_prompt,over", [("tiny_full", 9, {}), ("tiny_full", 31, {}), ("tiny", 33, {}), ("tiny_full", 65, {}), ("tiny", 129, {}),
+                                                ("tiny", 70, {"n_ff": 10240}), ("tiny_full", 30, {"n_ff": 10240}), ("tiny", 1303, {}),
+                                                ("tiny", 61, {"n_head": 12, "n_head_kv": 4}), ("tiny_full", 50, {"n_head_kv": 8}), ("tiny", 45, {"head_dim_full": 512})])
+def test_ragged_prompts_leave_the_same_cache_and_logits(lg, ob, gpu_required, model_path, name, n_prompt, over):
+    """Blocks of any width (padded inside the kernels only), the gate/up shapes of 64 x 64 tiles, more key tiles than the
+    attention keeps in LDS, query groups that leave units idle (three heads per kv head) or one head each, 512-wide heads."""
+    path, spec = model_path(name, **over)
+    check_wide_prefill(lg, ob, path, spec, f"{name} {over}", n_prompt)
