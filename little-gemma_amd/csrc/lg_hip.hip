@@ -815,9 +815,8 @@ extern "C" void lg_hip_model_destroy(lg_hip_model *m) {
 // when they are too many for LDS.
 static int wide_attn_tiles(const lg_hip_model *m, const Layer &y, int rows, int pos) {
     const int rg = lg_wide_attn_rows(m->H / y.nkv), all = ((pos + rows - 1) >> 5) + 1;
-    if (!(y.is_local && m->window > 0)) return all;
-    const int t = (m->window + rg - 1 + 31) / 32 + 1;
-    return t < all ? t : all;
+    const int t = (y.is_local && m->window > 0) ? (m->window + rg - 1 + 31) / 32 + 1 : all;
+    return ((t < all ? t : all) + 3) & ~3;
 }
 static size_t wide_attn_scratch(const lg_hip_model *m, const Layer &y, int rows, int pos) {
     const int rg = lg_wide_attn_rows(m->H / y.nkv), tiles = wide_attn_tiles(m, y, rows, pos);
@@ -1606,8 +1605,8 @@ static int launch_wide_mm(Launcher &lx, int cls, const uint8_t *w, const int8_t 
 template <int HD>
 static void launch_wide_attn(Launcher &lx, const WideAttn &a, int groups) {
     const dim3 grid(groups, a.nkv);
-    if (a.tiles <= LG_WA_TILES) LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, true>), grid, dim3(LG_WG), lg_wide_attn_lds(a.tiles), a, lx.m->ctl);
-    else                        LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false>), grid, dim3(LG_WG), 0, a, lx.m->ctl);
+    if (a.tiles <= LG_WA_TILES) LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, true>), grid, dim3(LG_WA_WG), lg_wide_attn_lds(a.tiles), a, lx.m->ctl);
+    else                        LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false>), grid, dim3(LG_WA_WG), 0, a, lx.m->ctl);
 }
 
 // One block of `rows` prompt positions from pos on (tokens in device memory): the launch sequence of a verify step with
@@ -1933,7 +1932,8 @@ extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *tok
     if (pos0 < 0 || n > kv->max_seq - pos0) return fail(-2, "positions %d..%lld do not fit a cache of %d", pos0, (long long)pos0 + n - 1, kv->max_seq);
     for (int i = 0; i < n; ++i) if (toks[i] < 0 || toks[i] >= m->n_vocab) return fail(-2, "token id %d outside the vocabulary of %d", toks[i], m->n_vocab);
     HIP_TRY(hipSetDevice(m->device));
-    const bool wide_ok = !m->target && m->wide_prefill;
+    bool wide_ok = !m->target && m->wide_prefill;
+    for (size_t L = 0; L < kv->seq.size(); ++L) wide_ok = wide_ok && (size_t)kv->seq[L] * kv->kv_dim[L] * 2 < ((size_t)1 << 31);   // (the prompt kernels address a layer's cache with 32 bits)
     const int cap = m->sched_cap * LG_HIP_MAX_ROWS;        // tokens the staging holds
     for (int at = 0; at < n;) {
         // the tokens go over once, the blocks follow each other on the stream and the host waits at the end

@@ -424,57 +424,63 @@ __global__ __launch_bounds__(LG_WG) void lg_k_wide_quant(const float *x, int row
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Attention of a wide block.  A workgroup is 4 wavefronts on 16 units = (rows, query heads) of one kv head.  Both products
-// run on v_mfma_f32_16x16x1_4b_f32, whose every step is one fma per output (K = 1), so the defined chains are exactly its
-// accumulation order:
-//  * scores: the instruction's four blocks are the four chains c of a score (dims 4g + c, g ascending), a step per g; a
-//    lane ends up with all four chains of its outputs and adds (a0+a1)+(a2+a3).  The wavefronts take key tiles in turn.
-//    Queries stay in registers; K rows come straight from the cache, 64 bytes of a row by four lanes, and are dealt to the
-//    chains by a 4 x 4 exchange over the four 16-lane rows.
-//  * values: the four blocks are 16 dims each, a step per key slot (masked slots have weight 0); a wavefront takes 64 dims
-//    and walks the tiles in order, adding each tile's result to the running sum with the weight exp(m_tile - M).
+// Attention of a wide block.  A workgroup is 8 wavefronts on 16 units = (rows, query heads) of one kv head.  Both products
+// run on f32 matrix instructions whose accumulation is the defined chain:
+//  * scores: the four blocks of v_mfma_f32_16x16x1_4b_f32 (one fma per output and step, subnormals included) are the four
+//    chains c of a score (dims 4g + c), a step per g ascending; a lane ends up with all four chains of its outputs and adds
+//    (a0+a1)+(a2+a3).  Queries wait in LDS chain by chain; K rows come straight from the cache, 64 bytes of a row by four
+//    lanes, and are dealt to the chains by a 4 x 4 exchange over the four 16-lane rows.  The wavefronts take key tiles in
+//    turn, the next tile's rows in flight.  (v_mfma_f32_16x16x4_f32, k = four steps of a chain, adds in the same order and
+//    needs no exchange, but its operands come as 8-byte pieces of a row, twice the cache accesses: 47 -> 54 us.)
+//  * values: the same instruction, its four blocks are four consecutive tiles, a step per key slot (masked slots have
+//    weight 0), the columns 16 dims; a wavefront takes 32 dims as two such products, so that one 4-byte load per lane feeds
+//    two steps, and adds the tiles' results to the running sum in tile order with the weights exp(m_tile - M).
 // The weights e of a row's tiles, their maxima and sums wait in LDS between the two (EL: up to LG_WA_TILES tiles; more: in
-// the cache's scratch).  On vector units the same block took a kernel per phase, and the tiles' results (1 KiB per tile
-// and head) went through memory: 56 + 15 us per layer and 512 rows at the E4B shape.
-#define LG_WA_TILES 36
+// the cache's scratch).  Bound by the matrix cores (8 to 9 thousand cycles per 16 units and tile) and the exponentials.
+// Eight wavefronts rather than four: one workgroup is all the LDS holds on a CU, and with two wavefronts on a SIMD one
+// loads, deals and exponentiates while the other multiplies.  500 rows of a 512-wide window of 256-wide heads (8 over 2):
+// 65 -> 43 us; 512 rows of a 1024-wide one (16 over 8): 232 -> 137 us; all of 4093 positions (16 over 1): 584 -> 400 us.
+#define LG_WA_TILES 44
+#define LG_WA_WG 512
 struct WideAttn {
     const float *q;              // [rows][H*hd] normed + rotated
     const uint16_t *kc, *vc;     // cache of the layer this one reads
     int H, nkv, seq, kv_dim, window, rows;
     float *scratch;              // !EL: per group tiles * 16 * 34 floats
-    int tiles;                   // tiles a group can touch
+    int tiles;                   // tiles a group can touch, rounded up to a multiple of four
     uint8_t *xq;                 // wide digits of the result, width H*hd
 };
 static inline int lg_wide_attn_rows(int G) { return 16 / G; }
+static inline size_t lg_wide_attn_lds(int tiles) { return (size_t)tiles * 16 * 38 * 4; }
 __device__ __forceinline__ float lg_max16(float v) {
     v = lg_max8(v);
     return fmaxf(v, lg_dpp_f<LG_DPP_MIRROR16>(v));
 }
+// 4 x 4 exchange over the four 16-lane rows of a wavefront: lane row c holds x0..x3 and receives element c of the rows
+// 0..3 in o[0..3].
+__device__ __forceinline__ void lg_deal4(uint32_t x0, uint32_t x1, uint32_t x2, uint32_t x3, uint32_t (&o)[4]) {
+    const lg_u2 p = __builtin_amdgcn_permlane32_swap(x0, x2, false, false), q = __builtin_amdgcn_permlane32_swap(x1, x3, false, false);
+    const lg_u2 x = __builtin_amdgcn_permlane16_swap(p.x, q.x, false, false), y = __builtin_amdgcn_permlane16_swap(p.y, q.y, false, false);
+    o[0] = x.x; o[1] = x.y; o[2] = y.x; o[3] = y.y;
+}
 template <int HD, bool EL>
-__global__ __launch_bounds__(LG_WG, HD > 256 ? 1 : 2) void lg_k_wide_attn(WideAttn a, const StepCtl *ctl) {
+__global__ __launch_bounds__(LG_WA_WG, 2) void lg_k_wide_attn(WideAttn a, const StepCtl *ctl) {
     extern __shared__ __align__(16) unsigned char smem[];
-    constexpr int NS = HD / 32;                               // 64-byte pieces of a K row
+    constexpr int NW = LG_WA_WG / 64;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), n = lane & 15, c = lane >> 4;
     const int G = a.H / a.nkv, RG = 16 / G, U = RG * G, kvh = blockIdx.y, row0 = blockIdx.x * RG;
     const int pos = ctl->pos;
     int rlast = row0 + RG - 1;
     if (rlast >= a.rows) rlast = a.rows - 1;
-    const int tfirst = lg_win_start(pos + row0, a.window) >> 5, tlast = (pos + rlast) >> 5, nt = tlast - tfirst + 1;
-    // e: [tile][16 units][36] (a 16-byte multiple off the 128-byte bank period), m and l: [tile][16]
+    const int tfirst = lg_win_start(pos + row0, a.window) >> 5, tlast = (pos + rlast) >> 5;
+    const int nt = (tlast - tfirst + 4) & ~3;                 // tiles past the last one are masked throughout
+    // e: [tile][16 units][ES] (36: off the bank period), weights m and sums l: [tile][16]
     constexpr int ES = EL ? 36 : 32;
     float *eb = EL ? (float *)smem : a.scratch + ((size_t)blockIdx.x * a.nkv + kvh) * a.tiles * (16 * 34);
-    float *mb = eb + (size_t)(EL ? nt : a.tiles) * 16 * ES, *lb = mb + (size_t)(EL ? nt : a.tiles) * 16;
-    __shared__ float mx[16][17];
+    float *mb = eb + (size_t)a.tiles * 16 * ES, *lb = mb + (size_t)a.tiles * 16;
+    __shared__ float mx[16][LG_WA_WG / 16 + 1];
     __shared__ __align__(16) float ob[16][HD + 4];
     {
-        // this lane's query elements: unit n, chain c
-        const int ur = n / G, uh = n - ur * G;
-        int qr = row0 + ur;
-        if (n >= U || qr > rlast) qr = rlast;
-        const float *qp = a.q + (size_t)qr * a.H * HD + (size_t)(kvh * G + (n < U ? uh : 0)) * HD + c;
-        float qv[HD / 4];
-        #pragma unroll
-        for (int g = 0; g < HD / 4; ++g) qv[g] = qp[4 * g];
         // validity of this lane's outputs: units 4c + i
         int us[4], up[4];
         #pragma unroll
@@ -484,34 +490,66 @@ __global__ __launch_bounds__(LG_WG, HD > 256 ? 1 : 2) void lg_k_wide_attn(WideAt
             up[i] = on ? pos + r : -1;
             us[i] = on ? lg_win_start(pos + r, a.window) : 0;
         }
-        for (int t = tfirst + wave; t <= tlast; t += 4) {
-            const int t0 = t << 5, ring0 = t0 % a.seq;
-            int r0 = ring0 + n, r1 = ring0 + 16 + n;          // ring rows of this lane's two keys
-            if (r0 >= a.seq) r0 -= a.seq;
-            if (r1 >= a.seq) r1 -= a.seq;
-            if (a.seq < 32) { r0 %= a.seq; r1 %= a.seq; }
+        // a tile's K rows (512-wide heads: half of them) are requested as soon as the ones before them have been dealt
+        constexpr int NS = HD / 32, CH = NS < 8 ? NS : 8;     // 64-byte pieces of a K row
+        uint4 w0[CH], w1[CH];
+        auto request = [&](int t, int s0) {
+            const int ring0 = (t << 5) % a.seq;
+            int r0 = ring0 + n, r1 = ring0 + 16 + n;          // ring rows of this lane's two keys (a ring is a multiple of 32 rows, or as long as the positions go)
+            if (r0 >= a.seq) r0 = a.seq - 1;
+            if (r1 >= a.seq) r1 = a.seq - 1;
             const uint16_t *k0 = a.kc + (size_t)r0 * a.kv_dim + (size_t)kvh * HD + c * 8, *k1 = a.kc + (size_t)r1 * a.kv_dim + (size_t)kvh * HD + c * 8;
-            uint4 w0[NS], w1[NS];
             #pragma unroll
-            for (int s = 0; s < NS; ++s) { w0[s] = *(const uint4 *)(k0 + s * 32); w1[s] = *(const uint4 *)(k1 + s * 32); }
+            for (int s = 0; s < CH; ++s) { w0[s] = *(const uint4 *)(k0 + (s0 + s) * 32); w1[s] = *(const uint4 *)(k1 + (s0 + s) * 32); }
+        };
+        request(tfirst + wave, 0);
+        // the units' query rows into LDS, chain by chain: [unit][i % 4][i / 4] (in registers a wave's copy of them spilled)
+        for (int i = threadIdx.x; i < 16 * (HD / 4); i += LG_WA_WG) {
+            const int u = i / (HD / 4), j = i - u * (HD / 4), ur = u / G;
+            int qr = row0 + ur;
+            if (u >= U || qr > rlast) qr = rlast;
+            const float4 f = *(const float4 *)(a.q + (size_t)qr * a.H * HD + (size_t)(kvh * G + (u < U ? u - ur * G : 0)) * HD + 4 * j);
+            float *qd = &ob[u][j];
+            qd[0] = f.x; qd[HD / 4] = f.y; qd[2 * (HD / 4)] = f.z; qd[3 * (HD / 4)] = f.w;
+        }
+        __syncthreads();
+        const float *qs = &ob[n][c * (HD / 4)];               // this lane's query elements: unit n, chain c
+        for (int t = tfirst + wave; t < tfirst + nt; t += NW) {
+            const int t0 = t << 5;
+            if (t > tlast) {                                  // a tile that only fills up the last four
+                float *et = eb + (size_t)(t - tfirst) * 16 * ES;
+                for (int i = lane; i < 16 * 32; i += 64) et[(i >> 5) * ES + (i & 31)] = 0.0f;
+                if (lane < 16) { mb[(t - tfirst) * 16 + lane] = -INFINITY; lb[(t - tfirst) * 16 + lane] = 0.0f; }
+                continue;
+            }
             lg_v16f d0 = {}, d1 = {};
             #pragma unroll
-            for (int s = 0; s < NS; ++s) {
+            for (int s0 = 0; s0 < NS; s0 += CH) {
                 // dims 32s + 8c + 0..7 of a key -> the same key's dims 32s + 4g + c, g = 0..7, as f16 pairs in g order
-                auto deal = [](uint4 w, uint32_t (&o)[4]) {
-                    uint32_t a0 = __builtin_amdgcn_perm(w.z, w.x, 0x05040100u), a1 = __builtin_amdgcn_perm(w.z, w.x, 0x07060302u);
-                    uint32_t a2 = __builtin_amdgcn_perm(w.w, w.y, 0x05040100u), a3 = __builtin_amdgcn_perm(w.w, w.y, 0x07060302u);
-                    const lg_u2 p = __builtin_amdgcn_permlane32_swap(a0, a2, false, false), q = __builtin_amdgcn_permlane32_swap(a1, a3, false, false);
-                    const lg_u2 x = __builtin_amdgcn_permlane16_swap(p.x, q.x, false, false), y = __builtin_amdgcn_permlane16_swap(p.y, q.y, false, false);
-                    o[0] = x.x; o[1] = x.y; o[2] = y.x; o[3] = y.y;
-                };
-                uint32_t o0[4], o1[4];
-                deal(w0[s], o0); deal(w1[s], o1);
+                uint32_t o0[CH][4], o1[CH][4];
                 #pragma unroll
-                for (int g = 0; g < 8; ++g) {
-                    const float b0 = lg_h2f((uint16_t)(o0[g >> 1] >> (16 * (g & 1)))), b1 = lg_h2f((uint16_t)(o1[g >> 1] >> (16 * (g & 1))));
-                    d0 = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[8 * s + g], b0, d0, 0, 0, 0);
-                    d1 = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[8 * s + g], b1, d1, 0, 0, 0);
+                for (int s = 0; s < CH; ++s) {
+                    auto deal = [](uint4 w, uint32_t (&o)[4]) {
+                        lg_deal4(__builtin_amdgcn_perm(w.z, w.x, 0x05040100u), __builtin_amdgcn_perm(w.z, w.x, 0x07060302u),
+                                 __builtin_amdgcn_perm(w.w, w.y, 0x05040100u), __builtin_amdgcn_perm(w.w, w.y, 0x07060302u), o);
+                    };
+                    deal(w0[s], o0[s]); deal(w1[s], o1[s]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                if (s0 + CH < NS) request(t, s0 + CH);
+                else request(t + NW, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                #pragma unroll
+                for (int s = 0; s < CH; ++s) {
+                    const float4 qa = *(const float4 *)(qs + 8 * (s0 + s)), qb = *(const float4 *)(qs + 8 * (s0 + s) + 4);
+                    if (s & 1) __builtin_amdgcn_sched_barrier(0);      // (else all of them are fetched at once and spill)
+                    const float qv[8] = { qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w };
+                    #pragma unroll
+                    for (int g = 0; g < 8; ++g) {
+                        const float b0 = lg_h2f((uint16_t)(o0[s][g >> 1] >> (16 * (g & 1)))), b1 = lg_h2f((uint16_t)(o1[s][g >> 1] >> (16 * (g & 1))));
+                        d0 = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[g], b0, d0, 0, 0, 0);
+                        d1 = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[g], b1, d1, 0, 0, 0);
+                    }
                 }
             }
             float *et = eb + (size_t)(t - tfirst) * 16 * ES, *mt = mb + (t - tfirst) * 16, *lt = lb + (t - tfirst) * 16;
@@ -533,61 +571,65 @@ __global__ __launch_bounds__(LG_WG, HD > 256 ? 1 : 2) void lg_k_wide_attn(WideAt
     {   // the units' maxima over their tiles, then m -> the tile's weight exp(m - M)
         const int u = threadIdx.x & 15, k = threadIdx.x >> 4;
         float m = -INFINITY;
-        for (int t = k; t < nt; t += 16) m = fmaxf(m, mb[t * 16 + u]);
+        for (int t = k; t < nt; t += LG_WA_WG / 16) m = fmaxf(m, mb[t * 16 + u]);
         mx[u][k] = m;
         __syncthreads();
-        #pragma unroll
-        for (int i = 0; i < 16; ++i) m = fmaxf(m, mx[u][i]);
-        for (int t = k; t < nt; t += 16) { const float v = mb[t * 16 + u]; mb[t * 16 + u] = v == -INFINITY ? 0.0f : lg_expf(v - m); }
+        for (int i = 0; i < LG_WA_WG / 16; ++i) m = fmaxf(m, mx[u][i]);
+        for (int t = k; t < nt; t += LG_WA_WG / 16) { const float v = mb[t * 16 + u]; mb[t * 16 + u] = v == -INFINITY ? 0.0f : lg_expf(v - m); }
     }
     __syncthreads();
-    for (int dg = wave; dg < HD / 64; dg += 4) {
-        float o[16], L[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+    for (int dg = wave; dg < HD / 32; dg += NW) {
+        float o[2][4], L[4];
         #pragma unroll
-        for (int i = 0; i < 16; ++i) o[i] = 0.0f;
-        const __amdgpu_buffer_rsrc_t rv = lg_buffer_rsrc(a.vc + (size_t)kvh * HD + dg * 64);
-        const int vstep = a.kv_dim * 2;
-        uint16_t vb[2][16];
-        auto fetch = [&](uint16_t (&v)[16], int t, int hf) {  // value rows 16*hf .. +15 of a tile, dim dg*64 + lane
-            int r = ((t << 5) + 16 * hf) % a.seq;
+        for (int i = 0; i < 4; ++i) { o[0][i] = o[1][i] = 0.0f; L[i] = 0.0f; }
+        // value rows of this lane's tile t + c, dims dg*32 + 2n and 2n + 1: a run of 8 slots is requested three runs ahead.
+        // Buffer loads: the tile's place in the lane offset, the slot's in a scalar register (as flat loads their 64-bit
+        // addresses cost more vector instructions than the conversions); the buffer ends with the ring, slots past it read 0.
+        constexpr int RUN = 8, AHEAD = 3;
+        uint32_t v[AHEAD + 1][RUN];
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)a.vc, 0, (uint32_t)a.seq * (uint32_t)a.kv_dim * 2u, 0x00020000);
+        const int vcol = (kvh * HD + dg * 32 + 2 * n) * 2, vrow = a.kv_dim * 2;
+        auto fetch = [&](uint32_t (&d)[RUN], int t, int k0) {
+            const int off = (((t + c) << 5) % a.seq) * vrow + vcol;
             #pragma unroll
-            for (int k = 0; k < 16; ++k) {
-                v[k] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rv, lane * 2, __builtin_amdgcn_readfirstlane(r) * vstep, 0);
-                if (++r == a.seq) r = 0;
-            }
+            for (int k = 0; k < RUN; ++k) d[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rv, off, (k0 + k) * vrow, 0);
         };
-        fetch(vb[0], tfirst, 0);
-        for (int t = tfirst; t <= tlast; ++t) {
-            const float *et = eb + (size_t)(t - tfirst) * 16 * ES + n * ES;
-            const float4 w = *(const float4 *)(mb + (t - tfirst) * 16 + 4 * c), l = *(const float4 *)(lb + (t - tfirst) * 16 + 4 * c);
-            float4 e[8];
+        #pragma unroll
+        for (int i = 0; i < AHEAD; ++i) fetch(v[i], tfirst, RUN * i);
+        for (int t = 0; t < nt; t += 4) {
+            const float *et = eb + (size_t)(t + c) * 16 * ES + n * ES;
+            lg_v16f acc0 = {}, acc1 = {};
             #pragma unroll
-            for (int i = 0; i < 8; ++i) e[i] = *(const float4 *)(et + 4 * i);
-            fetch(vb[1], t, 1);
-            lg_v16f acc = {};
-            #pragma unroll
-            for (int k = 0; k < 16; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x1f32(((const float *)&e[k >> 2])[k & 3], lg_h2f(vb[0][k]), acc, 0, 0, 0);
-            if (t < tlast) fetch(vb[0], t + 1, 0);
-            #pragma unroll
-            for (int k = 0; k < 16; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x1f32(((const float *)&e[4 + (k >> 2)])[k & 3], lg_h2f(vb[1][k]), acc, 0, 0, 0);
-            const float wv[4] = { w.x, w.y, w.z, w.w }, lv[4] = { l.x, l.y, l.z, l.w };
-            #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                L[i] = lg_fmaf(lv[i], wv[i], L[i]);
+            for (int i = 0; i < 4; ++i) {                     // (four runs per tile: AHEAD + 1 buffers in turn)
+                if (i == 0) fetch(v[3], tfirst + t, 24);
+                else fetch(v[i - 1], tfirst + (t + 4 < nt ? t + 4 : t), RUN * (i - 1));
+                const float4 ea = *(const float4 *)(et + RUN * i), ec = *(const float4 *)(et + RUN * i + 4);
+                const float e[8] = { ea.x, ea.y, ea.z, ea.w, ec.x, ec.y, ec.z, ec.w };
                 #pragma unroll
-                for (int b = 0; b < 4; ++b) o[4 * b + i] = lg_fmaf(acc[4 * b + i], wv[i], o[4 * b + i]);
+                for (int k = 0; k < RUN; ++k) {
+                    acc0 = __builtin_amdgcn_mfma_f32_16x16x1f32(e[k], lg_h2f((uint16_t)(v[i][k] & 0xFFFF)), acc0, 0, 0, 0);
+                    acc1 = __builtin_amdgcn_mfma_f32_16x16x1f32(e[k], lg_h2f((uint16_t)(v[i][k] >> 16)), acc1, 0, 0, 0);
+                }
+            }
+            #pragma unroll
+            for (int b = 0; b < 4; ++b) {                     // tiles in order
+                const float4 w = *(const float4 *)(mb + (t + b) * 16 + 4 * c), l = *(const float4 *)(lb + (t + b) * 16 + 4 * c);
+                const float wv[4] = { w.x, w.y, w.z, w.w }, lv[4] = { l.x, l.y, l.z, l.w };
+                #pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    L[i] = lg_fmaf(lv[i], wv[i], L[i]);
+                    o[0][i] = lg_fmaf(acc0[4 * b + i], wv[i], o[0][i]);
+                    o[1][i] = lg_fmaf(acc1[4 * b + i], wv[i], o[1][i]);
+                }
             }
         }
         #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            #pragma unroll
-            for (int b = 0; b < 4; ++b) ob[4 * c + i][dg * 64 + 16 * b + n] = o[4 * b + i] / L[i];
+        for (int i = 0; i < 4; ++i) *(float2 *)(&ob[4 * c + i][dg * 32 + 2 * n]) = make_float2(o[0][i] / L[i], o[1][i] / L[i]);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < 16 * (HD / 4); i += LG_WG) {
+    for (int i = threadIdx.x; i < 16 * (HD / 4); i += LG_WA_WG) {
         const int u = i / (HD / 4), qd = i - u * (HD / 4), r = row0 + u / G;
         if (u >= U || r > rlast) continue;                   // (whole groups of 8 lanes)
         lg_wide_quant4(*(const float4 *)(&ob[u][qd * 4]), a.xq, a.H * HD >> 5, r, (kvh * G + u - u / G * G) * (HD / 32) + (qd >> 3));
     }
 }
-static inline size_t lg_wide_attn_lds(int tiles) { return (size_t)tiles * 16 * 38 * 4; }
