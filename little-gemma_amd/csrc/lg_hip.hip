@@ -9,6 +9,8 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <array>
+#include <chrono>
 #include <map>
 #include <mutex>
 #include <string>
@@ -166,6 +168,8 @@ enum KClass { KC_ROWS, KC_PMP, KC_QKV, KC_QKVPOST, KC_ATTN, KC_MERGE, KC_O, KC_G
 static const char *k_class_names[KC_COUNT] = { "rows_norm_quant", "ple_model_proj", "qkv", "qkv_post", "attn_tiles", "attn_merge",
     "attn_output", "gate_up_geglu", "ffn_down", "ple_gate", "ple_proj", "lm_head", "accept", "ffn_xcd", "ple_tail", "attn_tail" };
 
+// What a captured graph was captured for: the cache's id, the options, the block width and the rest of the options.
+typedef std::array<uint64_t, 3> GraphKey;
 struct Profile {
     bool on = false;
     std::vector<hipEvent_t> ev;        // pairs
@@ -209,6 +213,7 @@ struct lg_hip_model {
     int32_t *sched = nullptr, *out = nullptr, *adv = nullptr;
     int sched_cap = 0, sched_steps = 0, sched_rows = 0, sched_pos0 = 0, sched_loaded = 0;
     int32_t *pin = nullptr;            // pinned host staging
+    int reports = 0;                   // steps the host has waited for: the last one's StepCtl.report
     int last_rows = 0, last_adv = 0;
     int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0;
     // the feed-forward half of a layer as one XCD-partitioned launch (lg_xffn.h): built when the shape and the chip fit
@@ -237,7 +242,7 @@ struct lg_hip_model {
     float *slabs = nullptr, *xact = nullptr; // [8][max_rows][E] partial sums of ffn_down; [8][max_rows][max FF/8] gelu(gate)*up per XCD
     uint32_t *xq8 = nullptr;                 // [8][E/32][80] q8 rows per XCD
     XcdSync *xsync = nullptr;
-    std::map<std::string, hipGraphExec_t> graphs;
+    std::map<GraphKey, hipGraphExec_t> graphs;
     Profile prof;
     // a draft head (src/mtp.c) is a model whose layers own no cache: they read `target`'s
     lg_hip_model *target = nullptr;
@@ -784,8 +789,9 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
     if (dev_alloc(m, &m->sched, (size_t)m->sched_cap * LG_HIP_MAX_ROWS) || dev_alloc(m, &m->out, (size_t)m->sched_cap * LG_HIP_MAX_ROWS) ||
         dev_alloc(m, &m->adv, (size_t)m->sched_cap))
         return -7;
-    // pinned staging: step state at 0, a verify block's successors at 32 and accept count at 48, a block's or a prompt's tokens from 64
-    HIP_TRY(hipHostMalloc((void **)&m->pin, (64 + (size_t)m->sched_cap * LG_HIP_MAX_ROWS) * sizeof(int32_t), hipHostMallocDefault));
+    // pinned staging: a step's state at 0, a reported step's results at 32 (LG_REPORT_*), from 64 a prompt's tokens or the results of rounds
+    HIP_TRY(hipHostMalloc((void **)&m->pin, (64 + (size_t)m->sched_cap * (2 * LG_HIP_MAX_ROWS + 1)) * sizeof(int32_t), hipHostMallocDefault));
+    m->pin[32 + LG_REPORT_SEQ] = 0;
     HIP_TRY(hipDeviceSynchronize());
     m->committed = true;
     return 0;
@@ -873,12 +879,11 @@ extern "C" void lg_hip_kv_destroy(lg_hip_kv *kv) {
     (void)hipSetDevice(kv->m->device);
     (void)hipDeviceSynchronize();
     // graphs captured for this cache hold its pointers
-    const std::string tag = "kv" + std::to_string(kv->id) + ":";
     std::vector<lg_hip_model *> holders(kv->m->drafts);
     holders.push_back(kv->m);
     for (lg_hip_model *h : holders)
         for (auto it = h->graphs.begin(); it != h->graphs.end();) {
-            if (it->first.compare(0, tag.size(), tag) == 0) { (void)hipGraphExecDestroy(it->second); it = h->graphs.erase(it); }
+            if (it->first[0] == (uint64_t)kv->id) { (void)hipGraphExecDestroy(it->second); it = h->graphs.erase(it); }
             else ++it;
         }
     for (size_t L = 0; L < kv->k.size(); ++L) {
@@ -951,7 +956,7 @@ extern "C" int lg_hip_kv_restore_prefix(lg_hip_kv *kv, int n) {
     return 0;
 }
 
-__global__ void lg_k_set_ctl(StepCtl *ctl, int pos) { ctl->pos = pos; ctl->step = 0; ctl->err = 0; ctl->pad = 0; }
+__global__ void lg_k_set_ctl(StepCtl *ctl, int pos) { ctl->pos = pos; ctl->step = 0; ctl->err = 0; ctl->report = 0; }
 
 // ---- launching --------------------------------------------------------------------------------
 static size_t lds_mm(int M, int k) { return (size_t)M * k + (size_t)M * (k / 32) * 8; }
@@ -1573,7 +1578,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 LAUNCH(KC_HEAD, (lg_k_head_m<M>), dim3(grid), dim3(512), (size_t)(E / 32) * LG_MU_DWORDS * 4, LG_HEAD_FIELDS(LG_XA, h) 0);
         } else
         LAUNCH(KC_HEAD, (lg_k_mm_head<M>), dim3(grid), dim3(LG_WG), lds_mm(M, E), LG_HEAD_FIELDS(LG_XA, h) 0);
-        AcceptArgs c{ m->pval, m->pidx, grid, m->sched, m->out, m->adv, m->hidden_rows, m->g_hidden, E };
+        AcceptArgs c{ m->pval, m->pidx, grid, m->sched, m->out, m->adv, m->hidden_rows, m->g_hidden, E, m->pin + 32 };
         LAUNCH(KC_ACCEPT, (lg_k_accept<M>), dim3(1), dim3(LG_WG), 0, m->ctl, LG_ACCEPT_FIELDS(LG_XA, c) 0);
     } else if (!lx.rc && !dry) {
         hipLaunchKernelGGL(lg_k_advance, dim3(1), dim3(1), 0, m->stream, m->ctl, M);
@@ -1714,10 +1719,21 @@ static int enqueue_step_rows(lg_hip_model *m, lg_hip_kv *kv, int rows, bool with
     return fail(-2, "rows %d outside 1..%d", rows, LG_HIP_MAX_ROWS);
 }
 
+// what: 0 a block without its head, 1 a step, 2 a speculative round
+static GraphKey graph_key(const lg_hip_model *m, const lg_hip_kv *kv, int rows, int what) {
+    uint64_t o = 0;
+    auto put = [&](unsigned v, int bits) { o = o << bits | (v & ((1u << bits) - 1u)); };
+    put(what, 2); put(rows, 4); put(m->store_logits != 0, 1); put(m->draft_chain, 1); put(m->fuse_rows, 1); put(m->attn_rows, 1); put(m->attn_rows_fq, 1);
+    put(m->head_mfma, 1); put(m->down_kq, 1); put(m->xcd_ffn, 1); put(m->fork_ple, 1); put(m->rows_geglu, 1); put(m->tail_stamps != 0, 1);
+    put(m->tail_spread == 1 ? 1 : m->tail_spread ? 2 : 0, 2); put(m->xcd_tail, 2); put(m->down_m, 2); put(m->xcd_attn_tail, 2); put(m->merge_o, 2);
+    put(m->xffn_delay, 10);
+    return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices };
+}
+
 // launch one step, through a captured graph when enabled
 static int launch_step(lg_hip_model *m, lg_hip_kv *kv, int rows, bool with_head) {
     if (!m->use_graph || m->prof.on) return enqueue_step_rows(m, kv, rows, with_head);
-    const std::string key = "kv" + std::to_string(kv->id) + ":" + std::to_string(rows) + (with_head ? "h" : "p") + (m->store_logits ? "l" : "") + (m->draft_chain ? "c" : "") + (m->fuse_rows ? "" : "u") + (m->attn_rows ? "" : "r") + (m->attn_rows_fq ? "" : "q") + (m->head_mfma ? "" : "s") + (m->down_kq ? "" : "d") + (m->xcd_ffn ? "x" + std::to_string(m->xffn_delay) : "") + (m->fork_ple ? "" : "f") + "t" + std::to_string(m->xcd_tail) + (m->tail_spread == 1 ? "" : m->tail_spread ? "N" : "n") + (m->rows_geglu ? "g" : "") + (m->tail_stamps ? "s" : "") + (m->down_m ? "D" + std::to_string(m->down_m) : "") + "a" + std::to_string(m->xcd_attn_tail) + "o" + std::to_string(m->merge_o) + "." + std::to_string(m->merge_o_slices);
+    const GraphKey key = graph_key(m, kv, rows, with_head ? 1 : 0);
     auto it = m->graphs.find(key);
     if (it == m->graphs.end()) {
         hipGraph_t graph = nullptr;
@@ -1780,12 +1796,28 @@ static int step_err(const char *who, int err) {
                 (err & LG_XFFN_ERR_WAIT) ? "a hand-over that was given up " : "", err);
 }
 
-static int load_block(lg_hip_model *m, const int32_t *toks, int rows, int pos) {
-    StepCtl c{ pos, 0, 0, 0 };
-    memcpy(m->pin, &c, sizeof c);
-    memcpy(m->pin + 64, toks, (size_t)rows * 4);
-    HIP_TRY(hipMemcpyAsync(m->ctl, m->pin, sizeof c, hipMemcpyHostToDevice, m->stream));
-    HIP_TRY(hipMemcpyAsync(m->sched, m->pin + 64, (size_t)rows * 4, hipMemcpyHostToDevice, m->stream));
+// The step's state and tokens.  `report`: its accept kernel also writes its results to the host, who waits for them with
+// wait_report: two copies in front of a step and three behind it cost 20 to 30 us of it.
+static int load_block(lg_hip_model *m, const int32_t *toks, int rows, int pos, bool report) {
+    LoadArgs a{};
+    memcpy(a.tok, toks, (size_t)rows * 4);
+    if (report && ++m->reports == INT32_MAX) m->reports = 1;
+    hipLaunchKernelGGL(lg_k_load, dim3(1), dim3(1), 0, m->stream, m->ctl, m->sched, pos, rows, report ? m->reports : 0, a);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+static int wait_report(lg_hip_model *m, const char *who, int rows, int32_t *out, int32_t *adv) {
+    const int32_t *r = m->pin + 32;
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int spins = 0; __atomic_load_n(r + LG_REPORT_SEQ, __ATOMIC_ACQUIRE) != m->reports; ++spins) {
+        if ((spins & 1023) != 1023 || std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(50)) { __builtin_ia32_pause(); continue; }
+        HIP_TRY(hipStreamSynchronize(m->stream));           // far longer than a step takes: a slow device, or an error that this returns
+        if (__atomic_load_n(r + LG_REPORT_SEQ, __ATOMIC_ACQUIRE) != m->reports) return fail(-9, "%s: the step ended without its results", who);
+    }
+    const int rc = step_err(who, r[LG_REPORT_ERR]);
+    if (rc) return rc;
+    memcpy(out, r + LG_REPORT_OUT, (size_t)rows * 4);
+    *adv = r[LG_REPORT_ADV];
     return 0;
 }
 
@@ -1795,15 +1827,9 @@ extern "C" int lg_hip_forward_spec(lg_hip_model *m, lg_hip_kv *kv, const int32_t
     if (rc) return rc;
     if (!out || !adv) return fail(-1, "forward_spec: null output");
     HIP_TRY(hipSetDevice(m->device));
-    if ((rc = load_block(m, toks, rows, pos))) return rc;
+    if ((rc = load_block(m, toks, rows, pos, true))) return rc;
     if ((rc = launch_step(m, kv, rows, true))) return rc;
-    HIP_TRY(hipMemcpyAsync(m->pin + 32, m->out, (size_t)rows * 4, hipMemcpyDeviceToHost, m->stream));
-    HIP_TRY(hipMemcpyAsync(m->pin + 48, m->adv, 4, hipMemcpyDeviceToHost, m->stream));
-    HIP_TRY(hipMemcpyAsync(m->pin + 56, m->ctl, sizeof(StepCtl), hipMemcpyDeviceToHost, m->stream));
-    HIP_TRY(hipStreamSynchronize(m->stream));
-    if ((rc = step_err("forward_spec", m->pin[58]))) return rc;
-    memcpy(out, m->pin + 32, (size_t)rows * 4);
-    *adv = m->pin[48];
+    if ((rc = wait_report(m, "forward_spec", rows, out, adv))) return rc;
     m->last_rows = rows; m->last_adv = *adv;
     return 0;
 }
@@ -1839,15 +1865,13 @@ extern "C" int lg_hip_draft_step(lg_hip_model *d, lg_hip_kv *kv, int token, int 
     if (d->H > t->max_rows * t->H) return fail(-2, "draft_step: %d draft heads do not fit the target's attention scratch", d->H);
     HIP_TRY(hipSetDevice(d->device));
     int rc;
-    int32_t tk = token;
-    if ((rc = load_block(d, &tk, 1, pos))) return rc;
+    int32_t tk = token, adv;
+    if ((rc = load_block(d, &tk, 1, pos, true))) return rc;
     d->draft_chain = chain != 0;
     rc = launch_step(d, kv, 1, true);
     d->draft_chain = false;
     if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(d->pin + 32, d->out, 4, hipMemcpyDeviceToHost, d->stream));
-    HIP_TRY(hipStreamSynchronize(d->stream));
-    *tok_out = d->pin[32];
+    if ((rc = wait_report(d, "draft_step", 1, tok_out, &adv))) return rc;
     d->last_rows = 1; d->last_adv = 1;
     return 0;
 }
@@ -1888,11 +1912,12 @@ extern "C" int lg_hip_mtp_rounds(lg_hip_model *d, lg_hip_kv *kv, int token, int 
     HIP_TRY(hipSetDevice(t->device));
     int rc;
     int32_t tk = token;
-    if ((rc = load_block(t, &tk, 1, pos))) return rc;
+    if ((rc = load_block(t, &tk, 1, pos, false))) return rc;
     if (!t->use_graph || t->prof.on || d->prof.on) {
         for (int r = 0; r < n_rounds; ++r) if ((rc = enqueue_round(d, kv, rows, false))) return rc;
     } else {
-        const std::string key = "kv" + std::to_string(kv->id) + ":round" + std::to_string(rows) + (t->store_logits ? "l" : "") + (d->store_logits ? "L" : "") + (t->fuse_rows ? "" : "u") + (d->fuse_rows ? "" : "v") + (t->attn_rows ? "" : "r") + (t->attn_rows_fq ? "" : "q") + (t->head_mfma ? "" : "s") + (t->down_kq ? "" : "d") + (t->xcd_ffn ? "x" : "") + (t->fork_ple ? "" : "f") + "t" + std::to_string(t->xcd_tail) + (t->tail_spread == 1 ? "" : t->tail_spread ? "N" : "n") + (t->rows_geglu ? "g" : "") + (t->down_m ? "D" + std::to_string(t->down_m) : "") + "a" + std::to_string(t->xcd_attn_tail) + "o" + std::to_string(t->merge_o) + "." + std::to_string(t->merge_o_slices);
+        GraphKey key = graph_key(t, kv, rows, 2);
+        key[1] |= (uint64_t)(d->store_logits != 0) << 62 | (uint64_t)(d->fuse_rows != 0) << 63;
         auto it = d->graphs.find(key);            // kept by the head: the graph dies with it or with the cache
         if (it == d->graphs.end()) {
             hipGraph_t graph = nullptr;
@@ -1910,14 +1935,20 @@ extern "C" int lg_hip_mtp_rounds(lg_hip_model *d, lg_hip_kv *kv, int token, int 
         }
         for (int r = 0; r < n_rounds; ++r) HIP_TRY(hipGraphLaunch(it->second, t->stream));
     }
+    const size_t nb = (size_t)n_rounds * rows;
+    int32_t *res = t->pin + 64;
+    HIP_TRY(hipMemcpyAsync(t->pin, t->ctl, sizeof(StepCtl), hipMemcpyDeviceToHost, t->stream));
+    HIP_TRY(hipMemcpyAsync(res, t->sched, nb * 4, hipMemcpyDeviceToHost, t->stream));
+    HIP_TRY(hipMemcpyAsync(res + nb, t->out, nb * 4, hipMemcpyDeviceToHost, t->stream));
+    HIP_TRY(hipMemcpyAsync(res + 2 * nb, t->adv, (size_t)n_rounds * 4, hipMemcpyDeviceToHost, t->stream));
     HIP_TRY(hipStreamSynchronize(t->stream));
     StepCtl c;
-    HIP_TRY(hipMemcpy(&c, t->ctl, sizeof c, hipMemcpyDeviceToHost));
+    memcpy(&c, t->pin, sizeof c);
     if (c.step != n_rounds) return fail(-9, "mtp_rounds: %d of %d rounds ran", c.step, n_rounds);
     { const int erc = step_err("mtp_rounds", c.err); if (erc) return erc; }
-    HIP_TRY(hipMemcpy(blocks, t->sched, (size_t)n_rounds * rows * 4, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(out, t->out, (size_t)n_rounds * rows * 4, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(adv, t->adv, (size_t)n_rounds * 4, hipMemcpyDeviceToHost));
+    memcpy(blocks, res, nb * 4);
+    memcpy(out, res + nb, nb * 4);
+    memcpy(adv, res + 2 * nb, (size_t)n_rounds * 4);
     if (final_pos) *final_pos = c.pos;
     t->last_rows = rows; t->last_adv = adv[n_rounds - 1];
     t->sched_steps = 0;
@@ -2086,7 +2117,7 @@ extern "C" int lg_hip_profile_step(lg_hip_model *m, lg_hip_kv *kv, const int32_t
     double acc[KC_COUNT] = { 0 };
     int cnt[KC_COUNT] = { 0 };
     for (int r = 0; r < repeats + 1; ++r) {              // first pass warms up and is dropped
-        if ((rc = load_block(m, toks, rows, pos))) return rc;
+        if ((rc = load_block(m, toks, rows, pos, false))) return rc;
         m->prof.on = true;
         rc = enqueue_step_rows(m, kv, rows, true);
         m->prof.on = false;

@@ -16,7 +16,7 @@ struct StepCtl {            // device-resident step state
     int pos;                // position of row 0 of the current block
     int step;               // index of the current block in the token schedule
     int err;
-    int pad;
+    int report;             // not 0: the step's results also go to the host's memory, with this value behind them (lg_k_accept)
 };
 
 // ---------------------------------------------------------------------------------------------
@@ -907,15 +907,20 @@ struct AcceptArgs {
     int32_t *out;            // [n_steps][M]
     int32_t *adv;            // [n_steps]
     const float *hidden_rows; float *g_hidden; int E;
+    int32_t *host;           // pinned host words (LG_REPORT_*)
 };
-#define LG_ACCEPT_FIELDS(X, v) X(const float *, pval, pval, v) X(const int *, pidx, pidx, v) X(int, n_part, n_part, v) X(int, E, E, v) X(const int32_t *, toks, toks, v) X(const float *, hidden_rows, hidden_rows, v) X(int32_t *, out, out, v) X(int32_t *, adv, adv, v) X(float *, g_hidden, g_hidden, v)
+#define LG_REPORT_OUT 0      // where a reported step's results lie: successors of its rows,
+#define LG_REPORT_ADV 16     // its accept count,
+#define LG_REPORT_ERR 17     // StepCtl.err,
+#define LG_REPORT_SEQ 24     // StepCtl.report, written last
+#define LG_ACCEPT_FIELDS(X, v) X(const float *, pval, pval, v) X(const int *, pidx, pidx, v) X(int, n_part, n_part, v) X(int, E, E, v) X(const int32_t *, toks, toks, v) X(const float *, hidden_rows, hidden_rows, v) X(int32_t *, out, out, v) X(int32_t *, adv, adv, v) X(float *, g_hidden, g_hidden, v) X(int32_t *, host, host, v)
 template <int M>
 __global__ __launch_bounds__(LG_WG) void lg_k_accept(StepCtl *ctl, LG_ACCEPT_FIELDS(LG_XP, _) int p_end_) {
     AcceptArgs a; LG_ACCEPT_FIELDS(LG_XI, a)
     __shared__ float sv[LG_HIP_MAX_ROWS_DEV][LG_WG / 64];
     __shared__ int si[LG_HIP_MAX_ROWS_DEV][LG_WG / 64];
     __shared__ int s_adv;
-    const int step = ctl->step, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int step = ctl->step, report = ctl->report, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // the block's tokens and this thread's slice of every row's hidden state are requested with the partials: read
     // when they are needed (the tokens one after the other in the accept loop, the accepted row after it) each costs
     // a memory round trip of its own at the end of the step
@@ -967,6 +972,12 @@ __global__ __launch_bounds__(LG_WG) void lg_k_accept(StepCtl *ctl, LG_ACCEPT_FIE
         for (int j = 0; j < M; ++j) a.out[(size_t)step * M + j] = best[j];
         a.adv[step] = adv;
         s_adv = adv;
+        // a step that the host waits for: written from here, the results cost it no copies behind the step
+        if (report) {
+            for (int j = 0; j < M; ++j) a.host[LG_REPORT_OUT + j] = best[j];
+            a.host[LG_REPORT_ADV] = adv;
+            a.host[LG_REPORT_ERR] = ctl->err;
+        }
     }
     __syncthreads();
     const int adv = s_adv;
@@ -983,7 +994,18 @@ __global__ __launch_bounds__(LG_WG) void lg_k_accept(StepCtl *ctl, LG_ACCEPT_FIE
         for (int i = threadIdx.x; i < a.E; i += LG_WG) a.g_hidden[i] = a.hidden_rows[(size_t)(adv - 1) * a.E + i];
     }
     __syncthreads();
-    if (threadIdx.x == 0) { ctl->pos += adv; ctl->step = step + 1; }
+    if (threadIdx.x == 0) {
+        ctl->pos += adv; ctl->step = step + 1;
+        if (report) __hip_atomic_store(a.host + LG_REPORT_SEQ, report, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// A step's state and its block's tokens, as kernel arguments: one launch ahead of the step instead of two copies.
+struct LoadArgs { int32_t tok[LG_HIP_MAX_ROWS_DEV]; };
+__global__ void lg_k_load(StepCtl *ctl, int32_t *sched, int pos, int rows, int report, LoadArgs a) {
+    #pragma unroll
+    for (int j = 0; j < LG_HIP_MAX_ROWS_DEV; ++j) if (j < rows) sched[j] = a.tok[j];
+    ctl->pos = pos; ctl->step = 0; ctl->err = 0; ctl->report = report;
 }
 
 // Prefill blocks skip the head: only the position advances.
@@ -1016,6 +1038,7 @@ __global__ void lg_k_link(LinkArgs a) {
         a.hsched[0] = tok;
         a.hctl->pos = a.tctl->pos + a.phase - 1;
         a.hctl->step = 0;
+        a.hctl->report = 0;
     }
 }
 
