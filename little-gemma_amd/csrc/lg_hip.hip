@@ -755,7 +755,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         dev_alloc(m, &m->dout, 4 * R * E) || dev_alloc(m, &m->q_rot, R * max_qd) || dev_alloc(m, &m->hidden_rows, HR * E) || dev_alloc(m, &m->g_hidden, (size_t)E) ||
         dev_alloc(m, &m->aq, qb(max_qd)) || dev_alloc(m, &m->gq, qb(max_ff)) || dev_alloc(m, &m->hq, qb(E) + (size_t)12 * E) ||
         dev_alloc(m, &m->pval, HR * (m->n_vocab / 32)) || dev_alloc(m, &m->pidx, HR * (m->n_vocab / 32)) ||
-        dev_alloc(m, &m->logits, HR * m->n_vocab) || dev_alloc(m, &m->ctl, (size_t)1))
+        dev_alloc(m, &m->ctl, (size_t)1))
         return -7;
     if (m->ple && dev_alloc(m, &m->eq, qb(E) + (size_t)12 * E)) return -7;
     if (!m->target) {                        // hand-over state of the one-XCD kernels (lg_xtail.h)
@@ -783,6 +783,8 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         m->xcd_ffn = getenv("LG_HIP_XCD_FFN") && atoi(getenv("LG_HIP_XCD_FFN")) != 0;     // off unless asked for: the separate kernels are faster (see lg_xffn.h)
         m->xffn_delay = 0x100;
     }
+    // logits lie in pinned host memory: the head writes them across the bus while it runs (a copy behind the step cost 25 us a row)
+    HIP_TRY(hipHostMalloc((void **)&m->logits, HR * m->n_vocab * 4, hipHostMallocDefault));
     HIP_TRY(hipMemset(m->ctl, 0, sizeof(StepCtl)));
     HIP_TRY(hipMemset(m->g_hidden, 0, (size_t)E * 4));
     m->sched_cap = 4096;
@@ -805,6 +807,7 @@ extern "C" void lg_hip_model_destroy(lg_hip_model *m) {
     for (void *p : m->allocs) (void)hipFree(p);
     for (hipEvent_t e : m->prof.ev) (void)hipEventDestroy(e);
     if (m->pin) (void)hipHostFree(m->pin);
+    if (m->logits) (void)hipHostFree(m->logits);
     if (m->target) {
         auto &v = m->target->drafts;
         for (size_t i = 0; i < v.size(); ++i) if (v[i] == m) { v.erase(v.begin() + i); break; }
@@ -2019,7 +2022,7 @@ extern "C" int lg_hip_get_logits(lg_hip_model *m, int row, float *dst) {
     if (row < 0 || row >= m->last_rows) return fail(-2, "get_logits: row %d of a %d-row step", row, m->last_rows);
     HIP_TRY(hipSetDevice(m->device));
     HIP_TRY(hipStreamSynchronize(m->stream));
-    HIP_TRY(hipMemcpy(dst, m->logits + (size_t)row * m->n_vocab, (size_t)m->n_vocab * 4, hipMemcpyDeviceToHost));
+    memcpy(dst, m->logits + (size_t)row * m->n_vocab, (size_t)m->n_vocab * 4);
     return 0;
 }
 
