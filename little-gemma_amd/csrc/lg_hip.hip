@@ -862,16 +862,20 @@ extern "C" int lg_hip_kv_create(lg_hip_model *m, int max_seq, lg_hip_kv **out) {
     }
     const size_t slots = pbytes / ((size_t)max_hd * 4 + 8);
     kv->scratch_bytes = slots * max_hd * 4;
-    for (kv->prompt_rows = wide_rows_for(max_seq); kv->prompt_rows > LG_WIDE; kv->prompt_rows -= LG_WIDE) {
+    auto prompt_scratch = [&](int rows) {
         size_t most = 0;
         for (int L = 0; L < nl; ++L) {
-            const size_t n = wide_attn_scratch(m, m->L[L], kv->prompt_rows, max_seq - kv->prompt_rows > 0 ? max_seq - kv->prompt_rows : 0);
+            const size_t n = wide_attn_scratch(m, m->L[L], rows, max_seq > rows ? max_seq - rows : 0);
             most = n > most ? n : most;
         }
-        if (most <= kv->scratch_bytes) break;
-    }
+        return most;
+    };
+    kv->prompt_rows = wide_rows_for(max_seq);
+    while (kv->prompt_rows > LG_WIDE && prompt_scratch(kv->prompt_rows) > kv->scratch_bytes) kv->prompt_rows -= LG_WIDE;
+    // partials of verify blocks of one or two rows (a long cache, a model committed for no more) are smaller than what 32 prompt rows need
+    if (prompt_scratch(kv->prompt_rows) > kv->scratch_bytes) kv->scratch_bytes = prompt_scratch(kv->prompt_rows);
     if (hipMalloc((void **)&kv->pm, slots * 4) != hipSuccess || hipMalloc((void **)&kv->pl, slots * 4) != hipSuccess ||
-        hipMalloc((void **)&kv->pacc, slots * max_hd * 4) != hipSuccess) { lg_hip_kv_destroy(kv); return fail(-7, "kv_create: out of device memory for attention partials"); }
+        hipMalloc((void **)&kv->pacc, kv->scratch_bytes) != hipSuccess) { lg_hip_kv_destroy(kv); return fail(-7, "kv_create: out of device memory for attention partials"); }
     HIP_TRY(hipDeviceSynchronize());
     *out = kv;
     return 0;

@@ -34,3 +34,24 @@ def test_ragged_prompts_leave_the_same_cache_and_logits(lg, ob, gpu_required, mo
     attention keeps in LDS, query groups that leave units idle (three heads per kv head) or one head each, 512-wide heads."""
     path, spec = model_path(name, **over)
     check_wide_prefill(lg, ob, path, spec, f"{name} {over}", n_prompt)
+
+
+def test_long_cache_of_a_model_for_single_rows(lg, ob, gpu_required, model_path):
+    """A model committed for one row with a cache too long for wide partials: the weights of 32 prompt rows over all its
+    tiles need more memory than the partials of single rows, and the cache has it.  Against the same prompt row by row."""
+    path, spec = model_path("tiny", n_head=16, n_head_kv=2, head_dim_full=512)
+    max_seq, n = 70000, 33
+    pos0 = max_seq - n - 1
+    prompt = np.random.default_rng(1).integers(1, spec["n_vocab"], n).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, max_seq, max_rows=1)
+    try:
+        got = []
+        for wide in (1, 0):
+            gpu.new_cache()
+            gpu.set_option("wide_prefill", wide)
+            print(f"33 positions at {pos0}, wide {wide}", flush=True)
+            gpu.prefill(prompt, pos0)
+            got.append([gpu.kv_read(L, w) for L in range(spec["n_layer"] - spec["shared_kv_layers"]) for w in (0, 1)])
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
+    finally:
+        gpu.close()
