@@ -472,7 +472,8 @@ __global__ __launch_bounds__(LG_WA_WG, 2) void lg_k_wide_attn(WideAttn a, const 
     const int pos = ctl->pos;
     int rlast = row0 + RG - 1;
     if (rlast >= a.rows) rlast = a.rows - 1;
-    const int tfirst = lg_win_start(pos + row0, a.window) >> 5, tlast = (pos + rlast) >> 5;
+    const int kfirst = lg_win_start(pos + row0, a.window), klast = pos + rlast;       // positions any row of the group sees
+    const int tfirst = kfirst >> 5, tlast = klast >> 5;
     const int nt = (tlast - tfirst + 4) & ~3;                 // tiles past the last one are masked throughout
     // e: [tile][16 units][ES] (36: off the bank period), weights m and sums l: [tile][16]
     constexpr int ES = EL ? 36 : 32;
@@ -605,6 +606,11 @@ __global__ __launch_bounds__(LG_WA_WG, 2) void lg_k_wide_attn(WideAttn a, const 
                 else fetch(v[i - 1], tfirst + (t + 4 < nt ? t + 4 : t), RUN * (i - 1));
                 const float4 ea = *(const float4 *)(et + RUN * i), ec = *(const float4 *)(et + RUN * i + 4);
                 const float e[8] = { ea.x, ea.y, ea.z, ea.w, ec.x, ec.y, ec.z, ec.w };
+                if (t == 0 || t + 4 >= nt) {                  // rows that no row of the group sees may hold anything (infinities too)
+                    const int p = ((tfirst + t + c) << 5) + RUN * i;
+                    #pragma unroll
+                    for (int k = 0; k < RUN; ++k) if (p + k < kfirst || p + k > klast) v[i][k] = 0;
+                }
                 #pragma unroll
                 for (int k = 0; k < RUN; ++k) {
                     acc0 = __builtin_amdgcn_mfma_f32_16x16x1f32(e[k], lg_h2f((uint16_t)(v[i][k] & 0xFFFF)), acc0, 0, 0, 0);

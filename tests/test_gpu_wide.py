@@ -36,6 +36,39 @@ def test_ragged_prompts_leave_the_same_cache_and_logits(lg, ob, gpu_required, mo
     check_wide_prefill(lg, ob, path, spec, f"{name} {over}", n_prompt)
 
 
+@pytest.mark.parametrize("name,pos0,n", [("tiny", 0, 45), ("tiny", 301, 70), ("tiny_full", 300, 33)])
+def test_rows_no_position_sees_may_hold_anything(lg, ob, gpu_required, model_path, name, pos0, n):
+    """Infinities and NaN in the cache rows behind the prompt and in front of its windows (what a discarded branch of a
+    conversation can leave) change no bit of what a prompt writes."""
+    path, spec = model_path(name)
+    rng = np.random.default_rng(n)
+    prompt = rng.integers(1, spec["n_vocab"], pos0 + n).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, 640, max_rows=4)
+    try:
+        got = []
+        for garbage in (0, 1):
+            gpu.new_cache()
+            if pos0:
+                gpu.prefill(prompt[:pos0], 0)
+            for L, y in enumerate(gpu.layers):
+                if L >= spec["n_layer"] - spec["shared_kv_layers"] or not garbage:
+                    continue
+                rows = gpu.kv_layout(L)[0]
+                seen = np.arange(max(0, pos0 + 1 - spec["sliding_window"]) if y["is_local"] else 0, pos0)
+                hidden = np.setdiff1d(np.arange(rows), seen % rows)
+                for which, bits in ((0, 0x7E00), (1, 0x7C00)):
+                    d = gpu.kv_read(L, which)
+                    d[hidden] = bits
+                    gpu.kv_write(L, which, d)
+            print(f"{name}: {n} positions at {pos0}, garbage {garbage}", flush=True)
+            gpu.prefill(prompt[pos0:], pos0)
+            got.append([gpu.kv_read(L, w)[np.arange(pos0, pos0 + n) % gpu.kv_layout(L)[0]]
+                        for L in range(spec["n_layer"] - spec["shared_kv_layers"]) for w in (0, 1)])
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
+    finally:
+        gpu.close()
+
+
 def test_long_cache_of_a_model_for_single_rows(lg, ob, gpu_required, model_path):
     """A model committed for one row with a cache too long for wide partials: the weights of 32 prompt rows over all its
     tiles need more memory than the partials of single rows, and the cache has it.  Against the same prompt row by row."""
