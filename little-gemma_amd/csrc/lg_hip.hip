@@ -1737,28 +1737,35 @@ static GraphKey graph_key(const lg_hip_model *m, const lg_hip_kv *kv, int rows, 
     return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices };
 }
 
-// launch one step, through a captured graph when enabled
+// What `enqueue` launches on the stream, as a graph.
+template <typename F>
+static int capture_graph(hipStream_t st, F enqueue, hipGraphExec_t *exec) {
+    hipGraph_t graph = nullptr;
+    HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+    const int rc = enqueue();
+    hipError_t e = hipStreamEndCapture(st, &graph);
+    if (rc) { if (graph) (void)hipGraphDestroy(graph); return rc; }
+    if (e != hipSuccess) return fail(-100 - (int)e, "hipStreamEndCapture: %s", hipGetErrorString(e));
+    e = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    if (e != hipSuccess) return fail(-100 - (int)e, "hipGraphInstantiate: %s", hipGetErrorString(e));
+    return 0;
+}
+
+// Launch one step, through a captured graph when enabled.  The first step of a (cache, width, options) runs as plain
+// launches, and its graph is captured behind them, while the device works on the step and the host would only wait
+// (a first decode step on a new cache, E4B shape: 3.95 -> 2.28 ms; capturing and instantiating 341 launches takes 1.5).
 static int launch_step(lg_hip_model *m, lg_hip_kv *kv, int rows, bool with_head) {
     if (!m->use_graph || m->prof.on) return enqueue_step_rows(m, kv, rows, with_head);
     const GraphKey key = graph_key(m, kv, rows, with_head ? 1 : 0);
     auto it = m->graphs.find(key);
-    if (it == m->graphs.end()) {
-        hipGraph_t graph = nullptr;
-        hipGraphExec_t exec = nullptr;
-        int rc = enqueue_step_rows(m, kv, rows, with_head, true);
-        if (rc) return rc;
-        HIP_TRY(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-        rc = enqueue_step_rows(m, kv, rows, with_head);
-        hipError_t e = hipStreamEndCapture(m->stream, &graph);
-        if (rc) { if (graph) (void)hipGraphDestroy(graph); return rc; }
-        if (e != hipSuccess) return fail(-100 - (int)e, "hipStreamEndCapture: %s", hipGetErrorString(e));
-        e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(graph);
-        if (e != hipSuccess) return fail(-100 - (int)e, "hipGraphInstantiate: %s", hipGetErrorString(e));
-        it = m->graphs.emplace(key, exec).first;
-    }
-    HIP_TRY(hipGraphLaunch(it->second, m->stream));
-    return 0;
+    if (it != m->graphs.end()) { HIP_TRY(hipGraphLaunch(it->second, m->stream)); return 0; }
+    hipGraphExec_t exec = nullptr;
+    int rc = enqueue_step_rows(m, kv, rows, with_head, true);
+    if (!rc) rc = enqueue_step_rows(m, kv, rows, with_head);
+    if (!rc) rc = capture_graph(m->stream, [&]() { return enqueue_step_rows(m, kv, rows, with_head); }, &exec);
+    if (!rc) m->graphs.emplace(key, exec);
+    return rc;
 }
 
 static int check_block(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int n, int rows, int pos) {
@@ -1926,21 +1933,15 @@ extern "C" int lg_hip_mtp_rounds(lg_hip_model *d, lg_hip_kv *kv, int token, int 
         GraphKey key = graph_key(t, kv, rows, 2);
         key[1] |= (uint64_t)(d->store_logits != 0) << 62 | (uint64_t)(d->fuse_rows != 0) << 63;
         auto it = d->graphs.find(key);            // kept by the head: the graph dies with it or with the cache
-        if (it == d->graphs.end()) {
-            hipGraph_t graph = nullptr;
+        int r = 0;
+        if (it == d->graphs.end()) {               // the first round as launches, its graph while the device works on it
             hipGraphExec_t exec = nullptr;
-            if ((rc = enqueue_round(d, kv, rows, true))) return rc;
-            HIP_TRY(hipStreamBeginCapture(t->stream, hipStreamCaptureModeThreadLocal));
-            rc = enqueue_round(d, kv, rows, false);
-            hipError_t e = hipStreamEndCapture(t->stream, &graph);
-            if (rc) { if (graph) (void)hipGraphDestroy(graph); return rc; }
-            if (e != hipSuccess) return fail(-100 - (int)e, "hipStreamEndCapture: %s", hipGetErrorString(e));
-            e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(graph);
-            if (e != hipSuccess) return fail(-100 - (int)e, "hipGraphInstantiate: %s", hipGetErrorString(e));
+            if ((rc = enqueue_round(d, kv, rows, true)) || (rc = enqueue_round(d, kv, rows, false)) ||
+                (rc = capture_graph(t->stream, [&]() { return enqueue_round(d, kv, rows, false); }, &exec))) return rc;
             it = d->graphs.emplace(key, exec).first;
+            r = 1;
         }
-        for (int r = 0; r < n_rounds; ++r) HIP_TRY(hipGraphLaunch(it->second, t->stream));
+        for (; r < n_rounds; ++r) HIP_TRY(hipGraphLaunch(it->second, t->stream));
     }
     const size_t nb = (size_t)n_rounds * rows;
     int32_t *res = t->pin + 64;
