@@ -1614,11 +1614,20 @@ static int launch_wide_mm(Launcher &lx, int cls, const uint8_t *w, const int8_t 
     else                LAUNCH(cls, (lg_k_wide_mm<2, 4, DUMP>), grid, block, lds, a, out, dots);
     return parts;
 }
+// Up to 128 workgroups (half of the chip) with 12 tiles and more: scores and values as two launches over more workgroups (200
+// rows, 100 workgroups: 41 -> 39 us in a 512-wide window, 175 -> 113 us over 100 tiles; with 130 workgroups 42 -> 55 us, with 8
+// tiles 23 us both ways).  Score workgroups take 4 tiles, or up to 16 while there are more than 512 of them.
 template <int HD>
-static void launch_wide_attn(Launcher &lx, const WideAttn &a, int groups) {
+static void launch_wide_attn(Launcher &lx, const WideAttn &a, int groups, size_t scratch_bytes) {
     const dim3 grid(groups, a.nkv);
-    if (a.tiles <= LG_WA_TILES) LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, true>), grid, dim3(LG_WA_WG), lg_wide_attn_lds(a.tiles), a, lx.m->ctl);
-    else                        LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false>), grid, dim3(LG_WA_WG), 0, a, lx.m->ctl);
+    const int wgs = groups * a.nkv;
+    if (wgs <= 128 && a.tiles >= 12 && a.tiles <= LG_WA_SPLIT_MAX && (size_t)wgs * a.tiles * (16 * 34 * 4) <= scratch_bytes) {
+        int chunk = 4;
+        while (chunk < 16 && wgs * (a.tiles / chunk) > 512) chunk *= 2;
+        LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false, 1>), dim3(groups, a.nkv, (a.tiles + chunk - 1) / chunk), dim3(LG_WA_SPLIT_WG), 0, a, lx.m->ctl);
+        LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false, 2>), dim3(groups, a.nkv, HD > 128 ? HD / 128 : 1), dim3(LG_WA_SPLIT_WG), (size_t)a.tiles * 64, a, lx.m->ctl);
+    } else if (a.tiles <= LG_WA_TILES) LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, true>), grid, dim3(LG_WA_WG), lg_wide_attn_lds(a.tiles), a, lx.m->ctl);
+    else                               LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false>), grid, dim3(LG_WA_WG), 0, a, lx.m->ctl);
 }
 
 // One block of `rows` prompt positions from pos on (tokens in device memory): the launch sequence of a verify step with
@@ -1671,10 +1680,10 @@ static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, i
         const WideAttn a{ m->q_rot, kv->k[y.src], kv->v[y.src], H, y.nkv, kv->seq[y.src], y.kd, window, rows, kv->pacc,
                           wide_attn_tiles(m, y, rows, pos), (uint8_t *)m->aq };
         switch (y.hd) {
-            case 512: launch_wide_attn<512>(lx, a, groups); break;
-            case 256: launch_wide_attn<256>(lx, a, groups); break;
-            case 128: launch_wide_attn<128>(lx, a, groups); break;
-            default:  launch_wide_attn<64>(lx, a, groups);
+            case 512: launch_wide_attn<512>(lx, a, groups, kv->scratch_bytes); break;
+            case 256: launch_wide_attn<256>(lx, a, groups, kv->scratch_bytes); break;
+            case 128: launch_wide_attn<128>(lx, a, groups, kv->scratch_bytes); break;
+            default:  launch_wide_attn<64>(lx, a, groups, kv->scratch_bytes);
         }
         pend_parts = launch_wide_mm<false>(lx, KC_O, y.wo_w, m->aq, y.qd, E, rows, m->dout, nullptr);
         pend_dout = m->dout; pend_w = y.post_attn;

@@ -440,8 +440,16 @@ __global__ __launch_bounds__(LG_WG) void lg_k_wide_quant(const float *x, int row
 // Eight wavefronts rather than four: one workgroup is all the LDS holds on a CU, and with two wavefronts on a SIMD one
 // loads, deals and exponentiates while the other multiplies.  500 rows of a 512-wide window of 256-wide heads (8 over 2):
 // 65 -> 43 us; 512 rows of a 1024-wide one (16 over 8): 232 -> 137 us; all of 4093 positions (16 over 1): 584 -> 400 us.
+// In memory the weights are requested with the value rows, runs ahead (512 rows at 3500, 16 heads over 8: 474 -> 450 us).
+//
+// PHASE 1 and 2 are the two halves as kernels of their own, for blocks whose groups do not fill the chip: the time of a
+// workgroup is a matter of its tiles (22 rows at position 3000 take 40 us on 12 workgroups, 487 rows 45 on 244).  PHASE 1 deals the
+// tiles of a group to gridDim.z workgroups of four wavefronts, PHASE 2 the dims, 128 to a workgroup: each wavefront has a
+// matrix core of its own.  22 rows at 3000: 512-wide window 40 -> 29 us, all positions 171 -> 74 us; at 20000 1083 -> 355 us.
 #define LG_WA_TILES 44
 #define LG_WA_WG 512
+#define LG_WA_SPLIT_WG 256
+#define LG_WA_SPLIT_MAX 1024             // tiles whose weights PHASE 2 keeps in LDS
 struct WideAttn {
     const float *q;              // [rows][H*hd] normed + rotated
     const uint16_t *kc, *vc;     // cache of the layer this one reads
@@ -463,10 +471,11 @@ __device__ __forceinline__ void lg_deal4(uint32_t x0, uint32_t x1, uint32_t x2, 
     const lg_u2 x = __builtin_amdgcn_permlane16_swap(p.x, q.x, false, false), y = __builtin_amdgcn_permlane16_swap(p.y, q.y, false, false);
     o[0] = x.x; o[1] = x.y; o[2] = y.x; o[3] = y.y;
 }
-template <int HD, bool EL>
-__global__ __launch_bounds__(LG_WA_WG, 2) void lg_k_wide_attn(WideAttn a, const StepCtl *ctl) {
+template <int HD, bool EL, int PHASE = 0>
+__global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wide_attn(WideAttn a, const StepCtl *ctl) {
     extern __shared__ __align__(16) unsigned char smem[];
-    constexpr int NW = LG_WA_WG / 64;
+    constexpr int WG = PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, NW = WG / 64;
+    static_assert(PHASE == 0 || !EL, "the two kernels hand the weights over in memory");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), n = lane & 15, c = lane >> 4;
     const int G = a.H / a.nkv, RG = 16 / G, U = RG * G, kvh = blockIdx.y, row0 = blockIdx.x * RG;
     const int pos = ctl->pos;
@@ -479,9 +488,10 @@ __global__ __launch_bounds__(LG_WA_WG, 2) void lg_k_wide_attn(WideAttn a, const 
     constexpr int ES = EL ? 36 : 32;
     float *eb = EL ? (float *)smem : a.scratch + ((size_t)blockIdx.x * a.nkv + kvh) * a.tiles * (16 * 34);
     float *mb = eb + (size_t)a.tiles * 16 * ES, *lb = mb + (size_t)a.tiles * 16;
-    __shared__ float mx[16][LG_WA_WG / 16 + 1];
+    float *wb = PHASE == 2 ? (float *)smem : mb;              // the tiles' weights exp(m - M): several workgroups of values read the maxima
+    __shared__ float mx[16][WG / 16 + 1];
     __shared__ __align__(16) float ob[16][HD + 4];
-    {
+    if constexpr (PHASE != 2) {
         // validity of this lane's outputs: units 4c + i
         int us[4], up[4];
         #pragma unroll
@@ -503,9 +513,10 @@ __global__ __launch_bounds__(LG_WA_WG, 2) void lg_k_wide_attn(WideAttn a, const 
             #pragma unroll
             for (int s = 0; s < CH; ++s) { w0[s] = *(const uint4 *)(k0 + (s0 + s) * 32); w1[s] = *(const uint4 *)(k1 + (s0 + s) * 32); }
         };
-        request(tfirst + wave, 0);
+        const int t1 = tfirst + (PHASE ? blockIdx.z * NW : 0) + wave, step = PHASE ? gridDim.z * NW : NW;
+        request(t1, 0);
         // the units' query rows into LDS, chain by chain: [unit][i % 4][i / 4] (in registers a wave's copy of them spilled)
-        for (int i = threadIdx.x; i < 16 * (HD / 4); i += LG_WA_WG) {
+        for (int i = threadIdx.x; i < 16 * (HD / 4); i += WG) {
             const int u = i / (HD / 4), j = i - u * (HD / 4), ur = u / G;
             int qr = row0 + ur;
             if (u >= U || qr > rlast) qr = rlast;
@@ -515,7 +526,7 @@ __global__ __launch_bounds__(LG_WA_WG, 2) void lg_k_wide_attn(WideAttn a, const 
         }
         __syncthreads();
         const float *qs = &ob[n][c * (HD / 4)];               // this lane's query elements: unit n, chain c
-        for (int t = tfirst + wave; t < tfirst + nt; t += NW) {
+        for (int t = t1; t < tfirst + nt; t += step) {
             const int t0 = t << 5;
             if (t > tlast) {                                  // a tile that only fills up the last four
                 float *et = eb + (size_t)(t - tfirst) * 16 * ES;
@@ -538,7 +549,7 @@ __global__ __launch_bounds__(LG_WA_WG, 2) void lg_k_wide_attn(WideAttn a, const 
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 if (s0 + CH < NS) request(t, s0 + CH);
-                else request(t + NW, 0);
+                else request(t + step, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 #pragma unroll
                 for (int s = 0; s < CH; ++s) {
@@ -568,64 +579,85 @@ __global__ __launch_bounds__(LG_WA_WG, 2) void lg_k_wide_attn(WideAttn a, const 
             }
         }
     }
+    if constexpr (PHASE == 1) return;
     __syncthreads();
     {   // the units' maxima over their tiles, then m -> the tile's weight exp(m - M)
         const int u = threadIdx.x & 15, k = threadIdx.x >> 4;
         float m = -INFINITY;
-        for (int t = k; t < nt; t += LG_WA_WG / 16) m = fmaxf(m, mb[t * 16 + u]);
+        for (int t = k; t < nt; t += WG / 16) m = fmaxf(m, mb[t * 16 + u]);
         mx[u][k] = m;
         __syncthreads();
-        for (int i = 0; i < LG_WA_WG / 16; ++i) m = fmaxf(m, mx[u][i]);
-        for (int t = k; t < nt; t += LG_WA_WG / 16) { const float v = mb[t * 16 + u]; mb[t * 16 + u] = v == -INFINITY ? 0.0f : lg_expf(v - m); }
+        for (int i = 0; i < WG / 16; ++i) m = fmaxf(m, mx[u][i]);
+        for (int t = k; t < nt; t += WG / 16) { const float v = mb[t * 16 + u]; wb[t * 16 + u] = v == -INFINITY ? 0.0f : lg_expf(v - m); }
     }
     __syncthreads();
-    for (int dg = wave; dg < HD / 32; dg += NW) {
+    const int ndg = PHASE == 2 ? HD / 32 / gridDim.z : HD / 32, dg0 = PHASE == 2 ? blockIdx.z * ndg : 0;      // runs of 32 dims of this workgroup
+    for (int dg = dg0 + wave; dg < dg0 + ndg; dg += NW) {
         float o[2][4], L[4];
         #pragma unroll
         for (int i = 0; i < 4; ++i) { o[0][i] = o[1][i] = 0.0f; L[i] = 0.0f; }
-        // value rows of this lane's tile t + c, dims dg*32 + 2n and 2n + 1: a run of 8 slots is requested three runs ahead.
+        // A run is 8 slots of this lane's tile 4g + c (value rows, dims dg*32 + 2n and 2n + 1; !EL: their weights as well, which
+        // come from memory too): requested AHEAD runs ahead, a group of four tiles is four runs.
         // Buffer loads: the tile's place in the lane offset, the slot's in a scalar register (as flat loads their 64-bit
         // addresses cost more vector instructions than the conversions); the buffer ends with the ring, slots past it read 0.
-        constexpr int RUN = 8, AHEAD = 3;
-        uint32_t v[AHEAD + 1][RUN];
+        constexpr int RUN = 8, NB = PHASE == 2 ? 8 : 4, AHEAD = NB - 1;
+        uint32_t v[NB][RUN];
+        float4 ev[EL ? 1 : NB][2];
+        const int ng = nt >> 2;
         const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)a.vc, 0, (uint32_t)a.seq * (uint32_t)a.kv_dim * 2u, 0x00020000);
         const int vcol = (kvh * HD + dg * 32 + 2 * n) * 2, vrow = a.kv_dim * 2;
-        auto fetch = [&](uint32_t (&d)[RUN], int t, int k0) {
-            const int off = (((t + c) << 5) % a.seq) * vrow + vcol;
+        auto fetch = [&](int buf, int g, int i) {
+            g = g < ng ? g : ng - 1;
+            const int off = (((tfirst + 4 * g + c) << 5) % a.seq) * vrow + vcol;
             #pragma unroll
-            for (int k = 0; k < RUN; ++k) d[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rv, off, (k0 + k) * vrow, 0);
+            for (int k = 0; k < RUN; ++k) v[buf][k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rv, off, (RUN * i + k) * vrow, 0);
+            if constexpr (!EL) {
+                const float *et = eb + ((size_t)(4 * g + c) * 16 + n) * ES + RUN * i;
+                ev[buf][0] = *(const float4 *)et; ev[buf][1] = *(const float4 *)(et + 4);
+            }
         };
         #pragma unroll
-        for (int i = 0; i < AHEAD; ++i) fetch(v[i], tfirst, RUN * i);
-        for (int t = 0; t < nt; t += 4) {
-            const float *et = eb + (size_t)(t + c) * 16 * ES + n * ES;
-            lg_v16f acc0 = {}, acc1 = {};
+        for (int i = 0; i < AHEAD; ++i) fetch(i, i >> 2, i & 3);
+        for (int g0 = 0; g0 < ng; g0 += NB / 4) {
             #pragma unroll
-            for (int i = 0; i < 4; ++i) {                     // (four runs per tile: AHEAD + 1 buffers in turn)
-                if (i == 0) fetch(v[3], tfirst + t, 24);
-                else fetch(v[i - 1], tfirst + (t + 4 < nt ? t + 4 : t), RUN * (i - 1));
-                const float4 ea = *(const float4 *)(et + RUN * i), ec = *(const float4 *)(et + RUN * i + 4);
-                const float e[8] = { ea.x, ea.y, ea.z, ea.w, ec.x, ec.y, ec.z, ec.w };
-                if (t == 0 || t + 4 >= nt) {                  // rows that no row of the group sees may hold anything (infinities too)
-                    const int p = ((tfirst + t + c) << 5) + RUN * i;
+            for (int h = 0; h < NB / 4; ++h) {
+                const int g = g0 + h, t = 4 * g;
+                if (g >= ng) break;
+                float4 w4[4], l4[4];
+                auto tile_weights = [&]() {
                     #pragma unroll
-                    for (int k = 0; k < RUN; ++k) if (p + k < kfirst || p + k > klast) v[i][k] = 0;
-                }
-                #pragma unroll
-                for (int k = 0; k < RUN; ++k) {
-                    acc0 = __builtin_amdgcn_mfma_f32_16x16x1f32(e[k], lg_h2f((uint16_t)(v[i][k] & 0xFFFF)), acc0, 0, 0, 0);
-                    acc1 = __builtin_amdgcn_mfma_f32_16x16x1f32(e[k], lg_h2f((uint16_t)(v[i][k] >> 16)), acc1, 0, 0, 0);
-                }
-            }
-            #pragma unroll
-            for (int b = 0; b < 4; ++b) {                     // tiles in order
-                const float4 w = *(const float4 *)(mb + (t + b) * 16 + 4 * c), l = *(const float4 *)(lb + (t + b) * 16 + 4 * c);
-                const float wv[4] = { w.x, w.y, w.z, w.w }, lv[4] = { l.x, l.y, l.z, l.w };
+                    for (int b = 0; b < 4; ++b) { w4[b] = *(const float4 *)(wb + (t + b) * 16 + 4 * c); l4[b] = *(const float4 *)(lb + (t + b) * 16 + 4 * c); }
+                };
+                if constexpr (!EL) tile_weights();
+                lg_v16f acc0 = {}, acc1 = {};
                 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    L[i] = lg_fmaf(lv[i], wv[i], L[i]);
-                    o[0][i] = lg_fmaf(acc0[4 * b + i], wv[i], o[0][i]);
-                    o[1][i] = lg_fmaf(acc1[4 * b + i], wv[i], o[1][i]);
+                    const int cur = 4 * h + i;
+                    fetch((cur + AHEAD) % NB, g + ((i + AHEAD) >> 2), (i + AHEAD) & 3);
+                    const float *et = eb + ((size_t)(t + c) * 16 + n) * ES + RUN * i;
+                    const float4 ea = EL ? *(const float4 *)et : ev[EL ? 0 : cur][0], ec = EL ? *(const float4 *)(et + 4) : ev[EL ? 0 : cur][1];
+                    const float e[8] = { ea.x, ea.y, ea.z, ea.w, ec.x, ec.y, ec.z, ec.w };
+                    if (g == 0 || g + 1 == ng) {              // rows that no row of the group sees may hold anything (infinities too)
+                        const int p = ((tfirst + t + c) << 5) + RUN * i;
+                        #pragma unroll
+                        for (int k = 0; k < RUN; ++k) if (p + k < kfirst || p + k > klast) v[cur][k] = 0;
+                    }
+                    #pragma unroll
+                    for (int k = 0; k < RUN; ++k) {
+                        acc0 = __builtin_amdgcn_mfma_f32_16x16x1f32(e[k], lg_h2f((uint16_t)(v[cur][k] & 0xFFFF)), acc0, 0, 0, 0);
+                        acc1 = __builtin_amdgcn_mfma_f32_16x16x1f32(e[k], lg_h2f((uint16_t)(v[cur][k] >> 16)), acc1, 0, 0, 0);
+                    }
+                }
+                if constexpr (EL) tile_weights();
+                #pragma unroll
+                for (int b = 0; b < 4; ++b) {                 // tiles in order
+                    const float wv[4] = { w4[b].x, w4[b].y, w4[b].z, w4[b].w }, lv[4] = { l4[b].x, l4[b].y, l4[b].z, l4[b].w };
+                    #pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        L[i] = lg_fmaf(lv[i], wv[i], L[i]);
+                        o[0][i] = lg_fmaf(acc0[4 * b + i], wv[i], o[0][i]);
+                        o[1][i] = lg_fmaf(acc1[4 * b + i], wv[i], o[1][i]);
+                    }
                 }
             }
         }
@@ -633,8 +665,8 @@ __global__ __launch_bounds__(LG_WA_WG, 2) void lg_k_wide_attn(WideAttn a, const 
         for (int i = 0; i < 4; ++i) *(float2 *)(&ob[4 * c + i][dg * 32 + 2 * n]) = make_float2(o[0][i] / L[i], o[1][i] / L[i]);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < 16 * (HD / 4); i += LG_WA_WG) {
-        const int u = i / (HD / 4), qd = i - u * (HD / 4), r = row0 + u / G;
+    for (int i = threadIdx.x; i < 16 * 8 * ndg; i += WG) {
+        const int u = i / (8 * ndg), qd = 8 * dg0 + i - u * (8 * ndg), r = row0 + u / G;
         if (u >= U || r > rlast) continue;                   // (whole groups of 8 lanes)
         lg_wide_quant4(*(const float4 *)(&ob[u][qd * 4]), a.xq, a.H * HD >> 5, r, (kvh * G + u - u / G * G) * (HD / 32) + (qd >> 3));
     }

@@ -88,3 +88,35 @@ def test_long_cache_of_a_model_for_single_rows(lg, ob, gpu_required, model_path)
         assert all(np.array_equal(a, b) for a, b in zip(*got))
     finally:
         gpu.close()
+
+
+@pytest.mark.parametrize("name,pos0,n,over", [("tiny", 351, 9, {}), ("tiny", 352, 33, {"sliding_window": 512}), ("tiny_full", 1500, 40, {}), ("tiny", 3000, 22, {"head_dim": 256, "sliding_window": 1024}),
+                                              ("tiny", 700, 250, {"head_dim_full": 512}), ("tiny", 701, 61, {"n_head": 12, "n_head_kv": 4, "sliding_window": 512}),
+                                              ("tiny", 1471, 260, {}), ("tiny", 32735, 24, {}), ("tiny", 32760, 24, {})])
+def test_few_rows_late_in_a_context(lg, ob, gpu_required, model_path, name, pos0, n, over):
+    """Scores and values as two kernels: from 12 tiles on, heads of 64 to 512 dims, windows and whole contexts, three heads per
+    kv head, on both sides of the rows (128 workgroups) and the tiles (1024) up to which they are used.  Against the same
+    rows through verify blocks, bit for bit; the cache rows in front are drawn."""
+    path, spec = model_path(name, **over)
+    rng = np.random.default_rng(pos0 + n)
+    prompt = rng.integers(1, spec["n_vocab"], n).astype(np.int32)
+    owners = spec["n_layer"] - spec["shared_kv_layers"]
+    gpu = lg.hiplib.HipBackend(path, pos0 + n + 2, max_rows=8)
+    try:
+        front = {}
+        for L in range(owners):
+            rows, width = gpu.kv_layout(L)
+            front[L] = rng.normal(0, 0.5, (2, rows, width)).astype(np.float16).view(np.uint16)
+        got = []
+        for wide in (1, 0):
+            gpu.new_cache()
+            gpu.set_option("wide_prefill", wide)
+            for L in front:
+                for which in (0, 1):
+                    gpu.kv_write(L, which, front[L][which])
+            print(f"{name} {over}: {n} positions at {pos0}, wide {wide}", flush=True)
+            gpu.prefill(prompt, pos0)
+            got.append([gpu.kv_read(L, w) for L in range(owners) for w in (0, 1)] + [gpu.forward(5, pos0 + n, spec["n_vocab"]).view(np.uint32)])
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
+    finally:
+        gpu.close()
