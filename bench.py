@@ -454,8 +454,7 @@ def main():
                             "draft_ms_per_step": 1e3 * t_draft / a.mtp_steps, "verify_ms_per_step": 1e3 * t_verify / a.mtp_steps,
                             "ms_per_step": 1e3 * (t_draft + t_verify) / a.mtp_steps, "tokens_per_step": emitted / a.mtp_steps,
                             "head": "synthetic gemma4-assistant (4 blocks, 256 wide), host round trip per draft"}
-    # prompt processing on the matrix cores: 32-row blocks through the int8 MFMA kernels (a fresh cache, host clock
-    # around a synchronised call; the first call captures the graph and is not timed)
+    # prompt processing on the matrix cores, blocks of up to 512 rows (a fresh cache, host clock around a synchronised call)
     if a.prefill > 0:
         prng = np.random.default_rng(a.seed + 1)
         ptoks = prng.integers(1, info["n_vocab"], a.prefill).astype(np.int32)
@@ -467,7 +466,7 @@ def main():
         dt = time.time() - t0
         macs = sum(c["bytes"] for c in prof if c["name"] != "lm_head" and c["name"] != "attn_tiles") / (18.0 / 32.0)   # weights touched per position
         line["prefill"] = {"positions": int(a.prefill), "ms": 1e3 * dt, "tok_per_s": a.prefill / dt,
-                           "kernel": "v_mfma_i32_32x32x32_i8, 512-row blocks", "int8_TOPs": 2.0 * macs * a.prefill / dt / 1e12,
+                           "kernel": "v_mfma_scale_f32_32x32x64_f8f6f4, 512-row blocks", "int8_TOPs": 2.0 * macs * a.prefill / dt / 1e12,
                            "mfma_peak_TOPs": 5000.0, "mfma_utilisation": 2.0 * macs * a.prefill / dt / 5.0e15}
     gpu.close()
     try:
