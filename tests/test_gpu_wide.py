@@ -1,10 +1,13 @@
 """The kernels of prompt blocks (lg_wide.h) at the sizes where they can go wrong: every workgroup shape of the matmul, weight
 rows that are no multiple of its 64-row tile, ragged activation rows, and prompts of every remainder through blocks of
 their own width, against the oracle bit for bit."""
+import os
+import shutil
+
 import numpy as np
 import pytest
 
-from conftest import random_q4_0
+from conftest import gguf_tensor_span, random_q4_0
 from test_gpu_kernels import oracle_matmul
 from test_gpu_prefill import check_wide_prefill
 
@@ -118,5 +121,79 @@ def test_few_rows_late_in_a_context(lg, ob, gpu_required, model_path, name, pos0
             gpu.prefill(prompt, pos0)
             got.append([gpu.kv_read(L, w) for L in range(owners) for w in (0, 1)] + [gpu.forward(5, pos0 + n, spec["n_vocab"]).view(np.uint32)])
         assert all(np.array_equal(a, b) for a, b in zip(*got))
+    finally:
+        gpu.close()
+
+
+def nan_rows(a):
+    """binary16 bit patterns with every NaN as one pattern (which NaN comes out of a sum is not defined)."""
+    return np.where((a & 0x7FFF) > 0x7C00, 0x7E00, a)
+
+
+@pytest.mark.parametrize("name,pos0,n,over", [("tiny", 301, 45, {}), ("tiny_full", 301, 33, {}), ("tiny", 400, 61, {"head_dim": 256}), ("tiny", 301, 37, {"n_head": 12, "n_head_kv": 4}),
+                                              ("tiny", 701, 61, {"sliding_window": 512}), ("tiny", 1700, 300, {"sliding_window": 1536})])
+def test_an_infinity_reaches_only_rows_that_see_it(lg, ob, gpu_required, model_path, name, pos0, n, over):
+    """Value rows of infinities and NaN at the start of a window, seen by the prompt's first two rows and by none after them (rows
+    that share a workgroup's products): the next layer's cache rows of the others keep their bits, and those of the two are what
+    verify blocks make of them.  With all weights in LDS, in memory, and as two kernels; three heads per kv head."""
+    path, spec = model_path(name, **over)
+    rng = np.random.default_rng(pos0 + n)
+    prompt = rng.integers(1, spec["n_vocab"], n).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, pos0 + n + 2, max_rows=8)
+    try:
+        front = {}
+        for L in (0, 1):
+            rows, width = gpu.kv_layout(L)
+            front[L] = rng.normal(0, 0.5, (2, rows, width)).astype(np.float16).view(np.uint16)
+        at = (pos0 + 2 - spec["sliding_window"]) % front[0].shape[1]
+        odd = front[0][1].copy()
+        odd[at, 0::5], odd[at, 1::5], odd[at, 7::5] = 0x7C00, 0xFC00, 0x7E00
+        got = {}
+        for wide, v0 in ((1, front[0][1]), (1, odd), (0, odd)):
+            gpu.new_cache()
+            gpu.set_option("wide_prefill", wide)
+            for L in front:
+                gpu.kv_write(L, 0, front[L][0])
+                gpu.kv_write(L, 1, v0 if L == 0 else front[L][1])
+            print(f"{name} {over}: {n} positions at {pos0}, wide {wide}, infinities {v0 is odd}", flush=True)
+            gpu.prefill(prompt, pos0)
+            ring = gpu.kv_layout(1)[0]
+            got[wide, v0 is odd] = [gpu.kv_read(1, w)[np.arange(pos0, pos0 + n) % ring] for w in (0, 1)]
+        for plain, wide, narrow in zip(got[1, False], got[1, True], got[0, True]):
+            assert np.array_equal(wide[2:], plain[2:])
+            assert np.array_equal(nan_rows(wide), nan_rows(narrow)) and ((wide[:2] & 0x7FFF) > 0x7C00).all()
+    finally:
+        gpu.close()
+
+
+@pytest.mark.parametrize("name,n,j,over", [("tiny", 45, 18, {}), ("tiny_full", 33, 10, {}), ("tiny", 130, 34, {"head_dim_full": 512}), ("tiny", 37, 13, {"n_head": 12, "n_head_kv": 4})])
+def test_a_row_of_nan_reaches_no_row_before_it(lg, ob, gpu_required, model_path, model_dir, name, n, j, over):
+    """A prompt token whose embedding is infinite: the cache rows of the positions in front of it, in every layer, are those of the
+    same prompt with another token there, and all of them those that verify blocks leave."""
+    src, spec = model_path(name, **over)
+    path = os.path.join(str(model_dir), os.path.basename(src) + ".odd")
+    shutil.copyfile(src, path)
+    off, nbytes, dims = gguf_tensor_span(path, "token_embd.weight")
+    odd = 77
+    with open(path, "r+b") as f:
+        for b in range(dims[0] // 32):
+            f.seek(off + odd * (nbytes // dims[1]) + b * 18)
+            f.write(b"\x00\x7c")                          # the block's scale: +inf
+    prompt = np.random.default_rng(n).integers(100, spec["n_vocab"], n).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, n + 2, max_rows=8)
+    try:
+        got = []
+        for wide, token in ((1, prompt[j]), (1, odd), (0, odd)):
+            gpu.new_cache()
+            gpu.set_option("wide_prefill", wide)
+            p = prompt.copy()
+            p[j] = token
+            print(f"{name} {over}: {n} positions, token {token} at {j}, wide {wide}", flush=True)
+            gpu.prefill(p, 0)
+            got.append([gpu.kv_read(L, w)[:n] for L in range(spec["n_layer"] - spec["shared_kv_layers"]) for w in (0, 1)])
+        for plain, wide, narrow in zip(*got):
+            assert np.array_equal(wide[:j], plain[:j])
+            assert np.array_equal(nan_rows(wide), nan_rows(narrow))
+        assert all(((a[j:] & 0x7FFF) > 0x7C00).all() for a in got[1][2:])
     finally:
         gpu.close()
