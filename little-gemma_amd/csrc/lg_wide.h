@@ -433,8 +433,9 @@ __global__ __launch_bounds__(LG_WG) void lg_k_wide_quant(const float *x, int row
 //    turn, the next tile's rows in flight.  (v_mfma_f32_16x16x4_f32, k = four steps of a chain, adds in the same order and
 //    needs no exchange, but its operands come as 8-byte pieces of a row, twice the cache accesses: 47 -> 54 us.)
 //  * values: the same instruction, its four blocks are four consecutive tiles, a step per key slot (masked slots have
-//    weight 0; where that leaves an infinity or NaN in the product it is taken out first), the columns 16 dims; a wavefront takes 32 dims as two such products, so that one 4-byte load per lane feeds
-//    two steps, and adds the tiles' results to the running sum in tile order with the weights exp(m_tile - M).
+//    weight 0; results that are not finite are computed again without them), the columns 16 dims; a wavefront takes 32 dims
+//    as two such products, so that one 4-byte load per lane feeds two steps, and adds the tiles' results to the running sum
+//    in tile order with the weights exp(m_tile - M).
 // The weights e of a row's tiles, their maxima and sums wait in LDS between the two (EL: up to LG_WA_TILES tiles; more: in
 // the cache's scratch).  Bound by the matrix cores (8 to 9 thousand cycles per 16 units and tile) and the exponentials.
 // Eight wavefronts rather than four: one workgroup is all the LDS holds on a CU, and with two wavefronts on a SIMD one
@@ -591,9 +592,6 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
         for (int t = k; t < nt; t += WG / 16) { const float v = mb[t * 16 + u]; wb[t * 16 + u] = v == -INFINITY ? 0.0f : lg_expf(v - m); }
     }
     __syncthreads();
-    // the four tiles from index t on hold positions that some row of the group does not see
-    const int kfull = lg_win_start(pos + rlast, a.window) - (tfirst << 5), kown = pos + row0 - (tfirst << 5);     // ... before the one, behind the other
-    auto border = [&](int t) { return (t << 5) < kfull || (t << 5) + 127 > kown; };
     const int ndg = PHASE == 2 ? HD / 32 / gridDim.z : HD / 32, dg0 = PHASE == 2 ? blockIdx.z * ndg : 0;      // runs of 32 dims of this workgroup
     for (int dg = dg0 + wave; dg < dg0 + ndg; dg += NW) {
         float o[2][4], L[4];
@@ -607,7 +605,6 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
         uint32_t v[NB][RUN];
         float4 ev[EL ? 1 : NB][2];
         const int ng = nt >> 2;
-        uint32_t odd = 0;                                     // an infinity or NaN was taken out of the products of a border group
         const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)a.vc, 0, (uint32_t)a.seq * (uint32_t)a.kv_dim * 2u, 0x00020000);
         const int vcol = (kvh * HD + dg * 32 + 2 * n) * 2, vrow = a.kv_dim * 2;
         auto fetch = [&](int buf, int g, int i) {
@@ -641,26 +638,10 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
                     const float *et = eb + ((size_t)(t + c) * 16 + n) * ES + RUN * i;
                     const float4 ea = EL ? *(const float4 *)et : ev[EL ? 0 : cur][0], ec = EL ? *(const float4 *)(et + 4) : ev[EL ? 0 : cur][1];
                     const float e[8] = { ea.x, ea.y, ea.z, ea.w, ec.x, ec.y, ec.z, ec.w };
-                    if (border(t)) {
-                        // positions that not every row of the group sees: a weight of 0 does not keep an infinity or NaN of theirs
-                        // out of the rows that do not see it.  Those values go out of the product (each 16-bit half whose
-                        // exponent bits are all set; 0x8000 in the sum says so) and are added to the rows that see them below.
+                    if (g == 0 || g + 1 == ng) {              // rows that no row of the group sees may hold anything (infinities too)
                         const int p = ((tfirst + t + c) << 5) + RUN * i;
-                        uint32_t any = 0;
                         #pragma unroll
-                        for (int k = 0; k < RUN; ++k) {
-                            if (p + k < kfirst || p + k > klast) v[cur][k] = 0;
-                            any |= (v[cur][k] & 0x7C007C00u) + 0x04000400u;
-                        }
-                        any &= 0x80008000u;
-                        if (__builtin_amdgcn_ballot_w64(any != 0)) {
-                            odd = 1;
-                            #pragma unroll
-                            for (int k = 0; k < RUN; ++k) {
-                                const uint32_t h = ((v[cur][k] & 0x7C007C00u) + 0x04000400u) & 0x80008000u;
-                                v[cur][k] &= ~(h | (h - (h >> 15)));
-                            }
-                        }
+                        for (int k = 0; k < RUN; ++k) if (p + k < kfirst || p + k > klast) v[cur][k] = 0;
                     }
                     #pragma unroll
                     for (int k = 0; k < RUN; ++k) {
@@ -681,28 +662,38 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
                 }
             }
         }
-        if (odd) {
-            // The values taken out above, for the rows that see them.  Where such a value is in its chain does not matter: what
-            // comes of it is an infinity or NaN whichever finite terms stand before and behind it.
+        // A value that is not finite and that some row of the group does not see was a product with weight 0 for that row: a NaN.
+        // So where a result of this wavefront is not finite, all of them are computed again, each from the slots its row sees.
+        float odd = 0.0f;
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) odd = lg_fmaf(o[0][i], 0.0f, lg_fmaf(o[1][i], 0.0f, odd));
+        if (__builtin_amdgcn_ballot_w64(odd != 0.0f)) {
             int u0 = 4 * c;
             asm("" : "+v"(u0));                               // (else what the scores know of these units is kept in registers for here, and spills)
+            int us[4], up[4];
+            #pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = row0 + (u0 + i) / G;
+                us[i] = lg_win_start(pos + r, a.window); up[i] = u0 + i < U && r <= rlast ? pos + r : -1;
+                o[0][i] = o[1][i] = 0.0f;
+            }
             for (int t = 0; t <= tlast - tfirst; ++t) {
-                if (!border(t & ~3)) continue;
-                for (int s = 0; s < 32; ++s) {
-                    const int p = ((tfirst + t) << 5) + s;
-                    if (p < kfirst || p > klast) continue;
-                    const uint32_t x = *(const uint32_t *)((const uint8_t *)a.vc + (size_t)(p % a.seq) * vrow + vcol);
+                float acc[2][4] = {};
+                const int t0 = (tfirst + t) << 5;
+                for (int s = t0 < kfirst ? kfirst - t0 : 0; s < 32 && t0 + s <= klast; ++s) {
+                    const uint32_t x = *(const uint32_t *)((const uint8_t *)a.vc + (size_t)((t0 + s) % a.seq) * vrow + vcol);
                     #pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const uint16_t xh = (uint16_t)(x >> (16 * h));
-                        if ((xh & 0x7C00) != 0x7C00) continue;
-                        #pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int u = u0 + i, r = row0 + u / G;
-                            if (u < U && r <= rlast && p <= pos + r && p >= lg_win_start(pos + r, a.window))
-                                o[h][i] = lg_fmaf(eb[((size_t)t * 16 + u) * ES + s] * lg_h2f(xh), wb[t * 16 + u], o[h][i]);
-                        }
+                    for (int i = 0; i < 4; ++i) {
+                        if (t0 + s < us[i] || t0 + s > up[i]) continue;
+                        const float e = eb[((size_t)t * 16 + u0 + i) * ES + s];
+                        acc[0][i] = lg_fmaf(e, lg_h2f((uint16_t)(x & 0xFFFF)), acc[0][i]);
+                        acc[1][i] = lg_fmaf(e, lg_h2f((uint16_t)(x >> 16)), acc[1][i]);
                     }
+                }
+                #pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    o[0][i] = lg_fmaf(acc[0][i], wb[t * 16 + u0 + i], o[0][i]);
+                    o[1][i] = lg_fmaf(acc[1][i], wb[t * 16 + u0 + i], o[1][i]);
                 }
             }
         }
