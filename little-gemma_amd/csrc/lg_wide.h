@@ -35,11 +35,12 @@ typedef float lg_v32f __attribute__((ext_vector_type(32)));
 #define LG_WIDE_ROWS 512                   // rows of the widest block
 #define LG_WIDE_MID  128                   // the widest block of a short cache
 
-// 6-bit float code (sign, 3 exponent bits of bias 3, 2 mantissa bits) of an integer -8..8 given as a float
+// 6-bit float code (sign, 3 exponent bits of bias 3, 2 mantissa bits) of an integer -8..8 given as a float; of any other
+// value, six bits
 __device__ __forceinline__ uint32_t lg_e3m2(float v) {
     const uint32_t u = __float_as_uint(v);
     const int e = (int)((u & 0x7FFFFFFFu) >> 21) - (124 << 2);
-    return (uint32_t)(e > 0 ? e : 0) | ((u >> 26) & 0x20u);
+    return (uint32_t)(e < 0 ? 0 : e > 31 ? 31 : e) | ((u >> 26) & 0x20u);
 }
 // Where the digits of (row j, block b) of a wide activation buffer of nb blocks per row live: dword d (0..5) of the hi
 // (half = 0) or lo (half = 1) digits, and the row's scale.
@@ -59,11 +60,14 @@ __device__ __forceinline__ void lg_wide_quant4(float4 h, uint8_t *q, int nb, int
     amax = lg_max_n(amax, 8);
     const float d = lg_div127(amax);
     const float id = d > 0.0f ? 1.0f / d : 0.0f;
-    const float v[4] = { lg_rintf(h.x * id), lg_rintf(h.y * id), lg_rintf(h.z * id), lg_rintf(h.w * id) };
+    const float p[4] = { h.x * id, h.y * id, h.z * id, h.w * id };
     uint32_t hi = 0, lo = 0;
     #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const float fh = floorf((v[i] + 8.0f) * 0.0625f), fl = lg_fmaf(-16.0f, fh, v[i]);
+        // a NaN becomes 0, as in the conversion to int8, and the values next to it keep their digits (an infinity among the 32
+        // makes their scale a NaN, so that the block does not pass for finite)
+        const float v = p[i] == p[i] ? lg_rintf(p[i]) : 0.0f;
+        const float fh = floorf((v + 8.0f) * 0.0625f), fl = lg_fmaf(-16.0f, fh, v);
         hi |= lg_e3m2(fh) << (6 * i);
         lo |= lg_e3m2(fl) << (6 * i);
     }

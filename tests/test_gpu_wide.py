@@ -29,6 +29,29 @@ def test_wide_matmul_shapes(lg, ob, gpu_required, m, k, rows):
     assert np.array_equal(r["out"].view(np.uint32), out.view(np.uint32))
 
 
+@pytest.mark.parametrize("k", [256, 2560, 5120])
+def test_wide_q8_of_values_that_are_not_finite(lg, gpu_required, k):
+    """NaN and infinities in the activations: q8 values, scales and products of a wide block are those that blocks of 8 rows get.
+    (A NaN counts as 0 beside finite neighbours; an infinity makes its block's scale a NaN.)"""
+    rng = np.random.default_rng(k)
+    m = 64
+    w = random_q4_0(rng, m, k)
+    x = rng.normal(0, 1, (32, k)).astype(np.float32)
+    for j in range(24):                                   # NaN at every place of a lane's four values, in several lanes
+        x[j, 32 * (j % 8) + j] = np.nan
+    x[24, 7], x[25, 40], x[26, 100] = np.inf, -np.inf, np.nan
+    x[26, 101] = np.inf
+    x[27, 64:96] = np.nan
+    print(f"wide q8 of NaN k={k}", flush=True)
+    wide = lg.hiplib.matmul_q4q8(w, k, m, x)
+    parts = [lg.hiplib.matmul_q4q8(w, k, m, np.ascontiguousarray(x[j:j + 8])) for j in range(0, 32, 8)]
+    for key in ("xq", "xsum", "xd", "out"):
+        want = np.concatenate([p[key].reshape(8, -1) for p in parts])
+        got = wide[key].reshape(32, -1)
+        assert np.array_equal(got, want, equal_nan=key in ("xd", "out")), key
+    assert np.isfinite(wide["out"].reshape(32, m)[:24]).all() and np.isnan(wide["out"].reshape(32, m)[24:28]).all()
+
+
 @pytest.mark.parametrize("name,n_prompt,over", [("tiny_full", 9, {}), ("tiny_full", 31, {}), ("tiny", 33, {}), ("tiny_full", 65, {}), ("tiny", 129, {}),
                                                 ("tiny", 70, {"n_ff": 10240}), ("tiny_full", 30, {"n_ff": 10240}), ("tiny", 1303, {}),
                                                 ("tiny", 61, {"n_head": 12, "n_head_kv": 4}), ("tiny_full", 50, {"n_head_kv": 8}), ("tiny", 45, {"head_dim_full": 512})])
