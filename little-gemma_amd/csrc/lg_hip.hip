@@ -242,7 +242,7 @@ struct lg_hip_model {
     float *slabs = nullptr, *xact = nullptr; // [8][max_rows][E] partial sums of ffn_down; [8][max_rows][max FF/8] gelu(gate)*up per XCD
     uint32_t *xq8 = nullptr;                 // [8][E/32][80] q8 rows per XCD
     XcdSync *xsync = nullptr;
-    std::map<GraphKey, hipGraphExec_t> graphs;
+    std::map<GraphKey, hipGraphExec_t> graphs;           // null: launched as it is (capture_behind)
     Profile prof;
     // a draft head (src/mtp.c) is a model whose layers own no cache: they read `target`'s
     lg_hip_model *target = nullptr;
@@ -803,7 +803,7 @@ extern "C" void lg_hip_model_destroy(lg_hip_model *m) {
     if (!m) return;
     (void)hipSetDevice(m->device);
     (void)hipDeviceSynchronize();
-    for (auto &g : m->graphs) (void)hipGraphExecDestroy(g.second);
+    for (auto &g : m->graphs) if (g.second) (void)hipGraphExecDestroy(g.second);
     for (void *p : m->allocs) (void)hipFree(p);
     for (hipEvent_t e : m->prof.ev) (void)hipEventDestroy(e);
     if (m->pin) (void)hipHostFree(m->pin);
@@ -890,7 +890,7 @@ extern "C" void lg_hip_kv_destroy(lg_hip_kv *kv) {
     holders.push_back(kv->m);
     for (lg_hip_model *h : holders)
         for (auto it = h->graphs.begin(); it != h->graphs.end();) {
-            if (it->first[0] == (uint64_t)kv->id) { (void)hipGraphExecDestroy(it->second); it = h->graphs.erase(it); }
+            if (it->first[0] == (uint64_t)kv->id) { if (it->second) (void)hipGraphExecDestroy(it->second); it = h->graphs.erase(it); }
             else ++it;
         }
     for (size_t L = 0; L < kv->k.size(); ++L) {
@@ -1746,19 +1746,21 @@ static GraphKey graph_key(const lg_hip_model *m, const lg_hip_kv *kv, int rows, 
     return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices };
 }
 
-// What `enqueue` launches on the stream, as a graph.
+// What `enqueue` launches on the stream, as a graph for the calls to come.  The caller has just launched the same thing: it
+// ran, whether a graph of it can be made or not, so a failure here (no memory for the graph, say) is none of the call's.
+// Null then, and the calls to come launch it as it is.
 template <typename F>
-static int capture_graph(hipStream_t st, F enqueue, hipGraphExec_t *exec) {
+static hipGraphExec_t capture_behind(hipStream_t st, F enqueue) {
     hipGraph_t graph = nullptr;
-    HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    const int rc = enqueue();
-    hipError_t e = hipStreamEndCapture(st, &graph);
-    if (rc) { if (graph) (void)hipGraphDestroy(graph); return rc; }
-    if (e != hipSuccess) return fail(-100 - (int)e, "hipStreamEndCapture: %s", hipGetErrorString(e));
-    e = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    if (e != hipSuccess) return fail(-100 - (int)e, "hipGraphInstantiate: %s", hipGetErrorString(e));
-    return 0;
+    hipGraphExec_t exec = nullptr;
+    if (hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) == hipSuccess) {
+        const int rc = enqueue();
+        const hipError_t e = hipStreamEndCapture(st, &graph);
+        if (rc || e != hipSuccess || hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess) exec = nullptr;
+        if (graph) (void)hipGraphDestroy(graph);
+    }
+    if (!exec) (void)hipGetLastError();                       // (else the next launch would report it)
+    return exec;
 }
 
 // Launch one step, through a captured graph when enabled.  The first step of a (cache, width, options) runs as plain
@@ -1768,12 +1770,14 @@ static int launch_step(lg_hip_model *m, lg_hip_kv *kv, int rows, bool with_head)
     if (!m->use_graph || m->prof.on) return enqueue_step_rows(m, kv, rows, with_head);
     const GraphKey key = graph_key(m, kv, rows, with_head ? 1 : 0);
     auto it = m->graphs.find(key);
-    if (it != m->graphs.end()) { HIP_TRY(hipGraphLaunch(it->second, m->stream)); return 0; }
-    hipGraphExec_t exec = nullptr;
+    if (it != m->graphs.end()) {
+        if (!it->second) return enqueue_step_rows(m, kv, rows, with_head);
+        HIP_TRY(hipGraphLaunch(it->second, m->stream));
+        return 0;
+    }
     int rc = enqueue_step_rows(m, kv, rows, with_head, true);
     if (!rc) rc = enqueue_step_rows(m, kv, rows, with_head);
-    if (!rc) rc = capture_graph(m->stream, [&]() { return enqueue_step_rows(m, kv, rows, with_head); }, &exec);
-    if (!rc) m->graphs.emplace(key, exec);
+    if (!rc) m->graphs.emplace(key, capture_behind(m->stream, [&]() { return enqueue_step_rows(m, kv, rows, with_head); }));
     return rc;
 }
 
@@ -1944,13 +1948,14 @@ extern "C" int lg_hip_mtp_rounds(lg_hip_model *d, lg_hip_kv *kv, int token, int 
         auto it = d->graphs.find(key);            // kept by the head: the graph dies with it or with the cache
         int r = 0;
         if (it == d->graphs.end()) {               // the first round as launches, its graph while the device works on it
-            hipGraphExec_t exec = nullptr;
-            if ((rc = enqueue_round(d, kv, rows, true)) || (rc = enqueue_round(d, kv, rows, false)) ||
-                (rc = capture_graph(t->stream, [&]() { return enqueue_round(d, kv, rows, false); }, &exec))) return rc;
-            it = d->graphs.emplace(key, exec).first;
+            if ((rc = enqueue_round(d, kv, rows, true)) || (rc = enqueue_round(d, kv, rows, false))) return rc;
+            it = d->graphs.emplace(key, capture_behind(t->stream, [&]() { return enqueue_round(d, kv, rows, false); })).first;
             r = 1;
         }
-        for (; r < n_rounds; ++r) HIP_TRY(hipGraphLaunch(it->second, t->stream));
+        for (; r < n_rounds; ++r) {
+            if (it->second) HIP_TRY(hipGraphLaunch(it->second, t->stream));
+            else if ((rc = enqueue_round(d, kv, rows, false))) return rc;
+        }
     }
     const size_t nb = (size_t)n_rounds * rows;
     int32_t *res = t->pin + 64;

@@ -2,8 +2,11 @@
 src/cuda/model-cuda.cuh:703-720, src/cpu/model-cpu.c:477-478) and the sampling hook model_pick
 (include/model.h:105-111, src/cuda/mtp-kernel.cuh:103-118)."""
 import ctypes as C
+import json
 import os
 import shutil
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -243,3 +246,55 @@ def test_shared_tile_attention_prepares_its_own_rows(lg, ob, gpu_required, model
             assert np.array_equal(g[2].view(np.uint32), b[2].view(np.uint32)), opts
         for a, b in zip(cache, base_cache):
             assert np.array_equal(a, b), opts
+
+
+SESSION = """
+import ctypes, importlib, json, sys
+import numpy as np
+root, path, head, shim = sys.argv[1:]
+if shim:
+    ctypes.CDLL(shim, mode=ctypes.RTLD_GLOBAL)      # ahead of the runtime for every library loaded from here on
+sys.path.insert(0, root)
+lg = importlib.import_module("little-gemma_amd")
+gpu = lg.hiplib.HipBackend(path, 256, max_rows=4)
+t = gpu.mtp_open(head)
+gpu.prefill(np.arange(1, 31, dtype=np.int32), 0)
+res, tok, pos = [], 31, 30
+for _ in range(3):
+    adv, out = gpu.forward_spec(np.array([tok, 5, 6, 7], np.int32), pos)
+    pos, tok = pos + adv, int(out[adv - 1])
+    res.append([adv, out.tolist()])
+for _ in range(2):
+    blocks, out, adv, pos = gpu.mtp_rounds(t, tok, pos, 3, 3)
+    tok = int(out[-1, adv[-1] - 1])
+    res.append([blocks.tolist(), out.tolist(), adv.tolist(), pos])
+gpu.schedule(np.array([[tok, 1], [2, 3]], np.int32), pos)
+gpu.schedule_run(2)
+out, adv, pos = gpu.schedule_wait()
+res.append([out.tolist(), adv.tolist(), pos, gpu.mtp_draft(t, 9, pos), gpu.mtp_draft(t, 9, pos)])
+gpu.mtp_close(t)
+gpu.close()
+calls = ctypes.CDLL(shim).refused() if shim else 0
+print(json.dumps([calls, res]))
+"""
+
+
+def test_a_step_counts_though_no_graph_of_it_can_be_made(lg, gpu_required, model_path, model_dir):
+    """The first step of its kind runs as launches and its graph is made behind it.  In a process whose runtime refuses to make
+    one (a library in front of it answers hipGraphInstantiate with out of memory), steps, rounds, schedules and drafts give
+    what they give elsewhere: the step has run and the cache has moved, so its results must reach the caller."""
+    path, spec = model_path("tiny_full")
+    head = write_head(lg, model_dir, "tiny_full", spec)
+    src, shim = os.path.join(str(model_dir), "refuse.c"), os.path.join(str(model_dir), "librefuse.so")
+    with open(src, "w") as f:
+        f.write("static int n;\nint hipGraphInstantiate(void **e, void *g, void **m, char *b, unsigned long s) { (void)e; (void)g; (void)m; (void)b; (void)s; n++; return 2; }\n"
+                "int refused(void) { return n; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", shim, src], check=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    got = []
+    for s in ("", shim):
+        print(f"session {'without graphs' if s else 'with graphs'}", flush=True)
+        r = subprocess.run([sys.executable, "-c", SESSION, root, path, head, s], capture_output=True, text=True, timeout=100)
+        assert r.returncode == 0, r.stderr[-500:]
+        got.append(json.loads(r.stdout.splitlines()[-1]))
+    assert got[1][0] > 0 and got[1][1] == got[0][1]
