@@ -1614,13 +1614,29 @@ static int launch_wide_mm(Launcher &lx, int cls, const uint8_t *w, const int8_t 
     else                LAUNCH(cls, (lg_k_wide_mm<2, 4, DUMP>), grid, block, lds, a, out, dots);
     return parts;
 }
+// Whether a prompt block reaches value rows 2 GiB and more behind a layer's first one (524288 positions at the 12B shape), where
+// lg_k_wide_attn's 32-bit addresses end.  (It fetches value rows four tiles at a time.)
+static bool far_block(const lg_hip_kv *kv, const Layer &y, int rows, int pos) {
+    const long long reach = (long long)pos + rows + 127;
+    return (size_t)(reach < kv->seq[y.src] ? reach : kv->seq[y.src]) * y.kd * 2 >= (size_t)1 << 31;
+}
+// Such a block runs as verify blocks when it has heads of up to 256 there: their attention serves a tile to all rows (96 rows at
+// 524288 positions, 16 heads of 256 over 8: 34 ms against 104; 512-wide heads have no such kernel: 376 against 142, 16 over 2).
+static bool far_in_narrow_heads(const lg_hip_model *m, const lg_hip_kv *kv, int rows, int pos) {
+    for (const Layer &y : m->L) if (y.hd < 512 && far_block(kv, y, rows, pos)) return true;
+    return false;
+}
 // Up to 128 workgroups (half of the chip) with 12 tiles and more: scores and values as two launches over more workgroups (200
 // rows, 100 workgroups: 41 -> 39 us in a 512-wide window, 175 -> 113 us over 100 tiles; with 130 workgroups 42 -> 55 us, with 8
 // tiles 23 us both ways).  Score workgroups take 4 tiles, or up to 16 while there are more than 512 of them.
+// `far`: the block reaches value rows 2 GiB and more behind a layer's first one and takes 64-bit addresses (96 rows, 16 heads of 512
+// over 2, a million positions: 140.9 -> 141.7 ms).  Built for heads of 512; narrower ones go to verify blocks there (far_in_narrow_heads).
 template <int HD>
-static void launch_wide_attn(Launcher &lx, const WideAttn &a, int groups, size_t scratch_bytes) {
+static void launch_wide_attn(Launcher &lx, const WideAttn &a, int groups, bool far, size_t scratch_bytes) {
     const dim3 grid(groups, a.nkv);
     const int wgs = groups * a.nkv;
+    if constexpr (HD == 512)
+        if (far) { LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false, 0, true>), grid, dim3(LG_WA_WG), 0, a, lx.m->ctl); return; }
     if (wgs <= 128 && a.tiles >= 12 && a.tiles <= LG_WA_SPLIT_MAX && (size_t)wgs * a.tiles * (16 * 34 * 4) <= scratch_bytes) {
         int chunk = 4;
         while (chunk < 16 && wgs * (a.tiles / chunk) > 512) chunk *= 2;
@@ -1679,11 +1695,12 @@ static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, i
         const int rg = lg_wide_attn_rows(H / y.nkv), groups = (rows + rg - 1) / rg;
         const WideAttn a{ m->q_rot, kv->k[y.src], kv->v[y.src], H, y.nkv, kv->seq[y.src], y.kd, window, rows, kv->pacc,
                           wide_attn_tiles(m, y, rows, pos), (uint8_t *)m->aq };
+        const bool far = far_block(kv, y, rows, pos);
         switch (y.hd) {
-            case 512: launch_wide_attn<512>(lx, a, groups, kv->scratch_bytes); break;
-            case 256: launch_wide_attn<256>(lx, a, groups, kv->scratch_bytes); break;
-            case 128: launch_wide_attn<128>(lx, a, groups, kv->scratch_bytes); break;
-            default:  launch_wide_attn<64>(lx, a, groups, kv->scratch_bytes);
+            case 512: launch_wide_attn<512>(lx, a, groups, far, kv->scratch_bytes); break;
+            case 256: launch_wide_attn<256>(lx, a, groups, far, kv->scratch_bytes); break;
+            case 128: launch_wide_attn<128>(lx, a, groups, far, kv->scratch_bytes); break;
+            default:  launch_wide_attn<64>(lx, a, groups, far, kv->scratch_bytes);
         }
         pend_parts = launch_wide_mm<false>(lx, KC_O, y.wo_w, m->aq, y.qd, E, rows, m->dout, nullptr);
         pend_dout = m->dout; pend_w = y.post_attn;
@@ -1986,7 +2003,8 @@ extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *tok
     for (int i = 0; i < n; ++i) if (toks[i] < 0 || toks[i] >= m->n_vocab) return fail(-2, "token id %d outside the vocabulary of %d", toks[i], m->n_vocab);
     HIP_TRY(hipSetDevice(m->device));
     bool wide_ok = !m->target && m->wide_prefill;
-    for (size_t L = 0; L < kv->seq.size(); ++L) wide_ok = wide_ok && (size_t)kv->seq[L] * kv->kv_dim[L] * 2 < ((size_t)1 << 31);   // (the prompt kernels address a layer's cache with 32 bits)
+    // (attention that keeps its weights in LDS addresses a layer's cache with 32 bits, and reaches no row past LG_WIDE_ROWS + 32 (LG_WA_TILES + 4))
+    for (size_t L = 0; L < kv->seq.size(); ++L) wide_ok = wide_ok && (size_t)(LG_WIDE_ROWS + 32 * (LG_WA_TILES + 4)) * kv->kv_dim[L] * 2 < (size_t)1 << 31;
     const int cap = m->sched_cap * LG_HIP_MAX_ROWS;        // tokens the staging holds
     for (int at = 0; at < n;) {
         // the tokens go over once, the blocks follow each other on the stream and the host waits at the end
@@ -1996,12 +2014,13 @@ extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *tok
         for (int done = 0; done < part;) {
             const int left = part - done;
             int rows = left < kv->prompt_rows ? left : kv->prompt_rows, rc;
-            if (wide_ok && left > m->max_rows) rc = enqueue_prompt(m, kv, m->sched + done, rows, pos0 + at + done);
+            const bool wide = wide_ok && !far_in_narrow_heads(m, kv, rows, pos0 + at + done);
+            if (wide && left > m->max_rows) rc = enqueue_prompt(m, kv, m->sched + done, rows, pos0 + at + done);
             else {                                           // a remainder that fits a verify block
                 rows = left < m->max_rows ? left : m->max_rows;
                 if (done) HIP_TRY(hipMemcpyAsync(m->sched, m->pin + 64 + done, (size_t)rows * 4, hipMemcpyHostToDevice, m->stream));   // (its kernels read the schedule from its start)
                 hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, m->stream, m->ctl, pos0 + at + done);
-                rc = wide_ok ? enqueue_step_rows(m, kv, rows, false) : launch_step(m, kv, rows, false);    // (a single one: not worth a capture)
+                rc = wide ? enqueue_step_rows(m, kv, rows, false) : launch_step(m, kv, rows, false);    // (a single one: not worth a capture)
             }
             if (rc) return rc;
             done += rows;

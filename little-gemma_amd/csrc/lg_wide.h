@@ -476,7 +476,7 @@ __device__ __forceinline__ void lg_deal4(uint32_t x0, uint32_t x1, uint32_t x2, 
     const lg_u2 x = __builtin_amdgcn_permlane16_swap(p.x, q.x, false, false), y = __builtin_amdgcn_permlane16_swap(p.y, q.y, false, false);
     o[0] = x.x; o[1] = x.y; o[2] = y.x; o[3] = y.y;
 }
-template <int HD, bool EL, int PHASE = 0>
+template <int HD, bool EL, int PHASE = 0, bool FAR = false>
 __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wide_attn(WideAttn a, const StepCtl *ctl) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int WG = PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, NW = WG / 64;
@@ -605,17 +605,28 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
         // come from memory too): requested AHEAD runs ahead, a group of four tiles is four runs.
         // Buffer loads: the tile's place in the lane offset, the slot's in a scalar register (as flat loads their 64-bit
         // addresses cost more vector instructions than the conversions); the buffer ends with the ring, slots past it read 0.
+        // FAR: flat loads, for blocks that reach 2 GiB and more into a layer's value rows.
         constexpr int RUN = 8, NB = PHASE == 2 ? 8 : 4, AHEAD = NB - 1;
         uint32_t v[NB][RUN];
         float4 ev[EL ? 1 : NB][2];
         const int ng = nt >> 2;
-        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)a.vc, 0, (uint32_t)a.seq * (uint32_t)a.kv_dim * 2u, 0x00020000);
+        const uint64_t vbytes = (uint64_t)a.seq * a.kv_dim * 2;
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)a.vc, 0, (uint32_t)(vbytes < 0x7FFFFFFFu ? vbytes : 0x7FFFFFFFu), 0x00020000);
         const int vcol = (kvh * HD + dg * 32 + 2 * n) * 2, vrow = a.kv_dim * 2;
         auto fetch = [&](int buf, int g, int i) {
             g = g < ng ? g : ng - 1;
-            const int off = (((tfirst + 4 * g + c) << 5) % a.seq) * vrow + vcol;
-            #pragma unroll
-            for (int k = 0; k < RUN; ++k) v[buf][k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rv, off, (RUN * i + k) * vrow, 0);
+            const int ring0 = ((tfirst + 4 * g + c) << 5) % a.seq;
+            if constexpr (FAR) {
+                #pragma unroll
+                for (int k = 0; k < RUN; ++k) {
+                    const int r = ring0 + RUN * i + k < a.seq ? ring0 + RUN * i + k : a.seq - 1;       // (a slot past the ring is no position of the group: zeroed below)
+                    v[buf][k] = *(const uint32_t *)((const uint8_t *)a.vc + (size_t)r * vrow + vcol);
+                }
+            } else {
+                const int off = ring0 * vrow + vcol;
+                #pragma unroll
+                for (int k = 0; k < RUN; ++k) v[buf][k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rv, off, (RUN * i + k) * vrow, 0);
+            }
             if constexpr (!EL) {
                 const float *et = eb + ((size_t)(4 * g + c) * 16 + n) * ES + RUN * i;
                 ev[buf][0] = *(const float4 *)et; ev[buf][1] = *(const float4 *)(et + 4);

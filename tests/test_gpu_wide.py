@@ -3,6 +3,7 @@ rows that are no multiple of its 64-row tile, ragged activation rows, and prompt
 their own width, against the oracle bit for bit."""
 import os
 import shutil
+import time
 
 import numpy as np
 import pytest
@@ -218,5 +219,47 @@ def test_a_row_of_nan_reaches_no_row_before_it(lg, ob, gpu_required, model_path,
             assert np.array_equal(wide[:j], plain[:j])
             assert np.array_equal(nan_rows(wide), nan_rows(narrow))
         assert all(((a[j:] & 0x7FFF) > 0x7C00).all() for a in got[1][2:])
+    finally:
+        gpu.close()
+
+
+@pytest.mark.parametrize("hd", [512, 64])
+def test_prompt_blocks_on_a_cache_of_two_gibibytes_a_layer(lg, gpu_required, model_path, hd):
+    """Caches whose value rows pass 2 GiB per layer (524288 positions at the 12B shape; here rows of 8 and 2 KiB): a prompt across
+    that offset leaves the cache rows that verify blocks leave (heads of 512: by 64-bit addresses; of 64: as such blocks), and one at the start of the cache still runs in prompt blocks
+    (20 times fewer launches per token than 8-row blocks: half their time is far off)."""
+    heads = 8 if hd == 512 else 16
+    path, spec = model_path("tiny", n_head=heads, n_head_kv=heads, head_dim=hd, n_layer=2)
+    limit = (1 << 31) // (heads * hd * 2)                 # positions whose value rows fit 2 GiB
+    n = 90
+    pos0 = limit - 50
+    rng = np.random.default_rng(hd)
+    prompt = rng.integers(1, spec["n_vocab"], 480).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, limit + 300, max_rows=8)
+    try:
+        width = gpu.kv_layout(1)[1]
+        front = rng.normal(0, 0.5, (2, 700, width)).astype(np.float16).view(np.uint16)
+        got, took = [], []
+        for wide in (1, 0):
+            gpu.new_cache()
+            gpu.set_option("wide_prefill", wide)
+            for which in (0, 1):
+                gpu.kv_write(1, which, front[which], pos0 - 700)
+            print(f"{n} positions at {pos0}, heads of {hd}, wide {wide}", flush=True)
+            gpu.prefill(prompt[:n], pos0)
+            rows = [np.zeros((n, width), np.uint16) for _ in (0, 1)]
+            for which in (0, 1):
+                lg.hiplib.hip_check(gpu.H.lg_hip_kv_read(gpu.dkv, 1, which, pos0, n, rows[which]), "kv_read")
+            hidden = gpu.forward(5, pos0 + n, spec["n_vocab"])
+            got.append(rows + [hidden.view(np.uint32)])
+            gpu.prefill(prompt, 0)
+            t = []
+            for _ in range(5):
+                t0 = time.perf_counter()
+                gpu.prefill(prompt, 0)
+                t.append(time.perf_counter() - t0)
+            took.append(min(t))
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
+        assert took[0] < 0.5 * took[1], took
     finally:
         gpu.close()
