@@ -298,3 +298,66 @@ def test_a_step_counts_though_no_graph_of_it_can_be_made(lg, gpu_required, model
         assert r.returncode == 0, r.stderr[-500:]
         got.append(json.loads(r.stdout.splitlines()[-1]))
     assert got[1][0] > 0 and got[1][1] == got[0][1]
+
+
+def test_logits_rows_in_any_order(lg, gpu_required, model_path, model_dir):
+    """Rows are fetched when they are asked for, the next one ahead of time for a caller that takes them in turn: in order,
+    backwards, twice, with gaps, of the step before the last none; after blocks, schedules and drafts.  Each row against the
+    same token decoded alone."""
+    path, spec = model_path("tiny_full")
+    V = spec["n_vocab"]
+    head = write_head(lg, model_dir, "tiny_full", spec)
+    gpu = lg.hiplib.HipBackend(path, 128, max_rows=8)
+    t = gpu.mtp_open(head)
+    try:
+        gpu.prefill(np.arange(1, 21, dtype=np.int32), 0)
+        blocks = [np.arange(30, 38, dtype=np.int32), np.arange(50, 58, dtype=np.int32)]
+        want = []
+        for b in blocks:
+            want.append([gpu.forward(int(tok), 20 + j, V).view(np.uint32) for j, tok in enumerate(b)])
+        gpu.set_option("store_logits", 1)
+        orders = [range(8), range(7, -1, -1), (0, 1, 1, 2, 0, 1, 2, 5), (3,), (0,), (7, 0, 1, 2, 3, 4, 5, 6), ()]
+        for i, order in enumerate(orders):
+            adv = C.c_int32(0)
+            out = np.zeros(8, np.int32)
+            lg.hiplib.hip_check(gpu.H.lg_hip_forward_spec(gpu.dev, gpu.dkv, blocks[i & 1], 8, 20, out, C.byref(adv)), "forward_spec")
+            for j in order:
+                assert np.array_equal(gpu.logits_row(j, V).view(np.uint32), want[i & 1][j]), (i, j)
+        print("schedule", flush=True)
+        gpu.schedule(blocks[1][None], 20)
+        gpu.schedule_run(1)
+        for j in (0, 1, 4):
+            assert np.array_equal(gpu.logits_row(j, V).view(np.uint32), want[1][j])
+        gpu.schedule_wait()
+        with pytest.raises(lg.hiplib.HipError):
+            gpu.logits_row(8, V)
+        print("draft head", flush=True)
+        gpu.mtp_store_logits(t)
+        first = gpu.mtp_draft(t, 9, 24)
+        a = gpu.mtp_logits(t, V)
+        assert int(np.argmax(a)) == first and np.array_equal(a, gpu.mtp_logits(t, V))
+        second = gpu.mtp_draft(t, first, 25, chain=True)
+        assert int(np.argmax(gpu.mtp_logits(t, V))) == second
+    finally:
+        gpu.mtp_close(t)
+        gpu.close()
+
+
+def test_logits_nobody_reads_stay_on_the_device(lg, gpu_required, model_path):
+    """store_logits left on costs a scheduled step of 8 rows x 262144 logits what storing them in device memory does: 8 MiB across
+    the bus would take 130 us at the 64 GB/s of its link; half of that is the bound here."""
+    path, spec = model_path("tiny", n_vocab=262144)
+    gpu = lg.hiplib.HipBackend(path, 512, max_rows=8)
+    try:
+        gpu.prefill(np.arange(1, 21, dtype=np.int32), 0)
+        blocks = np.tile(np.arange(30, 38, dtype=np.int32), (20, 1))
+        us = {}
+        for on in (0, 1, 0, 1):
+            gpu.set_option("store_logits", on)
+            for _ in range(4):
+                gpu.schedule(blocks, 20)
+                us[on] = min(us.get(on, 1e9), gpu.schedule_time(20) * 1e3 / 20)
+        print(f"a step: {us[0]:.1f} us, with logits {us[1]:.1f} us", flush=True)
+        assert us[1] - us[0] < 65, us
+    finally:
+        gpu.close()
