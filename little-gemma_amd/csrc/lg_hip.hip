@@ -1853,13 +1853,22 @@ static int load_block(lg_hip_model *m, const int32_t *toks, int rows, int pos, b
     HIP_TRY(hipGetLastError());
     return 0;
 }
+// A process that asked the runtime to give the processor away while it waits (hipSetDeviceFlags: yield, blocking) waits for the
+// stream, which does so.  Every other one polls, as the runtime's own wait does, for up to 50 ms: far longer than a step takes.
 static int wait_report(lg_hip_model *m, const char *who, int rows, int32_t *out, int32_t *adv) {
     const int32_t *r = m->pin + 32;
+    auto there = [&]() { return __atomic_load_n(r + LG_REPORT_SEQ, __ATOMIC_ACQUIRE) == m->reports; };
+    unsigned flags = 0;
+    if (hipGetDeviceFlags(&flags) != hipSuccess) { (void)hipGetLastError(); flags = 0; }
+    const bool poll = !(flags & (hipDeviceScheduleYield | hipDeviceScheduleBlockingSync));
     const auto t0 = std::chrono::steady_clock::now();
-    for (int spins = 0; __atomic_load_n(r + LG_REPORT_SEQ, __ATOMIC_ACQUIRE) != m->reports; ++spins) {
-        if ((spins & 1023) != 1023 || std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(50)) { __builtin_ia32_pause(); continue; }
-        HIP_TRY(hipStreamSynchronize(m->stream));           // far longer than a step takes: a slow device, or an error that this returns
-        if (__atomic_load_n(r + LG_REPORT_SEQ, __ATOMIC_ACQUIRE) != m->reports) return fail(-9, "%s: the step ended without its results", who);
+    for (int spins = 0; poll && !there(); ++spins) {
+        if ((spins & 1023) == 1023 && std::chrono::steady_clock::now() - t0 >= std::chrono::milliseconds(50)) break;
+        __builtin_ia32_pause();
+    }
+    if (!there()) {                                          // (also a slow device, or an error that this returns)
+        HIP_TRY(hipStreamSynchronize(m->stream));
+        if (!there()) return fail(-9, "%s: the step ended without its results", who);
     }
     const int rc = step_err(who, r[LG_REPORT_ERR]);
     if (rc) return rc;

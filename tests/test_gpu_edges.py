@@ -7,6 +7,7 @@ import os
 import shutil
 import subprocess
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -360,4 +361,32 @@ def test_logits_nobody_reads_stay_on_the_device(lg, gpu_required, model_path):
         print(f"a step: {us[0]:.1f} us, with logits {us[1]:.1f} us", flush=True)
         assert us[1] - us[0] < 65, us
     finally:
+        gpu.close()
+
+
+def test_a_process_that_asked_for_blocking_waits_gets_them(lg, gpu_required, model_path):
+    """hipSetDeviceFlags(hipDeviceScheduleBlockingSync): the processor is given away during a step of some milliseconds (what is
+    left is the launch and the short while the runtime polls first), and the results are those of polling."""
+    path, spec = model_path("tiny", n_layer=64)
+    gpu = lg.hiplib.HipBackend(path, 256, max_rows=4)
+    hip = C.CDLL(None)
+    if not hasattr(hip, "hipSetDeviceFlags"):
+        hip = C.CDLL("libamdhip64.so")
+    before = C.c_uint(0)
+    assert hip.hipGetDeviceFlags(C.byref(before)) == 0
+    try:
+        gpu.prefill(np.arange(1, 21, dtype=np.int32), 0)
+        got, steps = [], 40
+        for flags in (before.value, 4, before.value):
+            assert hip.hipSetDeviceFlags(flags) == 0
+            gpu.forward_spec(np.array([5, 6, 7, 8], np.int32), 20)
+            cpu, wall = time.thread_time(), time.perf_counter()
+            res = [gpu.forward_spec(np.array([5, 6, 7, 8], np.int32), 20) for _ in range(steps)]
+            cpu, wall = time.thread_time() - cpu, time.perf_counter() - wall
+            print(f"flags {flags}: {wall / steps * 1e6:.0f} us a step, {cpu / steps * 1e6:.0f} us of the processor", flush=True)
+            got.append((cpu / wall, [(a, o.tolist()) for a, o in res]))
+        assert got[0][1] == got[1][1] == got[2][1]
+        assert got[1][0] < 0.6, got[1][0]
+    finally:
+        hip.hipSetDeviceFlags(before.value)
         gpu.close()
