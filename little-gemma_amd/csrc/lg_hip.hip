@@ -191,7 +191,7 @@ struct lg_hip_model {
     float eps = 0, base = 0, base_swa = 0, softcap = 0;
     std::vector<int> is_local, ffn_len, head_dim, n_head_kv;
     std::map<std::string, HostTensor> host;
-    bool committed = false;
+    bool committed = false, wide_built = false;    // wide_built: the matrices' wide forms exist
     // weights
     std::vector<Layer> L;
     uint8_t *emb = nullptr, *pmp = nullptr, *pte = nullptr;
@@ -202,7 +202,6 @@ struct lg_hip_model {
     float *output_norm = nullptr, *rope_freqs = nullptr, *proj_norm = nullptr;
     std::vector<void *> allocs;
     std::map<std::pair<int, int>, float *> rope_tabs;      // (is_local, hd) -> table
-    size_t weight_bytes = 0;
     // scratch
     float *x[2] = { nullptr, nullptr }, *qkv = nullptr, *dout = nullptr, *pmp_raw = nullptr, *hidden_rows = nullptr,
           *g_hidden = nullptr, *logits = nullptr, *pval = nullptr, *q_rot = nullptr;
@@ -298,6 +297,7 @@ extern "C" int lg_hip_model_create(const struct lg_hip_config *c, int device, lg
     if (const char *e = getenv("LG_HIP_ATTN_ROWS_FQ")) m->attn_rows_fq = atoi(e) != 0;
     if (const char *e = getenv("LG_HIP_ROWS_GEGLU")) m->rows_geglu = atoi(e) != 0;     // the row work ahead of gate/up inside the gate/up launch
     if (const char *e = getenv("LG_HIP_XCD_TAIL_SPREAD")) m->tail_spread = atoi(e);   // 0: the one-XCD tail as ple/32 x rows units of 4 wavefronts only; 2: as 8-wavefront units at 3 and 4 rows too
+    if (const char *e = getenv("LG_HIP_WIDE_PREFILL")) m->wide_prefill = atoi(e) != 0;     // 0: prompts in verify blocks, and none of the copies that prompt blocks read
     if (getenv("LG_HIP_NO_DOWN_KQ")) m->down_kq = 0;       // ffn_down of verify blocks by whole rows everywhere (comparison runs)
     hipError_t e = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&m->stream2, hipStreamNonBlocking);
@@ -341,7 +341,6 @@ static int upload_vec(lg_hip_model *m, const std::string &name, size_t n, bool r
     if (t->type != 0 || have != n) return fail(-6, "model_commit: %s must be f32 with %zu elements", name.c_str(), n);
     if (dev_alloc(m, out, n)) return -7;
     HIP_TRY(hipMemcpy(*out, t->data, n * 4, hipMemcpyHostToDevice));
-    m->weight_bytes += n * 4;
     return 0;
 }
 
@@ -374,7 +373,6 @@ static int upload_float_mat(lg_hip_model *m, const HostTensor *t, const std::str
     }
     if (dev_alloc(m, out, n)) return -7;
     HIP_TRY(hipMemcpy(*out, src, n * 4, hipMemcpyHostToDevice));
-    m->weight_bytes += n * 4;
     return 0;
 }
 // upload a tiled matrix whose virtual rows are given by `rows`
@@ -387,12 +385,12 @@ static int upload_tiled(lg_hip_model *m, const std::vector<const uint8_t *> &row
     else repack_rows(rows.data(), k, (int)rows.size(), stage.data());
     if (dev_alloc(m, out, bytes)) return -7;
     HIP_TRY(hipMemcpy(*out, stage.data(), bytes, hipMemcpyHostToDevice));
-    m->weight_bytes += bytes;
     return 0;
 }
-// the wide form of an uploaded matrix (prompt blocks; a draft head takes none): not counted into weight_bytes
+// the wide form of an uploaded matrix: 0.81 bytes a weight beside the 0.56 of its tiles.  Only prompt blocks read it: none for a
+// draft head, nor for a model whose option wide_prefill is off when it is committed.
 static int wide_form(lg_hip_model *m, const uint8_t *tiles, int k, int rows, bool rowblocks, uint8_t **out) {
-    if (m->target) return 0;
+    if (m->target || !m->wide_prefill) return 0;
     if (dev_alloc(m, out, lg_wide_bytes(k, rows))) return -7;
     const size_t n = (size_t)((rows + LG_WT - 1) / LG_WT * LG_WT) * (size_t)(k >> 5);
     hipLaunchKernelGGL(lg_k_wide_pack, dim3((unsigned)((n + LG_WG - 1) / LG_WG)), dim3(LG_WG), 0, nullptr, tiles, k, rows, rowblocks ? 1 : 0, *out);
@@ -563,13 +561,9 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         std::vector<const uint8_t *> rows;
         push_rows(rows, t, 0, m->n_vocab);
         if ((rc = upload_tiled(m, rows, E, &m->emb, stage))) return rc;
-        // a second copy in the order the matrix-core lm_head reads (the first also serves the embedding lookup);
-        // it is not counted into weight_bytes, which says what a step streams
-        if (max_rows >= 4 && m->n_vocab % 64 == 0 && lg_segments(E) == 8 && !getenv("LG_HIP_NO_HEAD_MFMA")) {
-            const size_t wb = m->weight_bytes;
+        // a second copy in the order the matrix-core lm_head reads (the first also serves the embedding lookup)
+        if (max_rows >= 4 && m->n_vocab % 64 == 0 && lg_segments(E) == 8 && !getenv("LG_HIP_NO_HEAD_MFMA"))
             if ((rc = upload_tiled(m, rows, E, &m->emb_rb, stage, true))) return rc;
-            m->weight_bytes = wb;
-        }
     }
     if ((rc = upload_vec(m, "output_norm.weight", E, true, &m->output_norm))) return rc;
     int hd_global = 0;
@@ -655,7 +649,6 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
             pack_o_chains(rows.data(), y.qd, E, stage.data());
             if (dev_alloc(m, &y.wo_ch, stage.size())) return -7;
             HIP_TRY(hipMemcpy(y.wo_ch, stage.data(), stage.size(), hipMemcpyHostToDevice));
-            m->weight_bytes += stage.size();
         }
         if (getenv("LG_HIP_MERGE_O") && atoi(getenv("LG_HIP_MERGE_O")) > 0 && !m->target && m->H == 8 && lg_segments(y.qd) == 8 && E % 64 == 0 && y.hd % 32 == 0 && y.hd <= 512 &&
             (rc = upload_tiled(m, rows, y.qd, &y.wo_rb, stage, true))) return rc;
@@ -686,7 +679,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
                 }
             }
         }
-        if (xffn) {                                               // (second copies: not counted into weight_bytes, which says what a step streams)
+        if (xffn) {                                               // (second copies)
             xstage.resize(256 * (xg.gu_bytes > xg.dn_bytes ? xg.gu_bytes : xg.dn_bytes));
             xffn_pack_gu((const uint8_t *)g->data, (const uint8_t *)u->data, xg, xstage.data());
             if (dev_alloc(m, &y.xgu, 256 * xg.gu_bytes)) return -7;
@@ -797,6 +790,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
     HIP_TRY(hipHostMalloc((void **)&m->pin, (64 + (size_t)m->sched_cap * (2 * LG_HIP_MAX_ROWS + 1)) * sizeof(int32_t), hipHostMallocDefault));
     m->pin[32 + LG_REPORT_SEQ] = 0;
     HIP_TRY(hipDeviceSynchronize());
+    m->wide_built = !m->target && m->wide_prefill;
     m->committed = true;
     return 0;
 }
@@ -1814,7 +1808,7 @@ extern "C" int lg_hip_set_option(lg_hip_model *m, const char *name, int value) {
     if (!strcmp(name, "store_logits")) m->store_logits = value != 0;
     else if (!strcmp(name, "head_mfma")) m->head_mfma = value != 0;
     else if (!strcmp(name, "use_graph")) m->use_graph = value != 0;
-    else if (!strcmp(name, "wide_prefill")) m->wide_prefill = value != 0;
+    else if (!strcmp(name, "wide_prefill")) m->wide_prefill = value != 0 && (!m->committed || m->wide_built);
     else if (!strcmp(name, "fuse_rows")) m->fuse_rows = value != 0;
     else if (!strcmp(name, "attn_rows")) m->attn_rows = value != 0;
     else if (!strcmp(name, "attn_rows_fq")) m->attn_rows_fq = value != 0;

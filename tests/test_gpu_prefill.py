@@ -2,6 +2,8 @@
 (v_mfma_i32_32x32x32_i8): the isolated matmul with 32 activation rows against the oracle
 (int32 block dots bit-exact, f32 bit-identical in this build's order), and whole prompts whose
 cache rows and next-token logits must equal the position-by-position oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -44,6 +46,40 @@ def test_wide_prefill_with_an_attention_output_of_32_segments(lg, ob, gpu_requir
     whose slabs the next row kernel adds (as ffn_down's are at the larger shapes)."""
     path, spec = model_path("tiny", n_head=80, n_head_kv=10)
     check_wide_prefill(lg, ob, path, spec, "tiny with 80 heads", 200)
+
+
+def free_bytes():
+    hip = C.CDLL(None)
+    if not hasattr(hip, "hipMemGetInfo"):
+        hip = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(0), C.c_size_t(0)
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_a_model_without_prompt_blocks_holds_no_copies_for_them(lg, gpu_required, model_path, monkeypatch):
+    """LG_HIP_WIDE_PREFILL=0: the 0.81 bytes a weight that prompt blocks read are not there, the option cannot be switched on
+    behind that, and a prompt leaves the same cache."""
+    path, spec = model_path("tiny", n_ff=8192)
+    qkv = spec["n_embd"] * (spec["n_head"] + 2 * spec["n_head_kv"]) * spec["head_dim"]
+    weights = spec["n_layer"] * (qkv + spec["n_head"] * spec["head_dim"] * spec["n_embd"] + 3 * spec["n_embd"] * spec["n_ff"])
+    prompt = np.arange(1, 101, dtype=np.int32)
+    lg.hiplib.HipBackend(path, 256, max_rows=4).close()   # (what the runtime takes for itself)
+    held, caches = [], []
+    for wide in ("1", "0"):
+        monkeypatch.setenv("LG_HIP_WIDE_PREFILL", wide)
+        before = free_bytes()
+        gpu = lg.hiplib.HipBackend(path, 256, max_rows=4)
+        try:
+            held.append(before - free_bytes())
+            gpu.set_option("wide_prefill", 1)
+            print(f"LG_HIP_WIDE_PREFILL={wide}: {held[-1] >> 20} MiB", flush=True)
+            gpu.prefill(prompt, 0)
+            caches.append([gpu.kv_read(L, w) for L in range(spec["n_layer"]) for w in (0, 1)])
+        finally:
+            gpu.close()
+    assert held[0] - held[1] > 0.75 * weights, (held, weights)
+    assert all(np.array_equal(a, b) for a, b in zip(*caches))
 
 
 def check_wide_prefill(lg, ob, path, spec, name, n_prompt):
