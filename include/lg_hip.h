@@ -61,12 +61,13 @@ void lg_hip_model_destroy(lg_hip_model *m);
 int  lg_hip_kv_create(lg_hip_model *m, int max_seq, lg_hip_kv **out);
 void lg_hip_kv_destroy(lg_hip_kv *kv);
 int  lg_hip_ring_rows(int window, int max_seq);
-/* What lg_hip_kv_create asks for besides the rings (no counterpart in the reference, whose attention
- * keeps its partials per launch): bytes of attention partials, one slot of (max, sum, max_hd
- * accumulators) per (row of the cache's widest block, head, key tile a block can touch).  The widest
- * PROMPT block of a cache (*wide_rows: 512, 128, 32, or 0 = verify-width blocks only) is the largest
- * whose partials stay within 2 GiB; any_global = the model has a layer without a sliding window.
- * Arithmetic only: callable without a device. */
+/* What lg_hip_kv_create may take besides the rings (no counterpart in the reference, whose attention
+ * keeps its partials per launch): the bytes of one slot of (max, sum, max_hd accumulators) per (row of
+ * *wide_rows prompt or max_rows verify rows, head, key tile a block can touch), *wide_rows = the largest of
+ * 512, 128, 32 and 0 with which that stays within 2 GiB.  It asks for what its blocks need within that: the
+ * slots of max_rows rows, and 34 floats per (query head of a prompt row, tile) where a prompt block's tiles
+ * do not fit on-chip memory; prompt blocks are as wide (up to 512, at least 32 rows) as this leaves room for.
+ * any_global = the model has a layer without a sliding window.  Arithmetic only: callable without a device. */
 size_t lg_hip_kv_partials(int max_seq, int window, int any_global, int max_rows, int n_head, int max_hd,
                           int *wide_rows, int *tiles_max);
 /* rows/width of an owning layer's K (== V) storage; *rows = 0 for a layer that shares. */
@@ -88,10 +89,10 @@ int  lg_hip_kv_restore_prefix(lg_hip_kv *kv, int n);
 int  lg_hip_forward_spec(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int n_rows, int pos,
                          int32_t *out, int32_t *adv);
 /* model_prefill (include/model.h:121): positions pos0..pos0+n-1, cache writes only, no head.
- * Runs as blocks of 512 rows (128 when the cache holds fewer than 1024 positions) whose matmuls use the int8
- * matrix cores (the reference's chunked prefill, src/cuda/prefill-kernel.cuh:631-675), then 128- and 32-row
- * blocks, then verify-width blocks for the tail; every block leaves the cache rows that position-by-position
- * decode would. */
+ * Runs as blocks of up to 512 rows (128 when the cache holds fewer than 1024 positions, fewer in very long
+ * caches: lg_hip_kv_partials) on the matrix cores (the reference's chunked prefill,
+ * src/cuda/prefill-kernel.cuh:631-675), a last block of max_rows rows and fewer as a verify block; every block
+ * leaves the cache rows that position-by-position decode would. */
 int  lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int n, int pos0);
 /* Post-output-norm hidden state of the last valid row of the latest verify step (n_embd
  * floats): what the reference keeps in g_hidden / model.last_hidden for the draft head
@@ -104,7 +105,8 @@ int  lg_hip_set_hidden_row(lg_hip_model *m, int row);
  * "store_logits" option is on (model_forward, include/model.h:98, needs them; the verify does not). */
 int  lg_hip_get_logits(lg_hip_model *m, int row, float *dst);
 /* Options: "store_logits" (0/1, default 0), "use_graph" (0/1, default 1), "wide_prefill" (0/1,
- * default 1: 0 sends the whole prompt through verify-width blocks). */
+ * default 1: 0 sends the whole prompt through verify-width blocks; set before the commit it also leaves out
+ * the copies of the matrices that prompt blocks read, and cannot be set to 1 afterwards). */
 int  lg_hip_set_option(lg_hip_model *m, const char *name, int value);
 /* Measurement aid (no reference counterpart): with the option "xcd_tail_stamps" on, every unit of the
  * one-XCD launches of a layer writes the device wall clock (100 MHz) at its 8 phase boundaries; this

@@ -9,6 +9,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <algorithm>
 #include <array>
 #include <chrono>
 #include <map>
@@ -49,17 +50,18 @@ extern "C" int lg_hip_device_count(void) {
     return n;
 }
 // The widest prompt block a cache of max_seq positions takes: LG_WIDE_ROWS for caches of 1024 positions and more,
-// LG_WIDE_MID below (a short cache does not pay 512 spare rows per sliding ring and 512 rows of attention partials)
+// LG_WIDE_MID below (a short cache does not pay 512 spare rows per sliding ring)
 static int wide_rows_for(int max_seq) { return max_seq >= 1024 ? LG_WIDE_ROWS : LG_WIDE_MID; }
 extern "C" int lg_hip_ring_rows(int window, int max_seq) {
     int r = (window + wide_rows_for(max_seq) + 31) / 32 * 32;   // window + spare for the widest block written before its queries run, tile multiple
     return r < max_seq ? r : max_seq;
 }
 
-// The attention partials of a cache: one (max, sum, hd accumulators) slot per (row of the widest block, head, key
-// tile any block can touch).  A global layer's block late in a long cache touches every tile, so at the widest
-// block the slots grow with rows x max_seq: the widest PROMPT block of a cache is stepped down (512, 128, 32 rows,
-// then verify-width blocks only) until the partials fit LG_PARTIALS_BUDGET.  Pure arithmetic, no device needed.
+// What the attention of a cache may take beside its rings: one (max, sum, hd accumulators) slot per (row of the widest block,
+// head, key tile any block can touch), the widest PROMPT block of a cache stepped down (512, 128, 32 rows, then verify-width
+// blocks only) until that fits LG_PARTIALS_BUDGET: late in a long cache a block touches every tile, and the slots grow with
+// rows x max_seq.  Verify blocks keep such partials; the weights that prompt blocks keep of a tile in memory take less than
+// them (34 floats a unit and tile), so that this bounds both: lg_hip_kv_create asks for what they need.  Pure arithmetic.
 #define LG_PARTIALS_BUDGET ((size_t)2 << 30)
 extern "C" size_t lg_hip_kv_partials(int max_seq, int window, int any_global, int max_rows, int n_head, int max_hd,
                                      int *wide_rows, int *tiles_max) {
@@ -256,9 +258,9 @@ struct lg_hip_model {
 
 struct lg_hip_kv {
     lg_hip_model *m = nullptr;
-    int max_seq = 0, tiles_max = 0, wide_rows = 0;      // wide_rows: the block the partials are sized for
-    int prompt_rows = 0;                                // widest prompt block: what the rings' spare rows and the partials' memory (as the scratch of lg_k_wide_attn) allow
-    size_t scratch_bytes = 0;
+    int max_seq = 0, tiles_max = 0;                     // tiles_max: stride of the partials, tiles a block can touch
+    int prompt_rows = 0;                                // widest prompt block: what the rings' spare rows and the memory that lg_hip_kv_partials grants the scratch of lg_k_wide_attn allow
+    size_t scratch_bytes = 0;                           // of pacc: accumulators of verify blocks, scratch of lg_k_wide_attn
     std::vector<int> seq, kv_dim;
     std::vector<uint16_t *> k, v, px_k, px_v;
     float *pm = nullptr, *pl = nullptr, *pacc = nullptr;
@@ -844,7 +846,7 @@ extern "C" int lg_hip_kv_create(lg_hip_model *m, int max_seq, lg_hip_kv **out) {
         if (y.hd > max_hd) max_hd = y.hd;
         if (!(y.is_local && m->window > 0)) any_global = 1;
     }
-    const size_t pbytes = lg_hip_kv_partials(max_seq, m->window, any_global, m->max_rows, m->H, max_hd, &kv->wide_rows, &kv->tiles_max);
+    const size_t pbytes = lg_hip_kv_partials(max_seq, m->window, any_global, m->max_rows, m->H, max_hd, nullptr, &kv->tiles_max);
     for (int L = 0; L < nl; ++L) {
         const Layer &y = m->L[L];
         kv->kv_dim[L] = y.kd;
@@ -856,20 +858,16 @@ extern "C" int lg_hip_kv_create(lg_hip_model *m, int max_seq, lg_hip_kv **out) {
         if (e1 != hipSuccess || e2 != hipSuccess) { lg_hip_kv_destroy(kv); return fail(-7, "kv_create: out of device memory at layer %d", L); }
         (void)hipMemset(kv->k[L], 0, bytes); (void)hipMemset(kv->v[L], 0, bytes);
     }
-    const size_t slots = pbytes / ((size_t)max_hd * 4 + 8);
-    kv->scratch_bytes = slots * max_hd * 4;
-    auto prompt_scratch = [&](int rows) {
-        size_t most = 0;
-        for (int L = 0; L < nl; ++L) {
-            const size_t n = wide_attn_scratch(m, m->L[L], rows, max_seq > rows ? max_seq - rows : 0);
-            most = n > most ? n : most;
-        }
-        return most;
-    };
+    const size_t slots = (size_t)m->max_rows * m->H * kv->tiles_max, grant = pbytes / ((size_t)max_hd * 4 + 8) * max_hd * 4;
+    auto most = [&](auto need) { size_t n = 0; for (const Layer &y : m->L) n = std::max(n, need(y)); return n; };
+    auto prompt_scratch = [&](int rows) { return most([&](const Layer &y) { return wide_attn_scratch(m, y, rows, max_seq > rows ? max_seq - rows : 0); }); };
     kv->prompt_rows = wide_rows_for(max_seq);
-    while (kv->prompt_rows > LG_WIDE && prompt_scratch(kv->prompt_rows) > kv->scratch_bytes) kv->prompt_rows -= LG_WIDE;
+    while (kv->prompt_rows > LG_WIDE && prompt_scratch(kv->prompt_rows) > grant) kv->prompt_rows -= LG_WIDE;
     // partials of verify blocks of one or two rows (a long cache, a model committed for no more) are smaller than what 32 prompt rows need
-    if (prompt_scratch(kv->prompt_rows) > kv->scratch_bytes) kv->scratch_bytes = prompt_scratch(kv->prompt_rows);
+    kv->scratch_bytes = std::max(slots * max_hd * 4, prompt_scratch(kv->prompt_rows));
+    // and the two-launch attention of few workgroups, within the same grant
+    kv->scratch_bytes = std::max(kv->scratch_bytes, std::min(grant, most([&](const Layer &y) {
+        return (size_t)LG_WA_SPLIT_GROUPS * std::min(wide_attn_tiles(m, y, kv->prompt_rows, max_seq > kv->prompt_rows ? max_seq - kv->prompt_rows : 0), LG_WA_SPLIT_MAX) * (16 * 34 * 4); })));
     if (hipMalloc((void **)&kv->pm, slots * 4) != hipSuccess || hipMalloc((void **)&kv->pl, slots * 4) != hipSuccess ||
         hipMalloc((void **)&kv->pacc, kv->scratch_bytes) != hipSuccess) { lg_hip_kv_destroy(kv); return fail(-7, "kv_create: out of device memory for attention partials"); }
     HIP_TRY(hipDeviceSynchronize());
@@ -1622,7 +1620,7 @@ static bool far_in_narrow_heads(const lg_hip_model *m, const lg_hip_kv *kv, int 
     for (const Layer &y : m->L) if (y.hd < 512 && far_block(kv, y, rows, pos)) return true;
     return false;
 }
-// Up to 128 workgroups (half of the chip) with 12 tiles and more: scores and values as two launches over more workgroups (200
+// Up to LG_WA_SPLIT_GROUPS workgroups (half of the chip) with 12 tiles and more: scores and values as two launches over more workgroups (200
 // rows, 100 workgroups: 41 -> 39 us in a 512-wide window, 175 -> 113 us over 100 tiles; with 130 workgroups 42 -> 55 us, with 8
 // tiles 23 us both ways).  Score workgroups take 4 tiles, or up to 16 while there are more than 512 of them.
 // `far`: the block reaches value rows 2 GiB and more behind a layer's first one and takes 64-bit addresses (96 rows, 16 heads of 512
@@ -1633,7 +1631,7 @@ static void launch_wide_attn(Launcher &lx, const WideAttn &a, int groups, bool f
     const int wgs = groups * a.nkv;
     if constexpr (HD == 512)
         if (far) { LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false, 0, true>), grid, dim3(LG_WA_WG), 0, a, lx.m->ctl); return; }
-    if (wgs <= 128 && a.tiles >= 12 && a.tiles <= LG_WA_SPLIT_MAX && (size_t)wgs * a.tiles * (16 * 34 * 4) <= scratch_bytes) {
+    if (wgs <= LG_WA_SPLIT_GROUPS && a.tiles >= 12 && a.tiles <= LG_WA_SPLIT_MAX && (size_t)wgs * a.tiles * (16 * 34 * 4) <= scratch_bytes) {
         int chunk = 4;
         while (chunk < 16 && wgs * (a.tiles / chunk) > 512) chunk *= 2;
         LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false, 1>), dim3(groups, a.nkv, (a.tiles + chunk - 1) / chunk), dim3(LG_WA_SPLIT_WG), 0, a, lx.m->ctl);

@@ -82,6 +82,30 @@ def test_a_model_without_prompt_blocks_holds_no_copies_for_them(lg, gpu_required
     assert all(np.array_equal(a, b) for a, b in zip(*caches))
 
 
+def test_a_cache_takes_what_its_blocks_need(lg, gpu_required, model_path):
+    """Beside its rings a cache of 4096 positions takes the partials of 8-row blocks (8 rows x 8 heads x 130 tiles x 258 floats,
+    9 MiB) and the weights that 512 prompt rows keep of their tiles (256 groups of units x 132 tiles x 544 floats, 70 MiB), not the
+    partials of 512 rows (524 MiB: what lg_hip_kv_partials allows it)."""
+    path, spec = model_path("tiny", head_dim=256)
+    lg.hiplib.HipBackend(path, 256, max_rows=8).close()
+    gpu = lg.hiplib.HipBackend(path, 256, max_rows=8)
+    try:
+        before = free_bytes()
+        kv = C.c_void_p()
+        lg.hiplib.hip_check(gpu.H.lg_hip_kv_create(C.c_void_p(gpu.dev), 4096, C.byref(kv)), "kv_create")
+        taken = before - free_bytes()
+        rows, width = C.c_int(), C.c_int()
+        for L in range(spec["n_layer"]):
+            lg.hiplib.hip_check(gpu.H.lg_hip_kv_layout(kv, L, C.byref(rows), C.byref(width)), "kv_layout")
+            taken -= 2 * rows.value * width.value * 2
+        gpu.H.lg_hip_kv_destroy.argtypes, gpu.H.lg_hip_kv_destroy.restype = [C.c_void_p], None
+        gpu.H.lg_hip_kv_destroy(kv)
+        print(f"beside the rings: {taken >> 20} MiB", flush=True)
+        assert taken < 110 << 20, taken
+    finally:
+        gpu.close()
+
+
 def check_wide_prefill(lg, ob, path, spec, name, n_prompt):
     rng = np.random.default_rng(n_prompt)
     prompt = rng.integers(1, spec["n_vocab"], n_prompt).astype(np.int32)
