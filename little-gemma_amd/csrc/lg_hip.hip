@@ -1047,7 +1047,7 @@ static int launch_mm(Launcher &lx, int cls, const MmArgs &a_in, bool slabs_ok = 
         // blocks of four and more rows whose consumer adds four slabs: cut by K quarter (a quarter of the activations
         // per workgroup, several workgroups per CU).  12B shape, 5 rows: ffn_down 16.9 -> 14.3 us, the rows kernel that
         // adds the slabs 6.6 -> 7.5 us, the step 3.814 -> 3.775 ms (2 and 5 wavefronts per workgroup: 3.827, 3.924)
-        if constexpr (M >= 4 && M <= LG_HIP_MAX_ROWS) {
+        if constexpr (M >= 4) {
             const int oct = (a.m + 7) / 8, W = 4;
             a.nthreads = 64 * W;
             LAUNCH(cls, (lg_k_mm_kq<M>), dim3((oct + W - 1) / W, 4), dim3(64 * W), (size_t)M * (a.k / 1024) * 320, LG_MM_FIELDS(LG_XA, a) 0);
@@ -1070,7 +1070,7 @@ static int launch_mm(Launcher &lx, int cls, const MmArgs &a_in, bool slabs_ok = 
     } else if (M >= 4 && a.k >= 2048 && !DUMP) {
         // blocks of four and more rows: two row groups per workgroup, the tiles of each cut over two wavefronts
         // (over four was no faster at 8 and 10 tiles per group)
-        if constexpr (M >= 4 && M <= LG_HIP_MAX_ROWS) {
+        if constexpr (M >= 4) {
             const size_t l2 = ((lds + 15) & ~(size_t)15) + (size_t)2 * M * 64 * 4;
             // (over four wavefronts from 12 tiles per group on: 12B shape, k = 3840 and 4096, 3.662 -> 3.645 ms per step)
             a.nthreads = (a.k >> 8) >= 12 ? 512 : 256;
@@ -1096,7 +1096,7 @@ static void launch_mmf(Launcher &lx, int cls, const MmfArgs &a) {
     LAUNCH(cls, (lg_k_mmf<MC>), dim3((a.m + LG_WG / 64 - 1) / (LG_WG / 64), (a.rows + MC - 1) / MC), dim3(LG_WG), 0, a);
 }
 static bool attention_rows_shared(int rows, int tiles, int nkv, int hd, int seq) {
-    return rows > 1 && rows <= LG_HIP_MAX_ROWS && hd <= 256 && seq >= 32 && tiles * nkv >= 256;
+    return rows > 1 && hd <= 256 && seq >= 32 && tiles * nkv >= 256;
 }
 // tiles per workgroup of lg_k_attn_rows: one, until the grid would exceed the three workgroups per CU that the
 // staged tile's LDS lets a CU hold; then as many as bring it back under that (at most four), each tile's rows in
@@ -1109,7 +1109,7 @@ static int attention_rows_tp(int tiles, int nkv) {
 // the XCD-partitioned feed-forward launch: 256 workgroups of 512 threads, the instantiation of the shape's class
 template <int M>
 static void launch_xffn(Launcher &lx, const XffnArgs &a, int cls) {
-    if constexpr (M >= 4 && M <= LG_HIP_MAX_ROWS) {
+    if constexpr (M >= 4) {
         const size_t lds = xffn_lds(lg_xffn_geo(a.E, a.FF), M);
         switch (cls) {
             case 0: LAUNCH(KC_FFN, (lg_k_ffn_xcd<M, 1, 2, 1, 8, 8>), dim3(256), dim3(LG_XFFN_THREADS), lds, LG_XFFN_FIELDS(LG_XA, a) 0); break;
@@ -1123,7 +1123,7 @@ static void launch_xffn(Launcher &lx, const XffnArgs &a, int cls) {
 // The per-layer-input block of a verify block of `rows` rows as the one-XCD launch lg_k_ple_tail: q4_0 matrices of the
 // 256-wide per-layer input, at most LG_XTAIL_UNITS (gate block, row) units, a chip whose workgroups are dealt over 8 XCDs
 static bool use_ple_tail(const lg_hip_model *m, int rows) {
-    if (!m->ple || !m->tsync || m->xcd_tail <= 0 || m->target || rows < 1 || rows > LG_HIP_MAX_ROWS) return false;
+    if (!m->ple || !m->tsync || m->xcd_tail <= 0 || m->target) return false;
     if (m->ple != 256 || (m->ple / 32) * rows > LG_XTAIL_UNITS || m->E % 256 || m->E > 4096 || (m->E + 1023) / 1024 > m->ple / 32) return false;
     const int U = (m->ple / 32) * rows;
     const bool spread = m->tail_spread && (rows >= 5 || rows <= 2);   // (lg_k_ple_tail_s: 8 wavefronts per unit, enough of them at every width)
@@ -1148,7 +1148,7 @@ static int merge_o_slices(const lg_hip_model *m, int rows) {
     return pick;
 }
 static bool use_merge_o(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
-    if (!y.wo_rb || m->merge_o <= 0 || rows > LG_HIP_MAX_ROWS || (m->merge_o == 1 && rows < 3)) return false;
+    if (!y.wo_rb || m->merge_o <= 0 || (m->merge_o == 1 && rows < 3)) return false;
     return tiles < 128 && merge_o_slices(m, rows) > 0;
 }
 static void launch_merge_o(Launcher &lx, const MergeOArgs &a) {
@@ -1162,7 +1162,7 @@ static void launch_merge_o(Launcher &lx, const MergeOArgs &a) {
 
 template <int M>
 static void launch_down_m(Launcher &lx, const DownMArgs &a) {
-    if constexpr (M >= 4 && M <= LG_HIP_MAX_ROWS) {
+    if constexpr (M >= 4) {
         const DownMGeo g = lg_down_m_geo(a.E, a.FF);
         const size_t lds = (size_t)8 * g.nitd * (LG_MU_DWORDS * 4) + (size_t)8 * g.ops * 8 * 32 * 4;
         if (g.ops == 1 && g.npairs <= 3) LAUNCH(KC_DOWN, (lg_k_down_m<M, 1, 3>), dim3(256), dim3(512), lds, LG_DOWNM_FIELDS(LG_XA, a) 0);
@@ -1172,31 +1172,30 @@ static void launch_down_m(Launcher &lx, const DownMArgs &a) {
     }
 }
 static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
-    if (!y.wo_ch || !m->tsync || m->xcd_attn_tail <= 0 || rows > LG_HIP_MAX_ROWS || (m->xcd_attn_tail == 1 && rows < 3)) return false;
+    if (!y.wo_ch || !m->tsync || m->xcd_attn_tail <= 0 || (m->xcd_attn_tail == 1 && rows < 3)) return false;
     const int slices = (m->E + 1023) / 1024;
     return tiles < 128 && m->H * rows <= 2 * LG_XCD_WGS && slices * rows <= LG_XCD_WGS && y.hd % 32 == 0 && y.hd <= 256;
 }
 template <int M>
 static void launch_attn_tail(Launcher &lx, const XattnTailArgs &a) {
-    if constexpr (M <= LG_HIP_MAX_ROWS) {
-        lg_hip_model *m = lx.m;
-        int np = 0, rb = 0;
-        if (!attn_tail_shape(a.g.H * a.g.hd, a.E, &np, &rb)) { lx.rc = fail(-2, "attn_tail: no instantiation for this shape"); return; }
-        const size_t lds = (size_t)(16 * np) * LG_MU_DWORDS * 4 + (size_t)8 * rb * 8 * 32 * 4;
-        const dim3 grid(LG_XCDS * LG_XCD_WGS);
-        if (np == 1 && rb == 1) LAUNCH(KC_ATAIL, (lg_k_attn_tail<M, 1, 1>), grid, dim3(512), lds, m->ctl, LG_XATTN_FIELDS(LG_XA, a) 0);
-        else if (np == 2 && rb == 1) LAUNCH(KC_ATAIL, (lg_k_attn_tail<M, 2, 1>), grid, dim3(512), lds, m->ctl, LG_XATTN_FIELDS(LG_XA, a) 0);
-        else LAUNCH(KC_ATAIL, (lg_k_attn_tail<M, 4, 3>), grid, dim3(512), lds, m->ctl, LG_XATTN_FIELDS(LG_XA, a) 0);
-    }
+    lg_hip_model *m = lx.m;
+    int np = 0, rb = 0;
+    if (!attn_tail_shape(a.g.H * a.g.hd, a.E, &np, &rb)) { lx.rc = fail(-2, "attn_tail: no instantiation for this shape"); return; }
+    const size_t lds = (size_t)(16 * np) * LG_MU_DWORDS * 4 + (size_t)8 * rb * 8 * 32 * 4;
+    const dim3 grid(LG_XCDS * LG_XCD_WGS);
+    if (np == 1 && rb == 1) LAUNCH(KC_ATAIL, (lg_k_attn_tail<M, 1, 1>), grid, dim3(512), lds, m->ctl, LG_XATTN_FIELDS(LG_XA, a) 0);
+    else if (np == 2 && rb == 1) LAUNCH(KC_ATAIL, (lg_k_attn_tail<M, 2, 1>), grid, dim3(512), lds, m->ctl, LG_XATTN_FIELDS(LG_XA, a) 0);
+    else LAUNCH(KC_ATAIL, (lg_k_attn_tail<M, 4, 3>), grid, dim3(512), lds, m->ctl, LG_XATTN_FIELDS(LG_XA, a) 0);
 }
 
 template <int M>
 static void launch_ple_tail(Launcher &lx, const XtailArgs &a) {
-    if constexpr (M <= LG_HIP_MAX_ROWS) {
+    lg_hip_model *m = lx.m;
+    const int E = a.r.g.k;
+    {
         // 5..8 rows: the form whose units fit one per CU (row j by 32 / M workgroups of 8 wavefronts); 1 and 2 rows: the
         // form that has enough wavefronts for the projection
-        lg_hip_model *m = lx.m;
-        const int E = a.r.g.k, W = M * (32 / M), G = (E / 8 + 8 * W - 1) / (8 * W);
+        const int W = M * (32 / M), G = (E / 8 + 8 * W - 1) / (8 * W);
         if ((m->tail_spread == 2 || (m->tail_spread && (M >= 5 || M <= 2))) && a.gf && a.r.g.ple == 256 && G >= 1 && G <= 3) {
             const size_t lds = (size_t)E * 5 / 4 + (size_t)M * a.r.g.ple * 5 / 4;
             const dim3 grid(LG_XCDS * W);
@@ -1221,33 +1220,30 @@ static void launch_ple_tail(Launcher &lx, const XtailArgs &a) {
             }
         }
     }
-    if constexpr (M <= LG_HIP_MAX_ROWS) {
-        lg_hip_model *m = lx.m;
-        const int E = a.r.g.k, U = (a.r.g.ple / 32) * M;
-        const int G = (E / 8 + 4 * U - 1) / (4 * U);
-        const size_t lds = (size_t)E * 5 / 4 + (size_t)M * a.r.g.ple * 5 / 4;
-        const dim3 grid(LG_XCDS * U);
-        // the U units wait for each other: all of them must be resident on the 32 CUs of one XCD at once
-        static int fits[5] = { 0, 0, 0, 0, 0 };              // per G: 0 unknown, 1 yes, -1 no (asked once, outside any capture)
-        if (G >= 1 && G <= 4 && !fits[G]) {
-            int per_cu = 0;
-            hipError_t e = hipErrorInvalidValue;
-            switch (G) {
-                case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail<M, 1>, LG_WG, lds); break;
-                case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail<M, 2>, LG_WG, lds); break;
-                case 3: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail<M, 3>, LG_WG, lds); break;
-                case 4: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail<M, 4>, LG_WG, lds); break;
-            }
-            fits[G] = (e == hipSuccess && per_cu * LG_XCD_WGS >= U) ? 1 : -1;
-        }
-        if (G < 1 || G > 4 || fits[G] < 0) { lx.rc = fail(-2, "ple_tail: %d units of %d row groups per wavefront do not fit one XCD", U, G); return; }
+    const int U = (a.r.g.ple / 32) * M;
+    const int G = (E / 8 + 4 * U - 1) / (4 * U);
+    const size_t lds = (size_t)E * 5 / 4 + (size_t)M * a.r.g.ple * 5 / 4;
+    const dim3 grid(LG_XCDS * U);
+    // the U units wait for each other: all of them must be resident on the 32 CUs of one XCD at once
+    static int fits[5] = { 0, 0, 0, 0, 0 };              // per G: 0 unknown, 1 yes, -1 no (asked once, outside any capture)
+    if (G >= 1 && G <= 4 && !fits[G]) {
+        int per_cu = 0;
+        hipError_t e = hipErrorInvalidValue;
         switch (G) {
-            case 1: LAUNCH(KC_TAIL, (lg_k_ple_tail<M, 1>), grid, dim3(LG_WG), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
-            case 2: LAUNCH(KC_TAIL, (lg_k_ple_tail<M, 2>), grid, dim3(LG_WG), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
-            case 3: LAUNCH(KC_TAIL, (lg_k_ple_tail<M, 3>), grid, dim3(LG_WG), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
-            case 4: LAUNCH(KC_TAIL, (lg_k_ple_tail<M, 4>), grid, dim3(LG_WG), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
-            default: lx.rc = fail(-2, "ple_tail: %d row groups per wavefront", G);
+            case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail<M, 1>, LG_WG, lds); break;
+            case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail<M, 2>, LG_WG, lds); break;
+            case 3: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail<M, 3>, LG_WG, lds); break;
+            case 4: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail<M, 4>, LG_WG, lds); break;
         }
+        fits[G] = (e == hipSuccess && per_cu * LG_XCD_WGS >= U) ? 1 : -1;
+    }
+    if (G < 1 || G > 4 || fits[G] < 0) { lx.rc = fail(-2, "ple_tail: %d units of %d row groups per wavefront do not fit one XCD", U, G); return; }
+    switch (G) {
+        case 1: LAUNCH(KC_TAIL, (lg_k_ple_tail<M, 1>), grid, dim3(LG_WG), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
+        case 2: LAUNCH(KC_TAIL, (lg_k_ple_tail<M, 2>), grid, dim3(LG_WG), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
+        case 3: LAUNCH(KC_TAIL, (lg_k_ple_tail<M, 3>), grid, dim3(LG_WG), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
+        case 4: LAUNCH(KC_TAIL, (lg_k_ple_tail<M, 4>), grid, dim3(LG_WG), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
+        default: lx.rc = fail(-2, "ple_tail: %d row groups per wavefront", G);
     }
 }
 
@@ -1417,7 +1413,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             a.gx = tiles; a.gz = M;
             const bool shared = rows_shared(L);
             if (shared) {
-                if constexpr (M > 1 && M <= LG_HIP_MAX_ROWS) {
+                if constexpr (M > 1) {
                     const size_t lds = y.hd == 256 ? AttnRowsGeo<256>::bytes(M * G, fused_post) : y.hd == 128 ? AttnRowsGeo<128>::bytes(M * G, fused_post) : AttnRowsGeo<64>::bytes(M * G, fused_post);
                     const int tp = attention_rows_tp(tiles, y.nkv);
                     const dim3 grid((tiles + tp - 1) / tp, y.nkv);
@@ -1463,7 +1459,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 launch_merge_o(lx, f);
                 pend_dout = m->dout; pend_w = y.post_attn; pend_os = nullptr; pend_parts = 8;
             } else
-            if (M <= LG_HIP_MAX_ROWS && tiles >= 128 && y.hd % 64 == 0) LAUNCH(KC_MERGE, (lg_k_attn_merge_split<M>), dim3(H, M, y.hd / 64), dim3(LG_WG), 0, m->ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
+            if (tiles >= 128 && y.hd % 64 == 0) LAUNCH(KC_MERGE, (lg_k_attn_merge_split<M>), dim3(H, M, y.hd / 64), dim3(LG_WG), 0, m->ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
             else LAUNCH(KC_MERGE, (lg_k_attn_merge<M>), dim3(H, M), dim3(LG_WG), 0, m->ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
         }
         if (!merged_o) {   // attention output projection
@@ -1575,7 +1571,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         grid = (m->n_vocab / 64 + passes - 1) / passes;
         HeadArgs h{ head_m ? m->emb_rb : m->emb, E, m->n_vocab, passes, m->hq, m->softcap, m->store_logits ? m->logits : nullptr, m->pval, m->pidx };
         if (head_m) {
-            if constexpr (M >= 4 && M <= LG_HIP_MAX_ROWS)
+            if constexpr (M >= 4)
                 LAUNCH(KC_HEAD, (lg_k_head_m<M>), dim3(grid), dim3(512), (size_t)(E / 32) * LG_MU_DWORDS * 4, LG_HEAD_FIELDS(LG_XA, h) 0);
         } else
         LAUNCH(KC_HEAD, (lg_k_mm_head<M>), dim3(grid), dim3(LG_WG), lds_mm(M, E), LG_HEAD_FIELDS(LG_XA, h) 0);
@@ -1596,17 +1592,21 @@ static WideShape wide_shape(int m, int rows, int parts) {
     if (((m + LG_WT - 1) / LG_WT) * ((rows + 31) / 32) * parts <= 256) return { 1, 8 };
     return { rows <= 32 ? 1 : 2, 4 };
 }
-template <bool DUMP>
-static int launch_wide_mm(Launcher &lx, int cls, const uint8_t *w, const int8_t *q, int k, int m, int rows, float *out, int32_t *dots) {
-    const int parts = lg_segments(k) / 8;
+struct WideLaunch { WideMm a; WideShape c; dim3 grid, block; size_t lds; };
+static WideLaunch wide_launch(const uint8_t *w, const int8_t *q, int k, int m, int rows, int parts) {
     const WideShape c = wide_shape(m, rows, parts);
     const WideMm a{ w, (const uint8_t *)q, k, m, rows, (rows + 32 * c.tb - 1) / (32 * c.tb), parts };
-    const dim3 grid(lg_wide_grid(m, a.nb_tiles, parts)), block(64 * c.wv);
-    const size_t lds = (size_t)c.wv * 2 * c.tb * 4096;
-    if (c.wv == 8)      LAUNCH(cls, (lg_k_wide_mm<1, 8, DUMP>), grid, block, lds, a, out, dots);
-    else if (c.tb == 1) LAUNCH(cls, (lg_k_wide_mm<1, 4, DUMP>), grid, block, lds, a, out, dots);
-    else                LAUNCH(cls, (lg_k_wide_mm<2, 4, DUMP>), grid, block, lds, a, out, dots);
-    return parts;
+    return { a, c, dim3(lg_wide_grid(m, a.nb_tiles, parts)), dim3(64 * c.wv), (size_t)c.wv * 2 * c.tb * 4096 };
+}
+// k18, k14, k24: the kernel's builds for 32 activation rows by eight and by four wavefronts and for 64 by four
+#define LAUNCH_WIDE(cls, l, k18, k14, k24, ...) do { if (l.c.wv == 8) LAUNCH(cls, k18, l.grid, l.block, l.lds, l.a, __VA_ARGS__); \
+    else if (l.c.tb == 1) LAUNCH(cls, k14, l.grid, l.block, l.lds, l.a, __VA_ARGS__); \
+    else LAUNCH(cls, k24, l.grid, l.block, l.lds, l.a, __VA_ARGS__); } while (0)
+template <bool DUMP>
+static int launch_wide_mm(Launcher &lx, int cls, const uint8_t *w, const int8_t *q, int k, int m, int rows, float *out, int32_t *dots) {
+    const WideLaunch l = wide_launch(w, q, k, m, rows, lg_segments(k) / 8);
+    LAUNCH_WIDE(cls, l, (lg_k_wide_mm<1, 8, DUMP>), (lg_k_wide_mm<1, 4, DUMP>), (lg_k_wide_mm<2, 4, DUMP>), out, dots);
+    return l.a.parts;
 }
 // Whether a prompt block reaches value rows 2 GiB and more behind a layer's first one (524288 positions at the 12B shape), where
 // lg_k_wide_attn's 32-bit addresses end.  (It fetches value rows four tiles at a time.)
@@ -1699,15 +1699,8 @@ static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, i
         pend_parts = launch_wide_mm<false>(lx, KC_O, y.wo_w, m->aq, y.qd, E, rows, m->dout, nullptr);
         pend_dout = m->dout; pend_w = y.post_attn;
         row_work(y.ffn_norm, m->hq);
-        {
-            const WideShape c = wide_shape(2 * y.nff, rows, 1);
-            const WideMm g{ y.wgu_w, (const uint8_t *)m->hq, E, 2 * y.nff, rows, (rows + 32 * c.tb - 1) / (32 * c.tb), 1 };
-            const dim3 grid(lg_wide_grid(g.m, g.nb_tiles, 1)), block(64 * c.wv);
-            const size_t lds = (size_t)c.wv * 2 * c.tb * 4096;
-            if (c.wv == 8)      LAUNCH(KC_GATEUP, (lg_k_wide_geglu<1, 8>), grid, block, lds, g, (uint8_t *)m->gq);
-            else if (c.tb == 1) LAUNCH(KC_GATEUP, (lg_k_wide_geglu<1, 4>), grid, block, lds, g, (uint8_t *)m->gq);
-            else                LAUNCH(KC_GATEUP, (lg_k_wide_geglu<2, 4>), grid, block, lds, g, (uint8_t *)m->gq);
-        }
+        const WideLaunch gu = wide_launch(y.wgu_w, m->hq, E, 2 * y.nff, rows, 1);
+        LAUNCH_WIDE(KC_GATEUP, gu, (lg_k_wide_geglu<1, 8>), (lg_k_wide_geglu<1, 4>), (lg_k_wide_geglu<2, 4>), (uint8_t *)m->gq);
         pend_parts = launch_wide_mm<false>(lx, KC_DOWN, y.wdown_w, m->gq, y.nff, E, rows, m->dout, nullptr);
         pend_dout = m->dout; pend_w = y.post_ffw; pend_os = m->ple ? nullptr : y.out_scale;
         if (!m->ple) continue;
@@ -1719,12 +1712,10 @@ static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, i
             launch_mmf<LG_HIP_MAX_ROWS>(lx, KC_PLEPROJ, pr);
             pend_parts = 1;
         } else {
-            const WideShape c = wide_shape(m->ple, rows, 1);
-            const WideMm g{ y.winp_w, (const uint8_t *)m->hq, E, m->ple, rows, (rows + 32 * c.tb - 1) / (32 * c.tb), 1 };
-            const dim3 grid(lg_wide_grid(g.m, g.nb_tiles, 1)), block(64 * c.wv);
-            const size_t lds = (size_t)c.wv * 2 * c.tb * 4096;
-            if (c.wv == 8) LAUNCH(KC_PLEGATE, (lg_k_wide_plegate<1, 8>), grid, block, lds, g, m->pmp_raw, L, nl, (uint8_t *)m->pq);
-            else           LAUNCH(KC_PLEGATE, (lg_k_wide_plegate<2, 4>), grid, block, lds, g, m->pmp_raw, L, nl, (uint8_t *)m->pq);
+            // (256 gate rows: at most 4 weight tiles x 16 activation tiles, always eight wavefronts)
+            static_assert((256 / LG_WT) * (LG_WIDE_ROWS / 32) <= 256, "lg_k_wide_plegate is built for tiles of 64 x 32 by eight wavefronts");
+            const WideLaunch g = wide_launch(y.winp_w, m->hq, E, m->ple, rows, 1);
+            LAUNCH(KC_PLEGATE, (lg_k_wide_plegate<1, 8>), g.grid, g.block, g.lds, g.a, m->pmp_raw, L, nl, (uint8_t *)m->pq);
             pend_parts = launch_wide_mm<false>(lx, KC_PLEPROJ, y.wproj_w, m->pq, m->ple, E, rows, m->dout, nullptr);
         }
         pend_dout = m->dout; pend_w = y.post_norm; pend_os = y.out_scale;
@@ -2347,8 +2338,9 @@ extern "C" int lg_hip_matmul_q4q8(const void *w, int k, int mrows, const float *
                                   int8_t *xq, float *xd, int32_t *xsum, int repeats, float *kernel_ms) {
     if (!w || !x) return fail(-1, "matmul: null input");
     const bool wide = rows > LG_HIP_MAX_ROWS && rows % LG_WIDE == 0 && rows <= LG_WIDE_ROWS;     // row tiles through the kernels of prompt blocks
-    if (rows < 1 || (rows > LG_HIP_MAX_ROWS && !wide) || !lg_hip_repacked_bytes(k, mrows) || (!wide && lds_mm(rows, k) > 160 * 1024) || (rows > LG_HIP_MAX_ROWS && !wide))
-        return fail(-2, "matmul: rows %d (1..%d, or a multiple of %d), k %d (multiple of 256, rows*k*1.25 <= 160 KiB), m %d (multiple of 8)", rows, LG_HIP_MAX_ROWS, LG_WIDE, k, mrows);
+    if (rows < 1 || (rows > LG_HIP_MAX_ROWS && !wide) || !lg_hip_repacked_bytes(k, mrows) || (!wide && lds_mm(rows, k) > 160 * 1024))
+        return fail(-2, "matmul: rows %d (1..%d, or a multiple of %d up to %d), k %d (multiple of 256; up to %d rows: rows*k*1.25 <= 160 KiB), m %d (multiple of 8)",
+                    rows, LG_HIP_MAX_ROWS, LG_WIDE, LG_WIDE_ROWS, k, LG_HIP_MAX_ROWS, mrows);
     if (lg_hip_device_count() < 1) return fail(-3, "matmul: no HIP device");
     const int nb = k / 32;
     std::vector<uint8_t> tiled(lg_hip_repacked_bytes(k, mrows));
@@ -2494,7 +2486,7 @@ static int enqueue_attention(hipStream_t st, const AttnArgs &a_in, const MergeAr
     AttnArgs a = a_in;
     a.gx = tiles; a.gz = M;                               // the grid of lg_k_attn, which reads it from its arguments
     if (attention_rows_shared(M, tiles, a.nkv, a.hd, a.seq)) {
-        if constexpr (M > 1 && M <= LG_HIP_MAX_ROWS) {
+        if constexpr (M > 1) {
             const int units = M * (a.H / a.nkv);
             const size_t l2 = a.hd == 256 ? AttnRowsGeo<256>::bytes(units) : a.hd == 128 ? AttnRowsGeo<128>::bytes(units) : AttnRowsGeo<64>::bytes(units);
             int rc = a.hd == 256 ? set_lds(lg_k_attn_rows<M, 256>, l2) : a.hd == 128 ? set_lds(lg_k_attn_rows<M, 128>, l2) : set_lds(lg_k_attn_rows<M, 64>, l2);
@@ -2506,7 +2498,7 @@ static int enqueue_attention(hipStream_t st, const AttnArgs &a_in, const MergeAr
             else                  hipLaunchKernelGGL((lg_k_attn_rows<M, 64>), grid, dim3(LG_WG), l2, st, ctl, tp, LG_ATTN_FIELDS(LG_XA, a) 0);
         }
     } else hipLaunchKernelGGL((lg_k_attn<false, 1>), dim3(tiles, a.nkv, M), dim3(LG_WG), lds, st, ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
-    if (M <= LG_HIP_MAX_ROWS && tiles >= 128 && a.hd % 64 == 0) hipLaunchKernelGGL((lg_k_attn_merge_split<M>), dim3(a.H, M, a.hd / 64), dim3(LG_WG), 0, st, ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
+    if (tiles >= 128 && a.hd % 64 == 0) hipLaunchKernelGGL((lg_k_attn_merge_split<M>), dim3(a.H, M, a.hd / 64), dim3(LG_WG), 0, st, ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
     else hipLaunchKernelGGL((lg_k_attn_merge<M>), dim3(a.H, M), dim3(LG_WG), 0, st, ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
     return 0;
 }
