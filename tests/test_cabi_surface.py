@@ -74,8 +74,8 @@ def test_ring_rows_agree_with_the_oracle(lg, ob):
 
 
 def test_attention_partials_of_a_cache_stay_within_their_budget(lg):
-    """The byte count lg_hip_kv_create asks for beside the rings, at the E4B and 12B shapes (8 verify rows): the
-    widest prompt block steps down with the cache length so that rows x heads x key tiles x (head_dim + 2) floats
+    """The most that lg_hip_kv_create asks for beside the rings, at the E4B and 12B shapes (8 verify rows): the block
+    width it is counted for steps down with the cache length so that rows x heads x key tiles x (head_dim + 2) floats
     never pass 2 GiB; the closed form is recomputed here from the returned block width."""
     import ctypes as C
     H = lg.hiplib.load_hip()

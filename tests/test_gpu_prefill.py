@@ -1,7 +1,7 @@
-"""GPU parity of the wide (32-row) blocks that prefill runs on the matrix cores
-(v_mfma_i32_32x32x32_i8): the isolated matmul with 32 activation rows against the oracle
-(int32 block dots bit-exact, f32 bit-identical in this build's order), and whole prompts whose
-cache rows and next-token logits must equal the position-by-position oracle."""
+"""GPU parity of the blocks that prompts run in (lg_wide.h: v_mfma_scale_f32_32x32x64_f8f6f4 on 6-bit floats): the isolated
+matmul with 32 activation rows against the oracle (integer block dots exact, f32 bit-identical in this build's order), and
+whole prompts whose cache rows and next-token logits must equal the position-by-position oracle; and the memory that prompt
+blocks take."""
 import ctypes as C
 
 import numpy as np
@@ -33,10 +33,9 @@ def test_wide_matmul_matches_oracle(lg, ob, gpu_required, m, k):
 @pytest.mark.parametrize("name,n_prompt", [("tiny", 97), ("tiny_full", 200), ("tiny", 32), ("tiny_full", 427), ("tiny", 128), ("tiny_full_f32", 200), ("tiny_full_f16", 171),
                                            ("tiny", 1100), ("tiny_full", 1061)])
 def test_wide_prefill_leaves_the_same_cache_and_logits(lg, ob, gpu_required, model_path, name, n_prompt):
-    """A prompt through 512-row blocks (caches of 1024 positions and more; the two long prompts also wrap the
-    640-row sliding rings), 128-row blocks, 32-row blocks and a verify-width tail against one oracle forward per position:
-    every cache row identical, the logits of the next position identical; and identical to the same
-    prompt pushed through 8-row blocks only."""
+    """A prompt in blocks of up to 512 rows (caches of 1024 positions and more; the two long prompts also wrap the 640-row sliding
+    rings) or 128 rows and one block of any width for the rest, against one oracle forward per position: every cache row
+    identical, the logits of the next position identical; and identical to the same prompt pushed through 8-row blocks only."""
     path, spec = model_path(name)
     check_wide_prefill(lg, ob, path, spec, name, n_prompt)
 
