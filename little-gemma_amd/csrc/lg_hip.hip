@@ -1464,7 +1464,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         }
         if (!merged_o) {   // attention output projection
             MmArgs a{ y.wo, y.qd, E, m->dout, m->aq, nullptr };
-            pend_parts = launch_mm<M, false>(lx, KC_O, a);      // (four slabs for a wide block when n_head * head_dim > 4096)
+            pend_parts = launch_mm<M, false>(lx, KC_O, a);
             pend_dout = m->dout; pend_w = y.post_attn; pend_os = nullptr;
         }
         {   // feed-forward: gate/up + GeGLU, then down
