@@ -823,17 +823,21 @@ __global__ __launch_bounds__(LG_WG) void lg_k_attn_rows(const StepCtl *ctl, int 
     }
 }
 
-// lg_k_attn_merge for rows with very many tiles: one workgroup of four wavefronts per (head, row, 64 dims).  The
+// lg_k_attn_merge for rows with very many tiles: one workgroup of NW wavefronts per (head, row, 64 dims).  The
 // merge is one fma chain over the tiles ascending, and walked by a single wavefront its time is the instruction issue
-// of 2 loads + 2 fma per tile, tile after tile.  Here the tiles go in rounds of 256: wavefront w requests the 64
-// partials of tiles 64w..64w+63 of the round at once (all four wavefronts' loads in flight together) while the
+// of 2 loads + 2 fma per tile, tile after tile.  Here the tiles go in rounds of 64*NW: wavefront w requests the 64
+// partials of tiles 64w..64w+63 of the round at once (all wavefronts' loads in flight together) while the
 // workgroup computes the round's weights exp(m_t - M) into LDS; then the chain passes through the wavefronts in
 // order, each running its 64 fma back to back from registers and handing (L, o) to the next through LDS.  Same
 // order, same bits: weights exp(m_t - M), L and the output as fma chains over the tiles ascending, divide, q8.
-template <int M>
-__global__ __launch_bounds__(LG_WG) void lg_k_attn_merge_split(const StepCtl *ctl, LG_MERGE_FIELDS(LG_XP, _) int p_end_) {
+// NW: a round is a memory round trip and then its turns, so caches that hold more tiles take more wavefronts (merge_waves in
+// lg_hip.hip).  8 rows, 8 heads of 256, 626 tiles: four wavefronts in 3 rounds 21.6 us, sixteen in one 14.6; 5 rows, 16 heads, 257
+// tiles (a second round for the last of them): 13.0 -> 9.5 us with eight.
+template <int M, int NW>
+__global__ __launch_bounds__(64 * NW, 4) void lg_k_attn_merge_split(const StepCtl *ctl, LG_MERGE_FIELDS(LG_XP, _) int p_end_) {
     MergeArgs a; LG_MERGE_FIELDS(LG_XI, a)
-    __shared__ float wts[256], pls[256], hand[2][64], wmx[4];
+    constexpr int U = 64, WG = 64 * NW;
+    __shared__ __align__(16) float wts[WG], pls[WG], hand[2][64], wmx[NW];
     const int head = blockIdx.x, j = blockIdx.y, hd = a.hd, qd = a.H * hd, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int d = blockIdx.z * 64 + lane;                     // hd is a multiple of 64
     const int pos = ctl->pos + a.pos_off, pj = pos + j;
@@ -841,13 +845,13 @@ __global__ __launch_bounds__(LG_WG) void lg_k_attn_merge_split(const StepCtl *ct
     const int lo = (lg_win_start(pj, a.window) >> 5) - first, hi = (pj >> 5) - first;
     const size_t base = ((size_t)j * a.H + head) * a.tiles_max + lo;
     const int nt = hi - lo + 1;
-    constexpr int U = 64;
     float pa[U];
     // (buffer loads: the row's partials as the base in scalar registers, the lane's dim as the lane offset, the tile's
     // offset in a scalar register; a flat load each cost a dozen vector instructions of 64-bit address arithmetic)
     const __amdgpu_buffer_rsrc_t rp = lg_buffer_rsrc(a.pacc + base * hd);
     auto fetch = [&](int t0_) {                               // tiles t0 .. t0+63 of this row (past the end: the last one again)
         const int t0 = __builtin_amdgcn_readfirstlane(t0_);
+        if (NW > 4 && t0 >= nt) return;                       // (a wavefront without a tile in this round)
         #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int n = t0 + u < nt ? t0 + u : nt - 1;
@@ -856,31 +860,44 @@ __global__ __launch_bounds__(LG_WG) void lg_k_attn_merge_split(const StepCtl *ct
     };
     fetch(wave * U);                                          // the partials do not depend on the weights
     float mx = -INFINITY;
-    for (int n = threadIdx.x; n < nt; n += LG_WG) mx = fmaxf(mx, a.pm[base + n]);
+    for (int n = threadIdx.x; n < nt; n += WG) mx = fmaxf(mx, a.pm[base + n]);
     mx = lg_max_n(mx, 64);
     if (lane == 0) wmx[wave] = mx;
     __syncthreads();
-    mx = fmaxf(fmaxf(wmx[0], wmx[1]), fmaxf(wmx[2], wmx[3]));
+    #pragma unroll
+    for (int w = 0; w < NW; ++w) mx = fmaxf(mx, wmx[w]);
     float L = 0.0f, o = 0.0f;
-    for (int r0 = 0; r0 < nt; r0 += 4 * U) {
+    for (int r0 = 0; r0 < nt; r0 += WG) {
         if (r0 > 0) fetch(r0 + wave * U);
         {   // the round's weights and sums (one tile per thread)
             const int n = r0 + (int)threadIdx.x;
             if (n < nt) { wts[threadIdx.x] = lg_expf(a.pm[base + n] - mx); pls[threadIdx.x] = a.pl[base + n]; }
         }
         __syncthreads();
-        #pragma unroll
-        for (int turn = 0; turn < 4; ++turn) {
-            if (wave == turn && r0 + turn * U < nt) {
+        for (int turn = 0; turn < NW && r0 + turn * U < nt; ++turn) {
+            if (wave == turn) {
                 if (r0 + turn > 0) { L = hand[0][lane]; o = hand[1][lane]; }
+                // weights and sums four tiles at a time, requested ahead of their fma (tile by tile under a guard a turn
+                // was 64 trips to LDS: 2 us of its time)
+                constexpr int AHEAD = 2;
+                float4 w4[AHEAD], l4[AHEAD];
                 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    if (r0 + turn * U + u < nt) {             // (a guard, not a break: the partials stay in registers)
-                        const float wn = wts[turn * U + u];
-                        L = lg_fmaf(pls[turn * U + u], wn, L);
-                        o = lg_fmaf(pa[u], wn, o);
+                for (int g = 0; g < AHEAD; ++g) { w4[g] = *(const float4 *)(wts + turn * U + 4 * g); l4[g] = *(const float4 *)(pls + turn * U + 4 * g); }
+                auto chain = [&](auto full) {
+                    #pragma unroll
+                    for (int g = 0; g < U / 4; ++g) {
+                        const float wv[4] = { w4[g % AHEAD].x, w4[g % AHEAD].y, w4[g % AHEAD].z, w4[g % AHEAD].w };
+                        const float lv[4] = { l4[g % AHEAD].x, l4[g % AHEAD].y, l4[g % AHEAD].z, l4[g % AHEAD].w };
+                        if (g + AHEAD < U / 4) { w4[g % AHEAD] = *(const float4 *)(wts + turn * U + 4 * (g + AHEAD)); l4[g % AHEAD] = *(const float4 *)(pls + turn * U + 4 * (g + AHEAD)); }
+                        #pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float Ln = lg_fmaf(lv[i], wv[i], L), on = lg_fmaf(pa[4 * g + i], wv[i], o);
+                            const bool in = full || r0 + turn * U + 4 * g + i < nt;
+                            L = in ? Ln : L; o = in ? on : o;
+                        }
                     }
-                }
+                };
+                if (r0 + (turn + 1) * U <= nt) chain(std::true_type{}); else chain(std::false_type{});
                 hand[0][lane] = L; hand[1][lane] = o;
             }
             __syncthreads();

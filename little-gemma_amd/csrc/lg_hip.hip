@@ -1106,6 +1106,16 @@ static int attention_rows_tp(int tiles, int nkv) {
     return tp < 1 ? 1 : tp > 4 ? 4 : tp;
 }
 
+// wavefronts of lg_k_attn_merge_split: a round of 64 tiles each covers the cache's tiles, while the CUs hold all workgroups
+// at once (128 registers a wavefront: one workgroup of 16 wavefronts per CU, two of eight)
+static int merge_waves(int tiles, int wgs) {
+    return tiles <= 256 ? 4 : tiles <= 512 || wgs > cu_count() ? 8 : 16;
+}
+#define MERGE_SPLIT(M, go, H, hd, tiles) do { const dim3 grid_(H, M, (hd) / 64); const int nw_ = merge_waves(tiles, (H) * (M) * ((hd) / 64)); \
+    if (nw_ == 4)      go((lg_k_attn_merge_split<M, 4>), grid_, dim3(256)); \
+    else if (nw_ == 8) go((lg_k_attn_merge_split<M, 8>), grid_, dim3(512)); \
+    else               go((lg_k_attn_merge_split<M, 16>), grid_, dim3(1024)); } while (0)
+
 // the XCD-partitioned feed-forward launch: 256 workgroups of 512 threads, the instantiation of the shape's class
 template <int M>
 static void launch_xffn(Launcher &lx, const XffnArgs &a, int cls) {
@@ -1459,8 +1469,11 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 launch_merge_o(lx, f);
                 pend_dout = m->dout; pend_w = y.post_attn; pend_os = nullptr; pend_parts = 8;
             } else
-            if (tiles >= 128 && y.hd % 64 == 0) LAUNCH(KC_MERGE, (lg_k_attn_merge_split<M>), dim3(H, M, y.hd / 64), dim3(LG_WG), 0, m->ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
-            else LAUNCH(KC_MERGE, (lg_k_attn_merge<M>), dim3(H, M), dim3(LG_WG), 0, m->ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
+            if (tiles >= 128 && y.hd % 64 == 0) {
+#define GO(k, grid, block) LAUNCH(KC_MERGE, k, grid, block, 0, m->ctl, LG_MERGE_FIELDS(LG_XA, g) 0)
+                MERGE_SPLIT(M, GO, H, y.hd, tiles);
+#undef GO
+            } else LAUNCH(KC_MERGE, (lg_k_attn_merge<M>), dim3(H, M), dim3(LG_WG), 0, m->ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
         }
         if (!merged_o) {   // attention output projection
             MmArgs a{ y.wo, y.qd, E, m->dout, m->aq, nullptr };
@@ -2498,8 +2511,11 @@ static int enqueue_attention(hipStream_t st, const AttnArgs &a_in, const MergeAr
             else                  hipLaunchKernelGGL((lg_k_attn_rows<M, 64>), grid, dim3(LG_WG), l2, st, ctl, tp, LG_ATTN_FIELDS(LG_XA, a) 0);
         }
     } else hipLaunchKernelGGL((lg_k_attn<false, 1>), dim3(tiles, a.nkv, M), dim3(LG_WG), lds, st, ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
-    if (tiles >= 128 && a.hd % 64 == 0) hipLaunchKernelGGL((lg_k_attn_merge_split<M>), dim3(a.H, M, a.hd / 64), dim3(LG_WG), 0, st, ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
-    else hipLaunchKernelGGL((lg_k_attn_merge<M>), dim3(a.H, M), dim3(LG_WG), 0, st, ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
+    if (tiles >= 128 && a.hd % 64 == 0) {
+#define GO(k, grid, block) hipLaunchKernelGGL(HIP_KERNEL_NAME(k), grid, block, 0, st, ctl, LG_MERGE_FIELDS(LG_XA, g) 0)
+        MERGE_SPLIT(M, GO, a.H, a.hd, tiles);
+#undef GO
+    } else hipLaunchKernelGGL((lg_k_attn_merge<M>), dim3(a.H, M), dim3(LG_WG), 0, st, ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
     return 0;
 }
 

@@ -266,6 +266,24 @@ def test_attention_other_geometries(lg, ob, gpu_required, H, KV, hd, rows):
     assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("H,KV,hd,rows,tiles,off", [
+    (4, 1, 64, 2, 256, 31), (4, 1, 64, 3, 257, 0), (4, 1, 64, 8, 512, 17), (4, 2, 64, 1, 513, 0), (4, 1, 128, 5, 576, 31), (2, 1, 64, 4, 1024, 30),
+    (2, 1, 64, 4, 1025, 3), (16, 8, 256, 8, 514, 9)])
+def test_attention_over_many_tiles(lg, ob, gpu_required, H, KV, hd, rows, tiles, off):
+    """Lengths around the borders of the ordered merge's builds of 4, 8 and 16 wavefronts (up to 256, 512, more tiles; 8 where more
+    workgroups than CUs take part), whole and partial rounds and turns of 64 tiles, against the oracle's one chain: same bits."""
+    rng = np.random.default_rng(tiles * 8 + rows)
+    pos = (tiles - 1) * 32 + off - (rows - 1)                 # the last row's last slot of the last tile is `off`
+    seq = tiles * 32
+    kc = rng.normal(0, 1, (seq, KV * hd)).astype(np.float16).view(np.uint16)
+    vc = rng.normal(0, 1, (seq, KV * hd)).astype(np.float16).view(np.uint16)
+    q = (rng.normal(0, 1, (rows, H * hd)) * 0.1).astype(np.float32)
+    print(f"attention H={H} KV={KV} hd={hd} rows={rows} tiles={tiles} off={off}", flush=True)
+    out, _ = lg.hiplib.attention(q, kc, vc, H, KV, hd, 0, pos)
+    want = oracle_attention(ob, q, kc, vc, H, KV, hd, 0, pos)
+    assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
+
+
 def test_bad_arguments_are_refused(lg, gpu_required):
     rng = np.random.default_rng(1)
     with pytest.raises(lg.hiplib.HipError):
