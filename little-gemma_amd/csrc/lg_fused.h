@@ -494,106 +494,73 @@ __global__ __launch_bounds__(320, 2) void lg_k_mm_kq(LG_MM_FIELDS(LG_XP, _) int 
 
 // ---------------------------------------------------------------------------------------------
 // Attention tiles of a verify block for layers with many tiles (long global contexts, wide sliding windows):
-// one workgroup per (tile, kv head) serves ALL rows of the block against one staged K/V tile, where lg_k_attn
-// runs a workgroup per row and stages every tile once per row.  FQ = false: the queries arrive normed and rotated
+// a workgroup serves ALL rows of the block against its tiles, where lg_k_attn runs a workgroup per row and stages
+// every tile once per row.  FQ = false: the queries arrive normed and rotated
 // (lg_k_qkv_post has run and has written the block's K/V rows to the cache).  FQ = true: the kernel does that work
 // itself from the raw projections, one launch less per layer: every workgroup norms and rotates the M*G queries of
-// its kv head (a wavefront per query, written in the staged order), and the one workgroup whose tile holds rows of
-// the block builds those K/V rows straight into its LDS tile and stores them to the cache (K row r by wavefront
+// its kv head (a wavefront per query), and the workgroup whose tiles hold rows of
+// the block builds those K/V rows into LDS and stores them to the cache (K row r by wavefront
 // r % 4, V row r by wavefront 3 - r % 4; the ring has spare rows, so no row another workgroup reads is overwritten).
 // Same arithmetic and order as
 // lg_k_attn: score = (a0+a1)+(a2+a3) over four fma chains, tile max / exp / 32-lane tree sum, value accumulation
 // over the slots ascending; the partials go to the same slots and lg_k_attn_merge finishes them.
 //
-// A unit is one (row, query head) pair, M*G of them; a wavefront takes the units wave, wave + 4, ... three at a
-// time, so that one LDS read of a K (V) row serves three units and 6 (12) independent fma chains are in flight.
-// K is staged in reader order (the lane of key slot sl and chain pair hf finds its hd/4 dwords as consecutive
-// 16-byte units); the queries are read 16 bytes at a time, the same address in all lanes of a half.  Every slot of
-// a tile goes through the value chains: slots outside a row's keys have exponential zero and zeroed or finite
-// values, and fma(0, v, acc) is acc for every acc that a chain started at +0 can hold.
-//
-// A workgroup takes `tp` consecutive tiles; the next tile's rows are requested into registers before the current
-// tile is computed, so the memory latency of all tiles but the first is covered.
-
-// fmaf(x, (float)h, acc) with h the low (high) f16 half of a packed pair: one instruction; the conversion is exact
-// and the sum rounds once, as the two-instruction form does.  The compiler picks this instruction by itself when a
-// converted value feeds one fma; written out here because each key/value element feeds one fma per unit.
-__device__ __forceinline__ float lg_fma_hlo(float x, uint32_t hp, float acc) {
-    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel_hi:[0,1,0]" : "+v"(acc) : "v"(x), "v"(hp));
-    return acc;
-}
-__device__ __forceinline__ float lg_fma_hhi(float x, uint32_t hp, float acc) {
-    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "+v"(acc) : "v"(x), "v"(hp));
-    return acc;
-}
-
+// A unit is one (row, query head) pair, M*G of them, in groups of 16.  Both products run on v_mfma_f32_16x16x1_4b_f32,
+// one fma per output and step as in lg_k_wide_attn: the four blocks of a score step are its four chains, those of a value
+// step (one slot) are four runs of 16 dims.  A workgroup is two pairs of wavefronts.  Up to 16 units: a pair to a tile, two
+// tiles to a workgroup; more: a pair to a unit group of one tile.  The wavefronts of a pair take 16 keys each, then half of
+// the dims each.  K and V go from the cache straight into registers in operand order (16 bytes of a K row by four lanes,
+// dealt to the chains by lg_deal4; a run of a value row, one slot after another), all requested at the start, so the tile's
+// memory round trip passes under the preparation of the queries; LDS holds only queries, weights and the block's own rows.
+// Bound by its products (32 cycles each, 128 to a wavefront and tile) and about 500 vector instructions beside them, which run
+// one after the other; without the tile's loads and the partials' stores it takes 28 of its 33 us.  On the vector units, every K and V
+// row through LDS and three units to a read, LDS reads bounded it.  8 rows of 8 heads over 2 at 20011 keys 61 -> 33 us, 5 rows of
+// 16 over 8 at 8192 keys 42 -> 31, at 2048 keys of 8 over 2 15.2 -> 14.2; a 1024-key window of 16 over 8: 12.3 -> 13.1 (two
+// tiles to a workgroup, 136 workgroups).
+// Slots outside a row's keys have weight zero and zeroed values (or ones that another row of the block sees), and
+// fma(0, v, acc) is acc for every acc that a chain started at +0 can hold.
 template <int HD>
 struct AttnRowsGeo {
-    static constexpr int KSD = HD / 2 + 4;                    // dwords per staged K row (16-byte reads of 8 slots cover all banks)
-    static constexpr int VST = HD + 8;                        // halves per staged V row
-    static size_t bytes(int units, bool fq = false) {         // fq: a vector of staging per wavefront for the rotary
-        return (size_t)units * HD * 4 + (size_t)32 * KSD * 4 + (size_t)32 * VST * 2 + (size_t)units * 32 * 4 + (fq ? (size_t)(LG_WG / 64) * HD * 4 : 0);
+    static constexpr int QST = HD + 4;                        // floats per staged query: [chain][HD/4], off the bank period
+    static constexpr int EST = 36;                            // floats per unit's weights of a tile
+    static size_t bytes(int units, bool fq) {         // fq: the block's K and V rows, and a vector of staging per wavefront for the rotary
+        return (size_t)((units + 15) / 16) * 16 * QST * 4 + (size_t)2 * 16 * EST * 4 + (fq ? (size_t)2 * LG_HIP_MAX_ROWS_DEV * HD * 2 + (size_t)(LG_WG / 64) * HD * 4 : 0);
     }
 };
+// tiles a workgroup takes at a time
+__host__ __device__ static inline int lg_attn_rows_tiles(int units) { return units <= 16 ? 2 : 1; }
 template <int M, int HD, bool FQ = false>
-__global__ __launch_bounds__(LG_WG) void lg_k_attn_rows(const StepCtl *ctl, int tp, LG_ATTN_FIELDS(LG_XP, _) int p_end_) {
+__global__ __launch_bounds__(LG_WG, 2) void lg_k_attn_rows(const StepCtl *ctl, LG_ATTN_FIELDS(LG_XP, _) int p_end_) {
     AttnArgs a; LG_ATTN_FIELDS(LG_XI, a)
     using Geo = AttnRowsGeo<HD>;
     extern __shared__ __align__(16) unsigned char smem[];
-    const int G = a.H / a.nkv, units = M * G;
-    float *qs = (float *)smem;                                // [unit][hf][HD/2]: element i at hf = (i%4)/2, 2*(i/4) + i%2
-    uint32_t *kt = (uint32_t *)(qs + (size_t)units * HD);     // [32][KSD]: row sl = [hf][HD/4 dwords]
-    uint16_t *vt = (uint16_t *)(kt + 32 * Geo::KSD);          // [32][VST]
-    float *es = (float *)(vt + 32 * Geo::VST);                // [unit][32]
-    float *hv = es + (size_t)units * 32;                      // FQ: [wavefront][HD] staging of the rotary
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    __shared__ float mxs[4][16], lsum[4][16];                 // a wavefront's maxima and sums over its 16 keys
+    const int G = a.H / a.nkv, units = M * G, ng = (units + 15) >> 4;
+    float *qs = (float *)smem;                                // [unit][c][HD/4]: element i at c = i % 4, i / 4
+    float *es = qs + (size_t)ng * 16 * Geo::QST;              // [pair][unit][EST]
+    uint16_t *nk = (uint16_t *)(es + 2 * 16 * Geo::EST);      // FQ: the block's K rows, then its V rows, [M][HD] each
+    uint16_t *nv = nk + (size_t)LG_HIP_MAX_ROWS_DEV * HD;
+    float *hv = (float *)(nv + (size_t)LG_HIP_MAX_ROWS_DEV * HD);       // FQ: [wavefront][HD] staging of the rotary
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), pair = wave >> 1, half = wave & 1;
+    const int n = lane & 15, c = lane >> 4;
     const int kvh = blockIdx.y;
     const int pos0 = ctl->pos + a.pos_off, plast = pos0 + M - 1;
     // FQ: positions tnew..plast are rows of the block itself (none when the layer reads another layer's cache)
     const int tnew = (FQ && a.kcw) ? ctl->pos : 0x7FFFFFFF;
     const int start0 = lg_win_start(pos0, a.window), first = start0 >> 5, last = plast >> 5;
-    const int b0 = blockIdx.x * tp;                           // tiles first + b0 .. first + b0 + tp - 1
-    if (first + b0 > last) return;                            // no row of the block has keys here
-    constexpr int U4R = HD / 8;                               // 16-byte units per K/V row
-    constexpr int KL = (32 * U4R + LG_WG - 1) / LG_WG;        // 16-byte units of K (and of V) per thread
-    static_assert(32 * U4R % LG_WG == 0 || 32 * U4R < LG_WG, "tile staging assumes whole passes");
-    uint4 kq[KL], vq[KL];
-    auto fetch = [&](int bx) {
-        const int r0 = ((first + bx) << 5) % a.seq;
-        #pragma unroll
-        for (int u = 0; u < KL; ++u) {
-            const int idx = min((int)threadIdx.x + u * LG_WG, 32 * U4R - 1), row = idx / U4R, u4 = idx - row * U4R;
-            int rr = r0 + row; if (rr >= a.seq) rr -= a.seq;
-            const size_t go = (size_t)rr * a.kv_dim + (size_t)kvh * HD + u4 * 8;
-            kq[u] = a.kc4s(go); vq[u] = a.vc4s(go);
-        }
-    };
-    auto stash = [&](int bx) {
-        // slots outside the keys of every row of the block are zeroed (their exponentials are zero, and zero times
-        // a finite value leaves the sums as they are; stale bits that read as infinities would not)
-        const int t0 = (first + bx) << 5, slo = start0 - t0, shi = plast - t0;
-        #pragma unroll
-        for (int u = 0; u < KL; ++u) {
-            const int idx = (int)threadIdx.x + u * LG_WG, row = idx / U4R, u4 = idx - row * U4R;
-            if (32 * U4R < LG_WG && idx >= 32 * U4R) continue;
-            if (FQ && t0 + row >= tnew && row <= shi) continue;               // a row of the block: built below, not in the cache yet
-            const uint32_t mk = (row >= slo && row <= shi) ? 0xFFFFFFFFu : 0u;
-            uint32_t *d = kt + row * Geo::KSD + 2 * u4;
-            *(uint2 *)d = make_uint2(kq[u].x & mk, kq[u].z & mk);             // chains 0,1 of two groups of four dims
-            *(uint2 *)(d + HD / 4) = make_uint2(kq[u].y & mk, kq[u].w & mk);  // chains 2,3
-            *(uint4 *)(vt + row * Geo::VST + u4 * 8) = make_uint4(vq[u].x & mk, vq[u].y & mk, vq[u].z & mk, vq[u].w & mk);
-        }
-    };
+    // the workgroup's tiles: tw from first + tw * b on, b = blockIdx.x, blockIdx.x + gx, ...
+    const int tw = ng == 1 ? 2 : 1, gx = a.gx, b0 = blockIdx.x, nb = (last - first + tw) / tw;
+    if (b0 >= nb) return;                                     // no row of the block has keys here
+    auto mine = [&](int t) { return (((t >> 5) - first) / tw) % gx == b0; };      // position t lies in a tile of this workgroup
+
     constexpr int JOBS = 2 * ((M + 3) / 4);                   // FQ: K and V rows of the block one wavefront may have to build
     constexpr int QBATCH = 4;                                 // FQ: queries one wavefront prepares at a time
     HeadVec<1> hj[FQ ? JOBS : 1], hq[FQ ? QBATCH : 1], wk, wq;
     RopeVals<1> rv;
+    const bool any = FQ && tnew <= plast && (mine(tnew) || mine(plast));         // this workgroup's tiles hold rows of the block (at most two tiles do)
     if constexpr (FQ) {
         // What the preparation reads is requested ahead of the tile (loads return in order): the block's projections
         // come from the cache levels, the tile from memory, so the queries are prepared while the tile is on its way.
-        // Raw rows of the block that fall into this workgroup's tiles are requested here too and used when their tile
-        // is staged.
-        const int tlo = (first + b0) << 5, thi = ((first + b0 + tp) << 5) - 1;
         rv = lg_rope_load<1>(a.rope_tab, a.rope_ff, HD);
         wq = lg_head_load<1>(a.q_norm, HD);
         #pragma unroll
@@ -601,19 +568,43 @@ __global__ __launch_bounds__(LG_WG) void lg_k_attn_rows(const StepCtl *ctl, int 
             const int u = wave + b * (LG_WG / 64) < units ? wave + b * (LG_WG / 64) : min(wave, units - 1), j = u / G, g = u - j * G;
             hq[b] = lg_head_load<1>(a.qkv + (size_t)j * a.ld + (size_t)(kvh * G + g) * HD, HD);
         }
-        const bool any = tnew <= plast && plast >= tlo && tnew <= thi;
         wk = lg_head_load<1>(any ? a.k_norm : a.q_norm, HD);  // (no K rows to build: k_norm may not exist)
         #pragma unroll
         for (int u = 0; u < JOBS; ++u) {                      // first half of the slots: K rows wave, wave+4; second half: V rows 3-wave, 7-wave
             const bool isv = u >= JOBS / 2;
             const int r = (isv ? 3 - wave : wave) + 4 * (u % (JOBS / 2)), t = tnew + r;
-            if (any && r < M && t >= tlo && t <= thi) hj[u] = lg_head_load<1>(a.qkv + (size_t)r * a.ld + (isv ? a.v_off : a.k_off) + (size_t)kvh * HD, HD);
+            if (any && r < M && mine(t)) hj[u] = lg_head_load<1>(a.qkv + (size_t)r * a.ld + (isv ? a.v_off : a.k_off) + (size_t)kvh * HD, HD);
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    fetch(b0);
+    // a tile: this lane's key (K row, 64-byte pieces by four lanes) and its dims of every slot's value row
+    constexpr int NS = HD / 32, NK = HD >= 128 ? HD / 128 : 1;          // pieces of a K row; value products per slot and wavefront
+    uint4 kw[NS];
+    uint32_t vw[32];
+    const int vd = (HD >= 128 ? half * (HD / 2) : 0) + NK * lane;       // this lane's first dim (64-wide heads: both wavefronts all of them)
+    auto tile_of = [&](int b) { const int t = first + b * tw + (ng == 1 ? pair : 0); return t <= last ? t : last; };
+    // (a tile lies within the ring in one piece: a ring is a multiple of 32 rows, or as long as the positions go.  Rows past its
+    // end are no keys of any row: the last row again, and zeros.)
+    auto fetch_k = [&](int b) {
+        const int rr = (tile_of(b) << 5) % a.seq + 16 * half + n;
+        const size_t ko = (size_t)(rr < a.seq ? rr : a.seq - 1) * a.kv_dim + (size_t)kvh * HD + c * 8;
+        #pragma unroll
+        for (int s = 0; s < NS; ++s) kw[s] = a.kc4(ko + 32 * s);
+    };
+    auto fetch_v = [&](int b) {                               // buffer loads: the slot's row in a scalar register
+        const int r0 = (tile_of(b) << 5) % a.seq, vrow = a.kv_dim * 2, left = a.seq - r0;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)(a.vc + (size_t)r0 * a.kv_dim), 0, (left < 32 ? left : 32) * vrow, 0x00020000);
+        const int vo = (kvh * HD + vd) * 2;
+        #pragma unroll
+        for (int s = 0; s < 32; ++s) {
+            if constexpr (NK == 2) vw[s] = __builtin_amdgcn_raw_buffer_load_b32(rs, vo, s * vrow, 0);
+            else vw[s] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, vo, s * vrow, 0);
+        }
+    };
+    fetch_k(b0);
+    fetch_v(b0);
+    __builtin_amdgcn_sched_barrier(0);
     if constexpr (FQ) {
-        __builtin_amdgcn_sched_barrier(0);
         // a batch in stages, so that the sums and the rotary of its queries overlap: norms of all, each into its own
         // slot of qs in natural order; all rotary pairs read back; then the slots rewritten in the staged order
         // (a unit past the last repeats the batch's first one, a slot of this wavefront, and stores nothing)
@@ -631,13 +622,13 @@ __global__ __launch_bounds__(LG_WG) void lg_k_attn_rows(const StepCtl *ctl, int 
             for (int b = 0; b < QBATCH; ++b) nq[b] = lg_head_norm<1>(hq[b], wq, true, HD, a.eps);
             #pragma unroll
             for (int b = 0; b < QBATCH; ++b)
-                if (4 * lane < HD) *(float4 *)(qs + (size_t)unit_of(base, b) * HD + 4 * lane) = nq[b].x[0];
+                if (4 * lane < HD) *(float4 *)(qs + (size_t)unit_of(base, b) * Geo::QST + 4 * lane) = nq[b].x[0];
             lg_wave_lds_sync();
             float lo[QBATCH][2], hi[QBATCH][2];
             #pragma unroll
             for (int b = 0; b < QBATCH; ++b) {
                 const int u = unit_of(base, b), j = u / G;
-                const float *vec = qs + (size_t)u * HD;
+                const float *vec = qs + (size_t)u * Geo::QST;
                 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
                     const int p = min(lane + 64 * i, HD / 2 - 1);
@@ -652,19 +643,52 @@ __global__ __launch_bounds__(LG_WG) void lg_k_attn_rows(const StepCtl *ctl, int 
             #pragma unroll
             for (int b = 0; b < QBATCH; ++b) {
                 const int u = base + b * (LG_WG / 64);
-                float *qd = qs + (size_t)unit_of(base, b) * HD;
+                float *qd = qs + (size_t)unit_of(base, b) * Geo::QST;
                 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
                     const int p = lane + 64 * i, p1 = p + HD / 2;
                     if (u >= units || p >= HD / 2) continue;
-                    // element i sits at hf = (i%4)/2, 2*(i/4) + i%2
-                    qd[((p & 3) >> 1) * (HD / 2) + 2 * (p >> 2) + (p & 1)] = lo[b][i];
-                    qd[((p1 & 3) >> 1) * (HD / 2) + 2 * (p1 >> 2) + (p1 & 1)] = hi[b][i];
+                    qd[(p & 3) * (HD / 4) + (p >> 2)] = lo[b][i];
+                    qd[(p1 & 3) * (HD / 4) + (p1 >> 2)] = hi[b][i];
                 }
             }
             lg_wave_lds_sync();
         }
-    } else {   // the queries, once per workgroup (their loads follow the first tile's before any store)
+        if (any) {                                            // the rows of the block in the workgroup's tiles
+            float *vec = hv + (size_t)wave * HD;
+            HeadVec<1> nr[JOBS];
+            bool on[JOBS];
+            #pragma unroll
+            for (int u = 0; u < JOBS; ++u) {                  // the norms of all of them first: their sums overlap
+                const bool isv = u >= JOBS / 2;
+                const int r = (isv ? 3 - wave : wave) + 4 * (u % (JOBS / 2)), t = tnew + r;
+                on[u] = r < M && mine(t);
+                if (on[u]) nr[u] = lg_head_norm<1>(hj[u], wk, !isv, HD, a.eps);
+            }
+            #pragma unroll
+            for (int u = 0; u < JOBS; ++u) {
+                const bool isv = u >= JOBS / 2;
+                const int r = (isv ? 3 - wave : wave) + 4 * (u % (JOBS / 2)), t = tnew + r;
+                if (!on[u]) continue;
+                const size_t coff = (size_t)(t % a.seq) * a.kv_dim + (size_t)kvh * HD;
+                if (isv) {                                    // V: no rotary, straight from the registers
+                    if (4 * lane < HD) {
+                        const uint2 h4 = make_uint2((uint32_t)lg_f2h(nr[u].x[0].x) | ((uint32_t)lg_f2h(nr[u].x[0].y) << 16),
+                                                    (uint32_t)lg_f2h(nr[u].x[0].z) | ((uint32_t)lg_f2h(nr[u].x[0].w) << 16));
+                        *(uint2 *)(nv + r * HD + 4 * lane) = h4;
+                        *(uint2 *)(a.vcw + coff + 4 * lane) = h4;
+                    }
+                } else {
+                    uint16_t *row = nk + r * HD, *crow = a.kcw + coff;
+                    lg_head_rope<1>(nr[u], HD, t, rv, vec, [&](int p, float lo, float hi) {
+                        const uint16_t hl = lg_f2h(lo), hh = lg_f2h(hi);
+                        row[p] = hl; row[p + HD / 2] = hh;
+                        crow[p] = hl; crow[p + HD / 2] = hh;
+                    });
+                }
+            }
+        }
+    } else {   // the queries, once per workgroup
         constexpr int QB = 4;                                 // float4 of query per thread and pass
         const int nq4 = units * (HD / 4);
         for (int base = 0; base < nq4; base += QB * LG_WG) {
@@ -680,145 +704,129 @@ __global__ __launch_bounds__(LG_WG) void lg_k_attn_rows(const StepCtl *ctl, int 
                 const int idx = base + (int)threadIdx.x + i * LG_WG;
                 if (idx < nq4) {
                     const int u = idx / (HD / 4), g4 = idx - u * (HD / 4);
-                    float *qd = qs + (size_t)u * HD + 2 * g4;
-                    *(float2 *)qd = make_float2(qreg[i].x, qreg[i].y);
-                    *(float2 *)(qd + HD / 2) = make_float2(qreg[i].z, qreg[i].w);
+                    float *qd = qs + (size_t)u * Geo::QST + g4;
+                    qd[0] = qreg[i].x; qd[HD / 4] = qreg[i].y; qd[2 * (HD / 4)] = qreg[i].z; qd[3 * (HD / 4)] = qreg[i].w;
                 }
             }
         }
     }
-    constexpr int NWV = LG_WG / 64, UB = 3;
-    for (int i = 0; i < tp; ++i) {
-        const int bx = b0 + i, n = first + bx, t0 = n << 5;
-        if (n > last) break;
-        if (i > 0) __syncthreads();                           // the previous tile has been read by every wavefront
-        if constexpr (FQ) {                                   // rows of the block in this tile: built while the tile is on its way (stash leaves their slots alone)
-            if (tnew <= plast && tnew <= t0 + 31 && plast >= t0) {            // this tile holds rows of the block
-                float *vec = hv + (size_t)wave * HD;
-                HeadVec<1> nr[JOBS];
-                int slj[JOBS];
-                #pragma unroll
-                for (int u = 0; u < JOBS; ++u) {              // the norms of all of them first: their sums overlap
-                    const bool isv = u >= JOBS / 2;
-                    const int r = (isv ? 3 - wave : wave) + 4 * (u % (JOBS / 2)), sl = tnew + r - t0;
-                    slj[u] = (r < M && sl >= 0 && sl <= 31) ? sl : -1;
-                    if (slj[u] >= 0) nr[u] = lg_head_norm<1>(hj[u], wk, !isv, HD, a.eps);
-                }
-                #pragma unroll
-                for (int u = 0; u < JOBS; ++u) {
-                    const bool isv = u >= JOBS / 2;
-                    const int sl = slj[u], t = t0 + sl;
-                    if (sl < 0) continue;
-                    const size_t coff = (size_t)(t % a.seq) * a.kv_dim + (size_t)kvh * HD;
-                    if (isv) {                                // V: no rotary, straight from the registers
-                        if (4 * lane < HD) {
-                            const uint2 h4 = make_uint2((uint32_t)lg_f2h(nr[u].x[0].x) | ((uint32_t)lg_f2h(nr[u].x[0].y) << 16),
-                                                        (uint32_t)lg_f2h(nr[u].x[0].z) | ((uint32_t)lg_f2h(nr[u].x[0].w) << 16));
-                            *(uint2 *)(vt + sl * Geo::VST + 4 * lane) = h4;
-                            *(uint2 *)(a.vcw + coff + 4 * lane) = h4;
-                        }
-                    } else {
-                        uint16_t *row = (uint16_t *)(kt + sl * Geo::KSD), *crow = a.kcw + coff;
-                        lg_head_rope<1>(nr[u], HD, t, rv, vec, [&](int p, float lo, float hi) {
-                            const int p1 = p + HD / 2;        // dims 4g, 4g+1 in dword g of the first half, 4g+2, 4g+3 of the second
-                            const uint16_t hl = lg_f2h(lo), hh = lg_f2h(hi);
-                            row[2 * (((p & 3) >> 1) * (HD / 4) + (p >> 2)) + (p & 1)] = hl;
-                            row[2 * (((p1 & 3) >> 1) * (HD / 4) + (p1 >> 2)) + (p1 & 1)] = hh;
-                            crow[p] = hl; crow[p1] = hh;
-                        });
-                    }
-                }
-            }
+    __syncthreads();
+    for (int it = 0; it < ng; it += 2) {                      // unit groups of the pair (more than two: heads of more than 4 to a kv head)
+        const int ug = ng == 1 ? 0 : it + pair;
+        int us[4], up[4];                                     // keys that units 4c + i see: us..up
+        size_t pi[4];                                         // their partials' slots, less the tile
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int u = 16 * ug + 4 * c + i, j = u / G;
+            up[i] = u < units ? pos0 + j : -1;
+            us[i] = u < units ? lg_win_start(pos0 + j, a.window) : 0;
+            pi[i] = u < units ? ((size_t)j * a.H + kvh * G + (u - j * G)) * a.tiles_max : 0;
         }
-        stash(bx);
-        __syncthreads();
-        if (i + 1 < tp && n + 1 <= last) fetch(bx + 1);
-        {   // scores
-            const int sl = lane & 31, hf = lane >> 5, t = t0 + sl;
-            const uint32_t *ks = kt + sl * Geo::KSD + hf * (HD / 4);
-            for (int ub = wave; ub < units; ub += UB * NWV) {
-                int un[UB];
-                const float *qr[UB];
-                float ax[UB], ay[UB];
-                #pragma unroll
-                for (int b = 0; b < UB; ++b) {                // (a missing unit repeats the first one and stores nothing)
-                    un[b] = ub + b * NWV < units ? ub + b * NWV : ub;
-                    qr[b] = qs + (size_t)un[b] * HD + hf * (HD / 2);
-                    ax[b] = 0.0f; ay[b] = 0.0f;
-                }
-                #pragma unroll 2
-                for (int u = 0; u < HD / 16; ++u) {
-                    const uint4 k4 = *(const uint4 *)(ks + 4 * u);
+        const float *qr = qs + (size_t)(16 * (ug < ng ? ug : 0) + n) * Geo::QST + c * (HD / 4);
+        float *ep = es + (size_t)pair * 16 * Geo::EST;
+        if (it > 0) { fetch_k(b0); fetch_v(b0); }
+        for (int bb = b0; bb < nb; bb += gx) {
+            const int tile = tile_of(bb), bx = tile - first, t0 = tile << 5;
+            const bool act = ug < ng && (ng > 1 || first + bb * tw + pair <= last);      // (the others compute what nobody stores)
+            if constexpr (FQ) if (any && t0 + 31 >= tnew) {           // rows of the block in this tile: from LDS, they are not in the cache yet
+                const int rk = t0 + 16 * half + n - tnew;
+                if (rk >= 0 && rk < M) {
                     #pragma unroll
-                    for (int b = 0; b < UB; ++b) {
-                        const float4 p0 = *(const float4 *)(qr[b] + 8 * u), p1 = *(const float4 *)(qr[b] + 8 * u + 4);
-                        ax[b] = lg_fma_hlo(p0.x, k4.x, ax[b]); ay[b] = lg_fma_hhi(p0.y, k4.x, ay[b]);
-                        ax[b] = lg_fma_hlo(p0.z, k4.y, ax[b]); ay[b] = lg_fma_hhi(p0.w, k4.y, ay[b]);
-                        ax[b] = lg_fma_hlo(p1.x, k4.z, ax[b]); ay[b] = lg_fma_hhi(p1.y, k4.z, ay[b]);
-                        ax[b] = lg_fma_hlo(p1.z, k4.w, ax[b]); ay[b] = lg_fma_hhi(p1.w, k4.w, ay[b]);
-                    }
+                    for (int s = 0; s < NS; ++s) kw[s] = *(const uint4 *)(nk + rk * HD + 32 * s + 8 * c);
                 }
                 #pragma unroll
-                for (int b = 0; b < UB; ++b) {
-                    if (b > 0 && un[b] == ub) continue;
-                    const int unit = un[b], j = unit / G, pj = pos0 + j, startj = lg_win_start(pj, a.window);
-                    if (n < (startj >> 5) || n > (pj >> 5)) continue;         // tile outside this row's keys (wavefront-uniform)
-                    const bool valid = t >= startj && t <= pj;
-                    float s = lg_add_x32(ax[b] + ay[b]);      // (a0+a1) + (a2+a3): the two halves sit 32 lanes apart
-                    if (!valid) s = -INFINITY;
-                    const float mx = lg_max_n(s, 32);
-                    const float e = valid ? lg_expf(s - mx) : 0.0f;
-                    const float l = lg_sum32(e);
-                    if (hf == 0) es[unit * 32 + sl] = e;
-                    if (lane == 0) {
-                        const size_t pi = ((size_t)j * a.H + kvh * G + (unit - j * G)) * a.tiles_max + bx;
-                        a.pm[pi] = mx; a.pl[pi] = l;
-                    }
+                for (int s = 0; s < 32; ++s) {
+                    const int r = t0 + s - tnew;
+                    if (r >= 0 && r < M) { if constexpr (NK == 2) vw[s] = *(const uint32_t *)(nv + r * HD + vd); else vw[s] = nv[r * HD + vd]; }
                 }
             }
-        }
-        __syncthreads();
-        {   // values (lane = 4 dims)
-            const uint16_t *vl = vt + (4 * lane < HD ? 4 * lane : 0);
-            for (int ub = wave; ub < units; ub += UB * NWV) {
-                int un[UB];
-                bool on[UB];
-                const float *er[UB];
-                float4 acc[UB];
+            // slots outside the keys of every row of the block are zeroed (their weights are zero, and zero times
+            // a finite value leaves the sums as they are; stale bits that read as infinities would not)
+            if (t0 < start0 || t0 + 31 > plast) {
                 #pragma unroll
-                for (int b = 0; b < UB; ++b) {
-                    un[b] = ub + b * NWV < units ? ub + b * NWV : ub;
-                    const int j = un[b] / G, pj = pos0 + j, startj = lg_win_start(pj, a.window);
-                    on[b] = !(n < (startj >> 5) || n > (pj >> 5)) && !(b > 0 && un[b] == ub);
-                    er[b] = es + un[b] * 32;                  // (a unit that skipped the scores has stale rows here: never stored)
-                    acc[b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                }
-                #pragma unroll 2
-                for (int u4 = 0; u4 < 8; ++u4) {
-                    float ev[UB][4];
-                    #pragma unroll
-                    for (int b = 0; b < UB; ++b) {
-                        const float4 e4 = *(const float4 *)(er[b] + 4 * u4);
-                        ev[b][0] = e4.x; ev[b][1] = e4.y; ev[b][2] = e4.z; ev[b][3] = e4.w;
-                    }
-                    #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const uint2 v = *(const uint2 *)(vl + (4 * u4 + q) * Geo::VST);
-                        #pragma unroll
-                        for (int b = 0; b < UB; ++b) {
-                            acc[b].x = lg_fma_hlo(ev[b][q], v.x, acc[b].x); acc[b].y = lg_fma_hhi(ev[b][q], v.x, acc[b].y);
-                            acc[b].z = lg_fma_hlo(ev[b][q], v.y, acc[b].z); acc[b].w = lg_fma_hhi(ev[b][q], v.y, acc[b].w);
-                        }
-                    }
-                }
+                for (int s = 0; s < 32; ++s) vw[s] = (t0 + s >= start0 && t0 + s <= plast) ? vw[s] : 0;
+            }
+            lg_v16f d = {};
+            // dims 32s + 8c + 0..7 of the key -> its dims 32s + 4g + c, g = 0..7.  A product that waits for the conversion in
+            // front of it takes 52 cycles instead of 32, so a piece is dealt and converted before the products of the one ahead of it.
+            float kf[2][8];
+            float4 qv[2][2];
+            auto piece = [&](int s) {
+                uint32_t o[4];
+                lg_deal4(__builtin_amdgcn_perm(kw[s].z, kw[s].x, 0x05040100u), __builtin_amdgcn_perm(kw[s].z, kw[s].x, 0x07060302u),
+                         __builtin_amdgcn_perm(kw[s].w, kw[s].y, 0x05040100u), __builtin_amdgcn_perm(kw[s].w, kw[s].y, 0x07060302u), o);
                 #pragma unroll
-                for (int b = 0; b < UB; ++b) {
-                    if (!on[b]) continue;
-                    const int unit = un[b], j = unit / G;
-                    const size_t pi = ((size_t)j * a.H + kvh * G + (unit - j * G)) * a.tiles_max + bx;
-                    if (4 * lane < HD) *(float4 *)(a.pacc + pi * HD + 4 * lane) = acc[b];
+                for (int g = 0; g < 8; ++g) kf[s & 1][g] = lg_h2f((uint16_t)(o[g >> 1] >> (16 * (g & 1))));
+            };
+            qv[0][0] = *(const float4 *)qr; qv[0][1] = *(const float4 *)(qr + 4);
+            piece(0);
+            #pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                if (s + 1 < NS) { qv[(s + 1) & 1][0] = *(const float4 *)(qr + 8 * (s + 1)); qv[(s + 1) & 1][1] = *(const float4 *)(qr + 8 * (s + 1) + 4); piece(s + 1); }
+                __builtin_amdgcn_sched_barrier(0);
+                const float4 qa = qv[s & 1][0], qb = qv[s & 1][1];
+                const float qe[8] = { qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w };
+                #pragma unroll
+                for (int g = 0; g < 8; ++g) d = __builtin_amdgcn_mfma_f32_16x16x1f32(qe[g], kf[s & 1][g], d, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            fetch_k(bb + gx);                                 // the next tile's K rows (past the last tile: the last one's again)
+            const int p = t0 + 16 * half + n;
+            float sc[4], m[4];
+            #pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                sc[i] = p >= us[i] && p <= up[i] ? (d[i] + d[4 + i]) + (d[8 + i] + d[12 + i]) : -INFINITY;
+                m[i] = lg_max16(sc[i]);
+                if (n == 0) mxs[wave][4 * c + i] = m[i];
+            }
+            __syncthreads();
+            #pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                m[i] = fmaxf(m[i], mxs[wave ^ 1][4 * c + i]);
+                const float e = p >= us[i] && p <= up[i] ? lg_expf(sc[i] - m[i]) : 0.0f;
+                const float l = lg_sum16(e);
+                ep[(4 * c + i) * Geo::EST + 16 * half + n] = e;
+                if (n == 0) lsum[wave][4 * c + i] = l;
+            }
+            __syncthreads();
+            lg_v16f acc[NK] = {};
+            float vf[2][4][NK];                               // (four slots converted ahead, as above)
+            float4 e4[2];
+            auto slots = [&](int s4) {
+                e4[s4 & 1] = *(const float4 *)(ep + n * Geo::EST + 4 * s4);
+                #pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    asm volatile("" : "+v"(vw[4 * s4 + q]));  // (converted here: else ahead of the scores, which then wait for every load and store)
+                    #pragma unroll
+                    for (int k = 0; k < NK; ++k) vf[s4 & 1][q][k] = lg_h2f((uint16_t)(vw[4 * s4 + q] >> (16 * k)));
+                }
+            };
+            slots(0);
+            #pragma unroll
+            for (int s4 = 0; s4 < 8; ++s4) {
+                if (s4 + 1 < 8) slots(s4 + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                const float ev[4] = { e4[s4 & 1].x, e4[s4 & 1].y, e4[s4 & 1].z, e4[s4 & 1].w };
+                #pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    #pragma unroll
+                    for (int k = 0; k < NK; ++k) acc[k] = __builtin_amdgcn_mfma_f32_16x16x1f32(ev[q], vf[s4 & 1][q][k], acc[k], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            #pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (!act || tile < (us[i] >> 5) || tile > (up[i] >> 5)) continue;        // no key of the unit's row in this tile
+                const size_t ti = pi[i] + bx;
+                if (half == 0 && n == 0) { a.pm[ti] = m[i]; a.pl[ti] = lsum[wave][4 * c + i] + lsum[wave ^ 1][4 * c + i]; }
+                if (HD < 128 && half != 0) continue;
+                float *dst = a.pacc + ti * HD + (HD >= 128 ? half * (HD / 2) : 0) + NK * n;
+                #pragma unroll
+                for (int b = 0; b < 4; ++b) {                 // block b: dims 16b + n, NK of them each
+                    if constexpr (NK == 2) *(float2 *)(dst + 32 * b) = make_float2(acc[0][4 * b + i], acc[1][4 * b + i]);
+                    else dst[16 * b] = acc[0][4 * b + i];
                 }
             }
+            fetch_v(bb + gx);
         }
     }
 }

@@ -1095,15 +1095,15 @@ static void launch_mmf(Launcher &lx, int cls, const MmfArgs &a) {
     constexpr int MC = M < 8 ? M : 8;
     LAUNCH(cls, (lg_k_mmf<MC>), dim3((a.m + LG_WG / 64 - 1) / (LG_WG / 64), (a.rows + MC - 1) / MC), dim3(LG_WG), 0, a);
 }
-static bool attention_rows_shared(int rows, int tiles, int nkv, int hd, int seq) {
-    return rows > 1 && hd <= 256 && seq >= 32 && tiles * nkv >= 256;
+// `reach`: the positions that the rows go to; a ring of other than a multiple of 32 rows has tiles around its end, which only
+// the kernel per row takes (this library's own rings are multiples of 32: reach 0)
+static bool attention_rows_shared(int rows, int tiles, int nkv, int hd, int seq, int reach) {
+    return rows > 1 && hd <= 256 && seq >= 32 && (seq % 32 == 0 || reach <= seq) && tiles * nkv >= 256;
 }
-// tiles per workgroup of lg_k_attn_rows: one, until the grid would exceed the three workgroups per CU that the
-// staged tile's LDS lets a CU hold; then as many as bring it back under that (at most four), each tile's rows in
-// flight while the tile before it is computed
-static int attention_rows_tp(int tiles, int nkv) {
-    const int tp = (tiles * nkv + 3 * 256 - 1) / (3 * 256);
-    return tp < 1 ? 1 : tp > 4 ? 4 : tp;
+// workgroups of lg_k_attn_rows per kv head: three to a CU at most (its registers hold no more), each walking its share of the tiles
+static int attention_rows_wgs(int tiles, int units, int nkv) {
+    const int steps = (tiles + lg_attn_rows_tiles(units) - 1) / lg_attn_rows_tiles(units), cap = 3 * cu_count() / nkv;
+    return steps < cap ? steps : cap > 1 ? cap : 1;
 }
 
 // wavefronts of lg_k_attn_merge_split: a round of 64 tiles each covers the cache's tiles, while the CUs hold all workgroups
@@ -1382,7 +1382,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
     };
     auto rows_shared = [&](int L) {
         const Layer &y = m->L[L];
-        return pos_off == 0 && m->attn_rows && attention_rows_shared(M, layer_tiles(L), y.nkv, y.hd, kv->seq[y.src]);
+        return pos_off == 0 && m->attn_rows && attention_rows_shared(M, layer_tiles(L), y.nkv, y.hd, kv->seq[y.src], 0);
     };
     for (int L = 0; L < nl && !lx.rc; ++L) {
         const Layer &y = m->L[L];
@@ -1395,15 +1395,10 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             else { rows(y.attn_norm, nullptr); launch_mm<M, false>(lx, KC_QKV, a); }
             // blocks of the model itself, up to LG_HIP_MAX_ROWS rows: the attention kernel does this part as well
             fused_post = pos_off == 0 || !y.owns;    // (a draft head's layers own no cache: queries only)
-            // ... unless the layer has so many (tile, kv head) pairs that one workgroup per pair can serve all rows of
-            // the block against one staged tile (long global contexts, wide windows): the rows then arrive prepared
-            // (that kernel prepares them itself while it has few workgroups: each of them repeats the preparation of its kv
-            // head's queries, which a layer of many hundred workgroups pays for with more than the launch it saves: 12B
-            // shape, 8192 keys, 688 workgroups: 36 -> 43 us; a 1024-key window, 272 workgroups: 11 -> 13.5 us against 4.2)
-            if (rows_shared(L)) {
-                const int tiles = layer_tiles(L), tp = attention_rows_tp(tiles, y.nkv);
-                if (!m->attn_rows_fq || ((tiles + tp - 1) / tp) * y.nkv > 2 * cu_count()) fused_post = false;
-            }
+            // (so does the one for layers whose workgroups serve all rows of the block, unless more than two workgroups a CU would each
+            // prepare more than 16 queries: 8 rows x 4 heads at 20011 keys 2595 -> 2580 us a step with a launch of its own, but 5 rows x
+            // 2 heads at 8192 keys 3361 -> 3384)
+            if (rows_shared(L) && (!m->attn_rows_fq || (M * (H / y.nkv) > 16 && attention_rows_wgs(layer_tiles(L), M * (H / y.nkv), y.nkv) * y.nkv > 2 * cu_count()))) fused_post = false;
             QkvPostArgs p{};
             p.qkv = m->qkv; p.ld = y.qkv_m; p.k_off = y.k_off; p.v_off = y.v_off;
             p.H = H; p.nkv = y.nkv; p.hd = y.hd;
@@ -1425,19 +1420,19 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             if (shared) {
                 if constexpr (M > 1) {
                     const size_t lds = y.hd == 256 ? AttnRowsGeo<256>::bytes(M * G, fused_post) : y.hd == 128 ? AttnRowsGeo<128>::bytes(M * G, fused_post) : AttnRowsGeo<64>::bytes(M * G, fused_post);
-                    const int tp = attention_rows_tp(tiles, y.nkv);
-                    const dim3 grid((tiles + tp - 1) / tp, y.nkv);
+                    const dim3 grid(attention_rows_wgs(tiles, M * G, y.nkv), y.nkv);
+                    a.gx = (int)grid.x;
                     if (fused_post) {
                         a.qkv = m->qkv; a.ld = y.qkv_m; a.k_off = y.k_off; a.v_off = y.v_off;
                         a.q_norm = y.q_norm; a.k_norm = y.k_norm; a.rope_tab = y.rope_tab; a.rope_ff = y.rope_ff;
                         a.kcw = y.owns ? kv->k[L] : nullptr; a.vcw = y.owns ? kv->v[L] : nullptr; a.eps = m->eps;
-                        if (y.hd == 256)      LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 256, true>), grid, dim3(LG_WG), lds, m->ctl, tp, LG_ATTN_FIELDS(LG_XA, a) 0);
-                        else if (y.hd == 128) LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 128, true>), grid, dim3(LG_WG), lds, m->ctl, tp, LG_ATTN_FIELDS(LG_XA, a) 0);
-                        else                  LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 64, true>), grid, dim3(LG_WG), lds, m->ctl, tp, LG_ATTN_FIELDS(LG_XA, a) 0);
+                        if (y.hd == 256)      LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 256, true>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
+                        else if (y.hd == 128) LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 128, true>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
+                        else                  LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 64, true>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
                     } else
-                    if (y.hd == 256)      LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 256>), grid, dim3(LG_WG), lds, m->ctl, tp, LG_ATTN_FIELDS(LG_XA, a) 0);
-                    else if (y.hd == 128) LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 128>), grid, dim3(LG_WG), lds, m->ctl, tp, LG_ATTN_FIELDS(LG_XA, a) 0);
-                    else                  LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 64>), grid, dim3(LG_WG), lds, m->ctl, tp, LG_ATTN_FIELDS(LG_XA, a) 0);
+                    if (y.hd == 256)      LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 256>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
+                    else if (y.hd == 128) LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 128>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
+                    else                  LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 64>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
                 }
             } else
             if (fused_post) {
@@ -2495,20 +2490,20 @@ extern "C" int lg_hip_ple_inputs(const float *pmp, const float *proj_norm, const
 // (the same choice of kernels as a verify step makes: many (tile, kv head) pairs -> one workgroup per pair serves all
 // rows; many tiles per row -> the merge is cut by dims)
 template <int M>
-static int enqueue_attention(hipStream_t st, const AttnArgs &a_in, const MergeArgs &g, StepCtl *ctl, int tiles, size_t lds) {
+static int enqueue_attention(hipStream_t st, const AttnArgs &a_in, const MergeArgs &g, StepCtl *ctl, int tiles, int pos, size_t lds) {
     AttnArgs a = a_in;
     a.gx = tiles; a.gz = M;                               // the grid of lg_k_attn, which reads it from its arguments
-    if (attention_rows_shared(M, tiles, a.nkv, a.hd, a.seq)) {
+    if (attention_rows_shared(M, tiles, a.nkv, a.hd, a.seq, pos + M)) {
         if constexpr (M > 1) {
             const int units = M * (a.H / a.nkv);
-            const size_t l2 = a.hd == 256 ? AttnRowsGeo<256>::bytes(units) : a.hd == 128 ? AttnRowsGeo<128>::bytes(units) : AttnRowsGeo<64>::bytes(units);
+            const size_t l2 = a.hd == 256 ? AttnRowsGeo<256>::bytes(units, false) : a.hd == 128 ? AttnRowsGeo<128>::bytes(units, false) : AttnRowsGeo<64>::bytes(units, false);
             int rc = a.hd == 256 ? set_lds(lg_k_attn_rows<M, 256>, l2) : a.hd == 128 ? set_lds(lg_k_attn_rows<M, 128>, l2) : set_lds(lg_k_attn_rows<M, 64>, l2);
             if (rc) return rc;
-            const int tp = attention_rows_tp(tiles, a.nkv);
-            const dim3 grid((tiles + tp - 1) / tp, a.nkv);
-            if (a.hd == 256)      hipLaunchKernelGGL((lg_k_attn_rows<M, 256>), grid, dim3(LG_WG), l2, st, ctl, tp, LG_ATTN_FIELDS(LG_XA, a) 0);
-            else if (a.hd == 128) hipLaunchKernelGGL((lg_k_attn_rows<M, 128>), grid, dim3(LG_WG), l2, st, ctl, tp, LG_ATTN_FIELDS(LG_XA, a) 0);
-            else                  hipLaunchKernelGGL((lg_k_attn_rows<M, 64>), grid, dim3(LG_WG), l2, st, ctl, tp, LG_ATTN_FIELDS(LG_XA, a) 0);
+            const dim3 grid(attention_rows_wgs(tiles, units, a.nkv), a.nkv);
+            a.gx = (int)grid.x;
+            if (a.hd == 256)      hipLaunchKernelGGL((lg_k_attn_rows<M, 256>), grid, dim3(LG_WG), l2, st, ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
+            else if (a.hd == 128) hipLaunchKernelGGL((lg_k_attn_rows<M, 128>), grid, dim3(LG_WG), l2, st, ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
+            else                  hipLaunchKernelGGL((lg_k_attn_rows<M, 64>), grid, dim3(LG_WG), l2, st, ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
         }
     } else hipLaunchKernelGGL((lg_k_attn<false, 1>), dim3(tiles, a.nkv, M), dim3(LG_WG), lds, st, ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
     if (tiles >= 128 && a.hd % 64 == 0) {
@@ -2520,7 +2515,7 @@ static int enqueue_attention(hipStream_t st, const AttnArgs &a_in, const MergeAr
 }
 
 template <int M>
-static int attention_rows(hipStream_t st, AttnArgs a, MergeArgs g, StepCtl *ctl, int tiles, int repeats, float *kernel_ms) {
+static int attention_rows(hipStream_t st, AttnArgs a, MergeArgs g, StepCtl *ctl, int tiles, int pos, int repeats, float *kernel_ms) {
     const size_t lds = attn_lds(a.H / a.nkv, a.hd, false);
     int rc = set_lds(lg_k_attn<false, 1>, lds);
     if (rc) return rc;
@@ -2529,7 +2524,7 @@ static int attention_rows(hipStream_t st, AttnArgs a, MergeArgs g, StepCtl *ctl,
         HIP_TRY(hipEventCreate(&e0)); HIP_TRY(hipEventCreate(&e1));
         for (int r = 0; r < repeats + 1; ++r) {
             if (r == 1) HIP_TRY(hipEventRecord(e0, st));
-            const int erc = enqueue_attention<M>(st, a, g, ctl, tiles, lds);
+            const int erc = enqueue_attention<M>(st, a, g, ctl, tiles, pos, lds);
             if (erc) return erc;
         }
         HIP_TRY(hipEventRecord(e1, st));
@@ -2578,7 +2573,7 @@ extern "C" int lg_hip_attention(const float *q, const uint16_t *kc, const uint16
     HIP_TRY(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     int rc = 0;
     switch (rows) {
-#define CASE(M) case M: rc = attention_rows<M>(st, a, g, ctl, tiles, repeats, kernel_ms); break;
+#define CASE(M) case M: rc = attention_rows<M>(st, a, g, ctl, tiles, pos, repeats, kernel_ms); break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
 #undef CASE
     }
@@ -2609,9 +2604,9 @@ extern "C" size_t lg_hip_attention_noalloc_limit(void) { return LG_NOALLOC_BYTES
 // this first; the entry point calls it by itself on its first use on a device.
 template <int M>
 static int noalloc_raise_rows() {
-    int rc = set_lds(lg_k_attn_rows<M, 256>, AttnRowsGeo<256>::bytes(M * 8));
-    if (!rc) rc = set_lds(lg_k_attn_rows<M, 128>, AttnRowsGeo<128>::bytes(M * 8));
-    if (!rc) rc = set_lds(lg_k_attn_rows<M, 64>, AttnRowsGeo<64>::bytes(M * 8));
+    int rc = set_lds(lg_k_attn_rows<M, 256>, AttnRowsGeo<256>::bytes(M * 8, false));
+    if (!rc) rc = set_lds(lg_k_attn_rows<M, 128>, AttnRowsGeo<128>::bytes(M * 8, false));
+    if (!rc) rc = set_lds(lg_k_attn_rows<M, 64>, AttnRowsGeo<64>::bytes(M * 8, false));
     return rc;
 }
 extern "C" int lg_hip_attention_noalloc_init(void) {
@@ -2676,7 +2671,7 @@ extern "C" int lg_hip_attention_noalloc(const float *d_q, const uint16_t *d_kc, 
     // cleared; only the step state is set, by a kernel (a caller may be capturing this stream)
     hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, st, ctl, pos);
     switch (rows) {
-#define CASE(M) case M: rc = enqueue_attention<M>(st, a, g, ctl, tiles, lds); break;
+#define CASE(M) case M: rc = enqueue_attention<M>(st, a, g, ctl, tiles, pos, lds); break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
 #undef CASE
     }

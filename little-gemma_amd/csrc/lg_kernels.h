@@ -1196,9 +1196,6 @@ struct AttnArgs {
     int gx, gz;              // lg_k_attn: its launch dimensions x and z (as arguments they arrive with the others)
     __device__ __forceinline__ uint4 kc4(size_t off) const { return *(const uint4 *)(kc + off); }
     __device__ __forceinline__ uint4 vc4(size_t off) const { return *(const uint4 *)(vc + off); }
-    // for the kernels that stage a tile once for all the rows of a block: no second reader, so non-temporal
-    __device__ __forceinline__ uint4 kc4s(size_t off) const { return lg_ldw16(kc + off); }
-    __device__ __forceinline__ uint4 vc4s(size_t off) const { return lg_ldw16(vc + off); }
 };
 #define LG_ATTN_FIELDS(X, v) X(int, gx, gx, v) X(int, gz, gz, v) X(int, hd, hd, v) X(int, window, window, v) X(int, pos_off, pos_off, v) X(int, seq, seq, v) X(int, kv_dim, kv_dim, v) X(const uint16_t *, kc, kc, v) X(const uint16_t *, vc, vc, v) X(int, H, H, v) X(int, nkv, nkv, v) X(const float *, qkv, qkv, v) X(const float *, q_norm, q_norm, v) X(const float *, k_norm, k_norm, v) X(const float *, rope_tab, rope_tab, v) X(const float *, rope_ff, rope_ff, v) X(int, ld, ld, v) X(int, k_off, k_off, v) X(int, v_off, v_off, v) X(uint16_t *, kcw, kcw, v) X(uint16_t *, vcw, vcw, v) X(const float *, q, q, v) X(float *, pm, pm, v) X(float *, pl, pl, v) X(float *, pacc, pacc, v) X(int, tiles_max, tiles_max, v) X(float, eps, eps, v)
 

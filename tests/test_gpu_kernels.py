@@ -284,6 +284,25 @@ def test_attention_over_many_tiles(lg, ob, gpu_required, H, KV, hd, rows, tiles,
     assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("H,KV,hd,rows,window,seq,pos", [
+    (12, 2, 256, 7, 4100, 4128, 9000),     # 42 units (three groups), a window that begins and ends inside tiles
+    (16, 2, 128, 8, 0, 4161, 4150),        # 64 units, a cache that ends inside its last tile
+    (8, 1, 64, 2, 8200, 8224, 20001),      # 16 units: one group, two tiles at a time, an odd number of tiles
+    (16, 8, 256, 5, 1024, 1536, 1533),     # the 12B shape's window, at a ring's end
+    (4, 4, 256, 8, 2048, 2101, 6300),      # a ring of other than a multiple of 32 rows: the kernel per row
+    (8, 8, 64, 3, 1024, 1088, 40)])        # few keys in a wide window
+def test_attention_of_all_rows_of_a_block(lg, ob, gpu_required, H, KV, hd, rows, window, seq, pos):
+    """256 and more (tile, kv head) pairs: a workgroup serves all rows, units in groups of 16 on the matrix cores; same bits as the oracle."""
+    rng = np.random.default_rng(H * 100 + rows)
+    kc = rng.normal(0, 1, (seq, KV * hd)).astype(np.float16).view(np.uint16)
+    vc = rng.normal(0, 1, (seq, KV * hd)).astype(np.float16).view(np.uint16)
+    q = (rng.normal(0, 1, (rows, H * hd)) * 0.1).astype(np.float32)
+    print(f"attention H={H} KV={KV} hd={hd} rows={rows} window={window} seq={seq} pos={pos}", flush=True)
+    out, _ = lg.hiplib.attention(q, kc, vc, H, KV, hd, window, pos)
+    want = oracle_attention(ob, q, kc, vc, H, KV, hd, window, pos)
+    assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
+
+
 def test_bad_arguments_are_refused(lg, gpu_required):
     rng = np.random.default_rng(1)
     with pytest.raises(lg.hiplib.HipError):
