@@ -280,6 +280,89 @@ __global__ __launch_bounds__(LG_WG) void lg_k_mmf(MmfArgs a) {
     }
 }
 
+// The residual update ahead of the per-layer gate and the gate itself in one launch (verify blocks of models that keep the gate
+// in a float type; lg_k_rows_plegate does the same for q4_0): workgroup (i, y) forms the updated rows 4y..4y+3, x + rmsnorm(dout) * w_post,
+// in LDS, repeating what lg_k_rows does, and its wavefronts run row i of the gate against one of them each in
+// lg_k_mmf's order.  Workgroups 0..3 store the updated rows.  A kernel boundary and a loop of dependent loads less: the gate's 256 rows were 64
+// workgroups that fetched weights and rows step by step.  E4B width, 4 rows: 4.3 + 8.2 -> 6.3 us.
+struct RowsMmfArgs {
+    const float *x, *dout, *w_post;    // [M][k], [M][k] (four slabs of it when dparts = 4), [k]
+    int          dparts;
+    float       *x_out;                // [M][k]
+    float        eps;
+    const float *w; int k, m;          // gate [m][k], k a multiple of 256
+    const float *ipl; int ipl_ld;      // [M][ipl_ld], at the layer's slice
+    float       *out;                  // [M][m]
+};
+#define LG_RMMF_ROWS 4                     // rows of a workgroup
+template <int M>
+__global__ __launch_bounds__(LG_WG) void lg_k_rows_mmf(RowsMmfArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    float4 *rl = (float4 *)smem;                              // [RB][k/4]
+    constexpr int RB = M < LG_RMMF_ROWS ? M : LG_RMMF_ROWS;
+    __shared__ float red[RB][4];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), i = blockIdx.x, j0 = M > RB ? (int)blockIdx.y * RB : 0, nq = a.k >> 2, nit = a.k >> 8;
+    float4 wp[LG_ROWV], gw[LG_MAXV], xv[RB][LG_ROWV], dv[RB][LG_ROWV];
+    #pragma unroll
+    for (int r = 0; r < RB; ++r) {                            // (past the block: its last row again, never stored)
+        const int j = min(j0 + r, M - 1);
+        const float4 *xr = (const float4 *)(a.x + (size_t)j * a.k), *dr = (const float4 *)(a.dout + (size_t)j * a.k);
+        #pragma unroll
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) { dv[r][v] = dr[t + 256 * v]; xv[r][v] = xr[t + 256 * v]; }
+    }
+    #pragma unroll
+    for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) wp[v] = ((const float4 *)a.w_post)[t + 256 * v];
+    #pragma unroll
+    for (int v = 0; v < LG_MAXV; ++v) if (v < nit) gw[v] = ((const float4 *)(a.w + (size_t)i * a.k))[lane + 64 * v];
+    const float iplv = a.ipl[(size_t)min(j0 + wave, M - 1) * a.ipl_ld + i];
+    __builtin_amdgcn_sched_barrier(0);
+    if (a.dparts == 4) {                                      // top of the K-segment tree of a matmul cut by K quarter
+        const size_t slab = (size_t)M * nq;
+        #pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            const float4 *dr = (const float4 *)(a.dout + (size_t)min(j0 + r, M - 1) * a.k);
+            #pragma unroll
+            for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) {
+                const float4 p1 = dr[slab + t + 256 * v], p2 = dr[2 * slab + t + 256 * v], p3 = dr[3 * slab + t + 256 * v], p0 = dv[r][v];
+                dv[r][v] = make_float4((p0.x + p1.x) + (p2.x + p3.x), (p0.y + p1.y) + (p2.y + p3.y), (p0.z + p1.z) + (p2.z + p3.z), (p0.w + p1.w) + (p2.w + p3.w));
+            }
+        }
+    }
+    #pragma unroll
+    for (int r = 0; r < RB; ++r) {
+        float ss = 0.0f;
+        #pragma unroll
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) ss = lg_sumsq4(dv[r][v], ss);
+        ss = lg_wave_sum64(ss);
+        if (lane == 0) red[r][wave] = ss;
+    }
+    __syncthreads();
+    #pragma unroll
+    for (int r = 0; r < RB; ++r) {
+        const float ss = (red[r][0] + red[r][1]) + (red[r][2] + red[r][3]);
+        const float sc = 1.0f / sqrtf(ss / (float)a.k + a.eps);
+        #pragma unroll
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) {
+            const float4 w = wp[v], d = dv[r][v];
+            float4 x = xv[r][v];
+            x.x = x.x + d.x * sc * w.x;  x.y = x.y + d.y * sc * w.y;
+            x.z = x.z + d.z * sc * w.z;  x.w = x.w + d.w * sc * w.w;
+            rl[r * nq + t + 256 * v] = x;
+            if (i == r && j0 + r < M) ((float4 *)(a.x_out + (size_t)(j0 + r) * a.k))[t + 256 * v] = x;
+        }
+    }
+    __syncthreads();
+    if (wave >= RB || j0 + wave >= M) return;
+    float acc = 0.0f;
+    #pragma unroll
+    for (int v = 0; v < LG_MAXV; ++v) if (v < nit) {
+        const float4 x = rl[wave * nq + lane + 64 * v], w = gw[v];
+        acc = lg_fmaf(w.x, x.x, acc); acc = lg_fmaf(w.y, x.y, acc); acc = lg_fmaf(w.z, x.z, acc); acc = lg_fmaf(w.w, x.w, acc);
+    }
+    acc = lg_wave_sum64(acc);
+    if (lane == 0) a.out[(size_t)(j0 + wave) * a.m + i] = lg_gelu(acc) * iplv;
+}
+
 // ---------------------------------------------------------------------------------------------
 // lm_head for verify blocks of 4..8 rows on the matrix cores: lg_k_geglu_m's tile loop (row-block tiles of the
 // vocabulary matrix, a wavefront = 64 vocabulary rows x one of the 8 K segments, two v_mfma_i32_32x32x32_i8 per

@@ -1531,9 +1531,16 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         if (m->ple) join();
         if (m->ple && y.winp_f) {   // per-layer embedding block, matrices kept in a float type: residual update, then the
             // gate on the f32 rows (gelu(.) * ipl in its epilogue), then the projection of the f32 gate rows
+            if (have_x && pend_dout && !pend_os && (pend_parts == 1 || pend_parts == 4)) {
+                RowsMmfArgs f{ m->x[cur], pend_dout, pend_w, pend_parts, m->x[cur ^ 1], m->eps, y.winp_f, E, m->ple, m->pmp_raw + (size_t)L * m->ple, m->ple * nl, m->pgf };
+                LAUNCH(KC_PLEGATE, lg_k_rows_mmf<M>, dim3(m->ple, (M + LG_RMMF_ROWS - 1) / LG_RMMF_ROWS), dim3(LG_WG), (size_t)(M < LG_RMMF_ROWS ? M : LG_RMMF_ROWS) * E * 4, f);
+                cur ^= 1;
+                pend_dout = pend_w = pend_os = nullptr; pend_parts = 1;
+            } else {
             rows(nullptr, nullptr);
             MmfArgs g{ y.winp_f, E, m->ple, m->x[cur], E, M, m->pgf, m->ple, m->pmp_raw + (size_t)L * m->ple, m->ple * nl };
             launch_mmf<M>(lx, KC_PLEGATE, g);
+            }
             MmfArgs p{ y.wproj_f, m->ple, E, m->pgf, m->ple, M, m->dout, E, nullptr, 0 };
             launch_mmf<M>(lx, KC_PLEPROJ, p);
             pend_dout = m->dout; pend_w = y.post_norm; pend_os = y.out_scale;
