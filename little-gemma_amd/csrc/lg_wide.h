@@ -15,8 +15,9 @@
 //    correctly rounded product (subnormals included).  One instruction serves the two 32-row halves of a weight tile,
 //    and a lane loads one scale per block where the vector form loads the 16 scales of its outputs through LDS.
 //
-// Measured issue bound per 32x32x32 block and SIMD: 60 cycles of vector work, 66 of matrix work, two wavefronts
-// overlapping them (int8 with sub, mul and fma: 163 cycles).
+// Measured issue bound per 32x32x32 block and SIMD: 36 cycles of fma (two wavefronts: 2.25 each), 32 of the dot and 32 of half a
+// scale product.  The f32 product runs on the vector unit's multipliers and keeps it from everything else, and with both
+// wavefronts busy the dots do not overlap the fma either: 100 cycles, of which the loop reaches 126 (int8 with sub, mul and fma: 163).
 //
 // A workgroup is 4 wavefronts and owns 64 weight rows x 32*TB activation rows; wavefront w runs the K segments 2w and
 // 2w+1, so the wavefronts share no operands, the main loop has no barrier and the operands come straight from L2; LDS
@@ -186,14 +187,13 @@ __device__ __forceinline__ void lg_wide_tile(const WideMm &a, int at, int bt, in
                 mine[(t * 4 + g) * 64 + lane] = make_float4(p[t / TB][t % TB][4 * g], p[t / TB][t % TB][4 * g + 1], p[t / TB][t % TB][4 * g + 2], p[t / TB][t % TB][4 * g + 3]);
         clear();
     };
-    // A step is (block, activation tile): its scale products S, its two dots D0 and D1, and the 32 fma that use them.
-    // The matrix instructions of step q+1 are issued between the fma of step q (S ahead of the first 16, D0 ahead of
-    // the second, D1 behind them: each into registers that have just been read), so that neither pipe waits for the
-    // other; left to the compiler a wavefront issues one matrix instruction, waits it out and then does its fma
-    // (gate/up of 512 rows at the E4B shape: 91 us that way).
-    constexpr int NS = TB == 1 ? 4 : 2;                       // blocks in flight (even: a step's S alternates)
+    // A step is (block, activation tile): its two dots D0 and D1, its scale products S, and the 32 fma that use them.  S keeps the
+    // vector unit from everything else while it runs, so it has one set of registers; the dots of the next step are issued
+    // behind the fma that read this step's.  (With S of the next step issued ahead of this step's fma, 30 registers more: prompts
+    // 0.5 to 1.2% slower.)  The last blocks run apart from the loop, which always requests.
+    constexpr int NS = TB == 2 ? 2 : 4;                       // blocks in flight (32-row tiles with 6 or 8: a prompt of 23 tokens 5980 -> 6100, 6260 us)
     Ops o[NS];
-    lg_v32f S[2];
+    lg_v32f S;
     lg_v16f D0, D1;
     lg_v8i a0, a1;
     float dw, xd[2];
@@ -210,44 +210,47 @@ __device__ __forceinline__ void lg_wide_tile(const WideMm &a, int at, int bt, in
     for (int i = 0; i < NS; ++i) fetch(o[i], i < last ? i : last);
     clear();
     take(o[0]);
-    S[0] = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, xd[0], z32, 0, 0, 0);
     D0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a0, o[0].b[0], z16, 3, 3, 0, 127, 0, sb);
     D1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a1, o[0].b[0], z16, 3, 3, 0, 127, 0, sb);
-    for (int it = 0; it < nblk; it += NS) {
+    auto block = [&](int it, int u, bool more) {              // block it + u; `more`: its registers receive block it + u + NS
+        if (WV == 4 && it + u == nit) segment_end();
         #pragma unroll
-        for (int u = 0; u < NS; ++u) {
-            if ((NS > 2 || WV == 8) && it + u >= nblk) break;   // (two segments: an even count)
-            if (WV == 4 && it + u == nit) segment_end();
-            #pragma unroll
-            for (int t = 0; t < TB; ++t) {
-                const int cur = TB == 2 ? t : (u & 1), nxt = cur ^ 1;
-                const Ops &on = t + 1 < TB ? o[u] : o[(u + 1) % NS];
-                const int tn = t + 1 < TB ? t + 1 : 0;
-                if (tn == 0) take(on);
-                S[nxt] = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, xd[tn], z32, 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-                if (DUMP) {
-                    const int an = (bt * TB + t) * 32 + n;
-                    if (an < a.rows)
-                        for (int i = 0; i < 16; ++i) {
-                            const int row = at * LG_WT + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-                            if (row < a.m) dots[((size_t)an * a.m + row) * nb + kb0 + it + u] = (int)D0[i];
-                            if (row + 32 < a.m) dots[((size_t)an * a.m + row + 32) * nb + kb0 + it + u] = (int)D1[i];
-                        }
-                }
-                #pragma unroll
-                for (int i = 0; i < 16; ++i) p[0][t][i] = lg_fmaf(S[cur][i], D0[i], p[0][t][i]);
-                __builtin_amdgcn_sched_barrier(0);
-                D0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a0, on.b[tn], z16, 3, 3, 0, 127, 0, sb);
-                __builtin_amdgcn_sched_barrier(0);
-                #pragma unroll
-                for (int i = 0; i < 16; ++i) p[1][t][i] = lg_fmaf(S[cur][16 + i], D1[i], p[1][t][i]);
-                __builtin_amdgcn_sched_barrier(0);
-                D1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a1, on.b[tn], z16, 3, 3, 0, 127, 0, sb);
-                if (t == (TB == 2 ? 0 : TB - 1)) { const int nx = it + u + NS; fetch(o[u], nx < last ? nx : last); }
-                __builtin_amdgcn_sched_barrier(0);
+        for (int t = 0; t < TB; ++t) {
+            const Ops &on = t + 1 < TB ? o[u] : o[(u + 1) % NS];
+            const int tn = t + 1 < TB ? t + 1 : 0;
+            S = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, xd[t], z32, 0, 0, 0);
+            if (tn == 0) take(on);
+            __builtin_amdgcn_sched_barrier(0);
+            if (DUMP) {
+                const int an = (bt * TB + t) * 32 + n;
+                if (an < a.rows)
+                    for (int i = 0; i < 16; ++i) {
+                        const int row = at * LG_WT + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+                        if (row < a.m) dots[((size_t)an * a.m + row) * nb + kb0 + it + u] = (int)D0[i];
+                        if (row + 32 < a.m) dots[((size_t)an * a.m + row + 32) * nb + kb0 + it + u] = (int)D1[i];
+                    }
             }
+            #pragma unroll
+            for (int i = 0; i < 16; ++i) p[0][t][i] = lg_fmaf(S[i], D0[i], p[0][t][i]);
+            __builtin_amdgcn_sched_barrier(0);
+            D0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a0, on.b[tn], z16, 3, 3, 0, 127, 0, sb);
+            __builtin_amdgcn_sched_barrier(0);
+            #pragma unroll
+            for (int i = 0; i < 16; ++i) p[1][t][i] = lg_fmaf(S[16 + i], D1[i], p[1][t][i]);
+            __builtin_amdgcn_sched_barrier(0);
+            D1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a1, on.b[tn], z16, 3, 3, 0, 127, 0, sb);
+            if (more && t == (TB == 2 ? 0 : TB - 1)) { const int nx = it + u + NS; fetch(o[u], nx < last ? nx : last); }
+            __builtin_amdgcn_sched_barrier(0);
         }
+    };
+    int it = 0;
+    for (; it + NS < nblk; it += NS) {
+        #pragma unroll
+        for (int u = 0; u < NS; ++u) block(it, u, true);
+    }
+    #pragma unroll
+    for (int u = 0; u < NS; ++u) {                            // the last NS blocks at most: nothing left to request
+        if (it + u < nblk) block(it, u, false);             // (a guard, not a break: the operands stay in registers)
     }
     #pragma unroll
     for (int t = 0; t < 2 * TB; ++t)
