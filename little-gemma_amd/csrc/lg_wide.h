@@ -510,20 +510,21 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
             up[i] = on ? pos + r : -1;
             us[i] = on ? lg_win_start(pos + r, a.window) : 0;
         }
-        // a tile's K rows (512-wide heads: half of them) are requested as soon as the ones before them have been dealt
-        constexpr int NS = HD / 32, CH = NS < 8 ? NS : 8;     // 64-byte pieces of a K row
+        // pieces of a tile's K rows are requested as soon as the ones CH ahead of them have been dealt
+        constexpr int NS = HD / 32, CH = NS < 8 ? NS : 8;     // 64-byte pieces of a K row; in flight
         uint4 w0[CH], w1[CH];
-        auto request = [&](int t, int s0) {
+        auto rows_of = [&](int t, const uint16_t *&k0, const uint16_t *&k1) {
             const int ring0 = (t << 5) % a.seq;
             int r0 = ring0 + n, r1 = ring0 + 16 + n;          // ring rows of this lane's two keys (a ring is a multiple of 32 rows, or as long as the positions go)
             if (r0 >= a.seq) r0 = a.seq - 1;
             if (r1 >= a.seq) r1 = a.seq - 1;
-            const uint16_t *k0 = a.kc + (size_t)r0 * a.kv_dim + (size_t)kvh * HD + c * 8, *k1 = a.kc + (size_t)r1 * a.kv_dim + (size_t)kvh * HD + c * 8;
-            #pragma unroll
-            for (int s = 0; s < CH; ++s) { w0[s] = *(const uint4 *)(k0 + (s0 + s) * 32); w1[s] = *(const uint4 *)(k1 + (s0 + s) * 32); }
+            k0 = a.kc + (size_t)r0 * a.kv_dim + (size_t)kvh * HD + c * 8; k1 = a.kc + (size_t)r1 * a.kv_dim + (size_t)kvh * HD + c * 8;
         };
         const int t1 = tfirst + (PHASE ? blockIdx.z * NW : 0) + wave, step = PHASE ? gridDim.z * NW : NW;
-        request(t1, 0);
+        const uint16_t *k0, *k1, *n0, *n1;                    // of this tile, of the next one
+        rows_of(t1, n0, n1);
+        #pragma unroll
+        for (int s = 0; s < CH; ++s) { w0[s] = *(const uint4 *)(n0 + s * 32); w1[s] = *(const uint4 *)(n1 + s * 32); }
         // the units' query rows into LDS, chain by chain: [unit][i % 4][i / 4] (in registers a wave's copy of them spilled)
         for (int i = threadIdx.x; i < 16 * (HD / 4); i += WG) {
             const int u = i / (HD / 4), j = i - u * (HD / 4), ur = u / G;
@@ -544,34 +545,38 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
                 continue;
             }
             lg_v16f d0 = {}, d1 = {};
-            #pragma unroll
-            for (int s0 = 0; s0 < NS; s0 += CH) {
-                // dims 32s + 8c + 0..7 of a key -> the same key's dims 32s + 4g + c, g = 0..7, as f16 pairs in g order
-                uint32_t o0[CH][4], o1[CH][4];
-                #pragma unroll
-                for (int s = 0; s < CH; ++s) {
-                    auto deal = [](uint4 w, uint32_t (&o)[4]) {
-                        lg_deal4(__builtin_amdgcn_perm(w.z, w.x, 0x05040100u), __builtin_amdgcn_perm(w.z, w.x, 0x07060302u),
-                                 __builtin_amdgcn_perm(w.w, w.y, 0x05040100u), __builtin_amdgcn_perm(w.w, w.y, 0x07060302u), o);
-                    };
-                    deal(w0[s], o0[s]); deal(w1[s], o1[s]);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                if (s0 + CH < NS) request(t, s0 + CH);
-                else request(t + step, 0);
-                __builtin_amdgcn_sched_barrier(0);
-                #pragma unroll
-                for (int s = 0; s < CH; ++s) {
-                    const float4 qa = *(const float4 *)(qs + 8 * (s0 + s)), qb = *(const float4 *)(qs + 8 * (s0 + s) + 4);
-                    if (s & 1) __builtin_amdgcn_sched_barrier(0);      // (else all of them are fetched at once and spill)
-                    const float qv[8] = { qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w };
+            k0 = n0; k1 = n1;
+            rows_of(t + step, n0, n1);
+            // dims 32s + 8c + 0..7 of a key -> the same key's dims 32s + 4g + c, g = 0..7.  A product that waits for the conversion in front
+            // of it takes 52 cycles instead of 32, so a piece is dealt and converted ahead of the products of the one before it.
+            float f0[2][8], f1[2][8];
+            float4 qv[2][2];
+            auto piece = [&](int s) {
+                auto deal = [](uint4 w, float (&f)[8]) {
+                    uint32_t o[4];
+                    lg_deal4(__builtin_amdgcn_perm(w.z, w.x, 0x05040100u), __builtin_amdgcn_perm(w.z, w.x, 0x07060302u),
+                             __builtin_amdgcn_perm(w.w, w.y, 0x05040100u), __builtin_amdgcn_perm(w.w, w.y, 0x07060302u), o);
                     #pragma unroll
-                    for (int g = 0; g < 8; ++g) {
-                        const float b0 = lg_h2f((uint16_t)(o0[s][g >> 1] >> (16 * (g & 1)))), b1 = lg_h2f((uint16_t)(o1[s][g >> 1] >> (16 * (g & 1))));
-                        d0 = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[g], b0, d0, 0, 0, 0);
-                        d1 = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[g], b1, d1, 0, 0, 0);
-                    }
+                    for (int g = 0; g < 8; ++g) f[g] = lg_h2f((uint16_t)(o[g >> 1] >> (16 * (g & 1))));
+                };
+                deal(w0[s % CH], f0[s & 1]); deal(w1[s % CH], f1[s & 1]);
+                const int i = s + CH;
+                w0[s % CH] = *(const uint4 *)(i < NS ? k0 + i * 32 : n0 + (i - NS) * 32); w1[s % CH] = *(const uint4 *)(i < NS ? k1 + i * 32 : n1 + (i - NS) * 32);
+                qv[s & 1][0] = *(const float4 *)(qs + 8 * s); qv[s & 1][1] = *(const float4 *)(qs + 8 * s + 4);
+            };
+            piece(0);
+            #pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                if (s + 1 < NS) piece(s + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                const float4 qa = qv[s & 1][0], qb = qv[s & 1][1];
+                const float qe[8] = { qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w };
+                #pragma unroll
+                for (int g = 0; g < 8; ++g) {
+                    d0 = __builtin_amdgcn_mfma_f32_16x16x1f32(qe[g], f0[s & 1][g], d0, 0, 0, 0);
+                    d1 = __builtin_amdgcn_mfma_f32_16x16x1f32(qe[g], f1[s & 1][g], d1, 0, 0, 0);
                 }
+                __builtin_amdgcn_sched_barrier(0);
             }
             float *et = eb + (size_t)(t - tfirst) * 16 * ES, *mt = mb + (t - tfirst) * 16, *lt = lb + (t - tfirst) * 16;
             const int p0 = t0 + n, p1 = p0 + 16;
@@ -662,11 +667,16 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
                         #pragma unroll
                         for (int k = 0; k < RUN; ++k) if (p + k < kfirst || p + k > klast) v[cur][k] = 0;
                     }
+                    float vl[RUN], vh[RUN];                   // (converted ahead of the run's products, as above)
+                    #pragma unroll
+                    for (int k = 0; k < RUN; ++k) { vl[k] = lg_h2f((uint16_t)(v[cur][k] & 0xFFFF)); vh[k] = lg_h2f((uint16_t)(v[cur][k] >> 16)); }
+                    __builtin_amdgcn_sched_barrier(0);
                     #pragma unroll
                     for (int k = 0; k < RUN; ++k) {
-                        acc0 = __builtin_amdgcn_mfma_f32_16x16x1f32(e[k], lg_h2f((uint16_t)(v[cur][k] & 0xFFFF)), acc0, 0, 0, 0);
-                        acc1 = __builtin_amdgcn_mfma_f32_16x16x1f32(e[k], lg_h2f((uint16_t)(v[cur][k] >> 16)), acc1, 0, 0, 0);
+                        acc0 = __builtin_amdgcn_mfma_f32_16x16x1f32(e[k], vl[k], acc0, 0, 0, 0);
+                        acc1 = __builtin_amdgcn_mfma_f32_16x16x1f32(e[k], vh[k], acc1, 0, 0, 0);
                     }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
                 if constexpr (EL) tile_weights();
                 #pragma unroll
