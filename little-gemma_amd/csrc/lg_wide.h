@@ -448,6 +448,8 @@ __global__ __launch_bounds__(LG_WG) void lg_k_wide_quant(const float *x, int row
 // Eight wavefronts rather than four: one workgroup is all the LDS holds on a CU, and with two wavefronts on a SIMD one
 // loads, deals and exponentiates while the other multiplies.  500 rows of a 512-wide window of 256-wide heads (8 over 2):
 // 65 -> 43 us; 512 rows of a 1024-wide one (16 over 8): 232 -> 137 us; all of 4093 positions (16 over 1): 584 -> 400 us.
+// Pieces and runs converted ahead of their products: the 1024-wide window 132 -> 119 us; the first value runs requested ahead of
+// the synchronisations: 332 rows at 3001 11.73 -> 11.70 ms a prompt.
 // In memory the weights are requested with the value rows, runs ahead (512 rows at 3500, 16 heads over 8: 474 -> 450 us).
 //
 // PHASE 1 and 2 are the two halves as kernels of their own, for blocks whose groups do not fill the chip: the time of a
@@ -594,6 +596,47 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
         }
     }
     if constexpr (PHASE == 1) return;
+    // Value rows.  A run is 8 slots of this lane's tile 4g + c (dims dg*32 + 2n and 2n + 1; !EL: the weights as well, which
+    // come from memory too): requested AHEAD runs ahead, a group of four tiles is four runs.  The first runs do not wait for the
+    // weights: they are requested here, ahead of the synchronisations.
+    // Buffer loads: the tile's place in the lane offset, the slot's in a scalar register (as flat loads their 64-bit
+    // addresses cost more vector instructions than the conversions); the buffer ends with the ring, slots past it read 0.
+    // FAR: flat loads, for blocks that reach 2 GiB and more into a layer's value rows.
+    constexpr int RUN = 8, NB = PHASE == 2 ? 8 : 4, AHEAD = NB - 1;
+    uint32_t v[NB][RUN];
+    float4 ev[EL ? 1 : NB][2];
+    const int ng = nt >> 2, vrow = a.kv_dim * 2;
+    const uint64_t vbytes = (uint64_t)a.seq * a.kv_dim * 2;
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)a.vc, 0, (uint32_t)(vbytes < 0x7FFFFFFFu ? vbytes : 0x7FFFFFFFu), 0x00020000);
+    auto fetch_v = [&](int vcol, int buf, int g, int i) {
+        g = g < ng ? g : ng - 1;
+        const int ring0 = ((tfirst + 4 * g + c) << 5) % a.seq;
+        if constexpr (FAR) {
+            #pragma unroll
+            for (int k = 0; k < RUN; ++k) {
+                const int r = ring0 + RUN * i + k < a.seq ? ring0 + RUN * i + k : a.seq - 1;       // (a slot past the ring is no position of the group: zeroed below)
+                v[buf][k] = *(const uint32_t *)((const uint8_t *)a.vc + (size_t)r * vrow + vcol);
+            }
+        } else {
+            const int off = ring0 * vrow + vcol;
+            #pragma unroll
+            for (int k = 0; k < RUN; ++k) v[buf][k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rv, off, (RUN * i + k) * vrow, 0);
+        }
+    };
+    auto fetch_e = [&](int buf, int g, int i) {
+        if constexpr (!EL) {
+            g = g < ng ? g : ng - 1;
+            const float *et = eb + ((size_t)(4 * g + c) * 16 + n) * ES + RUN * i;
+            ev[buf][0] = *(const float4 *)et; ev[buf][1] = *(const float4 *)(et + 4);
+        }
+    };
+    const int ndg = PHASE == 2 ? HD / 32 / gridDim.z : HD / 32, dg0 = PHASE == 2 ? blockIdx.z * ndg : 0;      // runs of 32 dims of this workgroup
+    auto first_runs = [&](int dg) {
+        #pragma unroll
+        for (int i = 0; i < AHEAD; ++i) fetch_v((kvh * HD + dg * 32 + 2 * n) * 2, i, i >> 2, i & 3);
+    };
+    if (wave < ndg) first_runs(dg0 + wave);
+    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     {   // the units' maxima over their tiles, then m -> the tile's weight exp(m - M)
         const int u = threadIdx.x & 15, k = threadIdx.x >> 4;
@@ -605,44 +648,14 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
         for (int t = k; t < nt; t += WG / 16) { const float v = mb[t * 16 + u]; wb[t * 16 + u] = v == -INFINITY ? 0.0f : lg_expf(v - m); }
     }
     __syncthreads();
-    const int ndg = PHASE == 2 ? HD / 32 / gridDim.z : HD / 32, dg0 = PHASE == 2 ? blockIdx.z * ndg : 0;      // runs of 32 dims of this workgroup
     for (int dg = dg0 + wave; dg < dg0 + ndg; dg += NW) {
         float o[2][4], L[4];
         #pragma unroll
         for (int i = 0; i < 4; ++i) { o[0][i] = o[1][i] = 0.0f; L[i] = 0.0f; }
-        // A run is 8 slots of this lane's tile 4g + c (value rows, dims dg*32 + 2n and 2n + 1; !EL: their weights as well, which
-        // come from memory too): requested AHEAD runs ahead, a group of four tiles is four runs.
-        // Buffer loads: the tile's place in the lane offset, the slot's in a scalar register (as flat loads their 64-bit
-        // addresses cost more vector instructions than the conversions); the buffer ends with the ring, slots past it read 0.
-        // FAR: flat loads, for blocks that reach 2 GiB and more into a layer's value rows.
-        constexpr int RUN = 8, NB = PHASE == 2 ? 8 : 4, AHEAD = NB - 1;
-        uint32_t v[NB][RUN];
-        float4 ev[EL ? 1 : NB][2];
-        const int ng = nt >> 2;
-        const uint64_t vbytes = (uint64_t)a.seq * a.kv_dim * 2;
-        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)a.vc, 0, (uint32_t)(vbytes < 0x7FFFFFFFu ? vbytes : 0x7FFFFFFFu), 0x00020000);
-        const int vcol = (kvh * HD + dg * 32 + 2 * n) * 2, vrow = a.kv_dim * 2;
-        auto fetch = [&](int buf, int g, int i) {
-            g = g < ng ? g : ng - 1;
-            const int ring0 = ((tfirst + 4 * g + c) << 5) % a.seq;
-            if constexpr (FAR) {
-                #pragma unroll
-                for (int k = 0; k < RUN; ++k) {
-                    const int r = ring0 + RUN * i + k < a.seq ? ring0 + RUN * i + k : a.seq - 1;       // (a slot past the ring is no position of the group: zeroed below)
-                    v[buf][k] = *(const uint32_t *)((const uint8_t *)a.vc + (size_t)r * vrow + vcol);
-                }
-            } else {
-                const int off = ring0 * vrow + vcol;
-                #pragma unroll
-                for (int k = 0; k < RUN; ++k) v[buf][k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rv, off, (RUN * i + k) * vrow, 0);
-            }
-            if constexpr (!EL) {
-                const float *et = eb + ((size_t)(4 * g + c) * 16 + n) * ES + RUN * i;
-                ev[buf][0] = *(const float4 *)et; ev[buf][1] = *(const float4 *)(et + 4);
-            }
-        };
+        const int vcol = (kvh * HD + dg * 32 + 2 * n) * 2;
+        if (dg != dg0 + wave) first_runs(dg);
         #pragma unroll
-        for (int i = 0; i < AHEAD; ++i) fetch(i, i >> 2, i & 3);
+        for (int i = 0; i < AHEAD; ++i) fetch_e(i, i >> 2, i & 3);
         for (int g0 = 0; g0 < ng; g0 += NB / 4) {
             #pragma unroll
             for (int h = 0; h < NB / 4; ++h) {
@@ -658,7 +671,8 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
                 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int cur = 4 * h + i;
-                    fetch((cur + AHEAD) % NB, g + ((i + AHEAD) >> 2), (i + AHEAD) & 3);
+                    fetch_v(vcol, (cur + AHEAD) % NB, g + ((i + AHEAD) >> 2), (i + AHEAD) & 3);
+                    fetch_e((cur + AHEAD) % NB, g + ((i + AHEAD) >> 2), (i + AHEAD) & 3);
                     const float *et = eb + ((size_t)(t + c) * 16 + n) * ES + RUN * i;
                     const float4 ea = EL ? *(const float4 *)et : ev[EL ? 0 : cur][0], ec = EL ? *(const float4 *)(et + 4) : ev[EL ? 0 : cur][1];
                     const float e[8] = { ea.x, ea.y, ea.z, ea.w, ec.x, ec.y, ec.z, ec.w };
