@@ -1637,7 +1637,9 @@ static bool far_in_narrow_heads(const lg_hip_model *m, const lg_hip_kv *kv, int 
 }
 // Up to LG_WA_SPLIT_GROUPS workgroups (half of the chip) with 12 tiles and more: scores and values as two launches over more workgroups (200
 // rows, 100 workgroups: 41 -> 39 us in a 512-wide window, 175 -> 113 us over 100 tiles; with 130 workgroups 42 -> 55 us, with 8
-// tiles 23 us both ways).  Score workgroups take 4 tiles, or up to 16 while there are more than 512 of them.
+// tiles 23 us both ways).  Where the weights wait in memory anyway, also wherever the last round of workgroups would leave a fifth of
+// the CU time unused (332 rows at 3001, 166 workgroups: a prompt's 11.68 -> 11.55 ms; 300 rows at 3001, 304 workgroups: 22.18 -> 21.41 ms; with 256 or 512
+// of them 0.5% slower).  Score workgroups take 4 tiles, or up to 16 while there are more than 512 of them.
 // `far`: the block reaches value rows 2 GiB and more behind a layer's first one and takes 64-bit addresses (96 rows, 16 heads of 512
 // over 2, a million positions: 140.9 -> 141.7 ms).  Built for heads of 512; narrower ones go to verify blocks there (far_in_narrow_heads).
 template <int HD>
@@ -1646,7 +1648,9 @@ static void launch_wide_attn(Launcher &lx, const WideAttn &a, int groups, bool f
     const int wgs = groups * a.nkv;
     if constexpr (HD == 512)
         if (far) { LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false, 0, true>), grid, dim3(LG_WA_WG), 0, a, lx.m->ctl); return; }
-    if (wgs <= LG_WA_SPLIT_GROUPS && a.tiles >= 12 && a.tiles <= LG_WA_SPLIT_MAX && (size_t)wgs * a.tiles * (16 * 34 * 4) <= scratch_bytes) {
+    const int round = cu_count(), rounds = (wgs + round - 1) / round;       // one such workgroup of eight wavefronts to a CU
+    const bool split = wgs <= LG_WA_SPLIT_GROUPS || (a.tiles > LG_WA_TILES && 5 * wgs < 4 * rounds * round);
+    if (split && a.tiles >= 12 && a.tiles <= LG_WA_SPLIT_MAX && (size_t)wgs * a.tiles * (16 * 34 * 4) <= scratch_bytes) {
         int chunk = 4;
         while (chunk < 16 && wgs * (a.tiles / chunk) > 512) chunk *= 2;
         LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false, 1>), dim3(groups, a.nkv, (a.tiles + chunk - 1) / chunk), dim3(LG_WA_SPLIT_WG), 0, a, lx.m->ctl);

@@ -119,10 +119,10 @@ def test_long_cache_of_a_model_for_single_rows(lg, ob, gpu_required, model_path)
 
 @pytest.mark.parametrize("name,pos0,n,over", [("tiny", 351, 9, {}), ("tiny", 352, 33, {"sliding_window": 512}), ("tiny_full", 1500, 40, {}), ("tiny", 3000, 22, {"head_dim": 256, "sliding_window": 1024}),
                                               ("tiny", 700, 250, {"head_dim_full": 512}), ("tiny", 701, 61, {"n_head": 12, "n_head_kv": 4, "sliding_window": 512}),
-                                              ("tiny", 1471, 260, {}), ("tiny", 32735, 24, {}), ("tiny", 32760, 24, {})])
+                                              ("tiny", 1471, 260, {}), ("tiny", 1471, 420, {}), ("tiny", 32735, 24, {}), ("tiny", 32760, 24, {})])
 def test_few_rows_late_in_a_context(lg, ob, gpu_required, model_path, name, pos0, n, over):
     """Scores and values as two kernels: from 12 tiles on, heads of 64 to 512 dims, windows and whole contexts, three heads per
-    kv head, on both sides of the rows (128 workgroups) and the tiles (1024) up to which they are used.  Against the same
+    kv head, on both sides of the rows (128 workgroups, 205 of 256 beyond 44 tiles) and the tiles (1024) up to which they are used.  Against the same
     rows through verify blocks, bit for bit; the cache rows in front are drawn."""
     path, spec = model_path(name, **over)
     rng = np.random.default_rng(pos0 + n)
