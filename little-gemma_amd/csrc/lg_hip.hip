@@ -1662,6 +1662,8 @@ static void launch_wide_attn(Launcher &lx, const WideAttn &a, int groups, bool f
 // One block of `rows` prompt positions from pos on (tokens in device memory): the launch sequence of a verify step with
 // the kernels of lg_wide.h.  Launched as it is, not captured: a prompt's blocks differ in width and tile counts, and the
 // host stays ahead of launches of this size.
+// Rows of a prompt block up to which a row's work is cut over its slices and the per-layer gate does the row work ahead of it.
+#define WIDE_FEW_ROWS 64
 static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int rows, int pos) {
     Launcher lx{ m, false };
     const int E = m->E, H = m->H, nl = m->n_layer;
@@ -1678,7 +1680,8 @@ static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, i
         s.dout = pend_dout; s.w_post = pend_w; s.os = pend_os; s.dparts = pend_parts;
         s.w_pre = w_pre;
         if (pend_dout || !have_x) s.x_out = m->x[cur ^ 1];
-        LAUNCH(KC_ROWS, lg_k_wide_rows, dim3(rows), dim3(LG_WG), 0, s, rows);
+        s.slices = rows <= WIDE_FEW_ROWS ? (E + 1023) / 1024 : 1;
+        LAUNCH(KC_ROWS, lg_k_wide_rows, dim3(rows, s.slices), dim3(LG_WG), 0, s, rows);
         if (s.x_out) cur ^= 1;
         have_x = true; pend_dout = pend_w = pend_os = nullptr; pend_parts = 1;
     };
@@ -1723,7 +1726,8 @@ static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, i
         pend_parts = launch_wide_mm<false>(lx, KC_DOWN, y.wdown_w, m->gq, y.nff, E, rows, m->dout, nullptr);
         pend_dout = m->dout; pend_w = y.post_ffw; pend_os = m->ple ? nullptr : y.out_scale;
         if (!m->ple) continue;
-        row_work(nullptr, y.winp_f ? nullptr : m->hq);
+        const bool rows_in_gate = !y.winp_f && rows <= WIDE_FEW_ROWS;
+        if (!rows_in_gate) row_work(nullptr, y.winp_f ? nullptr : m->hq);
         if (y.winp_f) {
             MmfArgs g{ y.winp_f, E, m->ple, m->x[cur], E, rows, m->pgf, m->ple, m->pmp_raw + (size_t)L * m->ple, m->ple * nl };
             launch_mmf<LG_HIP_MAX_ROWS>(lx, KC_PLEGATE, g);
@@ -1733,8 +1737,15 @@ static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, i
         } else {
             // (256 gate rows: at most 4 weight tiles x 16 activation tiles, always eight wavefronts)
             static_assert((256 / LG_WT) * (LG_WIDE_ROWS / 32) <= 256, "lg_k_wide_plegate is built for tiles of 64 x 32 by eight wavefronts");
-            const WideLaunch g = wide_launch(y.winp_w, m->hq, E, m->ple, rows, 1);
-            LAUNCH(KC_PLEGATE, (lg_k_wide_plegate<1, 8>), g.grid, g.block, g.lds, g.a, m->pmp_raw, L, nl, (uint8_t *)m->pq);
+            if (rows_in_gate) {
+                RowsPleGateArgs r{ PleGateArgs{ y.winp, E, m->ple, nullptr, m->pmp_raw, L, nl, m->pq }, m->x[cur], pend_dout, pend_w, m->x[cur ^ 1], m->eps, pend_parts };
+                LAUNCH(KC_PLEGATE, lg_k_wide_rows_plegate, dim3(m->ple / 32, rows), dim3(LG_WG), (size_t)E * 5 / 4, r, rows);
+                cur ^= 1;
+                pend_os = nullptr;
+            } else {
+                const WideLaunch g = wide_launch(y.winp_w, m->hq, E, m->ple, rows, 1);
+                LAUNCH(KC_PLEGATE, (lg_k_wide_plegate<1, 8>), g.grid, g.block, g.lds, g.a, m->pmp_raw, L, nl, (uint8_t *)m->pq);
+            }
             pend_parts = launch_wide_mm<false>(lx, KC_PLEPROJ, y.wproj_w, m->pq, m->ple, E, rows, m->dout, nullptr);
         }
         pend_dout = m->dout; pend_w = y.post_norm; pend_os = y.out_scale;

@@ -728,9 +728,10 @@ struct RowsPleGateArgs {
 // lg_k_ple_tail as the first phase of a longer kernel).  xnew receives the lane's float4s of the updated residual;
 // after_requests runs once every load of the body has been requested (a caller's own loads go there: loads return
 // in the order they were requested, and the row's must not wait behind them).
-template <int M, typename Hook>
-__device__ __forceinline__ void lg_rows_plegate_body(const RowsPleGateArgs &a, int gb, int j, unsigned char *smem, float *gbuf, float *red,
-                                                     float4 (&xnew)[LG_ROWV], bool write_x, Hook &&after_requests) {
+// `rows`: of the block.  sink(gbuf) runs at the end with the 32 gated values in LDS (lg_plegate_q8: their q8 for verify blocks).
+template <typename Hook, typename Sink>
+__device__ __forceinline__ void lg_rows_plegate_body(const RowsPleGateArgs &a, int rows, int gb, int j, unsigned char *smem, float *gbuf, float *red,
+                                                     float4 (&xnew)[LG_ROWV], bool write_x, Hook &&after_requests, Sink &&sink) {
     int8_t *lq = (int8_t *)smem;                              // one row: [E] int8, then [E/32] {scale, sum}
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, E = a.g.k, nit = E >> 8, ple = a.g.ple;
     float2 *lds = (float2 *)(smem + (size_t)E);
@@ -747,7 +748,7 @@ __device__ __forceinline__ void lg_rows_plegate_body(const RowsPleGateArgs &a, i
         #pragma unroll
         for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) { xv[v] = xr[t + 256 * v]; dv[v] = dr[t + 256 * v]; wp[v] = wr[t + 256 * v]; }
         if (a.dparts == 4) {                                  // the top two levels of the tree of an ffn_down cut by K quarter
-            const size_t slab = (size_t)M * nq;
+            const size_t slab = (size_t)rows * nq;
             #pragma unroll
             for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) {
                 const float4 p1 = dr[slab + t + 256 * v], p2 = dr[2 * slab + t + 256 * v], p3 = dr[3 * slab + t + 256 * v], p0 = dv[v];
@@ -756,7 +757,7 @@ __device__ __forceinline__ void lg_rows_plegate_body(const RowsPleGateArgs &a, i
             }
         }
         if (a.dparts == 8) {                                  // the top three levels of the K-segment tree of an ffn_down cut over the 8 XCDs
-            const size_t slab = (size_t)M * nq;
+            const size_t slab = (size_t)rows * nq;
             #pragma unroll
             for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) {
                 const float4 *b = dr + t + 256 * v;
@@ -816,13 +817,18 @@ __device__ __forceinline__ void lg_rows_plegate_body(const RowsPleGateArgs &a, i
         if (c == 0) gbuf[wave * 8 + (lane >> 3)] = lg_gelu(p) * iplv;
     }
     __syncthreads();
+    sink(gbuf);
+}
+template <int M>
+__device__ __forceinline__ void lg_plegate_q8(const PleGateArgs &g, int gb, int j, const float *gbuf) {
+    const int ple = g.ple;
     if (threadIdx.x < 32) {
         const int i = threadIdx.x;
         float d; int sum;
         const int q = lg_quant1_32lanes(gbuf[i], &d, &sum);
         const ActLayout lay = lg_act_layout(ple);
-        a.g.pq[(size_t)j * ple + lg_act_unit(lay, gb * 2 + (i >> 4)) * 16 + (i & 15)] = (int8_t)q;
-        if (i == 0) lg_q8_ds<M>(a.g.pq, ple)[(size_t)j * (ple >> 5) + lg_act_block(lay, gb)] = make_float2(d, __int_as_float(sum));
+        g.pq[(size_t)j * ple + lg_act_unit(lay, gb * 2 + (i >> 4)) * 16 + (i & 15)] = (int8_t)q;
+        if (i == 0) lg_q8_ds<M>(g.pq, ple)[(size_t)j * (ple >> 5) + lg_act_block(lay, gb)] = make_float2(d, __int_as_float(sum));
     }
 }
 template <int M>
@@ -831,7 +837,7 @@ __global__ __launch_bounds__(LG_WG) void lg_k_rows_plegate(LG_RPG_FIELDS(LG_XP, 
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float gbuf[32], red[4];
     float4 xnew[LG_ROWV];
-    lg_rows_plegate_body<M>(a, (int)blockIdx.x, (int)blockIdx.y, smem, gbuf, red, xnew, blockIdx.x == 0, [] {});
+    lg_rows_plegate_body(a, M, (int)blockIdx.x, (int)blockIdx.y, smem, gbuf, red, xnew, blockIdx.x == 0, [] {}, [&](const float *v) { lg_plegate_q8<M>(a.g, blockIdx.x, blockIdx.y, v); });
 }
 
 // lm_head: each workgroup walks `passes` blocks of 64 vocabulary rows (4 wavefronts x 2 groups

@@ -344,11 +344,26 @@ __global__ __launch_bounds__(64 * WV, 2) void lg_k_wide_plegate(WideMm a, const 
     }
 }
 
-// Row kernel of a wide block (lg_k_rows of verify blocks, one workgroup per row, the result as wide digits): residual
-// update, norm, q8.  dparts = 4: dout is four [rows][E] slabs.
+// Per-layer gate of a block of few rows, the residual update ahead of it inside: lg_k_rows_plegate of verify blocks with the result as wide
+// digits, a workgroup per (32 gate rows, block row).  On 64 x 32 tiles 256 gate rows are four workgroups, whose CUs pull a quarter of
+// the matrix and all of the block's digits each: 22 rows at the E4B width 5.0 us for the rows and 9.4 for the gate -> 7.5.
+__global__ __launch_bounds__(LG_WG) void lg_k_wide_rows_plegate(RowsPleGateArgs a, int rows) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ __align__(16) float gbuf[32];
+    __shared__ float red[4];
+    const int gb = blockIdx.x, j = blockIdx.y;
+    float4 xnew[LG_ROWV];
+    lg_rows_plegate_body(a, rows, gb, j, smem, gbuf, red, xnew, gb == 0, [] {}, [&](const float *v) {
+        if (threadIdx.x < 8) lg_wide_quant4(((const float4 *)v)[threadIdx.x], (uint8_t *)a.g.pq, a.g.ple >> 5, j, gb);
+    });
+}
+
+// Row kernel of a wide block (lg_k_rows of verify blocks, the result as wide digits): residual
+// update, norm, q8.  dparts = 4: dout is four [rows][E] slabs.  A workgroup per row, or (blocks of few rows) one per slice of it:
+// each forms the row's sums, stores and quantizes the float4s t + 256 * blockIdx.y of its lanes.
 __global__ __launch_bounds__(LG_WG) void lg_k_wide_rows(RowArgs s, int rows) {
     __shared__ float red[2][4];
-    const int t = threadIdx.x, j = blockIdx.x, E = s.E, nq = E >> 2;
+    const int t = threadIdx.x, j = blockIdx.x, E = s.E, nq = E >> 2, vs = s.slices > 1 ? (int)blockIdx.y : -1;
     float4 xv[LG_ROWV], dv[LG_ROWV], wpost[LG_ROWV], wpre[LG_ROWV];
     if (!s.x) {
         const int tok = s.toks[j];
@@ -401,7 +416,7 @@ __global__ __launch_bounds__(LG_WG) void lg_k_wide_rows(RowArgs s, int rows) {
     if (s.x_out) {
         float4 *xo = (float4 *)(s.x_out + (size_t)j * E);
         #pragma unroll
-        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) xo[t + 256 * v] = xv[v];
+        for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq && (vs < 0 || v == vs)) xo[t + 256 * v] = xv[v];
     }
     if (s.w_pre) {
         float ss = 0.0f;
@@ -419,6 +434,7 @@ __global__ __launch_bounds__(LG_WG) void lg_k_wide_rows(RowArgs s, int rows) {
     #pragma unroll
     for (int v = 0; v < LG_ROWV; ++v) {
         if (t + 256 * v >= nq) break;                        // nq is a multiple of 64: whole wavefronts
+        if (vs >= 0 && v != vs) continue;
         lg_wide_quant4(xv[v], (uint8_t *)s.q, E >> 5, j, (t + 256 * v) >> 3);
     }
 }

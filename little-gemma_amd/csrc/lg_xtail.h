@@ -85,13 +85,13 @@ __global__ __launch_bounds__(LG_WG) void lg_k_ple_tail(StepCtl *ctl, LG_XTAIL_FI
     float4 wpost2[LG_ROWV], wpre[LG_ROWV];
     float osv = 1.0f;
     float4 xv[LG_ROWV];
-    lg_rows_plegate_body<M>(a.r, gb, j, smem, gbuf, red[0], xv, false, [&] {
+    lg_rows_plegate_body(a.r, M, gb, j, smem, gbuf, red[0], xv, false, [&] {
         lg_mm_fetch<G, 1>(pwt, wgp, 0, 1, lane);
         const float4 *w2 = (const float4 *)a.w_post2, *w3 = (const float4 *)a.w_pre;
         #pragma unroll
         for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) { wpost2[v] = w2[t + 256 * v]; wpre[v] = w3[t + 256 * v]; }
         if (a.os) osv = a.os[0];
-    });
+    }, [&](const float *v) { lg_plegate_q8<M>(a.r.g, gb, j, v); });
     stamp(1);
     // ---- hand-over: every unit's 32 gated values of its row are in the XCD's L2 ----
     int8_t *lq2 = (int8_t *)(smem + (size_t)E * 5 / 4);       // [M][ple] int8, [M][ple/32] {scale, sum}

@@ -53,12 +53,13 @@ def test_wide_q8_of_values_that_are_not_finite(lg, gpu_required, k):
     assert np.isfinite(wide["out"].reshape(32, m)[:24]).all() and np.isnan(wide["out"].reshape(32, m)[24:28]).all()
 
 
-@pytest.mark.parametrize("name,n_prompt,over", [("tiny_full", 9, {}), ("tiny_full", 31, {}), ("tiny", 33, {}), ("tiny_full", 65, {}), ("tiny", 129, {}),
+@pytest.mark.parametrize("name,n_prompt,over", [("tiny_full", 9, {}), ("tiny_full", 31, {}), ("tiny", 33, {}), ("tiny_full", 65, {}), ("tiny", 129, {}), ("tiny", 130, {}), ("tiny_full", 97, {}), ("tiny_full", 98, {}), ("tiny_full", 34, {"n_embd": 1280}),
                                                 ("tiny", 70, {"n_ff": 10240}), ("tiny_full", 30, {"n_ff": 10240}), ("tiny", 1303, {}),
                                                 ("tiny", 61, {"n_head": 12, "n_head_kv": 4}), ("tiny_full", 50, {"n_head_kv": 8}), ("tiny", 45, {"head_dim_full": 512})])
 def test_ragged_prompts_leave_the_same_cache_and_logits(lg, ob, gpu_required, model_path, name, n_prompt, over):
     """Blocks of any width (padded inside the kernels only), the gate/up shapes of 64 x 64 tiles, more key tiles than the
-    attention keeps in LDS, query groups that leave units idle (three heads per kv head) or one head each, 512-wide heads."""
+    attention keeps in LDS, query groups that leave units idle (three heads per kv head) or one head each, 512-wide heads; widths around those up to which
+    the per-layer gate does the row work ahead of it and small matrices are cut by K quarter."""
     path, spec = model_path(name, **over)
     check_wide_prefill(lg, ob, path, spec, f"{name} {over}", n_prompt)
 
