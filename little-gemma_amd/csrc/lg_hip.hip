@@ -1602,14 +1602,19 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
 // A matmul of a prompt block (lg_wide.h).  The workgroup's shape: 64 weight rows x 64 activation rows by four wavefronts
 // of two K segments each; 32 activation rows when the block has no more; and where 64 x 32 tiles would leave some CU
 // without a workgroup, eight wavefronts of one segment on such a tile (3072 x 2560, 32 rows, 48 workgroups: 8.8 -> 7.1 us).
-struct WideShape { int tb, wv; };
-static WideShape wide_shape(int m, int rows, int parts) {
-    if (((m + LG_WT - 1) / LG_WT) * ((rows + 31) / 32) * parts <= 256) return { 1, 8 };
-    return { rows <= 32 ? 1 : 2, 4 };
+// `slabs`: the consumer adds four slabs, so that a matrix of 8 segments may be cut by K quarter too: workgroups of two wavefronts,
+// where a quarter of the CUs would do for whole rows (a CU pulls 48 GB/s: 22 rows, 3072 x 2560 on 48 CUs 9.1 us, on 192 6.2).
+struct WideShape { int tb, wv, parts; };
+static WideShape wide_shape(int k, int m, int rows, bool slabs) {
+    const int parts = lg_segments(k) / 8, tiles = ((m + LG_WT - 1) / LG_WT) * ((rows + 31) / 32);
+    if (slabs && parts == 1 && tiles * 4 <= 256 && 4 * rows <= LG_WIDE_ROWS) return { 1, 2, 4 };      // (the slabs lie in a buffer of LG_WIDE_ROWS rows)
+    if (tiles * parts <= 256) return { 1, 8, parts };
+    return { rows <= 32 ? 1 : 2, 4, parts };
 }
 struct WideLaunch { WideMm a; WideShape c; dim3 grid, block; size_t lds; };
-static WideLaunch wide_launch(const uint8_t *w, const int8_t *q, int k, int m, int rows, int parts) {
-    const WideShape c = wide_shape(m, rows, parts);
+static WideLaunch wide_launch(const uint8_t *w, const int8_t *q, int k, int m, int rows, bool slabs = false) {
+    const WideShape c = wide_shape(k, m, rows, slabs);
+    const int parts = c.parts;
     const WideMm a{ w, (const uint8_t *)q, k, m, rows, (rows + 32 * c.tb - 1) / (32 * c.tb), parts };
     return { a, c, dim3(lg_wide_grid(m, a.nb_tiles, parts)), dim3(64 * c.wv), (size_t)c.wv * 2 * c.tb * 4096 };
 }
@@ -1618,9 +1623,10 @@ static WideLaunch wide_launch(const uint8_t *w, const int8_t *q, int k, int m, i
     else if (l.c.tb == 1) LAUNCH(cls, k14, l.grid, l.block, l.lds, l.a, __VA_ARGS__); \
     else LAUNCH(cls, k24, l.grid, l.block, l.lds, l.a, __VA_ARGS__); } while (0)
 template <bool DUMP>
-static int launch_wide_mm(Launcher &lx, int cls, const uint8_t *w, const int8_t *q, int k, int m, int rows, float *out, int32_t *dots) {
-    const WideLaunch l = wide_launch(w, q, k, m, rows, lg_segments(k) / 8);
-    LAUNCH_WIDE(cls, l, (lg_k_wide_mm<1, 8, DUMP>), (lg_k_wide_mm<1, 4, DUMP>), (lg_k_wide_mm<2, 4, DUMP>), out, dots);
+static int launch_wide_mm(Launcher &lx, int cls, const uint8_t *w, const int8_t *q, int k, int m, int rows, float *out, int32_t *dots, bool slabs = false) {
+    const WideLaunch l = wide_launch(w, q, k, m, rows, slabs);
+    if (l.c.wv == 2) LAUNCH(cls, (lg_k_wide_mm<1, 2, DUMP>), l.grid, l.block, l.lds, l.a, out, dots);
+    else LAUNCH_WIDE(cls, l, (lg_k_wide_mm<1, 8, DUMP>), (lg_k_wide_mm<1, 4, DUMP>), (lg_k_wide_mm<2, 4, DUMP>), out, dots);
     return l.a.parts;
 }
 // Whether a prompt block reaches value rows 2 GiB and more behind a layer's first one (524288 positions at the 12B shape), where
@@ -1659,11 +1665,13 @@ static void launch_wide_attn(Launcher &lx, const WideAttn &a, int groups, bool f
     else                               LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false>), grid, dim3(LG_WA_WG), 0, a, lx.m->ctl);
 }
 
+// Rows of a prompt block up to which a row's work is cut over its slices (22 rows 5.0 -> 4.2 us a launch; 99 rows of the 12B shape: a prompt
+// 9251 -> 9286 us), and up to which the per-layer gate does the row work ahead of it (96 rows: 6862 -> 6751 us a prompt, 127: 6937 -> 7012).
+#define WIDE_SLICE_ROWS 64
+#define WIDE_GATE_ROWS 96
 // One block of `rows` prompt positions from pos on (tokens in device memory): the launch sequence of a verify step with
 // the kernels of lg_wide.h.  Launched as it is, not captured: a prompt's blocks differ in width and tile counts, and the
 // host stays ahead of launches of this size.
-// Rows of a prompt block up to which a row's work is cut over its slices and the per-layer gate does the row work ahead of it.
-#define WIDE_FEW_ROWS 64
 static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int rows, int pos) {
     Launcher lx{ m, false };
     const int E = m->E, H = m->H, nl = m->n_layer;
@@ -1680,7 +1688,7 @@ static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, i
         s.dout = pend_dout; s.w_post = pend_w; s.os = pend_os; s.dparts = pend_parts;
         s.w_pre = w_pre;
         if (pend_dout || !have_x) s.x_out = m->x[cur ^ 1];
-        s.slices = rows <= WIDE_FEW_ROWS ? (E + 1023) / 1024 : 1;
+        s.slices = rows <= WIDE_SLICE_ROWS ? (E + 1023) / 1024 : 1;
         LAUNCH(KC_ROWS, lg_k_wide_rows, dim3(rows, s.slices), dim3(LG_WG), 0, s, rows);
         if (s.x_out) cur ^= 1;
         have_x = true; pend_dout = pend_w = pend_os = nullptr; pend_parts = 1;
@@ -1699,8 +1707,9 @@ static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, i
         const Layer &y = m->L[L];
         const int window = (y.is_local && m->window > 0) ? m->window : 0;
         row_work(y.attn_norm, m->hq);
-        launch_wide_mm<false>(lx, KC_QKV, y.wqkv_w, m->hq, E, y.qkv_m, rows, m->qkv, nullptr);
         QkvPostArgs p{};
+        p.parts = launch_wide_mm<false>(lx, KC_QKV, y.wqkv_w, m->hq, E, y.qkv_m, rows, m->qkv, nullptr, true);
+        p.slab = (size_t)rows * y.qkv_m;
         p.qkv = m->qkv; p.ld = y.qkv_m; p.k_off = y.k_off; p.v_off = y.v_off;
         p.H = H; p.nkv = y.nkv; p.hd = y.hd;
         p.q_norm = y.q_norm; p.k_norm = y.k_norm; p.rope_tab = y.rope_tab; p.rope_ff = y.rope_ff;
@@ -1718,15 +1727,15 @@ static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, i
             case 128: launch_wide_attn<128>(lx, a, groups, far, kv->scratch_bytes); break;
             default:  launch_wide_attn<64>(lx, a, groups, far, kv->scratch_bytes);
         }
-        pend_parts = launch_wide_mm<false>(lx, KC_O, y.wo_w, m->aq, y.qd, E, rows, m->dout, nullptr);
+        pend_parts = launch_wide_mm<false>(lx, KC_O, y.wo_w, m->aq, y.qd, E, rows, m->dout, nullptr, true);
         pend_dout = m->dout; pend_w = y.post_attn;
         row_work(y.ffn_norm, m->hq);
-        const WideLaunch gu = wide_launch(y.wgu_w, m->hq, E, 2 * y.nff, rows, 1);
+        const WideLaunch gu = wide_launch(y.wgu_w, m->hq, E, 2 * y.nff, rows);
         LAUNCH_WIDE(KC_GATEUP, gu, (lg_k_wide_geglu<1, 8>), (lg_k_wide_geglu<1, 4>), (lg_k_wide_geglu<2, 4>), (uint8_t *)m->gq);
         pend_parts = launch_wide_mm<false>(lx, KC_DOWN, y.wdown_w, m->gq, y.nff, E, rows, m->dout, nullptr);
         pend_dout = m->dout; pend_w = y.post_ffw; pend_os = m->ple ? nullptr : y.out_scale;
         if (!m->ple) continue;
-        const bool rows_in_gate = !y.winp_f && rows <= WIDE_FEW_ROWS;
+        const bool rows_in_gate = !y.winp_f && rows <= WIDE_GATE_ROWS;
         if (!rows_in_gate) row_work(nullptr, y.winp_f ? nullptr : m->hq);
         if (y.winp_f) {
             MmfArgs g{ y.winp_f, E, m->ple, m->x[cur], E, rows, m->pgf, m->ple, m->pmp_raw + (size_t)L * m->ple, m->ple * nl };
@@ -1743,7 +1752,7 @@ static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, i
                 cur ^= 1;
                 pend_os = nullptr;
             } else {
-                const WideLaunch g = wide_launch(y.winp_w, m->hq, E, m->ple, rows, 1);
+                const WideLaunch g = wide_launch(y.winp_w, m->hq, E, m->ple, rows);
                 LAUNCH(KC_PLEGATE, (lg_k_wide_plegate<1, 8>), g.grid, g.block, g.lds, g.a, m->pmp_raw, L, nl, (uint8_t *)m->pq);
             }
             pend_parts = launch_wide_mm<false>(lx, KC_PLEPROJ, y.wproj_w, m->pq, m->ple, E, rows, m->dout, nullptr);

@@ -1062,6 +1062,7 @@ struct QkvPostArgs {
     uint16_t *kc, *vc;       // this layer's cache (nullptr when it shares another layer's)
     int seq, kv_dim;
     float eps;
+    int parts; size_t slab;       // 4: qkv is four slabs of partial sums, added here as (p0+p1)+(p2+p3)
 };
 // One head vector (hd <= 512 floats) per wavefront, in two steps so that a wavefront with several vectors to do
 // has all their loads in flight first.  lg_head_load: 4 consecutive elements per lane (and 4 more at +256).
@@ -1165,7 +1166,15 @@ __global__ __launch_bounds__(64) void lg_k_qkv_post(QkvPostArgs a, const StepCtl
     const int head = isq ? job : (job - a.H) % a.nkv;
     const float *src = a.qkv + (size_t)j * a.ld + (isq ? (size_t)head * hd : (size_t)(isv ? a.v_off : a.k_off) + (size_t)head * hd);
     const float *w = isq ? a.q_norm : (isv ? nullptr : a.k_norm);
-    const HeadVec<2> h = lg_head_load<2>(src, hd);
+    HeadVec<2> h = lg_head_load<2>(src, hd);
+    if (a.parts == 4) {                                       // four slabs of a matmul cut by K quarter: the top of the segment tree
+        const HeadVec<2> h1 = lg_head_load<2>(src + a.slab, hd), h2 = lg_head_load<2>(src + 2 * a.slab, hd), h3 = lg_head_load<2>(src + 3 * a.slab, hd);
+        #pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            const float4 x0 = h.x[v], x1 = h1.x[v], x2 = h2.x[v], x3 = h3.x[v];
+            h.x[v] = make_float4((x0.x + x1.x) + (x2.x + x3.x), (x0.y + x1.y) + (x2.y + x3.y), (x0.z + x1.z) + (x2.z + x3.z), (x0.w + x1.w) + (x2.w + x3.w));
+        }
+    }
     const HeadVec<2> wv = w ? lg_head_load<2>(w, hd) : h;
     const RopeVals<2> rv = lg_rope_load<2>(a.rope_tab, a.rope_ff, hd);
     lg_head_finish<2>(h, wv, w != nullptr, hd, a.eps, !isv, pos, rv, vec);

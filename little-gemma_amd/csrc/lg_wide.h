@@ -140,14 +140,15 @@ static inline int lg_wide_grid(int m, int nb_tiles, int parts) {
     return 8 * ((nt + per - 1) / per) * nb_tiles;
 }
 
-// The tile's sums.  WV wavefronts: wavefront w runs the 8/WV segments from 8*part + w*8/WV of the K range and leaves their
+// The tile's sums.  WV wavefronts: wavefront w runs the 8/WV segments from 8*part + w*8/WV of the K range (WV = 2: segment 2*part + w) and leaves their
 // sum in lds[w][(ta*TB + tb)*4 + g][lane] as float4 (weight rows 32*ta + 8*g + 4*h + 0..3 of the tile, activation row
 // 32*tb + n, lane = 32*h + n).  Synchronised on return.
 template <int TB, int WV, bool DUMP>
 __device__ __forceinline__ void lg_wide_tile(const WideMm &a, int at, int bt, int part, float4 *lds, int32_t *dots) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31;
-    const int nb = a.k >> 5, nit = nb / (8 * a.parts);
-    const int kb0 = (8 * part + 8 / WV * __builtin_amdgcn_readfirstlane(wave)) * nit;
+    constexpr int SEG = WV == 2 ? 2 : 8;                      // segments of a workgroup (two: a matrix of 8 cut by K quarter)
+    const int nb = a.k >> 5, nit = nb / (SEG * a.parts);
+    const int kb0 = (SEG * part + SEG / WV * __builtin_amdgcn_readfirstlane(wave)) * nit;
     const __amdgpu_buffer_rsrc_t rw = lg_buffer_rsrc(a.w + ((size_t)at * nb + kb0) * LG_WTILE);
     const int sub = TB == 1 ? (bt & 1) : 0;
     const __amdgpu_buffer_rsrc_t rq = lg_buffer_rsrc(a.q + ((size_t)(TB == 1 ? bt >> 1 : bt) * nb + kb0) * LG_QTILE);
@@ -197,7 +198,7 @@ __device__ __forceinline__ void lg_wide_tile(const WideMm &a, int at, int bt, in
     lg_v16f D0, D1;
     lg_v8i a0, a1;
     float dw, xd[2];
-    const int nblk = 8 / WV * nit, last = nblk - 1;
+    const int nblk = SEG / WV * nit, last = nblk - 1;
     auto take = [&](const Ops &q) {                           // a block's weight operands: each 32-row half in both K halves
         #pragma unroll
         for (int i = 0; i < 6; ++i) { const lg_u2 r = lg_pair32(q.a[i]); a0[i] = (int)r.x; a1[i] = (int)r.y; }
@@ -266,6 +267,10 @@ __device__ __forceinline__ void lg_wide_tile(const WideMm &a, int at, int bt, in
 template <int TB, int WV>
 __device__ __forceinline__ float4 lg_wide_sum(const float4 *lds, int u) {
     const int lane = threadIdx.x & 63, st = 2 * TB * 4 * 64;
+    if constexpr (WV == 2) {
+        const float4 a = lds[u * 64 + lane], b = lds[st + u * 64 + lane];
+        return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+    }
     auto quad = [&](int w) {
         const float4 *l = lds + (size_t)w * st + u * 64 + lane;
         const float4 a = l[0], b = l[st], c = l[2 * st], d = l[3 * st];
