@@ -510,9 +510,24 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
     static_assert(PHASE == 0 || !EL, "the two kernels hand the weights over in memory");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), n = lane & 15, c = lane >> 4;
     const int G = a.H / a.nkv, RG = 16 / G, U = RG * G, kvh = blockIdx.y, row0 = blockIdx.x * RG;
-    const int pos = ctl->pos;
+    const int gi = 256 / G + 1;                               // u / G = u * gi >> 8 for u < 16
     int rlast = row0 + RG - 1;
     if (rlast >= a.rows) rlast = a.rows - 1;
+    // the units' query rows are requested first: neither the position nor the K rows are needed for them, and loads return in order
+    // (behind the first tile's rows they were in LDS 4.0 us into a launch of few workgroups: 22 rows of 8 heads of 256 16.0 -> 14.7 us)
+    constexpr int QL = 16 * (HD / 4) / WG;                    // float4 of query per thread (64-wide heads: every second thread)
+    float4 qf[QL < 1 ? 1 : QL];
+    if constexpr (PHASE != 2) {
+        #pragma unroll
+        for (int k = 0; k < (QL < 1 ? 1 : QL); ++k) {
+            const int i = threadIdx.x + k * WG, u = (i / (HD / 4)) & 15, j = i % (HD / 4), ur = u * gi >> 8;
+            int qr = row0 + ur;
+            if (u >= U || qr > rlast) qr = rlast;
+            qf[k] = *(const float4 *)(a.q + (size_t)qr * a.H * HD + (size_t)(kvh * G + (u < U ? u - ur * G : 0)) * HD + 4 * j);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    const int pos = ctl->pos;
     const int kfirst = lg_win_start(pos + row0, a.window), klast = pos + rlast;       // positions any row of the group sees
     const int tfirst = kfirst >> 5, tlast = klast >> 5;
     const int nt = (tlast - tfirst + 4) & ~3;                 // tiles past the last one are masked throughout
@@ -528,7 +543,7 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
         int us[4], up[4];
         #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int u = 4 * c + i, r = row0 + u / G;
+            const int u = 4 * c + i, r = row0 + (u * gi >> 8);
             const bool on = u < U && r <= rlast;
             up[i] = on ? pos + r : -1;
             us[i] = on ? lg_win_start(pos + r, a.window) : 0;
@@ -548,13 +563,13 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
         rows_of(t1, n0, n1);
         #pragma unroll
         for (int s = 0; s < CH; ++s) { w0[s] = *(const uint4 *)(n0 + s * 32); w1[s] = *(const uint4 *)(n1 + s * 32); }
-        // the units' query rows into LDS, chain by chain: [unit][i % 4][i / 4] (in registers a wave's copy of them spilled)
-        for (int i = threadIdx.x; i < 16 * (HD / 4); i += WG) {
-            const int u = i / (HD / 4), j = i - u * (HD / 4), ur = u / G;
-            int qr = row0 + ur;
-            if (u >= U || qr > rlast) qr = rlast;
-            const float4 f = *(const float4 *)(a.q + (size_t)qr * a.H * HD + (size_t)(kvh * G + (u < U ? u - ur * G : 0)) * HD + 4 * j);
-            float *qd = &ob[u][j];
+        // the query rows into LDS, chain by chain: [unit][i % 4][i / 4] (in registers a wave's copy of them spilled)
+        #pragma unroll
+        for (int k = 0; k < (QL < 1 ? 1 : QL); ++k) {
+            const int i = threadIdx.x + k * WG;
+            if (QL < 1 && i >= 16 * (HD / 4)) break;
+            const float4 f = qf[k];
+            float *qd = &ob[i / (HD / 4)][i % (HD / 4)];
             qd[0] = f.x; qd[HD / 4] = f.y; qd[2 * (HD / 4)] = f.z; qd[3 * (HD / 4)] = f.w;
         }
         __syncthreads();
@@ -766,8 +781,8 @@ __global__ __launch_bounds__(PHASE ? LG_WA_SPLIT_WG : LG_WA_WG, 2) void lg_k_wid
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 16 * 8 * ndg; i += WG) {
-        const int u = i / (8 * ndg), qd = 8 * dg0 + i - u * (8 * ndg), r = row0 + u / G;
+        const int u = i / (8 * ndg), qd = 8 * dg0 + i - u * (8 * ndg), ur = u * gi >> 8, r = row0 + ur;
         if (u >= U || r > rlast) continue;                   // (whole groups of 8 lanes)
-        lg_wide_quant4(*(const float4 *)(&ob[u][qd * 4]), a.xq, a.H * HD >> 5, r, (kvh * G + u - u / G * G) * (HD / 32) + (qd >> 3));
+        lg_wide_quant4(*(const float4 *)(&ob[u][qd * 4]), a.xq, a.H * HD >> 5, r, (kvh * G + u - ur * G) * (HD / 32) + (qd >> 3));
     }
 }
