@@ -1320,7 +1320,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
     };
     auto rows_mm = [&](const float *w_pre, const MmArgs &a, int cls) {      // rows(w_pre) then an 8-segment matmul of the result
         if constexpr (M <= LG_FUSE_ROWS_MAX) {
-            constexpr int NW = 1;
+            constexpr int NW = 4;                            // row groups per workgroup, which all repeat the row work (12B shape, 1024 groups: one 2746 us a decode step, two 2670, four 2648; 5 or 10 MB matrices: no difference)
             RowsMmArgs f{ a, row_work(w_pre) };
             const dim3 grid((a.m / 8 + NW - 1) / NW);
             const size_t lds = lds_mm(M, a.k);
