@@ -158,8 +158,8 @@ __global__ __launch_bounds__(LG_WG) void lg_k_rows_mm(LG_ROWSMM_FIELDS(LG_XP, _)
 }
 
 // ---------------------------------------------------------------------------------------------
-// Plain 8-segment matmul for blocks of several rows, the K range of every row group cut over KP wavefronts.
-// With four or more rows the dot phase of lg_k_mm is bound by the instruction issue of its one wavefront per row
+// Plain 8-segment matmul, the K range of every row group cut over KP wavefronts.
+// With one row a wavefront that takes its tiles two at a time waits for memory again and again; with four or more the dot phase of lg_k_mm is bound by the instruction issue of its one wavefront per row
 // group (about 125 instructions per tile at five rows, ten tiles at k = 2560) while half of the chip's SIMDs have
 // nothing to do.  Here wavefront (group, part) takes the tiles [part*nit/KP, (part+1)*nit/KP) of its group: it
 // requests all of them at once, forms the exact block dots and the scale products of its tiles, and the float

@@ -1059,18 +1059,21 @@ static int launch_mm(Launcher &lx, int cls, const MmArgs &a_in, bool slabs_ok = 
         const int cus = cu_count();
         const int W = (ngroups % 5 == 0 && ngroups / 5 <= cus && ngroups / 4 > cus) ? 5 : 4;
         // chunks of four tiles for the longest rows (15 tiles per lane at k = 15360: 3.96 against 4.00 ms per step at
-        // the 12B shape), of two otherwise (10 tiles at k = 10240: 2.602 against 2.618 ms at the E4B shape)
+        // the 12B shape), of two otherwise (10 tiles at k = 10240: 2.602 against 2.618 ms at the E4B shape); one and two rows leave
+        // registers for four (1849 -> 1832 and 1966 -> 1954 us; of eight 1851 and 1988)
         a.nthreads = 64 * W;
-        if ((a.k >> 5) / 32 >= 12) LAUNCH(cls, (lg_k_mm<M, 32, 1, DUMP, 4>), dim3((ngroups + W - 1) / W), dim3(64 * W), lds, LG_MM_FIELDS(LG_XA, a) 0);
+        if ((a.k >> 5) / 32 >= 12 || M <= 2) LAUNCH(cls, (lg_k_mm<M, 32, 1, DUMP, 4>), dim3((ngroups + W - 1) / W), dim3(64 * W), lds, LG_MM_FIELDS(LG_XA, a) 0);
         else                       LAUNCH(cls, (lg_k_mm<M, 32, 1, DUMP>), dim3((ngroups + W - 1) / W), dim3(64 * W), lds, LG_MM_FIELDS(LG_XA, a) 0);
     } else if (ngroups >= 4096) {
         const int W = 4;
         a.nthreads = 64 * W;
         LAUNCH(cls, (lg_k_mm<M, 8, 2, DUMP>), dim3((ngroups + 2 * W - 1) / (2 * W)), dim3(64 * W), lds, LG_MM_FIELDS(LG_XA, a) 0);
-    } else if (M >= 4 && a.k >= 2048 && !DUMP) {
-        // blocks of four and more rows: two row groups per workgroup, the tiles of each cut over two wavefronts
-        // (over four was no faster at 8 and 10 tiles per group)
-        if constexpr (M >= 4) {
+    } else if (a.k >= 2048 && !DUMP) {
+        // two row groups per workgroup, the tiles of each cut over two wavefronts, which request all of theirs at once
+        // (over four was no faster at 8 and 10 tiles per group).  For one row too: a wavefront that takes its tiles two at a time
+        // waits for memory five times (E4B shape, decode 1960 -> 1850 us a step, 2 rows 2050 -> 1960, 3 rows 2125 -> 2034; 12B shape
+        // 2646 -> 2545, 3 rows 3216 -> 3007)
+        if constexpr (!DUMP) {
             const size_t l2 = ((lds + 15) & ~(size_t)15) + (size_t)2 * M * 64 * 4;
             // (over four wavefronts from 12 tiles per group on: 12B shape, k = 3840 and 4096, 3.662 -> 3.645 ms per step)
             a.nthreads = (a.k >> 8) >= 12 ? 512 : 256;
