@@ -142,8 +142,11 @@ __global__ __launch_bounds__(LG_WG) void lg_k_rows_mm(LG_ROWSMM_FIELDS(LG_XP, _)
     const int gi = g0 < ngroups ? g0 : ngroups - 1;
     const uint8_t *wg[1] = { a.mm.w + (size_t)gi * nit * LG_TILE };
     const int row[1] = { gi * 8 + lane / 8 };
-    WChunk<1> first;
-    if (wave < NW) lg_mm_fetch<1>(first, wg, 0, nit, lane);
+    // tiles in flight: what is requested here arrives under the row work (12B shape, 15 tiles, one row: two 2540 us a decode step, four 2479,
+    // eight 2470, sixteen 2509)
+    constexpr int RU = NV == 1 ? 2 : M == 1 ? 8 : 4;          // (rows of up to 1024 values have four tiles at most: 22047 -> 22115 us for 8 draft rounds with eight)
+    WChunk<1, RU> first;
+    if (wave < NW) lg_mm_fetch<1, RU>(first, wg, 0, nit, lane);
     const ActLayout lay = lg_act_layout(k);
     lg_rows_fused<M, NV, 1, lg_rows_batch(M, NV, 40)>(a.rows, blockIdx.x == 0, red, [&](int j, int quad, uint32_t packed, float d, int sum) {
         *(uint32_t *)(lq + (size_t)j * k + (size_t)lg_act_unit(lay, quad >> 2) * 16 + (quad & 3) * 4) = packed;
@@ -152,7 +155,7 @@ __global__ __launch_bounds__(LG_WG) void lg_k_rows_mm(LG_ROWSMM_FIELDS(LG_XP, _)
     __syncthreads();
     if (wave >= NW || g0 >= ngroups) return;
     float acc[1][M];
-    lg_mm_groups<M, 8, 1, false>(wg, first, nit, lq, lds, k, acc, lane, nullptr, a.mm.m, row);
+    lg_mm_groups<M, 8, 1, false, RU>(wg, first, nit, lq, lds, k, acc, lane, nullptr, a.mm.m, row);
     const int c = lane & 7;
     if (c < M) a.mm.out[(size_t)c * a.mm.m + row[0]] = lg_pick<M>(acc[0], c);
 }

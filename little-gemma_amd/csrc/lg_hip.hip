@@ -1312,7 +1312,8 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
     // whose residual is already in memory.  NV = float4 per lane of a row.
     const int NVr = (E + 1023) / 1024;
     // (blocks of one or two rows: wider ones pay more for the repeated row work than for the launch, see lg_fused.h)
-    auto can_fuse = [&]() { return M <= LG_FUSE_ROWS_MAX && have_x && m->fuse_rows && pend_parts == 1; };
+    // (two rows of more than 3072 values: 12B shape, 2862 us a step inside the matmul, 2840 ahead of it)
+    auto can_fuse = [&]() { return (M == 1 || (M <= LG_FUSE_ROWS_MAX && NVr <= 3)) && have_x && m->fuse_rows && pend_parts == 1; };
     auto row_work = [&](const float *w_pre) {
         RowWork r{ m->x[cur], pend_dout, pend_w, pend_os, m->x[cur ^ 1], w_pre, E, m->eps };
         return r;
