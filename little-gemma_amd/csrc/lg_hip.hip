@@ -1068,7 +1068,7 @@ static int launch_mm(Launcher &lx, int cls, const MmArgs &a_in, bool slabs_ok = 
         const int W = 4;
         a.nthreads = 64 * W;
         LAUNCH(cls, (lg_k_mm<M, 8, 2, DUMP>), dim3((ngroups + 2 * W - 1) / (2 * W)), dim3(64 * W), lds, LG_MM_FIELDS(LG_XA, a) 0);
-    } else if (a.k >= 2048 && !DUMP) {
+    } else if (a.k >= 2048 && a.k <= 4096 && !DUMP) {         // (longer rows of 8 segments, a head's pre-projection: more than the 16 tiles a group holds)
         // two row groups per workgroup, the tiles of each cut over two wavefronts, which request all of theirs at once
         // (over four was no faster at 8 and 10 tiles per group).  For one row too: a wavefront that takes its tiles two at a time
         // waits for memory five times (E4B shape, decode 1960 -> 1850 us a step, 2 rows 2050 -> 1960, 3 rows 2125 -> 2034; 12B shape
