@@ -604,7 +604,9 @@ __global__ __launch_bounds__(320, 2) void lg_k_mm_kq(LG_MM_FIELDS(LG_XP, _) int 
 // 16 over 8 at 8192 keys 42 -> 31, at 2048 keys of 8 over 2 15.2 -> 14.2; a 1024-key window of 16 over 8: 12.3 -> 13.1 (two
 // tiles to a workgroup, 136 workgroups).
 // Slots outside a row's keys have weight zero and zeroed values (or ones that another row of the block sees), and
-// fma(0, v, acc) is acc for every acc that a chain started at +0 can hold.
+// fma(0, v, acc) is acc for every acc that a chain started at +0 can hold and every finite v; a tile that gives results that
+// are not finite where the rows' keys differ is computed again without those slots (5 rows of 16 over 8 at 8192 keys: a step
+// 3386 -> 3396 us for the test of the results, which is out of the way of the tiles in between).
 template <int HD>
 struct AttnRowsGeo {
     static constexpr int QST = HD + 4;                        // floats per staged query: [chain][HD/4], off the bank period
@@ -898,6 +900,43 @@ __global__ __launch_bounds__(LG_WG, 2) void lg_k_attn_rows(const StepCtl *ctl, L
                     #pragma unroll
                     for (int k = 0; k < NK; ++k) acc[k] = __builtin_amdgcn_mfma_f32_16x16x1f32(ev[q], vf[s4 & 1][q][k], acc[k], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
+            }
+            // Where the rows' keys may differ within the tile (its slots up to M - 1 behind the first key and M - 1 ahead of the last), a
+            // value that is not finite was a product with weight 0 for the units that do not see its slot: a NaN.  So where a result of
+            // this wavefront is not finite there, all of them are computed again, each from the slots its row sees (the block's own rows
+            // from LDS, the others from the cache).
+            if (__builtin_expect(t0 < start0 + M - 1 || t0 + 31 > plast - (M - 1), 0)) {
+                float o4[4] = {};
+                #pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    #pragma unroll
+                    for (int k = 0; k < NK; ++k) o4[i & 3] = lg_fmaf(acc[k][i], 0.0f, o4[i & 3]);
+                const float odd = (o4[0] + o4[1]) + (o4[2] + o4[3]);
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd != 0.0f) != 0, 0)) {
+                    int n2 = n, c2 = c;
+                    asm volatile("" : "+v"(n2), "+v"(c2));            // (else the addresses of this block are computed ahead of the scores and kept in registers)
+                    const int d0 = (HD >= 128 ? half * (HD / 2) : 0) + NK * n2;
+                    const float *eu = ep + (size_t)(4 * c2) * Geo::EST;
+                    #pragma unroll
+                    for (int k = 0; k < NK; ++k) acc[k] = lg_v16f{};
+                    for (int t = t0 < start0 ? start0 : t0; t <= plast && t < t0 + 32; ++t) {
+                        const uint16_t *vr = (FQ && t >= tnew ? nv + (t - tnew) * HD : a.vc + (size_t)(t % a.seq) * a.kv_dim + (size_t)kvh * HD) + d0;
+                        uint16_t v[4][NK];
+                        #pragma unroll
+                        for (int b = 0; b < 4; ++b)
+                            #pragma unroll
+                            for (int k = 0; k < NK; ++k) v[b][k] = vr[16 * NK * b + k];
+                        #pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            if (t < us[i] || t > up[i]) continue;
+                            const float e = eu[i * Geo::EST + t - t0];
+                            #pragma unroll
+                            for (int b = 0; b < 4; ++b)
+                                #pragma unroll
+                                for (int k = 0; k < NK; ++k) acc[k][4 * b + i] = lg_fmaf(e, lg_h2f(v[b][k]), acc[k][4 * b + i]);
+                        }
+                    }
+                }
             }
             #pragma unroll
             for (int i = 0; i < 4; ++i) {

@@ -14,6 +14,7 @@ import pytest
 
 from conftest import gguf_tensor_span
 from test_gpu_draft import write_head
+from test_gpu_wide import nan_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -247,6 +248,46 @@ def test_shared_tile_attention_prepares_its_own_rows(lg, ob, gpu_required, model
             assert np.array_equal(g[2].view(np.uint32), b[2].view(np.uint32)), opts
         for a, b in zip(cache, base_cache):
             assert np.array_equal(a, b), opts
+
+
+@pytest.mark.parametrize("n0,j,fq", [(2100, 0, 1), (2100, 3, 1), (2100, 7, 1), (2100, 3, 0), (20, 3, 1), (20, 4, 0)])
+def test_a_block_row_of_nan_reaches_no_row_before_it(lg, gpu_required, model_path, model_dir, n0, j, fq):
+    """Verify blocks whose rows share an attention tile (256 and more (tile, kv head) pairs), with a token whose embedding is
+    infinite at row j of the block that a tile boundary cuts, behind a whole window and in the first keys of one: the cache rows in
+    front of it, in every layer, are those of the same block with another token there, and all of them those of the attention kernel
+    per row."""
+    src, spec = model_path("tiny_full", n_head_kv=4, sliding_window=2048)
+    path = os.path.join(str(model_dir), "tiny_full_infinite_token.gguf")
+    shutil.copyfile(src, path)
+    off, nbytes, dims = gguf_tensor_span(path, "token_embd.weight")
+    odd = 77
+    with open(path, "r+b") as f:
+        for b in range(dims[0] // 32):
+            f.seek(off + odd * (nbytes // dims[1]) + b * 18)
+            f.write(b"\x00\x7c")                          # the block's scale: +inf
+    n = 16                                                # two blocks of 8 rows, the second over a tile boundary
+    prompt = np.random.default_rng(j).integers(100, spec["n_vocab"], n0 + n).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, 2160, max_rows=8)
+    try:
+        got = []
+        for shared, token in ((1, int(prompt[n0 + 8 + j])), (1, odd), (0, odd)):
+            gpu.new_cache()
+            gpu.set_option("wide_prefill", 1)
+            gpu.prefill(prompt[:n0], 0)
+            gpu.set_option("wide_prefill", 0)
+            gpu.set_option("attn_rows", shared)
+            gpu.set_option("attn_rows_fq", fq)
+            blocks = prompt[n0:].copy()
+            blocks[8 + j] = token
+            print(f"token {token} at row {j}, shared tiles {shared}, own preparation {fq}", flush=True)
+            gpu.prefill(blocks, n0)
+            got.append([gpu.kv_read(L, w)[np.arange(n0, n0 + n) % gpu.kv_layout(L)[0]] for L in range(spec["n_layer"] - spec["shared_kv_layers"]) for w in (0, 1)])
+        for plain, shared, per_row in zip(*got):
+            assert np.array_equal(shared[:8 + j], plain[:8 + j])
+            assert np.array_equal(nan_rows(shared), nan_rows(per_row))
+        assert all(((a[8 + j] & 0x7FFF) > 0x7C00).any() for a in got[1][2:])
+    finally:
+        gpu.close()
 
 
 SESSION = """

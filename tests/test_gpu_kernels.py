@@ -303,6 +303,51 @@ def test_attention_of_all_rows_of_a_block(lg, ob, gpu_required, H, KV, hd, rows,
     assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
 
 
+def nan_bits(a):
+    """The bits of floats, every NaN as one pattern (which NaN comes out of a sum is not defined)."""
+    return np.where(np.isnan(a), np.uint32(0x7FC00000), a.view(np.uint32))
+
+
+@pytest.mark.parametrize("H,KV,hd,rows,window,seq,pos", [
+    (12, 2, 256, 7, 4100, 4128, 9000),     # three groups of units, the window's ends inside tiles, the ring wrapped
+    (8, 2, 256, 4, 4096, 4608, 4607),      # one group, the rows' last tile wraps to the ring's start
+    (16, 8, 256, 5, 1024, 1536, 1533),     # the rows' last tiles on both sides of the ring's end
+    (16, 2, 128, 8, 0, 4192, 4150),        # a whole context, stale rows behind it
+    (8, 1, 64, 2, 8200, 8224, 20001),      # an odd number of tiles
+    (16, 4, 256, 8, 2048, 2560, 2050)])    # two groups of units
+def test_attention_values_that_are_not_finite(lg, ob, gpu_required, H, KV, hd, rows, window, seq, pos):
+    """256 and more (tile, kv head) pairs, where the rows of a block share a tile.  Infinities and NaN in the K and V rows that no row
+    of the block sees change no bit; in the value row that only the first row still sees and in the one that only the last row sees
+    they reach those rows alone; in one that all rows see, all of them.  Each against the oracle's row by row."""
+    rng = np.random.default_rng(H * 100 + rows)
+    kc = rng.normal(0, 1, (seq, KV * hd)).astype(np.float16).view(np.uint16)
+    vc = rng.normal(0, 1, (seq, KV * hd)).astype(np.float16).view(np.uint16)
+    q = (rng.normal(0, 1, (rows, H * hd)) * 0.1).astype(np.float32)
+    run = lambda k, v: lg.hiplib.attention(q, k, v, H, KV, hd, window, pos)[0]  # noqa: E731
+    start = max(0, pos - window + 1) if window else 0
+    seen = np.zeros(seq, bool)
+    seen[np.arange(start, pos + rows) % seq] = True
+    assert not seen.all()
+    stale_k, stale_v = kc.copy(), vc.copy()
+    stale_k[~seen] = 0x7E00
+    stale_v[~seen, 0::3], stale_v[~seen, 1::3], stale_v[~seen, 2::3] = 0x7C00, 0xFC00, 0x7E00
+    print(f"attention H={H} KV={KV} hd={hd} rows={rows} window={window} seq={seq} pos={pos}: stale rows", flush=True)
+    plain = run(stale_k, stale_v)
+    want = oracle_attention(ob, q, kc, vc, H, KV, hd, window, pos)
+    assert np.isfinite(plain).all() and np.array_equal(plain.view(np.uint32), want.view(np.uint32))
+    first_only = bool(window) and start > 0                  # (else every row sees the first key)
+    for name, at, sees in (("the first key", start, np.arange(rows) == 0 if first_only else np.ones(rows, bool)),
+                           ("the last row's", pos + rows - 1, np.arange(rows) == rows - 1),
+                           ("a row that all see", pos, np.ones(rows, bool))):
+        odd = stale_v.copy()
+        odd[at % seq, 0::5], odd[at % seq, 1::5], odd[at % seq, 7::5] = 0x7C00, 0xFC00, 0x7E00
+        print(f"  {name}", flush=True)
+        got = run(stale_k, odd)
+        assert np.array_equal(got[~sees].view(np.uint32), plain[~sees].view(np.uint32)), name
+        assert not np.isfinite(got[sees]).all(1).any(), name
+        assert np.array_equal(nan_bits(got), nan_bits(oracle_attention(ob, q, stale_k, odd, H, KV, hd, window, pos))), name
+
+
 def test_bad_arguments_are_refused(lg, gpu_required):
     rng = np.random.default_rng(1)
     with pytest.raises(lg.hiplib.HipError):
