@@ -267,6 +267,7 @@ struct lg_hip_kv {
     unsigned id = 0;
 };
 static unsigned g_kv_ids = 0;
+static int cu_count();
 
 template <typename T>
 static int dev_alloc(lg_hip_model *m, T **p, size_t n) {
@@ -284,6 +285,7 @@ extern "C" int lg_hip_model_create(const struct lg_hip_config *c, int device, lg
     if (c->n_embd_per_layer % 32) return fail(-2, "model_create: per-layer embedding width %d must be a multiple of 256 or 0", c->n_embd_per_layer);
     if (lg_hip_device_count() <= device) return fail(-3, "model_create: no HIP device %d (the verify step has no CPU path)", device);
     HIP_TRY(hipSetDevice(device));
+    if (cu_count() <= 0) return fail(-3, "model_create: device %d does not tell its number of compute units", device);      // (launches are cut by it)
     lg_hip_model *m = new lg_hip_model();
     m->device = device;
     m->n_layer = c->n_layer; m->E = c->n_embd; m->H = c->n_head; m->n_vocab = c->n_vocab;
@@ -404,7 +406,6 @@ static void push_rows(std::vector<const uint8_t *> &rows, const HostTensor *t, u
     for (uint64_t r = r0; r < r0 + n; ++r) rows.push_back((const uint8_t *)t->data + r * rb);
 }
 
-static int cu_count();
 
 // ---- weight streams of the XCD-partitioned feed-forward kernel (lg_xffn.h) --------------------------
 // Shapes it is instantiated for: { gate/up operands per workgroup, blocks per gate/up segment (capacity), ffn_down
@@ -1025,10 +1026,10 @@ static void launch_timed(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds
     else hipLaunchKernelGGL(kernel, grid, block, lds, lx.stream(), __VA_ARGS__); \
     lx.end(); } } while (0)
 
-// Compute units of the current device (asked once).
+// Compute units of the current device (asked until it answers); 0 when it does not, and then no model is created.
 static int cu_count() {
-    static int n = -1;
-    if (n < 0) {
+    static int n = 0;
+    if (n <= 0) {
         int dev = 0, v = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) v = 0;
         n = v;

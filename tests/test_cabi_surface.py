@@ -5,6 +5,7 @@ import os
 import re
 import shutil
 import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -109,6 +110,42 @@ def test_compute_calls_fail_loudly_without_a_device(lg, model_path):
     path, _ = model_path("tiny")
     with pytest.raises(lg.hiplib.HipError, match="no HIP device"):
         lg.hiplib.HipBackend(path, 64)
+
+
+RUNTIME_WITHOUT_A_COUNT = """
+int hipGetDeviceCount(int *n) { *n = 1; return 0; }
+int hipSetDevice(int d) { return d; }
+int hipGetDevice(int *d) { *d = 0; return 0; }
+int hipDeviceGetAttribute(int *v, int what, int d) { *v = 0; return 1 + 0 * (what + d); }
+int hipStreamCreateWithFlags(void **s, unsigned f) { *s = (void *)0; return 0 * f; }
+int hipEventCreateWithFlags(void **e, unsigned f) { *e = (void *)0; return 0 * f; }
+"""
+CREATE = """
+import ctypes as C, sys
+H = C.CDLL(sys.argv[1])
+H.lg_hip_last_error.restype = C.c_char_p
+class Config(C.Structure):
+    _fields_ = [(n, C.c_int32) for n in "n_layer n_embd n_head n_vocab sliding_window n_embd_per_layer n_kv_start".split()] + [
+        (n, C.c_float) for n in "rms_eps rope_freq_base rope_freq_base_swa logit_softcap".split()] + [
+        (n, C.POINTER(C.c_int32)) for n in "is_local ffn_len head_dim n_head_kv".split()]
+one = lambda v: (C.c_int32 * 1)(v)
+c = Config(1, 256, 4, 256, 0, 0, 1, 1e-6, 1e4, 1e4, 0.0, one(0), one(512), one(64), one(1))
+m = C.c_void_p()
+print(H.lg_hip_device_count(), H.lg_hip_model_create(C.byref(c), 0, C.byref(m)), bool(m), H.lg_hip_last_error().decode(), flush=True)
+"""
+
+
+@pytest.mark.skipif(has_gpu() or not shutil.which("gcc"), reason="stands in for the HIP runtime of a machine without a GPU")
+def test_no_model_on_a_device_that_does_not_tell_its_compute_units(lg, tmp_path):
+    """The launches of a prompt are cut by the number of compute units; a model without it would divide by zero there."""
+    lg.hiplib.load_hip()
+    src, stub = tmp_path / "runtime.c", str(tmp_path / "runtime.so")
+    src.write_text(RUNTIME_WITHOUT_A_COUNT)
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", stub], check=True)
+    env = dict(os.environ, LD_PRELOAD=" ".join(filter(None, (stub, os.environ.get("LD_PRELOAD")))))
+    so = os.path.join(ROOT, "little-gemma_amd", "csrc", "liblg_hip.so")
+    r = subprocess.run([sys.executable, "-c", CREATE, so], env=env, capture_output=True, text=True, timeout=60)
+    assert r.stdout.startswith("1 -3 False ") and "compute units" in r.stdout, (r.stdout, r.stderr)
 
 
 def test_model_hip_compiles_against_the_reference_headers():
