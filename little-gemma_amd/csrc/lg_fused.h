@@ -601,15 +601,147 @@ __global__ __launch_bounds__(320, 2) void lg_k_mm_kq(LG_MM_FIELDS(LG_XP, _) int 
 // Bound by its products (32 cycles each, 128 to a wavefront and tile) and about 500 vector instructions beside them, which run
 // one after the other; without the tile's loads and the partials' stores it takes 28 of its 33 us.  On the vector units, every K and V
 // row through LDS and three units to a read, LDS reads bounded it.  8 rows of 8 heads over 2 at 20011 keys 61 -> 33 us, 5 rows of
-// 16 over 8 at 8192 keys 42 -> 31, at 2048 keys of 8 over 2 15.2 -> 14.2; a 1024-key window of 16 over 8: 12.3 -> 13.1 (two
-// tiles to a workgroup, 136 workgroups).
+// 16 over 8 at 8192 keys 42 -> 31, at 2048 keys of 8 over 2 15.2 -> 14.2.
 // Slots outside a row's keys have weight zero and zeroed values (or ones that another row of the block sees), and
 // fma(0, v, acc) is acc for every acc that a chain started at +0 can hold and every finite v; a tile that gives results that
 // are not finite where the rows' keys differ is computed again without those slots (5 rows of 16 over 8 at 8192 keys: a step
 // 3386 -> 3396 us for the test of the results, which is out of the way of the tiles in between).
+//
+// Few units on few tiles go to lg_k_attn_few below.
+
+// What both kernels do themselves where FQ: the queries of the workgroup's kv head, and the block's K and V rows that lie in its tiles
+// (`mine`: whether position t does).  The queries arrive in LDS as [unit][c][HD/4], element i at c = i % 4, i / 4, QST floats a unit.
+template <int M, int HD>
+struct AttnRowsPrep {
+    static constexpr int QST = HD + 4;                        // floats per staged query: off the bank period
+    static constexpr int JOBS = 2 * ((M + 3) / 4);            // K and V rows of the block one wavefront may have to build
+    static constexpr int QBATCH = 4;                          // queries one wavefront prepares at a time
+    HeadVec<1> hj[JOBS], hq[QBATCH], wk, wq;
+    RopeVals<1> rv;
+    // What the preparation reads is requested ahead of the tile (loads return in order): the block's projections
+    // come from the cache levels, the tile from memory, so the queries are prepared while the tile is on its way.
+    template <typename Mine>
+    __device__ __forceinline__ void request(const AttnArgs &a, int kvh, int G, int wave, int tnew, bool any, Mine &&mine) {
+        const int units = M * G;
+        rv = lg_rope_load<1>(a.rope_tab, a.rope_ff, HD);
+        wq = lg_head_load<1>(a.q_norm, HD);
+        #pragma unroll
+        for (int b = 0; b < QBATCH; ++b) {                    // unit u = (row j, head g), by wavefront u % 4
+            const int u = wave + b * (LG_WG / 64) < units ? wave + b * (LG_WG / 64) : min(wave, units - 1), j = u / G, g = u - j * G;
+            hq[b] = lg_head_load<1>(a.qkv + (size_t)j * a.ld + (size_t)(kvh * G + g) * HD, HD);
+        }
+        wk = lg_head_load<1>(any ? a.k_norm : a.q_norm, HD);  // (no K rows to build: k_norm may not exist)
+        #pragma unroll
+        for (int u = 0; u < JOBS; ++u) {                      // first half of the slots: K rows wave, wave+4; second half: V rows 3-wave, 7-wave
+            const bool isv = u >= JOBS / 2;
+            const int r = (isv ? 3 - wave : wave) + 4 * (u % (JOBS / 2)), t = tnew + r;
+            if (any && r < M && mine(t)) hj[u] = lg_head_load<1>(a.qkv + (size_t)r * a.ld + (isv ? a.v_off : a.k_off) + (size_t)kvh * HD, HD);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __device__ __forceinline__ void queries(const AttnArgs &a, const StepCtl *ctl, int kvh, int G, int wave, int lane, float *qs) {
+        const int units = M * G;
+        // a batch in stages, so that the sums and the rotary of its queries overlap: norms of all, each into its own
+        // slot of qs in natural order; all rotary pairs read back; then the slots rewritten in the staged order
+        // (a unit past the last repeats the batch's first one, a slot of this wavefront, and stores nothing)
+        auto unit_of = [&](int base, int b) { return base + b * (LG_WG / 64) < units ? base + b * (LG_WG / 64) : base; };
+        for (int base = wave; base < units; base += QBATCH * (LG_WG / 64)) {
+            if (base != wave) {
+                #pragma unroll
+                for (int b = 0; b < QBATCH; ++b) {
+                    const int u = unit_of(base, b), j = u / G, g = u - j * G;
+                    hq[b] = lg_head_load<1>(a.qkv + (size_t)j * a.ld + (size_t)(kvh * G + g) * HD, HD);
+                }
+            }
+            HeadVec<1> nq[QBATCH];
+            #pragma unroll
+            for (int b = 0; b < QBATCH; ++b) nq[b] = lg_head_norm<1>(hq[b], wq, true, HD, a.eps);
+            #pragma unroll
+            for (int b = 0; b < QBATCH; ++b)
+                if (4 * lane < HD) *(float4 *)(qs + (size_t)unit_of(base, b) * QST + 4 * lane) = nq[b].x[0];
+            lg_wave_lds_sync();
+            float lo[QBATCH][2], hi[QBATCH][2];
+            #pragma unroll
+            for (int b = 0; b < QBATCH; ++b) {
+                const int u = unit_of(base, b), j = u / G;
+                const float *vec = qs + (size_t)u * QST;
+                #pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int p = min(lane + 64 * i, HD / 2 - 1);
+                    const float ang = (float)(ctl->pos + j) * rv.tab[i] / rv.ff[i];
+                    float sn, cs;
+                    lg_sincosf(ang, &sn, &cs);
+                    const float x0 = vec[p], x1 = vec[p + HD / 2];
+                    lo[b][i] = x0 * cs - x1 * sn; hi[b][i] = x0 * sn + x1 * cs;
+                }
+            }
+            lg_wave_lds_sync();                               // (LDS serves a wavefront in order: every read above is ahead of the stores below)
+            #pragma unroll
+            for (int b = 0; b < QBATCH; ++b) {
+                const int u = base + b * (LG_WG / 64);
+                float *qd = qs + (size_t)unit_of(base, b) * QST;
+                #pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int p = lane + 64 * i, p1 = p + HD / 2;
+                    if (u >= units || p >= HD / 2) continue;
+                    qd[(p & 3) * (HD / 4) + (p >> 2)] = lo[b][i];
+                    qd[(p1 & 3) * (HD / 4) + (p1 >> 2)] = hi[b][i];
+                }
+            }
+            lg_wave_lds_sync();
+        }
+    }
+    // k_row(r, t, lo, hi per rotary pair p), v_row(r, t, the lane's four values as f16)
+    template <typename Mine, typename KRow, typename VRow>
+    __device__ __forceinline__ void rows(const AttnArgs &a, int wave, int lane, int tnew, float *vec, Mine &&mine, KRow &&k_row, VRow &&v_row) {
+        HeadVec<1> nr[JOBS];
+        bool on[JOBS];
+        #pragma unroll
+        for (int u = 0; u < JOBS; ++u) {                      // the norms of all of them first: their sums overlap
+            const bool isv = u >= JOBS / 2;
+            const int r = (isv ? 3 - wave : wave) + 4 * (u % (JOBS / 2)), t = tnew + r;
+            on[u] = r < M && mine(t);
+            if (on[u]) nr[u] = lg_head_norm<1>(hj[u], wk, !isv, HD, a.eps);
+        }
+        #pragma unroll
+        for (int u = 0; u < JOBS; ++u) {
+            const bool isv = u >= JOBS / 2;
+            const int r = (isv ? 3 - wave : wave) + 4 * (u % (JOBS / 2)), t = tnew + r;
+            if (!on[u]) continue;
+            if (isv) {                                        // V: no rotary, straight from the registers
+                if (4 * lane < HD) v_row(r, t, make_uint2((uint32_t)lg_f2h(nr[u].x[0].x) | ((uint32_t)lg_f2h(nr[u].x[0].y) << 16),
+                                                          (uint32_t)lg_f2h(nr[u].x[0].z) | ((uint32_t)lg_f2h(nr[u].x[0].w) << 16)));
+            } else lg_head_rope<1>(nr[u], HD, t, rv, vec, [&](int p, float lo, float hi) { k_row(r, t, p, lg_f2h(lo), lg_f2h(hi)); });
+        }
+    }
+    // FQ = false: the queries as lg_k_qkv_post left them
+    __device__ static __forceinline__ void copy_queries(const AttnArgs &a, int kvh, int G, float *qs) {
+        const int units = M * G;
+        constexpr int QB = 4;                                 // float4 of query per thread and pass
+        const int nq4 = units * (HD / 4);
+        for (int base = 0; base < nq4; base += QB * LG_WG) {
+            float4 qreg[QB];
+            #pragma unroll
+            for (int i = 0; i < QB; ++i) {
+                const int idx = min(base + (int)threadIdx.x + i * LG_WG, nq4 - 1);
+                const int u = idx / (HD / 4), g4 = idx - u * (HD / 4), j = u / G, g = u - j * G;
+                qreg[i] = *(const float4 *)(a.q + (size_t)j * a.H * HD + (size_t)(kvh * G + g) * HD + 4 * g4);
+            }
+            #pragma unroll
+            for (int i = 0; i < QB; ++i) {
+                const int idx = base + (int)threadIdx.x + i * LG_WG;
+                if (idx < nq4) {
+                    const int u = idx / (HD / 4), g4 = idx - u * (HD / 4);
+                    float *qd = qs + (size_t)u * QST + g4;
+                    qd[0] = qreg[i].x; qd[HD / 4] = qreg[i].y; qd[2 * (HD / 4)] = qreg[i].z; qd[3 * (HD / 4)] = qreg[i].w;
+                }
+            }
+        }
+    }
+};
 template <int HD>
 struct AttnRowsGeo {
-    static constexpr int QST = HD + 4;                        // floats per staged query: [chain][HD/4], off the bank period
+    static constexpr int QST = HD + 4;
     static constexpr int EST = 36;                            // floats per unit's weights of a tile
     static size_t bytes(int units, bool fq) {         // fq: the block's K and V rows, and a vector of staging per wavefront for the rotary
         return (size_t)((units + 15) / 16) * 16 * QST * 4 + (size_t)2 * 16 * EST * 4 + (fq ? (size_t)2 * LG_HIP_MAX_ROWS_DEV * HD * 2 + (size_t)(LG_WG / 64) * HD * 4 : 0);
@@ -641,30 +773,9 @@ __global__ __launch_bounds__(LG_WG, 2) void lg_k_attn_rows(const StepCtl *ctl, L
     if (b0 >= nb) return;                                     // no row of the block has keys here
     auto mine = [&](int t) { return (((t >> 5) - first) / tw) % gx == b0; };      // position t lies in a tile of this workgroup
 
-    constexpr int JOBS = 2 * ((M + 3) / 4);                   // FQ: K and V rows of the block one wavefront may have to build
-    constexpr int QBATCH = 4;                                 // FQ: queries one wavefront prepares at a time
-    HeadVec<1> hj[FQ ? JOBS : 1], hq[FQ ? QBATCH : 1], wk, wq;
-    RopeVals<1> rv;
     const bool any = FQ && tnew <= plast && (mine(tnew) || mine(plast));         // this workgroup's tiles hold rows of the block (at most two tiles do)
-    if constexpr (FQ) {
-        // What the preparation reads is requested ahead of the tile (loads return in order): the block's projections
-        // come from the cache levels, the tile from memory, so the queries are prepared while the tile is on its way.
-        rv = lg_rope_load<1>(a.rope_tab, a.rope_ff, HD);
-        wq = lg_head_load<1>(a.q_norm, HD);
-        #pragma unroll
-        for (int b = 0; b < QBATCH; ++b) {                    // unit u = (row j, head g), by wavefront u % 4
-            const int u = wave + b * (LG_WG / 64) < units ? wave + b * (LG_WG / 64) : min(wave, units - 1), j = u / G, g = u - j * G;
-            hq[b] = lg_head_load<1>(a.qkv + (size_t)j * a.ld + (size_t)(kvh * G + g) * HD, HD);
-        }
-        wk = lg_head_load<1>(any ? a.k_norm : a.q_norm, HD);  // (no K rows to build: k_norm may not exist)
-        #pragma unroll
-        for (int u = 0; u < JOBS; ++u) {                      // first half of the slots: K rows wave, wave+4; second half: V rows 3-wave, 7-wave
-            const bool isv = u >= JOBS / 2;
-            const int r = (isv ? 3 - wave : wave) + 4 * (u % (JOBS / 2)), t = tnew + r;
-            if (any && r < M && mine(t)) hj[u] = lg_head_load<1>(a.qkv + (size_t)r * a.ld + (isv ? a.v_off : a.k_off) + (size_t)kvh * HD, HD);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
+    AttnRowsPrep<M, HD> prep;
+    if constexpr (FQ) prep.request(a, kvh, G, wave, tnew, any, mine);
     // a tile: this lane's key (K row, 64-byte pieces by four lanes) and its dims of every slot's value row
     constexpr int NS = HD / 32, NK = HD >= 128 ? HD / 128 : 1;          // pieces of a K row; value products per slot and wavefront
     uint4 kw[NS];
@@ -693,111 +804,18 @@ __global__ __launch_bounds__(LG_WG, 2) void lg_k_attn_rows(const StepCtl *ctl, L
     fetch_v(b0);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (FQ) {
-        // a batch in stages, so that the sums and the rotary of its queries overlap: norms of all, each into its own
-        // slot of qs in natural order; all rotary pairs read back; then the slots rewritten in the staged order
-        // (a unit past the last repeats the batch's first one, a slot of this wavefront, and stores nothing)
-        auto unit_of = [&](int base, int b) { return base + b * (LG_WG / 64) < units ? base + b * (LG_WG / 64) : base; };
-        for (int base = wave; base < units; base += QBATCH * (LG_WG / 64)) {
-            if (base != wave) {
-                #pragma unroll
-                for (int b = 0; b < QBATCH; ++b) {
-                    const int u = unit_of(base, b), j = u / G, g = u - j * G;
-                    hq[b] = lg_head_load<1>(a.qkv + (size_t)j * a.ld + (size_t)(kvh * G + g) * HD, HD);
-                }
-            }
-            HeadVec<1> nq[QBATCH];
-            #pragma unroll
-            for (int b = 0; b < QBATCH; ++b) nq[b] = lg_head_norm<1>(hq[b], wq, true, HD, a.eps);
-            #pragma unroll
-            for (int b = 0; b < QBATCH; ++b)
-                if (4 * lane < HD) *(float4 *)(qs + (size_t)unit_of(base, b) * Geo::QST + 4 * lane) = nq[b].x[0];
-            lg_wave_lds_sync();
-            float lo[QBATCH][2], hi[QBATCH][2];
-            #pragma unroll
-            for (int b = 0; b < QBATCH; ++b) {
-                const int u = unit_of(base, b), j = u / G;
-                const float *vec = qs + (size_t)u * Geo::QST;
-                #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const int p = min(lane + 64 * i, HD / 2 - 1);
-                    const float ang = (float)(ctl->pos + j) * rv.tab[i] / rv.ff[i];
-                    float sn, cs;
-                    lg_sincosf(ang, &sn, &cs);
-                    const float x0 = vec[p], x1 = vec[p + HD / 2];
-                    lo[b][i] = x0 * cs - x1 * sn; hi[b][i] = x0 * sn + x1 * cs;
-                }
-            }
-            lg_wave_lds_sync();                               // (LDS serves a wavefront in order: every read above is ahead of the stores below)
-            #pragma unroll
-            for (int b = 0; b < QBATCH; ++b) {
-                const int u = base + b * (LG_WG / 64);
-                float *qd = qs + (size_t)unit_of(base, b) * Geo::QST;
-                #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const int p = lane + 64 * i, p1 = p + HD / 2;
-                    if (u >= units || p >= HD / 2) continue;
-                    qd[(p & 3) * (HD / 4) + (p >> 2)] = lo[b][i];
-                    qd[(p1 & 3) * (HD / 4) + (p1 >> 2)] = hi[b][i];
-                }
-            }
-            lg_wave_lds_sync();
-        }
-        if (any) {                                            // the rows of the block in the workgroup's tiles
-            float *vec = hv + (size_t)wave * HD;
-            HeadVec<1> nr[JOBS];
-            bool on[JOBS];
-            #pragma unroll
-            for (int u = 0; u < JOBS; ++u) {                  // the norms of all of them first: their sums overlap
-                const bool isv = u >= JOBS / 2;
-                const int r = (isv ? 3 - wave : wave) + 4 * (u % (JOBS / 2)), t = tnew + r;
-                on[u] = r < M && mine(t);
-                if (on[u]) nr[u] = lg_head_norm<1>(hj[u], wk, !isv, HD, a.eps);
-            }
-            #pragma unroll
-            for (int u = 0; u < JOBS; ++u) {
-                const bool isv = u >= JOBS / 2;
-                const int r = (isv ? 3 - wave : wave) + 4 * (u % (JOBS / 2)), t = tnew + r;
-                if (!on[u]) continue;
-                const size_t coff = (size_t)(t % a.seq) * a.kv_dim + (size_t)kvh * HD;
-                if (isv) {                                    // V: no rotary, straight from the registers
-                    if (4 * lane < HD) {
-                        const uint2 h4 = make_uint2((uint32_t)lg_f2h(nr[u].x[0].x) | ((uint32_t)lg_f2h(nr[u].x[0].y) << 16),
-                                                    (uint32_t)lg_f2h(nr[u].x[0].z) | ((uint32_t)lg_f2h(nr[u].x[0].w) << 16));
-                        *(uint2 *)(nv + r * HD + 4 * lane) = h4;
-                        *(uint2 *)(a.vcw + coff + 4 * lane) = h4;
-                    }
-                } else {
-                    uint16_t *row = nk + r * HD, *crow = a.kcw + coff;
-                    lg_head_rope<1>(nr[u], HD, t, rv, vec, [&](int p, float lo, float hi) {
-                        const uint16_t hl = lg_f2h(lo), hh = lg_f2h(hi);
-                        row[p] = hl; row[p + HD / 2] = hh;
-                        crow[p] = hl; crow[p + HD / 2] = hh;
-                    });
-                }
-            }
-        }
-    } else {   // the queries, once per workgroup
-        constexpr int QB = 4;                                 // float4 of query per thread and pass
-        const int nq4 = units * (HD / 4);
-        for (int base = 0; base < nq4; base += QB * LG_WG) {
-            float4 qreg[QB];
-            #pragma unroll
-            for (int i = 0; i < QB; ++i) {
-                const int idx = min(base + (int)threadIdx.x + i * LG_WG, nq4 - 1);
-                const int u = idx / (HD / 4), g4 = idx - u * (HD / 4), j = u / G, g = u - j * G;
-                qreg[i] = *(const float4 *)(a.q + (size_t)j * a.H * HD + (size_t)(kvh * G + g) * HD + 4 * g4);
-            }
-            #pragma unroll
-            for (int i = 0; i < QB; ++i) {
-                const int idx = base + (int)threadIdx.x + i * LG_WG;
-                if (idx < nq4) {
-                    const int u = idx / (HD / 4), g4 = idx - u * (HD / 4);
-                    float *qd = qs + (size_t)u * Geo::QST + g4;
-                    qd[0] = qreg[i].x; qd[HD / 4] = qreg[i].y; qd[2 * (HD / 4)] = qreg[i].z; qd[3 * (HD / 4)] = qreg[i].w;
-                }
-            }
-        }
-    }
+        prep.queries(a, ctl, kvh, G, wave, lane, qs);
+        if (any) prep.rows(a, wave, lane, tnew, hv + (size_t)wave * HD, mine,       // the rows of the block in the workgroup's tiles
+            [&](int r, int t, int p, uint16_t lo, uint16_t hi) {
+                uint16_t *row = nk + r * HD + p, *crow = a.kcw + (size_t)(t % a.seq) * a.kv_dim + (size_t)kvh * HD + p;
+                row[0] = lo; row[HD / 2] = hi;
+                crow[0] = lo; crow[HD / 2] = hi;
+            },
+            [&](int r, int t, uint2 h4) {
+                *(uint2 *)(nv + r * HD + 4 * lane) = h4;
+                *(uint2 *)(a.vcw + (size_t)(t % a.seq) * a.kv_dim + (size_t)kvh * HD + 4 * lane) = h4;
+            });
+    } else AttnRowsPrep<M, HD>::copy_queries(a, kvh, G, qs);      // once per workgroup
     __syncthreads();
     for (int it = 0; it < ng; it += 2) {                      // unit groups of the pair (more than two: heads of more than 4 to a kv head)
         const int ug = ng == 1 ? 0 : it + pair;
@@ -954,6 +972,191 @@ __global__ __launch_bounds__(LG_WG, 2) void lg_k_attn_rows(const StepCtl *ctl, L
             fetch_v(bb + gx);
         }
     }
+}
+
+// The same for few units (attention_rows_few in lg_hip.hip): on the vector units, a workgroup to a tile, K and V rows through LDS.
+// lg_k_attn_rows pays for 16 units, leaves CUs without a workgroup where it takes two tiles at a time, and the registers of its operands
+// let a CU overlap the preparation of one workgroup with the tiles of another only twice.  A wavefront takes the units wave, wave + 4 and wave + 8, so that one LDS read of a K (V) row serves three units and 6
+// (12) independent fma chains are in flight; bound by those fma and their LDS reads.  K is staged in reader order (the lane of key slot sl
+// and chain pair hf finds its hd/4 dwords as consecutive 16-byte units).
+// Tiles and merge, 256-wide heads, 32 tiles of 8 kv heads: 10 units 13.9 -> 12.4 us, 4 units 13.3 -> 11.3; 33 tiles 14.0 -> 13.7 and 13.3 -> 12.7;
+// whole steps (the kernels prepare the rows themselves): 12B shape, 5 rows at 3000 keys 3266 -> 3120 us, 2 rows at 1100 2837 -> 2705.
+#define LG_ATTN_FEW 12                     // units: three to a wavefront
+// fmaf(x, (float)h, acc) with h the low (high) f16 half of a packed pair: one instruction; the conversion is exact
+// and the sum rounds once, as the two-instruction form does.  The compiler picks this instruction by itself when a
+// converted value feeds one fma; written out here because each key/value element feeds one fma per unit.
+__device__ __forceinline__ float lg_fma_hlo(float x, uint32_t hp, float acc) {
+    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel_hi:[0,1,0]" : "+v"(acc) : "v"(x), "v"(hp));
+    return acc;
+}
+__device__ __forceinline__ float lg_fma_hhi(float x, uint32_t hp, float acc) {
+    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "+v"(acc) : "v"(x), "v"(hp));
+    return acc;
+}
+template <int HD>
+struct AttnFewGeo {
+    static constexpr int QST = HD + 4;
+    static constexpr int KSD = HD / 2 + 4;                    // dwords per staged K row (16-byte reads of 8 slots cover all banks)
+    static constexpr int VST = HD + 8;                        // halves per staged V row
+    static constexpr size_t bytes(int units, bool fq) {       // fq: a vector of staging per wavefront for the rotary
+        return (size_t)units * QST * 4 + (size_t)32 * KSD * 4 + (size_t)32 * VST * 2 + (size_t)units * 32 * 4 + (fq ? (size_t)(LG_WG / 64) * HD * 4 : 0);
+    }
+};
+static_assert(AttnFewGeo<256>::bytes(LG_ATTN_FEW, false) <= 48 * 1024, "lg_hip_attention_noalloc raises no limit for this kernel");
+template <int M, int HD, bool FQ = false>
+__global__ __launch_bounds__(LG_WG) void lg_k_attn_few(const StepCtl *ctl, LG_ATTN_FIELDS(LG_XP, _) int p_end_) {
+    AttnArgs a; LG_ATTN_FIELDS(LG_XI, a)
+    using Geo = AttnFewGeo<HD>;
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int NW = LG_WG / 64, UB = LG_ATTN_FEW / NW;
+    const int G = a.H / a.nkv, units = M * G;
+    float *qs = (float *)smem;                                // [unit][c][HD/4]
+    uint32_t *kt = (uint32_t *)(qs + (size_t)units * Geo::QST);         // [32][KSD]: row sl = [hf][HD/4 dwords]
+    uint16_t *vt = (uint16_t *)(kt + 32 * Geo::KSD);          // [32][VST]
+    float *es = (float *)(vt + 32 * Geo::VST);                // [unit][32]
+    float *hv = es + (size_t)units * 32;                      // FQ: [wavefront][HD] staging of the rotary
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int kvh = blockIdx.y;
+    const int pos0 = ctl->pos + a.pos_off, plast = pos0 + M - 1;
+    const int tnew = (FQ && a.kcw) ? ctl->pos : 0x7FFFFFFF;   // FQ: positions tnew..plast are rows of the block itself
+    const int start0 = lg_win_start(pos0, a.window), first = start0 >> 5;
+    const int bx = blockIdx.x, tile = first + bx, t0 = tile << 5;
+    if (t0 > plast) return;                                   // no row of the block has keys here
+    auto mine = [&](int t) { return t >> 5 == tile; };
+    const bool any = FQ && tnew <= plast && t0 + 31 >= tnew;  // the tile holds rows of the block
+    AttnRowsPrep<M, HD> prep;
+    if constexpr (FQ) prep.request(a, kvh, G, wave, tnew, any, mine);
+    constexpr int U4R = HD / 8;                               // 16-byte units per K/V row
+    constexpr int KL = (32 * U4R + LG_WG - 1) / LG_WG;        // 16-byte units of K (and of V) per thread
+    static_assert(32 * U4R % LG_WG == 0, "tile staging assumes whole passes");
+    uint4 kq[KL], vq[KL];
+    {   // (a tile lies within the ring in one piece; rows past its end are no keys of any row)
+        const int r0 = t0 % a.seq;
+        #pragma unroll
+        for (int u = 0; u < KL; ++u) {
+            const int idx = (int)threadIdx.x + u * LG_WG, row = idx / U4R, u4 = idx - row * U4R;
+            const size_t go = (size_t)(r0 + row < a.seq ? r0 + row : a.seq - 1) * a.kv_dim + (size_t)kvh * HD + u4 * 8;
+            kq[u] = lg_ldw16(a.kc + go); vq[u] = lg_ldw16(a.vc + go);         // (no second reader: non-temporal)
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (FQ) {
+        prep.queries(a, ctl, kvh, G, wave, lane, qs);
+        if (any) prep.rows(a, wave, lane, tnew, hv + (size_t)wave * HD, mine,
+            [&](int r, int t, int p, uint16_t lo, uint16_t hi) {
+                const int p1 = p + HD / 2;                    // dims 4g, 4g+1 in dword g of the first half, 4g+2, 4g+3 of the second
+                uint16_t *row = (uint16_t *)(kt + (t - t0) * Geo::KSD), *crow = a.kcw + (size_t)(t % a.seq) * a.kv_dim + (size_t)kvh * HD;
+                row[2 * (((p & 3) >> 1) * (HD / 4) + (p >> 2)) + (p & 1)] = lo;
+                row[2 * (((p1 & 3) >> 1) * (HD / 4) + (p1 >> 2)) + (p1 & 1)] = hi;
+                crow[p] = lo; crow[p1] = hi;
+            },
+            [&](int r, int t, uint2 h4) {
+                *(uint2 *)(vt + (t - t0) * Geo::VST + 4 * lane) = h4;
+                *(uint2 *)(a.vcw + (size_t)(t % a.seq) * a.kv_dim + (size_t)kvh * HD + 4 * lane) = h4;
+            });
+    } else AttnRowsPrep<M, HD>::copy_queries(a, kvh, G, qs);
+    {   // the tile into LDS.  Slots outside the keys of every row of the block are zeroed (their weights are zero, and zero times a
+        // finite value leaves the sums as they are; stale bits that read as infinities would not)
+        const int slo = start0 - t0, shi = plast - t0;
+        #pragma unroll
+        for (int u = 0; u < KL; ++u) {
+            const int idx = (int)threadIdx.x + u * LG_WG, row = idx / U4R, u4 = idx - row * U4R;
+            if (FQ && t0 + row >= tnew && row <= shi) continue;               // a row of the block: built above, not in the cache yet
+            const uint32_t mk = (row >= slo && row <= shi) ? 0xFFFFFFFFu : 0u;
+            uint32_t *d = kt + row * Geo::KSD + 2 * u4;
+            *(uint2 *)d = make_uint2(kq[u].x & mk, kq[u].z & mk);             // chains 0,1 of two groups of four dims
+            *(uint2 *)(d + HD / 4) = make_uint2(kq[u].y & mk, kq[u].w & mk);  // chains 2,3
+            *(uint4 *)(vt + row * Geo::VST + u4 * 8) = make_uint4(vq[u].x & mk, vq[u].y & mk, vq[u].z & mk, vq[u].w & mk);
+        }
+    }
+    __syncthreads();
+    // this wavefront's units, the slots that they see (a missing unit repeats the first one and stores nothing), and their partials
+    const bool some = wave < units;
+    int un[UB], lo[UB], hi[UB];
+    bool on[UB];
+    size_t pi[UB];
+    #pragma unroll
+    for (int b = 0; b < UB; ++b) {
+        const bool there = wave + b * NW < units;
+        un[b] = there ? wave + b * NW : some ? wave : 0;
+        const int j = un[b] / G, pj = pos0 + j;
+        lo[b] = lg_win_start(pj, a.window) - t0; hi[b] = pj - t0;
+        on[b] = there && lo[b] < 32 && hi[b] >= 0;            // the row has keys in this tile
+        pi[b] = ((size_t)j * a.H + kvh * G + (un[b] - j * G)) * a.tiles_max + bx;
+    }
+    if (some) {   // scores
+        const int sl = lane & 31, hf = lane >> 5;
+        const uint32_t *ks = kt + sl * Geo::KSD + hf * (HD / 4);
+        const float *qr[UB];
+        float ax[UB], ay[UB];
+        #pragma unroll
+        for (int b = 0; b < UB; ++b) { qr[b] = qs + (size_t)un[b] * Geo::QST + hf * (HD / 2); ax[b] = 0.0f; ay[b] = 0.0f; }
+        #pragma unroll 2
+        for (int u = 0; u < HD / 16; ++u) {
+            const uint4 k4 = *(const uint4 *)(ks + 4 * u);
+            #pragma unroll
+            for (int b = 0; b < UB; ++b) {                    // chains 2 hf and 2 hf + 1
+                const float4 p0 = *(const float4 *)(qr[b] + 4 * u), p1 = *(const float4 *)(qr[b] + HD / 4 + 4 * u);
+                ax[b] = lg_fma_hlo(p0.x, k4.x, ax[b]); ay[b] = lg_fma_hhi(p1.x, k4.x, ay[b]);
+                ax[b] = lg_fma_hlo(p0.y, k4.y, ax[b]); ay[b] = lg_fma_hhi(p1.y, k4.y, ay[b]);
+                ax[b] = lg_fma_hlo(p0.z, k4.z, ax[b]); ay[b] = lg_fma_hhi(p1.z, k4.z, ay[b]);
+                ax[b] = lg_fma_hlo(p0.w, k4.w, ax[b]); ay[b] = lg_fma_hhi(p1.w, k4.w, ay[b]);
+            }
+        }
+        #pragma unroll
+        for (int b = 0; b < UB; ++b) {
+            if (!on[b]) continue;
+            const bool valid = sl >= lo[b] && sl <= hi[b];
+            float s = lg_add_x32(ax[b] + ay[b]);              // (a0+a1) + (a2+a3): the two halves sit 32 lanes apart
+            if (!valid) s = -INFINITY;
+            const float mx = lg_max_n(s, 32);
+            const float e = valid ? lg_expf(s - mx) : 0.0f;
+            const float l = lg_sum32(e);
+            if (hf == 0) es[un[b] * 32 + sl] = e;
+            if (lane == 0) { a.pm[pi[b]] = mx; a.pl[pi[b]] = l; }
+        }
+    }
+    __syncthreads();
+    if (!some) return;
+    // values (lane = 4 dims).  A slot that a row does not see has weight 0 for it; where another row of the block has a value there that
+    // is not finite, their product is a NaN.  So where the rows' keys may differ within the tile and a result is not finite, they are
+    // computed again with zeros in those slots (always with zeros there: 0.4 us more for the first and the last tile, which the merge waits for).
+    const uint16_t *vl = vt + (4 * lane < HD ? 4 * lane : 0);
+    float4 acc[UB];
+    auto values = [&](auto masked) {
+        #pragma unroll
+        for (int b = 0; b < UB; ++b) acc[b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        #pragma unroll 2
+        for (int u4 = 0; u4 < 8; ++u4) {
+            float ev[UB][4];
+            #pragma unroll
+            for (int b = 0; b < UB; ++b) {                    // (a unit that has no keys here has stale weights: never stored)
+                const float4 e4 = *(const float4 *)(es + un[b] * 32 + 4 * u4);
+                ev[b][0] = e4.x; ev[b][1] = e4.y; ev[b][2] = e4.z; ev[b][3] = e4.w;
+            }
+            #pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint2 v4 = *(const uint2 *)(vl + (4 * u4 + q) * Geo::VST);
+                #pragma unroll
+                for (int b = 0; b < UB; ++b) {
+                    uint2 v = v4;
+                    if constexpr (decltype(masked)::value) if (4 * u4 + q < lo[b] || 4 * u4 + q > hi[b]) v = make_uint2(0u, 0u);
+                    acc[b].x = lg_fma_hlo(ev[b][q], v.x, acc[b].x); acc[b].y = lg_fma_hhi(ev[b][q], v.x, acc[b].y);
+                    acc[b].z = lg_fma_hlo(ev[b][q], v.y, acc[b].z); acc[b].w = lg_fma_hhi(ev[b][q], v.y, acc[b].w);
+                }
+            }
+        }
+    };
+    values(std::false_type{});
+    if (__builtin_expect(t0 < start0 + M - 1 || t0 + 31 > plast - (M - 1), 0)) {
+        float odd = 0.0f;
+        #pragma unroll
+        for (int b = 0; b < UB; ++b) odd = lg_fmaf(acc[b].x, 0.0f, lg_fmaf(acc[b].y, 0.0f, lg_fmaf(acc[b].z, 0.0f, lg_fmaf(acc[b].w, 0.0f, odd))));
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd != 0.0f) != 0, 0)) values(std::true_type{});
+    }
+    #pragma unroll
+    for (int b = 0; b < UB; ++b)
+        if (on[b] && 4 * lane < HD) *(float4 *)(a.pacc + pi[b] * HD + 4 * lane) = acc[b];
 }
 
 // lg_k_attn_merge for rows with very many tiles: one workgroup of NW wavefronts per (head, row, 64 dims).  The

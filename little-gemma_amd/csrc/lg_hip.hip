@@ -1104,6 +1104,13 @@ static void launch_mmf(Launcher &lx, int cls, const MmfArgs &a) {
 static bool attention_rows_shared(int rows, int tiles, int nkv, int hd, int seq, int reach) {
     return rows > 1 && hd <= 256 && seq >= 32 && (seq % 32 == 0 || reach <= seq) && tiles * nkv >= 256;
 }
+// ... by lg_k_attn_few: up to 9 tiles a CU where the kernel prepares the block's rows itself (whole steps, lg_k_attn_rows against it: 12B shape,
+// 4 rows, 1840 (tile, kv head) pairs 3204 -> 3136 us; E4B shape, 3 rows, 2052 pairs 2192 -> 2161; 12B, 4112 pairs, 6 rows at 14000 keys
+// 3523 -> 3551, 5 at 8192 3350 -> 3295), up to three where the rows arrive prepared (768 pairs, 5 rows of 16 over 8: 256-wide heads 24.4 -> 24.6 us,
+// 64-wide 16.7 -> 17.1, 2 rows 22.4 -> 20.7 and 16.2 -> 15.9; 1600 pairs, 5 rows 34.0 -> 36.9)
+static bool attention_rows_few(int tiles, int units, int nkv, bool prepares) {
+    return units <= LG_ATTN_FEW && tiles * nkv <= (prepares ? 9 : 3) * cu_count();
+}
 // workgroups of lg_k_attn_rows per kv head: three to a CU at most (its registers hold no more), each walking its share of the tiles
 static int attention_rows_wgs(int tiles, int units, int nkv) {
     const int steps = (tiles + lg_attn_rows_tiles(units) - 1) / lg_attn_rows_tiles(units), cap = 3 * cu_count() / nkv;
@@ -1424,20 +1431,25 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             const bool shared = rows_shared(L);
             if (shared) {
                 if constexpr (M > 1) {
-                    const size_t lds = y.hd == 256 ? AttnRowsGeo<256>::bytes(M * G, fused_post) : y.hd == 128 ? AttnRowsGeo<128>::bytes(M * G, fused_post) : AttnRowsGeo<64>::bytes(M * G, fused_post);
-                    const dim3 grid(attention_rows_wgs(tiles, M * G, y.nkv), y.nkv);
+                    const bool few = attention_rows_few(tiles, M * G, y.nkv, fused_post);
+                    const size_t lds = few ? y.hd == 256 ? AttnFewGeo<256>::bytes(M * G, fused_post) : y.hd == 128 ? AttnFewGeo<128>::bytes(M * G, fused_post) : AttnFewGeo<64>::bytes(M * G, fused_post)
+                                           : y.hd == 256 ? AttnRowsGeo<256>::bytes(M * G, fused_post) : y.hd == 128 ? AttnRowsGeo<128>::bytes(M * G, fused_post) : AttnRowsGeo<64>::bytes(M * G, fused_post);
+                    const dim3 grid(few ? tiles : attention_rows_wgs(tiles, M * G, y.nkv), y.nkv);
                     a.gx = (int)grid.x;
+#define ATTN_ROWS(...) do { if (few) LAUNCH(KC_ATTN, (lg_k_attn_few<M, __VA_ARGS__>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0); \
+                            else     LAUNCH(KC_ATTN, (lg_k_attn_rows<M, __VA_ARGS__>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0); } while (0)
                     if (fused_post) {
                         a.qkv = m->qkv; a.ld = y.qkv_m; a.k_off = y.k_off; a.v_off = y.v_off;
                         a.q_norm = y.q_norm; a.k_norm = y.k_norm; a.rope_tab = y.rope_tab; a.rope_ff = y.rope_ff;
                         a.kcw = y.owns ? kv->k[L] : nullptr; a.vcw = y.owns ? kv->v[L] : nullptr; a.eps = m->eps;
-                        if (y.hd == 256)      LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 256, true>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
-                        else if (y.hd == 128) LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 128, true>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
-                        else                  LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 64, true>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
+                        if (y.hd == 256)      ATTN_ROWS(256, true);
+                        else if (y.hd == 128) ATTN_ROWS(128, true);
+                        else                  ATTN_ROWS(64, true);
                     } else
-                    if (y.hd == 256)      LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 256>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
-                    else if (y.hd == 128) LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 128>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
-                    else                  LAUNCH(KC_ATTN, (lg_k_attn_rows<M, 64>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
+                    if (y.hd == 256)      ATTN_ROWS(256);
+                    else if (y.hd == 128) ATTN_ROWS(128);
+                    else                  ATTN_ROWS(64);
+#undef ATTN_ROWS
                 }
             } else
             if (fused_post) {
@@ -2532,14 +2544,18 @@ static int enqueue_attention(hipStream_t st, const AttnArgs &a_in, const MergeAr
     if (attention_rows_shared(M, tiles, a.nkv, a.hd, a.seq, pos + M)) {
         if constexpr (M > 1) {
             const int units = M * (a.H / a.nkv);
-            const size_t l2 = a.hd == 256 ? AttnRowsGeo<256>::bytes(units, false) : a.hd == 128 ? AttnRowsGeo<128>::bytes(units, false) : AttnRowsGeo<64>::bytes(units, false);
-            int rc = a.hd == 256 ? set_lds(lg_k_attn_rows<M, 256>, l2) : a.hd == 128 ? set_lds(lg_k_attn_rows<M, 128>, l2) : set_lds(lg_k_attn_rows<M, 64>, l2);
-            if (rc) return rc;
-            const dim3 grid(attention_rows_wgs(tiles, units, a.nkv), a.nkv);
+            const bool few = attention_rows_few(tiles, units, a.nkv, false);
+            const dim3 grid(few ? tiles : attention_rows_wgs(tiles, units, a.nkv), a.nkv);
             a.gx = (int)grid.x;
-            if (a.hd == 256)      hipLaunchKernelGGL((lg_k_attn_rows<M, 256>), grid, dim3(LG_WG), l2, st, ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
-            else if (a.hd == 128) hipLaunchKernelGGL((lg_k_attn_rows<M, 128>), grid, dim3(LG_WG), l2, st, ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
-            else                  hipLaunchKernelGGL((lg_k_attn_rows<M, 64>), grid, dim3(LG_WG), l2, st, ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
+            int rc = 0;
+#define ATTN_ROWS(HD) do { const size_t l2 = few ? AttnFewGeo<HD>::bytes(units, false) : AttnRowsGeo<HD>::bytes(units, false); \
+    if (few) { if (!(rc = set_lds(lg_k_attn_few<M, HD>, l2))) hipLaunchKernelGGL((lg_k_attn_few<M, HD>), grid, dim3(LG_WG), l2, st, ctl, LG_ATTN_FIELDS(LG_XA, a) 0); } \
+    else if (!(rc = set_lds(lg_k_attn_rows<M, HD>, l2))) hipLaunchKernelGGL((lg_k_attn_rows<M, HD>), grid, dim3(LG_WG), l2, st, ctl, LG_ATTN_FIELDS(LG_XA, a) 0); } while (0)
+            if (a.hd == 256)      ATTN_ROWS(256);
+            else if (a.hd == 128) ATTN_ROWS(128);
+            else                  ATTN_ROWS(64);
+#undef ATTN_ROWS
+            if (rc) return rc;
         }
     } else hipLaunchKernelGGL((lg_k_attn<false, 1>), dim3(tiles, a.nkv, M), dim3(LG_WG), lds, st, ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
     if (tiles >= 128 && a.hd % 64 == 0) {

@@ -187,15 +187,17 @@ def test_every_kernel_choice_gives_the_same_bits(lg, gpu_required, model_path, m
             assert np.array_equal(a, b), opt
 
 
-@pytest.mark.parametrize("rows", [5, 8, 2])
-def test_shared_tile_attention_prepares_its_own_rows(lg, ob, gpu_required, model_path, rows):
-    """Layers with 256 and more (tile, kv head) pairs take the attention kernel that stages a tile once for all rows
-    of a block; it norms and rotates the block's queries and builds the block's K/V rows itself.  A 2048-key window
+@pytest.mark.parametrize("rows,over", [(5, {}), (8, {}), (2, {}), (5, {"head_dim": 256, "head_dim_full": 256}), (8, {"head_dim_full": 256}), (8, {"n_head": 4}),
+                                       (7, {"head_dim": 128}), (5, {"n_head": 16}), (3, {"n_head": 20, "head_dim": 128})])
+def test_shared_tile_attention_prepares_its_own_rows(lg, ob, gpu_required, model_path, rows, over):
+    """Layers with 256 and more (tile, kv head) pairs take the attention kernels whose workgroups serve all rows of a block (up to 12
+    units of (row, query head) on so few tiles on the vector units, more on the matrix cores); they norm and rotate the block's queries and
+    build the block's K/V rows themselves.  A 2048-key window
     on 4 KV heads (66 tiles) and a global context of the same length, layers that own their cache and layers that
     read another's, a block that starts 2 positions before a tile boundary (its rows fall into two tiles) and the
     next one after it: against the oracle, and bit for bit against the same step with lg_k_qkv_post run ahead
     (attn_rows_fq = 0) and with the per-row attention kernel (attn_rows = 0)."""
-    path, spec = model_path("tiny_full", n_head_kv=4, sliding_window=2048)
+    path, spec = model_path("tiny_full", **dict({"n_head_kv": 4, "sliding_window": 2048}, **over))
     V, E = spec["n_vocab"], spec["n_embd"]
     rng = np.random.default_rng(90 + rows)
     n0 = 65 * 32 + 30
@@ -250,13 +252,14 @@ def test_shared_tile_attention_prepares_its_own_rows(lg, ob, gpu_required, model
             assert np.array_equal(a, b), opts
 
 
-@pytest.mark.parametrize("n0,j,fq", [(2100, 0, 1), (2100, 3, 1), (2100, 7, 1), (2100, 3, 0), (20, 3, 1), (20, 4, 0)])
-def test_a_block_row_of_nan_reaches_no_row_before_it(lg, gpu_required, model_path, model_dir, n0, j, fq):
+@pytest.mark.parametrize("n0,j,fq,n_head", [(2100, 0, 1, 8), (2100, 3, 1, 8), (2100, 7, 1, 8), (2100, 3, 0, 8), (20, 3, 1, 8), (20, 4, 0, 8),
+                                            (2100, 0, 1, 4), (2100, 7, 1, 4), (2100, 3, 0, 4), (20, 3, 1, 4)])
+def test_a_block_row_of_nan_reaches_no_row_before_it(lg, gpu_required, model_path, model_dir, n0, j, fq, n_head):
     """Verify blocks whose rows share an attention tile (256 and more (tile, kv head) pairs), with a token whose embedding is
     infinite at row j of the block that a tile boundary cuts, behind a whole window and in the first keys of one: the cache rows in
     front of it, in every layer, are those of the same block with another token there, and all of them those of the attention kernel
     per row."""
-    src, spec = model_path("tiny_full", n_head_kv=4, sliding_window=2048)
+    src, spec = model_path("tiny_full", n_head=n_head, n_head_kv=4, sliding_window=2048)
     path = os.path.join(str(model_dir), "tiny_full_infinite_token.gguf")
     shutil.copyfile(src, path)
     off, nbytes, dims = gguf_tensor_span(path, "token_embd.weight")
@@ -288,6 +291,43 @@ def test_a_block_row_of_nan_reaches_no_row_before_it(lg, gpu_required, model_pat
         assert all(((a[8 + j] & 0x7FFF) > 0x7C00).any() for a in got[1][2:])
     finally:
         gpu.close()
+
+
+@pytest.mark.parametrize("n_head,hd,rows,pairs", [(16, 64, 8, 101), (16, 256, 8, 101), (16, 128, 5, 150), (8, 64, 8, 101), (16, 256, 5, 142)])
+def test_block_rows_in_a_later_tile_of_their_workgroup(lg, gpu_required, model_path, n_head, hd, rows, pairs):
+    """Long global layers of 8 kv heads whose pairs of tiles outnumber the workgroups that the CUs hold (96 per kv head): a block over the
+    border between two pairs, prepared inside the attention kernel by the workgroups that walk to them as their second pair (16 units; 10 where
+    the tiles are too many for lg_k_attn_few; the last two cases go there), against lg_k_qkv_post ahead of it (attn_rows_fq = 0) and the kernel
+    per row (attn_rows = 0).  The keys in front are drawn."""
+    path, spec = model_path("tiny", n_head=n_head, n_head_kv=8, head_dim_full=hd)
+    n0 = 64 * pairs - 2
+    blk = np.random.default_rng(rows).integers(0, spec["n_vocab"], rows).astype(np.int32)
+
+    def run(**opts):
+        gpu = lg.hiplib.HipBackend(path, n0 + 40, max_rows=8)
+        try:
+            rng = np.random.default_rng(5)
+            for L in range(spec["n_layer"]):
+                shape = gpu.kv_read(L, 0).shape
+                for w in (0, 1):
+                    gpu.kv_write(L, w, rng.normal(0, 1, shape).astype(np.float16).view(np.uint16))
+            for k, v in opts.items():
+                gpu.set_option(k, v)
+            gpu.set_option("store_logits", 1)
+            adv, out = gpu.forward_spec(blk, n0)
+            return adv, out.copy(), np.stack([gpu.logits_row(j, spec["n_vocab"]) for j in range(rows)]), [gpu.kv_read(L, w).copy() for L in range(spec["n_layer"]) for w in (0, 1)]
+        finally:
+            gpu.close()
+
+    got = []
+    for opts in ({"attn_rows": 0}, {"attn_rows_fq": 0}, {}):
+        print(f"n_head={n_head} hd={hd} rows={rows} pairs={pairs}: {opts}", flush=True)
+        got.append(run(**opts))
+    assert np.isfinite(got[0][2]).all()
+    for g in got[1:]:
+        assert g[0] == got[0][0] and np.array_equal(g[1], got[0][1])
+        assert np.array_equal(g[2].view(np.uint32), got[0][2].view(np.uint32))
+        assert all(np.array_equal(a, b) for a, b in zip(g[3], got[0][3]))
 
 
 SESSION = """

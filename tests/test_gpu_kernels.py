@@ -290,9 +290,19 @@ def test_attention_over_many_tiles(lg, ob, gpu_required, H, KV, hd, rows, tiles,
     (8, 1, 64, 2, 8200, 8224, 20001),      # 16 units: one group, two tiles at a time, an odd number of tiles
     (16, 8, 256, 5, 1024, 1536, 1533),     # the 12B shape's window, at a ring's end
     (4, 4, 256, 8, 2048, 2101, 6300),      # a ring of other than a multiple of 32 rows: the kernel per row
-    (8, 8, 64, 3, 1024, 1088, 40)])        # few keys in a wide window
+    (8, 8, 64, 3, 1024, 1088, 40),         # few keys in a wide window
+    (12, 4, 256, 4, 2048, 2560, 6300),     # 12 units, the most of lg_k_attn_few, 66 tiles of 4 kv heads
+    (12, 4, 256, 5, 2048, 2560, 6300),     # 15 units there
+    (16, 8, 256, 5, 3068, 3136, 9627),     # 96 tiles of 8 kv heads, the most of lg_k_attn_few
+    (16, 8, 256, 5, 3072, 3136, 9627),     # 97
+    (16, 8, 256, 2, 0, 1100, 1098),        # 35 tiles, the cache and the keys end inside the last one
+    (16, 8, 128, 3, 1024, 1536, 1533), (4, 4, 128, 8, 2048, 2560, 2049), (8, 8, 64, 8, 1024, 1100, 1092), (32, 16, 64, 2, 512, 576, 575),
+    (8, 1, 256, 2, 8160, 8224, 20001),     # 256 tiles of one kv head, 16 units
+    (64, 8, 64, 8, 0, 4160, 4150),         # 64 units, more tiles than workgroups at a time
+    (16, 8, 64, 8, 6300, 6368, 9000)])     # 16 units, more pairs of tiles than workgroups at a time
 def test_attention_of_all_rows_of_a_block(lg, ob, gpu_required, H, KV, hd, rows, window, seq, pos):
-    """256 and more (tile, kv head) pairs: a workgroup serves all rows, units in groups of 16 on the matrix cores; same bits as the oracle."""
+    """256 and more (tile, kv head) pairs: a workgroup serves all rows, units in groups of 16 on the matrix cores or few of them on the
+    vector units; same bits as the oracle."""
     rng = np.random.default_rng(H * 100 + rows)
     kc = rng.normal(0, 1, (seq, KV * hd)).astype(np.float16).view(np.uint16)
     vc = rng.normal(0, 1, (seq, KV * hd)).astype(np.float16).view(np.uint16)
@@ -314,7 +324,9 @@ def nan_bits(a):
     (16, 8, 256, 5, 1024, 1536, 1533),     # the rows' last tiles on both sides of the ring's end
     (16, 2, 128, 8, 0, 4192, 4150),        # a whole context, stale rows behind it
     (8, 1, 64, 2, 8200, 8224, 20001),      # an odd number of tiles
-    (16, 4, 256, 8, 2048, 2560, 2050)])    # two groups of units
+    (16, 4, 256, 8, 2048, 2560, 2050),     # two groups of units
+    (16, 8, 256, 8, 2048, 2112, 5005),     # one group of 256-wide heads, two tiles at a time
+    (12, 4, 128, 4, 2048, 2560, 6300), (8, 8, 64, 8, 1024, 1152, 3007), (8, 4, 256, 2, 2050, 2560, 2559)])       # few units: on the vector units
 def test_attention_values_that_are_not_finite(lg, ob, gpu_required, H, KV, hd, rows, window, seq, pos):
     """256 and more (tile, kv head) pairs, where the rows of a block share a tile.  Infinities and NaN in the K and V rows that no row
     of the block sees change no bit; in the value row that only the first row still sees and in the one that only the last row sees
