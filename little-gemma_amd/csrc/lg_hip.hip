@@ -2343,21 +2343,22 @@ static int read_back_wide(const uint8_t *dq, int rows, int k, int8_t *xq, float 
         }
     return 0;
 }
+// (as the q/k/v and the attention output projection of a prompt are launched; *parts: slabs of the result)
 static int matmul_wide(hipStream_t st, const uint8_t *dw, uint8_t *dwide, int k, int mrows, int rows, const float *dx, float *dout, int32_t *ddots,
-                       int8_t *dq, int repeats, float *kernel_ms) {
+                       int8_t *dq, int repeats, float *kernel_ms, int *parts) {
     const size_t np = (size_t)((mrows + LG_WT - 1) / LG_WT * LG_WT) * (k / 32);
     hipLaunchKernelGGL(lg_k_wide_pack, dim3((unsigned)((np + LG_WG - 1) / LG_WG)), dim3(LG_WG), 0, st, dw, k, mrows, 0, dwide);
     hipLaunchKernelGGL(lg_k_wide_quant, dim3((rows * (k / 32) * 8 + LG_WG - 1) / LG_WG), dim3(LG_WG), 0, st, dx, rows, k, (uint8_t *)dq);
     lg_hip_model shim;
     shim.stream = st;
     Launcher lx{ &shim, false };
-    if (ddots) launch_wide_mm<true>(lx, 0, dwide, dq, k, mrows, rows, dout, ddots);
+    if (ddots) launch_wide_mm<true>(lx, 0, dwide, dq, k, mrows, rows, dout, ddots, true);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     auto body = [&]() -> int {
         HIP_TRY(hipEventCreate(&e0)); HIP_TRY(hipEventCreate(&e1));
-        launch_wide_mm<false>(lx, 0, dwide, dq, k, mrows, rows, dout, nullptr);
+        *parts = launch_wide_mm<false>(lx, 0, dwide, dq, k, mrows, rows, dout, nullptr, true);
         HIP_TRY(hipEventRecord(e0, st));
-        for (int r = 0; r < repeats; ++r) launch_wide_mm<false>(lx, 0, dwide, dq, k, mrows, rows, dout, nullptr);
+        for (int r = 0; r < repeats; ++r) launch_wide_mm<false>(lx, 0, dwide, dq, k, mrows, rows, dout, nullptr, true);
         if (lx.rc) return lx.rc;
         HIP_TRY(hipEventRecord(e1, st));
         HIP_TRY(hipStreamSynchronize(st));
@@ -2411,10 +2412,11 @@ extern "C" int lg_hip_matmul_q4q8(const void *w, int k, int mrows, const float *
     HIP_TRY(hipMemcpy(dx, x, (size_t)rows * k * 4, hipMemcpyHostToDevice));
     hipStream_t st;
     HIP_TRY(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+    int parts = 1;
     if (wide) {
         uint8_t *dwide;
         if (sc.get(&dwide, lg_wide_bytes(k, mrows))) rc = -7;
-        else rc = matmul_wide(st, dw, dwide, k, mrows, rows, dx, dout, ddots, dq, repeats, kernel_ms);
+        else rc = matmul_wide(st, dw, dwide, k, mrows, rows, dx, dout, ddots, dq, repeats, kernel_ms, &parts);
     } else switch (rows) {
 #define CASE(M) case M: rc = matmul_rows<M>(st, dw, k, mrows, dx, dout, ddots, dq, repeats, kernel_ms); break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
@@ -2422,11 +2424,11 @@ extern "C" int lg_hip_matmul_q4q8(const void *w, int k, int mrows, const float *
     }
     (void)hipStreamDestroy(st);
     if (rc) return rc;
-    if (out && wide && lg_segments(k) == 32) {             // four slabs of partial sums: the top of the segment tree is added here
-        std::vector<float> parts((size_t)4 * rows * mrows);
-        HIP_TRY(hipMemcpy(parts.data(), dout, parts.size() * 4, hipMemcpyDeviceToHost));
+    if (out && parts == 4) {                               // four slabs of partial sums: the top of the segment tree is added here
+        std::vector<float> slabs((size_t)4 * rows * mrows);
+        HIP_TRY(hipMemcpy(slabs.data(), dout, slabs.size() * 4, hipMemcpyDeviceToHost));
         const size_t n = (size_t)rows * mrows;
-        for (size_t i = 0; i < n; ++i) out[i] = (parts[i] + parts[n + i]) + (parts[2 * n + i] + parts[3 * n + i]);
+        for (size_t i = 0; i < n; ++i) out[i] = (slabs[i] + slabs[n + i]) + (slabs[2 * n + i] + slabs[3 * n + i]);
     } else if (out) HIP_TRY(hipMemcpy(out, dout, (size_t)rows * mrows * 4, hipMemcpyDeviceToHost));
     if (dots) HIP_TRY(hipMemcpy(dots, ddots, (size_t)rows * mrows * nb * 4, hipMemcpyDeviceToHost));
     // the device keeps activation rows in the matmul's own order; hand them back in natural order

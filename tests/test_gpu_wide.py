@@ -15,9 +15,11 @@ from test_gpu_prefill import check_wide_prefill
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m,k,rows", [(20480, 256, 32), (20480, 512, 64), (8200, 3840, 96), (264, 2560, 512), (2560, 5120, 160), (4160, 256, 480)])
+@pytest.mark.parametrize("m,k,rows", [(20480, 256, 32), (20480, 512, 64), (8200, 3840, 96), (264, 2560, 512), (2560, 5120, 160), (4160, 256, 480),
+                                      (3072, 2560, 32), (1000, 4096, 96), (72, 4352, 128), (8, 256, 32), (2048, 2560, 64), (2056, 2560, 64), (264, 256, 160)])
 def test_wide_matmul_shapes(lg, ob, gpu_required, m, k, rows):
-    """64 x 32 tiles by four and by eight wavefronts, 64 x 64 tiles, a last weight tile of 8 rows, 32 K segments."""
+    """64 x 32 tiles by two wavefronts (8 K segments in four parts, up to 64 tiles and 128 rows), by four and by eight, 64 x 64 tiles, a last
+    weight tile of 8 rows, 32 K segments; rows of 8 segments of an odd number of blocks, of one."""
     rng = np.random.default_rng(m + k + rows)
     w = random_q4_0(rng, m, k)
     x = rng.normal(0, 1, (rows, k)).astype(np.float32)
