@@ -165,7 +165,8 @@ __global__ __launch_bounds__(LG_WG) void lg_k_rows_mm(LG_ROWSMM_FIELDS(LG_XP, _)
 // With one row a wavefront that takes its tiles two at a time waits for memory again and again; with four or more the dot phase of lg_k_mm is bound by the instruction issue of its one wavefront per row
 // group (about 125 instructions per tile at five rows, ten tiles at k = 2560) while half of the chip's SIMDs have
 // nothing to do.  Here wavefront (group, part) takes the tiles [part*nit/KP, (part+1)*nit/KP) of its group: it
-// requests all of them at once, forms the exact block dots and the scale products of its tiles, and the float
+// requests all of them at once (and tiles of the next part or the group's last one up to TMAX, which it does not use: none there under a guard
+// 1827 -> 1886 us a decode step of the E4B shape, its own last one again 2208 -> 2220 at five rows), forms the exact block dots and the scale products of its tiles, and the float
 // chain p = fma(xd*dw, (float)dot, p) then runs through the parts in order (part p starts from the value part
 // p-1 left in LDS), so every sum is formed in the order of lg_mm_groups and the result is the same bits.
 template <int M, int KP>

@@ -1340,7 +1340,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 case 1: LAUNCH(cls, (lg_k_rows_mm<M, 1, NW>), grid, dim3(LG_WG), lds, LG_ROWSMM_FIELDS(LG_XA, f) 0); break;
                 case 2: LAUNCH(cls, (lg_k_rows_mm<M, 2, NW>), grid, dim3(LG_WG), lds, LG_ROWSMM_FIELDS(LG_XA, f) 0); break;
                 case 3: LAUNCH(cls, (lg_k_rows_mm<M, 3, NW>), grid, dim3(LG_WG), lds, LG_ROWSMM_FIELDS(LG_XA, f) 0); break;
-                default: LAUNCH(cls, (lg_k_rows_mm<M, 4, NW>), grid, dim3(LG_WG), lds, LG_ROWSMM_FIELDS(LG_XA, f) 0); break;
+                default: if constexpr (M == 1) LAUNCH(cls, (lg_k_rows_mm<M, 4, NW>), grid, dim3(LG_WG), lds, LG_ROWSMM_FIELDS(LG_XA, f) 0);      // (two such rows: can_fuse)
             }
             row_work_done();
         }
@@ -1621,6 +1621,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
 // without a workgroup, eight wavefronts of one segment on such a tile (3072 x 2560, 32 rows, 48 workgroups: 8.8 -> 7.1 us).
 // `slabs`: the consumer adds four slabs, so that a matrix of 8 segments may be cut by K quarter too: workgroups of two wavefronts,
 // where a quarter of the CUs would do for whole rows (a CU pulls 48 GB/s: 22 rows, 3072 x 2560 on 48 CUs 9.1 us, on 192 6.2).
+// 256: the compute units of a whole device, as a constant because the per-layer gate is built for the shape that it gives.
 struct WideShape { int tb, wv, parts; };
 static WideShape wide_shape(int k, int m, int rows, bool slabs) {
     const int parts = lg_segments(k) / 8, tiles = ((m + LG_WT - 1) / LG_WT) * ((rows + 31) / 32);

@@ -1208,7 +1208,9 @@ struct AttnArgs {
     const float *q_norm, *k_norm, *rope_tab, *rope_ff;
     uint16_t *kcw, *vcw;     // this layer's own cache, to receive the block's rows (nullptr: it reads another layer's)
     float eps;
-    int gx, gz;              // lg_k_attn: its launch dimensions x and z (as arguments they arrive with the others)
+    // lg_k_attn: its launch dimensions x and z (as arguments they arrive with the others).  lg_k_attn_rows: gx workgroups of a kv head
+    // share its tiles, so it has to be the launch's x there too
+    int gx, gz;
     __device__ __forceinline__ uint4 kc4(size_t off) const { return *(const uint4 *)(kc + off); }
     __device__ __forceinline__ uint4 vc4(size_t off) const { return *(const uint4 *)(vc + off); }
 };

@@ -481,7 +481,7 @@ __global__ __launch_bounds__(LG_WG) void lg_k_wide_quant(const float *x, int row
 #define LG_WA_WG 512
 #define LG_WA_SPLIT_WG 256
 #define LG_WA_SPLIT_MAX 1024             // tiles whose weights PHASE 2 keeps in LDS
-#define LG_WA_SPLIT_GROUPS 128           // groups of units (x kv heads) up to which the two kernels are launched
+#define LG_WA_SPLIT_GROUPS 128           // groups of units (x kv heads) up to which the two kernels are launched for any number of tiles (more: launch_wide_attn)
 struct WideAttn {
     const float *q;              // [rows][H*hd] normed + rotated
     const uint16_t *kc, *vc;     // cache of the layer this one reads
