@@ -977,12 +977,12 @@ __global__ __launch_bounds__(LG_WG, 2) void lg_k_attn_rows(const StepCtl *ctl, L
 
 // The same for few units (attention_rows_few in lg_hip.hip): on the vector units, a workgroup to a tile, K and V rows through LDS.
 // lg_k_attn_rows pays for 16 units, leaves CUs without a workgroup where it takes two tiles at a time, and the registers of its operands
-// let a CU overlap the preparation of one workgroup with the tiles of another only twice.  A wavefront takes the units wave, wave + 4 and wave + 8, so that one LDS read of a K (V) row serves three units and 6
-// (12) independent fma chains are in flight; bound by those fma and their LDS reads.  K is staged in reader order (the lane of key slot sl
+// let a CU overlap the preparation of one workgroup with the tiles of another only twice.  A wavefront takes the units wave, wave + 4 and wave + 8 (UB = 4: and wave + 12), so that one LDS read of a K (V) row serves three units
+// and 6 (12) independent fma chains are in flight; bound by those fma and their LDS reads.  K is staged in reader order (the lane of key slot sl
 // and chain pair hf finds its hd/4 dwords as consecutive 16-byte units).
 // Tiles and merge, 256-wide heads, 32 tiles of 8 kv heads: 10 units 13.9 -> 12.4 us, 4 units 13.3 -> 11.3; 33 tiles 14.0 -> 13.7 and 13.3 -> 12.7;
 // whole steps (the kernels prepare the rows themselves): 12B shape, 5 rows at 3000 keys 3266 -> 3120 us, 2 rows at 1100 2837 -> 2705.
-#define LG_ATTN_FEW 12                     // units: three to a wavefront
+#define LG_ATTN_FEW 12                     // units: three to a wavefront (UB = 4: 16)
 // fmaf(x, (float)h, acc) with h the low (high) f16 half of a packed pair: one instruction; the conversion is exact
 // and the sum rounds once, as the two-instruction form does.  The compiler picks this instruction by itself when a
 // converted value feeds one fma; written out here because each key/value element feeds one fma per unit.
@@ -1004,12 +1004,12 @@ struct AttnFewGeo {
     }
 };
 static_assert(AttnFewGeo<256>::bytes(LG_ATTN_FEW, false) <= 48 * 1024, "lg_hip_attention_noalloc raises no limit for this kernel");
-template <int M, int HD, bool FQ = false>
+template <int M, int HD, bool FQ = false, int UB = LG_ATTN_FEW / 4>
 __global__ __launch_bounds__(LG_WG) void lg_k_attn_few(const StepCtl *ctl, LG_ATTN_FIELDS(LG_XP, _) int p_end_) {
     AttnArgs a; LG_ATTN_FIELDS(LG_XI, a)
     using Geo = AttnFewGeo<HD>;
     extern __shared__ __align__(16) unsigned char smem[];
-    constexpr int NW = LG_WG / 64, UB = LG_ATTN_FEW / NW;
+    constexpr int NW = LG_WG / 64;
     const int G = a.H / a.nkv, units = M * G;
     float *qs = (float *)smem;                                // [unit][c][HD/4]
     uint32_t *kt = (uint32_t *)(qs + (size_t)units * Geo::QST);         // [32][KSD]: row sl = [hf][HD/4 dwords]

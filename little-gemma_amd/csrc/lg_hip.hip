@@ -1107,9 +1107,11 @@ static bool attention_rows_shared(int rows, int tiles, int nkv, int hd, int seq,
 // ... by lg_k_attn_few: up to 9 tiles a CU where the kernel prepares the block's rows itself (whole steps, lg_k_attn_rows against it: 12B shape,
 // 4 rows, 1840 (tile, kv head) pairs 3204 -> 3136 us; E4B shape, 3 rows, 2052 pairs 2192 -> 2161; 12B, 4112 pairs, 6 rows at 14000 keys
 // 3523 -> 3551, 5 at 8192 3350 -> 3295), up to three where the rows arrive prepared (768 pairs, 5 rows of 16 over 8: 256-wide heads 24.4 -> 24.6 us,
-// 64-wide 16.7 -> 17.1, 2 rows 22.4 -> 20.7 and 16.2 -> 15.9; 1600 pairs, 5 rows 34.0 -> 36.9)
+// 64-wide 16.7 -> 17.1, 2 rows 22.4 -> 20.7 and 16.2 -> 15.9; 1600 pairs, 5 rows 34.0 -> 36.9).  13 to 16 units: up to three, where it prepares
+// (12B shape, 7 and 8 rows at 3000 keys 3687 -> 3604 and 3766 -> 3698 us, up to nine at 7000 keys 3816 -> 3844 and 3860 -> 3907)
 static bool attention_rows_few(int tiles, int units, int nkv, bool prepares) {
-    return units <= LG_ATTN_FEW && tiles * nkv <= (prepares ? 9 : 3) * cu_count();
+    const int per_cu = units <= LG_ATTN_FEW ? (prepares ? 9 : 3) : units <= 16 && prepares ? 3 : 0;
+    return tiles * nkv <= per_cu * cu_count();
 }
 // workgroups of lg_k_attn_rows per kv head: three to a CU at most (its registers hold no more), each walking its share of the tiles
 static int attention_rows_wgs(int tiles, int units, int nkv) {
@@ -1436,8 +1438,10 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                                            : y.hd == 256 ? AttnRowsGeo<256>::bytes(M * G, fused_post) : y.hd == 128 ? AttnRowsGeo<128>::bytes(M * G, fused_post) : AttnRowsGeo<64>::bytes(M * G, fused_post);
                     const dim3 grid(few ? tiles : attention_rows_wgs(tiles, M * G, y.nkv), y.nkv);
                     a.gx = (int)grid.x;
-#define ATTN_ROWS(...) do { if (few) LAUNCH(KC_ATTN, (lg_k_attn_few<M, __VA_ARGS__>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0); \
-                            else     LAUNCH(KC_ATTN, (lg_k_attn_rows<M, __VA_ARGS__>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0); } while (0)
+#define ATTN_ROWS(HD, FQ) do { \
+    if constexpr (FQ && 16 / M * M > LG_ATTN_FEW) if (few && M * G > LG_ATTN_FEW) { LAUNCH(KC_ATTN, (lg_k_attn_few<M, HD, FQ, 4>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0); break; } \
+    if (few) LAUNCH(KC_ATTN, (lg_k_attn_few<M, HD, FQ>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0); \
+    else     LAUNCH(KC_ATTN, (lg_k_attn_rows<M, HD, FQ>), grid, dim3(LG_WG), lds, m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0); } while (0)
                     if (fused_post) {
                         a.qkv = m->qkv; a.ld = y.qkv_m; a.k_off = y.k_off; a.v_off = y.v_off;
                         a.q_norm = y.q_norm; a.k_norm = y.k_norm; a.rope_tab = y.rope_tab; a.rope_ff = y.rope_ff;
@@ -1446,9 +1450,9 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                         else if (y.hd == 128) ATTN_ROWS(128, true);
                         else                  ATTN_ROWS(64, true);
                     } else
-                    if (y.hd == 256)      ATTN_ROWS(256);
-                    else if (y.hd == 128) ATTN_ROWS(128);
-                    else                  ATTN_ROWS(64);
+                    if (y.hd == 256)      ATTN_ROWS(256, false);
+                    else if (y.hd == 128) ATTN_ROWS(128, false);
+                    else                  ATTN_ROWS(64, false);
 #undef ATTN_ROWS
                 }
             } else

@@ -190,7 +190,7 @@ def test_every_kernel_choice_gives_the_same_bits(lg, gpu_required, model_path, m
 @pytest.mark.parametrize("rows,over", [(5, {}), (8, {}), (2, {}), (5, {"head_dim": 256, "head_dim_full": 256}), (8, {"head_dim_full": 256}), (8, {"n_head": 4}),
                                        (7, {"head_dim": 128}), (5, {"n_head": 16}), (3, {"n_head": 20, "head_dim": 128})])
 def test_shared_tile_attention_prepares_its_own_rows(lg, ob, gpu_required, model_path, rows, over):
-    """Layers with 256 and more (tile, kv head) pairs take the attention kernels whose workgroups serve all rows of a block (up to 12
+    """Layers with 256 and more (tile, kv head) pairs take the attention kernels whose workgroups serve all rows of a block (up to 16
     units of (row, query head) on so few tiles on the vector units, more on the matrix cores); they norm and rotate the block's queries and
     build the block's K/V rows themselves.  A 2048-key window
     on 4 KV heads (66 tiles) and a global context of the same length, layers that own their cache and layers that
@@ -253,7 +253,7 @@ def test_shared_tile_attention_prepares_its_own_rows(lg, ob, gpu_required, model
 
 
 @pytest.mark.parametrize("n0,j,fq,n_head", [(2100, 0, 1, 8), (2100, 3, 1, 8), (2100, 7, 1, 8), (2100, 3, 0, 8), (20, 3, 1, 8), (20, 4, 0, 8),
-                                            (2100, 0, 1, 4), (2100, 7, 1, 4), (2100, 3, 0, 4), (20, 3, 1, 4)])
+                                            (2100, 0, 1, 4), (2100, 7, 1, 4), (2100, 3, 0, 4), (20, 3, 1, 4), (2100, 0, 1, 12), (2100, 7, 1, 12), (20, 3, 1, 12)])
 def test_a_block_row_of_nan_reaches_no_row_before_it(lg, gpu_required, model_path, model_dir, n0, j, fq, n_head):
     """Verify blocks whose rows share an attention tile (256 and more (tile, kv head) pairs), with a token whose embedding is
     infinite at row j of the block that a tile boundary cuts, behind a whole window and in the first keys of one: the cache rows in
@@ -297,7 +297,7 @@ def test_a_block_row_of_nan_reaches_no_row_before_it(lg, gpu_required, model_pat
 def test_block_rows_in_a_later_tile_of_their_workgroup(lg, gpu_required, model_path, n_head, hd, rows, pairs):
     """Long global layers of 8 kv heads whose pairs of tiles outnumber the workgroups that the CUs hold (96 per kv head): a block over the
     border between two pairs, prepared inside the attention kernel by the workgroups that walk to them as their second pair (16 units; 10 where
-    the tiles are too many for lg_k_attn_few; the last two cases go there), against lg_k_qkv_post ahead of it (attn_rows_fq = 0) and the kernel
+    the tiles are too many for lg_k_attn_few; the last two cases are those of 8 and 10 units that go there), against lg_k_qkv_post ahead of it (attn_rows_fq = 0) and the kernel
     per row (attn_rows = 0).  The keys in front are drawn."""
     path, spec = model_path("tiny", n_head=n_head, n_head_kv=8, head_dim_full=hd)
     n0 = 64 * pairs - 2
