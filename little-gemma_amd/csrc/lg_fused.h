@@ -1121,7 +1121,7 @@ __global__ __launch_bounds__(LG_WG) void lg_k_attn_few(const StepCtl *ctl, LG_AT
     if (!some) return;
     // values (lane = 4 dims).  A slot that a row does not see has weight 0 for it; where another row of the block has a value there that
     // is not finite, their product is a NaN.  So where the rows' keys may differ within the tile and a result is not finite, they are
-    // computed again with zeros in those slots (always with zeros there: 0.4 us more for the first and the last tile, which the merge waits for).
+    // computed again with zeros in those slots (always with zeros there: 0.4 to 1.1 us more for the first and the last tile, which the merge waits for).
     const uint16_t *vl = vt + (4 * lane < HD ? 4 * lane : 0);
     float4 acc[UB];
     auto values = [&](auto masked) {
