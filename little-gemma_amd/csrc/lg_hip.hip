@@ -1687,9 +1687,11 @@ static void launch_wide_attn(Launcher &lx, const WideAttn &a, int groups, bool f
     else                               LAUNCH(KC_ATTN, (lg_k_wide_attn<HD, false>), grid, dim3(LG_WA_WG), 0, a, lx.m->ctl);
 }
 
-// Rows of a prompt block up to which a row's work is cut over its slices (22 rows 5.0 -> 4.2 us a launch; 99 rows of the 12B shape: a prompt
-// 9251 -> 9286 us), and up to which the per-layer gate does the row work ahead of it (96 rows: 6862 -> 6751 us a prompt, 127: 6937 -> 7012).
-#define WIDE_SLICE_ROWS 64
+// Rows of a prompt block up to which a row's work is cut over its slices, and up to which the per-layer gate does the row work ahead of it.
+// Prompts of 33 to 256 tokens with either always and never (never -> always, us): slices, E4B shape, 32 rows 5394 -> 5334, 64 5970 -> 5902,
+// 79 6590 -> 6548, 96 6637 -> 6589, 111 6737 -> 6775, 127 6779 -> 6841, 255 8544 -> 8716; 12B shape, 32 rows 6780 -> 6668, 96 8972 -> 8906,
+// 111 9040 -> 9076, 127 9110 -> 9183.  Gate, 32 rows 5570 -> 5343, 64 6045 -> 5916, 96 6724 -> 6657, 111 6746 -> 6800, 255 8558 -> 9011.
+#define WIDE_SLICE_ROWS 96
 #define WIDE_GATE_ROWS 96
 // One block of `rows` prompt positions from pos on (tokens in device memory): the launch sequence of a verify step with
 // the kernels of lg_wide.h.  Launched as it is, not captured: a prompt's blocks differ in width and tile counts, and the
