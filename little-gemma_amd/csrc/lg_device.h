@@ -96,14 +96,15 @@ __host__ __device__ static inline int lg_act_block(ActLayout a, int b) {
 // instruction; the partner patterns (swap inside pairs, swap pairs inside quads, mirror 8, mirror
 // 16) differ from xor-butterflies only in which lane of the already-uniform sub-group supplies the
 // value, so sums come out in the same adjacent-pair tree order (addition is commutative) and
-// max / integer sums are order-free anyway.
+// max / integer sums are order-free anyway.  Every lane has a partner, so the move needs no fallback value and folds into the
+// addition behind it (with a zero as the fallback it was two moves more: a 5-row step of the E4B shape 2206 -> 2200 us).
 template <int CTRL>
 __device__ __forceinline__ float lg_dpp_f(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
 }
 template <int CTRL>
 __device__ __forceinline__ int lg_dpp_i(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
+    return __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, true);
 }
 #define LG_DPP_SWAP1   0xB1     // quad_perm [1,0,3,2]
 #define LG_DPP_SWAP2   0x4E     // quad_perm [2,3,0,1]
@@ -181,6 +182,45 @@ __device__ __forceinline__ float lg_div127(float amax) {
     const float r = 1.0f / 127.0f;
     const float q0 = amax * r;
     return lg_fmaf(lg_fmaf(-127.0f, q0, amax), r, q0);
+}
+
+// The correctly rounded 1/d for normal d of 2^-100..2^100: the reciprocal instruction (1 ulp) and one Newton step, which leaves
+// r(1 + e) = (1 - e*e)/d with |e| < 2^-22 before its one rounding.  On this chip that rounds every d as the division does
+// (checked on it for all 2^23 mantissas; powers of two change nothing in this range): three instructions for its ten.
+__device__ __forceinline__ float lg_rcp_exact(float d) {
+    const float r = __builtin_amdgcn_rcpf(d);
+    return lg_fmaf(lg_fmaf(-d, r, 1.0f), r, r);
+}
+// 1/d, 0 where d is not positive: the factor of a q8 block.
+__device__ __forceinline__ float lg_inv_scale(float d) {
+    if (__float_as_uint(d) - 0x0D800000u < 0x64000000u) return lg_rcp_exact(d);          // 2^-100 <= d < 2^100
+    return d > 0.0f ? 1.0f / d : 0.0f;
+}
+
+// lg_gelu without branches, so that the gates of a lane overlap: the same value for every float (checked for all of them).  Both forms of the hyperbolic tangent are
+// computed and one chosen, the clamps that cannot bind there left out, 2/(e+1) as an exact reciprocal (e + 1 is 4.4 to 2^58).
+__device__ __forceinline__ float lg_gelu_d(float x) {
+    const float a = 0.7978845608028654f * (x + 0.044715f * x * x * x), ax = fabsf(a);
+    const float y = ax > 9.0f ? 20.0f : ax, y2 = y + y;       // e^40: 1 - 2/(e+1) is 1
+    const float n = lg_rintf(y2 * 1.44269504088896341f);
+    float r = lg_fmaf(n, -0.693145751953125f, y2);
+    r = lg_fmaf(n, -1.428606765330187045e-06f, r);
+    float p = 1.9875691500e-4f;
+    p = lg_fmaf(p, r, 1.3981999507e-3f);
+    p = lg_fmaf(p, r, 8.3334519073e-3f);
+    p = lg_fmaf(p, r, 4.1665795894e-2f);
+    p = lg_fmaf(p, r, 1.6666665459e-1f);
+    p = lg_fmaf(p, r, 5.0000001201e-1f);
+    const float e = (lg_fmaf(p, r * r, r) + 1.0f) * __uint_as_float((uint32_t)((int)n + 127) << 23);
+    const float t = lg_fmaf(-2.0f, lg_rcp_exact(e + 1.0f), 1.0f);
+    const float z = a * a;
+    float q = -5.70498872745e-3f;
+    q = lg_fmaf(q, z, 2.06390887954e-2f);
+    q = lg_fmaf(q, z, -5.37397155531e-2f);
+    q = lg_fmaf(q, z, 1.33314422036e-1f);
+    q = lg_fmaf(q, z, -3.33332819422e-1f);
+    const float s = lg_fmaf(q * z, a, a), th = ax < 0.625f ? s : __builtin_copysignf(t, a);
+    return 0.5f * x * (1.0f + th);
 }
 
 // q8 quantization of 32 consecutive values held as one float4 in each of 8 adjacent lanes:

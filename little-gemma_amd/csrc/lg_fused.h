@@ -279,7 +279,7 @@ __global__ __launch_bounds__(LG_WG) void lg_k_mmf(MmfArgs a) {
     for (int j = 0; j < MC; ++j) acc[j] = lg_wave_sum64(acc[j]);
     if (lane < MC && j0 + lane < a.rows) {
         float v = lg_pick<MC>(acc, lane);
-        if (a.ipl) v = lg_gelu(v) * a.ipl[(size_t)(j0 + lane) * a.ipl_ld + i];
+        if (a.ipl) v = lg_gelu_d(v) * a.ipl[(size_t)(j0 + lane) * a.ipl_ld + i];
         a.out[(size_t)(j0 + lane) * a.ldo + i] = v;
     }
 }
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(LG_WG) void lg_k_rows_mmf(RowsMmfArgs a) {
         acc = lg_fmaf(w.x, x.x, acc); acc = lg_fmaf(w.y, x.y, acc); acc = lg_fmaf(w.z, x.z, acc); acc = lg_fmaf(w.w, x.w, acc);
     }
     acc = lg_wave_sum64(acc);
-    if (lane == 0) a.out[(size_t)(j0 + wave) * a.m + i] = lg_gelu(acc) * iplv;
+    if (lane == 0) a.out[(size_t)(j0 + wave) * a.m + i] = lg_gelu_d(acc) * iplv;
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -2323,7 +2323,6 @@ static int read_back_wide(const uint8_t *dq, int rows, int k, int8_t *xq, float 
     const int nb = k / 32;
     std::vector<uint8_t> dev(lg_wide_q8_bytes(rows, k));
     HIP_TRY(hipMemcpy(dev.data(), dq, dev.size(), hipMemcpyDeviceToHost));
-    static const int mag[9] = { 0, 12, 16, 18, 20, 21, 22, 23, 24 };          // 6-bit codes of 0..8
     for (int j = 0; j < rows; ++j)
         for (int b = 0; b < nb; ++b) {
             const uint8_t *t = dev.data() + ((size_t)(j >> 6) * nb + b) * LG_QTILE;
@@ -2335,9 +2334,7 @@ static int read_back_wide(const uint8_t *dq, int rows, int k, int8_t *xq, float 
                 memcpy(bytes + 16, t + base + 1024 + lane * 8, 8);
                 for (int e = 0; e < 32; ++e) {
                     const int code = ((bytes[6 * e / 8] | (bytes[6 * e / 8 + 1] << 8)) >> (6 * e % 8)) & 63;
-                    int x = 0;
-                    for (int i = 0; i < 9; ++i) if (mag[i] == (code & 31)) x = i;
-                    v[half][e] = (code & 32) ? -x : x;
+                    v[half][e] = (code & 32) ? -(code & 31) : code & 31;
                 }
             }
             for (int e = 0; e < 32; ++e) {

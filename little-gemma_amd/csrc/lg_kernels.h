@@ -538,7 +538,7 @@ __global__ __launch_bounds__(512, 2) void lg_k_geglu_t(LG_GEGLU_FIELDS(LG_XP, _)
         const float gate = ((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]));
         const float up = ((u[0] + u[1]) + (u[2] + u[3])) + ((u[4] + u[5]) + (u[6] + u[7]));
         float d; int sum;
-        const int q = lg_quant1_32lanes(lg_gelu(gate) * up, &d, &sum);
+        const int q = lg_quant1_32lanes(lg_gelu_d(gate) * up, &d, &sum);
         const ActLayout lay = lg_act_layout(a.n_ff);          // order the ffn_down matmul reads
         a.gq[(size_t)j * a.n_ff + lg_act_unit(lay, t * 2 + (i >> 4)) * 16 + (i & 15)] = (int8_t)q;
         if (i == 0) lg_q8_ds<M>(a.gq, a.n_ff)[(size_t)j * (a.n_ff >> 5) + lg_act_block(lay, t)] = make_float2(d, __int_as_float(sum));
@@ -655,7 +655,7 @@ __global__ __launch_bounds__(512, 2) void lg_k_geglu_m(LG_GEGLU_FIELDS(LG_XP, _)
         const float gate = ((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]));
         const float up = ((u[0] + u[1]) + (u[2] + u[3])) + ((u[4] + u[5]) + (u[6] + u[7]));
         float d; int sum;
-        const int q = lg_quant1_32lanes(lg_gelu(gate) * up, &d, &sum);
+        const int q = lg_quant1_32lanes(lg_gelu_d(gate) * up, &d, &sum);
         if (a.gq_units == 2) {                                // block t of 80 dwords: row slot j's 32 bytes, dwords in the order 0 1 4 5 2 3 6 7
             int8_t *blk = a.gq + (size_t)t * (LG_MU_DWORDS * 4);
             const int dw = i >> 2;
@@ -814,7 +814,7 @@ __device__ __forceinline__ void lg_rows_plegate_body(const RowsPleGateArgs &a, i
             }
         }
         p = lg_sum_seg<8>(p);
-        if (c == 0) gbuf[wave * 8 + (lane >> 3)] = lg_gelu(p) * iplv;
+        if (c == 0) gbuf[wave * 8 + (lane >> 3)] = lg_gelu_d(p) * iplv;
     }
     __syncthreads();
     sink(gbuf);

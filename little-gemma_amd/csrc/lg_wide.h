@@ -5,10 +5,11 @@
 // contiguous K segments, then the adjacent-pair tree over the segments.  What is left to the vector units is the one
 // fma per output and block that this order needs; everything else of a block runs on the matrix cores:
 //
-//  * the dot, as v_mfma_scale_f32_32x32x64_f8f6f4 on 6-bit floats (e3m2, which holds every integer -8..8 exactly).
-//    A weight is one such value (its nibble - 8).  A q8 value q is two, q = 16*hi + lo with hi = (q+8) >> 4 in -8..8
-//    and lo in -8..7: the instruction's K = 64 is the block's 32 weights twice against its 32 hi and its 32 lo digits,
-//    and the factor 16 is the E8M0 scale of the first half.  Products and sums are integers below 2^15, so the result
+//  * the dot, as v_mfma_scale_f32_32x32x64_f8f6f4 on 6-bit floats (e2m3, whose codes 0..15 are the multiples 0..15 of 2^-3 and whose
+//    bit 5 is the sign: the code of an integer is its magnitude and its sign).  A weight is one such value (its nibble - 8).  A q8
+//    value q is two, the high and the low four bits of |q|, each with the sign of q: the instruction's K = 64 is the block's 32 weights
+//    twice against its 32 high and its 32 low digits.  The factors 16 of the high half and 2^3 of every code are the
+//    E8M0 scales.  Products and sums are integers below 2^15 (an integer times 2^-6 inside), so the result
 //    is the exact dot, already a float.  On int8 (v_mfma_i32_32x32x32_i8, the same 32 cycles) every output needs a
 //    subtraction to become (float)(dot - 8*sum).
 //  * the products xd*dw, as the outer product v_mfma_f32_32x32x1_2b_f32 with a zero accumulator: fma(x, y, 0) is the
@@ -36,12 +37,11 @@ typedef float lg_v32f __attribute__((ext_vector_type(32)));
 #define LG_WIDE_ROWS 512                   // rows of the widest block
 #define LG_WIDE_MID  128                   // the widest block of a short cache
 
-// 6-bit float code (sign, 3 exponent bits of bias 3, 2 mantissa bits) of an integer -8..8 given as a float; of any other
-// value, six bits
-__device__ __forceinline__ uint32_t lg_e3m2(float v) {
-    const uint32_t u = __float_as_uint(v);
-    const int e = (int)((u & 0x7FFFFFFFu) >> 21) - (124 << 2);
-    return (uint32_t)(e < 0 ? 0 : e > 31 ? 31 : e) | ((u >> 26) & 0x20u);
+// 6-bit float code of an integer -15..15: its value times 8, sign and magnitude
+__device__ __forceinline__ uint32_t lg_e2m3(int v) { return (uint32_t)(v < 0 ? -v : v) | (v < 0 ? 0x20u : 0u); }
+// four such codes in the bytes of x -> 24 bits
+__device__ __forceinline__ uint32_t lg_pack6(uint32_t x) {
+    return __builtin_amdgcn_udot4(x, 0x00004001u, __builtin_amdgcn_udot4(x, 0x40010000u, 0u, false) << 12, false);
 }
 // Where the digits of (row j, block b) of a wide activation buffer of nb blocks per row live: dword d (0..5) of the hi
 // (half = 0) or lo (half = 1) digits, and the row's scale.
@@ -55,23 +55,23 @@ __device__ __forceinline__ int lg_qscale(int j) { return 3072 + (j & 63) * 4; }
 __host__ __device__ static inline size_t lg_wide_q8_bytes(int rows, int k) { return (size_t)((rows + 63) / 64) * (size_t)(k >> 5) * LG_QTILE; }
 
 // q8 of 32 values held as one float4 in each of 8 adjacent lanes (lane % 8 = i holds elements 4i..4i+3 of block b of row
-// j), written as digits: the arithmetic of lg_quant4_8lanes.
+// j), written as digits: the arithmetic of lg_quant4_8lanes.  Bound by vector issue, next to which the matmuls that end in it run:
+// sign and magnitude take 26 instructions for four values where digits that are sums (e3m2 codes of q = 16*hi + lo) took 94.
+// With lg_gelu_d: 1000 tokens of the E4B shape 21.87 -> 21.46 ms, 4093 of the 12B shape 184.1 -> 181.0 ms.
 __device__ __forceinline__ void lg_wide_quant4(float4 h, uint8_t *q, int nb, int j, int b) {
     float amax = fmaxf(fmaxf(fabsf(h.x), fabsf(h.y)), fmaxf(fabsf(h.z), fabsf(h.w)));
     amax = lg_max_n(amax, 8);
     const float d = lg_div127(amax);
-    const float id = d > 0.0f ? 1.0f / d : 0.0f;
+    const float id = lg_inv_scale(d);
     const float p[4] = { h.x * id, h.y * id, h.z * id, h.w * id };
-    uint32_t hi = 0, lo = 0;
+    // |q| in the four bytes: a NaN becomes 0, as in the conversion to int8, and the values next to it keep their digits (an infinity
+    // among the 32 makes their scale a NaN, so that the block does not pass for finite).  Signs: bit 7 of the floats' last bytes.
+    uint32_t mag = 0;
     #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        // a NaN becomes 0, as in the conversion to int8, and the values next to it keep their digits (an infinity among the 32
-        // makes their scale a NaN, so that the block does not pass for finite)
-        const float v = p[i] == p[i] ? lg_rintf(p[i]) : 0.0f;
-        const float fh = floorf((v + 8.0f) * 0.0625f), fl = lg_fmaf(-16.0f, fh, v);
-        hi |= lg_e3m2(fh) << (6 * i);
-        lo |= lg_e3m2(fl) << (6 * i);
-    }
+    for (int i = 0; i < 4; ++i) mag = __builtin_amdgcn_cvt_pk_u8_f32(lg_rintf(fabsf(p[i])), i, mag);
+    const uint32_t sg = ((__builtin_amdgcn_perm(__float_as_uint(p[1]), __float_as_uint(p[0]), 0x0C0C0703u) |
+                          __builtin_amdgcn_perm(__float_as_uint(p[3]), __float_as_uint(p[2]), 0x07030C0Cu)) >> 2) & 0x20202020u;
+    const uint32_t hi = lg_pack6(((mag >> 4) & 0x0F0F0F0Fu) | sg), lo = lg_pack6((mag & 0x0F0F0F0Fu) | sg);
     // 24 bits per lane, four lanes make three dwords: lane k (k = 0..2 of the four) completes its bits with its neighbour's
     const int i = (int)threadIdx.x & 7, k = i & 3, dw = 3 * (i >> 2) + k;
     const uint32_t nh = (uint32_t)lg_dpp_i<0xF9>((int)hi), nl = (uint32_t)lg_dpp_i<0xF9>((int)lo);   // quad_perm [1,2,3,3]
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(LG_WG) void lg_k_wide_pack(const uint8_t *w, int k,
         #pragma unroll
         for (int e = 0; e < 32; ++e) {
             const int nib = e < 16 ? (qs[e] & 15) : (qs[e - 16] >> 4);
-            const uint64_t c = (uint64_t)lg_e3m2((float)(nib - 8)) << ((6 * e) & 31);
+            const uint64_t c = (uint64_t)lg_e2m3(nib - 8) << ((6 * e) & 31);
             out[(6 * e) >> 5] |= (uint32_t)c;
             if (((6 * e) & 31) > 26) out[((6 * e) >> 5) + 1] |= (uint32_t)(c >> 32);
         }
@@ -169,7 +169,7 @@ __device__ __forceinline__ void lg_wide_tile(const WideMm &a, int at, int bt, in
         }
         o.xs = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rq, vxs, qo, 0));
     };
-    const int sb = lane < 32 ? 131 : 127;                     // E8M0 scales of the K halves: 2^4 for the hi digits, 1 for the lo digits
+    const int sb = lane < 32 ? 134 : 130;                     // E8M0 scales of the K halves: 2^3 of the codes, 2^4 more for the high digits
     const lg_v16f z16 = {};
     const lg_v32f z32 = {};
     float p[2][TB][16];
@@ -211,8 +211,8 @@ __device__ __forceinline__ void lg_wide_tile(const WideMm &a, int at, int bt, in
     for (int i = 0; i < NS; ++i) fetch(o[i], i < last ? i : last);
     clear();
     take(o[0]);
-    D0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a0, o[0].b[0], z16, 3, 3, 0, 127, 0, sb);
-    D1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a1, o[0].b[0], z16, 3, 3, 0, 127, 0, sb);
+    D0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a0, o[0].b[0], z16, 2, 2, 0, 130, 0, sb);
+    D1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a1, o[0].b[0], z16, 2, 2, 0, 130, 0, sb);
     auto block = [&](int it, int u, bool more) {              // block it + u; `more`: its registers receive block it + u + NS
         if (WV == 4 && it + u == nit) segment_end();
         #pragma unroll
@@ -234,12 +234,12 @@ __device__ __forceinline__ void lg_wide_tile(const WideMm &a, int at, int bt, in
             #pragma unroll
             for (int i = 0; i < 16; ++i) p[0][t][i] = lg_fmaf(S[i], D0[i], p[0][t][i]);
             __builtin_amdgcn_sched_barrier(0);
-            D0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a0, on.b[tn], z16, 3, 3, 0, 127, 0, sb);
+            D0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a0, on.b[tn], z16, 2, 2, 0, 130, 0, sb);
             __builtin_amdgcn_sched_barrier(0);
             #pragma unroll
             for (int i = 0; i < 16; ++i) p[1][t][i] = lg_fmaf(S[16 + i], D1[i], p[1][t][i]);
             __builtin_amdgcn_sched_barrier(0);
-            D1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a1, on.b[tn], z16, 3, 3, 0, 127, 0, sb);
+            D1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a1, on.b[tn], z16, 2, 2, 0, 130, 0, sb);
             if (more && t == (TB == 2 ? 0 : TB - 1)) { const int nx = it + u + NS; fetch(o[u], nx < last ? nx : last); }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -315,7 +315,7 @@ __global__ __launch_bounds__(64 * WV, 2) void lg_k_wide_geglu(WideMm a, uint8_t 
         const int tb = u >> 2, g = u & 3;
         const float4 gv = lg_wide_sum<TB, WV>(lds, tb * 4 + g), uv = lg_wide_sum<TB, WV>(lds, (TB + tb) * 4 + g);
         *(float4 *)(vbuf + (32 * tb + n) * 36 + 8 * g + 4 * h) =
-            make_float4(lg_gelu(gv.x) * uv.x, lg_gelu(gv.y) * uv.y, lg_gelu(gv.z) * uv.z, lg_gelu(gv.w) * uv.w);
+            make_float4(lg_gelu_d(gv.x) * uv.x, lg_gelu_d(gv.y) * uv.y, lg_gelu_d(gv.z) * uv.z, lg_gelu_d(gv.w) * uv.w);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 32 * TB * 8; i += 64 * WV) {
@@ -340,7 +340,7 @@ __global__ __launch_bounds__(64 * WV, 2) void lg_k_wide_plegate(WideMm a, const 
         const int col = at * LG_WT + 32 * ta + 8 * g + 4 * h;
         const float4 p = *(const float4 *)(ipl + ((size_t)(an < a.rows ? an : a.rows - 1) * n_layer + layer) * a.m + col);
         *(float4 *)(vbuf + (ta * 32 * TB + 32 * tb + n) * 36 + 8 * g + 4 * h) =
-            make_float4(lg_gelu(v.x) * p.x, lg_gelu(v.y) * p.y, lg_gelu(v.z) * p.z, lg_gelu(v.w) * p.w);
+            make_float4(lg_gelu_d(v.x) * p.x, lg_gelu_d(v.y) * p.y, lg_gelu_d(v.z) * p.z, lg_gelu_d(v.w) * p.w);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 2 * 32 * TB * 8; i += 64 * WV) {

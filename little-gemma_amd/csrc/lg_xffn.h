@@ -417,7 +417,7 @@ __global__ __launch_bounds__(LG_XFFN_THREADS) void lg_k_ffn_xcd(LG_XFFN_FIELDS(L
             for (int k = 0; k < 8; ++k) { gg[k] = red[(k * M + j) * W + c]; uu[k] = red[(k * M + j) * W + g.CW + c]; }
             const float gate = ((gg[0] + gg[1]) + (gg[2] + gg[3])) + ((gg[4] + gg[5]) + (gg[6] + gg[7]));
             const float up = ((uu[0] + uu[1]) + (uu[2] + uu[3])) + ((uu[4] + uu[5]) + (uu[6] + uu[7]));
-            actbuf[i] = lg_gelu(gate) * up;
+            actbuf[i] = lg_gelu_d(gate) * up;
         }
         lg_rowsync(&rcnt, uses);
         // ---- B -> C

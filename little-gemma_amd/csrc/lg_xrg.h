@@ -258,7 +258,7 @@ __global__ __launch_bounds__(512, 4) void lg_k_rows_geglu(StepCtl *ctl, LG_RG_FI
         const float gate = ((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]));
         const float up = ((u[0] + u[1]) + (u[2] + u[3])) + ((u[4] + u[5]) + (u[6] + u[7]));
         float d; int sum;
-        const int q = lg_quant1_32lanes(lg_gelu(gate) * up, &d, &sum);
+        const int q = lg_quant1_32lanes(lg_gelu_d(gate) * up, &d, &sum);
         if (a.gq_units == 2) {                                // block t of 80 dwords: row slot j's 32 bytes, dwords in the order 0 1 4 5 2 3 6 7
             int8_t *blk = a.gq + (size_t)t * (LG_MU_DWORDS * 4);
             const int dw = i >> 2;

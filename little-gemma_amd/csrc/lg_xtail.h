@@ -354,7 +354,7 @@ __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FI
             }
         }
         pr = lg_sum_seg<8>(pr);
-        if (c == 0) a.gf[(size_t)j * ple + gg * 8 + (lane >> 3)] = lg_gelu(pr) * iplv;
+        if (c == 0) a.gf[(size_t)j * ple + gg * 8 + (lane >> 3)] = lg_gelu_d(pr) * iplv;
     }
     stamp(1);
     // ---- hand-over: every part's gated values of its row are in the XCD's L2 ----

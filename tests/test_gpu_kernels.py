@@ -397,3 +397,25 @@ def test_gate_up_geglu_matches_oracle(lg, ob, gpu_required, rows, E, FF):
     assert np.array_equal(r["asum"], asum), "sums"
     print(f"  kernel {1e3 * r['ms']:.2f} us", flush=True)
 
+
+
+@pytest.mark.parametrize("rows", [2, 8])
+def test_gelu_from_tiny_to_saturated_gates(lg, ob, gpu_required, rows):
+    """Gates of every size through gate/up: the polynomial around 0, the exponential, the step to 1 at 9 and gates whose cube
+    overflows.  The device's GELU has no branches and its own division: equal bits at every size."""
+    E, FF = 512, 2048
+    rng = np.random.default_rng(rows)
+    scale = np.array([1e-3, 0.05, 0.3, 1.0, 3.0, 10.0, 1e3, 1e14][:rows] if rows == 8 else [0.3, 5.0], np.float32)
+    x = rng.normal(0, 1, (rows, E)).astype(np.float32) * scale[:, None]
+    wg, wu = random_q4_0(rng, FF, E), random_q4_0(rng, FF, E)
+    print(f"gelu rows={rows}", flush=True)
+    r = lg.hiplib.gate_up_geglu(x, wg, wu, FF)
+    L = ob.lib()
+    gate, up = oracle_matmul(ob, wg, E, FF, x)[3], oracle_matmul(ob, wu, E, FF, x)[3]
+    for j in range(rows):
+        act = np.array([L.lgo_gelu(float(v), 1) for v in gate[j]], np.float32) * up[j]
+        aq, ad, asum = np.zeros(FF, np.int8), np.zeros(FF // 32, np.float32), np.zeros(FF // 32, np.int32)
+        L.lgo_quant_q8(act, FF, aq, ad, asum)
+        fin = np.isfinite(ad)
+        assert np.array_equal(r["ad"][j][fin].view(np.uint32), ad[fin].view(np.uint32)) and np.array_equal(np.isfinite(r["ad"][j]), fin)
+        assert np.array_equal(r["aq"][j].reshape(-1, 32)[fin], aq.reshape(-1, 32)[fin])
