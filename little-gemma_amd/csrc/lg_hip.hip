@@ -27,6 +27,7 @@
 #include "lg_xffn.h"
 #include "lg_xtail.h"
 #include "lg_xrg.h"
+#include "lg_narrow.h"
 
 static_assert(LG_HIP_MAX_ROWS == LG_HIP_MAX_ROWS_DEV, "row limits must agree");
 #define LG_FUSE_ROWS_MAX 2         // widest block whose q/k/v matmul does the preceding row work itself
@@ -218,7 +219,7 @@ struct lg_hip_model {
     int last_rows = 0, last_adv = 0;
     float *lstage = nullptr;           // pinned: two rows of logits on their way to a caller (lg_hip_get_logits), row j in half j % 2
     int lread = -1, lcoming = -1;      // the row of the latest step read last, and the one whose copy has been started
-    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0;
+    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1;
     // the feed-forward half of a layer as one XCD-partitioned launch (lg_xffn.h): built when the shape and the chip fit
     int xcd_ffn = 0;                         // option: use it (verify blocks of 4..8 rows)
     int down_m = 1;                          // option: ffn_down of 4..8-row blocks on the matrix cores (lg_k_down_m): 1 = the row group's four workgroups add
@@ -236,6 +237,7 @@ struct lg_hip_model {
     int xcd_tail = 1;                        // option: 0 off, 1 for blocks that do not fold the row work into q/k/v, 2 for every verify block
     XtailSync *tsync = nullptr;
     float *tgf = nullptr;                    // [LG_HIP_MAX_ROWS][ple] gated values of lg_k_ple_tail_s
+    NarrowSync *nsync = nullptr;             // hand-over state of lg_k_narrow (models it serves: narrow_shape)
     RgSync *rgsync = nullptr;                // flags and epoch base of lg_k_rows_geglu
     unsigned long long *tstamps = nullptr;   // [LG_XTAIL_UNITS][8] phase stamps of the last such launch (option xcd_tail_stamps)
     int tail_stamps = 0;
@@ -532,6 +534,15 @@ static bool attn_tail_shape(int qd, int E, int *np, int *rbs) {
     return (p == 1 && r == 1) || (p == 2 && r == 1) || (p == 4 && r == 3);
 }
 
+// Models whose layers lg_k_narrow serves: what its registers, LDS and 256 wavefronts hold, q4_0 matrices throughout
+static bool narrow_shape(const lg_hip_model *m) {
+    if (cu_count() != LG_XCDS * LG_XCD_WGS || m->E % 256 || m->E > LG_NARROW_E || m->H > LG_NARROW_WGS || (m->ple && m->ple != 256)) return false;
+    for (const Layer &y : m->L)
+        if (y.hd > LG_WG || y.hd % 64 || y.qd % 256 || y.qd > LG_NARROW_K || y.nff % 256 || y.nff > LG_NARROW_K || y.qkv_m % 8 || y.qkv_m > LG_NARROW_K ||
+            !y.wqkv || !y.wo || !y.wgu || !y.wdown || (m->ple && (!y.winp || !y.wproj))) return false;
+    return true;
+}
+
 static const float *rope_table(lg_hip_model *m, int is_local, int hd, int *rc) {
     auto key = std::make_pair(is_local, hd);
     auto it = m->rope_tabs.find(key);
@@ -765,6 +776,10 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         HIP_TRY(hipMemset(m->rgsync, 0, sizeof(RgSync)));
         HIP_TRY(hipMemset(m->aq, 0, qb(max_qd)));       // (row slots past the block are read as operand rows of the matrix cores)
         if (getenv("LG_HIP_XCD_TAIL")) m->xcd_tail = atoi(getenv("LG_HIP_XCD_TAIL"));
+    }
+    if (narrow_shape(m)) {
+        if (dev_alloc(m, &m->nsync, (size_t)1)) return -7;
+        HIP_TRY(hipMemset(m->nsync, 0, sizeof(NarrowSync)));
     }
     if (getenv("LG_HIP_XCD_ATTN_TAIL")) m->xcd_attn_tail = atoi(getenv("LG_HIP_XCD_ATTN_TAIL"));
     if (getenv("LG_HIP_DOWN_M")) m->down_m = atoi(getenv("LG_HIP_DOWN_M"));
@@ -1156,6 +1171,10 @@ static bool use_ple_tail(const lg_hip_model *m, int rows) {
     if (!spread && (m->E / 8 + 4 * U - 1) / (4 * U) > 4) return false;       // (few rows of a wide model: too few wavefronts for the projection)
     return cu_count() == LG_XCDS * LG_XCD_WGS;
 }
+// One row of a narrow model: a layer from the merge on, and the next layer's q/k/v, as one launch (every kernel choice left as it comes)
+static bool use_narrow(const lg_hip_model *m, int rows) {
+    return rows == 1 && m->narrow && m->nsync && m->fuse_rows && m->xcd_tail == 1 && m->tail_spread == 1 && !m->xcd_attn_tail && !m->merge_o && !m->fork_ple;
+}
 // Slices of the E output rows per (head, row) of lg_k_merge_o: a divisor of the E/64 chunks that leaves at most two
 // chunks per wavefront, the largest that keeps the launch within one workgroup per CU (else the smallest)
 static int merge_o_slices(const lg_hip_model *m, int rows) {
@@ -1349,6 +1368,8 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
     };
 
     const bool tail = use_ple_tail(m, M);
+    const bool narrow = use_narrow(m, M);
+    bool qkv_done = false;                         // the layer's projections have been done by the launch before it (lg_k_narrow)
     bool rows_done = false;                        // the row work ahead of the next matmul has been done by the launch before it
     bool join_ple = false;                         // the forked branch has to be waited for before its result is used
     if (m->ple) {
@@ -1404,7 +1425,8 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         bool fused_post = false, merged_o = false, ffn_rows_done = false;
         {   // q/k/v projections, then per-head norm, rotary and the K/V rows of this block
             MmArgs a{ y.wqkv, E, y.qkv_m, m->qkv, m->hq, nullptr };
-            if (rows_done) { launch_mm<M, false>(lx, KC_QKV, a); rows_done = false; }      // (the previous layer's tail did this layer's row work)
+            if (qkv_done) { qkv_done = rows_done = false; }
+            else if (rows_done) { launch_mm<M, false>(lx, KC_QKV, a); rows_done = false; }      // (the previous layer's tail did this layer's row work)
             else if (can_fuse()) rows_mm(y.attn_norm, a, KC_QKV);
             else { rows(y.attn_norm, nullptr); launch_mm<M, false>(lx, KC_QKV, a); }
             // blocks of the model itself, up to LG_HIP_MAX_ROWS rows: the attention kernel does this part as well
@@ -1466,6 +1488,23 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 LAUNCH(KC_ATTN, (lg_k_attn<false, 1>), dim3(tiles, y.nkv, M), dim3(LG_WG), attn_lds(G, y.hd, false), m->ctl, LG_ATTN_FIELDS(LG_XA, a) 0);
             }
             MergeArgs g{ kv->pm, kv->pl, kv->pacc, kv->tiles_max, H, y.hd, window, pos_off, m->aq, nullptr };
+            if constexpr (M == 1) if (narrow && (L + 1 < nl || with_head)) {
+                const bool last = L + 1 == nl;
+                NarrowArgs f{};
+                f.g = g; f.x = m->x[cur]; f.x_out = m->x[cur ^ 1];
+                f.wo = y.wo; f.wgu = y.wgu; f.wdn = y.wdown; f.winp = y.winp; f.wproj = y.wproj; f.wq = last ? nullptr : m->L[L + 1].wqkv;
+                f.post_attn = y.post_attn; f.ffn_norm = y.ffn_norm; f.post_ffw = y.post_ffw; f.post_norm = y.post_norm; f.os = y.out_scale;
+                f.w_pre = last ? m->output_norm : m->L[L + 1].attn_norm;
+                f.ipl = m->ple ? m->pmp_raw + (size_t)L * m->ple : nullptr;
+                f.qkv = m->qkv; f.h_out = last ? m->hidden_rows : nullptr; f.hq = m->hq;
+                f.E = E; f.qd = y.qd; f.FF = y.nff; f.qm = last ? 0 : m->L[L + 1].qkv_m; f.tiles = tiles; f.eps = m->eps;
+                f.sync = m->nsync; f.err = &m->ctl->err; f.err2 = draft ? &m->target->ctl->err : nullptr; f.spin_limit = 1 << 16;
+                if (m->ple) LAUNCH(KC_TAIL, lg_k_narrow<true>, dim3(LG_XCDS * LG_NARROW_WGS), dim3(512), 0, f, m->ctl);
+                else        LAUNCH(KC_TAIL, lg_k_narrow<false>, dim3(LG_XCDS * LG_NARROW_WGS), dim3(512), 0, f, m->ctl);
+                cur ^= 1;
+                rows_done = true; qkv_done = !last;
+                continue;
+            }
             merged_o = pos_off == 0 && use_merge_o(m, y, M, tiles);
             if (pos_off == 0 && have_x && use_attn_tail(m, y, M, tiles)) {
                 // merge, output projection and the row work ahead of gate/up as one launch on one XCD
@@ -1807,7 +1846,7 @@ static GraphKey graph_key(const lg_hip_model *m, const lg_hip_kv *kv, int rows, 
     put(what, 2); put(rows, 4); put(m->store_logits != 0, 1); put(m->draft_chain, 1); put(m->fuse_rows, 1); put(m->attn_rows, 1); put(m->attn_rows_fq, 1);
     put(m->head_mfma, 1); put(m->down_kq, 1); put(m->xcd_ffn, 1); put(m->fork_ple, 1); put(m->rows_geglu, 1); put(m->tail_stamps != 0, 1);
     put(m->tail_spread == 1 ? 1 : m->tail_spread ? 2 : 0, 2); put(m->xcd_tail, 2); put(m->down_m, 2); put(m->xcd_attn_tail, 2); put(m->merge_o, 2);
-    put(m->xffn_delay, 10);
+    put(m->xffn_delay, 10); put(m->narrow, 1);
     return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices };
 }
 
@@ -1866,6 +1905,7 @@ extern "C" int lg_hip_set_option(lg_hip_model *m, const char *name, int value) {
     else if (!strcmp(name, "attn_rows_fq")) m->attn_rows_fq = value != 0;
     else if (!strcmp(name, "xcd_tail_spread")) m->tail_spread = value;
     else if (!strcmp(name, "rows_geglu")) m->rows_geglu = value != 0;
+    else if (!strcmp(name, "narrow")) m->narrow = value != 0;
     else if (!strcmp(name, "down_kq")) m->down_kq = value != 0;
     else if (!strcmp(name, "xcd_ffn")) m->xcd_ffn = value != 0 && m->xffn_built;
     else if (!strcmp(name, "fork_ple")) m->fork_ple = value != 0;
@@ -2021,6 +2061,7 @@ extern "C" int lg_hip_mtp_rounds(lg_hip_model *d, lg_hip_kv *kv, int token, int 
     } else {
         GraphKey key = graph_key(t, kv, rows, 2);
         key[1] |= (uint64_t)(d->store_logits != 0) << 62 | (uint64_t)(d->fuse_rows != 0) << 63;
+        key[2] |= (uint64_t)(d->narrow != 0) << 63;
         auto it = d->graphs.find(key);            // kept by the head: the graph dies with it or with the cache
         int r = 0;
         if (it == d->graphs.end()) {               // the first round as launches, its graph while the device works on it
@@ -2197,9 +2238,12 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
     const double q = 18.0 / 32.0;                         // bytes per q4_0 weight
     for (int i = 0; i < KC_COUNT; ++i) b[i] = 0;
     if (m->ple) b[KC_PMP] = (double)m->E * m->ple * m->n_layer * (m->pmp_f ? 4.0 : q);
+    const bool narrow = use_narrow(m, rows);              // (everything but the attention and the first layer's projections)
     for (int L = 0; L < m->n_layer; ++L) {
         const Layer &y = m->L[L];
-        b[KC_QKV] += (double)m->E * y.qkv_m * q;
+        b[narrow && L ? KC_TAIL : KC_QKV] += (double)m->E * y.qkv_m * q;
+        if (narrow) b[KC_TAIL] += ((double)y.qd * m->E + 3.0 * m->E * y.nff + 2.0 * m->E * m->ple) * q;
+        else {
         {
             const int w = (y.is_local && m->window > 0) ? m->window : 0, st = (w > 0 && pos - w + 1 > 0) ? pos - w + 1 : 0;
             const int tiles = ((pos + rows - 1) >> 5) - (st >> 5) + 1;
@@ -2209,6 +2253,7 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
         else { b[KC_GATEUP] += 2.0 * m->E * y.nff * q; b[KC_DOWN] += (double)y.nff * m->E * q; }
         if (m->ple && !y.winp_f && use_ple_tail(m, rows)) b[KC_TAIL] += 2.0 * m->E * m->ple * q;
         else if (m->ple) { const double pq = y.winp_f ? 4.0 : q; b[KC_PLEGATE] += (double)m->E * m->ple * pq; b[KC_PLEPROJ] += (double)m->ple * m->E * pq; }
+        }
         const int window = (y.is_local && m->window > 0) ? m->window : 0;
         const int last = pos + rows - 1, start = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
         b[KC_ATTN] += 2.0 * (last - start + 1) * y.kd * 2.0;          // K and V rows, f16
