@@ -236,7 +236,7 @@ struct lg_hip_model {
     // the per-layer-input block and the next row work as one launch on one XCD (lg_xtail.h)
     int xcd_tail = 1;                        // option: 0 off, 1 for blocks that do not fold the row work into q/k/v, 2 for every verify block
     XtailSync *tsync = nullptr;
-    float *tgf = nullptr;                    // [LG_HIP_MAX_ROWS][ple] gated values of lg_k_ple_tail_s
+    uint2 *tgf = nullptr, *tpr = nullptr;    // [LG_HIP_MAX_ROWS][ple] and [LG_HIP_MAX_ROWS][E] its gated values and projections, tagged
     NarrowSync *nsync = nullptr;             // hand-over state of lg_k_narrow (models it serves: narrow_shape)
     RgSync *rgsync = nullptr;                // flags and epoch base of lg_k_rows_geglu
     unsigned long long *tstamps = nullptr;   // [LG_XTAIL_UNITS][8] phase stamps of the last such launch (option xcd_tail_stamps)
@@ -769,7 +769,11 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
     if (m->ple && dev_alloc(m, &m->eq, qb(E) + (size_t)12 * E)) return -7;
     if (!m->target) {                        // hand-over state of the one-XCD kernels (lg_xtail.h)
         if (dev_alloc(m, &m->tsync, (size_t)1) || dev_alloc(m, &m->tstamps, (size_t)2 * LG_XTAIL_UNITS * 8) ||
-            dev_alloc(m, &m->tgf, (size_t)LG_HIP_MAX_ROWS * (m->ple > 0 ? m->ple : 1))) return -7;
+            dev_alloc(m, &m->tgf, (size_t)LG_HIP_MAX_ROWS * (m->ple > 0 ? m->ple : 1)) || dev_alloc(m, &m->tpr, (size_t)LG_HIP_MAX_ROWS * (m->ple > 0 ? E : 1))) return -7;
+        if (m->ple > 0) {                    // (no tag of any launch)
+            HIP_TRY(hipMemset(m->tgf, 0, (size_t)LG_HIP_MAX_ROWS * m->ple * 8));
+            HIP_TRY(hipMemset(m->tpr, 0, (size_t)LG_HIP_MAX_ROWS * E * 8));
+        }
         HIP_TRY(hipMemset(m->tstamps, 0, (size_t)2 * LG_XTAIL_UNITS * 8 * 8));
         HIP_TRY(hipMemset(m->tsync, 0, sizeof(XtailSync)));
         if (dev_alloc(m, &m->rgsync, (size_t)1)) return -7;
@@ -1241,25 +1245,29 @@ static void launch_ple_tail(Launcher &lx, const XtailArgs &a) {
         if ((m->tail_spread == 2 || (m->tail_spread && (M >= 5 || M <= 2))) && a.gf && a.r.g.ple == 256 && G >= 1 && G <= 3) {
             const size_t lds = (size_t)E * 5 / 4 + (size_t)M * a.r.g.ple * 5 / 4;
             const dim3 grid(LG_XCDS * W);
-            static int fits[4] = { 0, 0, 0, 0 };              // per G: 0 unknown, 1 yes, -1 no (asked once, outside any capture)
-            if (!fits[G]) {
-                int per_cu = 0;
-                hipError_t e = hipErrorInvalidValue;
-                switch (G) {
-                    case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail_s<M, 1>, 512, lds); break;
-                    case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail_s<M, 2>, 512, lds); break;
-                    case 3: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail_s<M, 3>, 512, lds); break;
+            static int fits[2][4] = {};                       // per tiles of a gate row group (10, 16) and G: 0 unknown, 1 yes, -1 no (asked once, outside any capture)
+            auto launch = [&](auto nit_) {
+                constexpr int NIT = decltype(nit_)::value;
+                int &ok = fits[NIT == 10][G];
+                if (!ok) {
+                    int per_cu = 0;
+                    hipError_t e = hipErrorInvalidValue;
+                    switch (G) {
+                        case 1: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail_s<M, 1, NIT>, 512, lds); break;
+                        case 2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail_s<M, 2, NIT>, 512, lds); break;
+                        case 3: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lg_k_ple_tail_s<M, 3, NIT>, 512, lds); break;
+                    }
+                    ok = (e == hipSuccess && per_cu * LG_XCD_WGS >= W) ? 1 : -1;
                 }
-                fits[G] = (e == hipSuccess && per_cu * LG_XCD_WGS >= W) ? 1 : -1;
-            }
-            if (fits[G] > 0) {
+                if (ok < 0) return false;
                 switch (G) {
-                    case 1: LAUNCH(KC_TAIL, (lg_k_ple_tail_s<M, 1>), grid, dim3(512), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
-                    case 2: LAUNCH(KC_TAIL, (lg_k_ple_tail_s<M, 2>), grid, dim3(512), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
-                    case 3: LAUNCH(KC_TAIL, (lg_k_ple_tail_s<M, 3>), grid, dim3(512), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
+                    case 1: LAUNCH(KC_TAIL, (lg_k_ple_tail_s<M, 1, NIT>), grid, dim3(512), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
+                    case 2: LAUNCH(KC_TAIL, (lg_k_ple_tail_s<M, 2, NIT>), grid, dim3(512), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
+                    case 3: LAUNCH(KC_TAIL, (lg_k_ple_tail_s<M, 3, NIT>), grid, dim3(512), lds, m->ctl, LG_XTAIL_FIELDS(LG_XA, a) 0); break;
                 }
-                return;
-            }
+                return true;
+            };
+            if (E <= 2560 ? launch(std::integral_constant<int, 10>{}) : launch(std::integral_constant<int, 16>{})) return;
         }
     }
     const int U = (a.r.g.ple / 32) * M;
@@ -1613,7 +1621,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 const bool head_m = M >= 4 && m->emb_rb && m->head_mfma;
                 XtailArgs f{};
                 f.r = RowsPleGateArgs{ a, m->x[cur], pend_dout, pend_w, nullptr, m->eps, pend_parts };
-                f.pw = y.wproj; f.pout = m->dout; f.w_post2 = y.post_norm; f.os = y.out_scale;
+                f.pw = y.wproj; f.pout = m->tpr; f.w_post2 = y.post_norm; f.os = y.out_scale;
                 f.w_pre = last ? m->output_norm : m->L[L + 1].attn_norm;
                 f.x_out = m->x[cur ^ 1]; f.h_out = last ? m->hidden_rows : nullptr;
                 f.q = m->hq; f.q_units = last && head_m ? 2 : 0;

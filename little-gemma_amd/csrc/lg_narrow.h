@@ -18,7 +18,6 @@
 // 138 -> 100 us.  Sums, their order and every rounding are the separate kernels', lane for lane.  Tags carry the launch's number and the XCD id; a
 // wait is bounded, and what goes wrong lands in StepCtl.err, as in lg_xtail.h.
 #pragma once
-#include <type_traits>
 #include "lg_xtail.h"
 
 #define LG_NARROW_WGS 32            // one per CU of the XCD
@@ -43,8 +42,6 @@ struct NarrowArgs {
     int            spin_limit;
 };
 
-__device__ __forceinline__ void lg_ld4_wait2(lg_x4u &a, lg_x4u &b) { asm volatile("s_waitcnt vmcnt(0)" : "+v"(a), "+v"(b) :: "memory"); }
-
 template <bool PLE>
 __global__ __launch_bounds__(512, 2) void lg_k_narrow(NarrowArgs a, const StepCtl *ctl) {
     if (blockIdx.x & (LG_XCDS - 1)) return;
@@ -56,8 +53,7 @@ __global__ __launch_bounds__(512, 2) void lg_k_narrow(NarrowArgs a, const StepCt
     const int ge = u + LG_NARROW_WGS * (7 - wave);             // this wavefront's row group of 8 in every matmul (wavefront 0 merges: it has one last)
     const bool eg = ge < (E >> 3), qg = a.wq && ge < (a.qm >> 3);
     const uint32_t gen = a.sync->gen;
-    const int xcc = lg_xcc_id();
-    const uint32_t tag = ((gen + 1) << 4) | (uint32_t)xcc;
+    const uint32_t tag = lg_tag(gen, lg_xcc_id());
 
     // every load that depends on nothing
     struct Tiles { uint4 q[8]; uint32_t s[8]; } to, td;        // output, down
@@ -102,37 +98,17 @@ __global__ __launch_bounds__(512, 2) void lg_k_narrow(NarrowArgs a, const StepCt
     };
     NarrowSync &y = *a.sync;
     int err = 0;
-    // N 16-byte units of two tagged dwords each, loaded until every lane that takes some has the launch's
-    auto take = [&](const void *p, bool on, auto n_) {
-        constexpr int N = decltype(n_)::value;
-        struct { lg_x4u v[N]; } r;
-        for (int spins = 0;; ++spins) {
-            #pragma unroll
-            for (int i = 0; i < N; ++i) r.v[i] = lg_ld4_sc_issue<2>((const uint4 *)p + i);
-            if constexpr (N == 1) lg_ld4_wait1(r.v[0]); else lg_ld4_wait2(r.v[0], r.v[1]);
-            bool there = true, here = true;
-            #pragma unroll
-            for (int i = 0; i < N; ++i) {
-                there = there && ((r.v[i].y ^ tag) >> 4) == 0 && ((r.v[i].w ^ tag) >> 4) == 0;
-                here = here && r.v[i].y == tag && r.v[i].w == tag;
-            }
-            if (__all(there || !on)) { if (on && !here) err |= LG_XFFN_ERR_PLACE; break; }
-            if (spins >= a.spin_limit) { err |= LG_XFFN_ERR_WAIT; break; }
-        }
-        return r;
-    };
-    const std::integral_constant<int, 1> one; const std::integral_constant<int, 2> two;
-    auto put = [&](uint2 *p, float v) { *p = make_uint2(__float_as_uint(v), tag); };
+    auto put = [&](uint2 *p, float v) { lg_put(p, v, tag); };
     // q8 of k values into LDS: two words by each thread of wavefronts 0..3, a block's scale by a lane of wavefront 4
     auto take_q8 = [&](const NarrowQ8 &q, int k) {
         const int nw = k >> 3, ns = k >> 5;                    // 16-byte units of words (at most 256), of scales (at most 64)
         if (wave < 4) {
             const bool on = t < nw;
-            const auto r = take(q.w + 2 * (on ? t : 0), on, one);
+            const LgUnits<1> r = lg_take<1>([&](int) { return (const uint4 *)q.w + (on ? t : 0); }, on, tag, a.spin_limit, err);
             if (on) *(uint2 *)(lq + 8 * t) = make_uint2(r.v[0].x, r.v[0].z);
         } else if (wave == 4) {
             const bool on = lane < ns;
-            const auto r = take(q.s + (on ? lane : 0), on, one);
+            const LgUnits<1> r = lg_take<1>([&](int) { return q.s + (on ? lane : 0); }, on, tag, a.spin_limit, err);
             if (on) ((uint2 *)(lq + k))[lane] = make_uint2(r.v[0].x, r.v[0].z);
         }
         __syncthreads();
@@ -159,8 +135,8 @@ __global__ __launch_bounds__(512, 2) void lg_k_narrow(NarrowArgs a, const StepCt
     auto add_norm = [&](const uint2 *d, float4 w, bool scale, float *r) {
         float4 v = make_float4(0, 0, 0, 0);
         if (rowt) {
-            const auto q = take(d + 4 * t, true, two);
-            v = make_float4(__uint_as_float(q.v[0].x), __uint_as_float(q.v[0].z), __uint_as_float(q.v[1].x), __uint_as_float(q.v[1].z));
+            const LgUnits<2> q = lg_take<2>([&](int i) { return (const uint4 *)(d + 4 * t) + i; }, true, tag, a.spin_limit, err);
+            v = lg_units_float4(q.v[0], q.v[1]);
         }
         const float ss = lg_block_sum256_of512(rowt ? lg_sumsq4(v, 0.0f) : 0.0f, r), sc = 1.0f / sqrtf(ss / (float)E + a.eps);
         xv.x = xv.x + v.x * sc * w.x; xv.y = xv.y + v.y * sc * w.y; xv.z = xv.z + v.z * sc * w.z; xv.w = xv.w + v.w * sc * w.w;
@@ -301,13 +277,7 @@ __global__ __launch_bounds__(512, 2) void lg_k_narrow(NarrowArgs a, const StepCt
             p = lg_sum8(p);
             if (c == 0) put(y.gf + u * 8 + (lane >> 3), lg_gelu_d(p) * iplv);
         }
-        if (wave == 0) {
-            const auto v = take(y.gf + 4 * t, true, two);
-            float d; int sum;
-            const uint32_t packed = lg_quant4_8lanes(make_float4(__uint_as_float(v.v[0].x), __uint_as_float(v.v[0].z), __uint_as_float(v.v[1].x), __uint_as_float(v.v[1].z)), &d, &sum);
-            *(uint32_t *)(lgate + lg_q8_off<1>(256, 0, t >> 2, (t & 3) * 4)) = packed;
-            if ((t & 7) == 0) lg_q8_ds<1>(lgate, 256)[lg_q8_ds_idx<1>(256, 0, t >> 3)] = make_float2(d, __int_as_float(sum));
-        }
+        lg_take_gated<1>(y.gf, lgate, t, 512, tag, a.spin_limit, err);
         __syncthreads();
         if (eg) { const float p = lg_sum8(dot_tile(lgate, 256, 0, pjq, pjs, 0.0f)); if (c == 0) put(y.pr + ge * 8 + (lane >> 3), p); }
         add_norm(y.pr, w4, true, red[4]);

@@ -11,31 +11,37 @@
 // U = ple/32 x M workgroups i of the launch with i % 8 == 0 (the dispatcher deals workgroups to the XCDs in turn: one
 // XCD gets them all; the other 7U workgroups of the launch leave at once):
 //   phase 1 is lg_k_rows_plegate's body for unit (gate block, row); the unit keeps the updated residual row in registers;
-//   hand-over (the M x ple q8 values: 1.6 KB) ;
+//   hand-over (the M x ple gated values, which every unit quantizes) ;
 //   phase 2: the E/8 row groups of the projection dealt over the 4U wavefronts, weights requested at kernel start
 //   (they depend on nothing and are in registers long before the hand-over);
 //   hand-over (the [M][E] f32 outputs) ;
 //   phase 3: lg_k_rows' work for row j, by the units (v, j) of the row's first E/1024 gate blocks: each forms the row's
 //   sums and stores and quantizes the float4s t + 256 v of every lane (the slices of lg_k_rows).
 // Sums and quantization are the ones of the separate kernels, lane for lane: the results are bit-identical.
-// The flags carry the writer's XCD id; a unit that sees another id, or gives up a bounded wait, reports it in
+// A hand-over is one trip: every 8 bytes are a float and the launch's tag, stored together, and the reader loads them until
+// the tag is there (lg_take).  With a flag behind the acknowledged stores and the data loaded behind the flag it was four
+// trips, 1.25 us a hand-over at the E4B shape of 5 rows against 1.0, and 0.45 at one row; the launch 9.2 -> 8.3 us, 7.7 -> 6.5 at one
+// row (there also for the wavefronts without gate rows, which no longer request any), a step 2193 -> 2156 and 1832 -> 1776 us.
+// The tag carries the writer's XCD id; a unit that sees another id, or gives up a bounded wait, reports it in
 // StepCtl.err and goes on, so the kernel always ends and the host refuses the step.
 #pragma once
+#include <type_traits>
 #include "lg_kernels.h"
 #include "lg_xcd.h"
 #include "lg_xffn.h"
 
 #define LG_XTAIL_UNITS 64           // most units of a launch (lane i of a wavefront polls flag i)
 struct XtailSync {
-    uint32_t gen;                   // launches so far (advanced by unit 0 at the end of a launch); epochs 2 gen + 1, + 2
+    uint32_t gen;                   // launches so far (advanced by unit 0 at the end of a launch, when every unit has read it: unit 0 has taken
+                                    // values that all of them tagged); tag (gen + 1, XCD id), flags' epochs 2 gen + 1, + 2
     uint32_t pad[31];
-    uint32_t flags[2][LG_XTAIL_UNITS];
+    uint32_t flags[2][LG_XTAIL_UNITS];      // lg_k_attn_tail
 };
 
 struct XtailArgs {
     RowsPleGateArgs r;              // phase 1 (x_out is not written: the row stays in registers)
     const uint8_t *pw;              // phase 2: tiled projection weights [E][ple]
-    float         *pout;            // [M][E] its output (the XCD's L2 hands it from phase 2 to phase 3)
+    uint2         *pout;            // [M][E] its output, tagged (the XCD's L2 hands it from phase 2 to phase 3)
     const float   *w_post2, *os;    // phase 3: norm weight for pout, layer output scale (or nullptr)
     const float   *w_pre;           // norm weight applied before quantization
     float         *x_out, *h_out;   // [M][E] new residual; normed rows before quantization, or nullptr
@@ -44,15 +50,71 @@ struct XtailArgs {
     XtailSync     *sync;
     int            spin_limit;
     unsigned long long *stamps;     // nullptr, or [LG_XTAIL_UNITS][8] device wall-clock ticks at the phase boundaries of every unit (measurement runs)
-    float         *gf;              // lg_k_ple_tail_s: [M][ple] the gated values as floats (handed from phase 1 to phase 2 through the XCD's L2)
+    uint2         *gf;              // [M][ple] the gated values as tagged floats (handed from phase 1 to phase 2 through the XCD's L2)
 };
 #define LG_XTAIL_FIELDS(X, v) X(const float *, x, r.x, v) X(const float *, dout, r.dout, v) X(const float *, w_post, r.w_post, v) X(const uint8_t *, gw, r.g.w, v) \
     X(int, gk, r.g.k, v) X(int, gple, r.g.ple, v) X(int, dparts, r.dparts, v) X(XtailSync *, sync, sync, v) X(const float *, gipl, r.g.ipl, v) X(int, glayer, r.g.layer, v) \
     X(int, gnl, r.g.n_layer, v) X(int8_t *, gpq, r.g.pq, v) X(const uint8_t *, pw, pw, v) X(const float *, w_post2, w_post2, v) X(const float *, w_pre, w_pre, v) \
-    X(const float *, os, os, v) X(float *, pout, pout, v) X(float *, x_out, x_out, v) X(float *, h_out, h_out, v) X(int8_t *, q, q, v) X(int, q_units, q_units, v) \
-    X(float, eps, r.eps, v) X(int, spin_limit, spin_limit, v) X(unsigned long long *, stamps, stamps, v) X(float *, gf, gf, v)
+    X(const float *, os, os, v) X(uint2 *, pout, pout, v) X(float *, x_out, x_out, v) X(float *, h_out, h_out, v) X(int8_t *, q, q, v) X(int, q_units, q_units, v) \
+    X(float, eps, r.eps, v) X(int, spin_limit, spin_limit, v) X(unsigned long long *, stamps, stamps, v) X(uint2 *, gf, gf, v)
 
 __device__ __forceinline__ void lg_ld4_wait1(lg_x4u &a) { asm volatile("s_waitcnt vmcnt(0)" : "+v"(a) :: "memory"); }
+
+// Tagged hand-over.  A 16-byte unit is two (dword, tag) pairs, each stored by one 8-byte store; addr(i) is the lane's i-th unit.
+// All N are loaded, around the CU's L1, until every lane that is `on` finds the launch's number in all of its tags.
+template <int N> struct LgUnits { lg_x4u v[N]; };
+template <int N>
+__device__ __forceinline__ void lg_units_wait(LgUnits<N> &r) {
+    static_assert(N == 1 || N == 2 || N == 6 || N == 8, "units of a lane");
+    if constexpr (N == 1) asm volatile("s_waitcnt vmcnt(0)" : "+v"(r.v[0]) :: "memory");
+    if constexpr (N == 2) asm volatile("s_waitcnt vmcnt(0)" : "+v"(r.v[0]), "+v"(r.v[1]) :: "memory");
+    if constexpr (N == 6) asm volatile("s_waitcnt vmcnt(0)" : "+v"(r.v[0]), "+v"(r.v[1]), "+v"(r.v[2]), "+v"(r.v[3]), "+v"(r.v[4]), "+v"(r.v[5]) :: "memory");
+    if constexpr (N == 8) asm volatile("s_waitcnt vmcnt(0)" : "+v"(r.v[0]), "+v"(r.v[1]), "+v"(r.v[2]), "+v"(r.v[3]), "+v"(r.v[4]), "+v"(r.v[5]), "+v"(r.v[6]), "+v"(r.v[7]) :: "memory");
+}
+__device__ __forceinline__ uint32_t lg_tag(uint32_t gen, int xcc) { return ((gen + 1) << 4) | (uint32_t)xcc; }
+template <int N, typename A>
+__device__ __forceinline__ LgUnits<N> lg_take(A &&addr, bool on, uint32_t tag, int spin_limit, int &err) {
+    LgUnits<N> r;
+    for (int spins = 0;; ++spins) {
+        #pragma unroll
+        for (int i = 0; i < N; ++i) r.v[i] = lg_ld4_sc_issue<2>(addr(i));
+        lg_units_wait<N>(r);
+        uint32_t diff = 0;                                     // any bit of any tag that is not the launch's
+        #pragma unroll
+        for (int i = 0; i < N; ++i) diff |= (r.v[i].y ^ tag) | (r.v[i].w ^ tag);
+        if (__all(!on || (diff >> 4) == 0)) { if (on && diff) err |= LG_XFFN_ERR_PLACE; break; }
+        if (spins >= spin_limit) { err |= LG_XFFN_ERR_WAIT; break; }
+    }
+    return r;
+}
+__device__ __forceinline__ float4 lg_units_float4(lg_x4u a, lg_x4u b) { return make_float4(__uint_as_float(a.x), __uint_as_float(a.z), __uint_as_float(b.x), __uint_as_float(b.z)); }
+__device__ __forceinline__ void lg_put(uint2 *p, float v, uint32_t tag) { *p = make_uint2(__float_as_uint(v), tag); }
+// [M][256] gated values -> their q8 in LDS ([M][256] int8, then {scale, sum}): a float4 per lane, 8 lanes a block, 64 a row; thread t of nt
+template <int M>
+__device__ __forceinline__ void lg_take_gated(const uint2 *gf, int8_t *lq2, int t, int nt, uint32_t tag, int spin_limit, int &err) {
+    constexpr int PLE = 256;                                   // (the launch is made for ple == 256 only: constant layout arithmetic)
+    for (int i = t; i < M * 64; i += nt) {                     // (whole wavefronts)
+        const LgUnits<2> q = lg_take<2>([&](int k) { return (const uint4 *)(gf + 4 * i) + k; }, true, tag, spin_limit, err);
+        const int r = i >> 6, blk = (i & 63) >> 3, l8 = i & 7;
+        float d; int sum;
+        const uint32_t packed = lg_quant4_8lanes(lg_units_float4(q.v[0], q.v[1]), &d, &sum);
+        const ActLayout lay = lg_act_layout(PLE);
+        *(uint32_t *)(lq2 + (size_t)r * PLE + lg_act_unit(lay, blk * 2 + (l8 >> 2)) * 16 + (l8 & 3) * 4) = packed;
+        if (l8 == 0) lg_q8_ds<M>(lq2, PLE)[(size_t)r * (PLE >> 5) + lg_act_block(lay, blk)] = make_float2(d, __int_as_float(sum));
+    }
+}
+// a lane's float4s t + 256 v of a tagged row of nq float4s
+template <int N>
+__device__ __forceinline__ void lg_take_row_n(float4 (&dv)[LG_ROWV], const uint2 *row, int t, int nq, uint32_t tag, int spin_limit, int &err) {
+    const LgUnits<2 * N> q = lg_take<2 * N>([&](int i) { const int v = t + 256 * (i >> 1); return (const uint4 *)(row + 4 * (v < nq ? v : nq - 1)) + (i & 1); }, true, tag, spin_limit, err);
+    #pragma unroll
+    for (int v = 0; v < LG_ROWV; ++v) dv[v] = lg_units_float4(q.v[v < N ? 2 * v : 0], q.v[v < N ? 2 * v + 1 : 1]);
+}
+__device__ __forceinline__ void lg_take_row(float4 (&dv)[LG_ROWV], const uint2 *row, int t, int nq, uint32_t tag, int spin_limit, int &err) {
+    if (nq <= 256) lg_take_row_n<1>(dv, row, t, nq, tag, spin_limit, err);
+    else if (nq <= 768) lg_take_row_n<3>(dv, row, t, nq, tag, spin_limit, err);
+    else lg_take_row_n<4>(dv, row, t, nq, tag, spin_limit, err);
+}
 
 // G: most projection row groups per wavefront (E/8 groups over 4U wavefronts).
 template <int M, int G>
@@ -67,7 +129,8 @@ __global__ __launch_bounds__(LG_WG) void lg_k_ple_tail(StepCtl *ctl, LG_XTAIL_FI
     const uint32_t gen = a.sync->gen;
     auto stamp = [&](int i) { if (a.stamps && t == 0) a.stamps[(size_t)u * 8 + i] = wall_clock64(); };
     stamp(0);
-    const int xcc = lg_xcc_id();
+    const uint32_t tag = lg_tag(gen, lg_xcc_id());
+    int err = 0;
     // ---- phase 1, with this kernel's later loads requested behind its own ----
     const int groups = E >> 3, waves = 4 * U, gw = u * 4 + wave;
     const uint8_t *wgp[G];
@@ -75,7 +138,7 @@ __global__ __launch_bounds__(LG_WG) void lg_k_ple_tail(StepCtl *ctl, LG_XTAIL_FI
     bool live[G];
     #pragma unroll
     for (int g = 0; g < G; ++g) {
-        const int gi = gw + g * waves;
+        const int gi = g ? g * waves + wave * (U) + u : gw;         // (what does not come out even is spread over the units)
         live[g] = gi < groups;
         const int gc = live[g] ? gi : groups - 1;
         wgp[g] = a.pw + (size_t)gc * LG_TILE;                  // K = ple = 256: one tile per group of 8 rows
@@ -91,26 +154,12 @@ __global__ __launch_bounds__(LG_WG) void lg_k_ple_tail(StepCtl *ctl, LG_XTAIL_FI
         #pragma unroll
         for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) { wpost2[v] = w2[t + 256 * v]; wpre[v] = w3[t + 256 * v]; }
         if (a.os) osv = a.os[0];
-    }, [&](const float *v) { lg_plegate_q8<M>(a.r.g, gb, j, v); });
+    }, [&](const float *v) { if (t < 32) lg_put(a.gf + (size_t)j * ple + gb * 32 + t, v[t], tag); });
     stamp(1);
-    // ---- hand-over: every unit's 32 gated values of its row are in the XCD's L2 ----
+    // ---- hand-over: every unit's 32 gated values of its row ----
     int8_t *lq2 = (int8_t *)(smem + (size_t)E * 5 / 4);       // [M][ple] int8, [M][ple/32] {scale, sum}
-    lg_wait_vm();
-    __syncthreads();
-    if (wave == 0) {
-        const int err = lg_xcd_arrive_wait(a.sync->flags[0], u, true, U, 2 * gen + 1, xcc, a.spin_limit);
-        if (err && lane == 0) atomicOr(&ctl->err, err);
-    }
-    __syncthreads();
+    lg_take_gated<M>(a.gf, lq2, t, LG_WG, tag, a.spin_limit, err);
     stamp(2);
-    {
-        const int n16 = M * ple * 5 / 64;                      // 16-byte units of the q8 rows
-        for (int i = t; i < n16; i += LG_WG) {
-            lg_x4u v = lg_ld4_sc_issue<2>(a.r.g.pq + (size_t)i * 16);
-            lg_ld4_wait1(v);
-            *(lg_x4u *)(lq2 + (size_t)i * 16) = v;
-        }
-    }
     __syncthreads();
     stamp(3);
     // ---- phase 2: this wavefront's row groups of the projection ----
@@ -120,39 +169,19 @@ __global__ __launch_bounds__(LG_WG) void lg_k_ple_tail(StepCtl *ctl, LG_XTAIL_FI
         const int c = lane & 7;
         if (c < M) {
             #pragma unroll
-            for (int g = 0; g < G; ++g) if (live[g]) a.pout[(size_t)c * E + row[g]] = lg_pick<M>(acc[g], c);
+            for (int g = 0; g < G; ++g) if (live[g]) lg_put(a.pout + (size_t)c * E + row[g], lg_pick<M>(acc[g], c), tag);
         }
     }
-    // ---- hand-over: the projection's [M][E] is in the XCD's L2 ----
     const int slices = (E + 1023) >> 10;
     stamp(4);
-    lg_wait_vm();
-    __syncthreads();
-    if (gb >= slices) {                                        // this unit has no share of the row work: it arrives and leaves
-        if (t == 0) lg_st_sc<0>(a.sync->flags[1] + u, ((2 * gen + 2) << 4) | (uint32_t)xcc);
-        return;
-    }
-    if (wave == 0) {
-        const int err = lg_xcd_arrive_wait(a.sync->flags[1], u, true, U, 2 * gen + 2, xcc, a.spin_limit);
-        if (err && lane == 0) atomicOr(&ctl->err, err);
-    }
-    __syncthreads();
-    stamp(5);
-    // ---- phase 3: the row work of row j, this unit storing and quantizing slice gb ----
+    if (err) atomicOr(&ctl->err, err);
+    if (gb >= slices) return;                                  // this unit has no share of the row work
+    // ---- hand-over: the projection's row j; phase 3: the row work, this unit storing and quantizing slice gb ----
     float4 dv[LG_ROWV];
-    {
-        lg_x4u d0 = lg_x4u{ 0, 0, 0, 0 }, d1 = d0, d2 = d0, d3 = d0;
-        const float *pr = a.pout + (size_t)j * E;
-        const int last = nq - 1;
-        d0 = lg_ld4_sc_issue<2>(pr + 4 * min(t, last));
-        d1 = lg_ld4_sc_issue<2>(pr + 4 * min(t + 256, last));
-        d2 = lg_ld4_sc_issue<2>(pr + 4 * min(t + 512, last));
-        d3 = lg_ld4_sc_issue<2>(pr + 4 * min(t + 768, last));
-        lg_ld4_wait(d0, d1, d2, d3);
-        const lg_x4u d[4] = { d0, d1, d2, d3 };
-        #pragma unroll
-        for (int v = 0; v < LG_ROWV; ++v) dv[v] = make_float4(__uint_as_float(d[v].x), __uint_as_float(d[v].y), __uint_as_float(d[v].z), __uint_as_float(d[v].w));
-    }
+    err = 0;
+    lg_take_row(dv, a.pout + (size_t)j * E, t, nq, tag, a.spin_limit, err);
+    if (err) atomicOr(&ctl->err, err);
+    stamp(5);
     stamp(6);
     {
         float ss = 0.0f;
@@ -232,7 +261,7 @@ __device__ __forceinline__ float lg_block_sum256_of512(float v, float *scratch8)
 //   hand-over; every unit quantizes the M x ple floats into its LDS (the blocks, scales and sums of lg_k_rows_plegate);
 //   phase 2 and 3 as in lg_k_ple_tail, the projection's row groups dealt over 8 W wavefronts, the row work of row j by
 //   its parts 0 .. E/1024 - 1 (wavefronts 0..3).
-template <int M, int G>
+template <int M, int G, int NIT>
 __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FIELDS(LG_XP, _) int p_end_) {
     if (blockIdx.x & (LG_XCDS - 1)) return;
     XtailArgs a; LG_XTAIL_FIELDS(LG_XI, a)
@@ -250,7 +279,8 @@ __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FI
     const uint32_t gen = a.sync->gen;
     auto stamp = [&](int i) { if (a.stamps && t == 0) a.stamps[(size_t)u * 8 + i] = wall_clock64(); };
     stamp(0);
-    const int xcc = lg_xcc_id();
+    const uint32_t tag = lg_tag(gen, lg_xcc_id());
+    int err = 0;
     int8_t *lq = (int8_t *)smem;                               // the row: [E] int8, then [E/32] {scale, sum}
     float2 *lds = (float2 *)(smem + (size_t)E);
     int8_t *lq2 = (int8_t *)(smem + (size_t)E * 5 / 4);        // [M][ple] int8, [M][ple/32] {scale, sum}
@@ -280,24 +310,26 @@ __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FI
             }
         }
     }
-    uint4 wq[LG_MAXV]; uint32_t wsc[LG_MAXV];
-    {
+    uint4 wq[NIT]; uint32_t wsc[NIT];
+    float iplv = 0.0f;                                         // of this lane's gate column
+    if (gatew) {                                               // (a launch of one row has one such wavefront a unit: requested by all eight, the CU's
+                                                               // address unit is busy with them for a microsecond)
         const uint8_t *wg0 = a.r.g.w + (size_t)gg * nit * LG_TILE;
         #pragma unroll
-        for (int k = 0; k < LG_MAXV; ++k) {
+        for (int k = 0; k < NIT; ++k) {
             const int it = k < nit ? k : nit - 1;
             wq[k] = *(const uint4 *)(wg0 + (size_t)it * LG_TILE + lane * 16);
             wsc[k] = *(const uint16_t *)(wg0 + (size_t)it * LG_TILE + 1024 + lane * 2);
         }
+        iplv = a.r.g.ipl[(size_t)j * a.r.g.n_layer * ple + (size_t)a.r.g.layer * ple + gg * 8 + (lane >> 3)];
     }
-    const float iplv = a.r.g.ipl[(size_t)j * a.r.g.n_layer * ple + (size_t)a.r.g.layer * ple + gg * 8 + (lane >> 3)];   // of this lane's gate column
     const int groups = E >> 3, waves = 8 * W, gw = u * 8 + wave;
     const uint8_t *wgp[G];
     int row[G];
     bool live[G];
     #pragma unroll
     for (int g = 0; g < G; ++g) {
-        const int gi = gw + g * waves;
+        const int gi = g ? g * waves + wave * (W) + u : gw;         // (what does not come out even is spread over the units)
         live[g] = gi < groups;
         const int gc = live[g] ? gi : groups - 1;
         wgp[g] = a.pw + (size_t)gc * LG_TILE;                  // K = ple = 256: one tile per group of 8 rows
@@ -345,7 +377,7 @@ __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FI
         const int c = lane & 7;
         float pr = 0.0f;
         #pragma unroll
-        for (int k = 0; k < LG_MAXV; ++k) {
+        for (int k = 0; k < NIT; ++k) {
             if (k < nit) {                                     // (a guard, not a break: the arrays stay in registers)
                 const float2 ds = lds[k * 8 + c];
                 const int8_t *au = lq + (size_t)(k * 16 + c) * 16;
@@ -354,29 +386,12 @@ __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FI
             }
         }
         pr = lg_sum_seg<8>(pr);
-        if (c == 0) a.gf[(size_t)j * ple + gg * 8 + (lane >> 3)] = lg_gelu_d(pr) * iplv;
+        if (c == 0) lg_put(a.gf + (size_t)j * ple + gg * 8 + (lane >> 3), lg_gelu_d(pr) * iplv, tag);
     }
     stamp(1);
-    // ---- hand-over: every part's gated values of its row are in the XCD's L2 ----
-    lg_wait_vm();
-    __syncthreads();
-    if (wave == 0) {
-        const int err = lg_xcd_arrive_wait(a.sync->flags[0], u, true, W, 2 * gen + 1, xcc, a.spin_limit);
-        if (err && lane == 0) atomicOr(&ctl->err, err);
-    }
-    __syncthreads();
+    // ---- hand-over: every part's gated values; wavefront r quantizes row r ----
+    lg_take_gated<M>(a.gf, lq2, t, 512, tag, a.spin_limit, err);
     stamp(2);
-    if (wave < M) {                                            // wavefront r = row r: a float4 per lane, 8 lanes a block of 32
-        constexpr int PLE = 256;                               // (the launch is made for ple == 256 only: constant layout arithmetic)
-        lg_x4u v = lg_ld4_sc_issue<2>(a.gf + 4 * t);
-        lg_ld4_wait1(v);
-        const int r = wave, blk = lane >> 3, l8 = lane & 7;
-        float d; int sum;
-        const uint32_t packed = lg_quant4_8lanes(make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)), &d, &sum);
-        const ActLayout lay = lg_act_layout(PLE);
-        *(uint32_t *)(lq2 + (size_t)r * PLE + lg_act_unit(lay, blk * 2 + (l8 >> 2)) * 16 + (l8 & 3) * 4) = packed;
-        if (l8 == 0) lg_q8_ds<M>(lq2, PLE)[(size_t)r * (PLE >> 5) + lg_act_block(lay, blk)] = make_float2(d, __int_as_float(sum));
-    }
     __syncthreads();
     stamp(3);
     // ---- phase 2: this wavefront's row groups of the projection ----
@@ -386,39 +401,19 @@ __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FI
         const int c = lane & 7;
         if (c < M) {
             #pragma unroll
-            for (int g = 0; g < G; ++g) if (live[g]) a.pout[(size_t)c * E + row[g]] = lg_pick<M>(acc[g], c);
+            for (int g = 0; g < G; ++g) if (live[g]) lg_put(a.pout + (size_t)c * E + row[g], lg_pick<M>(acc[g], c), tag);
         }
     }
-    // ---- hand-over: the projection's [M][E] is in the XCD's L2 ----
     const int slices = (E + 1023) >> 10;
     stamp(4);
-    lg_wait_vm();
-    __syncthreads();
-    if (p >= slices) {                                         // this unit has no share of the row work: it arrives and leaves
-        if (t == 0) lg_st_sc<0>(a.sync->flags[1] + u, ((2 * gen + 2) << 4) | (uint32_t)xcc);
-        return;
-    }
-    if (wave == 0) {
-        const int err = lg_xcd_arrive_wait(a.sync->flags[1], u, true, W, 2 * gen + 2, xcc, a.spin_limit);
-        if (err && lane == 0) atomicOr(&ctl->err, err);
-    }
-    __syncthreads();
+    if (err) atomicOr(&ctl->err, err);
+    if (p >= slices) return;                                   // this unit has no share of the row work
+    // ---- hand-over: the projection's row j; phase 3: the row work, this unit storing and quantizing slice p (wavefronts 0..3;
+    //      the others only take part in the workgroup's barriers) ----
+    err = 0;
+    if (rowt) lg_take_row(dv, a.pout + (size_t)j * E, t, nq, tag, a.spin_limit, err);
+    if (err) atomicOr(&ctl->err, err);
     stamp(5);
-    // ---- phase 3: the row work of row j, this unit storing and quantizing slice p (wavefronts 0..3; the others only
-    //      take part in the workgroup's barriers) ----
-    if (rowt) {
-        lg_x4u d0 = lg_x4u{ 0, 0, 0, 0 }, d1 = d0, d2 = d0, d3 = d0;
-        const float *pr = a.pout + (size_t)j * E;
-        const int last = nq - 1;
-        d0 = lg_ld4_sc_issue<2>(pr + 4 * min(t, last));
-        d1 = lg_ld4_sc_issue<2>(pr + 4 * min(t + 256, last));
-        d2 = lg_ld4_sc_issue<2>(pr + 4 * min(t + 512, last));
-        d3 = lg_ld4_sc_issue<2>(pr + 4 * min(t + 768, last));
-        lg_ld4_wait(d0, d1, d2, d3);
-        const lg_x4u d[4] = { d0, d1, d2, d3 };
-        #pragma unroll
-        for (int v = 0; v < LG_ROWV; ++v) dv[v] = make_float4(__uint_as_float(d[v].x), __uint_as_float(d[v].y), __uint_as_float(d[v].z), __uint_as_float(d[v].w));
-    }
     stamp(6);
     {
         float ss = 0.0f;
