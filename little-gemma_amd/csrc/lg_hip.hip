@@ -28,6 +28,7 @@
 #include "lg_xtail.h"
 #include "lg_xrg.h"
 #include "lg_narrow.h"
+#include "lg_aout.h"
 
 static_assert(LG_HIP_MAX_ROWS == LG_HIP_MAX_ROWS_DEV, "row limits must agree");
 #define LG_FUSE_ROWS_MAX 2         // widest block whose q/k/v matmul does the preceding row work itself
@@ -219,7 +220,7 @@ struct lg_hip_model {
     int last_rows = 0, last_adv = 0;
     float *lstage = nullptr;           // pinned: two rows of logits on their way to a caller (lg_hip_get_logits), row j in half j % 2
     int lread = -1, lcoming = -1;      // the row of the latest step read last, and the one whose copy has been started
-    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1;
+    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1, attn_out = 1;
     // the feed-forward half of a layer as one XCD-partitioned launch (lg_xffn.h): built when the shape and the chip fit
     int xcd_ffn = 0;                         // option: use it (verify blocks of 4..8 rows)
     int down_m = 1;                          // option: ffn_down of 4..8-row blocks on the matrix cores (lg_k_down_m): 1 = the row group's four workgroups add
@@ -237,6 +238,7 @@ struct lg_hip_model {
     int xcd_tail = 1;                        // option: 0 off, 1 for blocks that do not fold the row work into q/k/v, 2 for every verify block
     XtailSync *tsync = nullptr;
     uint2 *tgf = nullptr, *tpr = nullptr;    // [LG_HIP_MAX_ROWS][ple] and [LG_HIP_MAX_ROWS][E] its gated values and projections, tagged
+    AttnOutSync *aosync = nullptr;           // hand-over state of lg_k_attn_out (models it serves)
     NarrowSync *nsync = nullptr;             // hand-over state of lg_k_narrow (models it serves: narrow_shape)
     RgSync *rgsync = nullptr;                // flags and epoch base of lg_k_rows_geglu
     unsigned long long *tstamps = nullptr;   // [LG_XTAIL_UNITS][8] phase stamps of the last such launch (option xcd_tail_stamps)
@@ -543,6 +545,11 @@ static bool narrow_shape(const lg_hip_model *m) {
     return true;
 }
 
+// Layers that lg_k_attn_out serves.  (Rows of up to 512 values: lg_k_narrow, or launches as short as this one.)
+static bool attn_out_shape(const lg_hip_model *m, const Layer &y) {
+    return m->E > LG_NARROW_E && m->E <= LG_AOUT_E && m->E % 256 == 0 && y.qd == LG_AOUT_K && y.hd % 64 == 0 && y.wo;
+}
+
 static const float *rope_table(lg_hip_model *m, int is_local, int hd, int *rc) {
     auto key = std::make_pair(is_local, hd);
     auto it = m->rope_tabs.find(key);
@@ -784,6 +791,13 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
     if (narrow_shape(m)) {
         if (dev_alloc(m, &m->nsync, (size_t)1)) return -7;
         HIP_TRY(hipMemset(m->nsync, 0, sizeof(NarrowSync)));
+    } else if (!m->target && cu_count() == LG_XCDS * LG_XCD_WGS) {
+        bool any = false;
+        for (const Layer &y : m->L) any = any || attn_out_shape(m, y);
+        if (any) {
+            if (dev_alloc(m, &m->aosync, (size_t)1)) return -7;
+            HIP_TRY(hipMemset(m->aosync, 0, sizeof(AttnOutSync)));
+        }
     }
     if (getenv("LG_HIP_XCD_ATTN_TAIL")) m->xcd_attn_tail = atoi(getenv("LG_HIP_XCD_ATTN_TAIL"));
     if (getenv("LG_HIP_DOWN_M")) m->down_m = atoi(getenv("LG_HIP_DOWN_M"));
@@ -1217,6 +1231,17 @@ static void launch_down_m(Launcher &lx, const DownMArgs &a) {
         else lx.rc = fail(-2, "down_m: no instantiation for this shape");
     }
 }
+// tiles a block of `rows` rows can touch (a sliding layer needs only its window's, not the cache's)
+static int step_tiles(const lg_hip_model *m, const lg_hip_kv *kv, const Layer &y, int rows, int pos_off) {
+    const int window = (y.is_local && m->window > 0) ? m->window + pos_off : 0;
+    if (window <= 0) return kv->tiles_max;
+    const int t = (window + rows - 1 + 31) / 32 + 1;
+    return t < kv->tiles_max ? t : kv->tiles_max;
+}
+// (tiles: what one wavefront holds; more of them, a global layer in a cache of more than 1280 positions, are merged by more of the chip)
+static bool use_attn_out(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
+    return rows <= LG_AOUT_ROWS && m->attn_out && m->aosync && attn_out_shape(m, y) && tiles <= LG_AOUT_TILES;
+}
 static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
     if (!y.wo_ch || !m->tsync || m->xcd_attn_tail <= 0 || (m->xcd_attn_tail == 1 && rows < 3)) return false;
     const int slices = (m->E + 1023) / 1024;
@@ -1416,13 +1441,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
     };
     // tiles a block of layer L can touch (a sliding layer needs only its window's, not the cache's), and whether the
     // layer takes the kernel that serves all rows of a block per (tile, kv head)
-    auto layer_tiles = [&](int L) {
-        const Layer &y = m->L[L];
-        const int window = (y.is_local && m->window > 0) ? m->window + pos_off : 0;
-        int tiles = kv->tiles_max;
-        if (window > 0) { const int t = (window + M - 1 + 31) / 32 + 1; if (t < tiles) tiles = t; }
-        return tiles;
-    };
+    auto layer_tiles = [&](int L) { return step_tiles(m, kv, m->L[L], M, pos_off); };
     auto rows_shared = [&](int L) {
         const Layer &y = m->L[L];
         return pos_off == 0 && m->attn_rows && attention_rows_shared(M, layer_tiles(L), y.nkv, y.hd, kv->seq[y.src], 0);
@@ -1524,6 +1543,17 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 launch_attn_tail<M>(lx, f);
                 cur ^= 1;
                 pend_dout = pend_w = pend_os = nullptr; pend_parts = 1;
+                merged_o = true; ffn_rows_done = true;
+            } else
+            if (!merged_o && pos_off == 0 && have_x && use_attn_out(m, y, M, tiles)) {
+                if constexpr (M <= LG_AOUT_ROWS) {
+                    AttnOutArgs f{};
+                    f.g = g; f.wo = y.wo; f.x = m->x[cur]; f.w_post = y.post_attn; f.w_pre = y.ffn_norm; f.x_out = m->x[cur ^ 1];
+                    f.q = m->hq; f.E = E; f.tiles = tiles; f.eps = m->eps; f.sync = m->aosync; f.spin_limit = 1 << 16;
+                    f.stamps = m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr;
+                    LAUNCH(KC_ATAIL, lg_k_attn_out<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(64 * (LG_AOUT_G + M)), 0, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
+                }
+                cur ^= 1;
                 merged_o = true; ffn_rows_done = true;
             } else
             if (merged_o) {
@@ -1854,7 +1884,7 @@ static GraphKey graph_key(const lg_hip_model *m, const lg_hip_kv *kv, int rows, 
     put(what, 2); put(rows, 4); put(m->store_logits != 0, 1); put(m->draft_chain, 1); put(m->fuse_rows, 1); put(m->attn_rows, 1); put(m->attn_rows_fq, 1);
     put(m->head_mfma, 1); put(m->down_kq, 1); put(m->xcd_ffn, 1); put(m->fork_ple, 1); put(m->rows_geglu, 1); put(m->tail_stamps != 0, 1);
     put(m->tail_spread == 1 ? 1 : m->tail_spread ? 2 : 0, 2); put(m->xcd_tail, 2); put(m->down_m, 2); put(m->xcd_attn_tail, 2); put(m->merge_o, 2);
-    put(m->xffn_delay, 10); put(m->narrow, 1);
+    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1);
     return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices };
 }
 
@@ -1914,6 +1944,7 @@ extern "C" int lg_hip_set_option(lg_hip_model *m, const char *name, int value) {
     else if (!strcmp(name, "xcd_tail_spread")) m->tail_spread = value;
     else if (!strcmp(name, "rows_geglu")) m->rows_geglu = value != 0;
     else if (!strcmp(name, "narrow")) m->narrow = value != 0;
+    else if (!strcmp(name, "attn_out")) m->attn_out = value != 0;
     else if (!strcmp(name, "down_kq")) m->down_kq = value != 0;
     else if (!strcmp(name, "xcd_ffn")) m->xcd_ffn = value != 0 && m->xffn_built;
     else if (!strcmp(name, "fork_ple")) m->fork_ple = value != 0;
@@ -2255,7 +2286,7 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
         {
             const int w = (y.is_local && m->window > 0) ? m->window : 0, st = (w > 0 && pos - w + 1 > 0) ? pos - w + 1 : 0;
             const int tiles = ((pos + rows - 1) >> 5) - (st >> 5) + 1;
-            b[use_attn_tail(m, y, rows, tiles) ? KC_ATAIL : use_merge_o(m, y, rows, tiles) ? KC_MERGE : KC_O] += (double)y.qd * m->E * q;
+            b[use_attn_tail(m, y, rows, tiles) ? KC_ATAIL : use_merge_o(m, y, rows, tiles) ? KC_MERGE : use_attn_out(m, y, rows, step_tiles(m, kv, y, rows, 0)) ? KC_ATAIL : KC_O] += (double)y.qd * m->E * q;
         }
         if (m->xffn_built && m->xcd_ffn && rows >= 4) b[KC_FFN] += 3.0 * m->E * y.nff * q;
         else { b[KC_GATEUP] += 2.0 * m->E * y.nff * q; b[KC_DOWN] += (double)y.nff * m->E * q; }
@@ -2268,7 +2299,6 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
     }
     b[KC_HEAD] = (double)m->E * m->n_vocab * q;
     b[KC_ROWS] = 0;
-    (void)kv;
 }
 
 extern "C" int lg_hip_profile_step(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int rows, int pos, int repeats,

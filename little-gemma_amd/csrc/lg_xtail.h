@@ -65,9 +65,10 @@ __device__ __forceinline__ void lg_ld4_wait1(lg_x4u &a) { asm volatile("s_waitcn
 template <int N> struct LgUnits { lg_x4u v[N]; };
 template <int N>
 __device__ __forceinline__ void lg_units_wait(LgUnits<N> &r) {
-    static_assert(N == 1 || N == 2 || N == 6 || N == 8, "units of a lane");
+    static_assert(N == 1 || N == 2 || N == 5 || N == 6 || N == 8, "units of a lane");
     if constexpr (N == 1) asm volatile("s_waitcnt vmcnt(0)" : "+v"(r.v[0]) :: "memory");
     if constexpr (N == 2) asm volatile("s_waitcnt vmcnt(0)" : "+v"(r.v[0]), "+v"(r.v[1]) :: "memory");
+    if constexpr (N == 5) asm volatile("s_waitcnt vmcnt(0)" : "+v"(r.v[0]), "+v"(r.v[1]), "+v"(r.v[2]), "+v"(r.v[3]), "+v"(r.v[4]) :: "memory");
     if constexpr (N == 6) asm volatile("s_waitcnt vmcnt(0)" : "+v"(r.v[0]), "+v"(r.v[1]), "+v"(r.v[2]), "+v"(r.v[3]), "+v"(r.v[4]), "+v"(r.v[5]) :: "memory");
     if constexpr (N == 8) asm volatile("s_waitcnt vmcnt(0)" : "+v"(r.v[0]), "+v"(r.v[1]), "+v"(r.v[2]), "+v"(r.v[3]), "+v"(r.v[4]), "+v"(r.v[5]), "+v"(r.v[6]), "+v"(r.v[7]) :: "memory");
 }
