@@ -1,30 +1,37 @@
-// lg_aout.h — attention merge, output projection and the row work ahead of gate/up as ONE launch on ONE XCD (blocks of 1..3 rows).
+// lg_aout.h — attention merge, output projection and the row work ahead of gate/up as ONE launch on ONE XCD (sliding layers).
 //
 // As separate launches these are three dependent steps of 8 to 320 workgroups, 4 us each from the predecessor's end, for 3 MB of weights.
 // The 32 CUs of one XCD pull those in 2 to 3 us, and hand over among themselves for less than a launch (lg_xcd.h).  Unit u of the 32:
-//   merge       64 dims of each row, a wavefront a row: what it loads comes first, the tiles' partials in registers   (lg_k_attn_merge)
+//   merge       64 dims of each row, a wavefront a row (two from 5 rows on: with more wavefronts than twelve the registers no longer hold the projection): what it loads comes first, the tiles' partials in
+//               registers   (lg_k_attn_merge)
 //   hand-over   the q8 of the rows, tagged (lg_take), to every unit's LDS: by the merging wavefronts
-//   projection  ten row groups of 8, a wavefront each, their weights in registers since the partials were requested   (lg_k_mm)
+//   projection  up to 3 rows (lg_k_attn_out): ten row groups of 8 on v_dot4, a wavefront each   (lg_k_mm)
+//               4 to 8 rows (lg_k_attn_out_m): up to three blocks of 32 rows on the matrix cores, a K segment to a wavefront   (lg_k_attn_tail)
+//               either way with the weights in registers, requested right behind the partials
 //   hand-over   the f32 rows, tagged, to the first rows x E/1024 units, which do the row work of lg_k_rows
 // Sums, their order and every rounding are the separate kernels', lane for lane.
-// Bound by the CU's one memory path: by the stamps of one row the q8 leaves at 2.1 us and is in every LDS at 3.6, when the 92 KB of
-// weights are through as well; rows at 5.6, end at 6.7.  E4B shape, the 35 sliding layers of 42: a step of one row 1776 -> 1703 us,
-// two 1880 -> 1829, three 1972 -> 1962; four 2070 -> 2080, five 2160 -> 2196, eight 2302 -> 2575 (the projection on v_dot4 by an eighth of the
-// chip: those keep the separate kernels).  With 4096 inputs, 276 KB a CU at rows of 3840, one row lost as well: 12B shape 2481 -> 2728.
-// Weights requested ahead of the partials: 1741 us.  Partials first, but the hand-over taken by the wavefronts that hold weights: 1712.
+// Bound by the CU's one memory path up to the projection, then by LDS (v_dot4) or the vector units (matrix cores).  By the stamps the q8 of
+// one row leaves at 1.9 us and is in every LDS at 3.4, when the 92 KB of weights are through as well; rows at 5.4, end at 6.4; five rows
+// 3.0, 4.8, 7.9 (the projection 2.3) and 8.9.  E4B shape, the 35 sliding layers of 42, a step: one row 1784 -> 1694 us, two 1883 -> 1812,
+// three 1985 -> 1944, four 2061 -> 2007, five 2162 -> 2125, six 2210 -> 2162, eight 2304 -> 2276.
+// v_dot4 at 4, 5, 8 rows: 2080, 2196, 2575 (every row group reads the rows from LDS again).  4096 inputs, 276 KB a CU at rows of 3840: a
+// step of the 12B shape 2481 -> 2728.  Weights requested ahead of the partials: one row 1741.  Partials first, but the hand-over
+// taken by the wavefronts that hold weights: 1712.  Five to eight rows with a wavefront per merge: the projection spills, 2202 at five.
 #pragma once
 #include "lg_narrow.h"
 
 #define LG_AOUT_TILES 40            // most tiles of a row: a wavefront holds them in registers
-#define LG_AOUT_BATCH 20            // ... the first so many requested at once, the others where there are more
+#define LG_AOUT_BATCH 20            // ... the first so many requested at once, the others where there are more; the most of lg_k_attn_out_m
 #define LG_AOUT_K 2048              // input of attn_output (8 tiles of a row group)
 #define LG_AOUT_E 2560              // widest row
 #define LG_AOUT_G (LG_AOUT_E / 8 / LG_XCD_WGS)     // row groups of a unit, a wavefront each
-#define LG_AOUT_ROWS 3              // widest block
-struct AttnOutSync { uint32_t gen, pad[31]; uint2 w[LG_AOUT_ROWS * LG_AOUT_K / 4]; uint4 s[LG_AOUT_ROWS * LG_AOUT_K / 32]; uint2 o[LG_AOUT_ROWS * LG_AOUT_E]; };
+#define LG_AOUT_DOT_ROWS 3          // widest block on v_dot4
+#define LG_AOUT_NV ((LG_AOUT_E + 1023) / 1024)     // float4 of a row per thread of 256
+struct AttnOutSync { uint32_t gen, pad[31]; uint2 w[LG_HIP_MAX_ROWS_DEV * LG_AOUT_K / 4]; uint4 s[LG_HIP_MAX_ROWS_DEV * LG_AOUT_K / 32]; uint2 o[LG_HIP_MAX_ROWS_DEV * LG_AOUT_E]; };
+static_assert(LG_AOUT_K == 64 * LG_XCD_WGS, "a merge of every row per unit");
 struct AttnOutArgs {
     MergeArgs      g;               // (xq, xf are not used)
-    const uint8_t *wo;              // segment tiles
+    const uint8_t *wo;              // segment tiles; lg_k_attn_out_m: the chains of lg_k_attn_tail
     const float   *x, *w_post, *w_pre;
     float         *x_out;
     int8_t        *q;
@@ -40,18 +47,140 @@ struct AttnOutArgs {
     X(float *, x_out, x_out, v) X(int8_t *, q, q, v) X(float, eps, eps, v) X(int, spin_limit, spin_limit, v) \
     X(unsigned long long *, stamps, stamps, v)
 
-// M: rows.  The first M wavefronts of a unit take a merge (row, 64 dims) each, the other ten a row group of 8
+// One wavefront's merge of 64 dims (number u of the row's) of row j, lane = dim: at most T tiles
+template <int T>
+struct AoutMerge {
+    float pm1, pl1, pv[T];
+    __device__ __forceinline__ void request(const AttnOutArgs &a, int u, int j, int lane) {
+        const int hd = a.g.hd, head = u * 64 / hd;
+        const size_t base = ((size_t)j * a.g.H + head) * a.g.tiles_max;
+        // (buffer loads, the tile's offset in a scalar register: as flat loads each takes a dozen instructions of address arithmetic)
+        const __amdgpu_buffer_rsrc_t acc = lg_buffer_rsrc(a.g.pacc + base * hd + (u * 64 - head * hd));
+        const int mine = lane < a.tiles ? lane : a.tiles - 1;
+        pm1 = a.g.pm[base + mine]; pl1 = a.g.pl[base + mine];
+        #pragma unroll
+        for (int n = 0; n < LG_AOUT_BATCH; ++n) pv[n] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(acc, lane * 4, (n < a.tiles ? n : a.tiles - 1) * hd * 4, 0));
+        if (T > LG_AOUT_BATCH && a.tiles > LG_AOUT_BATCH) {
+            #pragma unroll
+            for (int n = LG_AOUT_BATCH; n < T; ++n) pv[n] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(acc, lane * 4, (n < a.tiles ? n : a.tiles - 1) * hd * 4, 0));
+        }
+    }
+};
+// The merged values of rows j, j + 4, .. (N of them by one wavefront: their chains side by side)
+template <int T, int N>
+__device__ __forceinline__ void lg_aout_merge(const AoutMerge<T> (&m)[N], const AttnOutArgs &a, int pos, int j, int lane, float (&out)[N]) {
+    const int first = lg_win_start(pos, a.g.window) >> 5;
+    int lo[N], hi[N], lo_all = 0, hi_all = 64;
+    float wt[N], L[N], o[N];
+    #pragma unroll
+    for (int r = 0; r < N; ++r) {
+        lo[r] = (lg_win_start(pos + j + 4 * r, a.g.window) >> 5) - first; hi[r] = ((pos + j + 4 * r) >> 5) - first;
+        lo_all = lo[r] > lo_all ? lo[r] : lo_all; hi_all = hi[r] < hi_all ? hi[r] : hi_all;
+        const float mx = lg_max_n(lane >= lo[r] && lane <= hi[r] ? m[r].pm1 : -INFINITY, 64);
+        wt[r] = lg_expf(m[r].pm1 - mx); L[r] = o[r] = 0.0f;
+    }
+    auto add = [&](int r, int n) {
+        const float wn = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wt[r]), n)), ln = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(m[r].pl1), n));
+        L[r] = lg_fmaf(ln, wn, L[r]); o[r] = lg_fmaf(m[r].pv[n], wn, o[r]);
+    };
+    auto add4 = [&](int n) {                                   // in tile order
+        if (n >= lo_all && n + 3 <= hi_all) {
+            #pragma unroll
+            for (int i = 0; i < 4; ++i)
+                #pragma unroll
+                for (int r = 0; r < N; ++r) add(r, n + i);
+        } else {
+            #pragma unroll
+            for (int i = 0; i < 4; ++i)
+                #pragma unroll
+                for (int r = 0; r < N; ++r) if (n + i >= lo[r] && n + i <= hi[r]) add(r, n + i);
+        }
+    };
+    #pragma unroll
+    for (int n = 0; n < LG_AOUT_BATCH; n += 4) add4(n);
+    if (T > LG_AOUT_BATCH && a.tiles > LG_AOUT_BATCH) {
+        #pragma unroll
+        for (int n = LG_AOUT_BATCH; n < T; n += 4) add4(n);
+    }
+    #pragma unroll
+    for (int r = 0; r < N; ++r) out[r] = o[r] / L[r];
+}
+// four lanes' q8 values as a word
+__device__ __forceinline__ uint32_t lg_aout_word(int q) {
+    return (uint32_t)(lg_dpp_i<0x00>(q) & 255) | (uint32_t)(lg_dpp_i<0x55>(q) & 255) << 8 | (uint32_t)(lg_dpp_i<0xAA>(q) & 255) << 16 | (uint32_t)lg_dpp_i<0xFF>(q) << 24;
+}
+// 16-byte units of row j's q8 as they are handed over: four of words a lane, one of scales
+__device__ __forceinline__ LgUnits<5> lg_aout_take(const AttnOutSync &y, int j, int lane, uint32_t tag, int spin_limit, int &err) {
+    return lg_take<5>([&](int i) { return i < 4 ? (const uint4 *)y.w + j * (LG_AOUT_K >> 3) + i * 64 + lane : y.s + j * (LG_AOUT_K >> 5) + lane; }, true, tag, spin_limit, err);
+}
+// The row work ahead of gate/up (lg_k_rows) in a row unit: row j, this unit storing and quantizing the float4s t + 256 vr; every thread
+// of the workgroup calls, those with rowt (the first 256) have the row
+struct AoutRow {
+    float4 x[LG_AOUT_NV], w1[LG_AOUT_NV], w2[LG_AOUT_NV];
+    __device__ __forceinline__ void request(const AttnOutArgs &a, int j, int t) {
+        const int nq = a.E >> 2;
+        #pragma unroll
+        for (int v = 0; v < LG_AOUT_NV; ++v) if (t + 256 * v < nq) {
+            x[v] = ((const float4 *)(a.x + (size_t)j * a.E))[t + 256 * v]; w1[v] = ((const float4 *)a.w_post)[t + 256 * v]; w2[v] = ((const float4 *)a.w_pre)[t + 256 * v];
+        }
+    }
+    template <bool MFMA>
+    __device__ __forceinline__ void work(const AttnOutArgs &a, const float4 (&dv)[LG_ROWV], int j, int vr, bool rowt, int t, float *red0, float *red1) {
+        const int E = a.E, nq = E >> 2;
+        float ss = 0.0f;
+        if (rowt) {
+            #pragma unroll
+            for (int v = 0; v < LG_AOUT_NV; ++v) if (t + 256 * v < nq) ss = lg_sumsq4(dv[v], ss);
+        }
+        ss = lg_block_sum256_of512(ss, red0);
+        float sc = 1.0f / sqrtf(ss / (float)E + a.eps);
+        ss = 0.0f;
+        if (rowt) {
+            #pragma unroll
+            for (int v = 0; v < LG_AOUT_NV; ++v) if (t + 256 * v < nq) {
+                const float4 w = w1[v];
+                float4 r = x[v];
+                r.x = r.x + dv[v].x * sc * w.x;  r.y = r.y + dv[v].y * sc * w.y;
+                r.z = r.z + dv[v].z * sc * w.z;  r.w = r.w + dv[v].w * sc * w.w;
+                x[v] = r;
+                if (v == vr) ((float4 *)(a.x_out + (size_t)j * E))[t + 256 * v] = r;
+                ss = lg_sumsq4(r, ss);
+            }
+        }
+        ss = lg_block_sum256_of512(ss, red1);
+        sc = 1.0f / sqrtf(ss / (float)E + a.eps);
+        if (!rowt) return;
+        #pragma unroll
+        for (int v = 0; v < LG_AOUT_NV; ++v) {
+            if (t + 256 * v >= nq || v != vr) continue;
+            const float4 w = w2[v], h = make_float4(x[v].x * sc * w.x, x[v].y * sc * w.y, x[v].z * sc * w.z, x[v].w * sc * w.w);
+            float d; int sum;
+            const uint32_t packed = lg_quant4_8lanes(h, &d, &sum);
+            const int quad = t + 256 * v, dw = quad & 7;
+            if (MFMA) {                                        // (order of lg_k_geglu_m)
+                uint32_t *blk = (uint32_t *)a.q + (size_t)(quad >> 3) * LG_MU_DWORDS;
+                blk[j * 8 + ((dw & 1) | ((dw & 2) << 1) | ((dw & 4) >> 1))] = packed;
+                if ((t & 7) == 0) *(float2 *)(blk + 64 + 2 * j) = make_float2(d, 12582912.0f + (float)(8 * sum));
+            } else {                                           // (order of lg_k_geglu_t)
+                uint32_t *unit = (uint32_t *)a.q + (size_t)(quad >> 3) * 32;
+                unit[j * 8 + dw] = packed;
+                if ((t & 7) == 0) *(float2 *)(unit + 24 + 2 * j) = make_float2(d, __int_as_float(sum));
+            }
+        }
+    }
+};
+
+// M: rows.  The first M wavefronts of a unit take a merge each, the other ten a row group of 8
 template <int M>
 __global__ __launch_bounds__(64 * (LG_AOUT_G + M)) void lg_k_attn_out(StepCtl *ctl, LG_AOUT_FIELDS(LG_XP, _) int p_end_) {
-    constexpr int qd = LG_AOUT_K, NIT = qd >> 8, W = LG_AOUT_G + M, NV = (LG_AOUT_E + 1023) / 1024;
-    static_assert(qd == 64 * LG_XCD_WGS, "a merge of every row per unit");
+    constexpr int qd = LG_AOUT_K, NIT = qd >> 8, W = LG_AOUT_G + M;
     if (blockIdx.x & (LG_XCDS - 1)) return;
     AttnOutArgs a; LG_AOUT_FIELDS(LG_XI, a)
     __shared__ __align__(16) int8_t lq[M * qd * 5 / 4];        // [M][qd] int8, then [M][qd / 32] {scale, sum}: order of lg_act_layout
     __shared__ float red[2][W];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), c = lane & 7;
     const int u = blockIdx.x >> 3, E = a.E, nq = E >> 2, slices = (E + 1023) >> 10;
-    auto stamp = [&](int i) { if (a.stamps && lane == 0 && wave == 0) a.stamps[(size_t)u * 8 + i] = wall_clock64(); };
+    auto stamp = [&](int i) { if (a.stamps && t == 0) a.stamps[(size_t)u * 8 + i] = wall_clock64(); };
     stamp(0);
     const uint32_t gen = a.sync->gen;
     const uint32_t tag = lg_tag(gen, lg_xcc_id());
@@ -62,65 +191,26 @@ __global__ __launch_bounds__(64 * (LG_AOUT_G + M)) void lg_k_attn_out(StepCtl *c
     const int jr = u % M, vr = u / M;                          // the row unit's row and its float4s (row units: u < M * slices)
     const bool rowt = u < M * slices && t < LG_WG;
     uint4 wq[NIT]; uint32_t ws[NIT];
-    float4 xv[NV], w1[NV], w2[NV];
-    auto request_row = [&]() {
-        if (rowt) {
-            #pragma unroll
-            for (int v = 0; v < NV; ++v) if (t + 256 * v < nq) {
-                xv[v] = ((const float4 *)(a.x + (size_t)jr * E))[t + 256 * v]; w1[v] = ((const float4 *)a.w_post)[t + 256 * v]; w2[v] = ((const float4 *)a.w_pre)[t + 256 * v];
-            }
-        }
-    };
     // The partials are requested ahead of the CU's 92 KB of weights, which its one memory path takes 2 us for: behind them they arrive a
     // microsecond later.  (A wavefront meets the barrier in one branch or in the other.)
     if (wave < M) {
-        // ---- merge: 64 dims of a (row, head) ----
-        const int hd = a.g.hd, j = wave, head = u * 64 / hd;
-        const size_t base = ((size_t)j * a.g.H + head) * a.g.tiles_max;
-        const float *acc = a.g.pacc + base * hd + (u * 64 - head * hd) + lane;
-        const int mine = lane < a.tiles ? lane : a.tiles - 1;
-        const float pm1 = a.g.pm[base + mine], pl1 = a.g.pl[base + mine];
-        float pv[LG_AOUT_TILES];
-        #pragma unroll
-        for (int n = 0; n < LG_AOUT_BATCH; ++n) pv[n] = acc[(size_t)(n < a.tiles ? n : a.tiles - 1) * hd];
-        const bool more = a.tiles > LG_AOUT_BATCH;
-        if (more) {
-            #pragma unroll
-            for (int n = LG_AOUT_BATCH; n < LG_AOUT_TILES; ++n) pv[n] = acc[(size_t)(n < a.tiles ? n : a.tiles - 1) * hd];
-        }
-        const int pos = ctl->pos, first = lg_win_start(pos, a.g.window) >> 5, lo = (lg_win_start(pos + j, a.g.window) >> 5) - first, hi = ((pos + j) >> 5) - first;
+        const int j = wave;
+        AoutMerge<LG_AOUT_TILES> m[1];
+        m[0].request(a, u, j, lane);
+        const int pos = ctl->pos;
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
-        const float mx = lg_max_n(lane >= lo && lane <= hi ? pm1 : -INFINITY, 64), wt = lg_expf(pm1 - mx);
-        stamp(1);
-        float L = 0.0f, o = 0.0f;
-        auto add = [&](int n) {
-            const float wn = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wt), n)), ln = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(pl1), n));
-            L = lg_fmaf(ln, wn, L); o = lg_fmaf(pv[n], wn, o);
-        };
-        auto add4 = [&](int n) {                               // in tile order
-            if (n >= lo && n + 3 <= hi) { add(n); add(n + 1); add(n + 2); add(n + 3); }
-            else {
-                #pragma unroll
-                for (int i = 0; i < 4; ++i) if (n + i >= lo && n + i <= hi) add(n + i);
-            }
-        };
-        #pragma unroll
-        for (int n = 0; n < LG_AOUT_BATCH; n += 4) add4(n);
-        if (more) {
-            #pragma unroll
-            for (int n = LG_AOUT_BATCH; n < LG_AOUT_TILES; n += 4) add4(n);
-        }
-        float d; int sum;
-        const int q = lg_quant1_32lanes(o / L, &d, &sum), e = u * 64 + lane;
+        float v[1], d; int sum;
+        lg_aout_merge(m, a, pos, j, lane, v);
+        const int q = lg_quant1_32lanes(v[0], &d, &sum), e = u * 64 + lane;
         const ActLayout lay = lg_act_layout(qd);
-        const uint32_t w = (uint32_t)(lg_dpp_i<0x00>(q) & 255) | (uint32_t)(lg_dpp_i<0x55>(q) & 255) << 8 | (uint32_t)(lg_dpp_i<0xAA>(q) & 255) << 16 | (uint32_t)lg_dpp_i<0xFF>(q) << 24;
+        const uint32_t w = lg_aout_word(q);
         if ((e & 3) == 0) y.w[(j * qd >> 2) + lg_act_unit(lay, e >> 4) * 4 + ((e >> 2) & 3)] = make_uint2(w, tag);
         if ((e & 31) == 0) y.s[(j * qd >> 5) + lg_act_block(lay, e >> 5)] = make_uint4(__float_as_uint(d), tag, (uint32_t)sum, tag);
-        stamp(2);
+        stamp(1);
         // ---- hand-over: the whole row, to every unit.  (Loads return in order: a wavefront with weights on their way would wait for those first.) ----
-        const LgUnits<5> r = lg_take<5>([&](int i) { return i < 4 ? (const uint4 *)y.w + j * (qd >> 3) + i * 64 + lane : y.s + j * (qd >> 5) + lane; }, true, tag, a.spin_limit, err);
+        const LgUnits<5> r = lg_aout_take(y, j, lane, tag, a.spin_limit, err);
         #pragma unroll
         for (int i = 0; i < 4; ++i) *(uint2 *)(lq + j * qd + 512 * i + 8 * lane) = make_uint2(r.v[i].x, r.v[i].z);
         lg_q8_ds<M>(lq, qd)[j * (qd >> 5) + lane] = make_float2(__uint_as_float(r.v[4].x), __uint_as_float(r.v[4].z));
@@ -134,8 +224,9 @@ __global__ __launch_bounds__(64 * (LG_AOUT_G + M)) void lg_k_attn_out(StepCtl *c
         }
     }
     __syncthreads();
-    stamp(3);
-    request_row();
+    stamp(2);
+    AoutRow row;
+    if (rowt) row.request(a, jr, t);
     // ---- this wavefront's row group of the projection ----
     if (eg) {
         float p[M];
@@ -161,50 +252,138 @@ __global__ __launch_bounds__(64 * (LG_AOUT_G + M)) void lg_k_attn_out(StepCtl *c
         for (int j = 0; j < M; ++j) p[j] = lg_sum8(p[j]);
         if (c < M) lg_put(y.o + (size_t)c * E + ge * 8 + (lane >> 3), lg_pick<M>(p, c), tag);
     }
-    stamp(4);
+    stamp(3);
     if (err) atomicOr(&ctl->err, err);
     if (u >= M * slices) return;                               // this unit has no share of the row work
-    // ---- hand-over: the projection's row; the row work, this unit storing and quantizing slice vr (lg_k_rows) ----
+    // ---- hand-over: the projection's row; the row work ----
     float4 dv[LG_ROWV];
     err = 0;
     if (rowt) lg_take_row(dv, y.o + (size_t)jr * E, t, nq, tag, a.spin_limit, err);
     if (err) atomicOr(&ctl->err, err);
+    stamp(4);
+    row.work<false>(a, dv, jr, vr, rowt, t, red[0], red[1]);
     stamp(5);
-    float ss = 0.0f;
-    if (rowt) {
+    if (u == 0 && t == 0) a.sync->gen = gen + 1;
+}
+
+// Blocks of 4..8 rows: wavefronts 0..3 of a unit merge rows w and w + 4, the other eight run a K segment each of the row blocks u, u + 32,
+// u + 64 of 32 rows (a segment's activations are read once for the three: LDS would set the time otherwise)
+template <int M>
+__global__ __launch_bounds__(768) void lg_k_attn_out_m(StepCtl *ctl, LG_AOUT_FIELDS(LG_XP, _) int p_end_) {
+    constexpr int nb = LG_AOUT_K >> 5, NIT = nb / 8, NP = NIT / 2, RB = (LG_AOUT_E / 32 + LG_XCD_WGS - 1) / LG_XCD_WGS, W = 12;
+    if (blockIdx.x & (LG_XCDS - 1)) return;
+    AttnOutArgs a; LG_AOUT_FIELDS(LG_XI, a)
+    __shared__ __align__(16) unsigned char la[nb * LG_MU_DWORDS * 4];      // the rows as blocks of lg_k_geglu_m; slots past the block's rows hold anything
+    __shared__ float sums[8][RB][8][32], red[2][W];            // [segment][row block][row slot][row]
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), n = lane & 31, h = lane >> 5;
+    const int u = blockIdx.x >> 3, E = a.E, nq = E >> 2, nrb = E >> 5, slices = (E + 1023) >> 10;
+    auto stamp = [&](int i) { if (a.stamps && t == 0) a.stamps[(size_t)u * 8 + i] = wall_clock64(); };
+    stamp(0);
+    const uint32_t gen = a.sync->gen;
+    const uint32_t tag = lg_tag(gen, lg_xcc_id());
+    AttnOutSync &y = *a.sync;
+    int err = 0;
+    const int seg = wave - 4;
+    const int jr = u % M, vr = u / M;
+    const bool rowt = u < M * slices && t < LG_WG;
+    lg_x4u wq[RB][NP]; uint32_t ws[RB][NP];
+    if (wave < 4) {
+        const int e = u * 64 + lane, b = e >> 5, dw = (e >> 2) & 7;
+        auto merge = [&](auto two) {                           // rows wave and, of more than four, wave + 4
+            constexpr int N = decltype(two)::value ? 2 : 1;
+            AoutMerge<LG_AOUT_BATCH> m[N];
+            #pragma unroll
+            for (int r = 0; r < N; ++r) m[r].request(a, u, wave + 4 * r, lane);
+            const int pos = ctl->pos;
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            float v[N], d[N]; int q[N], sum[N];
+            lg_aout_merge(m, a, pos, wave, lane, v);
+            #pragma unroll
+            for (int r = 0; r < N; ++r) q[r] = lg_quant1_32lanes(v[r], &d[r], &sum[r]);
+            #pragma unroll
+            for (int r = 0; r < N; ++r) {
+                const int j = wave + 4 * r;
+                const uint32_t w = lg_aout_word(q[r]);
+                if ((e & 3) == 0) y.w[j * (LG_AOUT_K >> 2) + b * 8 + ((dw & 1) | ((dw & 2) << 1) | ((dw & 4) >> 1))] = make_uint2(w, tag);
+                if ((e & 31) == 0) y.s[j * nb + b] = make_uint4(__float_as_uint(d[r]), tag, __float_as_uint(12582912.0f + (float)(8 * sum[r])), tag);
+            }
+        };
+        if (wave + 4 < M) merge(std::true_type{}); else merge(std::false_type{});
+        stamp(1);
+        // ---- hand-over ----
+        for (int j = wave; j < M; j += 4) {
+            const LgUnits<5> r = lg_aout_take(y, j, lane, tag, a.spin_limit, err);
+            #pragma unroll
+            for (int i = 0; i < 4; ++i) *(uint2 *)(la + (i * 16 + (lane >> 2)) * (LG_MU_DWORDS * 4) + j * 32 + (lane & 3) * 8) = make_uint2(r.v[i].x, r.v[i].z);
+            *(uint2 *)(la + lane * (LG_MU_DWORDS * 4) + 256 + j * 8) = make_uint2(r.v[4].x, r.v[4].z);
+        }
+    } else {
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
         #pragma unroll
-        for (int v = 0; v < NV; ++v) if (t + 256 * v < nq) ss = lg_sumsq4(dv[v], ss);
-    }
-    ss = lg_block_sum256_of512(ss, red[0]);
-    float sc = 1.0f / sqrtf(ss / (float)E + a.eps);
-    ss = 0.0f;
-    if (rowt) {
-        #pragma unroll
-        for (int v = 0; v < NV; ++v) if (t + 256 * v < nq) {
-            const float4 w = w1[v];
-            float4 x = xv[v];
-            x.x = x.x + dv[v].x * sc * w.x;  x.y = x.y + dv[v].y * sc * w.y;
-            x.z = x.z + dv[v].z * sc * w.z;  x.w = x.w + dv[v].w * sc * w.w;
-            xv[v] = x;
-            if (v == vr) ((float4 *)(a.x_out + (size_t)jr * E))[t + 256 * v] = x;
-            ss = lg_sumsq4(x, ss);
+        for (int k = 0; k < RB; ++k) {
+            const int rb = u + LG_XCD_WGS * k;
+            if (rb < nrb) {
+                const uint8_t *cb = a.wo + ((size_t)rb * 8 + seg) * (NIT * 576);
+                #pragma unroll
+                for (int jp = 0; jp < NP; ++jp) {
+                    wq[k][jp] = __builtin_nontemporal_load((const lg_x4u *)(cb + (size_t)((jp * 2 + h) * 32 + n) * 16));
+                    ws[k][jp] = __builtin_nontemporal_load((const uint32_t *)(cb + (size_t)NIT * 512 + (size_t)(jp * 32 + n) * 4));
+                }
+            }
         }
     }
-    ss = lg_block_sum256_of512(ss, red[1]);
-    sc = 1.0f / sqrtf(ss / (float)E + a.eps);
-    if (rowt) {
+    __syncthreads();
+    stamp(2);
+    AoutRow row;
+    // ---- segment `seg` of the unit's row blocks ----
+    if (wave >= 4) {
+        lg_v16i magic;
         #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            if (t + 256 * v >= nq || v != vr) continue;
-            const float4 w = w2[v], h = make_float4(xv[v].x * sc * w.x, xv[v].y * sc * w.y, xv[v].z * sc * w.z, xv[v].w * sc * w.w);
-            float d; int sum;
-            const uint32_t packed = lg_quant4_8lanes(h, &d, &sum);
-            const int quad = t + 256 * v;
-            uint32_t *unit = (uint32_t *)a.q + (size_t)(quad >> 3) * 32;       // (order of lg_k_geglu_t)
-            unit[jr * 8 + (quad & 7)] = packed;
-            if ((t & 7) == 0) *(float2 *)(unit + 24 + 2 * jr) = make_float2(d, __int_as_float(sum));
+        for (int i = 0; i < 16; ++i) magic[i] = 0x4B400000;
+        asm volatile("" : "+v"(magic));
+        const int arow = n < 8 ? n : 7;
+        float p[RB][4];
+        #pragma unroll
+        for (int k = 0; k < RB; ++k)
+            #pragma unroll
+            for (int i = 0; i < 4; ++i) p[k][i] = 0.0f;
+        const unsigned char *ls = la + seg * NIT * (LG_MU_DWORDS * 4);
+        XffnAct nx = lg_xffn_act(ls, arow, h);
+        #pragma unroll
+        for (int s = 0; s < NIT; ++s) {
+            const XffnAct ac = nx;
+            if (s + 1 < NIT) nx = lg_xffn_act(ls + (s + 1) * (LG_MU_DWORDS * 4), arow, h);
+            #pragma unroll
+            for (int k = 0; k < RB; ++k) {
+                lg_v2u q; q.x = s & 1 ? wq[k][s >> 1].z : wq[k][s >> 1].x; q.y = s & 1 ? wq[k][s >> 1].w : wq[k][s >> 1].y;
+                lg_xffn_step(ac.av, ac.xd, ac.cf, q, lg_h2f((uint16_t)(s & 1 ? ws[k][s >> 1] >> 16 : ws[k][s >> 1])), magic, p[k]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
+        #pragma unroll
+        for (int k = 0; k < RB; ++k)
+            #pragma unroll
+            for (int i = 0; i < 4; ++i) sums[seg][k][4 * h + i][n] = p[k][i];
+    } else if (rowt) row.request(a, jr, t);                    // (in the branch without the projection's registers)
+    __syncthreads();
+    for (int idx = t; idx < RB * M * 32; idx += 64 * W) {      // the adjacent-pair tree over the 8 segments
+        const int k = idx / (M * 32), rem = idx - k * (M * 32), j = rem >> 5, i = rem & 31, rb = u + LG_XCD_WGS * k;
+        if (rb < nrb)
+            lg_put(y.o + (size_t)j * E + rb * 32 + i, ((sums[0][k][j][i] + sums[1][k][j][i]) + (sums[2][k][j][i] + sums[3][k][j][i])) +
+                                                      ((sums[4][k][j][i] + sums[5][k][j][i]) + (sums[6][k][j][i] + sums[7][k][j][i])), tag);
     }
-    stamp(6);
+    stamp(3);
+    if (err) atomicOr(&ctl->err, err);
+    if (u >= M * slices) return;
+    float4 dv[LG_ROWV];
+    err = 0;
+    if (rowt) lg_take_row(dv, y.o + (size_t)jr * E, t, nq, tag, a.spin_limit, err);
+    if (err) atomicOr(&ctl->err, err);
+    stamp(4);
+    row.work<true>(a, dv, jr, vr, rowt, t, red[0], red[1]);
+    stamp(5);
     if (u == 0 && t == 0) a.sync->gen = gen + 1;
 }

@@ -156,7 +156,7 @@ struct Layer {
     uint8_t *wqkv = nullptr, *wo = nullptr, *wgu = nullptr, *wdown = nullptr, *winp = nullptr, *wproj = nullptr;
     float *winp_f = nullptr, *wproj_f = nullptr;   // inp_gate / proj when the file keeps them in a float type (then winp / wproj are null)
     uint8_t *wdn_m = nullptr;                      // ffn_down again as the per-workgroup streams of lg_k_down_m
-    uint8_t *wo_ch = nullptr;                      // attn_output again as matrix-core chains [row block][segment]: lg_k_attn_tail
+    uint8_t *wo_ch = nullptr;                      // attn_output again as matrix-core chains [row block][segment]: lg_k_attn_tail, lg_k_attn_out_m
     // the matrices once more in the form of the prompt kernels (lg_wide.h)
     uint8_t *wqkv_w = nullptr, *wo_w = nullptr, *wgu_w = nullptr, *wdown_w = nullptr, *winp_w = nullptr, *wproj_w = nullptr;
     uint8_t *wo_rb = nullptr;                      // attn_output again as row-block tiles: the chains of lg_k_merge_o
@@ -664,8 +664,9 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         if ((rc = upload_tiled(m, rows, y.qd, &y.wo, stage))) return rc;
         if ((rc = wide_form(m, y.wo, y.qd, E, false, &y.wo_w))) return rc;
         // (8 query heads: the K segments of this projection are the heads, and the merge can run their chains itself)
-        if (getenv("LG_HIP_XCD_ATTN_TAIL") && atoi(getenv("LG_HIP_XCD_ATTN_TAIL")) > 0 && !m->target && attn_tail_shape(y.qd, E, nullptr, nullptr) &&
-            cu_count() == LG_XCDS * LG_XCD_WGS) {
+        if (!m->target && cu_count() == LG_XCDS * LG_XCD_WGS &&
+            ((getenv("LG_HIP_XCD_ATTN_TAIL") && atoi(getenv("LG_HIP_XCD_ATTN_TAIL")) > 0 && attn_tail_shape(y.qd, E, nullptr, nullptr)) ||
+             (max_rows > LG_AOUT_DOT_ROWS && attn_out_shape(m, y)))) {
             stage.resize((size_t)E * (y.qd / 32) * 18);
             pack_o_chains(rows.data(), y.qd, E, stage.data());
             if (dev_alloc(m, &y.wo_ch, stage.size())) return -7;
@@ -1240,10 +1241,10 @@ static int step_tiles(const lg_hip_model *m, const lg_hip_kv *kv, const Layer &y
 }
 // (tiles: what one wavefront holds; more of them, a global layer in a cache of more than 1280 positions, are merged by more of the chip)
 static bool use_attn_out(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
-    return rows <= LG_AOUT_ROWS && m->attn_out && m->aosync && attn_out_shape(m, y) && tiles <= LG_AOUT_TILES;
+    return m->attn_out && m->aosync && attn_out_shape(m, y) && (rows <= LG_AOUT_DOT_ROWS ? tiles <= LG_AOUT_TILES : y.wo_ch && tiles <= LG_AOUT_BATCH);
 }
 static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
-    if (!y.wo_ch || !m->tsync || m->xcd_attn_tail <= 0 || (m->xcd_attn_tail == 1 && rows < 3)) return false;
+    if (!y.wo_ch || !m->tsync || !attn_tail_shape(y.qd, m->E, nullptr, nullptr) || m->xcd_attn_tail <= 0 || (m->xcd_attn_tail == 1 && rows < 3)) return false;
     const int slices = (m->E + 1023) / 1024;
     return tiles < 128 && m->H * rows <= 2 * LG_XCD_WGS && slices * rows <= LG_XCD_WGS && y.hd % 32 == 0 && y.hd <= 256;
 }
@@ -1546,13 +1547,14 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 merged_o = true; ffn_rows_done = true;
             } else
             if (!merged_o && pos_off == 0 && have_x && use_attn_out(m, y, M, tiles)) {
-                if constexpr (M <= LG_AOUT_ROWS) {
-                    AttnOutArgs f{};
-                    f.g = g; f.wo = y.wo; f.x = m->x[cur]; f.w_post = y.post_attn; f.w_pre = y.ffn_norm; f.x_out = m->x[cur ^ 1];
-                    f.q = m->hq; f.E = E; f.tiles = tiles; f.eps = m->eps; f.sync = m->aosync; f.spin_limit = 1 << 16;
-                    f.stamps = m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr;
+                AttnOutArgs f{};
+                f.g = g; f.wo = M <= LG_AOUT_DOT_ROWS ? y.wo : y.wo_ch; f.x = m->x[cur]; f.w_post = y.post_attn; f.w_pre = y.ffn_norm; f.x_out = m->x[cur ^ 1];
+                f.q = m->hq; f.E = E; f.tiles = tiles; f.eps = m->eps; f.sync = m->aosync; f.spin_limit = 1 << 16;
+                f.stamps = m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr;
+                if constexpr (M <= LG_AOUT_DOT_ROWS)
                     LAUNCH(KC_ATAIL, lg_k_attn_out<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(64 * (LG_AOUT_G + M)), 0, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
-                }
+                else
+                    LAUNCH(KC_ATAIL, lg_k_attn_out_m<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(768), 0, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
                 cur ^= 1;
                 merged_o = true; ffn_rows_done = true;
             } else
