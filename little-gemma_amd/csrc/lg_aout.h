@@ -5,15 +5,15 @@
 //   merge       64 dims of each row, a wavefront a row (two from 5 rows on: with more wavefronts than twelve the registers no longer hold the projection): what it loads comes first, the tiles' partials in
 //               registers   (lg_k_attn_merge)
 //   hand-over   the q8 of the rows, tagged (lg_take), to every unit's LDS: by the merging wavefronts
-//   projection  up to 3 rows (lg_k_attn_out): ten row groups of 8 on v_dot4, a wavefront each   (lg_k_mm)
-//               4 to 8 rows (lg_k_attn_out_m): up to three blocks of 32 rows on the matrix cores, a K segment to a wavefront   (lg_k_attn_tail)
+//   projection  up to 2 rows, 3 of more than 20 tiles (lg_k_attn_out): ten row groups of 8 on v_dot4, a wavefront each   (lg_k_mm)
+//               3 to 8 rows (lg_k_attn_out_m): up to three blocks of 32 rows on the matrix cores, a K segment to a wavefront   (lg_k_attn_tail)
 //               either way with the weights in registers, requested right behind the partials
 //   hand-over   the f32 rows, tagged, to the first rows x E/1024 units, which do the row work of lg_k_rows
 // Sums, their order and every rounding are the separate kernels', lane for lane.
 // Bound by the CU's one memory path up to the projection, then by LDS (v_dot4) or the vector units (matrix cores).  By the stamps the q8 of
 // one row leaves at 1.9 us and is in every LDS at 3.4, when the 92 KB of weights are through as well; rows at 5.4, end at 6.4; five rows
 // 3.0, 4.8, 7.9 (the projection 2.3) and 8.9.  E4B shape, the 35 sliding layers of 42, a step: one row 1784 -> 1694 us, two 1883 -> 1812,
-// three 1985 -> 1944, four 2061 -> 2007, five 2162 -> 2125, six 2210 -> 2162, eight 2304 -> 2276.
+// three 1978 -> 1923 (on v_dot4 1935), four 2061 -> 2007, five 2162 -> 2125, six 2210 -> 2162, eight 2304 -> 2276.
 // v_dot4 at 4, 5, 8 rows: 2080, 2196, 2575 (every row group reads the rows from LDS again).  4096 inputs, 276 KB a CU at rows of 3840: a
 // step of the 12B shape 2481 -> 2728.  Weights requested ahead of the partials: one row 1741.  Partials first, but the hand-over
 // taken by the wavefronts that hold weights: 1712.  Five to eight rows with a wavefront per merge: the projection spills, 2202 at five.
@@ -266,7 +266,7 @@ __global__ __launch_bounds__(64 * (LG_AOUT_G + M)) void lg_k_attn_out(StepCtl *c
     if (u == 0 && t == 0) a.sync->gen = gen + 1;
 }
 
-// Blocks of 4..8 rows: wavefronts 0..3 of a unit merge rows w and w + 4, the other eight run a K segment each of the row blocks u, u + 32,
+// Blocks of 3..8 rows: wavefronts 0..3 of a unit merge rows w and w + 4, the other eight run a K segment each of the row blocks u, u + 32,
 // u + 64 of 32 rows (a segment's activations are read once for the three: LDS would set the time otherwise)
 template <int M>
 __global__ __launch_bounds__(768) void lg_k_attn_out_m(StepCtl *ctl, LG_AOUT_FIELDS(LG_XP, _) int p_end_) {
@@ -310,7 +310,8 @@ __global__ __launch_bounds__(768) void lg_k_attn_out_m(StepCtl *ctl, LG_AOUT_FIE
                 if ((e & 31) == 0) y.s[j * nb + b] = make_uint4(__float_as_uint(d[r]), tag, __float_as_uint(12582912.0f + (float)(8 * sum[r])), tag);
             }
         };
-        if (wave + 4 < M) merge(std::true_type{}); else merge(std::false_type{});
+        if (wave + 4 < M) merge(std::true_type{}); else if (wave < M) merge(std::false_type{});
+        else __builtin_amdgcn_s_barrier();
         stamp(1);
         // ---- hand-over ----
         for (int j = wave; j < M; j += 4) {
@@ -383,7 +384,7 @@ __global__ __launch_bounds__(768) void lg_k_attn_out_m(StepCtl *ctl, LG_AOUT_FIE
     if (rowt) lg_take_row(dv, y.o + (size_t)jr * E, t, nq, tag, a.spin_limit, err);
     if (err) atomicOr(&ctl->err, err);
     stamp(4);
-    row.work<true>(a, dv, jr, vr, rowt, t, red[0], red[1]);
+    row.work<(M > 3)>(a, dv, jr, vr, rowt, t, red[0], red[1]);
     stamp(5);
     if (u == 0 && t == 0) a.sync->gen = gen + 1;
 }

@@ -666,7 +666,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         // (8 query heads: the K segments of this projection are the heads, and the merge can run their chains itself)
         if (!m->target && cu_count() == LG_XCDS * LG_XCD_WGS &&
             ((getenv("LG_HIP_XCD_ATTN_TAIL") && atoi(getenv("LG_HIP_XCD_ATTN_TAIL")) > 0 && attn_tail_shape(y.qd, E, nullptr, nullptr)) ||
-             (max_rows > LG_AOUT_DOT_ROWS && attn_out_shape(m, y)))) {
+             (max_rows >= LG_AOUT_DOT_ROWS && attn_out_shape(m, y)))) {
             stage.resize((size_t)E * (y.qd / 32) * 18);
             pack_o_chains(rows.data(), y.qd, E, stage.data());
             if (dev_alloc(m, &y.wo_ch, stage.size())) return -7;
@@ -1547,14 +1547,15 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 merged_o = true; ffn_rows_done = true;
             } else
             if (!merged_o && pos_off == 0 && have_x && use_attn_out(m, y, M, tiles)) {
+                const bool chains = M > LG_AOUT_DOT_ROWS || (M == LG_AOUT_DOT_ROWS && y.wo_ch && tiles <= LG_AOUT_BATCH);
                 AttnOutArgs f{};
-                f.g = g; f.wo = M <= LG_AOUT_DOT_ROWS ? y.wo : y.wo_ch; f.x = m->x[cur]; f.w_post = y.post_attn; f.w_pre = y.ffn_norm; f.x_out = m->x[cur ^ 1];
+                f.g = g; f.wo = chains ? y.wo_ch : y.wo; f.x = m->x[cur]; f.w_post = y.post_attn; f.w_pre = y.ffn_norm; f.x_out = m->x[cur ^ 1];
                 f.q = m->hq; f.E = E; f.tiles = tiles; f.eps = m->eps; f.sync = m->aosync; f.spin_limit = 1 << 16;
                 f.stamps = m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr;
+                if constexpr (M >= LG_AOUT_DOT_ROWS)
+                    if (chains) LAUNCH(KC_ATAIL, lg_k_attn_out_m<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(768), 0, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
                 if constexpr (M <= LG_AOUT_DOT_ROWS)
-                    LAUNCH(KC_ATAIL, lg_k_attn_out<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(64 * (LG_AOUT_G + M)), 0, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
-                else
-                    LAUNCH(KC_ATAIL, lg_k_attn_out_m<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(768), 0, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
+                    if (!chains) LAUNCH(KC_ATAIL, lg_k_attn_out<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(64 * (LG_AOUT_G + M)), 0, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
                 cur ^= 1;
                 merged_o = true; ffn_rows_done = true;
             } else
