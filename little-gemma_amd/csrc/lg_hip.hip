@@ -173,7 +173,7 @@ static const char *k_class_names[KC_COUNT] = { "rows_norm_quant", "ple_model_pro
     "attn_output", "gate_up_geglu", "ffn_down", "ple_gate", "ple_proj", "lm_head", "accept", "ffn_xcd", "ple_tail", "attn_tail" };
 
 // What a captured graph was captured for: the cache's id, the options, the block width and the rest of the options.
-typedef std::array<uint64_t, 3> GraphKey;
+typedef std::array<uint64_t, 4> GraphKey;
 struct Profile {
     bool on = false;
     std::vector<hipEvent_t> ev;        // pairs
@@ -243,6 +243,7 @@ struct lg_hip_model {
     RgSync *rgsync = nullptr;                // flags and epoch base of lg_k_rows_geglu
     unsigned long long *tstamps = nullptr;   // [LG_XTAIL_UNITS][8] phase stamps of the last such launch (option xcd_tail_stamps)
     int tail_stamps = 0;
+    int wait_polls = 1 << 16;                // option: polls after which a kernel gives up a hand-over inside its launch
     bool xffn_built = false;                 // streams and working memory exist
     int xffn_cls = -1;                       // which instantiation serves the shape
     int xffn_delay = 0;                      // option: units of 64 clocks its compute wavefronts wait before they request their weights
@@ -992,7 +993,8 @@ extern "C" int lg_hip_kv_restore_prefix(lg_hip_kv *kv, int n) {
     return 0;
 }
 
-__global__ void lg_k_set_ctl(StepCtl *ctl, int pos) { ctl->pos = pos; ctl->step = 0; ctl->err = 0; ctl->report = 0; }
+// (first: of the call's blocks; what an earlier one reported stays)
+__global__ void lg_k_set_ctl(StepCtl *ctl, int pos, bool first) { ctl->pos = pos; ctl->step = 0; ctl->report = 0; if (first) ctl->err = 0; }
 
 // ---- launching --------------------------------------------------------------------------------
 static size_t lds_mm(int M, int k) { return (size_t)M * k + (size_t)M * (k / 32) * 8; }
@@ -1526,7 +1528,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 f.ipl = m->ple ? m->pmp_raw + (size_t)L * m->ple : nullptr;
                 f.qkv = m->qkv; f.h_out = last ? m->hidden_rows : nullptr; f.hq = m->hq;
                 f.E = E; f.qd = y.qd; f.FF = y.nff; f.qm = last ? 0 : m->L[L + 1].qkv_m; f.tiles = tiles; f.eps = m->eps;
-                f.sync = m->nsync; f.err = &m->ctl->err; f.err2 = draft ? &m->target->ctl->err : nullptr; f.spin_limit = 1 << 16;
+                f.sync = m->nsync; f.err = &m->ctl->err; f.err2 = draft ? &m->target->ctl->err : nullptr; f.spin_limit = m->wait_polls;
                 if (m->ple) LAUNCH(KC_TAIL, lg_k_narrow<true>, dim3(LG_XCDS * LG_NARROW_WGS), dim3(512), 0, f, m->ctl);
                 else        LAUNCH(KC_TAIL, lg_k_narrow<false>, dim3(LG_XCDS * LG_NARROW_WGS), dim3(512), 0, f, m->ctl);
                 cur ^= 1;
@@ -1540,7 +1542,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 f.g = g; f.wo = y.wo_ch; f.aq = (uint32_t *)m->aq; f.pout = m->dout;
                 f.x = m->x[cur]; f.w_post = y.post_attn; f.w_pre = y.ffn_norm; f.x_out = m->x[cur ^ 1];
                 f.q = m->hq; f.q_units = (M >= 4) ? 2 : 1; f.E = E; f.eps = m->eps;
-                f.sync = m->tsync; f.spin_limit = 1 << 16; f.stamps = m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr;
+                f.sync = m->tsync; f.spin_limit = m->wait_polls; f.stamps = m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr;
                 launch_attn_tail<M>(lx, f);
                 cur ^= 1;
                 pend_dout = pend_w = pend_os = nullptr; pend_parts = 1;
@@ -1550,7 +1552,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 const bool chains = M > LG_AOUT_DOT_ROWS || (M == LG_AOUT_DOT_ROWS && y.wo_ch && tiles <= LG_AOUT_BATCH);
                 AttnOutArgs f{};
                 f.g = g; f.wo = chains ? y.wo_ch : y.wo; f.x = m->x[cur]; f.w_post = y.post_attn; f.w_pre = y.ffn_norm; f.x_out = m->x[cur ^ 1];
-                f.q = m->hq; f.E = E; f.tiles = tiles; f.eps = m->eps; f.sync = m->aosync; f.spin_limit = 1 << 16;
+                f.q = m->hq; f.E = E; f.tiles = tiles; f.eps = m->eps; f.sync = m->aosync; f.spin_limit = m->wait_polls;
                 f.stamps = m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr;
                 if constexpr (M >= LG_AOUT_DOT_ROWS)
                     if (chains) LAUNCH(KC_ATAIL, lg_k_attn_out_m<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(768), 0, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
@@ -1584,7 +1586,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 // the whole half as one launch partitioned by XCD: row work, gate/up + GeGLU and the XCD's K share of
                 // ffn_down; the consumer adds the 8 slabs (the top of the segment tree)
                 XffnArgs f{ y.xgu, y.xdn, m->x[cur], pend_dout, pend_w, y.ffn_norm, m->x[cur ^ 1], m->slabs, m->xq8, m->xact,
-                            m->xsync, m->ctl, E, y.nff, m->eps, 1 << 18, m->xffn_delay, nullptr };
+                            m->xsync, m->ctl, E, y.nff, m->eps, 4 * m->wait_polls, m->xffn_delay, nullptr };
                 launch_xffn<M>(lx, f, m->xffn_cls);
                 cur ^= 1;
                 pend_dout = m->slabs; pend_parts = LG_XCDS; pend_w = y.post_ffw; pend_os = m->ple ? nullptr : y.out_scale;
@@ -1599,7 +1601,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 if (m->rows_geglu && m->rgsync && !ffn_rows_done && have_x && pend_dout && !pend_os && (pend_parts == 1 || pend_parts == 4) && (E == 2560 || E == 3840 || E == 512) &&
                     M * slices <= LG_RG_MAXP && L < LG_RG_STEP - 1) {
                     RowsGegluArgs f{ m->x[cur], pend_dout, pend_w, y.ffn_norm, m->x[cur ^ 1], m->hq, E, pend_parts, slices, m->eps,
-                                     y.wgu, y.nff, m->gq, dn_m ? 2 : 0, m->rgsync, L, 1 << 16, m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr };
+                                     y.wgu, y.nff, m->gq, dn_m ? 2 : 0, m->rgsync, L, m->wait_polls, m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr };
                     const dim3 grid(M * slices + y.nff / 32);
                     const size_t lds = (size_t)(E / 32) * LG_MU_DWORDS * 4;
                     if (E == 512)  LAUNCH(KC_GATEUP, (lg_k_rows_geglu<M, 2>), grid, dim3(512), lds, m->ctl, LG_RG_FIELDS(LG_XA, f) 0);
@@ -1620,7 +1622,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             }
             MmArgs d{ y.wdown, y.nff, E, m->dout, m->gq, nullptr };
             if (dn_m) {
-                DownMArgs dm{ y.wdn_m, (const uint32_t *)m->gq, m->dout, E, y.nff, m->down_m == 1 ? m->dmsync : nullptr, m->ctl, 1 << 16 };
+                DownMArgs dm{ y.wdn_m, (const uint32_t *)m->gq, m->dout, E, y.nff, m->down_m == 1 ? m->dmsync : nullptr, m->ctl, m->wait_polls };
                 launch_down_m<M>(lx, dm);
                 pend_parts = dm.sync ? 1 : 4;
             } else
@@ -1658,7 +1660,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 f.w_pre = last ? m->output_norm : m->L[L + 1].attn_norm;
                 f.x_out = m->x[cur ^ 1]; f.h_out = last ? m->hidden_rows : nullptr;
                 f.q = m->hq; f.q_units = last && head_m ? 2 : 0;
-                f.sync = m->tsync; f.spin_limit = 1 << 16; f.stamps = m->tail_stamps ? m->tstamps : nullptr;
+                f.sync = m->tsync; f.spin_limit = m->wait_polls; f.stamps = m->tail_stamps ? m->tstamps : nullptr;
                 f.gf = m->tgf;
                 launch_ple_tail<M>(lx, f);
                 cur ^= 1;
@@ -1694,7 +1696,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         AcceptArgs c{ m->pval, m->pidx, grid, m->sched, m->out, m->adv, m->hidden_rows, m->g_hidden, E, m->pin + 32 };
         LAUNCH(KC_ACCEPT, (lg_k_accept<M>), dim3(1), dim3(LG_WG), 0, m->ctl, LG_ACCEPT_FIELDS(LG_XA, c) 0);
     } else if (!lx.rc && !dry) {
-        hipLaunchKernelGGL(lg_k_advance, dim3(1), dim3(1), 0, m->stream, m->ctl, M);
+        hipLaunchKernelGGL(lg_k_advance, dim3(1), dim3(1), 0, m->stream, m->ctl, M, m->pin + 32);
     }
     return lx.rc;
 }
@@ -1776,14 +1778,14 @@ static void launch_wide_attn(Launcher &lx, const WideAttn &a, int groups, bool f
 // One block of `rows` prompt positions from pos on (tokens in device memory): the launch sequence of a verify step with
 // the kernels of lg_wide.h.  Launched as it is, not captured: a prompt's blocks differ in width and tile counts, and the
 // host stays ahead of launches of this size.
-static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int rows, int pos) {
+static int enqueue_prompt(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int rows, int pos, bool first) {
     Launcher lx{ m, false };
     const int E = m->E, H = m->H, nl = m->n_layer;
     int cur = 0;
     bool have_x = false;
     const float *pend_dout = nullptr, *pend_w = nullptr, *pend_os = nullptr;
     int pend_parts = 1;
-    hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, m->stream, m->ctl, pos);
+    hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, m->stream, m->ctl, pos, first);
     auto row_work = [&](const float *w_pre, int8_t *q) {
         RowArgs s{};
         s.E = E; s.eps = m->eps; s.toks = toks; s.q = q;
@@ -1887,8 +1889,8 @@ static GraphKey graph_key(const lg_hip_model *m, const lg_hip_kv *kv, int rows, 
     put(what, 2); put(rows, 4); put(m->store_logits != 0, 1); put(m->draft_chain, 1); put(m->fuse_rows, 1); put(m->attn_rows, 1); put(m->attn_rows_fq, 1);
     put(m->head_mfma, 1); put(m->down_kq, 1); put(m->xcd_ffn, 1); put(m->fork_ple, 1); put(m->rows_geglu, 1); put(m->tail_stamps != 0, 1);
     put(m->tail_spread == 1 ? 1 : m->tail_spread ? 2 : 0, 2); put(m->xcd_tail, 2); put(m->down_m, 2); put(m->xcd_attn_tail, 2); put(m->merge_o, 2);
-    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1);
-    return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices };
+    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->wait_polls, 17);
+    return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices, 0 };
 }
 
 // What `enqueue` launches on the stream, as a graph for the calls to come.  The caller has just launched the same thing: it
@@ -1956,6 +1958,7 @@ extern "C" int lg_hip_set_option(lg_hip_model *m, const char *name, int value) {
     else if (!strcmp(name, "merge_o")) m->merge_o = value < 0 ? 0 : value > 2 ? 2 : value;
     else if (!strcmp(name, "merge_o_slices")) m->merge_o_slices = value < 0 ? 0 : value;
     else if (!strcmp(name, "xcd_tail")) m->xcd_tail = value < 0 ? 0 : value > 2 ? 2 : value;
+    else if (!strcmp(name, "wait_polls")) m->wait_polls = value < 0 ? 0 : value > 1 << 16 ? 1 << 16 : value;
     else if (!strcmp(name, "xcd_tail_stamps")) m->tail_stamps = value != 0;
     else if (!strcmp(name, "xcd_ffn_delay")) m->xffn_delay = value < 0 ? 0 : value > 0x3FF ? 0x3FF : value;
     else return fail(-2, "set_option: unknown option %s", name);
@@ -2102,8 +2105,7 @@ extern "C" int lg_hip_mtp_rounds(lg_hip_model *d, lg_hip_kv *kv, int token, int 
         for (int r = 0; r < n_rounds; ++r) if ((rc = enqueue_round(d, kv, rows, false))) return rc;
     } else {
         GraphKey key = graph_key(t, kv, rows, 2);
-        key[1] |= (uint64_t)(d->store_logits != 0) << 62 | (uint64_t)(d->fuse_rows != 0) << 63;
-        key[2] |= (uint64_t)(d->narrow != 0) << 63;
+        key[3] = graph_key(d, kv, 1, 2)[1];
         auto it = d->graphs.find(key);            // kept by the head: the graph dies with it or with the cache
         int r = 0;
         if (it == d->graphs.end()) {               // the first round as launches, its graph while the device works on it
@@ -2148,6 +2150,8 @@ extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *tok
     // (attention that keeps its weights in LDS addresses a layer's cache with 32 bits, and reaches no row past LG_WIDE_ROWS + 32 (LG_WA_TILES + 4))
     for (size_t L = 0; L < kv->seq.size(); ++L) wide_ok = wide_ok && (size_t)(LG_WIDE_ROWS + 32 * (LG_WA_TILES + 4)) * kv->kv_dim[L] * 2 < (size_t)1 << 31;
     const int cap = m->sched_cap * LG_HIP_MAX_ROWS;        // tokens the staging holds
+    int32_t *err = m->pin + 32 + LG_REPORT_ERR;             // (written by the verify blocks among the call's, the prompt kernels wait for nobody)
+    __atomic_store_n(err, 0, __ATOMIC_RELAXED);
     for (int at = 0; at < n;) {
         // the tokens go over once, the blocks follow each other on the stream and the host waits at the end
         const int part = n - at < cap ? n - at : cap;
@@ -2157,11 +2161,12 @@ extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *tok
             const int left = part - done;
             int rows = left < kv->prompt_rows ? left : kv->prompt_rows, rc;
             const bool wide = wide_ok && !far_in_narrow_heads(m, kv, rows, pos0 + at + done);
-            if (wide && left > m->max_rows) rc = enqueue_prompt(m, kv, m->sched + done, rows, pos0 + at + done);
+            const bool first = at + done == 0;
+            if (wide && left > m->max_rows) rc = enqueue_prompt(m, kv, m->sched + done, rows, pos0 + at + done, first);
             else {                                           // a remainder that fits a verify block
                 rows = left < m->max_rows ? left : m->max_rows;
                 if (done) HIP_TRY(hipMemcpyAsync(m->sched, m->pin + 64 + done, (size_t)rows * 4, hipMemcpyHostToDevice, m->stream));   // (its kernels read the schedule from its start)
-                hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, m->stream, m->ctl, pos0 + at + done);
+                hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, m->stream, m->ctl, pos0 + at + done, first);
                 rc = wide ? enqueue_step_rows(m, kv, rows, false) : launch_step(m, kv, rows, false);    // (a single one: not worth a capture)
             }
             if (rc) return rc;
@@ -2170,7 +2175,7 @@ extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *tok
         at += part;
         HIP_TRY(hipStreamSynchronize(m->stream));
     }
-    return 0;
+    return step_err("prefill", __atomic_load_n(err, __ATOMIC_RELAXED));
 }
 
 extern "C" int lg_hip_tail_stamps(lg_hip_model *m, int which, unsigned long long *dst, int cap) {
@@ -2813,7 +2818,7 @@ extern "C" int lg_hip_attention_noalloc(const float *d_q, const uint16_t *d_kc, 
     hipStream_t st = (hipStream_t)stream;
     // every tile slot that the merge reads is written by the tile kernel of the same call, so nothing has to be
     // cleared; only the step state is set, by a kernel (a caller may be capturing this stream)
-    hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, st, ctl, pos);
+    hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, st, ctl, pos, true);
     switch (rows) {
 #define CASE(M) case M: rc = enqueue_attention<M>(st, a, g, ctl, tiles, pos, lds); break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)

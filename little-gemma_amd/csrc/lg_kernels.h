@@ -1014,8 +1014,8 @@ __global__ void lg_k_load(StepCtl *ctl, int32_t *sched, int pos, int rows, int r
     ctl->pos = pos; ctl->step = 0; ctl->err = 0; ctl->report = report;
 }
 
-// Prefill blocks skip the head: only the position advances.
-__global__ void lg_k_advance(StepCtl *ctl, int rows) { ctl->pos += rows; ctl->step += 1; }
+// Prefill blocks skip the head: the position advances, and the host, which waits for the stream, finds the error word.
+__global__ void lg_k_advance(StepCtl *ctl, int rows, int32_t *host) { ctl->pos += rows; ctl->step += 1; host[LG_REPORT_ERR] = ctl->err; }
 
 // Glue of a speculative round that stays on the device (the host loop it replaces: src/run.c:54-71): one thread
 // moves tokens between the draft head's and the target's step state, so that K chained drafts and the verify

@@ -1,0 +1,48 @@
+"""Launches whose workgroups wait for one another: a wait that is given up is reported by the call it happened in, and by no later one."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+W8 = dict(n_embd=768, n_head=8, head_dim=256, n_layer=2, n_ff=512, n_vocab=2048)
+
+
+@pytest.mark.parametrize("name,over,rows", [("tiny_full", {}, 1), ("tiny", W8, 2), ("tiny", W8, 3), ("tiny", W8, 8), ("tiny_full", {}, 4), ("tiny_full", {}, 5),
+                                            ("tiny", {"n_layer": 2, "n_ff": 8192, "n_embd": 2560}, 6)])
+def test_a_wait_given_up_is_reported_once(lg, ob, gpu_required, model_path, name, over, rows):
+    """One row of a narrow model, the attention output by v_dot4 and by the matrix cores, both forms of the layer tail, ffn_down over four
+    workgroups, each with no polls granted: a verify step, a schedule and prompts (in verify blocks, and with only the remainder in
+    one) return -9; with the polls back a prompt and a step are the oracle's."""
+    path, spec = model_path(name, **over)
+    rng = np.random.default_rng(rows)
+    V, n = spec["n_vocab"], 128 + rows                     # (one prompt block and a remainder)
+    toks = rng.integers(1, V, n).astype(np.int32)
+    blk = rng.integers(1, V, rows).astype(np.int32)
+    o = ob.Oracle(path)
+    gpu = lg.hiplib.HipBackend(path, n + 2 * rows, max_rows=max(rows, 4))
+    H = gpu.H
+    try:
+        out, adv = np.zeros(rows, np.int32), C.c_int32(0)
+        gpu.set_option("wait_polls", 0)
+        assert H.lg_hip_forward_spec(gpu.dev, gpu.dkv, blk, rows, 0, out, C.byref(adv)) == -9
+        assert b"given up" in H.lg_hip_last_error()
+        for wide, m in ((0, 2 * rows), (1, n)):
+            gpu.set_option("wide_prefill", wide)
+            print(f"{name} {over}: prompt of {m}, prompt blocks {wide}", flush=True)
+            assert H.lg_hip_prefill(gpu.dev, gpu.dkv, toks, m, 0) == -9
+        gpu.schedule(np.stack([blk, blk]), 0)
+        gpu.schedule_run(2)
+        with pytest.raises(lg.hiplib.HipError, match="given up"):
+            gpu.schedule_wait()
+        gpu.set_option("wait_polls", 1 << 16)
+        gpu.prefill(toks, 0)
+        okv = o.kv_new(n + 2 * rows, ob.I8)
+        o.prefill(okv, toks, 0, ob.I8)
+        got = gpu.forward_spec(blk, n)
+        want = o.forward_spec(okv, blk, n, ob.I8, want_hidden=True)
+        assert got[0] == want[0] and got[1].tolist()[:got[0]] == want[1].tolist()[:want[0]]
+        assert np.array_equal(gpu.last_hidden(spec["n_embd"]).view(np.uint32), want[2].view(np.uint32))
+    finally:
+        gpu.close(); o.close()
