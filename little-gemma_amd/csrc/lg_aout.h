@@ -27,7 +27,7 @@
 #define LG_AOUT_G (LG_AOUT_E / 8 / LG_XCD_WGS)     // row groups of a unit, a wavefront each
 #define LG_AOUT_DOT_ROWS 3          // widest block on v_dot4
 #define LG_AOUT_NV ((LG_AOUT_E + 1023) / 1024)     // float4 of a row per thread of 256
-struct AttnOutSync { uint32_t gen, pad[31]; uint2 w[LG_HIP_MAX_ROWS_DEV * LG_AOUT_K / 4]; uint4 s[LG_HIP_MAX_ROWS_DEV * LG_AOUT_K / 32]; uint2 o[LG_HIP_MAX_ROWS_DEV * LG_AOUT_E]; };
+struct AttnOutSync { uint2 w[LG_HIP_MAX_ROWS_DEV * LG_AOUT_K / 4]; uint4 s[LG_HIP_MAX_ROWS_DEV * LG_AOUT_K / 32]; uint2 o[LG_HIP_MAX_ROWS_DEV * LG_AOUT_E]; };
 static_assert(LG_AOUT_K == 64 * LG_XCD_WGS, "a merge of every row per unit");
 struct AttnOutArgs {
     MergeArgs      g;               // (xq, xf are not used)
@@ -38,11 +38,12 @@ struct AttnOutArgs {
     int            E, tiles;        // tiles: most that a row can see
     float          eps;
     AttnOutSync   *sync;
+    int            seq;             // number of this launch inside the step (the layer)
     int            spin_limit;
     unsigned long long *stamps;
 };
 #define LG_AOUT_FIELDS(X, v) X(const float *, pm, g.pm, v) X(const float *, pl, g.pl, v) X(const float *, pacc, g.pacc, v) X(int, tiles_max, g.tiles_max, v) \
-    X(int, H, g.H, v) X(int, hd, g.hd, v) X(int, window, g.window, v) X(int, tiles, tiles, v) X(const uint8_t *, wo, wo, v) X(AttnOutSync *, sync, sync, v) X(int, E, E, v) \
+    X(int, H, g.H, v) X(int, hd, g.hd, v) X(int, window, g.window, v) X(int, tiles, tiles, v) X(const uint8_t *, wo, wo, v) X(AttnOutSync *, sync, sync, v) X(int, seq, seq, v) X(int, E, E, v) \
     X(const float *, x, x, v) X(const float *, w_post, w_post, v) X(const float *, w_pre, w_pre, v) \
     X(float *, x_out, x_out, v) X(int8_t *, q, q, v) X(float, eps, eps, v) X(int, spin_limit, spin_limit, v) \
     X(unsigned long long *, stamps, stamps, v)
@@ -182,8 +183,7 @@ __global__ __launch_bounds__(64 * (LG_AOUT_G + M)) void lg_k_attn_out(StepCtl *c
     const int u = blockIdx.x >> 3, E = a.E, nq = E >> 2, slices = (E + 1023) >> 10;
     auto stamp = [&](int i) { if (a.stamps && t == 0) a.stamps[(size_t)u * 8 + i] = wall_clock64(); };
     stamp(0);
-    const uint32_t gen = a.sync->gen;
-    const uint32_t tag = lg_tag(gen, lg_xcc_id());
+    const uint32_t tag = lg_tag(ctl->launch + (uint32_t)a.seq, lg_xcc_id());
     AttnOutSync &y = *a.sync;
     int err = 0;
     const int ge = (wave - M) * LG_XCD_WGS + u;                // this wavefront's row group
@@ -263,7 +263,6 @@ __global__ __launch_bounds__(64 * (LG_AOUT_G + M)) void lg_k_attn_out(StepCtl *c
     stamp(4);
     row.work<false>(a, dv, jr, vr, rowt, t, red[0], red[1]);
     stamp(5);
-    if (u == 0 && t == 0) a.sync->gen = gen + 1;
 }
 
 // Blocks of 3..8 rows: wavefronts 0..3 of a unit merge rows w and w + 4, the other eight run a K segment each of the row blocks u, u + 32,
@@ -279,8 +278,7 @@ __global__ __launch_bounds__(768) void lg_k_attn_out_m(StepCtl *ctl, LG_AOUT_FIE
     const int u = blockIdx.x >> 3, E = a.E, nq = E >> 2, nrb = E >> 5, slices = (E + 1023) >> 10;
     auto stamp = [&](int i) { if (a.stamps && t == 0) a.stamps[(size_t)u * 8 + i] = wall_clock64(); };
     stamp(0);
-    const uint32_t gen = a.sync->gen;
-    const uint32_t tag = lg_tag(gen, lg_xcc_id());
+    const uint32_t tag = lg_tag(ctl->launch + (uint32_t)a.seq, lg_xcc_id());
     AttnOutSync &y = *a.sync;
     int err = 0;
     const int seg = wave - 4;
@@ -386,5 +384,4 @@ __global__ __launch_bounds__(768) void lg_k_attn_out_m(StepCtl *ctl, LG_AOUT_FIE
     stamp(4);
     row.work<(M > 3)>(a, dv, jr, vr, rowt, t, red[0], red[1]);
     stamp(5);
-    if (u == 0 && t == 0) a.sync->gen = gen + 1;
 }

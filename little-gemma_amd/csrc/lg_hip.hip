@@ -195,6 +195,7 @@ struct lg_hip_model {
     float eps = 0, base = 0, base_swa = 0, softcap = 0;
     std::vector<int> is_local, ffn_len, head_dim, n_head_kv;
     std::map<std::string, HostTensor> host;
+    bool numbered = false;             // every layer has a launch number of its own (StepCtl.launch): kernels whose workgroups wait for one another may run
     bool committed = false, wide_built = false;    // wide_built: the matrices' wide forms exist
     // weights
     std::vector<Layer> L;
@@ -240,7 +241,7 @@ struct lg_hip_model {
     uint2 *tgf = nullptr, *tpr = nullptr;    // [LG_HIP_MAX_ROWS][ple] and [LG_HIP_MAX_ROWS][E] its gated values and projections, tagged
     AttnOutSync *aosync = nullptr;           // hand-over state of lg_k_attn_out (models it serves)
     NarrowSync *nsync = nullptr;             // hand-over state of lg_k_narrow (models it serves: narrow_shape)
-    RgSync *rgsync = nullptr;                // flags and epoch base of lg_k_rows_geglu
+    RgSync *rgsync = nullptr;                // flags of lg_k_rows_geglu
     unsigned long long *tstamps = nullptr;   // [LG_XTAIL_UNITS][8] phase stamps of the last such launch (option xcd_tail_stamps)
     int tail_stamps = 0;
     int wait_polls = 1 << 16;                // option: polls after which a kernel gives up a hand-over inside its launch
@@ -293,6 +294,7 @@ extern "C" int lg_hip_model_create(const struct lg_hip_config *c, int device, lg
     if (cu_count() <= 0) return fail(-3, "model_create: device %d does not tell its number of compute units", device);      // (launches are cut by it)
     lg_hip_model *m = new lg_hip_model();
     m->device = device;
+    m->numbered = c->n_layer < LG_STEP_LAUNCHES;
     m->n_layer = c->n_layer; m->E = c->n_embd; m->H = c->n_head; m->n_vocab = c->n_vocab;
     m->window = c->sliding_window; m->ple = c->n_embd_per_layer; m->n_kv_start = c->n_kv_start;
     m->eps = c->rms_eps; m->base = c->rope_freq_base; m->base_swa = c->rope_freq_base_swa; m->softcap = c->logit_softcap;
@@ -539,7 +541,7 @@ static bool attn_tail_shape(int qd, int E, int *np, int *rbs) {
 
 // Models whose layers lg_k_narrow serves: what its registers, LDS and 256 wavefronts hold, q4_0 matrices throughout
 static bool narrow_shape(const lg_hip_model *m) {
-    if (cu_count() != LG_XCDS * LG_XCD_WGS || m->E % 256 || m->E > LG_NARROW_E || m->H > LG_NARROW_WGS || (m->ple && m->ple != 256)) return false;
+    if (!m->numbered || cu_count() != LG_XCDS * LG_XCD_WGS || m->E % 256 || m->E > LG_NARROW_E || m->H > LG_NARROW_WGS || (m->ple && m->ple != 256)) return false;
     for (const Layer &y : m->L)
         if (y.hd > LG_WG || y.hd % 64 || y.qd % 256 || y.qd > LG_NARROW_K || y.nff % 256 || y.nff > LG_NARROW_K || y.qkv_m % 8 || y.qkv_m > LG_NARROW_K ||
             !y.wqkv || !y.wo || !y.wgu || !y.wdown || (m->ple && (!y.winp || !y.wproj))) return false;
@@ -548,7 +550,7 @@ static bool narrow_shape(const lg_hip_model *m) {
 
 // Layers that lg_k_attn_out serves.  (Rows of up to 512 values: lg_k_narrow, or launches as short as this one.)
 static bool attn_out_shape(const lg_hip_model *m, const Layer &y) {
-    return m->E > LG_NARROW_E && m->E <= LG_AOUT_E && m->E % 256 == 0 && y.qd == LG_AOUT_K && y.hd % 64 == 0 && y.wo;
+    return m->numbered && m->E > LG_NARROW_E && m->E <= LG_AOUT_E && m->E % 256 == 0 && y.qd == LG_AOUT_K && y.hd % 64 == 0 && y.wo;
 }
 
 static const float *rope_table(lg_hip_model *m, int is_local, int hd, int *rc) {
@@ -1182,7 +1184,7 @@ static void launch_xffn(Launcher &lx, const XffnArgs &a, int cls) {
 // The per-layer-input block of a verify block of `rows` rows as the one-XCD launch lg_k_ple_tail: q4_0 matrices of the
 // 256-wide per-layer input, at most LG_XTAIL_UNITS (gate block, row) units, a chip whose workgroups are dealt over 8 XCDs
 static bool use_ple_tail(const lg_hip_model *m, int rows) {
-    if (!m->ple || !m->tsync || m->xcd_tail <= 0 || m->target) return false;
+    if (!m->ple || !m->tsync || !m->numbered || m->xcd_tail <= 0 || m->target) return false;
     if (m->ple != 256 || (m->ple / 32) * rows > LG_XTAIL_UNITS || m->E % 256 || m->E > 4096 || (m->E + 1023) / 1024 > m->ple / 32) return false;
     const int U = (m->ple / 32) * rows;
     const bool spread = m->tail_spread && (rows >= 5 || rows <= 2);   // (lg_k_ple_tail_s: 8 wavefronts per unit, enough of them at every width)
@@ -1246,7 +1248,7 @@ static bool use_attn_out(const lg_hip_model *m, const Layer &y, int rows, int ti
     return m->attn_out && m->aosync && attn_out_shape(m, y) && (rows <= LG_AOUT_DOT_ROWS ? tiles <= LG_AOUT_TILES : y.wo_ch && tiles <= LG_AOUT_BATCH);
 }
 static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
-    if (!y.wo_ch || !m->tsync || !attn_tail_shape(y.qd, m->E, nullptr, nullptr) || m->xcd_attn_tail <= 0 || (m->xcd_attn_tail == 1 && rows < 3)) return false;
+    if (!y.wo_ch || !m->tsync || !m->numbered || !attn_tail_shape(y.qd, m->E, nullptr, nullptr) || m->xcd_attn_tail <= 0 || (m->xcd_attn_tail == 1 && rows < 3)) return false;
     const int slices = (m->E + 1023) / 1024;
     return tiles < 128 && m->H * rows <= 2 * LG_XCD_WGS && slices * rows <= LG_XCD_WGS && y.hd % 32 == 0 && y.hd <= 256;
 }
@@ -1360,7 +1362,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         s.E = E; s.eps = m->eps; s.toks = m->sched; s.q = q_out ? q_out : m->hq;
         if (!have_x) {
             s.emb = m->emb; s.emb_seg = lg_segments(E); s.emb_nit = E / 32 / s.emb_seg; s.emb_scale = sqrtf((float)E);
-            if (m->rgsync) s.bump = &m->rgsync->base;          // the step's first kernel: a new range of epochs for lg_k_rows_geglu
+            s.bump = &m->ctl->launch;                          // the step's first kernel: a new range of launch numbers
         } else s.x = m->x[cur];
         s.dout = pend_dout; s.w_post = pend_w; s.os = pend_os; s.dparts = pend_parts;
         s.w_pre = w_pre; s.h_out = h_out;
@@ -1528,7 +1530,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 f.ipl = m->ple ? m->pmp_raw + (size_t)L * m->ple : nullptr;
                 f.qkv = m->qkv; f.h_out = last ? m->hidden_rows : nullptr; f.hq = m->hq;
                 f.E = E; f.qd = y.qd; f.FF = y.nff; f.qm = last ? 0 : m->L[L + 1].qkv_m; f.tiles = tiles; f.eps = m->eps;
-                f.sync = m->nsync; f.err = &m->ctl->err; f.err2 = draft ? &m->target->ctl->err : nullptr; f.spin_limit = m->wait_polls;
+                f.sync = m->nsync; f.seq = L; f.err = &m->ctl->err; f.err2 = draft ? &m->target->ctl->err : nullptr; f.spin_limit = m->wait_polls;
                 if (m->ple) LAUNCH(KC_TAIL, lg_k_narrow<true>, dim3(LG_XCDS * LG_NARROW_WGS), dim3(512), 0, f, m->ctl);
                 else        LAUNCH(KC_TAIL, lg_k_narrow<false>, dim3(LG_XCDS * LG_NARROW_WGS), dim3(512), 0, f, m->ctl);
                 cur ^= 1;
@@ -1542,7 +1544,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 f.g = g; f.wo = y.wo_ch; f.aq = (uint32_t *)m->aq; f.pout = m->dout;
                 f.x = m->x[cur]; f.w_post = y.post_attn; f.w_pre = y.ffn_norm; f.x_out = m->x[cur ^ 1];
                 f.q = m->hq; f.q_units = (M >= 4) ? 2 : 1; f.E = E; f.eps = m->eps;
-                f.sync = m->tsync; f.spin_limit = m->wait_polls; f.stamps = m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr;
+                f.sync = m->tsync; f.seq = L; f.spin_limit = m->wait_polls; f.stamps = m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr;
                 launch_attn_tail<M>(lx, f);
                 cur ^= 1;
                 pend_dout = pend_w = pend_os = nullptr; pend_parts = 1;
@@ -1552,7 +1554,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 const bool chains = M > LG_AOUT_DOT_ROWS || (M == LG_AOUT_DOT_ROWS && y.wo_ch && tiles <= LG_AOUT_BATCH);
                 AttnOutArgs f{};
                 f.g = g; f.wo = chains ? y.wo_ch : y.wo; f.x = m->x[cur]; f.w_post = y.post_attn; f.w_pre = y.ffn_norm; f.x_out = m->x[cur ^ 1];
-                f.q = m->hq; f.E = E; f.tiles = tiles; f.eps = m->eps; f.sync = m->aosync; f.spin_limit = m->wait_polls;
+                f.q = m->hq; f.E = E; f.tiles = tiles; f.eps = m->eps; f.sync = m->aosync; f.seq = L; f.spin_limit = m->wait_polls;
                 f.stamps = m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr;
                 if constexpr (M >= LG_AOUT_DOT_ROWS)
                     if (chains) LAUNCH(KC_ATAIL, lg_k_attn_out_m<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(768), 0, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
@@ -1586,7 +1588,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 // the whole half as one launch partitioned by XCD: row work, gate/up + GeGLU and the XCD's K share of
                 // ffn_down; the consumer adds the 8 slabs (the top of the segment tree)
                 XffnArgs f{ y.xgu, y.xdn, m->x[cur], pend_dout, pend_w, y.ffn_norm, m->x[cur ^ 1], m->slabs, m->xq8, m->xact,
-                            m->xsync, m->ctl, E, y.nff, m->eps, 4 * m->wait_polls, m->xffn_delay, nullptr };
+                            m->xsync, m->ctl, E, y.nff, m->eps, 4 * m->wait_polls, L, m->xffn_delay, nullptr };
                 launch_xffn<M>(lx, f, m->xffn_cls);
                 cur ^= 1;
                 pend_dout = m->slabs; pend_parts = LG_XCDS; pend_w = y.post_ffw; pend_os = m->ple ? nullptr : y.out_scale;
@@ -1598,8 +1600,8 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 // the row work as the first workgroups of the gate/up launch, whose other workgroups request their weights
                 // while it runs (lg_xrg.h); shapes whose K segment of E/256 tiles has a build
                 const int slices = (E + 1023) / 1024;
-                if (m->rows_geglu && m->rgsync && !ffn_rows_done && have_x && pend_dout && !pend_os && (pend_parts == 1 || pend_parts == 4) && (E == 2560 || E == 3840 || E == 512) &&
-                    M * slices <= LG_RG_MAXP && L < LG_RG_STEP - 1) {
+                if (m->rows_geglu && m->rgsync && m->numbered && !ffn_rows_done && have_x && pend_dout && !pend_os && (pend_parts == 1 || pend_parts == 4) && (E == 2560 || E == 3840 || E == 512) &&
+                    M * slices <= LG_RG_MAXP) {
                     RowsGegluArgs f{ m->x[cur], pend_dout, pend_w, y.ffn_norm, m->x[cur ^ 1], m->hq, E, pend_parts, slices, m->eps,
                                      y.wgu, y.nff, m->gq, dn_m ? 2 : 0, m->rgsync, L, m->wait_polls, m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr };
                     const dim3 grid(M * slices + y.nff / 32);
@@ -1622,7 +1624,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             }
             MmArgs d{ y.wdown, y.nff, E, m->dout, m->gq, nullptr };
             if (dn_m) {
-                DownMArgs dm{ y.wdn_m, (const uint32_t *)m->gq, m->dout, E, y.nff, m->down_m == 1 ? m->dmsync : nullptr, m->ctl, m->wait_polls };
+                DownMArgs dm{ y.wdn_m, (const uint32_t *)m->gq, m->dout, E, y.nff, m->down_m == 1 && m->numbered ? m->dmsync : nullptr, m->ctl, m->wait_polls, L };
                 launch_down_m<M>(lx, dm);
                 pend_parts = dm.sync ? 1 : 4;
             } else
@@ -1660,7 +1662,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 f.w_pre = last ? m->output_norm : m->L[L + 1].attn_norm;
                 f.x_out = m->x[cur ^ 1]; f.h_out = last ? m->hidden_rows : nullptr;
                 f.q = m->hq; f.q_units = last && head_m ? 2 : 0;
-                f.sync = m->tsync; f.spin_limit = m->wait_polls; f.stamps = m->tail_stamps ? m->tstamps : nullptr;
+                f.seq = L; f.spin_limit = m->wait_polls; f.stamps = m->tail_stamps ? m->tstamps : nullptr;
                 f.gf = m->tgf;
                 launch_ple_tail<M>(lx, f);
                 cur ^= 1;
@@ -2230,8 +2232,8 @@ extern "C" int lg_hip_schedule_load(lg_hip_model *m, const int32_t *toks, int n_
     HIP_TRY(hipSetDevice(m->device));
     HIP_TRY(hipStreamSynchronize(m->stream));
     HIP_TRY(hipMemcpy(m->sched, toks, (size_t)n_steps * rows * 4, hipMemcpyHostToDevice));
-    StepCtl c{ pos0, 0, 0, 0 };
-    HIP_TRY(hipMemcpy(m->ctl, &c, sizeof c, hipMemcpyHostToDevice));
+    StepCtl c{ pos0, 0, 0, 0, 0 };
+    HIP_TRY(hipMemcpy(m->ctl, &c, offsetof(StepCtl, launch), hipMemcpyHostToDevice));
     m->sched_steps = n_steps; m->sched_rows = rows; m->sched_pos0 = pos0; m->sched_loaded = n_steps;
     return 0;
 }
@@ -2711,7 +2713,7 @@ extern "C" int lg_hip_attention(const float *q, const uint16_t *kc, const uint16
     HIP_TRY(hipMemcpy(dq, q, (size_t)rows * qd * 4, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(dk, kc, (size_t)seq * kd * 2, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(dv, vc, (size_t)seq * kd * 2, hipMemcpyHostToDevice));
-    StepCtl c{ pos, 0, 0, 0 };
+    StepCtl c{ pos, 0, 0, 0, 0 };
     HIP_TRY(hipMemcpy(ctl, &c, sizeof c, hipMemcpyHostToDevice));
     AttnArgs a{};
     a.q = dq; a.H = n_head; a.nkv = n_head_kv; a.hd = hd;
@@ -2963,13 +2965,14 @@ extern "C" int lg_hip_down_m(const float *act, const void *down, int rows, int E
     lg_hip_model shim;
     shim.stream = st;
     Launcher lx{ &shim, false };
-    DownMArgs a{ dw, dq, dslabs, E, FF, join ? dsync : nullptr, ctl, 1 << 16 };
+    DownMArgs a{ dw, dq, dslabs, E, FF, join ? dsync : nullptr, ctl, 1 << 16, 0 };
     hipEvent_t e0 = nullptr, e1 = nullptr;
     auto body = [&]() -> int {
         HIP_TRY(hipEventCreate(&e0)); HIP_TRY(hipEventCreate(&e1));
         hipLaunchKernelGGL(lg_k_quant_mu, dim3((rows * (FF / 32) * 8 + LG_WG - 1) / LG_WG), dim3(LG_WG), 0, st, dx, rows, FF, dq);
         for (int r = 0; r < repeats + 1 && !lx.rc; ++r) {
             if (r == 1) HIP_TRY(hipEventRecord(e0, st));
+            a.seq = r;
             switch (rows) {
 #define CASE(M) case M: launch_down_m<M>(lx, a); break;
                 CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
@@ -3108,13 +3111,14 @@ extern "C" int lg_hip_ffn_xcd(const float *x, const float *dout, const float *w_
     if (flush_mb > 0 && sc.get(&dflush, (size_t)flush_mb << 20)) return -7;
     if (stamps && sc.get(&dstamps, (size_t)512 * LG_XFFN_STAMPS)) return -7;
     if (dstamps) HIP_TRY(hipMemset(dstamps, 0, (size_t)512 * LG_XFFN_STAMPS * 8));
-    XffnArgs f{ dgu, ddn, dx, dd, dwp, dwr, dxo, dslabs, dxq, dact, dsync, ctl, E, FF, eps, 1 << 16, delay_w, dstamps };
+    XffnArgs f{ dgu, ddn, dx, dd, dwp, dwr, dxo, dslabs, dxq, dact, dsync, ctl, E, FF, eps, 1 << 16, 0, delay_w, dstamps };
     hipEvent_t e0 = nullptr, e1 = nullptr;
     auto body = [&]() -> int {
         HIP_TRY(hipEventCreate(&e0)); HIP_TRY(hipEventCreate(&e1));
         for (int r = 0; r < repeats + 1 && !lx.rc; ++r) {
             if (r == 1) HIP_TRY(hipEventRecord(e0, st));
             if (dflush) HIP_TRY(hipMemsetAsync(dflush, r, (size_t)flush_mb << 20, st));
+            f.seq = r;
             switch (rows) {
 #define CASE(M) case M: launch_xffn<M>(lx, f, cls); break;
                 CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)

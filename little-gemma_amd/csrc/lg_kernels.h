@@ -17,7 +17,12 @@ struct StepCtl {            // device-resident step state
     int step;               // index of the current block in the token schedule
     int err;
     int report;             // not 0: the step's results also go to the host's memory, with this value behind them (lg_k_accept)
+    uint32_t launch;        // number of the step's first launch: advanced by LG_STEP_LAUNCHES by the step's first kernel (RowArgs.bump,
+                            // lg_k_draft_input) and by nothing else.  A launch whose workgroups wait for one another marks what it hands over with
+                            // launch + its layer: no earlier launch has used that number, and every workgroup of the launch finds the same one
+                            // whenever it starts, also when another of them has given up its wait and left
 };
+#define LG_STEP_LAUNCHES 256 // more than the layers of a model that has such launches
 
 // ---------------------------------------------------------------------------------------------
 // Row kernel: everything that happens to the M residual rows between two matmuls, one wavefront
@@ -53,9 +58,8 @@ struct RowArgs {
     int            E;
     float          eps;
     int            slices;   // workgroups per row (gridDim.y): as an argument it arrives with the others, the launch dimensions need a load of their own
-    uint32_t      *bump;     // nullptr, or a counter that the launch advances by LG_RG_STEP (the step's first kernel: epochs of lg_k_rows_geglu)
+    uint32_t      *bump;     // nullptr, or StepCtl.launch, which the launch advances (the step's first kernel)
 };
-#define LG_RG_STEP 256       // more than the launches of a step
 #define LG_ROW_FIELDS(X, v) X(const float *, x, x, v) X(const float *, dout, dout, v) X(const float *, w_post, w_post, v) X(const float *, w_pre, w_pre, v) X(int, E, E, v) X(int, dparts, dparts, v) X(int, slices, slices, v) X(const float *, os, os, v) X(float *, x_out, x_out, v) X(float *, h_out, h_out, v) X(int8_t *, q, q, v) X(int, q_units, q_units, v) X(float, eps, eps, v) X(const uint8_t *, emb, emb, v) X(const int32_t *, toks, toks, v) X(int, emb_nit, emb_nit, v) X(int, emb_seg, emb_seg, v) X(float, emb_scale, emb_scale, v) X(uint32_t *, bump, bump, v)
 
 // Sum over the 256 lanes of a workgroup in adjacent-pair tree order; every thread gets the result.
@@ -92,7 +96,7 @@ __global__ __launch_bounds__(LG_WG) void lg_k_rows(const StepCtl *ctl, LG_ROW_FI
     // float4 t + 256*y of each lane (the tail of the kernel is the longest part of it and splits freely)
     const int vs = s.slices > 1 ? (int)blockIdx.y : -1;
     const int E = s.E, nq = E >> 2;                          // float4 quads in a row; thread t owns quads t + 256*v
-    if (s.bump && blockIdx.x == 0 && blockIdx.y == 0 && t == 0) *s.bump += LG_RG_STEP;
+    if (s.bump && blockIdx.x == 0 && blockIdx.y == 0 && t == 0) *s.bump += LG_STEP_LAUNCHES;
     float4 xv[LG_ROWV], dv[LG_ROWV], wpost[LG_ROWV], wpre[LG_ROWV];
     // issue every load up front: one memory round trip for the whole row
     if (!s.x) {                                              // (rows that are token lookups have no residual yet)
@@ -281,8 +285,9 @@ struct DraftInArgs {
     int            nb;
     int8_t        *q;           // q8 activation buffer, one row of 2*nb
 };
-__global__ __launch_bounds__(LG_WG) void lg_k_draft_input(DraftInArgs a, const StepCtl *ctl) {
+__global__ __launch_bounds__(LG_WG) void lg_k_draft_input(DraftInArgs a, StepCtl *ctl) {
     const int quad = blockIdx.x * LG_WG + threadIdx.x, k = 2 * a.nb;
+    if (quad == 0) ctl->launch += LG_STEP_LAUNCHES;
     if (quad >= (k >> 2)) return;                            // k is a multiple of 256: whole wavefronts leave
     const int e = quad << 2;
     float4 v;

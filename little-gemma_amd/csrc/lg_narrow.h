@@ -27,7 +27,7 @@
 #define LG_NARROW_ONE 32            // ... by one wavefront
 // q8 rows as (4 values, tag) in the order of lg_act_layout and (scale, tag, sum, tag) a block; rows as (float, tag)
 struct NarrowQ8 { uint2 w[LG_NARROW_K / 4]; uint4 s[LG_NARROW_K / 32]; };
-struct NarrowSync { uint32_t gen, pad[31]; NarrowQ8 attn, act; uint2 o[LG_NARROW_E], d[LG_NARROW_E], pr[LG_NARROW_E], gf[256]; };
+struct NarrowSync { NarrowQ8 attn, act; uint2 o[LG_NARROW_E], d[LG_NARROW_E], pr[LG_NARROW_E], gf[256]; };
 struct NarrowArgs {
     MergeArgs      g;               // (xq, xf are not used)
     const float   *x;               // [E] residual
@@ -38,6 +38,7 @@ struct NarrowArgs {
     int            E, qd, FF, qm, tiles;      // tiles: most that the row can see
     float          eps;
     NarrowSync    *sync;
+    int            seq;             // number of this launch inside the step (the layer)
     int           *err, *err2;      // StepCtl.err of the model and (a draft head) of its target, or nullptr
     int            spin_limit;
 };
@@ -52,8 +53,7 @@ __global__ __launch_bounds__(512, 2) void lg_k_narrow(NarrowArgs a, const StepCt
     const bool rowt = t < nq;                                  // threads of the row work: a float4 of the row each (lane order of lg_k_rows)
     const int ge = u + LG_NARROW_WGS * (7 - wave);             // this wavefront's row group of 8 in every matmul (wavefront 0 merges: it has one last)
     const bool eg = ge < (E >> 3), qg = a.wq && ge < (a.qm >> 3);
-    const uint32_t gen = a.sync->gen;
-    const uint32_t tag = lg_tag(gen, lg_xcc_id());
+    const uint32_t tag = lg_tag(ctl->launch + (uint32_t)a.seq, lg_xcc_id());
 
     // every load that depends on nothing
     struct Tiles { uint4 q[8]; uint32_t s[8]; } to, td;        // output, down
@@ -302,5 +302,4 @@ __global__ __launch_bounds__(512, 2) void lg_k_narrow(NarrowArgs a, const StepCt
         }
     }
     if (err) { atomicOr(a.err, err); if (a.err2) atomicOr(a.err2, err); }
-    if (u == 0 && t == 0) y.gen = gen + 1;
 }

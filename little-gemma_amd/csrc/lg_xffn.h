@@ -44,8 +44,7 @@
 #include "lg_xcd.h"
 
 struct XcdSync {
-    uint32_t gen[LG_XCDS];                       // per group: launches so far (advanced by rank 0 at the end of a launch)
-    uint32_t flags[LG_XCDS][2][LG_XCD_WGS];      // per group and hand-over: (epoch << 4 | XCD id) of each rank's last arrival; epoch = 2 * gen + 1, + 2
+    uint32_t flags[LG_XCDS][2][LG_XCD_WGS];      // per group and hand-over: lg_tag of each rank's last arrival
 };
 
 struct XffnGeo {
@@ -98,10 +97,11 @@ struct XffnArgs {
     int E, FF;
     float eps;
     int spin_limit;
+    int seq;                       // number of this launch inside the step
     int delay_w;                   // the compute wavefronts sleep this many units of 64 clocks before they request their weights (the rows' loads go first)
     unsigned long long *stamps;    // nullptr, or [256][LG_XFFN_STAMPS] device wall-clock ticks at the phase boundaries of every workgroup (measurement runs)
 };
-#define LG_XFFN_FIELDS(X, v) X(const uint8_t *, wgu, wgu, v) X(const float *, x, x, v) X(const float *, dout, dout, v) X(const float *, w_post, w_post, v) X(const float *, w_pre, w_pre, v) X(int, E, E, v) X(int, FF, FF, v) X(XcdSync *, sync, sync, v) X(const uint8_t *, wdn, wdn, v) X(float *, x_out, x_out, v) X(float *, slabs, slabs, v) X(uint32_t *, xq, xq, v) X(float *, act, act, v) X(StepCtl *, ctl, ctl, v) X(float, eps, eps, v) X(int, spin_limit, spin_limit, v) X(int, delay_w, delay_w, v) X(unsigned long long *, stamps, stamps, v)
+#define LG_XFFN_FIELDS(X, v) X(const uint8_t *, wgu, wgu, v) X(const float *, x, x, v) X(const float *, dout, dout, v) X(const float *, w_post, w_post, v) X(const float *, w_pre, w_pre, v) X(int, E, E, v) X(int, FF, FF, v) X(XcdSync *, sync, sync, v) X(const uint8_t *, wdn, wdn, v) X(float *, x_out, x_out, v) X(float *, slabs, slabs, v) X(uint32_t *, xq, xq, v) X(float *, act, act, v) X(StepCtl *, ctl, ctl, v) X(float, eps, eps, v) X(int, spin_limit, spin_limit, v) X(int, seq, seq, v) X(int, delay_w, delay_w, v) X(unsigned long long *, stamps, stamps, v)
 #define LG_XFFN_STAMPS 16
 #define LG_XFFN_THREADS 768        // 8 compute wavefronts, 4 for the row work (the first of them serves the hand-overs)
 
@@ -115,16 +115,18 @@ __device__ __forceinline__ unsigned long long lg_ld_l2_u64(const void *p) {
     return __hip_atomic_load((const unsigned long long *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// What a workgroup of launch `number` (StepCtl.launch + its number inside the step) on XCD `xcc` marks its flags and values with
+__device__ __forceinline__ uint32_t lg_tag(uint32_t number, int xcc) { return ((number + 1) << 4) | (uint32_t)xcc; }
+
 // The hand-over wavefront's side of a flag barrier: publish this rank's arrival (its stores have been waited for),
-// then poll the flags of ranks 0..n-1 (lane i polls flag i) until all have reached `epoch`.  Returns 0, or the error
+// then poll the flags of ranks 0..n-1 (lane i polls flag i) until all hold the launch's number.  Returns 0, or the error
 // bits: a flag written from another XCD, or the bounded wait given up.
-__device__ __forceinline__ int lg_xcd_arrive_wait(uint32_t *flags, int rank, bool arrive, int n, uint32_t epoch, int xcc, int spin_limit) {
+__device__ __forceinline__ int lg_xcd_arrive_wait(uint32_t *flags, int rank, bool arrive, int n, uint32_t tag, int spin_limit) {
     const int lane = threadIdx.x & 63;
-    if (arrive && lane == 0) lg_st_sc<0>(flags + rank, (epoch << 4) | (uint32_t)xcc);
+    if (arrive && lane == 0) lg_st_sc<0>(flags + rank, tag);
     for (int spins = 0; spins < spin_limit; ++spins) {
-        const uint32_t f = lane < n ? lg_ld_sc<2>(flags + lane) : ((epoch << 4) | (uint32_t)xcc);
-        const bool there = (int)(((f >> 4) - epoch) << 4) >= 0;              // epochs are 28-bit counters that wrap
-        if (__all(there)) return __any((int)(f & 15) != xcc) ? LG_XFFN_ERR_PLACE : 0;
+        const uint32_t diff = (lane < n ? lg_ld_sc<2>(flags + lane) : tag) ^ tag;
+        if (__all((diff >> 4) == 0)) return __any(diff != 0) ? LG_XFFN_ERR_PLACE : 0;
     }
     return LG_XFFN_ERR_WAIT;
 }
@@ -321,9 +323,9 @@ __global__ __launch_bounds__(LG_XFFN_THREADS) void lg_k_ffn_xcd(LG_XFFN_FIELDS(L
         // ================= the row-work wavefronts: everything that is handed over through memory =================
         if (a.delay_w & 0x100) __builtin_amdgcn_s_setprio(3);        // (their few instructions ahead of the others')
         const int tt = t - 512;                                       // 0..255: the thread index of lg_k_rows
-        uint32_t uses = 0, gen = 0;
-        int xcc = 0, err = 0;
-        const uint32_t *genp = a.sync->gen + x;
+        uint32_t uses = 0, tag = 0;
+        int err = 0;
+        if (service) tag = lg_tag(a.ctl->launch + (uint32_t)a.seq, lg_xcc_id());
         if (row_wg) {
             // ---- A: this workgroup's row (the arithmetic and the lane assignment of lg_k_rows); its q8 goes to LDS in
             //      the 80-dword block order, from where the first of these wavefronts publishes it
@@ -335,7 +337,6 @@ __global__ __launch_bounds__(LG_XFFN_THREADS) void lg_k_ffn_xcd(LG_XFFN_FIELDS(L
                 #pragma unroll
                 for (int v = 0; v < LG_ROWV; ++v) if (tt + 256 * v < nq) { xv[v] = xr[tt + 256 * v]; dv[v] = dr[tt + 256 * v]; wpost[v] = wo[tt + 256 * v]; wpre[v] = wp[tt + 256 * v]; }
             }
-            if (service) gen = __hip_atomic_load(genp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // (behind the row's loads: it is needed after them)
             stamp(11);
             float ss = 0.0f;
             #pragma unroll
@@ -387,13 +388,10 @@ __global__ __launch_bounds__(LG_XFFN_THREADS) void lg_k_ffn_xcd(LG_XFFN_FIELDS(L
                 lg_wait_vm();                                         // the row is in the group's L2
             }
             stamp(15);
-        } else if (service) gen = lg_ld_sc<2>(genp);
+        }
         // ---- A -> B: the first wavefront publishes and polls, the others wait for it; then all four copy the group's
         //      q8 rows into LDS for the compute wavefronts
-        if (service) {
-            xcc = lg_xcc_id();
-            err |= lg_xcd_arrive_wait(flags1, r, row_wg, M, 2 * gen + 1, xcc, a.spin_limit);
-        }
+        if (service) err |= lg_xcd_arrive_wait(flags1, r, row_wg, M, tag, a.spin_limit);
         stamp(2);
         lg_rowsync(&rcnt, uses);
         {
@@ -425,7 +423,7 @@ __global__ __launch_bounds__(LG_XFFN_THREADS) void lg_k_ffn_xcd(LG_XFFN_FIELDS(L
             for (int i = lane; i < M * g.CW; i += 64) { const int j = i / g.CW; act[(size_t)j * g.C + r * g.CW + (i - j * g.CW)] = actbuf[i]; }
             lg_wait_vm();
             stamp(6);
-            err |= lg_xcd_arrive_wait(flags2, r, true, LG_XCD_WGS, 2 * gen + 2, xcc, a.spin_limit);
+            err |= lg_xcd_arrive_wait(flags2, r, true, LG_XCD_WGS, tag, a.spin_limit);
         }
         lg_rowsync(&rcnt, uses);
         stamp(7);
@@ -458,10 +456,7 @@ __global__ __launch_bounds__(LG_XFFN_THREADS) void lg_k_ffn_xcd(LG_XFFN_FIELDS(L
         }
         stamp(8);
         __syncthreads();                                              // (#3)
-        if (service && lane == 0) {
-            if (r == 0) lg_st_sc<0>(a.sync->gen + x, gen + 1);        // every rank of the group has read gen long ago (it passed B -> C)
-            if (err) atomicOr(&a.ctl->err, err);
-        }
+        if (service && lane == 0 && err) atomicOr(&a.ctl->err, err);
     }
     __syncthreads();                                                  // (#4: the chain sums of ffn_down are in LDS)
     for (int idx = t; idx < M * g.RW; idx += LG_XFFN_THREADS) {       // the group's levels of the segment tree, slab x
@@ -512,8 +507,7 @@ __host__ __device__ static inline DownMGeo lg_down_m_geo(int E, int FF) {
 // then holds the whole sums and the consumer reads a quarter of the bytes.  Only quarter 0 waits, for workgroups that
 // wait for nobody, so no residency is assumed; the wait is bounded and a flag from another XCD is reported (StepCtl.err).
 struct DownMSync {
-    uint32_t gen[64];            // per row group: launches so far (advanced by its quarter 0 once it has seen the flags)
-    uint32_t flags[64][4];       // (epoch << 4 | XCD id) of the quarter's last arrival, epoch = gen + 1
+    uint32_t flags[64][4];       // lg_tag of the quarter's last arrival
 };
 struct DownMArgs {
     const uint8_t *w;        // [256][wg_bytes]
@@ -523,9 +517,10 @@ struct DownMArgs {
     DownMSync *sync;         // nullptr: leave four slabs to the consumer
     StepCtl *ctl;
     int spin_limit;
+    int seq;                 // number of this launch inside the step
 };
 #define LG_DOWNM_FIELDS(X, v) X(const uint8_t *, w, w, v) X(const uint32_t *, act, act, v) X(int, E, E, v) X(int, FF, FF, v) X(float *, slabs, slabs, v) \
-    X(DownMSync *, sync, sync, v) X(StepCtl *, ctl, ctl, v) X(int, spin_limit, spin_limit, v)
+    X(DownMSync *, sync, sync, v) X(StepCtl *, ctl, ctl, v) X(int, spin_limit, spin_limit, v) X(int, seq, seq, v)
 // M: rows of the block; OPS: operands of 32 rows per workgroup; NDP: capacity in pairs of blocks of a segment.
 template <int M, int OPS, int NDP>
 __global__ __launch_bounds__(512) void lg_k_down_m(LG_DOWNM_FIELDS(LG_XP, _) int p_end_) {
@@ -535,7 +530,7 @@ __global__ __launch_bounds__(512) void lg_k_down_m(LG_DOWNM_FIELDS(LG_XP, _) int
     const int wg = blockIdx.x, r = wg & 63, q = wg >> 6;
     const int t = threadIdx.x, lane = t & 63, n = lane & 31, h = lane >> 5;
     const int s = __builtin_amdgcn_readfirstlane(t >> 6);             // segment 8q + s
-    const uint32_t gen = a.sync ? a.sync->gen[r] : 0u;
+    const uint32_t number = a.ctl->launch + (uint32_t)a.seq;
     unsigned char *la = smem + (size_t)s * g.nitd * (LG_MU_DWORDS * 4);                          // this wavefront's blocks
     float *red = (float *)(smem + (size_t)8 * g.nitd * (LG_MU_DWORDS * 4));                      // [8 segments][OPS][8 row slots][32]
     // the activation blocks of the segment first (they come from nearer), then the whole chain's weights
@@ -606,23 +601,20 @@ __global__ __launch_bounds__(512) void lg_k_down_m(LG_DOWNM_FIELDS(LG_XP, _) int
     }
     if (!a.sync) return;
     // ---- the row group's four slabs added here ----
-    const int xcc = lg_xcc_id();
-    const uint32_t epoch = gen + 1;
+    const uint32_t tag = lg_tag(number, lg_xcc_id());
     if (q != 0) {
         lg_wait_vm();
         __syncthreads();
-        if (t == 0) lg_st_sc<0>(&a.sync->flags[r][q], (epoch << 4) | (uint32_t)xcc);
+        if (t == 0) lg_st_sc<0>(&a.sync->flags[r][q], tag);
         return;
     }
     if (s == 0) {
         int err = LG_XFFN_ERR_WAIT;
         for (int spins = 0; spins < a.spin_limit; ++spins) {
-            const uint32_t f = (lane >= 1 && lane < 4) ? lg_ld_sc<2>(&a.sync->flags[r][lane]) : ((epoch << 4) | (uint32_t)xcc);
-            const bool there = (int)(((f >> 4) - epoch) << 4) >= 0;
-            if (__all(there)) { err = __any((int)(f & 15) != xcc) ? LG_XFFN_ERR_PLACE : 0; break; }
+            const uint32_t diff = ((lane >= 1 && lane < 4) ? lg_ld_sc<2>(&a.sync->flags[r][lane]) : tag) ^ tag;
+            if (__all((diff >> 4) == 0)) { err = __any(diff != 0) ? LG_XFFN_ERR_PLACE : 0; break; }
         }
         if (err && lane == 0) atomicOr(&a.ctl->err, err);
-        if (lane == 0) a.sync->gen[r] = epoch;
     }
     __syncthreads();
     if (on) {

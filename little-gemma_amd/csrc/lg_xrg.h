@@ -26,10 +26,7 @@
 // (acknowledged stores, flag, poll, load: four round trips) costs more than the kernel boundary it replaces, whose
 // launch gap the graph hides anyway.  Bit-identical; kept as an option, off (`rows_geglu`).
 //
-// A flag holds an epoch that no earlier launch has used: base + seq + 1, where `base` is advanced once per step by
-// the step's first kernel (the embedding rows: RowArgs.bump) and seq is the launch's number inside the step (the
-// layer).  Nothing changes `base` while a step's launches run, so every workgroup of a launch computes the same
-// epoch whenever it starts.
+// A flag holds an epoch that no earlier launch has used: StepCtl.launch + the launch's number inside the step + 1.
 #pragma once
 #include "lg_kernels.h"
 #include "lg_xcd.h"
@@ -40,8 +37,6 @@
 #define LG_RG_COPIES 32             // copies of the flags, a 128-byte line each: a gate/up workgroup polls copy (id % 32), so that
                                     // the polls of some hundred workgroups do not all queue at one memory channel
 struct RgSync {
-    uint32_t base;
-    uint32_t pad[31];
     uint32_t flags[LG_RG_COPIES][LG_RG_MAXP];
 };
 struct RowsGegluArgs {
@@ -71,7 +66,7 @@ __global__ __launch_bounds__(512, 4) void lg_k_rows_geglu(StepCtl *ctl, LG_RG_FI
     extern __shared__ __align__(16) unsigned char smem[];     // gate/up workgroups: [8 segments][NIT][80 dwords]
     __shared__ float red[8][LG_HIP_MAX_ROWS_DEV][64];
     const int P = M * a.slices;
-    const uint32_t epoch = a.sync->base + (uint32_t)a.seq + 1u;
+    const uint32_t epoch = ctl->launch + (uint32_t)a.seq + 1u;
     const int E = a.E;
     if ((int)blockIdx.x < P) {
         // ---- a row workgroup: row j, storing and quantizing the float4s t + 256 vs of every lane (lg_k_rows with a

@@ -32,10 +32,7 @@
 
 #define LG_XTAIL_UNITS 64           // most units of a launch (lane i of a wavefront polls flag i)
 struct XtailSync {
-    uint32_t gen;                   // launches so far (advanced by unit 0 at the end of a launch, when every unit has read it: unit 0 has taken
-                                    // values that all of them tagged); tag (gen + 1, XCD id), flags' epochs 2 gen + 1, + 2
-    uint32_t pad[31];
-    uint32_t flags[2][LG_XTAIL_UNITS];      // lg_k_attn_tail
+    uint32_t flags[2][LG_XTAIL_UNITS];      // lg_k_attn_tail: lg_tag of each unit's last arrival
 };
 
 struct XtailArgs {
@@ -47,13 +44,13 @@ struct XtailArgs {
     float         *x_out, *h_out;   // [M][E] new residual; normed rows before quantization, or nullptr
     int8_t        *q;               // q8 activation buffer of the result
     int            q_units;         // 0: rows in the order of lg_act_layout; 2: the 80-dword blocks of lg_k_geglu_m
-    XtailSync     *sync;
+    int            seq;             // number of this launch inside the step (the layer)
     int            spin_limit;
     unsigned long long *stamps;     // nullptr, or [LG_XTAIL_UNITS][8] device wall-clock ticks at the phase boundaries of every unit (measurement runs)
     uint2         *gf;              // [M][ple] the gated values as tagged floats (handed from phase 1 to phase 2 through the XCD's L2)
 };
 #define LG_XTAIL_FIELDS(X, v) X(const float *, x, r.x, v) X(const float *, dout, r.dout, v) X(const float *, w_post, r.w_post, v) X(const uint8_t *, gw, r.g.w, v) \
-    X(int, gk, r.g.k, v) X(int, gple, r.g.ple, v) X(int, dparts, r.dparts, v) X(XtailSync *, sync, sync, v) X(const float *, gipl, r.g.ipl, v) X(int, glayer, r.g.layer, v) \
+    X(int, gk, r.g.k, v) X(int, gple, r.g.ple, v) X(int, dparts, r.dparts, v) X(int, seq, seq, v) X(const float *, gipl, r.g.ipl, v) X(int, glayer, r.g.layer, v) \
     X(int, gnl, r.g.n_layer, v) X(int8_t *, gpq, r.g.pq, v) X(const uint8_t *, pw, pw, v) X(const float *, w_post2, w_post2, v) X(const float *, w_pre, w_pre, v) \
     X(const float *, os, os, v) X(uint2 *, pout, pout, v) X(float *, x_out, x_out, v) X(float *, h_out, h_out, v) X(int8_t *, q, q, v) X(int, q_units, q_units, v) \
     X(float, eps, r.eps, v) X(int, spin_limit, spin_limit, v) X(unsigned long long *, stamps, stamps, v) X(uint2 *, gf, gf, v)
@@ -72,7 +69,6 @@ __device__ __forceinline__ void lg_units_wait(LgUnits<N> &r) {
     if constexpr (N == 6) asm volatile("s_waitcnt vmcnt(0)" : "+v"(r.v[0]), "+v"(r.v[1]), "+v"(r.v[2]), "+v"(r.v[3]), "+v"(r.v[4]), "+v"(r.v[5]) :: "memory");
     if constexpr (N == 8) asm volatile("s_waitcnt vmcnt(0)" : "+v"(r.v[0]), "+v"(r.v[1]), "+v"(r.v[2]), "+v"(r.v[3]), "+v"(r.v[4]), "+v"(r.v[5]), "+v"(r.v[6]), "+v"(r.v[7]) :: "memory");
 }
-__device__ __forceinline__ uint32_t lg_tag(uint32_t gen, int xcc) { return ((gen + 1) << 4) | (uint32_t)xcc; }
 template <int N, typename A>
 __device__ __forceinline__ LgUnits<N> lg_take(A &&addr, bool on, uint32_t tag, int spin_limit, int &err) {
     LgUnits<N> r;
@@ -127,10 +123,9 @@ __global__ __launch_bounds__(LG_WG) void lg_k_ple_tail(StepCtl *ctl, LG_XTAIL_FI
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int E = a.r.g.k, ple = a.r.g.ple, nblk = ple >> 5, U = nblk * M, nq = E >> 2;
     const int u = blockIdx.x >> 3, gb = u % nblk, j = u / nblk;
-    const uint32_t gen = a.sync->gen;
     auto stamp = [&](int i) { if (a.stamps && t == 0) a.stamps[(size_t)u * 8 + i] = wall_clock64(); };
     stamp(0);
-    const uint32_t tag = lg_tag(gen, lg_xcc_id());
+    const uint32_t tag = lg_tag(ctl->launch + (uint32_t)a.seq, lg_xcc_id());
     int err = 0;
     // ---- phase 1, with this kernel's later loads requested behind its own ----
     const int groups = E >> 3, waves = 4 * U, gw = u * 4 + wave;
@@ -240,7 +235,6 @@ __global__ __launch_bounds__(LG_WG) void lg_k_ple_tail(StepCtl *ctl, LG_XTAIL_FI
         }
     }
     stamp(7);
-    if (u == 0 && t == 0) a.sync->gen = gen + 1;
 }
 
 // the sum over the 256 lanes of wavefronts 0..3 (order of lg_block_sum256) in a workgroup of 8 wavefronts that all call it
@@ -277,10 +271,9 @@ __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FI
     const int cnt = gbase + (p < gextra ? 1 : 0), g0 = p * gbase + (p < gextra ? p : gextra);
     const bool gatew = wave < cnt;
     const int gg = g0 + (gatew ? wave : 0);                    // this wavefront's gate row group
-    const uint32_t gen = a.sync->gen;
     auto stamp = [&](int i) { if (a.stamps && t == 0) a.stamps[(size_t)u * 8 + i] = wall_clock64(); };
     stamp(0);
-    const uint32_t tag = lg_tag(gen, lg_xcc_id());
+    const uint32_t tag = lg_tag(ctl->launch + (uint32_t)a.seq, lg_xcc_id());
     int err = 0;
     int8_t *lq = (int8_t *)smem;                               // the row: [E] int8, then [E/32] {scale, sum}
     float2 *lds = (float2 *)(smem + (size_t)E);
@@ -482,7 +475,6 @@ __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FI
         }
     }
     stamp(7);
-    if (u == 0 && t == 0) a.sync->gen = gen + 1;
 }
 
 // A second form was built and measured, and is not kept: 32 units of 8 gate rows and 8 wavefronts whatever the block
@@ -527,13 +519,14 @@ struct XattnTailArgs {
     int            E;
     float          eps;
     XtailSync     *sync;
+    int            seq;          // number of this launch inside the step (the layer)
     int            spin_limit;
     unsigned long long *stamps;
 };
 #define LG_XATTN_FIELDS(X, v) X(const float *, pm, g.pm, v) X(const float *, pl, g.pl, v) X(const float *, pacc, g.pacc, v) X(int, tiles_max, g.tiles_max, v) \
     X(int, H, g.H, v) X(int, hd, g.hd, v) X(int, window, g.window, v) X(int, pos_off, g.pos_off, v) X(const uint8_t *, wo, wo, v) X(XtailSync *, sync, sync, v) \
     X(const float *, x, x, v) X(const float *, w_post, w_post, v) X(const float *, w_pre, w_pre, v) X(uint32_t *, aq, aq, v) X(float *, pout, pout, v) \
-    X(float *, x_out, x_out, v) X(int8_t *, q, q, v) X(int, q_units, q_units, v) X(int, E, E, v) X(float, eps, eps, v) X(int, spin_limit, spin_limit, v) \
+    X(float *, x_out, x_out, v) X(int8_t *, q, q, v) X(int, q_units, q_units, v) X(int, E, E, v) X(float, eps, eps, v) X(int, spin_limit, spin_limit, v) X(int, seq, seq, v) \
     X(unsigned long long *, stamps, stamps, v)
 
 // Row blocks of a unit whose weights are requested with the merge's partials; the rest after the merge.  All of them early
@@ -559,8 +552,7 @@ __global__ __launch_bounds__(512) void lg_k_attn_tail(StepCtl *ctl, LG_XATTN_FIE
     const int slices = (E + 1023) >> 10, nrow = slices * M;
     const bool rowunit = u < nrow, rowlane = t < LG_WG;
     const int v_ = u / M, jr = u - v_ * M;
-    const uint32_t gen = a.sync->gen;
-    const int xcc = lg_xcc_id();
+    const uint32_t tag = lg_tag(ctl->launch + (uint32_t)a.seq, lg_xcc_id());
     auto stamp = [&](int i) { if (a.stamps && t == 0) a.stamps[(size_t)u * 8 + i] = wall_clock64(); };
     stamp(0);
     lg_v16i magic;
@@ -608,7 +600,7 @@ __global__ __launch_bounds__(512) void lg_k_attn_tail(StepCtl *ctl, LG_XATTN_FIE
     lg_wait_vm();
     __syncthreads();
     if (wave == 0) {
-        const int err = lg_xcd_arrive_wait(a.sync->flags[0], u, u < nmerge, nmerge, 2 * gen + 1, xcc, a.spin_limit);
+        const int err = lg_xcd_arrive_wait(a.sync->flags[0], u, u < nmerge, nmerge, tag, a.spin_limit);
         if (err && lane == 0) atomicOr(&ctl->err, err);
     }
     __syncthreads();
@@ -674,11 +666,11 @@ __global__ __launch_bounds__(512) void lg_k_attn_tail(StepCtl *ctl, LG_XATTN_FIE
     lg_wait_vm();
     __syncthreads();
     if (!rowunit) {
-        if (t == 0) lg_st_sc<0>(a.sync->flags[1] + u, ((2 * gen + 2) << 4) | (uint32_t)xcc);
+        if (t == 0) lg_st_sc<0>(a.sync->flags[1] + u, tag);
         return;
     }
     if (wave == 0) {
-        const int err = lg_xcd_arrive_wait(a.sync->flags[1], u, true, U, 2 * gen + 2, xcc, a.spin_limit);
+        const int err = lg_xcd_arrive_wait(a.sync->flags[1], u, true, U, tag, a.spin_limit);
         if (err && lane == 0) atomicOr(&ctl->err, err);
     }
     __syncthreads();
@@ -757,5 +749,4 @@ __global__ __launch_bounds__(512) void lg_k_attn_tail(StepCtl *ctl, LG_XATTN_FIE
         }
     }
     stamp(7);
-    if (u == 0 && t == 0) a.sync->gen = gen + 1;
 }

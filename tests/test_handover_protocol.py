@@ -1,0 +1,63 @@
+"""The marks of a hand-over inside a launch, as a model on the CPU: units that start at any time, values that carry the launch's number, waits
+that are given up.  What a launch takes has to be of that launch, whatever became of the launches before it."""
+import itertools
+
+import pytest
+
+UNITS, WAIT, STEP = 4, 3, 16
+
+
+class Memory:
+    """One slot per unit (value, tag), the word that the number is read from, the error word of a step."""
+
+    def __init__(self):
+        self.slots, self.word, self.err = [(None, 0)] * UNITS, 0, False
+
+
+def unit(m, u, launch, delay, advances):
+    """One unit of launch `launch`: starts `delay` turns late, reads the launch's number, stores its value with it, takes every unit's."""
+    for _ in range(delay):
+        yield
+    tag = m.word + 1
+    yield
+    m.slots[u] = (launch, tag)
+    yield
+    for _ in range(WAIT):
+        if all(t == tag for _, t in m.slots):
+            taken = [v for v, _ in m.slots]
+            assert all(v == launch for v in taken) or m.err, f"unit {u} of launch {launch} took {taken} and nothing was reported"
+            break
+        yield
+    else:
+        m.err = True
+    if advances and u == 0:
+        m.word += 1
+
+
+def run_steps(advances):
+    """Steps of one launch each: one with units that start when the others have left, then one with units that start a little late."""
+    refused = 0
+    for late in itertools.product((0, 3 * WAIT), repeat=UNITS):
+        for behind in itertools.product((0, WAIT - 1), repeat=UNITS):
+            m = Memory()
+            for launch, delays in enumerate(((0,) * UNITS, late, behind)):
+                m.err = False
+                if not advances:
+                    m.word += STEP                                      # the step's first kernel: before any launch that waits
+                live = [unit(m, u, launch, delays[u], advances) for u in range(UNITS)]
+                while live:                                             # (a launch ends when all of its units have)
+                    live = [g for g in live if next(g, "left") != "left"]
+                refused += m.err
+    assert refused                                                      # (somebody gave up)
+
+
+def test_a_number_of_the_step_stays_with_its_launch():
+    """StepCtl.launch: advanced between launches only."""
+    run_steps(advances=False)
+
+
+def test_a_number_that_a_unit_advances_can_leave_its_launch():
+    """The model sees the fault it is there for: unit 0 gives up and advances the word, a unit that starts later marks its value with
+    the next launch's number, which the next launch takes for its own."""
+    with pytest.raises(AssertionError, match="nothing was reported"):
+        run_steps(advances=True)
