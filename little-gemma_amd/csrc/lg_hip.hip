@@ -1531,8 +1531,12 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 f.qkv = m->qkv; f.h_out = last ? m->hidden_rows : nullptr; f.hq = m->hq;
                 f.E = E; f.qd = y.qd; f.FF = y.nff; f.qm = last ? 0 : m->L[L + 1].qkv_m; f.tiles = tiles; f.eps = m->eps;
                 f.sync = m->nsync; f.seq = L; f.err = &m->ctl->err; f.err2 = draft ? &m->target->ctl->err : nullptr; f.spin_limit = m->wait_polls;
-                if (m->ple) LAUNCH(KC_TAIL, lg_k_narrow<true>, dim3(LG_XCDS * LG_NARROW_WGS), dim3(512), 0, f, m->ctl);
-                else        LAUNCH(KC_TAIL, lg_k_narrow<false>, dim3(LG_XCDS * LG_NARROW_WGS), dim3(512), 0, f, m->ctl);
+                const dim3 grid(LG_XCDS * LG_NARROW_WGS);
+                if (tiles > LG_NARROW_LONG) {
+                    if (m->ple) LAUNCH(KC_TAIL, (lg_k_narrow<true, true>), grid, dim3(512), 0, f, m->ctl);
+                    else        LAUNCH(KC_TAIL, (lg_k_narrow<false, true>), grid, dim3(512), 0, f, m->ctl);
+                } else if (m->ple) LAUNCH(KC_TAIL, (lg_k_narrow<true, false>), grid, dim3(512), 0, f, m->ctl);
+                else               LAUNCH(KC_TAIL, (lg_k_narrow<false, false>), grid, dim3(512), 0, f, m->ctl);
                 cur ^= 1;
                 rows_done = true; qkv_done = !last;
                 continue;

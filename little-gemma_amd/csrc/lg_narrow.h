@@ -23,8 +23,9 @@
 #define LG_NARROW_WGS 32            // one per CU of the XCD
 #define LG_NARROW_E 512             // widest row
 #define LG_NARROW_K 2048            // longest input of attn_output and ffn_down
-#define LG_NARROW_TILES 128         // tiles merged at a time by a workgroup
+#define LG_NARROW_TILES 128         // tiles of a round of the merge by a workgroup
 #define LG_NARROW_ONE 32            // ... by one wavefront
+#define LG_NARROW_LONG 256          // tiles up to which a round at a time is the faster form at every position (100 positions in a cache of 4096: 140 us, 142 in rounds of two)
 // q8 rows as (4 values, tag) in the order of lg_act_layout and (scale, tag, sum, tag) a block; rows as (float, tag)
 struct NarrowQ8 { uint2 w[LG_NARROW_K / 4]; uint4 s[LG_NARROW_K / 32]; };
 struct NarrowSync { NarrowQ8 attn, act; uint2 o[LG_NARROW_E], d[LG_NARROW_E], pr[LG_NARROW_E], gf[256]; };
@@ -43,10 +44,14 @@ struct NarrowArgs {
     int            spin_limit;
 };
 
-template <bool PLE>
+// LONG: rows that can have more than LG_NARROW_LONG tiles, two rounds of them on their way at a time.  With the rounds of the other build, one after the
+// other, rows of very many tiles were slower than with the separate merge (4 layers of 512 values, every row 100000 positions: 546 us a step, 373
+// with these); one build for both cost a row of few tiles 0.25 us a launch.
+template <bool PLE, bool LONG>
 __global__ __launch_bounds__(512, 2) void lg_k_narrow(NarrowArgs a, const StepCtl *ctl) {
     if (blockIdx.x & (LG_XCDS - 1)) return;
-    __shared__ float part[LG_NARROW_TILES][64], wts[LG_NARROW_TILES], pls[LG_NARROW_TILES], wmx[8], red[PLE ? 6 : 4][8], pcol[2][8][64];
+    __shared__ __align__(16) float wts[LONG ? 2 : 1][LG_NARROW_TILES], pls[LONG ? 2 : 1][LG_NARROW_TILES];
+    __shared__ float part[LONG ? 2 : 1][LG_NARROW_TILES][64], wmx[8], red[PLE ? 6 : 4][8], pcol[2][8][64];
     __shared__ __align__(16) int8_t lq[LG_NARROW_K * 5 / 4], lrow[LG_NARROW_E * 5 / 4], lnat[LG_NARROW_E * 5 / 4], lgate[256 * 5 / 4];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), c = lane & 7;
     const int u = blockIdx.x >> 3, E = a.E, nq = E >> 2, nitE = E >> 8, nitQ = a.qd >> 8, nitF = a.FF >> 8;
@@ -159,7 +164,76 @@ __global__ __launch_bounds__(512, 2) void lg_k_narrow(NarrowArgs a, const StepCt
         const size_t base = (size_t)head * a.g.tiles_max;
         const float *acc = a.g.pacc + base * hd + (u * 64 - head * hd) + lane, *pm = a.g.pm + base, *pl = a.g.pl + base;
         float L = 0.0f, o = 0.0f;
-        if (a.tiles <= LG_NARROW_ONE) {                        // (a sliding window of 512, say)
+        if constexpr (LONG) {
+            // Rounds of 128 tiles, two of them on their way: the wavefronts request 16 each, wavefront 0 adds the values of a round from LDS and
+            // wavefront 1 the sums of its weights (the same two chains of fma in tile order).
+            float pv[2][LG_NARROW_TILES / 8], pmn[2], pln[2];
+            auto fetch = [&](auto k_, int c0) {
+                constexpr int k = decltype(k_)::value;
+                #pragma unroll
+                for (int i = 0; i < LG_NARROW_TILES / 8; ++i) { const int n = c0 + wave + 8 * i; pv[k][i] = acc[(size_t)(n < a.tiles ? n : a.tiles - 1) * hd]; }
+                if (c0 && t < LG_NARROW_TILES) { const int n = c0 + t < a.tiles ? c0 + t : a.tiles - 1; pmn[k] = pm[n]; pln[k] = pl[n]; }
+            };
+            constexpr std::integral_constant<int, 0> K0{}; constexpr std::integral_constant<int, 1> K1{};
+            const int mine = t < a.tiles ? t : a.tiles - 1;
+            pmn[0] = pm[mine]; pln[0] = pl[mine];
+            const int pos = ctl->pos + a.g.pos_off;
+            fetch(K0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            request();
+            const int hi = (pos >> 5) - (lg_win_start(pos, a.g.window) >> 5);
+            if (hi >= LG_NARROW_TILES) fetch(K1, LG_NARROW_TILES);
+            float mx = t <= hi ? pmn[0] : -INFINITY;
+            for (int n = t + 512; n <= hi; n += 4 * 512) {
+                float m4[4];
+                #pragma unroll
+                for (int i = 0; i < 4; ++i) m4[i] = pm[n + 512 * i <= hi ? n + 512 * i : n];
+                mx = fmaxf(fmaxf(fmaxf(mx, m4[0]), fmaxf(m4[1], m4[2])), m4[3]);
+            }
+            mx = lg_max_n(mx, 64);
+            if (lane == 0) wmx[wave] = mx;
+            __syncthreads();
+            mx = fmaxf(fmaxf(fmaxf(wmx[0], wmx[1]), fmaxf(wmx[2], wmx[3])), fmaxf(fmaxf(wmx[4], wmx[5]), fmaxf(wmx[6], wmx[7])));
+            // sum += src[tile] * weight[tile], tiles 0..cn-1 in order; the next eight tiles' reads ahead of the fma of the present ones
+            auto chain = [&](const float *src, auto stride, const float *w, int cn, float &sum) {
+                constexpr int ST = decltype(stride)::value;
+                float p8[2][8], w8[2][8];
+                auto read = [&](int k, int n0_) {
+                    const int n0 = n0_ < LG_NARROW_TILES ? n0_ : LG_NARROW_TILES - 8;
+                    #pragma unroll
+                    for (int i = 0; i < 8; ++i) { p8[k][i] = src[(n0 + i) * ST]; w8[k][i] = w[n0 + i]; }
+                };
+                auto add = [&](int k, int n0) {
+                    if (n0 + 8 <= cn) {
+                        #pragma unroll
+                        for (int i = 0; i < 8; ++i) sum = lg_fmaf(p8[k][i], w8[k][i], sum);
+                    } else {
+                        #pragma unroll
+                        for (int i = 0; i < 8; ++i) if (n0 + i < cn) sum = lg_fmaf(p8[k][i], w8[k][i], sum);
+                    }
+                };
+                read(0, 0);
+                for (int n0 = 0; n0 < cn; n0 += 16) { read(1, n0 + 8); add(0, n0); read(0, n0 + 16); add(1, n0 + 8); }
+            };
+            auto round = [&](auto k_, int c0) {                // (a round's place in LDS is written again behind the other round's barrier)
+                constexpr int k = decltype(k_)::value;
+                #pragma unroll
+                for (int i = 0; i < LG_NARROW_TILES / 8; ++i) part[k][wave + 8 * i][lane] = pv[k][i];
+                if (t < LG_NARROW_TILES && c0 + t <= hi) { wts[k][t] = lg_expf(pmn[k] - mx); pls[k][t] = pln[k]; }
+                __syncthreads();
+                if (c0 + 2 * LG_NARROW_TILES <= hi) fetch(k_, c0 + 2 * LG_NARROW_TILES);
+                const int cn = hi - c0 + 1 < LG_NARROW_TILES ? hi - c0 + 1 : LG_NARROW_TILES;
+                if (wave == 0) chain(&part[k][0][lane], std::integral_constant<int, 64>{}, wts[k], cn, o);
+                else if (wave == 1) chain(pls[k], std::integral_constant<int, 1>{}, wts[k], cn, L);
+            };
+            for (int c0 = 0; c0 <= hi; c0 += 2 * LG_NARROW_TILES) {
+                round(K0, c0);
+                if (c0 + LG_NARROW_TILES <= hi) round(K1, c0 + LG_NARROW_TILES);
+            }
+            if (wave == 1 && lane == 0) wmx[0] = L;            // (every wavefront has read the maxima before the first round's barrier)
+            __syncthreads();
+            L = wmx[0];
+        } else if (a.tiles <= LG_NARROW_ONE) {                        // (a sliding window of 512, say)
             // one wavefront by itself, while the others request: they are a microsecond at it, and a merge that all of them take part
             // in ends behind that (3.5 us into the launch, one wavefront's 2.8)
             if (wave == 0) {
@@ -199,8 +273,8 @@ __global__ __launch_bounds__(512, 2) void lg_k_narrow(NarrowArgs a, const StepCt
             mx = fmaxf(fmaxf(fmaxf(wmx[0], wmx[1]), fmaxf(wmx[2], wmx[3])), fmaxf(fmaxf(wmx[4], wmx[5]), fmaxf(wmx[6], wmx[7])));
             for (int c0 = 0; c0 <= hi; c0 += LG_NARROW_TILES) {
                 #pragma unroll
-                for (int i = 0; i < LG_NARROW_TILES / 8; ++i) part[wave + 8 * i][lane] = pv[i];
-                if (t < LG_NARROW_TILES && c0 + t <= hi) { wts[t] = lg_expf((c0 ? pm[c0 + t] : pm1) - mx); pls[t] = c0 ? pl[c0 + t] : pl1; }
+                for (int i = 0; i < LG_NARROW_TILES / 8; ++i) part[0][wave + 8 * i][lane] = pv[i];
+                if (t < LG_NARROW_TILES && c0 + t <= hi) { wts[0][t] = lg_expf((c0 ? pm[c0 + t] : pm1) - mx); pls[0][t] = c0 ? pl[c0 + t] : pl1; }
                 __syncthreads();
                 if (c0 + LG_NARROW_TILES <= hi) fetch(c0 + LG_NARROW_TILES);
                 if (wave == 0) {
@@ -208,7 +282,7 @@ __global__ __launch_bounds__(512, 2) void lg_k_narrow(NarrowArgs a, const StepCt
                     for (int n0 = 0; n0 < cn; n0 += 8) {          // in tile order; eight tiles' reads ahead of their fma
                         float p8[8], w8[8], l8[8];
                         #pragma unroll
-                        for (int i = 0; i < 8; ++i) { p8[i] = part[n0 + i][lane]; w8[i] = wts[n0 + i]; l8[i] = pls[n0 + i]; }
+                        for (int i = 0; i < 8; ++i) { p8[i] = part[0][n0 + i][lane]; w8[i] = wts[0][n0 + i]; l8[i] = pls[0][n0 + i]; }
                         #pragma unroll
                         for (int i = 0; i < 8; ++i) if (n0 + i < cn) { L = lg_fmaf(l8[i], w8[i], L); o = lg_fmaf(p8[i], w8[i], o); }
                     }
@@ -221,7 +295,7 @@ __global__ __launch_bounds__(512, 2) void lg_k_narrow(NarrowArgs a, const StepCt
             const int q = lg_quant1_32lanes(o / L, &d, &sum);
             put_q8(y.attn, a.qd, u * 64 + lane, q, d, sum);
         }
-        if (a.tiles <= LG_NARROW_ONE) request();
+        if (!LONG && a.tiles <= LG_NARROW_ONE) request();
     } else request();
     // ---- attention output ----
     take_q8(y.attn, a.qd);

@@ -8,10 +8,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("name,over,pos0", [
     ("tiny", {}, 0), ("tiny_full", {}, 100), ("tiny", {"n_embd": 256, "n_ff": 256}, 31), ("tiny_full", {"n_embd": 256, "n_ff": 1280}, 64),
     ("tiny", {"n_ff": 1280, "head_dim": 128}, 127), ("tiny", {"sliding_window": 512}, 1000), ("tiny", {"sliding_window": 1024}, 1500),
-    ("tiny", {}, 1023), ("tiny_full", {}, 4094), ("tiny", {}, 8250)])
+    ("tiny", {}, 1023), ("tiny_full", {}, 4094), ("tiny", {}, 8250), ("tiny_full", {}, 8190), ("tiny", {"local_period": 0}, 20478)])
 def test_a_layer_as_one_launch_equals_the_separate_kernels(lg, gpu_required, model_path, name, over, pos0):
     """Widths of one and two tiles a segment, feed-forward blocks on a part of the workgroups and on more than all of them, heads of 64 and
-    128, contexts of one tile, on both sides of 32 (the merge by one wavefront) and of 128 (the tiles of a round): logits, hidden state and
+    128, contexts of one tile, on both sides of 32 (the merge by one wavefront), of 128 (half a round of tiles), of 256 (a round) and of 640 (two and a half): logits, hidden state and
     cache rows of several steps, bit for bit.  The cache rows in front are drawn."""
     path, spec = model_path(name, **over)
     rng = np.random.default_rng(pos0)
