@@ -196,6 +196,8 @@ struct lg_hip_model {
     std::vector<int> is_local, ffn_len, head_dim, n_head_kv;
     std::map<std::string, HostTensor> host;
     bool numbered = false;             // every layer has a launch number of its own (StepCtl.launch): kernels whose workgroups wait for one another may run
+    std::vector<std::pair<void *, size_t>> marks;          // memory whose words carry launch numbers (mark_alloc)
+    int marked_steps = 0;                                  // steps since it was last cleared (count_steps)
     bool committed = false, wide_built = false;    // wide_built: the matrices' wide forms exist
     // weights
     std::vector<Layer> L;
@@ -279,6 +281,25 @@ template <typename T>
 static int dev_alloc(lg_hip_model *m, T **p, size_t n) {
     HIP_TRY(hipMalloc((void **)p, n * sizeof(T) ? n * sizeof(T) : 16));
     m->allocs.push_back((void *)*p);
+    return 0;
+}
+
+// Memory that workgroups of a launch hand data over in, every word or flag with the launch's number (lg_tag): zero, which is the number of no launch
+// (the last of a step's LG_STEP_LAUNCHES is not used)
+template <typename T>
+static int mark_alloc(lg_hip_model *m, T **p, size_t n = 1) {
+    if (dev_alloc(m, p, n)) return -7;
+    m->marks.emplace_back((void *)*p, n * sizeof(T));
+    HIP_TRY(hipMemset(*p, 0, n * sizeof(T)));
+    return 0;
+}
+// Called ahead of `steps` more steps of the model on its stream, never under capture.  A mark has 28 bits, so the numbers come round after 2^20 steps (half an hour
+// of steps of 1.7 ms), and what no launch has written since (the rows of a wider block, say) would then count as the present launch's.
+// Cleared every LG_MARK_STEPS it is never that old.
+static int count_steps(lg_hip_model *m, int steps) {
+    if ((m->marked_steps += steps) <= LG_MARK_STEPS) return 0;
+    m->marked_steps = steps;
+    for (auto &p : m->marks) HIP_TRY(hipMemsetAsync(p.first, 0, p.second, m->stream));
     return 0;
 }
 
@@ -699,8 +720,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
                 if (dev_alloc(m, &y.wdn_m, 256 * dg.wg_bytes)) return -7;
                 HIP_TRY(hipMemcpy(y.wdn_m, xstage.data(), 256 * dg.wg_bytes, hipMemcpyHostToDevice));
                 if (!m->dmsync) {
-                    if (dev_alloc(m, &m->dmsync, (size_t)1)) return -7;
-                    HIP_TRY(hipMemset(m->dmsync, 0, sizeof(DownMSync)));
+                    if (mark_alloc(m, &m->dmsync)) return -7;
                 }
             }
         }
@@ -779,29 +799,18 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         return -7;
     if (m->ple && dev_alloc(m, &m->eq, qb(E) + (size_t)12 * E)) return -7;
     if (!m->target) {                        // hand-over state of the one-XCD kernels (lg_xtail.h)
-        if (dev_alloc(m, &m->tsync, (size_t)1) || dev_alloc(m, &m->tstamps, (size_t)2 * LG_XTAIL_UNITS * 8) ||
-            dev_alloc(m, &m->tgf, (size_t)LG_HIP_MAX_ROWS * (m->ple > 0 ? m->ple : 1)) || dev_alloc(m, &m->tpr, (size_t)LG_HIP_MAX_ROWS * (m->ple > 0 ? E : 1))) return -7;
-        if (m->ple > 0) {                    // (no tag of any launch)
-            HIP_TRY(hipMemset(m->tgf, 0, (size_t)LG_HIP_MAX_ROWS * m->ple * 8));
-            HIP_TRY(hipMemset(m->tpr, 0, (size_t)LG_HIP_MAX_ROWS * E * 8));
-        }
+        if (mark_alloc(m, &m->tsync) || mark_alloc(m, &m->rgsync) || dev_alloc(m, &m->tstamps, (size_t)2 * LG_XTAIL_UNITS * 8) ||
+            (m->ple > 0 && (mark_alloc(m, &m->tgf, (size_t)LG_HIP_MAX_ROWS * m->ple) || mark_alloc(m, &m->tpr, (size_t)LG_HIP_MAX_ROWS * E)))) return -7;
         HIP_TRY(hipMemset(m->tstamps, 0, (size_t)2 * LG_XTAIL_UNITS * 8 * 8));
-        HIP_TRY(hipMemset(m->tsync, 0, sizeof(XtailSync)));
-        if (dev_alloc(m, &m->rgsync, (size_t)1)) return -7;
-        HIP_TRY(hipMemset(m->rgsync, 0, sizeof(RgSync)));
         HIP_TRY(hipMemset(m->aq, 0, qb(max_qd)));       // (row slots past the block are read as operand rows of the matrix cores)
         if (getenv("LG_HIP_XCD_TAIL")) m->xcd_tail = atoi(getenv("LG_HIP_XCD_TAIL"));
     }
     if (narrow_shape(m)) {
-        if (dev_alloc(m, &m->nsync, (size_t)1)) return -7;
-        HIP_TRY(hipMemset(m->nsync, 0, sizeof(NarrowSync)));
+        if (mark_alloc(m, &m->nsync)) return -7;
     } else if (!m->target && cu_count() == LG_XCDS * LG_XCD_WGS) {
         bool any = false;
         for (const Layer &y : m->L) any = any || attn_out_shape(m, y);
-        if (any) {
-            if (dev_alloc(m, &m->aosync, (size_t)1)) return -7;
-            HIP_TRY(hipMemset(m->aosync, 0, sizeof(AttnOutSync)));
-        }
+        if (any && mark_alloc(m, &m->aosync)) return -7;
     }
     if (getenv("LG_HIP_XCD_ATTN_TAIL")) m->xcd_attn_tail = atoi(getenv("LG_HIP_XCD_ATTN_TAIL"));
     if (getenv("LG_HIP_DOWN_M")) m->down_m = atoi(getenv("LG_HIP_DOWN_M"));
@@ -811,8 +820,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         return -7;
     if (xffn) {
         if (dev_alloc(m, &m->slabs, (size_t)LG_XCDS * max_rows * E) || dev_alloc(m, &m->xact, (size_t)LG_XCDS * max_rows * xg.C) ||
-            dev_alloc(m, &m->xq8, (size_t)LG_XCDS * xg.nb * LG_MU_DWORDS) || dev_alloc(m, &m->xsync, (size_t)1)) return -7;
-        HIP_TRY(hipMemset(m->xsync, 0, sizeof(XcdSync)));
+            dev_alloc(m, &m->xq8, (size_t)LG_XCDS * xg.nb * LG_MU_DWORDS) || mark_alloc(m, &m->xsync)) return -7;
         HIP_TRY(hipMemset(m->xq8, 0, (size_t)LG_XCDS * xg.nb * LG_MU_DWORDS * 4));        // row slots past the block are read as operand rows
         m->xffn_built = true; m->xffn_cls = xffn_class_of(xg);
         m->xcd_ffn = getenv("LG_HIP_XCD_FFN") && atoi(getenv("LG_HIP_XCD_FFN")) != 0;     // off unless asked for: the separate kernels are faster (see lg_xffn.h)
@@ -1921,6 +1929,8 @@ static hipGraphExec_t capture_behind(hipStream_t st, F enqueue) {
 // (a first decode step on a new cache, E4B shape: 3.95 -> 2.28 ms; capturing and instantiating 341 launches takes 1.5).
 static int launch_step(lg_hip_model *m, lg_hip_kv *kv, int rows, bool with_head) {
     m->lread = m->lcoming = -1;
+    int rc = count_steps(m, 1);
+    if (rc) return rc;
     if (!m->use_graph || m->prof.on) return enqueue_step_rows(m, kv, rows, with_head);
     const GraphKey key = graph_key(m, kv, rows, with_head ? 1 : 0);
     auto it = m->graphs.find(key);
@@ -1929,7 +1939,7 @@ static int launch_step(lg_hip_model *m, lg_hip_kv *kv, int rows, bool with_head)
         HIP_TRY(hipGraphLaunch(it->second, m->stream));
         return 0;
     }
-    int rc = enqueue_step_rows(m, kv, rows, with_head, true);
+    rc = enqueue_step_rows(m, kv, rows, with_head, true);
     if (!rc) rc = enqueue_step_rows(m, kv, rows, with_head);
     if (!rc) m->graphs.emplace(key, capture_behind(m->stream, [&]() { return enqueue_step_rows(m, kv, rows, with_head); }));
     return rc;
@@ -2107,6 +2117,7 @@ extern "C" int lg_hip_mtp_rounds(lg_hip_model *d, lg_hip_kv *kv, int token, int 
     int32_t tk = token;
     if ((rc = load_block(t, &tk, 1, pos, false))) return rc;
     t->lread = t->lcoming = d->lread = d->lcoming = -1;
+    if ((rc = count_steps(t, n_rounds)) || (rc = count_steps(d, n_rounds * (rows - 1)))) return rc;
     if (!t->use_graph || t->prof.on || d->prof.on) {
         for (int r = 0; r < n_rounds; ++r) if ((rc = enqueue_round(d, kv, rows, false))) return rc;
     } else {
@@ -2173,7 +2184,8 @@ extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *tok
                 rows = left < m->max_rows ? left : m->max_rows;
                 if (done) HIP_TRY(hipMemcpyAsync(m->sched, m->pin + 64 + done, (size_t)rows * 4, hipMemcpyHostToDevice, m->stream));   // (its kernels read the schedule from its start)
                 hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, m->stream, m->ctl, pos0 + at + done, first);
-                rc = wide ? enqueue_step_rows(m, kv, rows, false) : launch_step(m, kv, rows, false);    // (a single one: not worth a capture)
+                if (!wide) rc = launch_step(m, kv, rows, false);
+                else if (!(rc = count_steps(m, 1))) rc = enqueue_step_rows(m, kv, rows, false);         // (a single one: not worth a capture)
             }
             if (rc) return rc;
             done += rows;
@@ -2325,6 +2337,7 @@ extern "C" int lg_hip_profile_step(lg_hip_model *m, lg_hip_kv *kv, const int32_t
     int cnt[KC_COUNT] = { 0 };
     for (int r = 0; r < repeats + 1; ++r) {              // first pass warms up and is dropped
         if ((rc = load_block(m, toks, rows, pos, false))) return rc;
+        if ((rc = count_steps(m, 1))) return rc;
         m->prof.on = true;
         m->lread = m->lcoming = -1;
         rc = enqueue_step_rows(m, kv, rows, true);

@@ -23,6 +23,8 @@ struct StepCtl {            // device-resident step state
                             // whenever it starts, also when another of them has given up its wait and left
 };
 #define LG_STEP_LAUNCHES 256 // more than the layers of a model that has such launches
+#define LG_MARK_STEPS (1 << 19)  // steps after which the marks of launches are cleared: they come round after 2^28 launch numbers
+static_assert((uint64_t)2 * LG_MARK_STEPS * LG_STEP_LAUNCHES <= (uint64_t)1 << 28, "marks older than half their range are cleared");
 
 // ---------------------------------------------------------------------------------------------
 // Row kernel: everything that happens to the M residual rows between two matmuls, one wavefront

@@ -61,3 +61,25 @@ def test_a_number_that_a_unit_advances_can_leave_its_launch():
     the next launch's number, which the next launch takes for its own."""
     with pytest.raises(AssertionError, match="nothing was reported"):
         run_steps(advances=True)
+
+
+@pytest.mark.parametrize("cleared_every,sound", [(4, True), (7, True), (None, False)])
+def test_marks_that_come_round(cleared_every, sound):
+    """Marks of 8 steps: blocks whose last units' slots lie unused for any number of steps and are then waited for.  A slot that was last written
+    8 steps ago holds the present mark; cleared in less than that, no slot is that old."""
+    around = 8 * STEP
+    for idle in range(1, 20):
+        m, since, taken = Memory(), 0, True
+        for step in range(2 * idle + 2):
+            if cleared_every and since + 1 > cleared_every:
+                m.slots, since = [(None, 0)] * UNITS, 0
+            since += 1
+            tag = ((step + 1) * STEP + 1) % around              # (number + 1, as lg_tag has it)
+            wide = step % (idle + 1) == 0
+            taken &= not (wide and m.slots[UNITS - 1][1] == tag)  # there before the unit has stored it
+            for u in range(UNITS if wide else UNITS - 1):
+                m.slots[u] = (step, tag)
+        if not sound and not taken:
+            return
+        assert taken
+    assert sound
