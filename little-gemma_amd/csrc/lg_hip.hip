@@ -196,6 +196,9 @@ struct lg_hip_model {
     std::vector<int> is_local, ffn_len, head_dim, n_head_kv;
     std::map<std::string, HostTensor> host;
     bool numbered = false;             // every layer has a launch number of its own (StepCtl.launch): kernels whose workgroups wait for one another may run
+    struct Turns *turns = nullptr;                         // of its device
+    hipEvent_t ev_turn = nullptr;                          // end of the steps it has launched, for another model's to wait for
+    bool turn_recorded = false;                            // ev_turn holds the end of its latest step already
     std::vector<std::pair<void *, size_t>> marks;          // memory whose words carry launch numbers (mark_alloc)
     int marked_steps = 0;                                  // steps since it was last cleared (count_steps)
     bool committed = false, wide_built = false;    // wide_built: the matrices' wide forms exist
@@ -284,6 +287,53 @@ static int dev_alloc(lg_hip_model *m, T **p, size_t n) {
     return 0;
 }
 
+// Steps with launches whose workgroups wait for one another, of several models on a device.  Such a launch is sound when its workgroups are all resident
+// at some time: a waiting one keeps its CU, up to a whole one.  Two of them at a time, on the streams of two models, could each hold a part of an
+// XCD's 32 and wait for the rest until both give up.  So a step with such launches starts behind the end of the last one of another model; the
+// steps of one model are ordered by its stream.  With one model at work this is one uncontended lock a step.
+struct Turns {
+    std::mutex mu;                             // held while a step is launched or captured
+    lg_hip_model *last = nullptr;              // whose step with such launches was the latest
+};
+static Turns *turns_of(int device) {
+    static std::mutex mu;
+    static auto *all = new std::map<int, Turns>();         // (kept: models may outlive the library's static objects)
+    std::lock_guard<std::mutex> hold(mu);
+    return &(*all)[device];
+}
+// The lock under which a step of m (or a round of a draft head m) is launched; `waits`: with launches of that kind
+static int take_turn(lg_hip_model *m, bool waits, std::unique_lock<std::mutex> &turn) {
+    lg_hip_model *own = m->target ? m->target : m;         // (a draft head has its target's stream)
+    turn = std::unique_lock<std::mutex>(own->turns->mu);
+    if (!waits) return 0;
+    lg_hip_model *&last = own->turns->last;
+    if (last && last != own) {
+        if (!last->turn_recorded) HIP_TRY(hipEventRecord(last->ev_turn, last->stream));
+        last->turn_recorded = true;
+        HIP_TRY(hipStreamWaitEvent(own->stream, last->ev_turn, 0));
+    }
+    last = own;
+    own->turn_recorded = false;
+    return 0;
+}
+// Ahead of long work without such launches (a prompt's blocks), which another model's steps need not wait for
+static int mark_turn(lg_hip_model *m) {
+    std::lock_guard<std::mutex> turn(m->turns->mu);
+    if (m->turns->last != m || m->turn_recorded) return 0;
+    HIP_TRY(hipEventRecord(m->ev_turn, m->stream));
+    m->turn_recorded = true;
+    return 0;
+}
+// For a launch of that kind outside of any model, on a stream that is waited for before the lock is given back
+static int take_turn_alone(std::unique_lock<std::mutex> &turn) {
+    int device = 0;
+    HIP_TRY(hipGetDevice(&device));
+    Turns *t = turns_of(device);
+    turn = std::unique_lock<std::mutex>(t->mu);
+    if (t->last) HIP_TRY(hipStreamSynchronize(t->last->stream));
+    return 0;
+}
+
 // Memory that workgroups of a launch hand data over in, every word or flag with the launch's number (lg_tag): zero, which is the number of no launch
 // (the last of a step's LG_STEP_LAUNCHES is not used)
 template <typename T>
@@ -315,6 +365,7 @@ extern "C" int lg_hip_model_create(const struct lg_hip_config *c, int device, lg
     if (cu_count() <= 0) return fail(-3, "model_create: device %d does not tell its number of compute units", device);      // (launches are cut by it)
     lg_hip_model *m = new lg_hip_model();
     m->device = device;
+    m->turns = turns_of(device);
     m->numbered = c->n_layer < LG_STEP_LAUNCHES;
     m->n_layer = c->n_layer; m->E = c->n_embd; m->H = c->n_head; m->n_vocab = c->n_vocab;
     m->window = c->sliding_window; m->ple = c->n_embd_per_layer; m->n_kv_start = c->n_kv_start;
@@ -335,6 +386,7 @@ extern "C" int lg_hip_model_create(const struct lg_hip_config *c, int device, lg
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&m->stream2, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&m->ev_fork, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&m->ev_join, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&m->ev_turn, hipEventDisableTiming);
     if (e != hipSuccess) { delete m; return fail(-100 - (int)e, "hipStreamCreate: %s", hipGetErrorString(e)); }
     if (getenv("LG_HIP_FORK")) m->fork_ple = atoi(getenv("LG_HIP_FORK")) != 0;   // the per-layer inputs as a second branch (comparison runs)
     *out = m;
@@ -847,6 +899,10 @@ extern "C" void lg_hip_model_destroy(lg_hip_model *m) {
     if (!m) return;
     (void)hipSetDevice(m->device);
     (void)hipDeviceSynchronize();
+    {
+        std::lock_guard<std::mutex> turn(m->turns->mu);
+        if (m->turns->last == m) m->turns->last = nullptr;
+    }
     for (auto &g : m->graphs) if (g.second) (void)hipGraphExecDestroy(g.second);
     for (void *p : m->allocs) (void)hipFree(p);
     for (hipEvent_t e : m->prof.ev) (void)hipEventDestroy(e);
@@ -860,6 +916,7 @@ extern "C" void lg_hip_model_destroy(lg_hip_model *m) {
     if (m->stream2) (void)hipStreamDestroy(m->stream2);
     if (m->ev_fork) (void)hipEventDestroy(m->ev_fork);
     if (m->ev_join) (void)hipEventDestroy(m->ev_join);
+    if (m->ev_turn) (void)hipEventDestroy(m->ev_turn);
     for (lg_hip_model *d : m->drafts) { d->target = nullptr; d->stream = nullptr; }        // orphaned heads refuse to run
     delete m;
 }
@@ -1259,6 +1316,11 @@ static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int t
     if (!y.wo_ch || !m->tsync || !m->numbered || !attn_tail_shape(y.qd, m->E, nullptr, nullptr) || m->xcd_attn_tail <= 0 || (m->xcd_attn_tail == 1 && rows < 3)) return false;
     const int slices = (m->E + 1023) / 1024;
     return tiles < 128 && m->H * rows <= 2 * LG_XCD_WGS && slices * rows <= LG_XCD_WGS && y.hd % 32 == 0 && y.hd <= 256;
+}
+// Whether a step may hold launches whose workgroups wait for one another
+static bool step_waits(const lg_hip_model *m, int rows) {
+    return m->numbered && (use_narrow(m, rows) || (m->attn_out && m->aosync) || use_ple_tail(m, rows) || m->rows_geglu || m->xcd_attn_tail > 0 ||
+                           (rows >= 4 && ((m->down_m == 1 && m->dmsync) || m->xcd_ffn)));
 }
 template <int M>
 static void launch_attn_tail(Launcher &lx, const XattnTailArgs &a) {
@@ -1929,8 +1991,9 @@ static hipGraphExec_t capture_behind(hipStream_t st, F enqueue) {
 // (a first decode step on a new cache, E4B shape: 3.95 -> 2.28 ms; capturing and instantiating 341 launches takes 1.5).
 static int launch_step(lg_hip_model *m, lg_hip_kv *kv, int rows, bool with_head) {
     m->lread = m->lcoming = -1;
-    int rc = count_steps(m, 1);
-    if (rc) return rc;
+    std::unique_lock<std::mutex> turn;
+    int rc = take_turn(m, step_waits(m, rows), turn);
+    if (rc || (rc = count_steps(m, 1))) return rc;
     if (!m->use_graph || m->prof.on) return enqueue_step_rows(m, kv, rows, with_head);
     const GraphKey key = graph_key(m, kv, rows, with_head ? 1 : 0);
     auto it = m->graphs.find(key);
@@ -2117,20 +2180,27 @@ extern "C" int lg_hip_mtp_rounds(lg_hip_model *d, lg_hip_kv *kv, int token, int 
     int32_t tk = token;
     if ((rc = load_block(t, &tk, 1, pos, false))) return rc;
     t->lread = t->lcoming = d->lread = d->lcoming = -1;
+    const bool waits = step_waits(t, rows) || step_waits(d, 1);
     if ((rc = count_steps(t, n_rounds)) || (rc = count_steps(d, n_rounds * (rows - 1)))) return rc;
     if (!t->use_graph || t->prof.on || d->prof.on) {
-        for (int r = 0; r < n_rounds; ++r) if ((rc = enqueue_round(d, kv, rows, false))) return rc;
+        for (int r = 0; r < n_rounds; ++r) {
+            std::unique_lock<std::mutex> turn;
+            if ((rc = take_turn(t, waits, turn)) || (rc = enqueue_round(d, kv, rows, false))) return rc;
+        }
     } else {
         GraphKey key = graph_key(t, kv, rows, 2);
         key[3] = graph_key(d, kv, 1, 2)[1];
         auto it = d->graphs.find(key);            // kept by the head: the graph dies with it or with the cache
         int r = 0;
         if (it == d->graphs.end()) {               // the first round as launches, its graph while the device works on it
-            if ((rc = enqueue_round(d, kv, rows, true)) || (rc = enqueue_round(d, kv, rows, false))) return rc;
+            std::unique_lock<std::mutex> turn;
+            if ((rc = take_turn(t, waits, turn)) || (rc = enqueue_round(d, kv, rows, true)) || (rc = enqueue_round(d, kv, rows, false))) return rc;
             it = d->graphs.emplace(key, capture_behind(t->stream, [&]() { return enqueue_round(d, kv, rows, false); })).first;
             r = 1;
         }
         for (; r < n_rounds; ++r) {
+            std::unique_lock<std::mutex> turn;
+            if ((rc = take_turn(t, waits, turn))) return rc;
             if (it->second) HIP_TRY(hipGraphLaunch(it->second, t->stream));
             else if ((rc = enqueue_round(d, kv, rows, false))) return rc;
         }
@@ -2169,6 +2239,7 @@ extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *tok
     const int cap = m->sched_cap * LG_HIP_MAX_ROWS;        // tokens the staging holds
     int32_t *err = m->pin + 32 + LG_REPORT_ERR;             // (written by the verify blocks among the call's, the prompt kernels wait for nobody)
     __atomic_store_n(err, 0, __ATOMIC_RELAXED);
+    if (wide_ok && n > m->max_rows) { const int rc = mark_turn(m); if (rc) return rc; }
     for (int at = 0; at < n;) {
         // the tokens go over once, the blocks follow each other on the stream and the host waits at the end
         const int part = n - at < cap ? n - at : cap;
@@ -2179,13 +2250,15 @@ extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *tok
             int rows = left < kv->prompt_rows ? left : kv->prompt_rows, rc;
             const bool wide = wide_ok && !far_in_narrow_heads(m, kv, rows, pos0 + at + done);
             const bool first = at + done == 0;
+            std::unique_lock<std::mutex> turn;
             if (wide && left > m->max_rows) rc = enqueue_prompt(m, kv, m->sched + done, rows, pos0 + at + done, first);
             else {                                           // a remainder that fits a verify block
                 rows = left < m->max_rows ? left : m->max_rows;
                 if (done) HIP_TRY(hipMemcpyAsync(m->sched, m->pin + 64 + done, (size_t)rows * 4, hipMemcpyHostToDevice, m->stream));   // (its kernels read the schedule from its start)
                 hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, m->stream, m->ctl, pos0 + at + done, first);
                 if (!wide) rc = launch_step(m, kv, rows, false);
-                else if (!(rc = count_steps(m, 1))) rc = enqueue_step_rows(m, kv, rows, false);         // (a single one: not worth a capture)
+                else if (!(rc = take_turn(m, step_waits(m, rows), turn)) && !(rc = count_steps(m, 1)))
+                    rc = enqueue_step_rows(m, kv, rows, false);                                         // (a single one: not worth a capture)
             }
             if (rc) return rc;
             done += rows;
@@ -2337,10 +2410,12 @@ extern "C" int lg_hip_profile_step(lg_hip_model *m, lg_hip_kv *kv, const int32_t
     int cnt[KC_COUNT] = { 0 };
     for (int r = 0; r < repeats + 1; ++r) {              // first pass warms up and is dropped
         if ((rc = load_block(m, toks, rows, pos, false))) return rc;
-        if ((rc = count_steps(m, 1))) return rc;
+        std::unique_lock<std::mutex> turn;
+        if ((rc = take_turn(m, step_waits(m, rows), turn)) || (rc = count_steps(m, 1))) return rc;
         m->prof.on = true;
         m->lread = m->lcoming = -1;
         rc = enqueue_step_rows(m, kv, rows, true);
+        turn.unlock();
         m->prof.on = false;
         hipError_t e = hipStreamSynchronize(m->stream);
         if (!rc && e != hipSuccess) rc = fail(-100 - (int)e, "profile_step: %s", hipGetErrorString(e));
@@ -2943,6 +3018,8 @@ extern "C" int lg_hip_xcd_handover(int set_mode, int sel, int n, int store_scope
     if (sc.get(&a.flags, (size_t)64) || sc.get(&a.data, (size_t)2 * n * (a.words ? a.words : 1)) || sc.get(&a.res, (size_t)n * 4)) return -7;
     HIP_TRY(hipMemset(a.flags, 0, 256));
     HIP_TRY(hipMemset(a.res, 0xFF, (size_t)n * 16));
+    std::unique_lock<std::mutex> turn;
+    { const int rc = take_turn_alone(turn); if (rc) return rc; }
     HIP_TRY(hipDeviceSynchronize());
     const int combo = store_scope * 4 + load_scope;
     switch (combo) {
@@ -2977,6 +3054,8 @@ extern "C" int lg_hip_down_m(const float *act, const void *down, int rows, int E
     HIP_TRY(hipMemcpy(dw, stage.data(), 256 * g.wg_bytes, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(dx, act, (size_t)rows * FF * 4, hipMemcpyHostToDevice));
     HIP_TRY(hipMemset(dq, 0, (size_t)(FF / 32) * LG_MU_DWORDS * 4));
+    std::unique_lock<std::mutex> turn;
+    { const int rc = take_turn_alone(turn); if (rc) return rc; }
     hipStream_t st;
     HIP_TRY(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     lg_hip_model shim;
@@ -3116,6 +3195,8 @@ extern "C" int lg_hip_ffn_xcd(const float *x, const float *dout, const float *w_
     HIP_TRY(hipMemset(dsync, 0, sizeof(XcdSync)));
     HIP_TRY(hipMemset(dxq, 0, (size_t)LG_XCDS * g.nb * LG_MU_DWORDS * 4));
     HIP_TRY(hipMemset(ctl, 0, sizeof(StepCtl)));
+    std::unique_lock<std::mutex> turn;
+    { const int rc = take_turn_alone(turn); if (rc) return rc; }
     hipStream_t st;
     HIP_TRY(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     lg_hip_model shim;
