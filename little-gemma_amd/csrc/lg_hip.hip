@@ -694,7 +694,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
     // the XCD-partitioned feed-forward kernel: one shape for all layers, a chip of 256 CUs in 8 XCDs, blocks of 4+ rows
     XffnGeo xg = lg_xffn_geo(E, m->ffn_len[0]);
     // (its weight streams are second copies of the FFN matrices: built only when the option is asked for at commit)
-    bool xffn = max_rows >= 4 && !m->target && cu_count() == LG_XCDS * LG_XCD_WGS && xffn_class_of(xg) >= 0 &&
+    bool xffn = max_rows >= 4 && !m->target && m->numbered && cu_count() == LG_XCDS * LG_XCD_WGS && xffn_class_of(xg) >= 0 &&
                 getenv("LG_HIP_XCD_FFN") && atoi(getenv("LG_HIP_XCD_FFN")) != 0;
     for (int L = 1; L < nl && xffn; ++L) xffn = m->ffn_len[L] == m->ffn_len[0];
     std::vector<uint8_t> xstage;

@@ -46,3 +46,18 @@ def test_a_wait_given_up_is_reported_once(lg, ob, gpu_required, model_path, name
         assert np.array_equal(gpu.last_hidden(spec["n_embd"]).view(np.uint32), want[2].view(np.uint32))
     finally:
         gpu.close(); o.close()
+
+
+def test_more_layers_than_launch_numbers(lg, gpu_required, model_path, monkeypatch):
+    """256 layers: the numbers of two steps would overlap, so every kernel is one that waits for nobody, also where another was asked for."""
+    monkeypatch.setenv("LG_HIP_XCD_FFN", "1")
+    path, spec = model_path("tiny", n_layer=256, n_vocab=2048)
+    toks = np.random.default_rng(1).integers(1, spec["n_vocab"], 4).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, 64, max_rows=4)
+    try:
+        gpu.set_option("xcd_ffn", 1)
+        for rows in (1, 4):
+            launches = {k["name"]: k["launches"] for k in gpu.profile_step(toks[:rows], 0, 1)}
+            assert not any(launches.get(k, 0) for k in ("ffn_xcd", "ple_tail", "attn_tail")), launches
+    finally:
+        gpu.close()
