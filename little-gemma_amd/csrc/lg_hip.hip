@@ -1308,8 +1308,10 @@ static int step_tiles(const lg_hip_model *m, const lg_hip_kv *kv, const Layer &y
     const int t = (window + rows - 1 + 31) / 32 + 1;
     return t < kv->tiles_max ? t : kv->tiles_max;
 }
-// (tiles: what one wavefront holds; more of them, a global layer in a cache of more than 1280 positions, are merged by more of the chip)
+// (tiles: what one wavefront holds; more of them, a global layer in a cache of 1248 positions and more, are merged by more of the chip.  The row work
+// ahead of gate/up is part of this launch: asked for in another one, by rows_geglu or xcd_ffn, it stays there)
 static bool use_attn_out(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
+    if (rows >= 4 && ((m->rows_geglu && m->E == 2560) || (m->xcd_ffn && y.xgu))) return false;
     return m->attn_out && m->aosync && attn_out_shape(m, y) && (rows <= LG_AOUT_DOT_ROWS ? tiles <= LG_AOUT_TILES : y.wo_ch && tiles <= LG_AOUT_BATCH);
 }
 static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int tiles) {

@@ -42,3 +42,54 @@ def test_one_launch_equals_the_separate_kernels(lg, gpu_required, model_path, ov
         assert all(np.array_equal(a, b) for a, b in zip(*got))
     finally:
         gpu.close()
+
+
+def launches_of(gpu, toks, pos):
+    return {k["name"]: k["launches"] for k in gpu.profile_step(toks, pos, 1)}
+
+
+@pytest.mark.parametrize("window,cache", [(512, 607), (512, 608), (1024, 1247), (1024, 1248)])
+def test_every_width_takes_the_launch_that_its_tiles_allow(lg, gpu_required, model_path, window, cache):
+    """A sliding and a global layer: at most 40 tiles at 1 to 3 rows, 20 at 4 to 8.  (Each has to have run for the comparison above to mean anything.)"""
+    path, spec = model_path("tiny", **dict(W8, n_layer=2, n_ff=512, n_vocab=2048, sliding_window=window))
+    toks = np.random.default_rng(window).integers(1, spec["n_vocab"], 8).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, cache, max_rows=8)
+    try:
+        for rows in range(1, 9):
+            print(f"window {window}, cache {cache}, {rows} rows", flush=True)
+            every = cache // 32 + 2                              # (tiles_max of lg_hip_kv_partials)
+            tiles = (min((window + rows - 1 + 31) // 32 + 1, every), every)
+            got = launches_of(gpu, toks[:rows], 16)
+            want = sum(t <= (40 if rows <= 3 else 20) for t in tiles)
+            assert got.get("attn_tail", 0) == want and got.get("attn_output", 0) == 2 - want, (rows, got)
+    finally:
+        gpu.close()
+
+
+@pytest.mark.parametrize("rows", [4, 5, 8])
+def test_launches_asked_for_come_before_this_one(lg, gpu_required, model_path, monkeypatch, rows):
+    """The row work ahead of gate/up is in this launch, in the gate/up launch (rows_geglu) or in the feed-forward launch (xcd_ffn): the one that was
+    asked for does it, in every layer, with the same bits."""
+    monkeypatch.setenv("LG_HIP_XCD_FFN", "1")
+    path, spec = model_path("tiny", **dict(W8, n_layer=2, n_ff=10240, n_vocab=2048, sliding_window=512))
+    rng = np.random.default_rng(rows)
+    prompt, blk = rng.integers(1, spec["n_vocab"], 40).astype(np.int32), rng.integers(1, spec["n_vocab"], rows).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, 600, max_rows=8)
+    try:
+        gpu.set_option("store_logits", 1)
+        gpu.set_option("xcd_ffn", 0)
+        gpu.prefill(prompt, 0)
+        res, cnt = {}, {}
+        for name, opts in (("separate", dict(attn_out=0)), ("attn_out", {}), ("rows_geglu", dict(rows_geglu=1)), ("xcd_ffn", dict(xcd_ffn=1))):
+            print(f"{rows} rows, {name}", flush=True)
+            for k, v in dict(dict(attn_out=1, rows_geglu=0, xcd_ffn=0), **opts).items():
+                gpu.set_option(k, v)
+            gpu.forward_spec(blk, 40)
+            res[name] = [gpu.logits_row(j, spec["n_vocab"]).view(np.uint32) for j in range(rows)]
+            cnt[name] = launches_of(gpu, blk, 40)
+        assert all(np.array_equal(a, b) for r in res.values() for a, b in zip(r, res["separate"]))
+        n = {k: (c.get("rows_norm_quant", 0), c.get("attn_tail", 0), c.get("ffn_xcd", 0)) for k, c in cnt.items()}
+        alone = n["separate"][0]
+        assert n == {"separate": (alone, 0, 0), "attn_out": (alone - 2, 2, 0), "rows_geglu": (alone - 2, 0, 0), "xcd_ffn": (alone - 2, 0, 2)}, n
+    finally:
+        gpu.close()
