@@ -281,6 +281,9 @@ int    lg_hip_down_m(const float *act, const void *down_q4_0, int rows, int E, i
  * parity tests and timing. */
 int    lg_hip_gate_up_geglu(const float *x, const void *gate_q4_0, const void *up_q4_0, int rows, int E, int FF,
                             int8_t *aq, float *ad, int32_t *asum, int repeats, float *kernel_ms);
+/* Scalar functions of the kernels, one value each (tests): fn 0 = lg_rcp_exact (1/x, x of 2^-100..2^100), 1 = lg_inv_scale
+ * (1/x, or 0 where x is not positive: the factor of a q8 block), 2 = lg_gelu_d, 3 = lg_gelu of include/lg_math.h. */
+int    lg_hip_math(int fn, const float *x, size_t n, float *out);
 /* Host-side weight layout transform used by lg_hip_model_tensor, exposed for tests: q4_0 rows
  * -> the kernels' tile order.  dst needs lg_hip_repacked_bytes(k, m) bytes. */
 int    lg_hip_segments(int k);      /* K segments of a row of k weights: 8, or 32 when k/32 > 128 and a multiple of 32 */

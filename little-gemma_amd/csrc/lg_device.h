@@ -185,8 +185,9 @@ __device__ __forceinline__ float lg_div127(float amax) {
 }
 
 // The correctly rounded 1/d for normal d of 2^-100..2^100: the reciprocal instruction (1 ulp) and one Newton step, which leaves
-// r(1 + e) = (1 - e*e)/d with |e| < 2^-22 before its one rounding.  On this chip that rounds every d as the division does
-// (checked on it for all 2^23 mantissas; powers of two change nothing in this range): three instructions for its ten.
+// r(1 + e) = (1 - e*e)/d with |e| < 2^-22 before its one rounding: three instructions for the division's ten.  From a correctly rounded start that
+// rounds every d as the division does, from one an ulp high all but 32 of the 2^23 mantissas, from one an ulp low all but 1: at those
+// 33 it rests on what this chip's instruction returns.  lg_hip_math and its test cover all of them (powers of two change nothing in this range).
 __device__ __forceinline__ float lg_rcp_exact(float d) {
     const float r = __builtin_amdgcn_rcpf(d);
     return lg_fmaf(lg_fmaf(-d, r, 1.0f), r, r);

@@ -3036,6 +3036,26 @@ extern "C" int lg_hip_xcd_handover(int set_mode, int sel, int n, int store_scope
     return 0;
 }
 
+// ---- device functions on their own (tests) ----------------------------------------------------------
+__global__ void lg_k_math(int fn, const float *x, size_t n, float *out) {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+        out[i] = fn == 0 ? lg_rcp_exact(x[i]) : fn == 1 ? lg_inv_scale(x[i]) : fn == 2 ? lg_gelu_d(x[i]) : lg_gelu(x[i]);
+}
+extern "C" int lg_hip_math(int fn, const float *x, size_t n, float *out) {
+    if (!x || !out || n < 1) return fail(-1, "math: null argument");
+    if (fn < 0 || fn > 3) return fail(-2, "math: no function %d", fn);
+    if (lg_hip_device_count() < 1) return fail(-3, "math: no HIP device");
+    Scratch sc;
+    float *dx, *dout;
+    if (sc.get(&dx, n) || sc.get(&dout, n)) return -7;
+    HIP_TRY(hipMemcpy(dx, x, n * 4, hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(lg_k_math, dim3(2048), dim3(LG_WG), 0, nullptr, fn, dx, n, dout);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipDeviceSynchronize());
+    HIP_TRY(hipMemcpy(out, dout, n * 4, hipMemcpyDeviceToHost));
+    return 0;
+}
+
 // ---- the XCD-partitioned feed-forward half on its own (tests, timing) ------------------------------
 // x_out = x + rmsnorm(dout) * w_post; h = rmsnorm(x_out) * w_pre; act = gelu(gate . q8(h)) * (up . q8(h));
 // out = down . q8(act): lg_k_ffn_xcd on host data, the 8 slabs added here in tree order.

@@ -427,6 +427,16 @@ def ffn_xcd(x, dout, w_post, w_pre, gate_q4_0, up_q4_0, down_q4_0, FF, eps=1e-6,
     return dict(x_out=x_out, act=act, out=out, kernel_ms=ms.value, stamps=stamps)
 
 
+def math(fn, x):
+    """A scalar function of the kernels, value by value: 0 lg_rcp_exact, 1 lg_inv_scale, 2 lg_gelu_d, 3 lg_gelu."""
+    H = load_hip()
+    H.lg_hip_math.argtypes = [C.c_int, f32p, C.c_size_t, f32p]
+    x = np.ascontiguousarray(x, np.float32)
+    out = np.zeros(x.size, np.float32)
+    hip_check(H.lg_hip_math(fn, x, x.size, out), "math")
+    return out
+
+
 def ple_inputs(pmp, proj_norm, pte_q4_0, n_tok, toks, n_layer, ple, E, eps=1e-6):
     """Isolated per-layer-input kernel through the C ABI.  pmp: [rows, n_layer*ple] raw projection; pte_q4_0: n_tok
     q4_0 rows of n_layer*ple; toks: [rows].  Returns [rows, n_layer*ple]."""

@@ -419,3 +419,28 @@ def test_gelu_from_tiny_to_saturated_gates(lg, ob, gpu_required, rows):
         fin = np.isfinite(ad)
         assert np.array_equal(r["ad"][j][fin].view(np.uint32), ad[fin].view(np.uint32)) and np.array_equal(np.isfinite(r["ad"][j]), fin)
         assert np.array_equal(r["aq"][j].reshape(-1, 32)[fin], aq.reshape(-1, 32)[fin])
+
+
+@pytest.mark.parametrize("fn", [0, 1])
+@pytest.mark.parametrize("exponent", [-100, -1, 0, 99])
+def test_reciprocal_of_every_mantissa(lg, gpu_required, fn, exponent):
+    """lg_rcp_exact and lg_inv_scale against the IEEE quotient for all 2^23 mantissas, at both ends of their range too."""
+    x = (np.arange(1 << 23, dtype=np.uint32) | np.uint32((127 + exponent) << 23)).view(np.float32)
+    assert np.array_equal(lg.hiplib.math(fn, x).view(np.uint32), (np.float32(1) / x).view(np.uint32))
+
+
+def test_scale_factor_outside_the_short_form(lg, gpu_required):
+    """lg_inv_scale beside 2^-100 and 2^100, of denormal and huge scales, of 0, negative values, infinities and NaN: 1/d, 0 where d is not positive."""
+    edge = np.concatenate([np.nextafter(np.float32(2.0 ** e), np.float32(d), dtype=np.float32)[None] for e in (-100, 100, -126) for d in (0, np.inf)])
+    x = np.concatenate([edge, np.float32([2.0 ** -100, 2.0 ** 100, 2.0 ** -126, 2.0 ** -149, 2.0 ** -130, 3e38, 0.0, -0.0, -1.0, np.inf, -np.inf, np.nan])])
+    with np.errstate(divide="ignore", over="ignore"):
+        want = np.where(x > 0, np.float32(1) / x, np.float32(0)).astype(np.float32)
+    assert np.array_equal(lg.hiplib.math(1, x).view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("part", range(4))
+def test_gelu_without_branches_is_the_defined_one(lg, gpu_required, part):
+    """lg_gelu_d against lg_gelu, which the oracle shares, over the bit patterns of all floats (every 61st, 70 million), NaN for NaN."""
+    x = np.arange(part, 1 << 32, 4 * 61, dtype=np.uint64).astype(np.uint32).view(np.float32)
+    a, b = lg.hiplib.math(2, x), lg.hiplib.math(3, x)
+    assert np.array_equal(np.isnan(a), np.isnan(b)) and not (a.view(np.uint32) != b.view(np.uint32))[~np.isnan(b)].any()
