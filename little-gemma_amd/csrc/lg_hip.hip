@@ -11,6 +11,7 @@
 #include <string.h>
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <chrono>
 #include <map>
 #include <mutex>
@@ -277,7 +278,7 @@ struct lg_hip_kv {
     float *pm = nullptr, *pl = nullptr, *pacc = nullptr;
     unsigned id = 0;
 };
-static unsigned g_kv_ids = 0;
+static std::atomic<unsigned> g_kv_ids{0};      // (a thread per model creates caches; a graph is kept for a cache by its id)
 static int cu_count();
 
 template <typename T>
