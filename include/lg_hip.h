@@ -8,8 +8,8 @@
  *
  * Threading: one caller thread per model, like the reference backends
  * (src/cuda/model-cuda.cuh:724-726); calls on one model are not re-entrant.
- * Steps of several models on one device overlap only where no launch of theirs waits inside itself; the others run one
- * after another, in the order in which they were launched.  That holds within a process: two processes that drive one
+ * Of several models at work on one device, one at a time has launches that wait inside themselves; the steps of the
+ * others take separate kernels meanwhile, with the same results.  That holds within a process: two processes that drive one
  * device at the same time can keep each other's launches from getting all their workgroups, and the call then returns -9.
  * Device errors are returned, never exit(): the caller decides (model-hip.c prints and exits
  * like CUDA_CHECK, src/cuda/model-cuda.cuh:34-36).

@@ -15,6 +15,7 @@
 #include <chrono>
 #include <map>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <type_traits>
 #include <thread>
@@ -198,8 +199,10 @@ struct lg_hip_model {
     std::map<std::string, HostTensor> host;
     bool numbered = false;             // every layer has a launch number of its own (StepCtl.launch): kernels whose workgroups wait for one another may run
     struct Turns *turns = nullptr;                         // of its device
-    hipEvent_t ev_turn = nullptr;                          // end of the steps it has launched, for another model's to wait for
+    hipEvent_t ev_turn = nullptr;                          // end of the steps it has launched, for another model to ask about
     bool turn_recorded = false;                            // ev_turn holds the end of its latest step already
+    bool launching = false;                                // a step of it is being launched or captured: its stream is its own
+    bool plain = false;                                    // the step that is being launched takes the kernels that wait for nobody
     std::vector<std::pair<void *, size_t>> marks;          // memory whose words carry launch numbers (mark_alloc)
     int marked_steps = 0;                                  // steps since it was last cleared (count_steps)
     bool committed = false, wide_built = false;    // wide_built: the matrices' wide forms exist
@@ -288,12 +291,13 @@ static int dev_alloc(lg_hip_model *m, T **p, size_t n) {
     return 0;
 }
 
-// Steps with launches whose workgroups wait for one another, of several models on a device.  Such a launch is sound when its workgroups are all resident
+// Launches whose workgroups wait for one another, of several models on a device.  Such a launch is sound when its workgroups are all resident
 // at some time: a waiting one keeps its CU, up to a whole one.  Two of them at a time, on the streams of two models, could each hold a part of an
-// XCD's 32 and wait for the rest until both give up.  So a step with such launches starts behind the end of the last one of another model; the
-// steps of one model are ordered by its stream.  With one model at work this is one uncontended lock a step.
+// XCD's 32 and wait for the rest until both give up.  So one model has them at a time: the one whose latest such step has not ended yet.  A step of another
+// model takes the kernels that wait for nobody (same bits) and overlaps with it as streams do.  Two models of 512 values, a step each at a time: 106 us
+// with separate kernels in both, 162 when the steps of one waited for the other's, 97 and 80 so; of 2560 values and 5 rows 156, 316, 165 and 155.  With one model at work this is an uncontended lock twice a step.
 struct Turns {
-    std::mutex mu;                             // held while a step is launched or captured
+    std::mutex mu;                             // not held over launches: a thread that launches many steps would keep the others out
     lg_hip_model *last = nullptr;              // whose step with such launches was the latest
 };
 static Turns *turns_of(int device) {
@@ -302,22 +306,10 @@ static Turns *turns_of(int device) {
     std::lock_guard<std::mutex> hold(mu);
     return &(*all)[device];
 }
-// The lock under which a step of m (or a round of a draft head m) is launched; `waits`: with launches of that kind
-static int take_turn(lg_hip_model *m, bool waits, std::unique_lock<std::mutex> &turn) {
-    lg_hip_model *own = m->target ? m->target : m;         // (a draft head has its target's stream)
-    turn = std::unique_lock<std::mutex>(own->turns->mu);
-    if (!waits) return 0;
-    lg_hip_model *&last = own->turns->last;
-    if (last && last != own) {
-        if (!last->turn_recorded) HIP_TRY(hipEventRecord(last->ev_turn, last->stream));
-        last->turn_recorded = true;
-        HIP_TRY(hipStreamWaitEvent(own->stream, last->ev_turn, 0));
-    }
-    last = own;
-    own->turn_recorded = false;
-    return 0;
-}
-// Ahead of long work without such launches (a prompt's blocks), which another model's steps need not wait for
+static lg_hip_model *stream_owner(lg_hip_model *m) { return m->target ? m->target : m; }       // (a draft head has its target's stream)
+// Whether a step of m that is launched now may hold such launches
+static bool may_wait(const lg_hip_model *m) { return m->numbered && !(m->target ? m->target : m)->plain; }
+// Ahead of long work without such launches (a prompt's blocks): another model may have them meanwhile
 static int mark_turn(lg_hip_model *m) {
     std::lock_guard<std::mutex> turn(m->turns->mu);
     if (m->turns->last != m || m->turn_recorded) return 0;
@@ -330,7 +322,12 @@ static int take_turn_alone(std::unique_lock<std::mutex> &turn) {
     int device = 0;
     HIP_TRY(hipGetDevice(&device));
     Turns *t = turns_of(device);
-    turn = std::unique_lock<std::mutex>(t->mu);
+    for (;;) {
+        turn = std::unique_lock<std::mutex>(t->mu);
+        if (!t->last || !t->last->launching) break;
+        turn.unlock();
+        std::this_thread::yield();
+    }
     if (t->last) HIP_TRY(hipStreamSynchronize(t->last->stream));
     return 0;
 }
@@ -1250,7 +1247,7 @@ static void launch_xffn(Launcher &lx, const XffnArgs &a, int cls) {
 // The per-layer-input block of a verify block of `rows` rows as the one-XCD launch lg_k_ple_tail: q4_0 matrices of the
 // 256-wide per-layer input, at most LG_XTAIL_UNITS (gate block, row) units, a chip whose workgroups are dealt over 8 XCDs
 static bool use_ple_tail(const lg_hip_model *m, int rows) {
-    if (!m->ple || !m->tsync || !m->numbered || m->xcd_tail <= 0 || m->target) return false;
+    if (!m->ple || !m->tsync || !may_wait(m) || m->xcd_tail <= 0 || m->target) return false;
     if (m->ple != 256 || (m->ple / 32) * rows > LG_XTAIL_UNITS || m->E % 256 || m->E > 4096 || (m->E + 1023) / 1024 > m->ple / 32) return false;
     const int U = (m->ple / 32) * rows;
     const bool spread = m->tail_spread && (rows >= 5 || rows <= 2);   // (lg_k_ple_tail_s: 8 wavefronts per unit, enough of them at every width)
@@ -1262,7 +1259,7 @@ static bool use_ple_tail(const lg_hip_model *m, int rows) {
 }
 // One row of a narrow model: a layer from the merge on, and the next layer's q/k/v, as one launch (every kernel choice left as it comes)
 static bool use_narrow(const lg_hip_model *m, int rows) {
-    return rows == 1 && m->narrow && m->nsync && m->fuse_rows && m->xcd_tail == 1 && m->tail_spread == 1 && !m->xcd_attn_tail && !m->merge_o && !m->fork_ple;
+    return rows == 1 && m->narrow && m->nsync && may_wait(m) && m->fuse_rows && m->xcd_tail == 1 && m->tail_spread == 1 && !m->xcd_attn_tail && !m->merge_o && !m->fork_ple;
 }
 // Slices of the E output rows per (head, row) of lg_k_merge_o: a divisor of the E/64 chunks that leaves at most two
 // chunks per wavefront, the largest that keeps the launch within one workgroup per CU (else the smallest)
@@ -1313,18 +1310,52 @@ static int step_tiles(const lg_hip_model *m, const lg_hip_kv *kv, const Layer &y
 // ahead of gate/up is part of this launch: asked for in another one, by rows_geglu or xcd_ffn, it stays there)
 static bool use_attn_out(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
     if (rows >= 4 && ((m->rows_geglu && m->E == 2560) || (m->xcd_ffn && y.xgu))) return false;
-    return m->attn_out && m->aosync && attn_out_shape(m, y) && (rows <= LG_AOUT_DOT_ROWS ? tiles <= LG_AOUT_TILES : y.wo_ch && tiles <= LG_AOUT_BATCH);
+    return m->attn_out && m->aosync && may_wait(m) && attn_out_shape(m, y) && (rows <= LG_AOUT_DOT_ROWS ? tiles <= LG_AOUT_TILES : y.wo_ch && tiles <= LG_AOUT_BATCH);
 }
 static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
-    if (!y.wo_ch || !m->tsync || !m->numbered || !attn_tail_shape(y.qd, m->E, nullptr, nullptr) || m->xcd_attn_tail <= 0 || (m->xcd_attn_tail == 1 && rows < 3)) return false;
+    if (!y.wo_ch || !m->tsync || !may_wait(m) || !attn_tail_shape(y.qd, m->E, nullptr, nullptr) || m->xcd_attn_tail <= 0 || (m->xcd_attn_tail == 1 && rows < 3)) return false;
     const int slices = (m->E + 1023) / 1024;
     return tiles < 128 && m->H * rows <= 2 * LG_XCD_WGS && slices * rows <= LG_XCD_WGS && y.hd % 32 == 0 && y.hd <= 256;
 }
-// Whether a step may hold launches whose workgroups wait for one another
+// Whether a step has launches whose workgroups wait for one another, if it may
 static bool step_waits(const lg_hip_model *m, int rows) {
-    return m->numbered && (use_narrow(m, rows) || (m->attn_out && m->aosync) || use_ple_tail(m, rows) || m->rows_geglu || m->xcd_attn_tail > 0 ||
+    return may_wait(m) && (use_narrow(m, rows) || (m->attn_out && m->aosync) || use_ple_tail(m, rows) || m->rows_geglu || m->xcd_attn_tail > 0 ||
                            (rows >= 4 && ((m->down_m == 1 && m->dmsync) || m->xcd_ffn)));
 }
+// Held while a step of m is launched (or a round of `head` and m, its target); begin() finds out whether it may have such launches
+struct Turn {
+    lg_hip_model *own = nullptr;
+    int begin(lg_hip_model *m, int rows, const lg_hip_model *head = nullptr) {
+        own = stream_owner(m);
+        std::lock_guard<std::mutex> lock(own->turns->mu);
+        own->launching = true;
+        own->plain = false;
+        return step_waits(m, rows) || (head && step_waits(head, 1)) ? claim() : 0;
+    }
+    ~Turn() {
+        if (!own) return;
+        std::lock_guard<std::mutex> lock(own->turns->mu);
+        own->launching = false;
+    }
+    int claim() {
+        lg_hip_model *&last = own->turns->last;
+        if (last && last != own) {
+            if (last->launching) { own->plain = true; return 0; }
+            if (!last->turn_recorded) HIP_TRY(hipEventRecord(last->ev_turn, last->stream));
+            last->turn_recorded = true;
+            const hipError_t e = hipEventQuery(last->ev_turn);
+            if (e == hipErrorNotReady) {
+                (void)hipGetLastError();                   // (no error, and not to be found as one by the next launch)
+                own->plain = true;
+                return 0;
+            }
+            if (e != hipSuccess) return fail(-100 - (int)e, "hipEventQuery: %s", hipGetErrorString(e));
+        }
+        last = own;
+        own->turn_recorded = false;
+        return 0;
+    }
+};
 template <int M>
 static void launch_attn_tail(Launcher &lx, const XattnTailArgs &a) {
     lg_hip_model *m = lx.m;
@@ -1661,7 +1692,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             // verify blocks: 1..3 rows through v_dot4 with scalar operands, 4..8 rows through the matrix cores
             // (its float work per tile does not grow with the row count); each has its own activation order
             constexpr bool mfma = M >= 4;
-            if (mfma && m->xffn_built && m->xcd_ffn && y.xgu && have_x && pend_dout && pend_parts == 1 && !pend_os) {
+            if (mfma && m->xffn_built && m->xcd_ffn && may_wait(m) && y.xgu && have_x && pend_dout && pend_parts == 1 && !pend_os) {
                 // the whole half as one launch partitioned by XCD: row work, gate/up + GeGLU and the XCD's K share of
                 // ffn_down; the consumer adds the 8 slabs (the top of the segment tree)
                 XffnArgs f{ y.xgu, y.xdn, m->x[cur], pend_dout, pend_w, y.ffn_norm, m->x[cur ^ 1], m->slabs, m->xq8, m->xact,
@@ -1677,7 +1708,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 // the row work as the first workgroups of the gate/up launch, whose other workgroups request their weights
                 // while it runs (lg_xrg.h); shapes whose K segment of E/256 tiles has a build
                 const int slices = (E + 1023) / 1024;
-                if (m->rows_geglu && m->rgsync && m->numbered && !ffn_rows_done && have_x && pend_dout && !pend_os && (pend_parts == 1 || pend_parts == 4) && (E == 2560 || E == 3840 || E == 512) &&
+                if (m->rows_geglu && m->rgsync && may_wait(m) && !ffn_rows_done && have_x && pend_dout && !pend_os && (pend_parts == 1 || pend_parts == 4) && (E == 2560 || E == 3840 || E == 512) &&
                     M * slices <= LG_RG_MAXP) {
                     RowsGegluArgs f{ m->x[cur], pend_dout, pend_w, y.ffn_norm, m->x[cur ^ 1], m->hq, E, pend_parts, slices, m->eps,
                                      y.wgu, y.nff, m->gq, dn_m ? 2 : 0, m->rgsync, L, m->wait_polls, m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr };
@@ -1701,7 +1732,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             }
             MmArgs d{ y.wdown, y.nff, E, m->dout, m->gq, nullptr };
             if (dn_m) {
-                DownMArgs dm{ y.wdn_m, (const uint32_t *)m->gq, m->dout, E, y.nff, m->down_m == 1 && m->numbered ? m->dmsync : nullptr, m->ctl, m->wait_polls, L };
+                DownMArgs dm{ y.wdn_m, (const uint32_t *)m->gq, m->dout, E, y.nff, m->down_m == 1 && may_wait(m) ? m->dmsync : nullptr, m->ctl, m->wait_polls, L };
                 launch_down_m<M>(lx, dm);
                 pend_parts = dm.sync ? 1 : 4;
             } else
@@ -1968,7 +1999,7 @@ static GraphKey graph_key(const lg_hip_model *m, const lg_hip_kv *kv, int rows, 
     put(what, 2); put(rows, 4); put(m->store_logits != 0, 1); put(m->draft_chain, 1); put(m->fuse_rows, 1); put(m->attn_rows, 1); put(m->attn_rows_fq, 1);
     put(m->head_mfma, 1); put(m->down_kq, 1); put(m->xcd_ffn, 1); put(m->fork_ple, 1); put(m->rows_geglu, 1); put(m->tail_stamps != 0, 1);
     put(m->tail_spread == 1 ? 1 : m->tail_spread ? 2 : 0, 2); put(m->xcd_tail, 2); put(m->down_m, 2); put(m->xcd_attn_tail, 2); put(m->merge_o, 2);
-    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->wait_polls, 17);
+    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->wait_polls, 17); put(may_wait(m), 1);
     return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices, 0 };
 }
 
@@ -1994,8 +2025,8 @@ static hipGraphExec_t capture_behind(hipStream_t st, F enqueue) {
 // (a first decode step on a new cache, E4B shape: 3.95 -> 2.28 ms; capturing and instantiating 341 launches takes 1.5).
 static int launch_step(lg_hip_model *m, lg_hip_kv *kv, int rows, bool with_head) {
     m->lread = m->lcoming = -1;
-    std::unique_lock<std::mutex> turn;
-    int rc = take_turn(m, step_waits(m, rows), turn);
+    Turn turn;
+    int rc = turn.begin(m, rows);
     if (rc || (rc = count_steps(m, 1))) return rc;
     if (!m->use_graph || m->prof.on) return enqueue_step_rows(m, kv, rows, with_head);
     const GraphKey key = graph_key(m, kv, rows, with_head ? 1 : 0);
@@ -2183,30 +2214,23 @@ extern "C" int lg_hip_mtp_rounds(lg_hip_model *d, lg_hip_kv *kv, int token, int 
     int32_t tk = token;
     if ((rc = load_block(t, &tk, 1, pos, false))) return rc;
     t->lread = t->lcoming = d->lread = d->lcoming = -1;
-    const bool waits = step_waits(t, rows) || step_waits(d, 1);
     if ((rc = count_steps(t, n_rounds)) || (rc = count_steps(d, n_rounds * (rows - 1)))) return rc;
-    if (!t->use_graph || t->prof.on || d->prof.on) {
-        for (int r = 0; r < n_rounds; ++r) {
-            std::unique_lock<std::mutex> turn;
-            if ((rc = take_turn(t, waits, turn)) || (rc = enqueue_round(d, kv, rows, false))) return rc;
+    const bool graphs = t->use_graph && !t->prof.on && !d->prof.on;
+    for (int r = 0; r < n_rounds; ++r) {
+        Turn turn;
+        if ((rc = turn.begin(t, rows, d))) return rc;
+        if (!graphs) {
+            if ((rc = enqueue_round(d, kv, rows, false))) return rc;
+            continue;
         }
-    } else {
         GraphKey key = graph_key(t, kv, rows, 2);
         key[3] = graph_key(d, kv, 1, 2)[1];
         auto it = d->graphs.find(key);            // kept by the head: the graph dies with it or with the cache
-        int r = 0;
-        if (it == d->graphs.end()) {               // the first round as launches, its graph while the device works on it
-            std::unique_lock<std::mutex> turn;
-            if ((rc = take_turn(t, waits, turn)) || (rc = enqueue_round(d, kv, rows, true)) || (rc = enqueue_round(d, kv, rows, false))) return rc;
-            it = d->graphs.emplace(key, capture_behind(t->stream, [&]() { return enqueue_round(d, kv, rows, false); })).first;
-            r = 1;
-        }
-        for (; r < n_rounds; ++r) {
-            std::unique_lock<std::mutex> turn;
-            if ((rc = take_turn(t, waits, turn))) return rc;
-            if (it->second) HIP_TRY(hipGraphLaunch(it->second, t->stream));
-            else if ((rc = enqueue_round(d, kv, rows, false))) return rc;
-        }
+        if (it == d->graphs.end()) {               // the first of them as launches, its graph while the device works on it
+            if ((rc = enqueue_round(d, kv, rows, true)) || (rc = enqueue_round(d, kv, rows, false))) return rc;
+            d->graphs.emplace(key, capture_behind(t->stream, [&]() { return enqueue_round(d, kv, rows, false); }));
+        } else if (it->second) HIP_TRY(hipGraphLaunch(it->second, t->stream));
+        else if ((rc = enqueue_round(d, kv, rows, false))) return rc;
     }
     const size_t nb = (size_t)n_rounds * rows;
     int32_t *res = t->pin + 64;
@@ -2253,14 +2277,14 @@ extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *tok
             int rows = left < kv->prompt_rows ? left : kv->prompt_rows, rc;
             const bool wide = wide_ok && !far_in_narrow_heads(m, kv, rows, pos0 + at + done);
             const bool first = at + done == 0;
-            std::unique_lock<std::mutex> turn;
+            Turn turn;
             if (wide && left > m->max_rows) rc = enqueue_prompt(m, kv, m->sched + done, rows, pos0 + at + done, first);
             else {                                           // a remainder that fits a verify block
                 rows = left < m->max_rows ? left : m->max_rows;
                 if (done) HIP_TRY(hipMemcpyAsync(m->sched, m->pin + 64 + done, (size_t)rows * 4, hipMemcpyHostToDevice, m->stream));   // (its kernels read the schedule from its start)
                 hipLaunchKernelGGL(lg_k_set_ctl, dim3(1), dim3(1), 0, m->stream, m->ctl, pos0 + at + done, first);
                 if (!wide) rc = launch_step(m, kv, rows, false);
-                else if (!(rc = take_turn(m, step_waits(m, rows), turn)) && !(rc = count_steps(m, 1)))
+                else if (!(rc = turn.begin(m, rows)) && !(rc = count_steps(m, 1)))
                     rc = enqueue_step_rows(m, kv, rows, false);                                         // (a single one: not worth a capture)
             }
             if (rc) return rc;
@@ -2390,7 +2414,7 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
             const int tiles = ((pos + rows - 1) >> 5) - (st >> 5) + 1;
             b[use_attn_tail(m, y, rows, tiles) ? KC_ATAIL : use_merge_o(m, y, rows, tiles) ? KC_MERGE : use_attn_out(m, y, rows, step_tiles(m, kv, y, rows, 0)) ? KC_ATAIL : KC_O] += (double)y.qd * m->E * q;
         }
-        if (m->xffn_built && m->xcd_ffn && rows >= 4) b[KC_FFN] += 3.0 * m->E * y.nff * q;
+        if (m->xffn_built && m->xcd_ffn && may_wait(m) && rows >= 4) b[KC_FFN] += 3.0 * m->E * y.nff * q;
         else { b[KC_GATEUP] += 2.0 * m->E * y.nff * q; b[KC_DOWN] += (double)y.nff * m->E * q; }
         if (m->ple && !y.winp_f && use_ple_tail(m, rows)) b[KC_TAIL] += 2.0 * m->E * m->ple * q;
         else if (m->ple) { const double pq = y.winp_f ? 4.0 : q; b[KC_PLEGATE] += (double)m->E * m->ple * pq; b[KC_PLEPROJ] += (double)m->ple * m->E * pq; }
@@ -2413,12 +2437,12 @@ extern "C" int lg_hip_profile_step(lg_hip_model *m, lg_hip_kv *kv, const int32_t
     int cnt[KC_COUNT] = { 0 };
     for (int r = 0; r < repeats + 1; ++r) {              // first pass warms up and is dropped
         if ((rc = load_block(m, toks, rows, pos, false))) return rc;
-        std::unique_lock<std::mutex> turn;
-        if ((rc = take_turn(m, step_waits(m, rows), turn)) || (rc = count_steps(m, 1))) return rc;
+        std::optional<Turn> turn(std::in_place);
+        if ((rc = turn->begin(m, rows)) || (rc = count_steps(m, 1))) return rc;
         m->prof.on = true;
         m->lread = m->lcoming = -1;
         rc = enqueue_step_rows(m, kv, rows, true);
-        turn.unlock();
+        turn.reset();
         m->prof.on = false;
         hipError_t e = hipStreamSynchronize(m->stream);
         if (!rc && e != hipSuccess) rc = fail(-100 - (int)e, "profile_step: %s", hipGetErrorString(e));

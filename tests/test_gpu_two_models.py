@@ -1,4 +1,4 @@
-"""Two models at work at once on one device: steps whose workgroups wait for one another take turns, results are those of a model alone."""
+"""Two models at work at once on one device: one of them has launches whose workgroups wait for one another, results are those of a model alone."""
 import ctypes as C
 import threading
 

@@ -61,3 +61,36 @@ def test_more_layers_than_launch_numbers(lg, gpu_required, model_path, monkeypat
             assert not any(launches.get(k, 0) for k in ("ffn_xcd", "ple_tail", "attn_tail")), launches
     finally:
         gpu.close()
+
+
+@pytest.mark.parametrize("name,over", [("tiny_full", {"n_embd": 2560, "n_head": 8, "head_dim": 256, "head_dim_full": 0, "n_ff": 8192, "n_vocab": 2048}), ("tiny_full", {}),
+                                       ("tiny", {"n_embd": 2560, "n_head": 8, "head_dim": 256, "n_ff": 8192, "n_vocab": 2048}), ("tiny_full_bf16", {"n_ff": 8192})])
+def test_steps_without_such_launches_leave_the_same_bits(lg, gpu_required, model_path, name, over):
+    """What a step takes while another model has such launches: every kernel that waits for nobody, at every width, against the default's logits,
+    hidden state and cache rows."""
+    path, spec = model_path(name, **over)
+    rng = np.random.default_rng(4)
+    V, owners = spec["n_vocab"], spec["n_layer"] - spec["shared_kv_layers"]
+    prompt, toks = rng.integers(1, V, 70).astype(np.int32), rng.integers(1, V, 40).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, 160, max_rows=8)
+    got = []
+    try:
+        gpu.set_option("store_logits", 1)
+        for opts in (dict(narrow=1, attn_out=1, xcd_tail=1, down_m=1), dict(narrow=0, attn_out=0, xcd_tail=0, down_m=2)):
+            for k, v in opts.items():
+                gpu.set_option(k, v)
+            gpu.new_cache()
+            gpu.prefill(prompt, 0)
+            pos, res = 70, []
+            for rows in range(1, 9):
+                print(f"{name} {over} {opts}: {rows} rows", flush=True)
+                adv, out = gpu.forward_spec(toks[pos - 70:pos - 70 + rows], pos)
+                res += [out, gpu.last_hidden(spec["n_embd"])] + [gpu.logits_row(j, V) for j in range(rows)]
+                pos += rows
+            launches = {k["name"]: k["launches"] for k in gpu.profile_step(toks[:8], 100, 1)}
+            if not opts["narrow"]:
+                assert not any(launches.get(k, 0) for k in ("ple_tail", "attn_tail", "ffn_xcd")), launches
+            got.append([np.ascontiguousarray(r).view(np.uint8) for r in res + [gpu.kv_read(L, w) for L in range(owners) for w in (0, 1)]])
+    finally:
+        gpu.close()
+    assert all(np.array_equal(a, b) for a, b in zip(*got))

@@ -83,3 +83,56 @@ def test_marks_that_come_round(cleared_every, sound):
             return
         assert taken
     assert sound
+
+
+class Model:
+    """A caller thread and its stream: steps that were launched and have not ended, True for one with launches that wait."""
+
+    def __init__(self):
+        self.launching = self.plain = self.recorded = False
+        self.stream, self.mark = [], 0                          # mark: how many of the stream's steps lie ahead of the recorded event
+
+
+def caller(models, me, turns, steps, checks_launching):
+    """The calls of one model: begin (under the lock: one turn of the model here), then the launches, then the end."""
+    for _ in range(steps):
+        me.launching, me.plain = True, False
+        last = turns[0]
+        if last is not None and last is not me:
+            if checks_launching and last.launching:
+                me.plain = True
+            else:
+                if not last.recorded:
+                    last.recorded, last.mark = True, len(last.stream)
+                me.plain = last.mark > 0
+        if not me.plain:
+            turns[0], me.recorded = me, False
+        yield
+        me.stream.append(not me.plain)
+        yield
+        me.launching = False
+        assert sum(any(m.stream) for m in models) <= 1, "two models have launches that wait"
+        yield
+
+
+@pytest.mark.parametrize("checks_launching", [True, False])
+def test_one_model_at_a_time_has_launches_that_wait(checks_launching):
+    """Threads and streams in any order: the latest model with such launches keeps them until its stream has ended them.  Without the look at a step that
+    is still being launched the model sees the fault: the event lies ahead of it."""
+    import random
+    seen = False
+    for seed in range(400):
+        rng, turns, models = random.Random(seed), [None], [Model() for _ in range(3)]
+        live = [caller(models, m, turns, 6, checks_launching) for m in models]
+        try:
+            while live:
+                g = rng.choice(live)
+                if next(g, "left") == "left":
+                    live.remove(g)
+                m = rng.choice(models)
+                if m.stream and rng.random() < 0.4:             # the device ends a step
+                    m.stream.pop(0)
+                    m.mark = max(0, m.mark - 1)
+        except AssertionError:
+            seen = True
+    assert seen is not checks_launching
