@@ -47,6 +47,17 @@ static int fail(int code, const char *fmt, ...) {
 #define HIP_TRY(expr) do { hipError_t e_ = (expr); if (e_ != hipSuccess) \
     return fail(-100 - (int)e_, "%s failed: %s (%s:%d)", #expr, hipGetErrorString(e_), __FILE__, __LINE__); } while (0)
 
+// Copies and clears that are done when the call returns, on a model's own stream: the forms without a stream fail (hipErrorStreamCaptureImplicit)
+// while any other thread of the process captures, a step of another model, say.
+static hipError_t copy_now(hipStream_t st, void *dst, const void *src, size_t n, hipMemcpyKind kind) {
+    const hipError_t e = hipMemcpyAsync(dst, src, n, kind, st);
+    return e == hipSuccess ? hipStreamSynchronize(st) : e;
+}
+static hipError_t clear_now(hipStream_t st, void *dst, int value, size_t n) {
+    const hipError_t e = hipMemsetAsync(dst, value, n, st);
+    return e == hipSuccess ? hipStreamSynchronize(st) : e;
+}
+
 extern "C" const char *lg_hip_last_error(void) { return g_err; }
 extern "C" int lg_hip_device_count(void) {
     int n = 0;
@@ -338,7 +349,7 @@ template <typename T>
 static int mark_alloc(lg_hip_model *m, T **p, size_t n = 1) {
     if (dev_alloc(m, p, n)) return -7;
     m->marks.emplace_back((void *)*p, n * sizeof(T));
-    HIP_TRY(hipMemset(*p, 0, n * sizeof(T)));
+    HIP_TRY(clear_now(m->stream, *p, 0, n * sizeof(T)));
     return 0;
 }
 // Called ahead of `steps` more steps of the model on its stream, never under capture.  A mark has 28 bits, so the numbers come round after 2^20 steps (half an hour
@@ -422,7 +433,7 @@ static int upload_vec(lg_hip_model *m, const std::string &name, size_t n, bool r
     for (uint32_t i = 0; i < t->n_dims; ++i) have *= t->dims[i];
     if (t->type != 0 || have != n) return fail(-6, "model_commit: %s must be f32 with %zu elements", name.c_str(), n);
     if (dev_alloc(m, out, n)) return -7;
-    HIP_TRY(hipMemcpy(*out, t->data, n * 4, hipMemcpyHostToDevice));
+    HIP_TRY(copy_now(m->stream, *out, t->data, n * 4, hipMemcpyHostToDevice));
     return 0;
 }
 
@@ -454,7 +465,7 @@ static int upload_float_mat(lg_hip_model *m, const HostTensor *t, const std::str
         src = wide.data();
     }
     if (dev_alloc(m, out, n)) return -7;
-    HIP_TRY(hipMemcpy(*out, src, n * 4, hipMemcpyHostToDevice));
+    HIP_TRY(copy_now(m->stream, *out, src, n * 4, hipMemcpyHostToDevice));
     return 0;
 }
 // upload a tiled matrix whose virtual rows are given by `rows`
@@ -466,7 +477,7 @@ static int upload_tiled(lg_hip_model *m, const std::vector<const uint8_t *> &row
     if (rowblocks) repack_rowblocks(rows.data(), k, (int)rows.size(), stage.data());
     else repack_rows(rows.data(), k, (int)rows.size(), stage.data());
     if (dev_alloc(m, out, bytes)) return -7;
-    HIP_TRY(hipMemcpy(*out, stage.data(), bytes, hipMemcpyHostToDevice));
+    HIP_TRY(copy_now(m->stream, *out, stage.data(), bytes, hipMemcpyHostToDevice));
     return 0;
 }
 // the wide form of an uploaded matrix: 0.81 bytes a weight beside the 0.56 of its tiles.  Only prompt blocks read it: none for a
@@ -632,7 +643,7 @@ static const float *rope_table(lg_hip_model *m, int is_local, int hd, int *rc) {
     const float base = is_local ? m->base_swa : m->base;
     for (int i = 0; i < hd / 2; ++i) tab[i] = powf(base, -2.0f * (float)i / (float)hd);   // src/cpu/model-cpu.c:90
     float *d = nullptr;
-    if (hipMalloc((void **)&d, tab.size() * 4) != hipSuccess || hipMemcpy(d, tab.data(), tab.size() * 4, hipMemcpyHostToDevice) != hipSuccess) {
+    if (hipMalloc((void **)&d, tab.size() * 4) != hipSuccess || copy_now(m->stream, d, tab.data(), tab.size() * 4, hipMemcpyHostToDevice) != hipSuccess) {
         *rc = fail(-7, "model_commit: rope table upload failed");
         return nullptr;
     }
@@ -673,7 +684,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
             return fail(-6, "model_commit: per_layer_token_embd.weight must be q4_0 %llu x %d", (unsigned long long)total, m->n_vocab);
         const size_t bytes = (size_t)m->n_vocab * (total / 32) * 18;
         if (dev_alloc(m, &m->pte, bytes)) return -7;
-        HIP_TRY(hipMemcpy(m->pte, t->data, bytes, hipMemcpyHostToDevice));
+        HIP_TRY(copy_now(m->stream, m->pte, t->data, bytes, hipMemcpyHostToDevice));
         const HostTensor *p = find(m, "per_layer_model_proj.weight");
         if (float_typed(p)) {
             if ((rc = upload_float_mat(m, p, "per_layer_model_proj.weight", E, total, &m->pmp_f))) return rc;
@@ -744,7 +755,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
             stage.resize((size_t)E * (y.qd / 32) * 18);
             pack_o_chains(rows.data(), y.qd, E, stage.data());
             if (dev_alloc(m, &y.wo_ch, stage.size())) return -7;
-            HIP_TRY(hipMemcpy(y.wo_ch, stage.data(), stage.size(), hipMemcpyHostToDevice));
+            HIP_TRY(copy_now(m->stream, y.wo_ch, stage.data(), stage.size(), hipMemcpyHostToDevice));
         }
         if (getenv("LG_HIP_MERGE_O") && atoi(getenv("LG_HIP_MERGE_O")) > 0 && !m->target && m->H == 8 && lg_segments(y.qd) == 8 && E % 64 == 0 && y.hd % 32 == 0 && y.hd <= 512 &&
             (rc = upload_tiled(m, rows, y.qd, &y.wo_rb, stage, true))) return rc;
@@ -768,7 +779,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
                 xstage.resize(256 * dg.wg_bytes);
                 pack_down_m((const uint8_t *)d->data, dg, xstage.data());
                 if (dev_alloc(m, &y.wdn_m, 256 * dg.wg_bytes)) return -7;
-                HIP_TRY(hipMemcpy(y.wdn_m, xstage.data(), 256 * dg.wg_bytes, hipMemcpyHostToDevice));
+                HIP_TRY(copy_now(m->stream, y.wdn_m, xstage.data(), 256 * dg.wg_bytes, hipMemcpyHostToDevice));
                 if (!m->dmsync) {
                     if (mark_alloc(m, &m->dmsync)) return -7;
                 }
@@ -778,10 +789,10 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
             xstage.resize(256 * (xg.gu_bytes > xg.dn_bytes ? xg.gu_bytes : xg.dn_bytes));
             xffn_pack_gu((const uint8_t *)g->data, (const uint8_t *)u->data, xg, xstage.data());
             if (dev_alloc(m, &y.xgu, 256 * xg.gu_bytes)) return -7;
-            HIP_TRY(hipMemcpy(y.xgu, xstage.data(), 256 * xg.gu_bytes, hipMemcpyHostToDevice));
+            HIP_TRY(copy_now(m->stream, y.xgu, xstage.data(), 256 * xg.gu_bytes, hipMemcpyHostToDevice));
             xffn_pack_dn((const uint8_t *)d->data, xg, xstage.data());
             if (dev_alloc(m, &y.xdn, 256 * xg.dn_bytes)) return -7;
-            HIP_TRY(hipMemcpy(y.xdn, xstage.data(), 256 * xg.dn_bytes, hipMemcpyHostToDevice));
+            HIP_TRY(copy_now(m->stream, y.xdn, xstage.data(), 256 * xg.dn_bytes, hipMemcpyHostToDevice));
         }
         if (m->ple) {
             if (m->ple != 256) return fail(-2, "model_commit: per-layer width %d (256 is built)", m->ple);
@@ -851,8 +862,8 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
     if (!m->target) {                        // hand-over state of the one-XCD kernels (lg_xtail.h)
         if (mark_alloc(m, &m->tsync) || mark_alloc(m, &m->rgsync) || dev_alloc(m, &m->tstamps, (size_t)2 * LG_XTAIL_UNITS * 8) ||
             (m->ple > 0 && (mark_alloc(m, &m->tgf, (size_t)LG_HIP_MAX_ROWS * m->ple) || mark_alloc(m, &m->tpr, (size_t)LG_HIP_MAX_ROWS * E)))) return -7;
-        HIP_TRY(hipMemset(m->tstamps, 0, (size_t)2 * LG_XTAIL_UNITS * 8 * 8));
-        HIP_TRY(hipMemset(m->aq, 0, qb(max_qd)));       // (row slots past the block are read as operand rows of the matrix cores)
+        HIP_TRY(clear_now(m->stream, m->tstamps, 0, (size_t)2 * LG_XTAIL_UNITS * 8 * 8));
+        HIP_TRY(clear_now(m->stream, m->aq, 0, qb(max_qd)));       // (row slots past the block are read as operand rows of the matrix cores)
         if (getenv("LG_HIP_XCD_TAIL")) m->xcd_tail = atoi(getenv("LG_HIP_XCD_TAIL"));
     }
     if (narrow_shape(m)) {
@@ -871,15 +882,15 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
     if (xffn) {
         if (dev_alloc(m, &m->slabs, (size_t)LG_XCDS * max_rows * E) || dev_alloc(m, &m->xact, (size_t)LG_XCDS * max_rows * xg.C) ||
             dev_alloc(m, &m->xq8, (size_t)LG_XCDS * xg.nb * LG_MU_DWORDS) || mark_alloc(m, &m->xsync)) return -7;
-        HIP_TRY(hipMemset(m->xq8, 0, (size_t)LG_XCDS * xg.nb * LG_MU_DWORDS * 4));        // row slots past the block are read as operand rows
+        HIP_TRY(clear_now(m->stream, m->xq8, 0, (size_t)LG_XCDS * xg.nb * LG_MU_DWORDS * 4));        // row slots past the block are read as operand rows
         m->xffn_built = true; m->xffn_cls = xffn_class_of(xg);
         m->xcd_ffn = getenv("LG_HIP_XCD_FFN") && atoi(getenv("LG_HIP_XCD_FFN")) != 0;     // off unless asked for: the separate kernels are faster (see lg_xffn.h)
         m->xffn_delay = 0x100;
     }
     HIP_TRY(hipHostMalloc((void **)&m->lstage, (size_t)2 * m->n_vocab * 4, hipHostMallocDefault));
     memset(m->lstage, 0, (size_t)2 * m->n_vocab * 4);       // (the host's pages of it, 0.4 ms a MB when first touched)
-    HIP_TRY(hipMemset(m->ctl, 0, sizeof(StepCtl)));
-    HIP_TRY(hipMemset(m->g_hidden, 0, (size_t)E * 4));
+    HIP_TRY(clear_now(m->stream, m->ctl, 0, sizeof(StepCtl)));
+    HIP_TRY(clear_now(m->stream, m->g_hidden, 0, (size_t)E * 4));
     m->sched_cap = 4096;
     if (dev_alloc(m, &m->sched, (size_t)m->sched_cap * LG_HIP_MAX_ROWS) || dev_alloc(m, &m->out, (size_t)m->sched_cap * LG_HIP_MAX_ROWS) ||
         dev_alloc(m, &m->adv, (size_t)m->sched_cap))
@@ -957,7 +968,7 @@ extern "C" int lg_hip_kv_create(lg_hip_model *m, int max_seq, lg_hip_kv **out) {
         const size_t bytes = (size_t)kv->seq[L] * y.kd * 2;
         hipError_t e1 = hipMalloc((void **)&kv->k[L], bytes), e2 = hipMalloc((void **)&kv->v[L], bytes);
         if (e1 != hipSuccess || e2 != hipSuccess) { lg_hip_kv_destroy(kv); return fail(-7, "kv_create: out of device memory at layer %d", L); }
-        (void)hipMemset(kv->k[L], 0, bytes); (void)hipMemset(kv->v[L], 0, bytes);
+        (void)hipMemsetAsync(kv->k[L], 0, bytes, m->stream); (void)hipMemsetAsync(kv->v[L], 0, bytes, m->stream);
     }
     const size_t slots = (size_t)m->max_rows * m->H * kv->tiles_max, grant = pbytes / ((size_t)max_hd * 4 + 8) * max_hd * 4;
     auto most = [&](auto need) { size_t n = 0; for (const Layer &y : m->L) n = std::max(n, need(y)); return n; };
@@ -1015,7 +1026,7 @@ extern "C" int lg_hip_kv_write(lg_hip_kv *kv, int layer, int which, int row0, in
     if (rc) return rc;
     HIP_TRY(hipSetDevice(kv->m->device));
     HIP_TRY(hipStreamSynchronize(kv->m->stream));
-    HIP_TRY(hipMemcpy(base + off, src, bytes, hipMemcpyHostToDevice));
+    HIP_TRY(copy_now(kv->m->stream, base + off, src, bytes, hipMemcpyHostToDevice));
     return 0;
 }
 extern "C" int lg_hip_kv_read(const lg_hip_kv *kv, int layer, int which, int row0, int n, uint16_t *dst) {
@@ -1024,7 +1035,7 @@ extern "C" int lg_hip_kv_read(const lg_hip_kv *kv, int layer, int which, int row
     if (rc) return rc;
     HIP_TRY(hipSetDevice(kv->m->device));
     HIP_TRY(hipStreamSynchronize(kv->m->stream));
-    HIP_TRY(hipMemcpy(dst, base + off, bytes, hipMemcpyDeviceToHost));
+    HIP_TRY(copy_now(kv->m->stream, dst, base + off, bytes, hipMemcpyDeviceToHost));
     return 0;
 }
 extern "C" int lg_hip_kv_save_prefix(lg_hip_kv *kv, int n) {
@@ -1040,8 +1051,8 @@ extern "C" int lg_hip_kv_save_prefix(lg_hip_kv *kv, int n) {
         if (!bytes) continue;
         HIP_TRY(hipMalloc((void **)&kv->px_k[L], bytes));
         HIP_TRY(hipMalloc((void **)&kv->px_v[L], bytes));
-        HIP_TRY(hipMemcpy(kv->px_k[L], kv->k[L], bytes, hipMemcpyDeviceToDevice));
-        HIP_TRY(hipMemcpy(kv->px_v[L], kv->v[L], bytes, hipMemcpyDeviceToDevice));
+        HIP_TRY(copy_now(kv->m->stream, kv->px_k[L], kv->k[L], bytes, hipMemcpyDeviceToDevice));
+        HIP_TRY(copy_now(kv->m->stream, kv->px_v[L], kv->v[L], bytes, hipMemcpyDeviceToDevice));
     }
     return 0;
 }
@@ -2301,7 +2312,7 @@ extern "C" int lg_hip_tail_stamps(lg_hip_model *m, int which, unsigned long long
     if (cap < LG_XTAIL_UNITS * 8) return fail(-2, "tail_stamps: room for %d values needed", LG_XTAIL_UNITS * 8);
     HIP_TRY(hipSetDevice(m->device));
     HIP_TRY(hipStreamSynchronize(m->stream));
-    HIP_TRY(hipMemcpy(dst, m->tstamps + (size_t)which * LG_XTAIL_UNITS * 8, (size_t)LG_XTAIL_UNITS * 8 * 8, hipMemcpyDeviceToHost));
+    HIP_TRY(copy_now(m->stream, dst, m->tstamps + (size_t)which * LG_XTAIL_UNITS * 8, (size_t)LG_XTAIL_UNITS * 8 * 8, hipMemcpyDeviceToHost));
     return LG_XTAIL_UNITS;
 }
 
@@ -2309,7 +2320,7 @@ extern "C" int lg_hip_get_hidden(lg_hip_model *m, float *dst) {
     if (!m || !dst) return fail(-1, "get_hidden: null argument");
     HIP_TRY(hipSetDevice(m->device));
     HIP_TRY(hipStreamSynchronize(m->stream));
-    HIP_TRY(hipMemcpy(dst, m->g_hidden, (size_t)m->E * 4, hipMemcpyDeviceToHost));
+    HIP_TRY(copy_now(m->stream, dst, m->g_hidden, (size_t)m->E * 4, hipMemcpyDeviceToHost));
     return 0;
 }
 extern "C" int lg_hip_set_hidden_row(lg_hip_model *m, int row) {
@@ -2347,9 +2358,9 @@ extern "C" int lg_hip_schedule_load(lg_hip_model *m, const int32_t *toks, int n_
     for (size_t i = 0; i < (size_t)n_steps * rows; ++i) if (toks[i] < 0 || toks[i] >= m->n_vocab) return fail(-2, "schedule_load: token id %d outside the vocabulary", toks[i]);
     HIP_TRY(hipSetDevice(m->device));
     HIP_TRY(hipStreamSynchronize(m->stream));
-    HIP_TRY(hipMemcpy(m->sched, toks, (size_t)n_steps * rows * 4, hipMemcpyHostToDevice));
+    HIP_TRY(copy_now(m->stream, m->sched, toks, (size_t)n_steps * rows * 4, hipMemcpyHostToDevice));
     StepCtl c{ pos0, 0, 0, 0, 0 };
-    HIP_TRY(hipMemcpy(m->ctl, &c, offsetof(StepCtl, launch), hipMemcpyHostToDevice));
+    HIP_TRY(copy_now(m->stream, m->ctl, &c, offsetof(StepCtl, launch), hipMemcpyHostToDevice));
     m->sched_steps = n_steps; m->sched_rows = rows; m->sched_pos0 = pos0; m->sched_loaded = n_steps;
     return 0;
 }
@@ -2370,13 +2381,13 @@ extern "C" int lg_hip_schedule_wait(lg_hip_model *m, int32_t *out, int32_t *adv,
     HIP_TRY(hipSetDevice(m->device));
     HIP_TRY(hipStreamSynchronize(m->stream));
     StepCtl c;
-    HIP_TRY(hipMemcpy(&c, m->ctl, sizeof c, hipMemcpyDeviceToHost));
+    HIP_TRY(copy_now(m->stream, &c, m->ctl, sizeof c, hipMemcpyDeviceToHost));
     { const int erc = step_err("schedule_wait", c.err); if (erc) return erc; }
     // the step counter is device state: never copy more than the schedule that was loaded holds
     if (c.step < 0 || c.step > m->sched_loaded)
         return fail(-6, "schedule_wait: the device reports %d steps done, %d were loaded", c.step, m->sched_loaded);
-    if (out) HIP_TRY(hipMemcpy(out, m->out, (size_t)c.step * m->sched_rows * 4, hipMemcpyDeviceToHost));
-    if (adv) HIP_TRY(hipMemcpy(adv, m->adv, (size_t)c.step * 4, hipMemcpyDeviceToHost));
+    if (out) HIP_TRY(copy_now(m->stream, out, m->out, (size_t)c.step * m->sched_rows * 4, hipMemcpyDeviceToHost));
+    if (adv) HIP_TRY(copy_now(m->stream, adv, m->adv, (size_t)c.step * 4, hipMemcpyDeviceToHost));
     if (final_pos) *final_pos = c.pos;
     return c.step;
 }
