@@ -169,6 +169,57 @@ __global__ __launch_bounds__(LG_WG) void lg_k_rows_mm(LG_ROWSMM_FIELDS(LG_XP, _)
 // 1827 -> 1886 us a decode step of the E4B shape, its own last one again 2208 -> 2220 at five rows), forms the exact block dots and the scale products of its tiles, and the float
 // chain p = fma(xd*dw, (float)dot, p) then runs through the parts in order (part p starts from the value part
 // p-1 left in LDS), so every sum is formed in the order of lg_mm_groups and the result is the same bits.
+// Tiles it_lo .. it_lo + nt - 1 of a row group (wq, ws) against the rows in LDS; acc is whole in the last part's wavefront.  xch: [M][64] floats of the group
+template <int M, int KP, int TMAX>
+__device__ __forceinline__ void lg_mm_ks_sums(const uint4 (&wq)[TMAX], const uint32_t (&ws)[TMAX], int it_lo, int nt, int part, const int8_t *lq, const float2 *lds, int k, int lane, float *xch, float (&acc)[M]) {
+    const int c = lane & 7, nb = k >> 5;
+    float sc[TMAX][M], fd[TMAX][M];
+    #pragma unroll
+    for (int u = 0; u < TMAX; ++u) {
+        if (u >= nt) continue;                                // (a guard, not a break: the arrays stay in registers)
+        const int it = it_lo + u;
+        float2 ds[M]; int4 a0[M], a1[M];
+        #pragma unroll
+        for (int j = 0; j < M; ++j) {
+            ds[j] = lds[j * nb + it * 8 + c];
+            const int8_t *au = lq + (size_t)j * k + (size_t)(it * 16 + c) * 16;
+            a0[j] = *(const int4 *)au; a1[j] = *(const int4 *)(au + 8 * 16);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const float dw = lg_h2f((uint16_t)ws[u]);
+        #pragma unroll
+        for (int j = 0; j < M; ++j) {
+            fd[u][j] = (float)lg_block_dot(wq[u], a0[j], a1[j], __float_as_int(ds[j].y));
+            sc[u][j] = ds[j].x * dw;
+        }
+    }
+    #pragma unroll
+    for (int j = 0; j < M; ++j) acc[j] = 0.0f;
+    float *mine = xch + lane;
+    #pragma unroll
+    for (int p = 0; p < KP; ++p) {
+        if (part == p) {
+            if (p > 0) {
+                #pragma unroll
+                for (int j = 0; j < M; ++j) acc[j] = mine[j * 64];
+            }
+            #pragma unroll
+            for (int u = 0; u < TMAX; ++u) {
+                if (u >= nt) continue;
+                #pragma unroll
+                for (int j = 0; j < M; ++j) acc[j] = lg_fmaf(sc[u][j], fd[u][j], acc[j]);
+            }
+            if (p < KP - 1) {
+                #pragma unroll
+                for (int j = 0; j < M; ++j) mine[j * 64] = acc[j];
+            }
+        }
+        if (p < KP - 1) __syncthreads();
+    }
+    if (part != KP - 1) return;
+    #pragma unroll
+    for (int j = 0; j < M; ++j) acc[j] = lg_sum_seg<8>(acc[j]);
+}
 template <int M, int KP>
 __global__ __launch_bounds__(128 * KP) void lg_k_mm_ks(LG_MM_FIELDS(LG_XP, _) int p_end_) {
     MmArgs a; LG_MM_FIELDS(LG_XI, a)
@@ -193,54 +244,10 @@ __global__ __launch_bounds__(128 * KP) void lg_k_mm_ks(LG_MM_FIELDS(LG_XP, _) in
     __builtin_amdgcn_sched_barrier(0);
     lg_load_q8_commit<M>(rows, a.q_in, k, lq, 128 * KP);
     __syncthreads();
-    const int c = lane & 7;
-    float sc[TMAX][M], fd[TMAX][M];
-    #pragma unroll
-    for (int u = 0; u < TMAX; ++u) {
-        if (u >= nt) continue;                                // (a guard, not a break: the arrays stay in registers)
-        const int it = it_lo + u;
-        float2 ds[M]; int4 a0[M], a1[M];
-        #pragma unroll
-        for (int j = 0; j < M; ++j) {
-            ds[j] = lds[j * nb + it * 8 + c];
-            const int8_t *au = lq + (size_t)j * k + (size_t)(it * 16 + c) * 16;
-            a0[j] = *(const int4 *)au; a1[j] = *(const int4 *)(au + 8 * 16);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        const float dw = lg_h2f((uint16_t)ws[u]);
-        #pragma unroll
-        for (int j = 0; j < M; ++j) {
-            fd[u][j] = (float)lg_block_dot(wq[u], a0[j], a1[j], __float_as_int(ds[j].y));
-            sc[u][j] = ds[j].x * dw;
-        }
-    }
     float acc[M];
-    #pragma unroll
-    for (int j = 0; j < M; ++j) acc[j] = 0.0f;
-    float *mine = xch + (size_t)gsel * M * 64 + lane;
-    #pragma unroll
-    for (int p = 0; p < KP; ++p) {
-        if (part == p) {
-            if (p > 0) {
-                #pragma unroll
-                for (int j = 0; j < M; ++j) acc[j] = mine[j * 64];
-            }
-            #pragma unroll
-            for (int u = 0; u < TMAX; ++u) {
-                if (u >= nt) continue;
-                #pragma unroll
-                for (int j = 0; j < M; ++j) acc[j] = lg_fmaf(sc[u][j], fd[u][j], acc[j]);
-            }
-            if (p < KP - 1) {
-                #pragma unroll
-                for (int j = 0; j < M; ++j) mine[j * 64] = acc[j];
-            }
-        }
-        if (p < KP - 1) __syncthreads();
-    }
+    lg_mm_ks_sums<M, KP, TMAX>(wq, ws, it_lo, nt, part, lq, lds, k, lane, xch + (size_t)gsel * M * 64, acc);
     if (part != KP - 1 || g0 >= ngroups) return;
-    #pragma unroll
-    for (int j = 0; j < M; ++j) acc[j] = lg_sum_seg<8>(acc[j]);
+    const int c = lane & 7;
     if (c < M) a.out[(size_t)c * a.m + gi * 8 + (lane >> 3)] = lg_pick<M>(acc, c);
 }
 

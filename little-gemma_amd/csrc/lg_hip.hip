@@ -169,6 +169,7 @@ struct Layer {
     uint8_t *wqkv = nullptr, *wo = nullptr, *wgu = nullptr, *wdown = nullptr, *winp = nullptr, *wproj = nullptr;
     float *winp_f = nullptr, *wproj_f = nullptr;   // inp_gate / proj when the file keeps them in a float type (then winp / wproj are null)
     uint8_t *wdn_m = nullptr;                      // ffn_down again as the per-workgroup streams of lg_k_down_m
+    uint8_t *wqkv_ch = nullptr;                    // q/k/v again as such chains: lg_k_ple_tail_s of 4..8 rows
     uint8_t *wo_ch = nullptr;                      // attn_output again as matrix-core chains [row block][segment]: lg_k_attn_tail, lg_k_attn_out_m
     // the matrices once more in the form of the prompt kernels (lg_wide.h)
     uint8_t *wqkv_w = nullptr, *wo_w = nullptr, *wgu_w = nullptr, *wdown_w = nullptr, *winp_w = nullptr, *wproj_w = nullptr;
@@ -241,7 +242,7 @@ struct lg_hip_model {
     int last_rows = 0, last_adv = 0;
     float *lstage = nullptr;           // pinned: two rows of logits on their way to a caller (lg_hip_get_logits), row j in half j % 2
     int lread = -1, lcoming = -1;      // the row of the latest step read last, and the one whose copy has been started
-    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1, attn_out = 1;
+    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1, attn_out = 1, tail_qkv = 1;
     // the feed-forward half of a layer as one XCD-partitioned launch (lg_xffn.h): built when the shape and the chip fit
     int xcd_ffn = 0;                         // option: use it (verify blocks of 4..8 rows)
     int down_m = 1;                          // option: ffn_down of 4..8-row blocks on the matrix cores (lg_k_down_m): 1 = the row group's four workgroups add
@@ -259,6 +260,7 @@ struct lg_hip_model {
     int xcd_tail = 1;                        // option: 0 off, 1 for blocks that do not fold the row work into q/k/v, 2 for every verify block
     XtailSync *tsync = nullptr;
     uint2 *tgf = nullptr, *tpr = nullptr;    // [LG_HIP_MAX_ROWS][ple] and [LG_HIP_MAX_ROWS][E] its gated values and projections, tagged
+    FarRows *trows = nullptr;                // rows of lg_k_ple_tail_s on their way to the next layer's projections (option tail_qkv)
     AttnOutSync *aosync = nullptr;           // hand-over state of lg_k_attn_out (models it serves)
     NarrowSync *nsync = nullptr;             // hand-over state of lg_k_narrow (models it serves: narrow_shape)
     RgSync *rgsync = nullptr;                // flags of lg_k_rows_geglu
@@ -742,6 +744,13 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         }
         if ((rc = upload_tiled(m, rows, E, &y.wqkv, stage))) return rc;
         if ((rc = wide_form(m, y.wqkv, E, y.qkv_m, false, &y.wqkv_w))) return rc;
+        const HostTensor *ig = m->ple == 256 ? find(m, lname(L, "inp_gate.weight")) : nullptr;
+        if (ig && ig->type == 2 && !m->target && m->numbered && L > 0 && max_rows >= LG_TAIL_MFMA && E % 512 == 0 && E <= 4096 && y.qkv_m % 32 == 0 && cu_count() == LG_XCDS * LG_XCD_WGS) {
+            stage.resize((size_t)y.qkv_m * (E / 32) * 18);       // (once more: the chains that lg_k_ple_tail_s takes)
+            pack_o_chains(rows.data(), E, y.qkv_m, stage.data());
+            if (dev_alloc(m, &y.wqkv_ch, stage.size())) return -7;
+            HIP_TRY(copy_now(m->stream, y.wqkv_ch, stage.data(), stage.size(), hipMemcpyHostToDevice));
+        }
         rows.clear();
         const HostTensor *o = find(m, lname(L, "attn_output.weight"));
         if ((rc = check_mat(o, lname(L, "attn_output.weight"), y.qd, E))) return rc;
@@ -861,7 +870,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
     if (m->ple && dev_alloc(m, &m->eq, qb(E) + (size_t)12 * E)) return -7;
     if (!m->target) {                        // hand-over state of the one-XCD kernels (lg_xtail.h)
         if (mark_alloc(m, &m->tsync) || mark_alloc(m, &m->rgsync) || dev_alloc(m, &m->tstamps, (size_t)2 * LG_XTAIL_UNITS * 8) ||
-            (m->ple > 0 && (mark_alloc(m, &m->tgf, (size_t)LG_HIP_MAX_ROWS * m->ple) || mark_alloc(m, &m->tpr, (size_t)LG_HIP_MAX_ROWS * E)))) return -7;
+            (m->ple > 0 && (mark_alloc(m, &m->tgf, (size_t)LG_HIP_MAX_ROWS * m->ple) || mark_alloc(m, &m->tpr, (size_t)LG_HIP_MAX_ROWS * E) || mark_alloc(m, &m->trows)))) return -7;
         HIP_TRY(clear_now(m->stream, m->tstamps, 0, (size_t)2 * LG_XTAIL_UNITS * 8 * 8));
         HIP_TRY(clear_now(m->stream, m->aq, 0, qb(max_qd)));       // (row slots past the block are read as operand rows of the matrix cores)
         if (getenv("LG_HIP_XCD_TAIL")) m->xcd_tail = atoi(getenv("LG_HIP_XCD_TAIL"));
@@ -1255,13 +1264,21 @@ static void launch_xffn(Launcher &lx, const XffnArgs &a, int cls) {
     }
 }
 
+// Whether that launch is lg_k_ple_tail_s: 5 to 8 rows (its units fit one per CU), 1 and 2 (it has enough wavefronts for the projection), and 3 and 4 where
+// the next layer's projections are part of it
+static bool tail_spreads(const lg_hip_model *m, int rows) { return m->tail_spread && (rows >= 5 || rows <= 2 || m->tail_qkv || m->tail_spread == 2); }
+// ... which they are while the workgroups on the other seven XCDs, one to a CU, take 16 or 32 of their rows each
+static bool tail_does_qkv(const lg_hip_model *m, int rows, const Layer &next) {
+    return m->tail_qkv && m->trows && tail_spreads(m, rows) && next.qkv_m <= (LG_XCDS - 1) * rows * (LG_XCD_WGS / rows) * (rows >= LG_TAIL_MFMA ? 32 : 16) &&
+           (rows < LG_TAIL_MFMA || next.wqkv_ch);
+}
 // The per-layer-input block of a verify block of `rows` rows as the one-XCD launch lg_k_ple_tail: q4_0 matrices of the
 // 256-wide per-layer input, at most LG_XTAIL_UNITS (gate block, row) units, a chip whose workgroups are dealt over 8 XCDs
 static bool use_ple_tail(const lg_hip_model *m, int rows) {
     if (!m->ple || !m->tsync || !may_wait(m) || m->xcd_tail <= 0 || m->target) return false;
     if (m->ple != 256 || (m->ple / 32) * rows > LG_XTAIL_UNITS || m->E % 256 || m->E > 4096 || (m->E + 1023) / 1024 > m->ple / 32) return false;
     const int U = (m->ple / 32) * rows;
-    const bool spread = m->tail_spread && (rows >= 5 || rows <= 2);   // (lg_k_ple_tail_s: 8 wavefronts per unit, enough of them at every width)
+    const bool spread = tail_spreads(m, rows);               // (lg_k_ple_tail_s: 8 wavefronts per unit, enough of them at every width)
     // blocks of one and two rows: with lg_k_ple_tail_s the tail beats folding the next layer's row work into its q/k/v
     // matmul (E4B shape: 1.994 -> 1.958 ms at one row, 2.127 -> 2.032 at two); with lg_k_ple_tail alone it does not
     if (m->xcd_tail == 1 && rows <= LG_FUSE_ROWS_MAX && m->fuse_rows && !spread) return false;
@@ -1387,8 +1404,8 @@ static void launch_ple_tail(Launcher &lx, const XtailArgs &a) {
         // 5..8 rows: the form whose units fit one per CU (row j by 32 / M workgroups of 8 wavefronts); 1 and 2 rows: the
         // form that has enough wavefronts for the projection
         const int W = M * (32 / M), G = (E / 8 + 8 * W - 1) / (8 * W);
-        if ((m->tail_spread == 2 || (m->tail_spread && (M >= 5 || M <= 2))) && a.gf && a.r.g.ple == 256 && G >= 1 && G <= 3) {
-            const size_t lds = (size_t)E * 5 / 4 + (size_t)M * a.r.g.ple * 5 / 4;
+        if (tail_spreads(m, M) && a.gf && a.r.g.ple == 256 && G >= 1 && G <= 3) {
+            const size_t lds = lg_tail_s_lds(M, E, a.r.g.ple, a.qw != nullptr);
             const dim3 grid(LG_XCDS * W);
             static int fits[2][4] = {};                       // per tiles of a gate row group (10, 16) and G: 0 unknown, 1 yes, -1 no (asked once, outside any capture)
             auto launch = [&](auto nit_) {
@@ -1413,6 +1430,7 @@ static void launch_ple_tail(Launcher &lx, const XtailArgs &a) {
                 return true;
             };
             if (E <= 2560 ? launch(std::integral_constant<int, 10>{}) : launch(std::integral_constant<int, 16>{})) return;
+            if (a.qw) { lx.rc = fail(-2, "ple_tail: the units of %d rows do not fit one XCD", M); return; }
         }
     }
     const int U = (a.r.g.ple / 32) * M;
@@ -1782,7 +1800,11 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 f.x_out = m->x[cur ^ 1]; f.h_out = last ? m->hidden_rows : nullptr;
                 f.q = m->hq; f.q_units = last && head_m ? 2 : 0;
                 f.seq = L; f.spin_limit = m->wait_polls; f.stamps = m->tail_stamps ? m->tstamps : nullptr;
-                f.gf = m->tgf;
+                f.gf = m->tgf; f.rows = m->trows;
+                if (!last && tail_does_qkv(m, M, m->L[L + 1])) {
+                    f.qw = M >= LG_TAIL_MFMA ? m->L[L + 1].wqkv_ch : m->L[L + 1].wqkv; f.qm = m->L[L + 1].qkv_m; f.qout = m->qkv;
+                    qkv_done = true;
+                }
                 launch_ple_tail<M>(lx, f);
                 cur ^= 1;
                 pend_dout = pend_w = pend_os = nullptr; pend_parts = 1;
@@ -2010,7 +2032,7 @@ static GraphKey graph_key(const lg_hip_model *m, const lg_hip_kv *kv, int rows, 
     put(what, 2); put(rows, 4); put(m->store_logits != 0, 1); put(m->draft_chain, 1); put(m->fuse_rows, 1); put(m->attn_rows, 1); put(m->attn_rows_fq, 1);
     put(m->head_mfma, 1); put(m->down_kq, 1); put(m->xcd_ffn, 1); put(m->fork_ple, 1); put(m->rows_geglu, 1); put(m->tail_stamps != 0, 1);
     put(m->tail_spread == 1 ? 1 : m->tail_spread ? 2 : 0, 2); put(m->xcd_tail, 2); put(m->down_m, 2); put(m->xcd_attn_tail, 2); put(m->merge_o, 2);
-    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->wait_polls, 17); put(may_wait(m), 1);
+    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->tail_qkv, 1); put(m->wait_polls, 17); put(may_wait(m), 1);
     return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices, 0 };
 }
 
@@ -2074,6 +2096,7 @@ extern "C" int lg_hip_set_option(lg_hip_model *m, const char *name, int value) {
     else if (!strcmp(name, "rows_geglu")) m->rows_geglu = value != 0;
     else if (!strcmp(name, "narrow")) m->narrow = value != 0;
     else if (!strcmp(name, "attn_out")) m->attn_out = value != 0;
+    else if (!strcmp(name, "tail_qkv")) m->tail_qkv = value != 0;
     else if (!strcmp(name, "down_kq")) m->down_kq = value != 0;
     else if (!strcmp(name, "xcd_ffn")) m->xcd_ffn = value != 0 && m->xffn_built;
     else if (!strcmp(name, "fork_ple")) m->fork_ple = value != 0;
@@ -2417,7 +2440,7 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
     const bool narrow = use_narrow(m, rows);              // (everything but the attention and the first layer's projections)
     for (int L = 0; L < m->n_layer; ++L) {
         const Layer &y = m->L[L];
-        b[narrow && L ? KC_TAIL : KC_QKV] += (double)m->E * y.qkv_m * q;
+        b[L && (narrow || (!y.winp_f && use_ple_tail(m, rows) && tail_does_qkv(m, rows, y))) ? KC_TAIL : KC_QKV] += (double)m->E * y.qkv_m * q;
         if (narrow) b[KC_TAIL] += ((double)y.qd * m->E + 3.0 * m->E * y.nff + 2.0 * m->E * m->ple) * q;
         else {
         {

@@ -87,6 +87,7 @@ template <int M>
 __device__ __forceinline__ size_t lg_q8_off(int k, int j, int w, int byte) { return (size_t)j * k + (size_t)lg_act_unit(lg_act_layout(k), w) * 16 + byte; }
 template <int M>
 __device__ __forceinline__ size_t lg_q8_ds_idx(int k, int j, int b) { return (size_t)j * (k >> 5) + lg_act_block(lg_act_layout(k), b); }
+#define LG_MAXK_FAR 4096                    // widest row of FarRows
 #define LG_MU_DWORDS 80                     // dwords per block of the lg_k_geglu_m activation order
 #define LG_ROWV ((LG_MAXV + 3) / 4)        // float4 per thread of a residual row, 256 threads per row
 template <int M>

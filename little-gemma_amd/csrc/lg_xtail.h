@@ -22,11 +22,17 @@
 // the tag is there (lg_take).  With a flag behind the acknowledged stores and the data loaded behind the flag it was four
 // trips, 1.25 us a hand-over at the E4B shape of 5 rows against 1.0, and 0.45 at one row; the launch 9.2 -> 8.3 us, 7.7 -> 6.5 at one
 // row (there also for the wavefronts without gate rows, which no longer request any), a step 2193 -> 2156 and 1832 -> 1776 us.
+// The other 7U workgroups of lg_k_ple_tail_s are the next layer's q/k/v projections (TailQkv): their weights are in registers when the rows leave the one
+// XCD (FarRows, 0.9 us from the last unit's store to the last workgroup's LDS), and what was a launch of its own behind this one is 2 us of it: by the stamps five
+// rows are there at 8.3 us, taken at 9.4, multiplied at 10.5.  Steps of the E4B shape, one row 1759 -> 1731 us, four 2009 -> 1938, five 2115 -> 2058,
+// eight at 20011 2502 -> 2409.  On v_dot4 from four rows on (every row group reads the rows from LDS again): 2100 and 2504; the tail on all eight XCDs at once, so
+// that each has its rows in its own L2: its first phase takes 5.5 us for 4.2, 2168 and 2264 (eight at 777, for 2262).
 // The tag carries the writer's XCD id; a unit that sees another id, or gives up a bounded wait, reports it in
 // StepCtl.err and goes on, so the kernel always ends and the host refuses the step.
 #pragma once
 #include <type_traits>
 #include "lg_kernels.h"
+#include "lg_fused.h"
 #include "lg_xcd.h"
 #include "lg_xffn.h"
 
@@ -34,6 +40,62 @@
 struct XtailSync {
     uint32_t flags[2][LG_XTAIL_UNITS];      // lg_k_attn_tail: lg_tag of each unit's last arrival
 };
+
+// q8 rows that a launch hands from its one XCD to the workgroups on the other seven, two dwords of a row or a {scale, sum} pair to a unit, every dword
+// with the launch's tag (row j: k/8 units of dwords, then k/32 of pairs; either in the order in which the consumer keeps them in LDS).  Stored and loaded with
+// an agent's scope: through the writer's L2 to memory, and around the reader's.
+struct FarRows {
+    uint2 soon;                     // {-, tag}: the rows are on their way, from here on the waiting workgroups load them until they are there
+    uint2 pad[15];
+    uint4 u[LG_HIP_MAX_ROWS_DEV * LG_MAXK_FAR * 5 / 32];
+};
+__device__ __forceinline__ void lg_put_far(uint2 *p, uint32_t v, uint32_t tag) {
+    __hip_atomic_store((unsigned long long *)p, (unsigned long long)tag << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// MFMA: as the 80-dword blocks of lg_k_geglu_m, else in the order of lg_act_layout.  A lane's four values (quad of row j) and, by the first lane of a block, its pair
+template <bool MFMA>
+__device__ __forceinline__ void lg_put_far_q8(FarRows *f, int k, int j, int quad, uint32_t packed, float d, int sum, uint32_t tag) {
+    uint2 *row = (uint2 *)(f->u + (size_t)j * (k * 5 >> 5));
+    const ActLayout lay = lg_act_layout(k);
+    const int b = quad >> 3, dw = quad & 7;
+    lg_put_far(row + (MFMA ? b * 8 + ((dw & 1) | ((dw & 2) << 1) | ((dw & 4) >> 1)) : lg_act_unit(lay, quad >> 2) * 4 + (quad & 3)), packed, tag);
+    if (dw == 0) {
+        uint2 *p = row + (k >> 2) + 2 * (MFMA ? b : lg_act_block(lay, b));
+        lg_put_far(p, __float_as_uint(d), tag);
+        lg_put_far(p + 1, MFMA ? __float_as_uint(12582912.0f + (float)(8 * sum)) : (uint32_t)sum, tag);
+    }
+}
+// Wait until the rows are on their way (one load per wavefront and trip: workgroups that load the rows all the time keep the memory from the ones that make them)
+__device__ __forceinline__ int lg_wait_soon(const FarRows *f, uint32_t tag, int spin_limit) {
+    for (int spins = 0;; ++spins) {
+        const uint32_t diff = (uint32_t)(lg_ld_l2_u64(&f->soon) >> 32) ^ tag;
+        if ((diff >> 4) == 0) return 0;
+        if (spins >= spin_limit) return LG_XFFN_ERR_WAIT;
+        __builtin_amdgcn_s_sleep(1);
+    }
+}
+// Units at(i) of the rows, i = 0 .. total - 1, by nt threads, at most N of a thread, to `to(i)` in LDS (two dwords each)
+template <int N, typename A, typename P>
+__device__ __forceinline__ int lg_take_far_q8(const FarRows *f, int total, int t, int nt, uint32_t tag, int spin_limit, A &&at, P &&to) {
+    const __amdgpu_buffer_rsrc_t r = lg_buffer_rsrc(f->u);
+    lg_x4u v[N];
+    int err = 0, o[N];
+    #pragma unroll
+    for (int i = 0; i < N; ++i) o[i] = at(t + nt * i < total ? t + nt * i : total - 1) * 16;
+    for (int spins = 0;; ++spins) {
+        uint32_t diff = 0;
+        #pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = __builtin_bit_cast(lg_x4u, __builtin_amdgcn_raw_buffer_load_b128(r, o[i], 0, 16));      // (16: the scope bit sc1)
+        #pragma unroll
+        for (int i = 0; i < N; ++i) diff |= (v[i].y ^ tag) | (v[i].w ^ tag);
+        if (__all((diff >> 4) == 0)) break;
+        if (spins >= spin_limit) { err = LG_XFFN_ERR_WAIT; break; }
+        asm volatile("" ::: "memory");
+    }
+    #pragma unroll
+    for (int i = 0; i < N; ++i) if (t + nt * i < total) *(uint2 *)to(t + nt * i) = make_uint2(v[i].x, v[i].z);
+    return err;
+}
 
 struct XtailArgs {
     RowsPleGateArgs r;              // phase 1 (x_out is not written: the row stays in registers)
@@ -48,12 +110,18 @@ struct XtailArgs {
     int            spin_limit;
     unsigned long long *stamps;     // nullptr, or [LG_XTAIL_UNITS][8] device wall-clock ticks at the phase boundaries of every unit (measurement runs)
     uint2         *gf;              // [M][ple] the gated values as tagged floats (handed from phase 1 to phase 2 through the XCD's L2)
+    const uint8_t *qw;              // lg_k_ple_tail_s: the next layer's q/k/v projections are part of the launch (segment tiles; from LG_TAIL_MFMA rows on the chains
+                                    // of lg_k_attn_tail), or nullptr
+    int            qm;              // their rows
+    float         *qout;            // [M][qm]
+    FarRows       *rows;            // the rows that they take
 };
 #define LG_XTAIL_FIELDS(X, v) X(const float *, x, r.x, v) X(const float *, dout, r.dout, v) X(const float *, w_post, r.w_post, v) X(const uint8_t *, gw, r.g.w, v) \
     X(int, gk, r.g.k, v) X(int, gple, r.g.ple, v) X(int, dparts, r.dparts, v) X(int, seq, seq, v) X(const float *, gipl, r.g.ipl, v) X(int, glayer, r.g.layer, v) \
     X(int, gnl, r.g.n_layer, v) X(int8_t *, gpq, r.g.pq, v) X(const uint8_t *, pw, pw, v) X(const float *, w_post2, w_post2, v) X(const float *, w_pre, w_pre, v) \
     X(const float *, os, os, v) X(uint2 *, pout, pout, v) X(float *, x_out, x_out, v) X(float *, h_out, h_out, v) X(int8_t *, q, q, v) X(int, q_units, q_units, v) \
-    X(float, eps, r.eps, v) X(int, spin_limit, spin_limit, v) X(unsigned long long *, stamps, stamps, v) X(uint2 *, gf, gf, v)
+    X(float, eps, r.eps, v) X(int, spin_limit, spin_limit, v) X(unsigned long long *, stamps, stamps, v) X(uint2 *, gf, gf, v) \
+    X(const uint8_t *, qw, qw, v) X(int, qm, qm, v) X(float *, qout, qout, v) X(FarRows *, rows, rows, v)
 
 __device__ __forceinline__ void lg_ld4_wait1(lg_x4u &a) { asm volatile("s_waitcnt vmcnt(0)" : "+v"(a) :: "memory"); }
 
@@ -256,11 +324,142 @@ __device__ __forceinline__ float lg_block_sum256_of512(float v, float *scratch8)
 //   hand-over; every unit quantizes the M x ple floats into its LDS (the blocks, scales and sums of lg_k_rows_plegate);
 //   phase 2 and 3 as in lg_k_ple_tail, the projection's row groups dealt over 8 W wavefronts, the row work of row j by
 //   its parts 0 .. E/1024 - 1 (wavefronts 0..3).
+#define LG_TAIL_MFMA 4              // rows from which the projections are on the matrix cores
+// A workgroup's share of the next layer's q/k/v projections, the weights requested, and unpacked, while the rows are being made
+template <int M, int NIT, bool MFMA = (M >= LG_TAIL_MFMA)> struct TailQkv;
+// ... a block of 32 rows, a K segment to a wavefront (lg_k_attn_tail), which takes its part of the rows itself
+template <int M, int NIT>
+struct TailQkv<M, NIT, true> {
+    static constexpr int ROWS = 32, N = (NIT + 1) / 2;
+    lg_v4i b[NIT]; float dw[NIT];
+    __device__ __forceinline__ void request(const XtailArgs &a, int rank, int wave, int lane, int nit) {
+        const uint8_t *cb = a.qw + ((size_t)rank * 8 + wave) * (nit * 576);
+        lg_x4u q[N]; uint32_t s[N];
+        #pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const int at = 2 * u < nit ? u : 0;
+            q[u] = __builtin_nontemporal_load((const lg_x4u *)(cb + (size_t)(at * 64 + lane) * 16));
+            s[u] = __builtin_nontemporal_load((const uint32_t *)(cb + (size_t)nit * 512 + (size_t)(at * 32 + (lane & 31)) * 4));
+        }
+        #pragma unroll
+        for (int i = 0; i < NIT; ++i) {
+            const uint32_t x = i & 1 ? q[i >> 1].z : q[i >> 1].x, y = i & 1 ? q[i >> 1].w : q[i >> 1].y;
+            b[i].x = x & 0x0F0F0F0F; b[i].y = y & 0x0F0F0F0F; b[i].z = (x >> 4) & 0x0F0F0F0F; b[i].w = (y >> 4) & 0x0F0F0F0F;
+            dw[i] = lg_h2f((uint16_t)(i & 1 ? s[i >> 1] >> 16 : s[i >> 1]));
+            asm volatile("" : "+v"(b[i]), "+v"(dw[i]));
+        }
+    }
+    __device__ __forceinline__ int take(const XtailArgs &a, int wave, int lane, int nit, unsigned char *act, uint32_t tag) {
+        const int k = a.r.g.k, per = k * 5 >> 5, words = k >> 3, mine = nit * 5, first = wave * nit;
+        unsigned char *la = act + (size_t)first * (LG_MU_DWORDS * 4);
+        return lg_take_far_q8<(5 * NIT * M + 63) / 64>(a.rows, mine * M, lane, 64, tag, a.spin_limit, [&](int i) {
+            const int j = i / mine, w = i - j * mine;
+            return j * per + (w < 4 * nit ? 4 * first + w : words + first + w - 4 * nit);
+        }, [&](int i) {
+            const int j = i / mine, w = i - j * mine;
+            return w < 4 * nit ? la + (size_t)(w >> 2) * (LG_MU_DWORDS * 4) + j * 32 + (w & 3) * 8 : la + (size_t)(w - 4 * nit) * (LG_MU_DWORDS * 4) + 256 + j * 8;
+        });
+    }
+    // xch: 8 KB of LDS
+    __device__ __forceinline__ void finish(const XtailArgs &a, int rank, int wave, int t, int nit, const unsigned char *act, float *xch, int real) {
+        const int lane = t & 63, n = lane & 31, h = lane >> 5, arow = n < 8 ? n : 7;
+        lg_v16i magic;
+        #pragma unroll
+        for (int i = 0; i < 16; ++i) magic[i] = 0x4B400000;
+        asm volatile("" : "+v"(magic));
+        float p[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+        const unsigned char *ls = act + (size_t)wave * nit * (LG_MU_DWORDS * 4);
+        // (no branch on a shorter segment's end: its last block again, the result not taken)
+        auto block = [&](int i) { return lg_xffn_act(ls + (i < nit ? i : nit - 1) * (LG_MU_DWORDS * 4), arow, h); };
+        XffnAct ac[3] = { block(0), block(1), block(2) };
+        lg_v16i d[2];
+        d[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ac[0].av, b[0], magic, 0, 0, 0);
+        #pragma unroll
+        for (int i = 0; i < NIT; ++i) {                        // (the next block's dots on their way while this one's join the sums)
+            if (i + 1 < NIT) d[(i + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ac[(i + 1) % 3].av, b[i + 1 < NIT ? i + 1 : i], magic, 0, 0, 0);
+            const XffnAct &c = ac[i % 3];
+            #pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float v = lg_fmaf(c.xd[r] * dw[i], __int_as_float(d[i & 1][r]) - c.cf[r], p[r]);
+                p[r] = i < nit ? v : p[r];
+            }
+            asm volatile("" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]));
+            if (i + 3 < NIT) ac[i % 3] = block(i + 3);
+        }
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) xch[(wave * 8 + 4 * h + i) * 32 + n] = p[i];
+        __syncthreads();
+        if (t < 32 * M && real) {                              // the adjacent-pair tree over the 8 segments
+            const float *z = xch + t;
+            a.qout[(size_t)(t >> 5) * a.qm + rank * 32 + (t & 31)] = ((z[0] + z[256]) + (z[512] + z[768])) + ((z[1024] + z[1280]) + (z[1536] + z[1792]));
+        }
+    }
+};
+// ... two row groups of 8, the tiles of each over four wavefronts (lg_k_mm_ks<M, 4>)
+template <int M, int NIT>
+struct TailQkv<M, NIT, false> {
+    static constexpr int ROWS = 16, KP = 4, N = (NIT + KP - 1) / KP;
+    uint4 q[N]; uint32_t s[N];
+    __device__ __forceinline__ void request(const XtailArgs &a, int rank, int wave, int lane, int nit) {
+        const int g0 = rank * 2 + wave / KP, gi = g0 < a.qm >> 3 ? g0 : (a.qm >> 3) - 1, lo = wave % KP * nit / KP;
+        const uint8_t *wg = a.qw + (size_t)gi * nit * LG_TILE;
+        #pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const int it = lo + u < nit ? lo + u : nit - 1;
+            q[u] = lg_ldt16(wg, it, lane);
+            s[u] = lg_ldt2(wg, it, lane);
+        }
+    }
+    __device__ __forceinline__ int take(const XtailArgs &a, int wave, int lane, int nit, unsigned char *act, uint32_t tag) {
+        const int k = a.r.g.k, per = k * 5 >> 5, words = k >> 3;
+        const int err = lg_take_far_q8<(40 * NIT * M + 511) / 512>(a.rows, per * M, wave * 64 + lane, 512, tag, a.spin_limit, [&](int i) { return i; }, [&](int i) {
+            const int j = i / per, w = i - j * per;
+            return w < words ? act + (size_t)j * k + 8 * w : act + (size_t)M * k + ((size_t)j * (k >> 5) + (w - words)) * 8;
+        });
+        __syncthreads();
+        return err;
+    }
+    __device__ __forceinline__ void finish(const XtailArgs &a, int rank, int wave, int t, int nit, const unsigned char *act, float *xch, int real) {
+        const int lane = t & 63, k = a.r.g.k, gsel = wave / KP, part = wave % KP, lo = part * nit / KP, nt = (part + 1) * nit / KP - lo, g0 = rank * 2 + gsel;
+        float acc[M];
+        lg_mm_ks_sums<M, KP, N>(q, s, lo, nt, part, (const int8_t *)act, (const float2 *)(act + (size_t)M * k), k, lane, xch + (size_t)gsel * M * 64, acc);
+        if (part != KP - 1 || g0 >= a.qm >> 3) return;
+        const int c = lane & 7;
+        if (c < M && real) a.qout[(size_t)c * a.qm + g0 * 8 + (lane >> 3)] = lg_pick<M>(acc, c);
+    }
+};
+// bytes of LDS of lg_k_ple_tail_s; with the projections: the rows, 8 slots wide on the matrix cores, and 8 KB for sums
+static inline size_t lg_tail_s_lds(int M, int E, int ple, bool qkv) {
+    return (size_t)E * 5 / 4 + (size_t)M * ple * 5 / 4 + (qkv ? (size_t)(M >= LG_TAIL_MFMA ? 8 : M) * E * 5 / 4 + 8192 : 0);
+}
+template <int M, int NIT>
+__device__ __forceinline__ void lg_tail_qkv(const XtailArgs &a, int rank, unsigned char *act, uint32_t tag, StepCtl *ctl) {
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), E = a.r.g.k, nit = E >> 8;
+    float *xch = (float *)(act + (size_t)(M >= LG_TAIL_MFMA ? 8 : M) * E * 5 / 4);
+    TailQkv<M, NIT> qkv;
+    qkv.request(a, rank, wave, t & 63, nit);
+    __builtin_amdgcn_sched_barrier(0);
+    // The first time over whatever LDS holds, for nothing but the instructions: they are in the CU's cache when the rows are there (five rows 2068 -> 2061 us a step)
+    #pragma unroll 1
+    for (int real = 0; real < 2; ++real) {
+        if (real) {
+            int err = lg_wait_soon(a.rows, tag, a.spin_limit);
+            err |= qkv.take(a, wave, t & 63, nit, act, tag);
+            if (err) atomicOr(&ctl->err, err);
+        }
+        qkv.finish(a, rank, wave, t, nit, act, xch, real);
+        __syncthreads();
+    }
+}
 template <int M, int G, int NIT>
 __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FIELDS(LG_XP, _) int p_end_) {
-    if (blockIdx.x & (LG_XCDS - 1)) return;
     XtailArgs a; LG_XTAIL_FIELDS(LG_XI, a)
     extern __shared__ __align__(16) unsigned char smem[];
+    if (blockIdx.x & (LG_XCDS - 1)) {
+        const int rank = (blockIdx.x >> 3) * (LG_XCDS - 1) + (blockIdx.x & (LG_XCDS - 1)) - 1;
+        if (a.qw && rank * TailQkv<M, NIT>::ROWS < a.qm) lg_tail_qkv<M, NIT>(a, rank, smem, lg_tag(ctl->launch + (uint32_t)a.seq, 0), ctl);
+        return;
+    }
     __shared__ float red[3][8];
     constexpr int P = 32 / M;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -401,14 +600,14 @@ __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FI
     const int slices = (E + 1023) >> 10;
     stamp(4);
     if (err) atomicOr(&ctl->err, err);
-    if (p >= slices) return;                                   // this unit has no share of the row work
+    if (p >= slices) return;                    // this unit has no share of the row work
     // ---- hand-over: the projection's row j; phase 3: the row work, this unit storing and quantizing slice p (wavefronts 0..3;
     //      the others only take part in the workgroup's barriers) ----
     err = 0;
     if (rowt) lg_take_row(dv, a.pout + (size_t)j * E, t, nq, tag, a.spin_limit, err);
     if (err) atomicOr(&ctl->err, err);
+    if (a.qw && u == 0 && t == 0) lg_put_far(&a.rows->soon, 0, tag);
     stamp(5);
-    stamp(6);
     {
         float ss = 0.0f;
         if (rowt) {
@@ -463,7 +662,8 @@ __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FI
             float d; int sum;
             const uint32_t packed = lg_quant4_8lanes(xv[v], &d, &sum);
             const int quad = t + 256 * v;
-            if (a.q_units == 2) {
+            if (a.qw) lg_put_far_q8<(M >= LG_TAIL_MFMA)>(a.rows, E, j, quad, packed, d, sum, tag);
+            else if (a.q_units == 2) {
                 uint32_t *blk = (uint32_t *)a.q + (size_t)(quad >> 3) * LG_MU_DWORDS;
                 const int dw = quad & 7;
                 blk[j * 8 + ((dw & 1) | ((dw & 2) << 1) | ((dw & 4) >> 1))] = packed;
