@@ -14,6 +14,12 @@
 // one row leaves at 1.9 us and is in every LDS at 3.4, when the 92 KB of weights are through as well; rows at 5.4, end at 6.4; five rows
 // 3.0, 4.8, 7.9 (the projection 2.3) and 8.9.  E4B shape, the 35 sliding layers of 42, a step: one row 1784 -> 1694 us, two 1883 -> 1812,
 // three 1978 -> 1923 (on v_dot4 1935), four 2061 -> 2007, five 2162 -> 2125, six 2210 -> 2162, eight 2304 -> 2276.
+// The other 224 workgroups of the launch are gate/up and the GeGLU of the rows (lg_aout_geglu), which was a launch of its own behind this one.  By the stamps (two blocks
+// of columns to a workgroup) one row is done at 7.4 us (1.1 of it beside 29 MB of weights on their way), in every LDS at 8.2, multiplied at 9.9 and stored at 10.5; five
+// rows 9.8, 10.9, 13.3 and 13.8, where the two launches took 6.3 + 6.4 and 8.9 + 8.6.  Steps of the E4B shape (with the q/k/v projections in
+// lg_k_ple_tail_s as well): one row 1765 -> 1618 us, five 2113 -> 1946, eight at 20011 2497 -> 2327, four with bf16 per-layer matrices 2546 -> 2385.
+// With 32x32x32 products one row 1664, five 1983; with the rows' scales read from LDS for each product, 16 bytes of tags to 16 of values and
+// divisions in the way of a unit to its place 1658, 1966; a first pass over nothing to have the instructions in the CU's cache made the second wait for it.
 // v_dot4 at 4, 5, 8 rows: 2080, 2196, 2575 (every row group reads the rows from LDS again).  4096 inputs, 276 KB a CU at rows of 3840: a
 // step of the 12B shape 2481 -> 2728.  Weights requested ahead of the partials: one row 1741.  Partials first, but the hand-over
 // taken by the wavefronts that hold weights: 1712.  Five to eight rows with a wavefront per merge: the projection spills, 2202 at five.
@@ -28,6 +34,7 @@
 #define LG_AOUT_DOT_ROWS 3          // widest block on v_dot4
 #define LG_AOUT_NV ((LG_AOUT_E + 1023) / 1024)     // float4 of a row per thread of 256
 struct AttnOutSync { uint2 w[LG_HIP_MAX_ROWS_DEV * LG_AOUT_K / 4]; uint4 s[LG_HIP_MAX_ROWS_DEV * LG_AOUT_K / 32]; uint2 o[LG_HIP_MAX_ROWS_DEV * LG_AOUT_E]; };
+#define LG_AOUT_M_LDS ((size_t)(LG_AOUT_K / 32) * LG_MU_DWORDS * 4 + 8 * ((LG_AOUT_E / 32 + LG_XCD_WGS - 1) / LG_XCD_WGS) * 8 * 32 * 4)
 static_assert(LG_AOUT_K == 64 * LG_XCD_WGS, "a merge of every row per unit");
 struct AttnOutArgs {
     MergeArgs      g;               // (xq, xf are not used)
@@ -41,12 +48,135 @@ struct AttnOutArgs {
     int            seq;             // number of this launch inside the step (the layer)
     int            spin_limit;
     unsigned long long *stamps;
+    const uint8_t *gw;              // gate/up of the rows is part of the launch (row-block tiles), or nullptr
+    int            nff, gq_units;   // GegluArgs.n_ff, .gq_units
+    int8_t        *gq;
+    FarRows       *rows;            // the rows that it takes
 };
 #define LG_AOUT_FIELDS(X, v) X(const float *, pm, g.pm, v) X(const float *, pl, g.pl, v) X(const float *, pacc, g.pacc, v) X(int, tiles_max, g.tiles_max, v) \
     X(int, H, g.H, v) X(int, hd, g.hd, v) X(int, window, g.window, v) X(int, tiles, tiles, v) X(const uint8_t *, wo, wo, v) X(AttnOutSync *, sync, sync, v) X(int, seq, seq, v) X(int, E, E, v) \
     X(const float *, x, x, v) X(const float *, w_post, w_post, v) X(const float *, w_pre, w_pre, v) \
     X(float *, x_out, x_out, v) X(int8_t *, q, q, v) X(float, eps, eps, v) X(int, spin_limit, spin_limit, v) \
-    X(unsigned long long *, stamps, stamps, v)
+    X(unsigned long long *, stamps, stamps, v) X(const uint8_t *, gw, gw, v) X(int, nff, nff, v) X(int, gq_units, gq_units, v) X(int8_t *, gq, gq, v) X(FarRows *, rows, rows, v)
+
+// Gate/up and GeGLU of the rows by the workgroups on the other seven XCDs, for every width: a workgroup's one or two blocks of 32 FFN columns are in its
+// registers and LDS when the rows are there.  Wavefront (pair of K segments, gate or up): v_mfma_i32_16x16x64_i8 with a block of 32 K values of either segment in
+// its K range, rows 0..7 of its operand with the first segment's values and zeros, rows 8..15 with zeros and the second's, so that a product has
+// the dots of 16 weight rows with a block of either segment apart: half the matrix time of a 32x32x32 product, which has the dots of 32 weight rows with one block.
+#define LG_AOUT_NIT (LG_AOUT_E / 256)
+#define LG_AOUT_GU_WGS ((LG_XCDS - 1) * LG_XCD_WGS)
+#define LG_AOUT_GU_LDS ((size_t)8 * LG_AOUT_NIT * (LG_FAR_BLK + LG_TILE) + LG_AOUT_NIT * LG_FAR_BLK + 2 * 8 * 8 * 64 * 4)
+template <int N, typename F, int... X> __device__ __forceinline__ void lg_unroll_(F &&f, std::integer_sequence<int, X...>) { (f(std::integral_constant<int, X>{}), ...); }
+template <int N, typename F> __device__ __forceinline__ void lg_unroll(F &&f) { lg_unroll_<N>(f, std::make_integer_sequence<int, N>{}); }
+template <int M>
+__device__ __forceinline__ void lg_aout_geglu(const AttnOutArgs &a, int rank, unsigned char *smem, uint32_t tag, StepCtl *ctl) {
+    constexpr int NIT = LG_AOUT_NIT, BLK = LG_FAR_BLK, I = (M + 1) / 2;
+    const int t = threadIdx.x, lane = t & 63, c16 = lane & 15, hf = (lane >> 4) & 1, sg = lane >> 5, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int E = a.E, nb = E >> 5, nit = nb >> 3, nblk = a.nff >> 5, b1 = rank + LG_AOUT_GU_WGS;
+    if (rank >= nblk || wave >= 8) return;
+    const bool two = b1 < nblk;
+    const int seg = (wave >> 1) * 2 + sg, up = wave & 1;
+    unsigned char *zero = smem + (size_t)8 * NIT * BLK, *tiles = zero + NIT * BLK + (size_t)wave * NIT * LG_TILE;      // (tiles: of the second block, this wavefront's)
+    float (*red)[8][8][64] = (float (*)[8][8][64])(zero + (size_t)NIT * BLK + (size_t)8 * NIT * LG_TILE);             // [block][segment][row][gate 32, up 32]
+    uint4 q[NIT]; uint32_t sc[NIT];
+    // lane: a gate (or up) row of its segment's tile.  The 16-lane rows trade bytes: lane (row of 16, hf) then has nibble bytes 8 hf .. 8 hf + 7 of rows c16 and 16 + c16
+    auto fetch = [&](int b) {
+        const __amdgpu_buffer_rsrc_t rw = lg_buffer_rsrc(a.gw + (size_t)b * nb * LG_TILE);
+        const int at = seg * nit * LG_TILE, row = up * 32 + (lane & 31);
+        #pragma unroll
+        for (int i = 0; i < NIT; ++i) {
+            const int it = __builtin_amdgcn_readfirstlane(i < nit ? i : nit - 1) * LG_TILE;
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(rw, at + row * 16, it, 2);
+            q[i] = make_uint4(v[0], v[1], v[2], v[3]);
+            sc[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rw, at + 1024 + row * 2, it, 2);
+        }
+        #pragma unroll
+        for (int i = 0; i < NIT; ++i) {
+            const lg_v2u s0 = __builtin_amdgcn_permlane16_swap(q[i].x, q[i].z, false, false), s1 = __builtin_amdgcn_permlane16_swap(q[i].y, q[i].w, false, false);
+            const lg_v2u sd = __builtin_amdgcn_permlane16_swap(sc[i], sc[i], false, false);
+            q[i] = make_uint4(s0.x ^ 0x88888888u, s1.x ^ 0x88888888u, s0.y ^ 0x88888888u, s1.y ^ 0x88888888u);
+            sc[i] = (sd.x & 0xFFFF) | sd.y << 16;
+        }
+    };
+    if (two) {
+        fetch(b1);
+        #pragma unroll
+        for (int i = 0; i < NIT; ++i) { *(uint4 *)(tiles + i * LG_TILE + lane * 16) = q[i]; if (!hf) *(uint32_t *)(tiles + i * LG_TILE + 1024 + (sg * 16 + c16) * 4) = sc[i]; }
+    }
+    for (int i = t; i < NIT * BLK / 16; i += 512) ((uint4 *)zero)[i] = make_uint4(0, 0, 0, 0);
+    fetch(rank);
+    lg_v4i w0[NIT], w1[NIT];
+    #pragma unroll
+    for (int i = 0; i < NIT; ++i) {
+        w0[i] = lg_far_weights(q[i].x, q[i].y); w1[i] = lg_far_weights(q[i].z, q[i].w);
+        asm volatile("" : "+v"(w0[i]), "+v"(w1[i]), "+v"(sc[i]));
+    }
+    int err = lg_wait_soon(a.rows, tag, a.spin_limit);
+    err |= lg_take_far_segment<M, NIT>(a.rows, E, nit, wave, lane, smem + (size_t)wave * NIT * BLK, tag, a.spin_limit);
+    if (err) atomicOr(&ctl->err, err);
+    __syncthreads();
+    const unsigned char *ls = smem + (size_t)seg * NIT * BLK, *la = ((lane >> 3) & 1) == sg ? ls + (lane & 7) * 32 + hf * 16 : zero;
+    lg_v4i magic = { LG_FAR_MAGIC, LG_FAR_MAGIC, LG_FAR_MAGIC, LG_FAR_MAGIC };
+    asm volatile("" : "+v"(magic));
+    // lane i of a row of 16: the scales of block i of the row's segment and half; a product's are broadcast from there
+    float xd[I];
+    static_assert(NIT <= 16, "a block to a lane");
+    #pragma unroll
+    for (int r = 0; r < I; ++r) xd[r] = *(const float *)(ls + (c16 < NIT ? c16 : 0) * BLK + 256 + (4 * hf + r) * 4);
+    float p[2][2][I];                                          // [block][16 columns][row 2i + hf]
+    #pragma unroll
+    for (int i = 0; i < 4 * I; ++i) p[i / (2 * I)][i / I % 2][i % I] = 0.0f;
+    auto chains = [&](auto both, auto whole) {                 // one block, or two that share the reads of the rows
+        constexpr bool TWO = decltype(both)::value;
+        lg_unroll<NIT>([&](auto i_) {
+            constexpr int i = decltype(i_)::value;
+            const lg_v4i av = *(const lg_v4i *)(la + i * BLK);
+            auto join = [&](const lg_v4i &d, float dw, float (&z)[I]) {
+                #pragma unroll
+                for (int r = 0; r < I; ++r) {
+                    const float v = lg_fmaf(lg_row_bcast<i>(xd[r]) * dw, __int_as_float(d[r]) - LG_FAR_BIAS, z[r]);
+                    z[r] = decltype(whole)::value || i < nit ? v : z[r];      // (no branch on a shorter segment's end)
+                }
+            };
+            const lg_v4i d0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, w0[i], magic, 0, 0, 0), d1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, w1[i], magic, 0, 0, 0);
+            if (TWO) {
+                const uint4 w = *(const uint4 *)(tiles + i * LG_TILE + lane * 16);
+                const uint32_t dw = *(const uint32_t *)(tiles + i * LG_TILE + 1024 + (sg * 16 + c16) * 4);
+                const lg_v4i d2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, lg_far_weights(w.x, w.y), magic, 0, 0, 0), d3 = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, lg_far_weights(w.z, w.w), magic, 0, 0, 0);
+                join(d2, lg_h2f((uint16_t)dw), p[1][0]); join(d3, lg_h2f((uint16_t)(dw >> 16)), p[1][1]);
+            }
+            join(d0, lg_h2f((uint16_t)sc[i]), p[0][0]); join(d1, lg_h2f((uint16_t)(sc[i] >> 16)), p[0][1]);
+        });
+        #pragma unroll
+        for (int o = 0; o < (TWO ? 2 : 1); ++o)
+            #pragma unroll
+            for (int i = 0; i < I; ++i) { red[o][seg][2 * i + hf][up * 32 + c16] = p[o][0][i]; red[o][seg][2 * i + hf][up * 32 + 16 + c16] = p[o][1][i]; }
+    };
+    if (nit == NIT) { if (two) chains(std::true_type{}, std::true_type{}); else chains(std::false_type{}, std::true_type{}); }
+    else            { if (two) chains(std::true_type{}, std::false_type{}); else chains(std::false_type{}, std::false_type{}); }
+    __syncthreads();
+    {
+        for (int x = t >> 5; x < (two ? 2 * M : M); x += 16) {            // half-wavefront per row, one FFN column per lane
+            const int o = x >= M, j = x - (o ? M : 0), i = t & 31, b = o ? b1 : rank;
+            float g[8], u[8];
+            #pragma unroll
+            for (int c = 0; c < 8; ++c) { g[c] = red[o][c][j][i]; u[c] = red[o][c][j][32 + i]; }
+            const float gate = ((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7])), up = ((u[0] + u[1]) + (u[2] + u[3])) + ((u[4] + u[5]) + (u[6] + u[7]));
+            float d; int sum;
+            const int v = lg_quant1_32lanes(lg_gelu_d(gate) * up, &d, &sum);
+            if (a.gq_units == 2) {
+                int8_t *blk = a.gq + (size_t)b * (LG_MU_DWORDS * 4);
+                const int dw = i >> 2;
+                blk[(j * 8 + ((dw & 1) | ((dw & 2) << 1) | ((dw & 4) >> 1))) * 4 + (i & 3)] = (int8_t)v;
+                if (i == 0) *(float2 *)(blk + 256 + 8 * j) = make_float2(d, 12582912.0f + (float)(8 * sum));
+            } else {
+                const ActLayout lay = lg_act_layout(a.nff);
+                a.gq[(size_t)j * a.nff + lg_act_unit(lay, b * 2 + (i >> 4)) * 16 + (i & 15)] = (int8_t)v;
+                if (i == 0) lg_q8_ds<M>(a.gq, a.nff)[(size_t)j * (a.nff >> 5) + lg_act_block(lay, b)] = make_float2(d, __int_as_float(sum));
+            }
+        }
+    }
+}
 
 // One wavefront's merge of 64 dims (number u of the row's) of row j, lane = dim: at most T tiles
 template <int T>
@@ -126,7 +256,7 @@ struct AoutRow {
         }
     }
     template <bool MFMA>
-    __device__ __forceinline__ void work(const AttnOutArgs &a, const float4 (&dv)[LG_ROWV], int j, int vr, bool rowt, int t, float *red0, float *red1) {
+    __device__ __forceinline__ void work(const AttnOutArgs &a, const float4 (&dv)[LG_ROWV], int j, int vr, bool rowt, int t, float *red0, float *red1, uint32_t tag) {
         const int E = a.E, nq = E >> 2;
         float ss = 0.0f;
         if (rowt) {
@@ -158,7 +288,8 @@ struct AoutRow {
             float d; int sum;
             const uint32_t packed = lg_quant4_8lanes(h, &d, &sum);
             const int quad = t + 256 * v, dw = quad & 7;
-            if (MFMA) {                                        // (order of lg_k_geglu_m)
+            if (a.gw) lg_put_far_q8(a.rows, E, j, quad, packed, d, lg_far_tag(tag));
+            else if (MFMA) {                                   // (order of lg_k_geglu_m)
                 uint32_t *blk = (uint32_t *)a.q + (size_t)(quad >> 3) * LG_MU_DWORDS;
                 blk[j * 8 + ((dw & 1) | ((dw & 2) << 1) | ((dw & 4) >> 1))] = packed;
                 if ((t & 7) == 0) *(float2 *)(blk + 64 + 2 * j) = make_float2(d, 12582912.0f + (float)(8 * sum));
@@ -175,9 +306,14 @@ struct AoutRow {
 template <int M>
 __global__ __launch_bounds__(64 * (LG_AOUT_G + M)) void lg_k_attn_out(StepCtl *ctl, LG_AOUT_FIELDS(LG_XP, _) int p_end_) {
     constexpr int qd = LG_AOUT_K, NIT = qd >> 8, W = LG_AOUT_G + M;
-    if (blockIdx.x & (LG_XCDS - 1)) return;
     AttnOutArgs a; LG_AOUT_FIELDS(LG_XI, a)
-    __shared__ __align__(16) int8_t lq[M * qd * 5 / 4];        // [M][qd] int8, then [M][qd / 32] {scale, sum}: order of lg_act_layout
+    extern __shared__ __align__(16) unsigned char smem[];
+    if (blockIdx.x & (LG_XCDS - 1)) {
+        if constexpr (M < LG_AOUT_DOT_ROWS)
+            if (a.gw) lg_aout_geglu<M>(a, (blockIdx.x >> 3) * (LG_XCDS - 1) + (blockIdx.x & (LG_XCDS - 1)) - 1, smem, lg_tag(ctl->launch + (uint32_t)a.seq, 0), ctl);
+        return;
+    }
+    int8_t *lq = (int8_t *)smem;                               // [M][qd] int8, then [M][qd / 32] {scale, sum}: order of lg_act_layout
     __shared__ float red[2][W];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), c = lane & 7;
     const int u = blockIdx.x >> 3, E = a.E, nq = E >> 2, slices = (E + 1023) >> 10;
@@ -260,8 +396,9 @@ __global__ __launch_bounds__(64 * (LG_AOUT_G + M)) void lg_k_attn_out(StepCtl *c
     err = 0;
     if (rowt) lg_take_row(dv, y.o + (size_t)jr * E, t, nq, tag, a.spin_limit, err);
     if (err) atomicOr(&ctl->err, err);
+    if (a.gw && u == 0 && t == 0) lg_put_soon(a.rows, lg_far_tag(tag));
     stamp(4);
-    row.work<false>(a, dv, jr, vr, rowt, t, red[0], red[1]);
+    row.work<false>(a, dv, jr, vr, rowt, t, red[0], red[1], tag);
     stamp(5);
 }
 
@@ -270,10 +407,15 @@ __global__ __launch_bounds__(64 * (LG_AOUT_G + M)) void lg_k_attn_out(StepCtl *c
 template <int M>
 __global__ __launch_bounds__(768) void lg_k_attn_out_m(StepCtl *ctl, LG_AOUT_FIELDS(LG_XP, _) int p_end_) {
     constexpr int nb = LG_AOUT_K >> 5, NIT = nb / 8, NP = NIT / 2, RB = (LG_AOUT_E / 32 + LG_XCD_WGS - 1) / LG_XCD_WGS, W = 12;
-    if (blockIdx.x & (LG_XCDS - 1)) return;
     AttnOutArgs a; LG_AOUT_FIELDS(LG_XI, a)
-    __shared__ __align__(16) unsigned char la[nb * LG_MU_DWORDS * 4];      // the rows as blocks of lg_k_geglu_m; slots past the block's rows hold anything
-    __shared__ float sums[8][RB][8][32], red[2][W];            // [segment][row block][row slot][row]
+    extern __shared__ __align__(16) unsigned char smem[];
+    if (blockIdx.x & (LG_XCDS - 1)) {
+        if (a.gw) lg_aout_geglu<M>(a, (blockIdx.x >> 3) * (LG_XCDS - 1) + (blockIdx.x & (LG_XCDS - 1)) - 1, smem, lg_tag(ctl->launch + (uint32_t)a.seq, 0), ctl);
+        return;
+    }
+    unsigned char *la = smem;                                  // the rows as blocks of lg_k_geglu_m; slots past the block's rows hold anything
+    float (*sums)[RB][8][32] = (float (*)[RB][8][32])(smem + nb * LG_MU_DWORDS * 4);        // [segment][row block][row slot][row]
+    __shared__ float red[2][W];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), n = lane & 31, h = lane >> 5;
     const int u = blockIdx.x >> 3, E = a.E, nq = E >> 2, nrb = E >> 5, slices = (E + 1023) >> 10;
     auto stamp = [&](int i) { if (a.stamps && t == 0) a.stamps[(size_t)u * 8 + i] = wall_clock64(); };
@@ -381,7 +523,8 @@ __global__ __launch_bounds__(768) void lg_k_attn_out_m(StepCtl *ctl, LG_AOUT_FIE
     err = 0;
     if (rowt) lg_take_row(dv, y.o + (size_t)jr * E, t, nq, tag, a.spin_limit, err);
     if (err) atomicOr(&ctl->err, err);
+    if (a.gw && u == 0 && t == 0) lg_put_soon(a.rows, lg_far_tag(tag));
     stamp(4);
-    row.work<(M > 3)>(a, dv, jr, vr, rowt, t, red[0], red[1]);
+    row.work<(M > 3)>(a, dv, jr, vr, rowt, t, red[0], red[1], tag);
     stamp(5);
 }

@@ -242,7 +242,7 @@ struct lg_hip_model {
     int last_rows = 0, last_adv = 0;
     float *lstage = nullptr;           // pinned: two rows of logits on their way to a caller (lg_hip_get_logits), row j in half j % 2
     int lread = -1, lcoming = -1;      // the row of the latest step read last, and the one whose copy has been started
-    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1, attn_out = 1, tail_qkv = 1;
+    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1, attn_out = 1, tail_qkv = 1, attn_geglu = 1;
     // the feed-forward half of a layer as one XCD-partitioned launch (lg_xffn.h): built when the shape and the chip fit
     int xcd_ffn = 0;                         // option: use it (verify blocks of 4..8 rows)
     int down_m = 1;                          // option: ffn_down of 4..8-row blocks on the matrix cores (lg_k_down_m): 1 = the row group's four workgroups add
@@ -261,6 +261,7 @@ struct lg_hip_model {
     XtailSync *tsync = nullptr;
     uint2 *tgf = nullptr, *tpr = nullptr;    // [LG_HIP_MAX_ROWS][ple] and [LG_HIP_MAX_ROWS][E] its gated values and projections, tagged
     FarRows *trows = nullptr;                // rows of lg_k_ple_tail_s on their way to the next layer's projections (option tail_qkv)
+    FarRows *aorows = nullptr;               // rows of lg_k_attn_out on their way to gate/up (option attn_geglu)
     AttnOutSync *aosync = nullptr;           // hand-over state of lg_k_attn_out (models it serves)
     NarrowSync *nsync = nullptr;             // hand-over state of lg_k_narrow (models it serves: narrow_shape)
     RgSync *rgsync = nullptr;                // flags of lg_k_rows_geglu
@@ -880,7 +881,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
     } else if (!m->target && cu_count() == LG_XCDS * LG_XCD_WGS) {
         bool any = false;
         for (const Layer &y : m->L) any = any || attn_out_shape(m, y);
-        if (any && mark_alloc(m, &m->aosync)) return -7;
+        if (any && (mark_alloc(m, &m->aosync) || mark_alloc(m, &m->aorows))) return -7;
     }
     if (getenv("LG_HIP_XCD_ATTN_TAIL")) m->xcd_attn_tail = atoi(getenv("LG_HIP_XCD_ATTN_TAIL"));
     if (getenv("LG_HIP_DOWN_M")) m->down_m = atoi(getenv("LG_HIP_DOWN_M"));
@@ -1340,6 +1341,12 @@ static bool use_attn_out(const lg_hip_model *m, const Layer &y, int rows, int ti
     if (rows >= 4 && ((m->rows_geglu && m->E == 2560) || (m->xcd_ffn && y.xgu))) return false;
     return m->attn_out && m->aosync && may_wait(m) && attn_out_shape(m, y) && (rows <= LG_AOUT_DOT_ROWS ? tiles <= LG_AOUT_TILES : y.wo_ch && tiles <= LG_AOUT_BATCH);
 }
+// ... on the matrix cores: 4 rows and more, and three of up to 20 tiles
+static bool attn_out_chains(const Layer &y, int rows, int tiles) { return rows > LG_AOUT_DOT_ROWS || (rows == LG_AOUT_DOT_ROWS && y.wo_ch && tiles <= LG_AOUT_BATCH); }
+// ... with gate/up as part of the launch: two blocks of 32 FFN columns at most for a workgroup on the other seven XCDs; not beside the 13 wavefronts of lg_k_attn_out<3>
+static bool attn_out_geglu(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
+    return m->attn_geglu && m->aorows && y.wgu && y.nff / 32 <= 2 * LG_AOUT_GU_WGS && (rows < LG_AOUT_DOT_ROWS || attn_out_chains(y, rows, tiles));
+}
 static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
     if (!y.wo_ch || !m->tsync || !may_wait(m) || !attn_tail_shape(y.qd, m->E, nullptr, nullptr) || m->xcd_attn_tail <= 0 || (m->xcd_attn_tail == 1 && rows < 3)) return false;
     const int slices = (m->E + 1023) / 1024;
@@ -1587,7 +1594,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
     for (int L = 0; L < nl && !lx.rc; ++L) {
         const Layer &y = m->L[L];
         const int window = (y.is_local && m->window > 0) ? m->window + pos_off : 0;
-        bool fused_post = false, merged_o = false, ffn_rows_done = false;
+        bool fused_post = false, merged_o = false, ffn_rows_done = false, gate_up_done = false;
         {   // q/k/v projections, then per-head norm, rotary and the K/V rows of this block
             MmArgs a{ y.wqkv, E, y.qkv_m, m->qkv, m->hq, nullptr };
             if (qkv_done) { qkv_done = rows_done = false; }
@@ -1688,15 +1695,21 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 merged_o = true; ffn_rows_done = true;
             } else
             if (!merged_o && pos_off == 0 && have_x && use_attn_out(m, y, M, tiles)) {
-                const bool chains = M > LG_AOUT_DOT_ROWS || (M == LG_AOUT_DOT_ROWS && y.wo_ch && tiles <= LG_AOUT_BATCH);
+                const bool chains = attn_out_chains(y, M, tiles);
                 AttnOutArgs f{};
                 f.g = g; f.wo = chains ? y.wo_ch : y.wo; f.x = m->x[cur]; f.w_post = y.post_attn; f.w_pre = y.ffn_norm; f.x_out = m->x[cur ^ 1];
                 f.q = m->hq; f.E = E; f.tiles = tiles; f.eps = m->eps; f.sync = m->aosync; f.seq = L; f.spin_limit = m->wait_polls;
                 f.stamps = m->tail_stamps ? m->tstamps + LG_XTAIL_UNITS * 8 : nullptr;
+                if (attn_out_geglu(m, y, M, tiles)) {
+                    f.gw = y.wgu; f.nff = y.nff; f.gq = m->gq; f.gq_units = M >= 4 && m->down_m && y.wdn_m ? 2 : 0; f.rows = m->aorows;
+                    gate_up_done = true;
+                }
+                size_t lds = chains ? LG_AOUT_M_LDS : (size_t)M * LG_AOUT_K * 5 / 4;
+                if (gate_up_done) lds = std::max(lds, LG_AOUT_GU_LDS);
                 if constexpr (M >= LG_AOUT_DOT_ROWS)
-                    if (chains) LAUNCH(KC_ATAIL, lg_k_attn_out_m<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(768), 0, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
+                    if (chains) LAUNCH(KC_ATAIL, lg_k_attn_out_m<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(768), lds, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
                 if constexpr (M <= LG_AOUT_DOT_ROWS)
-                    if (!chains) LAUNCH(KC_ATAIL, lg_k_attn_out<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(64 * (LG_AOUT_G + M)), 0, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
+                    if (!chains) LAUNCH(KC_ATAIL, lg_k_attn_out<M>, dim3(LG_XCDS * LG_XCD_WGS), dim3(64 * (LG_AOUT_G + M)), lds, m->ctl, LG_AOUT_FIELDS(LG_XA, f) 0);
                 cur ^= 1;
                 merged_o = true; ffn_rows_done = true;
             } else
@@ -1751,7 +1764,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                     rows_in_geglu = true;
                 }
             }
-            if (rows_in_geglu) {
+            if (rows_in_geglu || gate_up_done) {
             } else {
             if (!ffn_rows_done) rows(y.ffn_norm, nullptr, mfma ? 2 : 1);
             if constexpr (mfma)
@@ -2032,7 +2045,7 @@ static GraphKey graph_key(const lg_hip_model *m, const lg_hip_kv *kv, int rows, 
     put(what, 2); put(rows, 4); put(m->store_logits != 0, 1); put(m->draft_chain, 1); put(m->fuse_rows, 1); put(m->attn_rows, 1); put(m->attn_rows_fq, 1);
     put(m->head_mfma, 1); put(m->down_kq, 1); put(m->xcd_ffn, 1); put(m->fork_ple, 1); put(m->rows_geglu, 1); put(m->tail_stamps != 0, 1);
     put(m->tail_spread == 1 ? 1 : m->tail_spread ? 2 : 0, 2); put(m->xcd_tail, 2); put(m->down_m, 2); put(m->xcd_attn_tail, 2); put(m->merge_o, 2);
-    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->tail_qkv, 1); put(m->wait_polls, 17); put(may_wait(m), 1);
+    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->tail_qkv, 1); put(m->attn_geglu, 1); put(m->wait_polls, 17); put(may_wait(m), 1);
     return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices, 0 };
 }
 
@@ -2097,6 +2110,7 @@ extern "C" int lg_hip_set_option(lg_hip_model *m, const char *name, int value) {
     else if (!strcmp(name, "narrow")) m->narrow = value != 0;
     else if (!strcmp(name, "attn_out")) m->attn_out = value != 0;
     else if (!strcmp(name, "tail_qkv")) m->tail_qkv = value != 0;
+    else if (!strcmp(name, "attn_geglu")) m->attn_geglu = value != 0;
     else if (!strcmp(name, "down_kq")) m->down_kq = value != 0;
     else if (!strcmp(name, "xcd_ffn")) m->xcd_ffn = value != 0 && m->xffn_built;
     else if (!strcmp(name, "fork_ple")) m->fork_ple = value != 0;
@@ -2448,8 +2462,9 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
             const int tiles = ((pos + rows - 1) >> 5) - (st >> 5) + 1;
             b[use_attn_tail(m, y, rows, tiles) ? KC_ATAIL : use_merge_o(m, y, rows, tiles) ? KC_MERGE : use_attn_out(m, y, rows, step_tiles(m, kv, y, rows, 0)) ? KC_ATAIL : KC_O] += (double)y.qd * m->E * q;
         }
+        const int tiles = step_tiles(m, kv, y, rows, 0);
         if (m->xffn_built && m->xcd_ffn && may_wait(m) && rows >= 4) b[KC_FFN] += 3.0 * m->E * y.nff * q;
-        else { b[KC_GATEUP] += 2.0 * m->E * y.nff * q; b[KC_DOWN] += (double)y.nff * m->E * q; }
+        else { b[use_attn_out(m, y, rows, tiles) && attn_out_geglu(m, y, rows, tiles) ? KC_ATAIL : KC_GATEUP] += 2.0 * m->E * y.nff * q; b[KC_DOWN] += (double)y.nff * m->E * q; }
         if (m->ple && !y.winp_f && use_ple_tail(m, rows)) b[KC_TAIL] += 2.0 * m->E * m->ple * q;
         else if (m->ple) { const double pq = y.winp_f ? 4.0 : q; b[KC_PLEGATE] += (double)m->E * m->ple * pq; b[KC_PLEPROJ] += (double)m->ple * m->E * pq; }
         }

@@ -41,42 +41,40 @@ struct XtailSync {
     uint32_t flags[2][LG_XTAIL_UNITS];      // lg_k_attn_tail: lg_tag of each unit's last arrival
 };
 
-// q8 rows that a launch hands from its one XCD to the workgroups on the other seven, two dwords of a row or a {scale, sum} pair to a unit, every dword
-// with the launch's tag (row j: k/8 units of dwords, then k/32 of pairs; either in the order in which the consumer keeps them in LDS).  Stored and loaded with
-// an agent's scope: through the writer's L2 to memory, and around the reader's.
+// q8 rows that a launch hands from its one XCD to the workgroups on the other seven, in units of 16 bytes: three dwords and the launch's number exclusive-or'ed
+// with them (a lane's 16 bytes travel together; were they ever seen apart, the fourth dword would not fit).  Stored and loaded with an agent's scope: through the
+// writer's L2 to memory, and around the reader's.  A block of 32 values is three units, its 8 dwords and its scale.  On v_dot4 (lg_take_far_rows) the sum
+// of the values is added up by the reader; on the matrix cores weights are signed and none is needed.
 struct FarRows {
     uint2 soon;                     // {-, tag}: the rows are on their way, from here on the waiting workgroups load them until they are there
     uint2 pad[15];
-    uint4 u[LG_HIP_MAX_ROWS_DEV * LG_MAXK_FAR * 5 / 32];
+    uint4 u[LG_HIP_MAX_ROWS_DEV * LG_MAXK_FAR / 32 * 3];
 };
-__device__ __forceinline__ void lg_put_far(uint2 *p, uint32_t v, uint32_t tag) {
-    __hip_atomic_store((unsigned long long *)p, (unsigned long long)tag << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ uint32_t lg_far_tag(uint32_t tag) { return tag & ~15u; }      // (the reader is on another XCD)
+__device__ __forceinline__ void lg_put_soon(FarRows *f, uint32_t tag) {
+    __hip_atomic_store((unsigned long long *)&f->soon, (unsigned long long)tag << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// MFMA: as the 80-dword blocks of lg_k_geglu_m, else in the order of lg_act_layout.  A lane's four values (quad of row j) and, by the first lane of a block, its pair
-template <bool MFMA>
-__device__ __forceinline__ void lg_put_far_q8(FarRows *f, int k, int j, int quad, uint32_t packed, float d, int sum, uint32_t tag) {
-    uint2 *row = (uint2 *)(f->u + (size_t)j * (k * 5 >> 5));
-    const ActLayout lay = lg_act_layout(k);
-    const int b = quad >> 3, dw = quad & 7;
-    lg_put_far(row + (MFMA ? b * 8 + ((dw & 1) | ((dw & 2) << 1) | ((dw & 4) >> 1)) : lg_act_unit(lay, quad >> 2) * 4 + (quad & 3)), packed, tag);
-    if (dw == 0) {
-        uint2 *p = row + (k >> 2) + 2 * (MFMA ? b : lg_act_block(lay, b));
-        lg_put_far(p, __float_as_uint(d), tag);
-        lg_put_far(p + 1, MFMA ? __float_as_uint(12582912.0f + (float)(8 * sum)) : (uint32_t)sum, tag);
-    }
+// A lane's four values (quad of row j) of a block that 8 lanes hold, d: its scale
+__device__ __forceinline__ void lg_put_far_q8(FarRows *f, int k, int j, int quad, uint32_t packed, float d, uint32_t tag) {
+    const uint32_t b = (uint32_t)lg_dpp_i<0x101>((int)packed), c = (uint32_t)lg_dpp_i<0x102>((int)packed);      // (row_shl: of the next lane and the one behind it)
+    const int dw = quad & 7;
+    if (dw % 3) return;                                        // lanes 0, 3 and 6 store
+    const uint32_t z = dw == 6 ? __float_as_uint(d) : c;
+    const __amdgpu_buffer_rsrc_t r = lg_buffer_rsrc(f->u);
+    lg_x4u v; v.x = packed; v.y = b; v.z = z; v.w = tag ^ packed ^ b ^ z;
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, ((j * (k >> 5) + (quad >> 3)) * 3 + dw / 3) * 16, 0, 16);      // (16: the scope bit sc1)
 }
 // Wait until the rows are on their way (one load per wavefront and trip: workgroups that load the rows all the time keep the memory from the ones that make them)
 __device__ __forceinline__ int lg_wait_soon(const FarRows *f, uint32_t tag, int spin_limit) {
     for (int spins = 0;; ++spins) {
-        const uint32_t diff = (uint32_t)(lg_ld_l2_u64(&f->soon) >> 32) ^ tag;
-        if ((diff >> 4) == 0) return 0;
+        if ((uint32_t)(lg_ld_l2_u64(&f->soon) >> 32) == tag) return 0;
         if (spins >= spin_limit) return LG_XFFN_ERR_WAIT;
         __builtin_amdgcn_s_sleep(1);
     }
 }
-// Units at(i) of the rows, i = 0 .. total - 1, by nt threads, at most N of a thread, to `to(i)` in LDS (two dwords each)
+// Units at(i), i = 0 .. total - 1, by nt threads, at most N of a thread; then put(i, unit)
 template <int N, typename A, typename P>
-__device__ __forceinline__ int lg_take_far_q8(const FarRows *f, int total, int t, int nt, uint32_t tag, int spin_limit, A &&at, P &&to) {
+__device__ __forceinline__ int lg_take_far(const FarRows *f, int total, int t, int nt, uint32_t tag, int spin_limit, A &&at, P &&put) {
     const __amdgpu_buffer_rsrc_t r = lg_buffer_rsrc(f->u);
     lg_x4u v[N];
     int err = 0, o[N];
@@ -85,17 +83,66 @@ __device__ __forceinline__ int lg_take_far_q8(const FarRows *f, int total, int t
     for (int spins = 0;; ++spins) {
         uint32_t diff = 0;
         #pragma unroll
-        for (int i = 0; i < N; ++i) v[i] = __builtin_bit_cast(lg_x4u, __builtin_amdgcn_raw_buffer_load_b128(r, o[i], 0, 16));      // (16: the scope bit sc1)
+        for (int i = 0; i < N; ++i) v[i] = __builtin_bit_cast(lg_x4u, __builtin_amdgcn_raw_buffer_load_b128(r, o[i], 0, 16));
         #pragma unroll
-        for (int i = 0; i < N; ++i) diff |= (v[i].y ^ tag) | (v[i].w ^ tag);
-        if (__all((diff >> 4) == 0)) break;
+        for (int i = 0; i < N; ++i) diff |= v[i].x ^ v[i].y ^ v[i].z ^ v[i].w ^ tag;
+        if (__all(diff == 0)) break;
         if (spins >= spin_limit) { err = LG_XFFN_ERR_WAIT; break; }
         asm volatile("" ::: "memory");
     }
     #pragma unroll
-    for (int i = 0; i < N; ++i) if (t + nt * i < total) *(uint2 *)to(t + nt * i) = make_uint2(v[i].x, v[i].z);
+    for (int i = 0; i < N; ++i) if (t + nt * i < total) put(t + nt * i, v[i]);
     return err;
 }
+// The rows in LDS for the matrix cores: a block of 32 values of all rows is LG_FAR_BLK bytes, 8 slots of 32 bytes (dwords in the order 0 1 4 5 2 3 6 7, the K halves
+// that a lane takes) and 8 scales.  Row j of 2i + h is in slot 4h + i, so that the lanes of either half h, which get slots 4h .. 4h + 3 of a product, have
+// (M + 1) / 2 results of rows and not four.
+#define LG_FAR_BLK 288
+__host__ __device__ static inline constexpr int lg_far_slot(int j) { return (j & 1) * 4 + (j >> 1); }
+// Wavefront `wave`'s K segment (nit blocks of 32, at most NIT) of M rows of k values, into the blocks at la.  A lane's units are the same of every row
+// that it takes (two at a time, where a half of the wavefront holds a row's units), so that nothing is left to compute when they arrive; what is past the rows
+// or the segment is its last once more.
+template <int M, int NIT>
+__device__ __forceinline__ int lg_take_far_segment(const FarRows *f, int k, int nit, int wave, int lane, unsigned char *la, uint32_t tag, int spin_limit) {
+    constexpr int H = 3 * NIT <= 32 ? 2 : 1, N = (M + H - 1) / H;                // rows of a trip, trips
+    const int h = H == 2 ? lane >> 5 : 0, x = H == 2 ? lane & 31 : lane, w = x < 3 * nit ? x : 3 * nit - 1, b = w / 3, e = w - 3 * b, nb = k >> 5;
+    auto pos = [](int m) { return (m & 1) | ((m & 2) << 1) | ((m & 4) >> 1); };
+    uint32_t *blk = (uint32_t *)(la + (size_t)b * LG_FAR_BLK), *s0 = blk + (H == 2 ? 32 * h : 0) + pos(3 * e), *s1 = blk + (H == 2 ? 32 * h : 0) + pos(3 * e + 1);
+    uint32_t *s2 = e == 2 ? blk + 64 + (H == 2 ? 4 * h : 0) : blk + (H == 2 ? 32 * h : 0) + pos(3 * e + 2);
+    const int st = e == 2 ? 1 : 8;                             // dwords from a slot to the next
+    const __amdgpu_buffer_rsrc_t r = lg_buffer_rsrc(f->u);
+    const int at = (wave * nit * 3 + w) * 16, row = nb * 48;
+    lg_x4u v[N];
+    int err = 0;
+    for (int spins = 0;; ++spins) {
+        uint32_t diff = 0;
+        #pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int j = H * i + h < M ? H * i + h : M - 1;   // (a lane's own only where the last trip has one row)
+            v[i] = __builtin_bit_cast(lg_x4u, __builtin_amdgcn_raw_buffer_load_b128(r, at + j * row, 0, 16));
+        }
+        #pragma unroll
+        for (int i = 0; i < N; ++i) diff |= v[i].x ^ v[i].y ^ v[i].z ^ v[i].w ^ tag;
+        if (__all(diff == 0)) break;
+        if (spins >= spin_limit) { err = LG_XFFN_ERR_WAIT; break; }
+        asm volatile("" ::: "memory");
+    }
+    #pragma unroll
+    for (int i = 0; i < N; ++i) {                              // (row H i + h: slot 4 h + i, or lg_far_slot(i))
+        const int z = H == 2 ? i : lg_far_slot(i);
+        s0[z * 8] = v[i].x; s1[z * 8] = v[i].y; s2[z * st] = v[i].z;
+    }
+    return err;
+}
+// Weights as the high nibbles of bytes, two's complement: their product with values is 16 times the dot, which the accumulators' start, the bits of 1.5 * 2^19,
+// turns into 786432 + dot, exactly
+#define LG_FAR_MAGIC 0x49400000
+#define LG_FAR_BIAS 786432.0f
+__device__ __forceinline__ lg_v4i lg_far_weights(uint32_t x, uint32_t y) {      // (nibbles of x and y: signed)
+    lg_v4i b; b.x = (x << 4) & 0xF0F0F0F0; b.y = (y << 4) & 0xF0F0F0F0; b.z = x & 0xF0F0F0F0; b.w = y & 0xF0F0F0F0;
+    return b;
+}
+template <int N> __device__ __forceinline__ float lg_row_bcast(float v) { return lg_dpp_f<0x150 + N>(v); }      // lane N of each row of 16
 
 struct XtailArgs {
     RowsPleGateArgs r;              // phase 1 (x_out is not written: the row stays in registers)
@@ -330,7 +377,7 @@ template <int M, int NIT, bool MFMA = (M >= LG_TAIL_MFMA)> struct TailQkv;
 // ... a block of 32 rows, a K segment to a wavefront (lg_k_attn_tail), which takes its part of the rows itself
 template <int M, int NIT>
 struct TailQkv<M, NIT, true> {
-    static constexpr int ROWS = 32, N = (NIT + 1) / 2;
+    static constexpr int ROWS = 32, N = (NIT + 1) / 2, I = (M + 1) / 2;
     lg_v4i b[NIT]; float dw[NIT];
     __device__ __forceinline__ void request(const XtailArgs &a, int rank, int wave, int lane, int nit) {
         const uint8_t *cb = a.qw + ((size_t)rank * 8 + wave) * (nit * 576);
@@ -343,51 +390,39 @@ struct TailQkv<M, NIT, true> {
         }
         #pragma unroll
         for (int i = 0; i < NIT; ++i) {
-            const uint32_t x = i & 1 ? q[i >> 1].z : q[i >> 1].x, y = i & 1 ? q[i >> 1].w : q[i >> 1].y;
-            b[i].x = x & 0x0F0F0F0F; b[i].y = y & 0x0F0F0F0F; b[i].z = (x >> 4) & 0x0F0F0F0F; b[i].w = (y >> 4) & 0x0F0F0F0F;
+            b[i] = lg_far_weights((i & 1 ? q[i >> 1].z : q[i >> 1].x) ^ 0x88888888u, (i & 1 ? q[i >> 1].w : q[i >> 1].y) ^ 0x88888888u);
             dw[i] = lg_h2f((uint16_t)(i & 1 ? s[i >> 1] >> 16 : s[i >> 1]));
             asm volatile("" : "+v"(b[i]), "+v"(dw[i]));
         }
     }
     __device__ __forceinline__ int take(const XtailArgs &a, int wave, int lane, int nit, unsigned char *act, uint32_t tag) {
-        const int k = a.r.g.k, per = k * 5 >> 5, words = k >> 3, mine = nit * 5, first = wave * nit;
-        unsigned char *la = act + (size_t)first * (LG_MU_DWORDS * 4);
-        return lg_take_far_q8<(5 * NIT * M + 63) / 64>(a.rows, mine * M, lane, 64, tag, a.spin_limit, [&](int i) {
-            const int j = i / mine, w = i - j * mine;
-            return j * per + (w < 4 * nit ? 4 * first + w : words + first + w - 4 * nit);
-        }, [&](int i) {
-            const int j = i / mine, w = i - j * mine;
-            return w < 4 * nit ? la + (size_t)(w >> 2) * (LG_MU_DWORDS * 4) + j * 32 + (w & 3) * 8 : la + (size_t)(w - 4 * nit) * (LG_MU_DWORDS * 4) + 256 + j * 8;
-        });
+        return lg_take_far_segment<M, NIT>(a.rows, a.r.g.k, nit, wave, lane, act + (size_t)wave * NIT * LG_FAR_BLK, tag, a.spin_limit);
     }
     // xch: 8 KB of LDS
     __device__ __forceinline__ void finish(const XtailArgs &a, int rank, int wave, int t, int nit, const unsigned char *act, float *xch, int real) {
         const int lane = t & 63, n = lane & 31, h = lane >> 5, arow = n < 8 ? n : 7;
         lg_v16i magic;
         #pragma unroll
-        for (int i = 0; i < 16; ++i) magic[i] = 0x4B400000;
+        for (int i = 0; i < 16; ++i) magic[i] = LG_FAR_MAGIC;
         asm volatile("" : "+v"(magic));
-        float p[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
-        const unsigned char *ls = act + (size_t)wave * nit * (LG_MU_DWORDS * 4);
-        // (no branch on a shorter segment's end: its last block again, the result not taken)
-        auto block = [&](int i) { return lg_xffn_act(ls + (i < nit ? i : nit - 1) * (LG_MU_DWORDS * 4), arow, h); };
-        XffnAct ac[3] = { block(0), block(1), block(2) };
+        float p[I];
+        #pragma unroll
+        for (int r = 0; r < I; ++r) p[r] = 0.0f;
+        const unsigned char *ls = act + (size_t)wave * NIT * LG_FAR_BLK, *la = ls + arow * 32 + h * 16;
         lg_v16i d[2];
-        d[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ac[0].av, b[0], magic, 0, 0, 0);
+        d[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(*(const lg_v4i *)la, b[0], magic, 0, 0, 0);
         #pragma unroll
         for (int i = 0; i < NIT; ++i) {                        // (the next block's dots on their way while this one's join the sums)
-            if (i + 1 < NIT) d[(i + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ac[(i + 1) % 3].av, b[i + 1 < NIT ? i + 1 : i], magic, 0, 0, 0);
-            const XffnAct &c = ac[i % 3];
+            if (i + 1 < NIT) d[(i + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(*(const lg_v4i *)(la + (i + 1) * LG_FAR_BLK), b[i + 1 < NIT ? i + 1 : i], magic, 0, 0, 0);
             #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float v = lg_fmaf(c.xd[r] * dw[i], __int_as_float(d[i & 1][r]) - c.cf[r], p[r]);
-                p[r] = i < nit ? v : p[r];
+            for (int r = 0; r < I; ++r) {
+                const float v = lg_fmaf(*(const float *)(ls + i * LG_FAR_BLK + 256 + (4 * h + r) * 4) * dw[i], __int_as_float(d[i & 1][r]) - LG_FAR_BIAS, p[r]);
+                p[r] = i < nit ? v : p[r];                     // (no branch on a shorter segment's end: what lies behind it is not taken)
+                asm volatile("" : "+v"(p[r]));
             }
-            asm volatile("" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]));
-            if (i + 3 < NIT) ac[i % 3] = block(i + 3);
         }
         #pragma unroll
-        for (int i = 0; i < 4; ++i) xch[(wave * 8 + 4 * h + i) * 32 + n] = p[i];
+        for (int i = 0; i < I; ++i) xch[(wave * 8 + 2 * i + h) * 32 + n] = p[i];
         __syncthreads();
         if (t < 32 * M && real) {                              // the adjacent-pair tree over the 8 segments
             const float *z = xch + t;
@@ -411,10 +446,17 @@ struct TailQkv<M, NIT, false> {
         }
     }
     __device__ __forceinline__ int take(const XtailArgs &a, int wave, int lane, int nit, unsigned char *act, uint32_t tag) {
-        const int k = a.r.g.k, per = k * 5 >> 5, words = k >> 3;
-        const int err = lg_take_far_q8<(40 * NIT * M + 511) / 512>(a.rows, per * M, wave * 64 + lane, 512, tag, a.spin_limit, [&](int i) { return i; }, [&](int i) {
-            const int j = i / per, w = i - j * per;
-            return w < words ? act + (size_t)j * k + 8 * w : act + (size_t)M * k + ((size_t)j * (k >> 5) + (w - words)) * 8;
+        // (a block's units by three lanes in a row of four, the fourth idle: its sum is added up across them)
+        const int k = a.r.g.k, nb = k >> 5;
+        const ActLayout lay = lg_act_layout(k);
+        const int err = lg_take_far<(32 * NIT * M + 511) / 512>(a.rows, nb * M * 4, wave * 64 + lane, 512, tag, a.spin_limit, [&](int i) { return (i >> 2) * 3 + min(i & 3, 2); }, [&](int i, const lg_x4u &v) {
+            const int e = i & 3, j = (i >> 2) / nb, b = (i >> 2) - j * nb;
+            int sum = e == 3 ? 0 : __builtin_amdgcn_sdot4((int)v.x, 0x01010101, __builtin_amdgcn_sdot4((int)v.y, 0x01010101, e == 2 ? 0 : __builtin_amdgcn_sdot4((int)v.z, 0x01010101, 0, false), false), false);
+            sum += lg_dpp_i<LG_DPP_SWAP1>(sum); sum += lg_dpp_i<LG_DPP_SWAP2>(sum);
+            auto put = [&](int m, uint32_t w) { *(uint32_t *)(act + (size_t)j * k + lg_act_unit(lay, b * 2 + (m >> 2)) * 16 + (m & 3) * 4) = w; };
+            if (e < 3) { put(3 * e, v.x); put(3 * e + 1, v.y); }
+            if (e < 2) put(3 * e + 2, v.z);
+            if (e == 2) *(float2 *)(act + (size_t)M * k + ((size_t)j * nb + lg_act_block(lay, b)) * 8) = make_float2(__uint_as_float(v.z), __int_as_float(sum));
         });
         __syncthreads();
         return err;
@@ -428,14 +470,17 @@ struct TailQkv<M, NIT, false> {
         if (c < M && real) a.qout[(size_t)c * a.qm + g0 * 8 + (lane >> 3)] = lg_pick<M>(acc, c);
     }
 };
+// bytes of the rows in LDS
+__host__ __device__ static inline size_t lg_tail_act(int M, int E) { return M >= LG_TAIL_MFMA ? (size_t)8 * (E <= 2560 ? 10 : 16) * LG_FAR_BLK : (size_t)M * E * 5 / 4; }
 // bytes of LDS of lg_k_ple_tail_s; with the projections: the rows, 8 slots wide on the matrix cores, and 8 KB for sums
 static inline size_t lg_tail_s_lds(int M, int E, int ple, bool qkv) {
-    return (size_t)E * 5 / 4 + (size_t)M * ple * 5 / 4 + (qkv ? (size_t)(M >= LG_TAIL_MFMA ? 8 : M) * E * 5 / 4 + 8192 : 0);
+    const size_t units = (size_t)E * 5 / 4 + (size_t)M * ple * 5 / 4, far = qkv ? lg_tail_act(M, E) + 8192 : 0;
+    return units > far ? units : far;
 }
 template <int M, int NIT>
 __device__ __forceinline__ void lg_tail_qkv(const XtailArgs &a, int rank, unsigned char *act, uint32_t tag, StepCtl *ctl) {
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), E = a.r.g.k, nit = E >> 8;
-    float *xch = (float *)(act + (size_t)(M >= LG_TAIL_MFMA ? 8 : M) * E * 5 / 4);
+    float *xch = (float *)(act + lg_tail_act(M, E));
     TailQkv<M, NIT> qkv;
     qkv.request(a, rank, wave, t & 63, nit);
     __builtin_amdgcn_sched_barrier(0);
@@ -606,7 +651,7 @@ __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FI
     err = 0;
     if (rowt) lg_take_row(dv, a.pout + (size_t)j * E, t, nq, tag, a.spin_limit, err);
     if (err) atomicOr(&ctl->err, err);
-    if (a.qw && u == 0 && t == 0) lg_put_far(&a.rows->soon, 0, tag);
+    if (a.qw && u == 0 && t == 0) lg_put_soon(a.rows, lg_far_tag(tag));
     stamp(5);
     {
         float ss = 0.0f;
@@ -662,7 +707,7 @@ __global__ __launch_bounds__(512) void lg_k_ple_tail_s(StepCtl *ctl, LG_XTAIL_FI
             float d; int sum;
             const uint32_t packed = lg_quant4_8lanes(xv[v], &d, &sum);
             const int quad = t + 256 * v;
-            if (a.qw) lg_put_far_q8<(M >= LG_TAIL_MFMA)>(a.rows, E, j, quad, packed, d, sum, tag);
+            if (a.qw) lg_put_far_q8(a.rows, E, j, quad, packed, d, lg_far_tag(tag));
             else if (a.q_units == 2) {
                 uint32_t *blk = (uint32_t *)a.q + (size_t)(quad >> 3) * LG_MU_DWORDS;
                 const int dw = quad & 7;
