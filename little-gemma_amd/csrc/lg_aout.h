@@ -66,6 +66,29 @@ struct AttnOutArgs {
 #define LG_AOUT_NIT (LG_AOUT_E / 256)
 #define LG_AOUT_GU_WGS ((LG_XCDS - 1) * LG_XCD_WGS)
 #define LG_AOUT_GU_LDS ((size_t)8 * LG_AOUT_NIT * (LG_FAR_BLK + LG_TILE) + LG_AOUT_NIT * LG_FAR_BLK + 2 * 8 * 8 * 64 * 4)
+// The segments' sums of one or two blocks of 32 FFN columns -> their GeGLU as q8: half-wavefront per row, one FFN column per lane
+template <int M>
+__device__ __forceinline__ void lg_far_geglu_out(const float (*red)[8][8][64], bool two, int b0, int b1, int t, int8_t *gq, int gq_units, int nff) {
+    for (int x = t >> 5; x < (two ? 2 * M : M); x += 16) {
+        const int o = x >= M, j = x - (o ? M : 0), i = t & 31, b = o ? b1 : b0;
+        float g[8], u[8];
+        #pragma unroll
+        for (int c = 0; c < 8; ++c) { g[c] = red[o][c][j][i]; u[c] = red[o][c][j][32 + i]; }
+        const float gate = ((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7])), up = ((u[0] + u[1]) + (u[2] + u[3])) + ((u[4] + u[5]) + (u[6] + u[7]));
+        float d; int sum;
+        const int v = lg_quant1_32lanes(lg_gelu_d(gate) * up, &d, &sum);
+        if (gq_units == 2) {
+            int8_t *blk = gq + (size_t)b * (LG_MU_DWORDS * 4);
+            const int dw = i >> 2;
+            blk[(j * 8 + ((dw & 1) | ((dw & 2) << 1) | ((dw & 4) >> 1))) * 4 + (i & 3)] = (int8_t)v;
+            if (i == 0) *(float2 *)(blk + 256 + 8 * j) = make_float2(d, 12582912.0f + (float)(8 * sum));
+        } else {
+            const ActLayout lay = lg_act_layout(nff);
+            gq[(size_t)j * nff + lg_act_unit(lay, b * 2 + (i >> 4)) * 16 + (i & 15)] = (int8_t)v;
+            if (i == 0) lg_q8_ds<M>(gq, nff)[(size_t)j * (nff >> 5) + lg_act_block(lay, b)] = make_float2(d, __int_as_float(sum));
+        }
+    }
+}
 template <int N, typename F, int... X> __device__ __forceinline__ void lg_unroll_(F &&f, std::integer_sequence<int, X...>) { (f(std::integral_constant<int, X>{}), ...); }
 template <int N, typename F> __device__ __forceinline__ void lg_unroll(F &&f) { lg_unroll_<N>(f, std::make_integer_sequence<int, N>{}); }
 template <int M>
@@ -155,27 +178,7 @@ __device__ __forceinline__ void lg_aout_geglu(const AttnOutArgs &a, int rank, un
     if (nit == NIT) { if (two) chains(std::true_type{}, std::true_type{}); else chains(std::false_type{}, std::true_type{}); }
     else            { if (two) chains(std::true_type{}, std::false_type{}); else chains(std::false_type{}, std::false_type{}); }
     __syncthreads();
-    {
-        for (int x = t >> 5; x < (two ? 2 * M : M); x += 16) {            // half-wavefront per row, one FFN column per lane
-            const int o = x >= M, j = x - (o ? M : 0), i = t & 31, b = o ? b1 : rank;
-            float g[8], u[8];
-            #pragma unroll
-            for (int c = 0; c < 8; ++c) { g[c] = red[o][c][j][i]; u[c] = red[o][c][j][32 + i]; }
-            const float gate = ((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7])), up = ((u[0] + u[1]) + (u[2] + u[3])) + ((u[4] + u[5]) + (u[6] + u[7]));
-            float d; int sum;
-            const int v = lg_quant1_32lanes(lg_gelu_d(gate) * up, &d, &sum);
-            if (a.gq_units == 2) {
-                int8_t *blk = a.gq + (size_t)b * (LG_MU_DWORDS * 4);
-                const int dw = i >> 2;
-                blk[(j * 8 + ((dw & 1) | ((dw & 2) << 1) | ((dw & 4) >> 1))) * 4 + (i & 3)] = (int8_t)v;
-                if (i == 0) *(float2 *)(blk + 256 + 8 * j) = make_float2(d, 12582912.0f + (float)(8 * sum));
-            } else {
-                const ActLayout lay = lg_act_layout(a.nff);
-                a.gq[(size_t)j * a.nff + lg_act_unit(lay, b * 2 + (i >> 4)) * 16 + (i & 15)] = (int8_t)v;
-                if (i == 0) lg_q8_ds<M>(a.gq, a.nff)[(size_t)j * (a.nff >> 5) + lg_act_block(lay, b)] = make_float2(d, __int_as_float(sum));
-            }
-        }
-    }
+    lg_far_geglu_out<M>(red, two, rank, b1, t, a.gq, a.gq_units, a.nff);
 }
 
 // One wavefront's merge of 64 dims (number u of the row's) of row j, lane = dim: at most T tiles

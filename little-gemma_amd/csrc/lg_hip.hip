@@ -31,6 +31,7 @@
 #include "lg_xrg.h"
 #include "lg_narrow.h"
 #include "lg_aout.h"
+#include "lg_mid.h"
 
 static_assert(LG_HIP_MAX_ROWS == LG_HIP_MAX_ROWS_DEV, "row limits must agree");
 #define LG_FUSE_ROWS_MAX 2         // widest block whose q/k/v matmul does the preceding row work itself
@@ -169,6 +170,7 @@ struct Layer {
     uint8_t *wqkv = nullptr, *wo = nullptr, *wgu = nullptr, *wdown = nullptr, *winp = nullptr, *wproj = nullptr;
     float *winp_f = nullptr, *wproj_f = nullptr;   // inp_gate / proj when the file keeps them in a float type (then winp / wproj are null)
     uint8_t *wdn_m = nullptr;                      // ffn_down again as the per-workgroup streams of lg_k_down_m
+    uint8_t *wqkv_pc = nullptr, *wo_pc = nullptr;  // q/k/v and attn_output again as chains of pairs of K segments (pack_pairs): lg_k_down_qkv, lg_k_o_geglu
     uint8_t *wqkv_ch = nullptr;                    // q/k/v again as such chains: lg_k_ple_tail_s of 4..8 rows
     uint8_t *wo_ch = nullptr;                      // attn_output again as matrix-core chains [row block][segment]: lg_k_attn_tail, lg_k_attn_out_m
     // the matrices once more in the form of the prompt kernels (lg_wide.h)
@@ -242,7 +244,7 @@ struct lg_hip_model {
     int last_rows = 0, last_adv = 0;
     float *lstage = nullptr;           // pinned: two rows of logits on their way to a caller (lg_hip_get_logits), row j in half j % 2
     int lread = -1, lcoming = -1;      // the row of the latest step read last, and the one whose copy has been started
-    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1, attn_out = 1, tail_qkv = 1, attn_geglu = 1;
+    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1, attn_out = 1, tail_qkv = 1, attn_geglu = 1, mid = 1;
     // the feed-forward half of a layer as one XCD-partitioned launch (lg_xffn.h): built when the shape and the chip fit
     int xcd_ffn = 0;                         // option: use it (verify blocks of 4..8 rows)
     int down_m = 1;                          // option: ffn_down of 4..8-row blocks on the matrix cores (lg_k_down_m): 1 = the row group's four workgroups add
@@ -260,6 +262,8 @@ struct lg_hip_model {
     int xcd_tail = 1;                        // option: 0 off, 1 for blocks that do not fold the row work into q/k/v, 2 for every verify block
     XtailSync *tsync = nullptr;
     uint2 *tgf = nullptr, *tpr = nullptr;    // [LG_HIP_MAX_ROWS][ple] and [LG_HIP_MAX_ROWS][E] its gated values and projections, tagged
+    uint2 *mido = nullptr, *midd = nullptr, *mids = nullptr;   // [max rows][E] the first products of lg_k_o_geglu and lg_k_down_qkv, [3][max rows][E] slabs of the latter, tagged (option mid)
+    FarRows *midro = nullptr, *midrd = nullptr;                // their rows
     FarRows *trows = nullptr;                // rows of lg_k_ple_tail_s on their way to the next layer's projections (option tail_qkv)
     FarRows *aorows = nullptr;               // rows of lg_k_attn_out on their way to gate/up (option attn_geglu)
     AttnOutSync *aosync = nullptr;           // hand-over state of lg_k_attn_out (models it serves)
@@ -615,6 +619,42 @@ static void pack_o_chains(const uint8_t *const *rows, int k, int m, uint8_t *dst
                 }
         }
 }
+// Chains of pairs of segments (lg_mid.h)
+static void pack_pairs(const uint8_t *const *rows, int k, int m, uint8_t *dst) {
+    const int nit = k / 256, nitp = (nit + 1) & ~1;
+    auto work = [&](int r0, int r1) {
+        for (int rb = r0; rb < r1; ++rb)
+            for (int sp = 0; sp < 4; ++sp) {
+                uint8_t *ub = dst + ((size_t)rb * 4 + sp) * nitp * 576;
+                for (int l = 0; l < 64; ++l)
+                    for (int it = 0; it < nit; ++it) {
+                        const int sg = l >> 5, hf = (l >> 4) & 1, c = l & 15;
+                        const uint8_t *blk = rows[rb * 16 + c] + (size_t)((2 * sp + sg) * nit + it) * 18;
+                        uint8_t *q = ub + (size_t)((it >> 1) * 64 + l) * 16 + (it & 1) * 8;
+                        for (int i = 0; i < 8; ++i) q[i] = blk[2 + 8 * hf + i] ^ 0x88;
+                        if (!hf) memcpy(ub + (size_t)nitp * 512 + (size_t)((it >> 1) * 32 + sg * 16 + c) * 4 + (it & 1) * 2, blk, 2);
+                    }
+            }
+    };
+    std::vector<std::thread> pool;
+    const int nt = m / 16 < 16 ? 1 : 8;
+    for (int t = 0; t < nt; ++t) pool.emplace_back(work, (int)((long long)(m / 16) * t / nt), (int)((long long)(m / 16) * (t + 1) / nt));
+    for (auto &th : pool) th.join();
+}
+static int upload_pairs(lg_hip_model *m, const std::vector<const uint8_t *> &rows, int k, uint8_t **out, std::vector<uint8_t> &stage) {
+    stage.assign(lg_pairs_bytes(k, (int)rows.size()), 0);
+    pack_pairs(rows.data(), k, (int)rows.size(), stage.data());
+    if (dev_alloc(m, out, stage.size())) return -7;
+    HIP_TRY(copy_now(m->stream, *out, stage.data(), stage.size(), hipMemcpyHostToDevice));
+    return 0;
+}
+// Models and layers that lg_k_o_geglu and lg_k_down_qkv serve: one workgroup to a CU takes an equal share of either product
+static bool mid_model(const lg_hip_model *m) { return m->numbered && !m->target && cu_count() == LG_XCDS * LG_XCD_WGS && m->E > LG_NARROW_E && m->E <= LG_MID_E && m->E % 256 == 0; }
+static bool mid_o_shape(const lg_hip_model *m, int qd, int nff) { return mid_model(m) && qd % 1024 == 0 && qd <= LG_MID_K && nff / 32 <= LG_OG_BLOCKS; }
+static bool mid_down_shape(const lg_hip_model *m, int nff, int next_qkv) {
+    return mid_model(m) && !m->ple && lg_segments(nff) == 32 && nff <= 1024 * LG_MID_NIT && next_qkv % 32 == 0 && next_qkv <= 32 * LG_XCDS * LG_XCD_WGS;
+}
+static bool mid_proj_shape(const lg_hip_model *m, int next_qkv) { return mid_model(m) && m->ple == 256 && m->E % 256 == 0 && next_qkv % 32 == 0 && next_qkv <= 32 * LG_XCDS * LG_XCD_WGS; }
 // shapes lg_k_attn_tail is instantiated for: pairs of blocks per chain, row blocks per unit
 static bool attn_tail_shape(int qd, int E, int *np, int *rbs) {
     if (qd % 512 || lg_segments(qd) != 8 || E % 256 || E > 4096) return false;
@@ -746,6 +786,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         if ((rc = upload_tiled(m, rows, E, &y.wqkv, stage))) return rc;
         if ((rc = wide_form(m, y.wqkv, E, y.qkv_m, false, &y.wqkv_w))) return rc;
         const HostTensor *ig = m->ple == 256 ? find(m, lname(L, "inp_gate.weight")) : nullptr;
+        if (L > 0 && (mid_down_shape(m, m->L[L - 1].nff, y.qkv_m) || (ig && ig->type != 2 && mid_proj_shape(m, y.qkv_m))) && (rc = upload_pairs(m, rows, E, &y.wqkv_pc, stage))) return rc;
         if (ig && ig->type == 2 && !m->target && m->numbered && L > 0 && max_rows >= LG_TAIL_MFMA && E % 512 == 0 && E <= 4096 && y.qkv_m % 32 == 0 && cu_count() == LG_XCDS * LG_XCD_WGS) {
             stage.resize((size_t)y.qkv_m * (E / 32) * 18);       // (once more: the chains that lg_k_ple_tail_s takes)
             pack_o_chains(rows.data(), E, y.qkv_m, stage.data());
@@ -758,6 +799,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         push_rows(rows, o, 0, E);
         if ((rc = upload_tiled(m, rows, y.qd, &y.wo, stage))) return rc;
         if ((rc = wide_form(m, y.wo, y.qd, E, false, &y.wo_w))) return rc;
+        if (mid_o_shape(m, y.qd, y.nff) && (rc = upload_pairs(m, rows, y.qd, &y.wo_pc, stage))) return rc;
         // (8 query heads: the K segments of this projection are the heads, and the merge can run their chains itself)
         if (!m->target && cu_count() == LG_XCDS * LG_XCD_WGS &&
             ((getenv("LG_HIP_XCD_ATTN_TAIL") && atoi(getenv("LG_HIP_XCD_ATTN_TAIL")) > 0 && attn_tail_shape(y.qd, E, nullptr, nullptr)) ||
@@ -876,6 +918,8 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         HIP_TRY(clear_now(m->stream, m->aq, 0, qb(max_qd)));       // (row slots past the block are read as operand rows of the matrix cores)
         if (getenv("LG_HIP_XCD_TAIL")) m->xcd_tail = atoi(getenv("LG_HIP_XCD_TAIL"));
     }
+    if (mid_model(m) && (mark_alloc(m, &m->mido, (size_t)LG_HIP_MAX_ROWS * E) || mark_alloc(m, &m->midd, (size_t)LG_HIP_MAX_ROWS * E) || mark_alloc(m, &m->mids, (size_t)3 * LG_HIP_MAX_ROWS * E) ||
+                         mark_alloc(m, &m->midro) || mark_alloc(m, &m->midrd))) return -7;
     if (narrow_shape(m)) {
         if (mark_alloc(m, &m->nsync)) return -7;
     } else if (!m->target && cu_count() == LG_XCDS * LG_XCD_WGS) {
@@ -1352,9 +1396,21 @@ static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int t
     const int slices = (m->E + 1023) / 1024;
     return tiles < 128 && m->H * rows <= 2 * LG_XCD_WGS && slices * rows <= LG_XCD_WGS && y.hd % 32 == 0 && y.hd <= 256;
 }
+// attn_output, row work and gate/up as one launch; not where one of the options does that row work elsewhere
+static bool use_mid_o(const lg_hip_model *m, const Layer &y, int rows) {
+    return m->mid && m->attn_out && m->mido && may_wait(m) && y.wo_pc && y.wgu && !(rows >= 4 && (m->rows_geglu || (m->xcd_ffn && y.xgu)));
+}
+// ffn_down, row work and the next layer's q/k/v projections as one launch (1 to 3 rows: with the whole rows in LDS)
+static bool use_mid_down(const lg_hip_model *m, const Layer &y, const Layer &next, int rows) {
+    if (!m->mid || !m->midd || !may_wait(m) || m->ple || !next.wqkv_pc) return false;
+    if (rows >= 4) return m->down_m == 1 && y.wdn_m && m->E > 2048 && lg_down_m_geo(m->E, y.nff).npairs <= LG_MID_NDP;
+    return lg_downqkv_lds(rows, y.nff) <= 160 * 1024;
+}
+// ... with the per-layer projection of a float type in ffn_down's place
+static bool use_mid_proj(const lg_hip_model *m, const Layer &next) { return m->mid && m->midd && may_wait(m) && m->ple && next.wqkv_pc; }
 // Whether a step has launches whose workgroups wait for one another, if it may
 static bool step_waits(const lg_hip_model *m, int rows) {
-    return may_wait(m) && (use_narrow(m, rows) || (m->attn_out && m->aosync) || use_ple_tail(m, rows) || m->rows_geglu || m->xcd_attn_tail > 0 ||
+    return may_wait(m) && (use_narrow(m, rows) || (m->attn_out && m->aosync) || (m->mid && m->mido) || use_ple_tail(m, rows) || m->rows_geglu || m->xcd_attn_tail > 0 ||
                            (rows >= 4 && ((m->down_m == 1 && m->dmsync) || m->xcd_ffn)));
 }
 // Held while a step of m is launched (or a round of `head` and m, its target); begin() finds out whether it may have such launches
@@ -1725,6 +1781,16 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
 #undef GO
             } else LAUNCH(KC_MERGE, (lg_k_attn_merge<M>), dim3(H, M), dim3(LG_WG), 0, m->ctl, LG_MERGE_FIELDS(LG_XA, g) 0);
         }
+        if (!merged_o && pos_off == 0 && have_x && use_mid_o(m, y, M)) {
+            OGegluArgs f{};
+            f.ow = y.wo_pc; f.act = m->aq; f.out = m->mido; f.gw = y.wgu; f.gq = m->gq; f.qd = y.qd; f.nff = y.nff;
+            f.gq_units = M >= 4 && m->down_m && y.wdn_m ? 2 : 0; f.seq = L;
+            f.r = MidRowArgs{ m->x[cur], y.post_attn, nullptr, y.ffn_norm, m->x[cur ^ 1], nullptr, m->midro, E, m->wait_polls, m->eps };
+            if (E <= 2560) LAUNCH(KC_O, (lg_k_o_geglu<M, 10>), dim3(LG_XCDS * LG_XCD_WGS), dim3(512), LG_OG_LDS(10), m->ctl, LG_OGEGLU_FIELDS(LG_XA, f) 0);
+            else           LAUNCH(KC_O, (lg_k_o_geglu<M, 15>), dim3(LG_XCDS * LG_XCD_WGS), dim3(512), LG_OG_LDS(15), m->ctl, LG_OGEGLU_FIELDS(LG_XA, f) 0);
+            cur ^= 1;
+            merged_o = true; ffn_rows_done = true; gate_up_done = true;
+        }
         if (!merged_o) {   // attention output projection
             MmArgs a{ y.wo, y.qd, E, m->dout, m->aq, nullptr };
             pend_parts = launch_mm<M, false>(lx, KC_O, a);
@@ -1773,6 +1839,16 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 LAUNCH(KC_GATEUP, (lg_k_geglu_t<M>), dim3(y.nff / 32), dim3(512), 0, LG_GEGLU_FIELDS(LG_XA, a) 0);
             }
             MmArgs d{ y.wdown, y.nff, E, m->dout, m->gq, nullptr };
+            if (pos_off == 0 && have_x && L + 1 < nl && use_mid_down(m, y, m->L[L + 1], M)) {
+                DownQkvArgs f{};
+                f.d = DownHere{ M >= 4 ? y.wdn_m : y.wdown, m->gq, y.nff, E, m->mids, m->midd, m->wait_polls };
+                f.r = MidRowArgs{ m->x[cur], y.post_ffw, y.out_scale, m->L[L + 1].attn_norm, m->x[cur ^ 1], nullptr, m->midrd, E, m->wait_polls, m->eps };
+                f.qw = m->L[L + 1].wqkv_pc; f.qout = m->qkv; f.qm = m->L[L + 1].qkv_m; f.seq = L;
+                LAUNCH(KC_ROWS, (lg_k_down_qkv<M, false>), dim3(LG_XCDS * LG_XCD_WGS), dim3(512), lg_downqkv_lds(M, y.nff), m->ctl, LG_DOWNQKV_FIELDS(LG_XA, f) 0);
+                cur ^= 1;
+                rows_done = qkv_done = true;
+                continue;
+            }
             if (dn_m) {
                 DownMArgs dm{ y.wdn_m, (const uint32_t *)m->gq, m->dout, E, y.nff, m->down_m == 1 && may_wait(m) ? m->dmsync : nullptr, m->ctl, m->wait_polls, L };
                 launch_down_m<M>(lx, dm);
@@ -1795,6 +1871,16 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             rows(nullptr, nullptr);
             MmfArgs g{ y.winp_f, E, m->ple, m->x[cur], E, M, m->pgf, m->ple, m->pmp_raw + (size_t)L * m->ple, m->ple * nl };
             launch_mmf<M>(lx, KC_PLEGATE, g);
+            }
+            if (pos_off == 0 && L + 1 < nl && use_mid_proj(m, m->L[L + 1])) {      // the projection, the row work behind it and the next layer's projections
+                DownQkvArgs f{};
+                f.d = DownHere{ (const uint8_t *)y.wproj_f, m->pgf, 0, E, nullptr, m->midd, m->wait_polls };
+                f.r = MidRowArgs{ m->x[cur], y.post_norm, y.out_scale, m->L[L + 1].attn_norm, m->x[cur ^ 1], nullptr, m->midrd, E, m->wait_polls, m->eps };
+                f.qw = m->L[L + 1].wqkv_pc; f.qout = m->qkv; f.qm = m->L[L + 1].qkv_m; f.seq = L;
+                LAUNCH(KC_ROWS, (lg_k_down_qkv<M, true>), dim3(LG_XCDS * LG_XCD_WGS), dim3(512), LG_DOWNQKV_ACT, m->ctl, LG_DOWNQKV_FIELDS(LG_XA, f) 0);
+                cur ^= 1;
+                rows_done = qkv_done = true;
+                continue;
             }
             MmfArgs p{ y.wproj_f, m->ple, E, m->pgf, m->ple, M, m->dout, E, nullptr, 0 };
             launch_mmf<M>(lx, KC_PLEPROJ, p);
@@ -2045,7 +2131,7 @@ static GraphKey graph_key(const lg_hip_model *m, const lg_hip_kv *kv, int rows, 
     put(what, 2); put(rows, 4); put(m->store_logits != 0, 1); put(m->draft_chain, 1); put(m->fuse_rows, 1); put(m->attn_rows, 1); put(m->attn_rows_fq, 1);
     put(m->head_mfma, 1); put(m->down_kq, 1); put(m->xcd_ffn, 1); put(m->fork_ple, 1); put(m->rows_geglu, 1); put(m->tail_stamps != 0, 1);
     put(m->tail_spread == 1 ? 1 : m->tail_spread ? 2 : 0, 2); put(m->xcd_tail, 2); put(m->down_m, 2); put(m->xcd_attn_tail, 2); put(m->merge_o, 2);
-    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->tail_qkv, 1); put(m->attn_geglu, 1); put(m->wait_polls, 17); put(may_wait(m), 1);
+    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->tail_qkv, 1); put(m->attn_geglu, 1); put(m->mid, 1); put(m->wait_polls, 17); put(may_wait(m), 1);
     return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices, 0 };
 }
 
@@ -2109,6 +2195,7 @@ extern "C" int lg_hip_set_option(lg_hip_model *m, const char *name, int value) {
     else if (!strcmp(name, "rows_geglu")) m->rows_geglu = value != 0;
     else if (!strcmp(name, "narrow")) m->narrow = value != 0;
     else if (!strcmp(name, "attn_out")) m->attn_out = value != 0;
+    else if (!strcmp(name, "mid")) m->mid = value != 0;
     else if (!strcmp(name, "tail_qkv")) m->tail_qkv = value != 0;
     else if (!strcmp(name, "attn_geglu")) m->attn_geglu = value != 0;
     else if (!strcmp(name, "down_kq")) m->down_kq = value != 0;
@@ -2454,7 +2541,7 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
     const bool narrow = use_narrow(m, rows);              // (everything but the attention and the first layer's projections)
     for (int L = 0; L < m->n_layer; ++L) {
         const Layer &y = m->L[L];
-        b[L && (narrow || (!y.winp_f && use_ple_tail(m, rows) && tail_does_qkv(m, rows, y))) ? KC_TAIL : KC_QKV] += (double)m->E * y.qkv_m * q;
+        b[L && (narrow || (!y.winp_f && use_ple_tail(m, rows) && tail_does_qkv(m, rows, y))) ? KC_TAIL : L && !narrow && (use_mid_down(m, m->L[L - 1], y, rows) || (y.winp_f && use_mid_proj(m, y))) ? KC_ROWS : KC_QKV] += (double)m->E * y.qkv_m * q;
         if (narrow) b[KC_TAIL] += ((double)y.qd * m->E + 3.0 * m->E * y.nff + 2.0 * m->E * m->ple) * q;
         else {
         {
@@ -2464,16 +2551,15 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
         }
         const int tiles = step_tiles(m, kv, y, rows, 0);
         if (m->xffn_built && m->xcd_ffn && may_wait(m) && rows >= 4) b[KC_FFN] += 3.0 * m->E * y.nff * q;
-        else { b[use_attn_out(m, y, rows, tiles) && attn_out_geglu(m, y, rows, tiles) ? KC_ATAIL : KC_GATEUP] += 2.0 * m->E * y.nff * q; b[KC_DOWN] += (double)y.nff * m->E * q; }
+        else { b[use_attn_out(m, y, rows, tiles) ? attn_out_geglu(m, y, rows, tiles) ? KC_ATAIL : KC_GATEUP : use_mid_o(m, y, rows) ? KC_O : KC_GATEUP] += 2.0 * m->E * y.nff * q; b[L + 1 < m->n_layer && use_mid_down(m, y, m->L[L + 1], rows) ? KC_ROWS : KC_DOWN] += (double)y.nff * m->E * q; }
         if (m->ple && !y.winp_f && use_ple_tail(m, rows)) b[KC_TAIL] += 2.0 * m->E * m->ple * q;
-        else if (m->ple) { const double pq = y.winp_f ? 4.0 : q; b[KC_PLEGATE] += (double)m->E * m->ple * pq; b[KC_PLEPROJ] += (double)m->ple * m->E * pq; }
+        else if (m->ple) { const double pq = y.winp_f ? 4.0 : q; b[KC_PLEGATE] += (double)m->E * m->ple * pq; b[L + 1 < m->n_layer && y.winp_f && use_mid_proj(m, m->L[L + 1]) ? KC_ROWS : KC_PLEPROJ] += (double)m->ple * m->E * pq; }
         }
         const int window = (y.is_local && m->window > 0) ? m->window : 0;
         const int last = pos + rows - 1, start = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
         b[KC_ATTN] += 2.0 * (last - start + 1) * y.kd * 2.0;          // K and V rows, f16
     }
     b[KC_HEAD] = (double)m->E * m->n_vocab * q;
-    b[KC_ROWS] = 0;
 }
 
 extern "C" int lg_hip_profile_step(lg_hip_model *m, lg_hip_kv *kv, const int32_t *toks, int rows, int pos, int repeats,

@@ -102,8 +102,8 @@ __host__ __device__ static inline constexpr int lg_far_slot(int j) { return (j &
 // Wavefront `wave`'s K segment (nit blocks of 32, at most NIT) of M rows of k values, into the blocks at la.  A lane's units are the same of every row
 // that it takes (two at a time, where a half of the wavefront holds a row's units), so that nothing is left to compute when they arrive; what is past the rows
 // or the segment is its last once more.
-template <int M, int NIT>
-__device__ __forceinline__ int lg_take_far_segment(const FarRows *f, int k, int nit, int wave, int lane, unsigned char *la, uint32_t tag, int spin_limit) {
+template <int M, int NIT, typename B>
+__device__ __forceinline__ int lg_take_far_segment(const FarRows *f, int k, int nit, int wave, int lane, unsigned char *la, uint32_t tag, int spin_limit, B &&behind) {
     constexpr int H = 3 * NIT <= 32 ? 2 : 1, N = (M + H - 1) / H;                // rows of a trip, trips
     const int h = H == 2 ? lane >> 5 : 0, x = H == 2 ? lane & 31 : lane, w = x < 3 * nit ? x : 3 * nit - 1, b = w / 3, e = w - 3 * b, nb = k >> 5;
     auto pos = [](int m) { return (m & 1) | ((m & 2) << 1) | ((m & 4) >> 1); };
@@ -114,18 +114,23 @@ __device__ __forceinline__ int lg_take_far_segment(const FarRows *f, int k, int 
     const int at = (wave * nit * 3 + w) * 16, row = nb * 48;
     lg_x4u v[N];
     int err = 0;
-    for (int spins = 0;; ++spins) {
-        uint32_t diff = 0;
+    auto load = [&] {
         #pragma unroll
         for (int i = 0; i < N; ++i) {
             const int j = H * i + h < M ? H * i + h : M - 1;   // (a lane's own only where the last trip has one row)
             v[i] = __builtin_bit_cast(lg_x4u, __builtin_amdgcn_raw_buffer_load_b128(r, at + j * row, 0, 16));
         }
+    };
+    load();
+    behind();                                                  // (further requests, behind the first load of the rows)
+    for (int spins = 0;; ++spins) {
+        uint32_t diff = 0;
         #pragma unroll
         for (int i = 0; i < N; ++i) diff |= v[i].x ^ v[i].y ^ v[i].z ^ v[i].w ^ tag;
         if (__all(diff == 0)) break;
         if (spins >= spin_limit) { err = LG_XFFN_ERR_WAIT; break; }
         asm volatile("" ::: "memory");
+        load();
     }
     #pragma unroll
     for (int i = 0; i < N; ++i) {                              // (row H i + h: slot 4 h + i, or lg_far_slot(i))
@@ -133,6 +138,10 @@ __device__ __forceinline__ int lg_take_far_segment(const FarRows *f, int k, int 
         s0[z * 8] = v[i].x; s1[z * 8] = v[i].y; s2[z * st] = v[i].z;
     }
     return err;
+}
+template <int M, int NIT>
+__device__ __forceinline__ int lg_take_far_segment(const FarRows *f, int k, int nit, int wave, int lane, unsigned char *la, uint32_t tag, int spin_limit) {
+    return lg_take_far_segment<M, NIT>(f, k, nit, wave, lane, la, tag, spin_limit, [] {});
 }
 // Weights as the high nibbles of bytes, two's complement: their product with values is 16 times the dot, which the accumulators' start, the bits of 1.5 * 2^19,
 // turns into 786432 + dot, exactly

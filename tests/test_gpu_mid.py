@@ -1,0 +1,78 @@
+"""A product, the row work behind it and the next product as one launch (lg_k_o_geglu, lg_k_down_qkv; option mid) against the separate kernels."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ALL = tuple(range(1, 9))
+
+
+# attn_output inputs of 4 to 16 blocks a segment, rows of 3 to 15, one and two column blocks to a workgroup; ffn_down's segments of 5 to 15 blocks
+@pytest.mark.parametrize("over,o,down", [
+    (dict(n_embd=768, n_head=16, n_ff=5120), ALL, (1, 2, 3)),                                        # (streams of ffn_down's matrix-core form: rows past 2048 values)
+    (dict(n_embd=1280, n_head=8, head_dim=128, n_ff=8192, n_head_kv=4), ALL, (1, 2, 3)),
+    (dict(n_embd=2304, n_head=12, head_dim=256, n_ff=5120), ALL, ALL),
+    (dict(n_embd=2560, n_head=16, head_dim=64, n_ff=10240, out_scale=0.9), ALL, ALL),
+    (dict(n_embd=3072, n_head=16, head_dim=256, n_head_kv=8, n_ff=15360), ALL, ALL),
+    (dict(n_embd=3840, n_head=16, head_dim=256, n_head_kv=8, n_ff=15360), ALL, ALL),
+    (dict(n_embd=3840, n_head=4, head_dim=256, n_ff=512), ALL, ()),                                 # 16 column blocks: most workgroups without one; ffn_down of 8 segments
+    (dict(n_embd=2560, n_head=20, n_head_kv=4, head_dim=256, n_ff=512), (), ())])                                # an input too wide
+def test_one_launch_equals_the_separate_kernels(lg, gpu_required, model_path, over, o, down):
+    """Every width: logits, hidden state and cache rows of steps in a row, bit for bit; and the launches say which form ran."""
+    path, spec = model_path("tiny", **dict(dict(n_layer=3, n_vocab=2048, sliding_window=64), **over))
+    rng = np.random.default_rng(spec["n_embd"] + spec["n_ff"])
+    prompt, toks = rng.integers(1, spec["n_vocab"], 90).astype(np.int32), rng.integers(1, spec["n_vocab"], 40).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, 2000, max_rows=8)
+    try:
+        gpu.set_option("store_logits", 1)
+        got = []
+        for on in (1, 0):
+            gpu.new_cache()
+            gpu.set_option("mid", on)
+            gpu.prefill(prompt, 0)
+            res, pos = [], len(prompt)
+            for rows in (1, 2, 3, 4, 5, 6, 7, 8, 1):
+                print(f"{over} at {pos}, {rows} rows, mid {on}", flush=True)
+                gpu.forward_spec(toks[pos - 90:pos - 90 + rows], pos)
+                res += [gpu.logits_row(j, spec["n_vocab"]) for j in range(rows)] + [gpu.last_hidden(spec["n_embd"])]
+                pos += rows
+            res += [gpu.kv_read(L, w) for L in range(3) for w in (0, 1)]
+            got.append([np.ascontiguousarray(r).view(np.uint8) for r in res])
+            for rows in ALL:
+                n = {k["name"]: k["launches"] for k in gpu.profile_step(toks[:rows], 90, 1)}
+                assert (n.get("gate_up_geglu", 0) == 0) == bool(on and rows in o), (rows, on, n)
+                assert n["qkv"] == (1 if on and rows in down else 3), (rows, on, n)
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
+    finally:
+        gpu.close()
+
+
+@pytest.mark.parametrize("name,over", [("tiny_full_bf16", dict(n_embd=768)), ("tiny_full_f32", dict(n_embd=2560, n_head=8, head_dim=256, head_dim_full=256, n_head_kv=2)),
+                                       ("tiny_full_f16", dict(n_embd=3840, n_head=16, head_dim=256, head_dim_full=256, n_head_kv=4))])
+def test_per_layer_projection_of_a_float_type(lg, gpu_required, model_path, name, over):
+    """The same launch with that projection as its first product: 3, 10 and 15 of its rows to a workgroup, shared-cache layers (queries only) and others behind it."""
+    path, spec = model_path(name, **dict(dict(n_layer=4, n_ff=512, n_vocab=2048), **over))
+    rng = np.random.default_rng(spec["n_embd"])
+    prompt, toks = rng.integers(1, spec["n_vocab"], 90).astype(np.int32), rng.integers(1, spec["n_vocab"], 40).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, 400, max_rows=8)
+    try:
+        gpu.set_option("store_logits", 1)
+        got = []
+        for on in (1, 0):
+            gpu.new_cache()
+            gpu.set_option("mid", on)
+            gpu.prefill(prompt, 0)
+            res, pos = [], len(prompt)
+            for rows in (1, 2, 3, 4, 5, 6, 7, 8, 1):
+                print(f"{name} {over} at {pos}, {rows} rows, mid {on}", flush=True)
+                gpu.forward_spec(toks[pos - 90:pos - 90 + rows], pos)
+                res += [gpu.logits_row(j, spec["n_vocab"]) for j in range(rows)] + [gpu.last_hidden(spec["n_embd"])]
+                pos += rows
+            res += [gpu.kv_read(L, w) for L in range(2) for w in (0, 1)]
+            got.append([np.ascontiguousarray(r).view(np.uint8) for r in res])
+            for rows in ALL:
+                n = {k["name"]: k["launches"] for k in gpu.profile_step(toks[:rows], 90, 1)}
+                assert n["qkv"] == (1 if on else 4), (rows, on, n)
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
+    finally:
+        gpu.close()
