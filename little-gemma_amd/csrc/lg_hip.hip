@@ -263,7 +263,7 @@ struct lg_hip_model {
     XtailSync *tsync = nullptr;
     uint2 *tgf = nullptr, *tpr = nullptr;    // [LG_HIP_MAX_ROWS][ple] and [LG_HIP_MAX_ROWS][E] its gated values and projections, tagged
     uint2 *mido = nullptr, *midd = nullptr, *mids = nullptr;   // [max rows][E] the first products of lg_k_o_geglu and lg_k_down_qkv, [3][max rows][E] slabs of the latter, tagged (option mid)
-    FarRows *midro = nullptr, *midrd = nullptr;                // their rows
+    FarRows *midro = nullptr, *midrd = nullptr, *midao = nullptr;                // their rows
     FarRows *trows = nullptr;                // rows of lg_k_ple_tail_s on their way to the next layer's projections (option tail_qkv)
     FarRows *aorows = nullptr;               // rows of lg_k_attn_out on their way to gate/up (option attn_geglu)
     AttnOutSync *aosync = nullptr;           // hand-over state of lg_k_attn_out (models it serves)
@@ -919,7 +919,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         if (getenv("LG_HIP_XCD_TAIL")) m->xcd_tail = atoi(getenv("LG_HIP_XCD_TAIL"));
     }
     if (mid_model(m) && (mark_alloc(m, &m->mido, (size_t)LG_HIP_MAX_ROWS * E) || mark_alloc(m, &m->midd, (size_t)LG_HIP_MAX_ROWS * E) || mark_alloc(m, &m->mids, (size_t)3 * LG_HIP_MAX_ROWS * E) ||
-                         mark_alloc(m, &m->midro) || mark_alloc(m, &m->midrd))) return -7;
+                         mark_alloc(m, &m->midro) || mark_alloc(m, &m->midao) || mark_alloc(m, &m->midrd))) return -7;
     if (narrow_shape(m)) {
         if (mark_alloc(m, &m->nsync)) return -7;
     } else if (!m->target && cu_count() == LG_XCDS * LG_XCD_WGS) {
@@ -1400,6 +1400,11 @@ static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int t
 static bool use_mid_o(const lg_hip_model *m, const Layer &y, int rows) {
     return m->mid && m->attn_out && m->mido && may_wait(m) && y.wo_pc && y.wgu && !(rows >= 4 && (m->rows_geglu || (m->xcd_ffn && y.xgu)));
 }
+// ... and the merge of attention's partials: up to LG_MID_MERGE_ROWS rows (more: no gain, see lg_k_o_geglu) of up to LG_AOUT_TILES tiles, which a wavefront holds in
+// registers.  (Rows of up to 2560 values have lg_k_attn_out.)
+static bool use_mid_merge(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
+    return rows <= LG_MID_MERGE_ROWS && use_mid_o(m, y, rows) && m->E > 2560 && tiles <= LG_AOUT_TILES && y.hd % 64 == 0;
+}
 // ffn_down, row work and the next layer's q/k/v projections as one launch (1 to 3 rows: with the whole rows in LDS)
 static bool use_mid_down(const lg_hip_model *m, const Layer &y, const Layer &next, int rows) {
     if (!m->mid || !m->midd || !may_wait(m) || m->ple || !next.wqkv_pc) return false;
@@ -1651,6 +1656,9 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         const Layer &y = m->L[L];
         const int window = (y.is_local && m->window > 0) ? m->window + pos_off : 0;
         bool fused_post = false, merged_o = false, ffn_rows_done = false, gate_up_done = false;
+        bool mid_merge = false;                                // the merge is left to lg_k_o_geglu, with these
+        MergeArgs mg{};
+        int mg_tiles = 0;
         {   // q/k/v projections, then per-head norm, rotary and the K/V rows of this block
             MmArgs a{ y.wqkv, E, y.qkv_m, m->qkv, m->hq, nullptr };
             if (qkv_done) { qkv_done = rows_done = false; }
@@ -1775,6 +1783,10 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 launch_merge_o(lx, f);
                 pend_dout = m->dout; pend_w = y.post_attn; pend_os = nullptr; pend_parts = 8;
             } else
+            if ((mid_merge = pos_off == 0 && have_x && use_mid_merge(m, y, M, tiles))) {
+                mg = g;
+                mg_tiles = tiles;
+            } else
             if (tiles >= 128 && y.hd % 64 == 0) {
 #define GO(k, grid, block) LAUNCH(KC_MERGE, k, grid, block, 0, m->ctl, LG_MERGE_FIELDS(LG_XA, g) 0)
                 MERGE_SPLIT(M, GO, H, y.hd, tiles);
@@ -1786,8 +1798,11 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             f.ow = y.wo_pc; f.act = m->aq; f.out = m->mido; f.gw = y.wgu; f.gq = m->gq; f.qd = y.qd; f.nff = y.nff;
             f.gq_units = M >= 4 && m->down_m && y.wdn_m ? 2 : 0; f.seq = L;
             f.r = MidRowArgs{ m->x[cur], y.post_attn, nullptr, y.ffn_norm, m->x[cur ^ 1], nullptr, m->midro, E, m->wait_polls, m->eps };
-            if (E <= 2560) LAUNCH(KC_O, (lg_k_o_geglu<M, 10>), dim3(LG_XCDS * LG_XCD_WGS), dim3(512), LG_OG_LDS(10), m->ctl, LG_OGEGLU_FIELDS(LG_XA, f) 0);
-            else           LAUNCH(KC_O, (lg_k_o_geglu<M, 15>), dim3(LG_XCDS * LG_XCD_WGS), dim3(512), LG_OG_LDS(15), m->ctl, LG_OGEGLU_FIELDS(LG_XA, f) 0);
+            f.g = mg; f.tiles = mg_tiles; f.arows = m->midao;
+            if constexpr (M <= LG_MID_MERGE_ROWS)
+                if (mid_merge) LAUNCH(KC_O, (lg_k_o_geglu<M, 15, true>), dim3(LG_XCDS * LG_XCD_WGS), dim3(512), LG_OG_LDS(15), m->ctl, LG_OGEGLU_FIELDS(LG_XA, f) 0);
+            if (E <= 2560)       LAUNCH(KC_O, (lg_k_o_geglu<M, 10, false>), dim3(LG_XCDS * LG_XCD_WGS), dim3(512), LG_OG_LDS(10), m->ctl, LG_OGEGLU_FIELDS(LG_XA, f) 0);
+            else if (!mid_merge) LAUNCH(KC_O, (lg_k_o_geglu<M, 15, false>), dim3(LG_XCDS * LG_XCD_WGS), dim3(512), LG_OG_LDS(15), m->ctl, LG_OGEGLU_FIELDS(LG_XA, f) 0);
             cur ^= 1;
             merged_o = true; ffn_rows_done = true; gate_up_done = true;
         }

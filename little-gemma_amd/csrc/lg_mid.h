@@ -19,6 +19,7 @@
 
 #define LG_MID_E 3840               // widest row
 #define LG_MID_K 4096               // widest input of attn_output
+#define LG_MID_MERGE_ROWS 3         // widest block whose merge is part of lg_k_o_geglu
 // Chains of pairs of K segments (host: pack_pairs): block of 16 rows, pair of segments, pairs of blocks of 32: 64 lanes x (8 + 8) nibble bytes of two blocks, signed (lane:
 // row c16, half hf of its 16 bytes, segment sg of the pair), then 32 (segment, row) x two f16 scales
 __host__ __device__ static inline size_t lg_pairs_bytes(int k, int m) { const int nit = k / 256, nitp = (nit + 1) & ~1; return (size_t)m / 16 * 4 * nitp * 576; }
@@ -375,10 +376,15 @@ struct OGegluArgs {
     const uint8_t *gw;              // row-block tiles
     int8_t        *gq;
     int            qd, nff, gq_units, seq;
+    MergeArgs      g;               // MG: attention's partials (xq, xf are not used),
+    FarRows       *arows;           // the rows they become
+    int            tiles;           // and the most tiles that a row can see
 };
 #define LG_OGEGLU_FIELDS(X, v) X(const int8_t *, act, act, v) X(const uint8_t *, ow, ow, v) X(int, qd, qd, v) X(int, E, r.E, v) X(const uint8_t *, gw, gw, v) X(int, nff, nff, v) X(int, seq, seq, v) \
     X(uint2 *, out, out, v) X(const float *, x, r.x, v) X(const float *, w_post, r.w_post, v) X(const float *, os, r.os, v) X(const float *, w_pre, r.w_pre, v) X(float *, x_out, r.x_out, v) \
-    X(FarRows *, rows, r.rows, v) X(float, eps, r.eps, v) X(int, spin_limit, r.spin_limit, v) X(int8_t *, gq, gq, v) X(int, gq_units, gq_units, v)
+    X(FarRows *, rows, r.rows, v) X(float, eps, r.eps, v) X(int, spin_limit, r.spin_limit, v) X(int8_t *, gq, gq, v) X(int, gq_units, gq_units, v) \
+    X(const float *, pm, g.pm, v) X(const float *, pl, g.pl, v) X(const float *, pacc, g.pacc, v) X(int, tiles_max, g.tiles_max, v) X(int, H, g.H, v) X(int, hd, g.hd, v) \
+    X(int, window, g.window, v) X(FarRows *, arows, arows, v) X(int, tiles, tiles, v)
 #define LG_OG_AHEAD 3                // ... of the column block that comes first: ahead of attn_output's products
 #define LG_OG_EARLY 5               // blocks of the first column block's tiles that are requested ahead of the rows
 #define LG_OG_LT 12                 // blocks of a segment of the second column block that wait in LDS (the others in registers)
@@ -386,7 +392,11 @@ struct OGegluArgs {
 #define LG_OG_LDS(NIT) (LG_OG_ACT(NIT) + (size_t)8 * ((NIT) < LG_OG_LT ? (NIT) : LG_OG_LT) * LG_TILE + 8192)
 #define LG_OG_BLOCKS (2 * LG_XCDS * LG_XCD_WGS - 32)      // two blocks of 32 FFN columns for each workgroup, one for the row units (8 rows x 4 slices)
 static_assert((size_t)9 * 16 * LG_FAR_BLK >= 2 * 8 * 8 * 64 * 4, "the sums of two column blocks take the rows' place");
-template <int M, int NIT>
+// MG (up to LG_MID_MERGE_ROWS rows): the merge of attention's partials (lg_k_attn_merge) is part of the launch too, 64 dims of a row by a wavefront, a workgroup
+// each; the q8 is handed over as the rows are.  12B shape at 3001, one to five rows, us a step: 2322 -> 2245, 2495 -> 2413, 2635 -> 2565, 2715 -> 2704, 2855 -> 2855
+// (the launch 18.0 -> 20.4 at one row, the 4.3 of the merge and its gap gone; 20.6 -> 24.4 at five, where 256 workgroups pull 31 KB of q8 each and a merge takes 4.9).
+// One row: gate/up's first tiles requested ahead of the q8 2276, `soon` put behind the q8 2255.
+template <int M, int NIT, bool MG>
 __global__ __launch_bounds__(512) void lg_k_o_geglu(StepCtl *ctl, LG_OGEGLU_FIELDS(LG_XP, _) int p_end_) {
     constexpr int BLK = LG_FAR_BLK, I = (M + 1) / 2, LT = NIT < LG_OG_LT ? NIT : LG_OG_LT;
     OGegluArgs a; LG_OGEGLU_FIELDS(LG_XI, a)
@@ -402,6 +412,12 @@ __global__ __launch_bounds__(512) void lg_k_o_geglu(StepCtl *ctl, LG_OGEGLU_FIEL
     const bool unit = u < M * slices, rowt = unit && t < 256;
     const int K = a.qd, na = K >> 8, nh = na >> 1, nbk = K >> 5;          // blocks of a segment, of half of it (even)
     const int j0 = u % M, vr = u / M;
+    const int mrow = K >> 6, mj = (int)blockIdx.x / mrow, mu = (int)blockIdx.x - mj * mrow;
+    const bool merges = MG && wave == 0 && (int)blockIdx.x < M * mrow;
+    AoutMerge<LG_AOUT_TILES> part[1];
+    AttnOutArgs ma;
+    ma.g = a.g; ma.tiles = a.tiles;
+    if (merges) part[0].request(ma, mu, mj, lane);
     MidRow row;
     if (rowt) row.request(a.r, j0, t);
     const int rb = min((int)blockIdx.x, (E >> 4) - 1);         // (workgroups without a share take the last one once more: no conditions, see lg_k_down_qkv)
@@ -409,10 +425,12 @@ __global__ __launch_bounds__(512) void lg_k_o_geglu(StepCtl *ctl, LG_OGEGLU_FIEL
     uint4 au[NU]; float as[NS];
     lg_x4u ow[4]; uint32_t os[4];
     {
-        #pragma unroll
-        for (int i = 0; i < NU; ++i) au[i] = ((const uint4 *)a.act)[min(t + 512 * i, M * (K >> 4) - 1)];
-        #pragma unroll
-        for (int i = 0; i < NS; ++i) as[i] = lg_q8_ds<M>(a.act, K)[min(t + 512 * i, M * nbk - 1)].x;
+        if constexpr (!MG) {
+            #pragma unroll
+            for (int i = 0; i < NU; ++i) au[i] = ((const uint4 *)a.act)[min(t + 512 * i, M * (K >> 4) - 1)];
+            #pragma unroll
+            for (int i = 0; i < NS; ++i) as[i] = lg_q8_ds<M>(a.act, K)[min(t + 512 * i, M * nbk - 1)].x;
+        }
         const uint8_t *cb = a.ow + ((size_t)rb * 4 + sp) * na * 576;
         #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -447,16 +465,30 @@ __global__ __launch_bounds__(512) void lg_k_o_geglu(StepCtl *ctl, LG_OGEGLU_FIEL
     {
         unsigned char *zero = smem + (size_t)8 * 16 * BLK;
         for (int i = t; i < 8 * BLK / 16; i += 512) ((uint4 *)zero)[i] = make_uint4(0, 0, 0, 0);
-        #pragma unroll
-        for (int i = 0; i < NU; ++i) {                         // (what is past the rows is their last unit once more)
-            const int at = min(t + 512 * i, M * (K >> 4) - 1), j = at / (K >> 4), p = at - j * (K >> 4);
-            unsigned char *o = smem + (size_t)((p & 7) * 16 + (p >> 4)) * BLK + lg_far_slot(j) * 32 + ((p >> 3) & 1) * 8;
-            *(uint2 *)o = make_uint2(au[i].x, au[i].y); *(uint2 *)(o + 16) = make_uint2(au[i].z, au[i].w);
-        }
-        #pragma unroll
-        for (int i = 0; i < NS; ++i) {
-            const int at = min(t + 512 * i, M * nbk - 1), j = at / nbk, p = at - j * nbk;
-            *(float *)(smem + (size_t)((p & 7) * 16 + (p >> 3)) * BLK + 256 + lg_far_slot(j) * 4) = as[i];
+        if constexpr (MG) {
+            if (merges) {
+                float v[1], d;
+                int sum;
+                lg_aout_merge(part, ma, ctl->pos, mj, lane, v);
+                asm volatile("" : "+v"(v[0]));
+                if (blockIdx.x == 0 && lane == 0) lg_put_soon(a.arows, tag);
+                lg_put_far_dims(a.arows, K, mj, mu, lane, lg_quant1_32lanes(v[0], &d, &sum), d, tag);
+            }
+            int err = lg_wait_soon(a.arows, tag, a.r.spin_limit);
+            err |= lg_take_far_segment<M, 16>(a.arows, K, na, wave, lane, smem + (size_t)wave * 16 * BLK, tag, a.r.spin_limit);
+            if (err) atomicOr(&ctl->err, err);
+        } else {
+            #pragma unroll
+            for (int i = 0; i < NU; ++i) {                     // (what is past the rows is their last unit once more)
+                const int at = min(t + 512 * i, M * (K >> 4) - 1), j = at / (K >> 4), p = at - j * (K >> 4);
+                unsigned char *o = smem + (size_t)((p & 7) * 16 + (p >> 4)) * BLK + lg_far_slot(j) * 32 + ((p >> 3) & 1) * 8;
+                *(uint2 *)o = make_uint2(au[i].x, au[i].y); *(uint2 *)(o + 16) = make_uint2(au[i].z, au[i].w);
+            }
+            #pragma unroll
+            for (int i = 0; i < NS; ++i) {
+                const int at = min(t + 512 * i, M * nbk - 1), j = at / nbk, p = at - j * nbk;
+                *(float *)(smem + (size_t)((p & 7) * 16 + (p >> 3)) * BLK + 256 + lg_far_slot(j) * 4) = as[i];
+            }
         }
         __syncthreads();
         #pragma unroll

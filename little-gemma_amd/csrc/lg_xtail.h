@@ -64,6 +64,15 @@ __device__ __forceinline__ void lg_put_far_q8(FarRows *f, int k, int j, int quad
     lg_x4u v; v.x = packed; v.y = b; v.z = z; v.w = tag ^ packed ^ b ^ z;
     __builtin_amdgcn_raw_buffer_store_b128(v, r, ((j * (k >> 5) + (quad >> 3)) * 3 + dw / 3) * 16, 0, 16);      // (16: the scope bit sc1)
 }
+// 64 values of row j (dims 64 u + lane) as q8 q, d their block's scale
+__device__ __forceinline__ void lg_put_far_dims(FarRows *f, int k, int j, int u, int lane, int q, float d, uint32_t tag) {
+    const uint32_t word = (uint32_t)(lg_dpp_i<0x00>(q) & 255) | (uint32_t)(lg_dpp_i<0x55>(q) & 255) << 8 | (uint32_t)(lg_dpp_i<0xAA>(q) & 255) << 16 | (uint32_t)lg_dpp_i<0xFF>(q) << 24;
+    const int l = lane < 6 ? lane : 5, b = l / 3, e = l - 3 * b, at = b * 32 + e * 12;          // lanes 0 .. 5 store a unit each
+    const uint32_t x = __shfl(word, at), y = __shfl(word, at + 4), w = __shfl(word, e < 2 ? at + 8 : at), s = __float_as_uint(__shfl(d, at)), z = e < 2 ? w : s;
+    const __amdgpu_buffer_rsrc_t r = lg_buffer_rsrc(f->u);
+    lg_x4u v; v.x = x; v.y = y; v.z = z; v.w = tag ^ x ^ y ^ z;
+    if (lane < 6) __builtin_amdgcn_raw_buffer_store_b128(v, r, ((j * (k >> 5) + 2 * u + b) * 3 + e) * 16, 0, 16);
+}
 // Wait until the rows are on their way (one load per wavefront and trip: workgroups that load the rows all the time keep the memory from the ones that make them)
 __device__ __forceinline__ int lg_wait_soon(const FarRows *f, uint32_t tag, int spin_limit) {
     for (int spins = 0;; ++spins) {

@@ -76,3 +76,40 @@ def test_per_layer_projection_of_a_float_type(lg, gpu_required, model_path, name
         assert all(np.array_equal(a, b) for a, b in zip(*got))
     finally:
         gpu.close()
+
+
+@pytest.mark.parametrize("over,pos0,cache,merges", [
+    (dict(n_embd=3840, n_head=16, head_dim=256, n_head_kv=8, sliding_window=1024), 3001, 3100, 1), (dict(n_embd=3072, n_head=16, head_dim=128, n_head_kv=4, sliding_window=608), 639, 700, 0),
+    (dict(n_embd=2816, n_head=16, head_dim=64, sliding_window=1184), 1200, 1214, 0), (dict(n_embd=2816, n_head=32, head_dim=64, n_head_kv=4, sliding_window=1312), 2400, 2500, 2),
+    (dict(n_embd=3840, n_head=4, head_dim=256), 0, 64, 0)])
+def test_merge_inside_the_launch(lg, gpu_required, model_path, over, pos0, cache, merges):
+    """Attention's partials merged by lg_k_o_geglu (1 to 3 rows): contexts of one tile, windows at and past the tiles of the first batch (20) and of all (40), global layers of more
+    tiles beside them; against the separate kernels, bit for bit.  The cache rows in front are drawn.  merges: layers of more tiles than that, which keep their own."""
+    path, spec = model_path("tiny", **dict(dict(n_layer=2, n_ff=512, n_vocab=2048), **over))
+    rng = np.random.default_rng(pos0)
+    gpu = lg.hiplib.HipBackend(path, cache, max_rows=8)
+    try:
+        gpu.set_option("store_logits", 1)
+        front = [rng.normal(0, 0.5, (2,) + gpu.kv_layout(L)).astype(np.float16).view(np.uint16) for L in range(2)]
+        toks = rng.integers(1, spec["n_vocab"], 20).astype(np.int32)
+        got = []
+        for on in (1, 0):
+            gpu.new_cache()
+            gpu.set_option("mid", on)
+            for L in range(2):
+                for which in (0, 1):
+                    gpu.kv_write(L, which, front[L][which])
+            res, pos = [], pos0
+            for rows in (1, 2, 3, 4, 1):
+                print(f"{over} at {pos}, {rows} rows, mid {on}", flush=True)
+                gpu.forward_spec(toks[pos - pos0:pos - pos0 + rows], pos)
+                res += [gpu.logits_row(j, spec["n_vocab"]) for j in range(rows)] + [gpu.last_hidden(spec["n_embd"])]
+                pos += rows
+            res += [gpu.kv_read(L, w) for L in range(2) for w in (0, 1)]
+            got.append([np.ascontiguousarray(r).view(np.uint8) for r in res])
+            for rows in (1, 2, 3, 4):
+                n = {k["name"]: k["launches"] for k in gpu.profile_step(toks[:rows], pos0, 1)}
+                assert n.get("attn_merge", 0) == (merges if on and rows < 4 else 2), (rows, on, n)
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
+    finally:
+        gpu.close()
