@@ -29,11 +29,11 @@ HBM_PEAK_GBS = 8000.0
 FLOOR_LAUNCH_US = 1.55          # a dependent kernel boundary inside a captured graph on this part (bench.py --launch-floor)
 FLOOR_STREAM_GBS = 6000.0       # what a plain streaming kernel sustains from HBM here
 i32a = np.ctypeslib.ndpointer(np.int32, flags="C_CONTIGUOUS")
-# HBM bytes per launch of the dominant kernel (gate/up + GeGLU at the E4B shape), from the FETCH_SIZE and
-# WRITE_SIZE counter runs summarised in the file named below (scaled by the copy-kernel calibration given
-# there): reads 29.40 MB for M = 5 (29.27 MB for M = 1), writes 0.15 MB (0.03 MB).  Counters cannot be read
+# HBM bytes per launch of the dominant kernel (at the E4B shape the launch of attention merge, attn_output, row work, gate/up
+# and GeGLU), from the FETCH_SIZE and WRITE_SIZE counter runs summarised in the file named below (scaled by the copy-kernel
+# calibration given there): reads 33.5 MB for M = 5 (32.5 MB for M = 1), writes 0.27 MB (0.07 MB).  Counters cannot be read
 # from inside this process, so the figure is quoted with its source; shapes without a counter run report null.
-MEASURED_TRAFFIC = {("e4b", "gate_up_geglu", 5): 29.41e6 + 0.07e6, ("e4b", "gate_up_geglu", 1): 29.27e6 + 0.03e6}
+MEASURED_TRAFFIC = {("e4b", "attn_tail", 5): 33.53e6 + 0.27e6, ("e4b", "attn_tail", 1): 32.51e6 + 0.07e6}
 TRAFFIC_SOURCE = "profiles/verify_step_e4b_rows5_hbm_counters.md"
 CTX = 2048
 WORKLOADS = {
@@ -343,8 +343,8 @@ def main():
     # per-kernel-class device time of one step (un-captured, start/stop events filled in by each launch)
     prof = gpu.profile_step(blocks[0], ctx, repeats=10)
     step_bytes = sum(c["bytes"] for c in prof)
-    # the roofline kernel: the class that moves the most bytes per step (gate/up + GeGLU: 47% of them at the E4B
-    # shape).  By device time several classes of a layer are within 10% of it (kernel_classes lists them all).
+    # the roofline kernel: the class that moves the most bytes per step (attn_output and gate/up of the sliding layers: 43% of
+    # them at the E4B shape).  By device time several classes of a layer are within 10% of it (kernel_classes lists them all).
     dom = max((c for c in prof if c["bytes"] > 0 and c["launches"] > 1), key=lambda c: c["bytes"])
     dom_gbs = dom["bytes"] / (dom["ms"] * 1e-3) / 1e9
     roofline = {"bound": "hbm", "kernel": dom["name"], "achieved": dom_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
@@ -364,16 +364,19 @@ def main():
         c["over_floor"] = (c["ms"] * 1e3 / c["floor_us"]) if c["floor_us"] > 0 else None
     floor_ms = sum(c["floor_us"] for c in prof) * 1e-3
     uncaptured_ms = sum(c["ms"] for c in prof)
-    # matrix-core utilisation of the verify step's one MFMA GEMM (gate/up for blocks of 4..8 rows): the weights of a
-    # launch (bytes / 0.5625 elements) times the block's rows are the useful MACs, the 8 row slots of the tiles the
-    # issued ones.  It is a bandwidth-bound kernel: the figure says how far the matrix cores are from mattering.
+    # matrix-core utilisation of the verify step's largest MFMA GEMM (gate/up for blocks of 4..8 rows, a launch of its own or, with
+    # attn_output, part of one): the weights of a launch (bytes / 0.5625 elements) times the block's rows are the useful MACs, the
+    # row slots of a product (8 of a launch of its own, 16 with half of them zeros in the other) the issued ones.  It is a
+    # bandwidth-bound kernel: the figure says how far the matrix cores are from mattering.
     mfma = None
-    gu = next((c for c in prof if c["name"] == "gate_up_geglu" and c["launches"] > 0), None)
+    gu = next((c for name in ("gate_up_geglu", "attn_tail", "attn_output") for c in prof if c["name"] == name and c["launches"] > 0 and c["bytes"] > 0), None)
     if gu and 4 <= a.rows <= 8:
         w_elems = gu["bytes"] / gu["launches"] / (18.0 / 32.0)
         sec = gu["ms"] / gu["launches"] * 1e-3
-        mfma = {"kernel": "gate_up_geglu (v_mfma_i32_32x32x32_i8, activations as the 8-row operand)",
-                "useful_int8_TOPs": 2.0 * w_elems * a.rows / sec / 1e12, "issued_int8_TOPs": 2.0 * w_elems * 8 / sec / 1e12,
+        alone = gu["name"] == "gate_up_geglu"
+        mfma = {"kernel": "gate_up_geglu (v_mfma_i32_32x32x32_i8, activations as the 8-row operand)" if alone else
+                          gu["name"] + " with gate_up_geglu (v_mfma_i32_16x16x64_i8, two K segments to a product)",
+                "useful_int8_TOPs": 2.0 * w_elems * a.rows / sec / 1e12, "issued_int8_TOPs": 2.0 * w_elems * (8 if alone else 16) / sec / 1e12,
                 "mfma_peak_TOPs": 5000.0, "mfma_utilisation": 2.0 * w_elems * a.rows / sec / 5.0e15}
     line = {
         "metric": ("verified tok/s (E4B-shape q4_0, block-4, ctx 2048) + achieved HBM GB/s vs peak" if a.workload == "e4b" and ctx == CTX else
