@@ -707,6 +707,24 @@ __global__ __launch_bounds__(64) void lg_k_ipl(IplArgs a, const StepCtl *ctl) {
                                                (p.z * sc * wn.z + tk[2]) * a.rsqrt2, (p.w * sc * wn.w + tk[3]) * a.rsqrt2);
 }
 
+// A row that arrives as four slabs of partial sums, dv the first one's: (p0 + p1) + (p2 + p3).  The other three are requested at once, by every lane (past the row its last
+// values again): under a condition per float4 each waited for the one before it, three trips instead of one (a prompt of 23 on
+// the E4B shape, 22 rows by lg_k_wide_rows_plegate: 4955 -> 4901 us; one of 4093 on the 12B shape, lg_k_wide_rows: 182.7 -> 182.3 ms).
+__device__ __forceinline__ void lg_add_slabs(float4 (&dv)[LG_ROWV], const float4 *row, size_t slab, int t, int nq) {
+    float4 p1[LG_ROWV], p2[LG_ROWV], p3[LG_ROWV];
+    #pragma unroll
+    for (int v = 0; v < LG_ROWV; ++v) {
+        const int at = t + 256 * v < nq ? t + 256 * v : nq - 1;
+        p1[v] = row[slab + at]; p2[v] = row[2 * slab + at]; p3[v] = row[3 * slab + at];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    #pragma unroll
+    for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) {
+        const float4 p0 = dv[v];
+        dv[v] = make_float4((p0.x + p1[v].x) + (p2[v].x + p3[v].x), (p0.y + p1[v].y) + (p2[v].y + p3[v].y),
+                            (p0.z + p1[v].z) + (p2[v].z + p3[v].z), (p0.w + p1[v].w) + (p2[v].w + p3[v].w));
+    }
+}
 // PLE gate: inp_gate matmul on the q8 of the updated residual, then gelu(.) * ipl and q8.
 struct PleGateArgs {
     const uint8_t *w;        // tiled inp_gate [ple][E]
@@ -755,15 +773,7 @@ __device__ __forceinline__ void lg_rows_plegate_body(const RowsPleGateArgs &a, i
         const float4 *wr = (const float4 *)a.w_post, *xr = (const float4 *)(a.x + (size_t)j * E), *dr = (const float4 *)(a.dout + (size_t)j * E);
         #pragma unroll
         for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) { xv[v] = xr[t + 256 * v]; dv[v] = dr[t + 256 * v]; wp[v] = wr[t + 256 * v]; }
-        if (a.dparts == 4) {                                  // the top two levels of the tree of an ffn_down cut by K quarter
-            const size_t slab = (size_t)rows * nq;
-            #pragma unroll
-            for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) {
-                const float4 p1 = dr[slab + t + 256 * v], p2 = dr[2 * slab + t + 256 * v], p3 = dr[3 * slab + t + 256 * v], p0 = dv[v];
-                dv[v] = make_float4((p0.x + p1.x) + (p2.x + p3.x), (p0.y + p1.y) + (p2.y + p3.y),
-                                    (p0.z + p1.z) + (p2.z + p3.z), (p0.w + p1.w) + (p2.w + p3.w));
-            }
-        }
+        if (a.dparts == 4) lg_add_slabs(dv, dr, (size_t)rows * nq, t, nq);      // the top two levels of the tree of an ffn_down cut by K quarter
         if (a.dparts == 8) {                                  // the top three levels of the K-segment tree of an ffn_down cut over the 8 XCDs
             const size_t slab = (size_t)rows * nq;
             #pragma unroll

@@ -388,20 +388,13 @@ __global__ __launch_bounds__(LG_WG) void lg_k_wide_rows(RowArgs s, int rows) {
         const float4 *dr = (const float4 *)(s.dout + (size_t)j * E), *wr = (const float4 *)s.w_post;
         #pragma unroll
         for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) { dv[v] = dr[t + 256 * v]; wpost[v] = wr[t + 256 * v]; }
-        if (s.dparts == 4) {
-            const size_t slab = (size_t)rows * nq;
-            #pragma unroll
-            for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) {
-                const float4 p1 = dr[slab + t + 256 * v], p2 = dr[2 * slab + t + 256 * v], p3 = dr[3 * slab + t + 256 * v], p0 = dv[v];
-                dv[v] = make_float4((p0.x + p1.x) + (p2.x + p3.x), (p0.y + p1.y) + (p2.y + p3.y), (p0.z + p1.z) + (p2.z + p3.z), (p0.w + p1.w) + (p2.w + p3.w));
-            }
-        }
     }
     if (s.w_pre) {
         const float4 *wr = (const float4 *)s.w_pre;
         #pragma unroll
         for (int v = 0; v < LG_ROWV; ++v) if (t + 256 * v < nq) wpre[v] = wr[t + 256 * v];
     }
+    if (s.dout && s.dparts == 4) lg_add_slabs(dv, (const float4 *)(s.dout + (size_t)j * E), (size_t)rows * nq, t, nq);
     if (s.dout) {
         float ss = 0.0f;
         #pragma unroll
