@@ -217,6 +217,7 @@ struct lg_hip_model {
     bool turn_recorded = false;                            // ev_turn holds the end of its latest step already
     bool launching = false;                                // a step of it is being launched or captured: its stream is its own
     bool plain = false;                                    // the step that is being launched takes the kernels that wait for nobody
+    bool prompting = false;                                // prompt blocks of it are under way (PromptTurn)
     std::vector<std::pair<void *, size_t>> marks;          // memory whose words carry launch numbers (mark_alloc)
     int marked_steps = 0;                                  // steps since it was last cleared (count_steps)
     bool committed = false, wide_built = false;    // wide_built: the matrices' wide forms exist
@@ -314,9 +315,16 @@ static int dev_alloc(lg_hip_model *m, T **p, size_t n) {
 // XCD's 32 and wait for the rest until both give up.  So one model has them at a time: the one whose latest such step has not ended yet.  A step of another
 // model takes the kernels that wait for nobody (same bits) and overlaps with it as streams do.  Two models of 512 values, a step each at a time: 106 us
 // with separate kernels in both, 162 when the steps of one waited for the other's, 97 and 80 so; of 2560 values and 5 rows 156, 316, 165 and 155.  With one model at work this is an uncontended lock twice a step.
+// A prompt's blocks wait for nobody, but their kernels run for milliseconds (of rows far into a long cache for tens of them), and their workgroups go on filling the CUs
+// that a waiting launch needs whole, up to all 256, while those of it that have a place hold theirs and poll, a bounded number of times: the
+// step would be refused.  So while a model has prompt blocks under way the others' steps take the separate kernels too, and the
+// blocks follow, on the device, what others have launched of the waiting kind before (PromptTurn).  12 layers of the E4B shape beside prompts of
+// 8176 tokens of 6 layers of the 12B shape: a decode step 2440 us and a prompt 71 ms with waiting launches in the steps, 1820 and 54 so (alone 447 and 50); 5 rows
+// 2555 and 81, 2170 and 57.
 struct Turns {
     std::mutex mu;                             // not held over launches: a thread that launches many steps would keep the others out
     lg_hip_model *last = nullptr;              // whose step with such launches was the latest
+    int prompts = 0;                           // models with prompt blocks under way
 };
 static Turns *turns_of(int device) {
     static std::mutex mu;
@@ -327,14 +335,6 @@ static Turns *turns_of(int device) {
 static lg_hip_model *stream_owner(lg_hip_model *m) { return m->target ? m->target : m; }       // (a draft head has its target's stream)
 // Whether a step of m that is launched now may hold such launches
 static bool may_wait(const lg_hip_model *m) { return m->numbered && !(m->target ? m->target : m)->plain; }
-// Ahead of long work without such launches (a prompt's blocks): another model may have them meanwhile
-static int mark_turn(lg_hip_model *m) {
-    std::lock_guard<std::mutex> turn(m->turns->mu);
-    if (m->turns->last != m || m->turn_recorded) return 0;
-    HIP_TRY(hipEventRecord(m->ev_turn, m->stream));
-    m->turn_recorded = true;
-    return 0;
-}
 // For a launch of that kind outside of any model, on a stream that is waited for before the lock is given back
 static int take_turn_alone(std::unique_lock<std::mutex> &turn) {
     int device = 0;
@@ -342,7 +342,7 @@ static int take_turn_alone(std::unique_lock<std::mutex> &turn) {
     Turns *t = turns_of(device);
     for (;;) {
         turn = std::unique_lock<std::mutex>(t->mu);
-        if (!t->last || !t->last->launching) break;
+        if (!t->prompts && (!t->last || !t->last->launching)) break;
         turn.unlock();
         std::this_thread::yield();
     }
@@ -1435,6 +1435,7 @@ struct Turn {
     }
     int claim() {
         lg_hip_model *&last = own->turns->last;
+        if (own->turns->prompts > own->prompting) { own->plain = true; return 0; }
         if (last && last != own) {
             if (last->launching) { own->plain = true; return 0; }
             if (!last->turn_recorded) HIP_TRY(hipEventRecord(last->ev_turn, last->stream));
@@ -1450,6 +1451,35 @@ struct Turn {
         last = own;
         own->turn_recorded = false;
         return 0;
+    }
+};
+// Held while prompt blocks of m are launched and run.  The caller waits for m's stream before it gives this back, and a failed call here.
+struct PromptTurn {
+    lg_hip_model *own = nullptr;
+    bool done = false;                         // the stream has been waited for
+    int begin(lg_hip_model *m) {
+        Turns *t = m->turns;
+        std::unique_lock<std::mutex> lock(t->mu);
+        (own = m)->prompting = true;
+        ++t->prompts;                          // (from here on no step of another model is launched with such launches)
+        while (t->last && t->last != m && t->last->launching) {
+            lock.unlock();
+            std::this_thread::yield();
+            lock.lock();
+        }
+        lg_hip_model *last = t->last;
+        if (!last || last == m) return 0;
+        if (!last->turn_recorded) HIP_TRY(hipEventRecord(last->ev_turn, last->stream));
+        last->turn_recorded = true;
+        HIP_TRY(hipStreamWaitEvent(m->stream, last->ev_turn, 0));
+        return 0;
+    }
+    ~PromptTurn() {
+        if (!own) return;
+        if (!done) (void)hipStreamSynchronize(own->stream);
+        std::lock_guard<std::mutex> lock(own->turns->mu);
+        own->prompting = false;
+        --own->turns->prompts;
     }
 };
 template <int M>
@@ -2416,7 +2446,8 @@ extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *tok
     const int cap = m->sched_cap * LG_HIP_MAX_ROWS;        // tokens the staging holds
     int32_t *err = m->pin + 32 + LG_REPORT_ERR;             // (written by the verify blocks among the call's, the prompt kernels wait for nobody)
     __atomic_store_n(err, 0, __ATOMIC_RELAXED);
-    if (wide_ok && n > m->max_rows) { const int rc = mark_turn(m); if (rc) return rc; }
+    PromptTurn prompt;
+    if (wide_ok && n > m->max_rows) { const int rc = prompt.begin(m); if (rc) return rc; }
     for (int at = 0; at < n;) {
         // the tokens go over once, the blocks follow each other on the stream and the host waits at the end
         const int part = n - at < cap ? n - at : cap;
@@ -2443,6 +2474,7 @@ extern "C" int lg_hip_prefill(lg_hip_model *m, lg_hip_kv *kv, const int32_t *tok
         at += part;
         HIP_TRY(hipStreamSynchronize(m->stream));
     }
+    prompt.done = true;
     return step_err("prefill", __atomic_load_n(err, __ATOMIC_RELAXED));
 }
 

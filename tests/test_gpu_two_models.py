@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 NARROW = dict(E=512, heads=8, nkv=2, hd=64, ff=1024, rows=1)             # lg_k_narrow
 WIDE = dict(E=2560, heads=8, nkv=2, hd=256, ff=2048, rows=5)             # lg_k_attn_out_m
 ONE = dict(WIDE, rows=2)                                                 # lg_k_attn_out
+JOINED = dict(E=3840, heads=16, nkv=8, hd=256, ff=5120, rows=5)          # lg_k_o_geglu, lg_k_down_qkv
 LAYERS, VOCAB, SEQ, FRONT = 3, 2048, 512, 130
 
 
@@ -51,7 +52,7 @@ class Served:
             for n, k in (("attn_q_norm", s["hd"]), ("attn_k_norm", s["hd"]), ("attn_norm", E), ("post_attention_norm", E), ("ffn_norm", E), ("post_ffw_norm", E)):
                 vec(b + n, k)
         assert H.lg_hip_model_commit(self.m, 8) == 0, H.lg_hip_last_error()
-        assert H.lg_hip_kv_create(self.m, SEQ, C.byref(self.kv)) == 0, H.lg_hip_last_error()
+        assert H.lg_hip_kv_create(self.m, s.get("seq", SEQ), C.byref(self.kv)) == 0, H.lg_hip_last_error()
         self.prompt = rng.integers(1, VOCAB, FRONT).astype(np.int32)
         self.blocks = rng.integers(1, VOCAB, (300, s["rows"])).astype(np.int32)
 
@@ -113,3 +114,51 @@ def test_two_threads_with_a_model_each(H, a, b):
     finally:
         for m in models:
             m.close()
+
+
+def launches(m, rows):
+    """Launches of a step by class."""
+    cap = 32
+    names, ms, n, by = (C.c_char_p * cap)(), np.zeros(cap, np.float32), np.zeros(cap, np.int32), np.zeros(cap, np.float64)
+    k = m.H.lg_hip_profile_step(m.m, m.kv, m.blocks[0][:rows], rows, FRONT, 1, names, ms, n, by, cap)
+    assert k > 0, m.H.lg_hip_last_error()
+    return {names[i].decode(): int(n[i]) for i in range(k)}
+
+
+def test_steps_beside_a_prompt_wait_for_nobody(H):
+    """A prompt's kernels hold the CUs for long: while another model has one under way a step has no launch whose workgroups wait for one another, and the same results."""
+    a, b = Served(H, JOINED, 1), Served(H, dict(WIDE, seq=4096), 2)
+    try:
+        rows = JOINED["rows"]
+        out, adv = np.zeros(rows, np.int32), C.c_int32(0)
+
+        def step():
+            assert H.lg_hip_forward_spec(a.m, a.kv, a.blocks[0], rows, FRONT, out, C.byref(adv)) == 0, H.lg_hip_last_error()
+            return out.copy()
+        assert H.lg_hip_prefill(a.m, a.kv, a.prompt, FRONT, 0) == 0
+        alone = step()
+        assert launches(a, rows).get("gate_up_geglu", 0) == 0
+        long = np.resize(b.prompt, 4000)
+        rcs, begun = [], threading.Event()
+
+        def prompts():
+            for _ in range(40):
+                begun.set()
+                rcs.append(H.lg_hip_prefill(b.m, b.kv, long, len(long), 0))
+        t = threading.Thread(target=prompts)
+        print("together", flush=True)
+        t.start()
+        begun.wait()
+        seen = []
+        while t.is_alive():
+            n = launches(a, rows).get("gate_up_geglu", 0)
+            assert np.array_equal(step(), alone)
+            if t.is_alive():
+                seen.append(n)
+        t.join()
+        assert rcs == [0] * 40 and len(seen) > 3
+        assert sum(n == LAYERS for n in seen) >= len(seen) - 2, seen    # (one may fall between two prompts)
+        assert launches(a, rows).get("gate_up_geglu", 0) == 0           # theirs again
+    finally:
+        a.close()
+        b.close()

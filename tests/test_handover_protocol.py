@@ -136,3 +136,83 @@ def test_one_model_at_a_time_has_launches_that_wait(checks_launching):
         except AssertionError:
             seen = True
     assert seen is not checks_launching
+
+
+class Device:
+    """Streams of (kind, what has to have ended before) in order; an entry runs when it is at the front of its stream and nothing is left to wait for."""
+
+    def __init__(self, n):
+        self.streams, self.done = [[] for _ in range(n)], [0] * n
+
+    def running(self):
+        return [s[0][0] for s in self.streams if s and (s[0][1] is None or self.done[s[0][1][0]] >= s[0][1][1])]
+
+    def end(self, i):
+        s = self.streams[i]
+        if s and (s[0][1] is None or self.done[s[0][1][0]] >= s[0][1][1]):
+            s.pop(0)
+            self.done[i] += 1
+
+
+def server(dev, ms, me, turns, rng, checks_prompts):
+    """The calls of one model: steps (as `caller` has them) and prompts, which the host waits for."""
+    for _ in range(8):
+        m = ms[me]
+        if rng.random() < 0.4:
+            dep = None
+            if checks_prompts:
+                m.prompting = True
+                yield
+                last = turns[0]
+                while last is not None and last != me and ms[last].launching:
+                    yield
+                    last = turns[0]
+                if last is not None and last != me:
+                    dep = (last, dev.done[last] + len(dev.streams[last]))
+            want = dev.done[me] + len(dev.streams[me]) + 2
+            for _ in range(2):
+                dev.streams[me].append(("prompt", dep))
+                yield
+            while dev.done[me] < want:
+                yield
+            m.prompting = False
+        else:
+            m.launching, m.plain = True, False
+            last = turns[0]
+            if checks_prompts and any(o.prompting for o in ms if o is not m):
+                m.plain = True
+            elif last is not None and last != me:
+                m.plain = ms[last].launching or "waiting" in [k for k, _ in dev.streams[last]]
+            if not m.plain:
+                turns[0] = me
+            yield
+            dev.streams[me].append(("plain" if m.plain else "waiting", None))
+            yield
+            m.launching = False
+        yield
+
+
+@pytest.mark.parametrize("checks_prompts", [True, False])
+def test_no_prompt_runs_beside_launches_that_wait(checks_prompts):
+    """Threads and streams in any order: a prompt's blocks and launches that wait are never on the device together.  Without the count of prompts, and the wait
+    of a prompt's stream for what was launched before it, the model sees them there."""
+    import random
+    together = twos = 0
+    for seed in range(400):
+        rng, turns, dev, ms = random.Random(seed), [None], Device(3), [Model() for _ in range(3)]
+        for m in ms:
+            m.prompting = False
+        live = [server(dev, ms, i, turns, rng, checks_prompts) for i in range(3)]
+        for _ in range(20000):
+            if not live:
+                break
+            g = rng.choice(live)
+            if next(g, "left") == "left":
+                live.remove(g)
+            if rng.random() < 0.5:
+                dev.end(rng.randrange(3))
+            on = dev.running()
+            together += "prompt" in on and "waiting" in on
+            twos += on.count("waiting") > 1
+        assert not live, "a thread waits for ever"
+    assert not twos and bool(together) is not checks_prompts
