@@ -1309,21 +1309,21 @@ static void launch_xffn(Launcher &lx, const XffnArgs &a, int cls) {
     }
 }
 
-// Whether that launch is lg_k_ple_tail_s: 5 to 8 rows (its units fit one per CU), 1 and 2 (it has enough wavefronts for the projection), and 3 and 4 where
-// the next layer's projections are part of it
-static bool tail_spreads(const lg_hip_model *m, int rows) { return m->tail_spread && (rows >= 5 || rows <= 2 || m->tail_qkv || m->tail_spread == 2); }
+// Whether the layer tail's launch is lg_k_ple_tail_s: 5 to 8 rows (its units fit one per CU), 1 and 2 (it has enough wavefronts for the projection), and 3 and 4 where
+// the next layer's projections are part of it (joins; without them it is no faster there: 12 layers of 768 values, four rows, 404 us a step and 395 with lg_k_ple_tail)
+static bool tail_spreads(const lg_hip_model *m, int rows, bool joins) { return m->tail_spread && (rows >= 5 || rows <= 2 || joins || m->tail_spread == 2); }
 // ... which they are while the workgroups on the other seven XCDs, one to a CU, take 16 or 32 of their rows each
 static bool tail_does_qkv(const lg_hip_model *m, int rows, const Layer &next) {
-    return m->tail_qkv && m->trows && tail_spreads(m, rows) && next.qkv_m <= (LG_XCDS - 1) * rows * (LG_XCD_WGS / rows) * (rows >= LG_TAIL_MFMA ? 32 : 16) &&
+    return m->tail_qkv && m->trows && m->tail_spread && next.qkv_m <= (LG_XCDS - 1) * rows * (LG_XCD_WGS / rows) * (rows >= LG_TAIL_MFMA ? 32 : 16) &&
            (rows < LG_TAIL_MFMA || next.wqkv_ch);
 }
 // The per-layer-input block of a verify block of `rows` rows as the one-XCD launch lg_k_ple_tail: q4_0 matrices of the
-// 256-wide per-layer input, at most LG_XTAIL_UNITS (gate block, row) units, a chip whose workgroups are dealt over 8 XCDs
-static bool use_ple_tail(const lg_hip_model *m, int rows) {
+// 256-wide per-layer input, at most LG_XTAIL_UNITS (gate block, row) units, a chip whose workgroups are dealt over 8 XCDs.  joins: with the next layer's projections
+static bool use_ple_tail(const lg_hip_model *m, int rows, bool joins) {
     if (!m->ple || !m->tsync || !may_wait(m) || m->xcd_tail <= 0 || m->target) return false;
     if (m->ple != 256 || (m->ple / 32) * rows > LG_XTAIL_UNITS || m->E % 256 || m->E > 4096 || (m->E + 1023) / 1024 > m->ple / 32) return false;
     const int U = (m->ple / 32) * rows;
-    const bool spread = tail_spreads(m, rows);               // (lg_k_ple_tail_s: 8 wavefronts per unit, enough of them at every width)
+    const bool spread = tail_spreads(m, rows, joins);        // (lg_k_ple_tail_s: 8 wavefronts per unit, enough of them at every width)
     // blocks of one and two rows: with lg_k_ple_tail_s the tail beats folding the next layer's row work into its q/k/v
     // matmul (E4B shape: 1.994 -> 1.958 ms at one row, 2.127 -> 2.032 at two); with lg_k_ple_tail alone it does not
     if (m->xcd_tail == 1 && rows <= LG_FUSE_ROWS_MAX && m->fuse_rows && !spread) return false;
@@ -1415,7 +1415,7 @@ static bool use_mid_down(const lg_hip_model *m, const Layer &y, const Layer &nex
 static bool use_mid_proj(const lg_hip_model *m, const Layer &next) { return m->mid && m->midd && may_wait(m) && m->ple && next.wqkv_pc; }
 // Whether a step has launches whose workgroups wait for one another, if it may
 static bool step_waits(const lg_hip_model *m, int rows) {
-    return may_wait(m) && (use_narrow(m, rows) || (m->attn_out && m->aosync) || (m->mid && m->mido) || use_ple_tail(m, rows) || m->rows_geglu || m->xcd_attn_tail > 0 ||
+    return may_wait(m) && (use_narrow(m, rows) || (m->attn_out && m->aosync) || (m->mid && m->mido) || use_ple_tail(m, rows, true) || m->rows_geglu || m->xcd_attn_tail > 0 ||
                            (rows >= 4 && ((m->down_m == 1 && m->dmsync) || m->xcd_ffn)));
 }
 // Held while a step of m is launched (or a round of `head` and m, its target); begin() finds out whether it may have such launches
@@ -1499,10 +1499,9 @@ static void launch_ple_tail(Launcher &lx, const XtailArgs &a) {
     lg_hip_model *m = lx.m;
     const int E = a.r.g.k;
     {
-        // 5..8 rows: the form whose units fit one per CU (row j by 32 / M workgroups of 8 wavefronts); 1 and 2 rows: the
-        // form that has enough wavefronts for the projection
+        // (row j by 32 / M workgroups of 8 wavefronts)
         const int W = M * (32 / M), G = (E / 8 + 8 * W - 1) / (8 * W);
-        if (tail_spreads(m, M) && a.gf && a.r.g.ple == 256 && G >= 1 && G <= 3) {
+        if (tail_spreads(m, M, a.qw != nullptr) && a.gf && a.r.g.ple == 256 && G >= 1 && G <= 3) {
             const size_t lds = lg_tail_s_lds(M, E, a.r.g.ple, a.qw != nullptr);
             const dim3 grid(LG_XCDS * W);
             static int fits[2][4] = {};                       // per tiles of a gate row group (10, 16) and G: 0 unknown, 1 yes, -1 no (asked once, outside any capture)
@@ -1636,7 +1635,6 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         }
     };
 
-    const bool tail = use_ple_tail(m, M);
     const bool narrow = use_narrow(m, M);
     bool qkv_done = false;                         // the layer's projections have been done by the launch before it (lg_k_narrow)
     bool rows_done = false;                        // the row work ahead of the next matmul has been done by the launch before it
@@ -1933,9 +1931,9 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
         } else
         if (m->ple) {   // per-layer embedding block
             PleGateArgs a{ y.winp, E, m->ple, m->hq, m->pmp_raw, L, nl, m->pq };
-            if (tail && (L + 1 < nl || with_head) && pend_dout && have_x && !pend_os) {
+            const bool last = L + 1 == nl, joins = !last && tail_does_qkv(m, M, m->L[L + 1]);
+            if (use_ple_tail(m, M, joins) && (!last || with_head) && pend_dout && have_x && !pend_os) {
                 // the whole block and the row work that follows it (the next layer's, or the head's) in one launch on one XCD
-                const bool last = L + 1 == nl;
                 const bool head_m = M >= 4 && m->emb_rb && m->head_mfma;
                 XtailArgs f{};
                 f.r = RowsPleGateArgs{ a, m->x[cur], pend_dout, pend_w, nullptr, m->eps, pend_parts };
@@ -1945,7 +1943,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
                 f.q = m->hq; f.q_units = last && head_m ? 2 : 0;
                 f.seq = L; f.spin_limit = m->wait_polls; f.stamps = m->tail_stamps ? m->tstamps : nullptr;
                 f.gf = m->tgf; f.rows = m->trows;
-                if (!last && tail_does_qkv(m, M, m->L[L + 1])) {
+                if (joins) {
                     f.qw = M >= LG_TAIL_MFMA ? m->L[L + 1].wqkv_ch : m->L[L + 1].wqkv; f.qm = m->L[L + 1].qkv_m; f.qout = m->qkv;
                     qkv_done = true;
                 }
@@ -2588,7 +2586,7 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
     const bool narrow = use_narrow(m, rows);              // (everything but the attention and the first layer's projections)
     for (int L = 0; L < m->n_layer; ++L) {
         const Layer &y = m->L[L];
-        b[L && (narrow || (!y.winp_f && use_ple_tail(m, rows) && tail_does_qkv(m, rows, y))) ? KC_TAIL : L && !narrow && (use_mid_down(m, m->L[L - 1], y, rows) || (y.winp_f && use_mid_proj(m, y))) ? KC_ROWS : KC_QKV] += (double)m->E * y.qkv_m * q;
+        b[L && (narrow || (!y.winp_f && tail_does_qkv(m, rows, y) && use_ple_tail(m, rows, true))) ? KC_TAIL : L && !narrow && (use_mid_down(m, m->L[L - 1], y, rows) || (y.winp_f && use_mid_proj(m, y))) ? KC_ROWS : KC_QKV] += (double)m->E * y.qkv_m * q;
         if (narrow) b[KC_TAIL] += ((double)y.qd * m->E + 3.0 * m->E * y.nff + 2.0 * m->E * m->ple) * q;
         else {
         {
@@ -2599,7 +2597,7 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
         const int tiles = step_tiles(m, kv, y, rows, 0);
         if (m->xffn_built && m->xcd_ffn && may_wait(m) && rows >= 4) b[KC_FFN] += 3.0 * m->E * y.nff * q;
         else { b[use_attn_out(m, y, rows, tiles) ? attn_out_geglu(m, y, rows, tiles) ? KC_ATAIL : KC_GATEUP : use_mid_o(m, y, rows) ? KC_O : KC_GATEUP] += 2.0 * m->E * y.nff * q; b[L + 1 < m->n_layer && use_mid_down(m, y, m->L[L + 1], rows) ? KC_ROWS : KC_DOWN] += (double)y.nff * m->E * q; }
-        if (m->ple && !y.winp_f && use_ple_tail(m, rows)) b[KC_TAIL] += 2.0 * m->E * m->ple * q;
+        if (m->ple && !y.winp_f && use_ple_tail(m, rows, L + 1 < m->n_layer && tail_does_qkv(m, rows, m->L[L + 1]))) b[KC_TAIL] += 2.0 * m->E * m->ple * q;
         else if (m->ple) { const double pq = y.winp_f ? 4.0 : q; b[KC_PLEGATE] += (double)m->E * m->ple * pq; b[L + 1 < m->n_layer && y.winp_f && use_mid_proj(m, m->L[L + 1]) ? KC_ROWS : KC_PLEPROJ] += (double)m->ple * m->E * pq; }
         }
         const int window = (y.is_local && m->window > 0) ? m->window : 0;

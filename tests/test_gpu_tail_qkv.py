@@ -44,3 +44,25 @@ def test_one_launch_equals_two(lg, gpu_required, model_path, over, fused):
         assert all(np.array_equal(a, b) for a, b in zip(*got))
     finally:
         gpu.close()
+
+
+@pytest.mark.parametrize("over,rows,joins", [
+    (dict(n_embd=768), 4, False),                                                                    # not on the matrix cores: q/k/v keep their launch
+    (dict(n_embd=1024, n_head=20, n_head_kv=4, head_dim=256, head_dim_full=256), 3, False),          # more rows than 16 to a workgroup
+    (dict(n_embd=1024, n_head=4, n_head_kv=1), 3, True)])
+def test_three_and_four_rows_take_the_form_that_joins_where_it_joins(lg, gpu_required, model_path, over, rows, joins):
+    """lg_k_ple_tail_s at 3 and 4 rows only with the projections in it.  The units' stamps say which form ran: 8 x 3 units of lg_k_ple_tail or 3 x 10 of lg_k_ple_tail_s
+    at three rows; at four lg_k_ple_tail alone has a phase 6.  (The last layer's, which joins nothing, is lg_k_ple_tail in either case.)"""
+    path, spec = model_path("tiny_full", **dict(dict(n_layer=4, n_ff=512, n_vocab=2048), **over))
+    toks = np.random.default_rng(rows).integers(1, spec["n_vocab"], rows).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, 64, max_rows=8)
+    try:
+        gpu.set_option("xcd_tail_stamps", 1)
+        gpu.forward_spec(toks, 0)
+        s = gpu.tail_stamps(0)
+        assert s[:24, 0].all()
+        if rows == 3:
+            assert s[24:30, 0].any() == joins and not s[30:, 0].any()
+        assert s[:, 6].any()
+    finally:
+        gpu.close()
