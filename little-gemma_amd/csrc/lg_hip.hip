@@ -1500,7 +1500,9 @@ static void launch_ple_tail(Launcher &lx, const XtailArgs &a) {
     const int E = a.r.g.k;
     {
         // (row j by 32 / M workgroups of 8 wavefronts)
-        const int W = M * (32 / M), G = (E / 8 + 8 * W - 1) / (8 * W);
+        constexpr int W = M * (32 / M);
+        const int G = (E / 8 + 8 * W - 1) / (8 * W);
+        static_assert((4096 / 8 + 8 * W - 1) / (8 * W) <= 3, "every row that use_ple_tail admits has an instantiation");
         if (tail_spreads(m, M, a.qw != nullptr) && a.gf && a.r.g.ple == 256 && G >= 1 && G <= 3) {
             const size_t lds = lg_tail_s_lds(M, E, a.r.g.ple, a.qw != nullptr);
             const dim3 grid(LG_XCDS * W);
@@ -1527,8 +1529,9 @@ static void launch_ple_tail(Launcher &lx, const XtailArgs &a) {
                 return true;
             };
             if (E <= 2560 ? launch(std::integral_constant<int, 10>{}) : launch(std::integral_constant<int, 16>{})) return;
-            if (a.qw) { lx.rc = fail(-2, "ple_tail: the units of %d rows do not fit one XCD", M); return; }
         }
+        // (the caller counts on q/k/v once it has asked for them, and the form below does not know of them)
+        if (a.qw) { lx.rc = fail(-2, "ple_tail: the units of %d rows of %d values do not fit one XCD with q/k/v", M, E); return; }
     }
     const int U = (a.r.g.ple / 32) * M;
     const int G = (E / 8 + 4 * U - 1) / (4 * U);
