@@ -245,7 +245,8 @@ struct lg_hip_model {
     int last_rows = 0, last_adv = 0;
     float *lstage = nullptr;           // pinned: two rows of logits on their way to a caller (lg_hip_get_logits), row j in half j % 2
     int lread = -1, lcoming = -1;      // the row of the latest step read last, and the one whose copy has been started
-    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1, attn_out = 1, tail_qkv = 1, attn_geglu = 1, mid = 1;
+    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1, attn_out = 1, tail_qkv = 1, attn_geglu = 1, mid = 2;
+    uint32_t mid_rows = 0;             // bit r: blocks of r rows have launches of lg_mid.h while mid is 2
     // the feed-forward half of a layer as one XCD-partitioned launch (lg_xffn.h): built when the shape and the chip fit
     int xcd_ffn = 0;                         // option: use it (verify blocks of 4..8 rows)
     int down_m = 1;                          // option: ffn_down of 4..8-row blocks on the matrix cores (lg_k_down_m): 1 = the row group's four workgroups add
@@ -655,6 +656,24 @@ static bool mid_down_shape(const lg_hip_model *m, int nff, int next_qkv) {
     return mid_model(m) && !m->ple && lg_segments(nff) == 32 && nff <= 1024 * LG_MID_NIT && next_qkv % 32 == 0 && next_qkv <= 32 * LG_XCDS * LG_XCD_WGS;
 }
 static bool mid_proj_shape(const lg_hip_model *m, int next_qkv) { return mid_model(m) && m->ple == 256 && m->E % 256 == 0 && next_qkv % 32 == 0 && next_qkv <= 32 * LG_XCDS * LG_XCD_WGS; }
+// Where the launches of lg_mid.h are faster than the ones they replace (models of 12 layers, one to eight rows, us a layer saved; option mid = 1: everywhere).
+// attn_output with gate/up pays for the hand-overs with work that the first product's rows, K values of attention, leave its 256 workgroups little of, and for
+// every block of a segment that its form is cut for and the rows have not (10 up to 2560 values, else 15: the loads and products are made all the same).
+//   full rows: 2560, K 2048 0.9 .. 0.3, K 4096 1.0 .. 2.6; 2304, K 3072 1.0 .. 1.4; 3840, K 4096 2.0 .. 1.0; K 1024 at four rows 0.5, 0.7, 0.3, at eight -0.4, -1.2, -2.1;
+//     3840, K 2048 at four rows 1.0, at eight -0.9
+//   one or two blocks short of 15: 3584 and 3328, K 4096, two rows 1.2 and 0.6, four 1.1 and 0.7, eight -0.3 and -1.0; K 1024 0.6 and 0.2, -0.8 and -1.3, -3.7 and -3.4
+//   others: 3072, FFN 11776, -0.4 .. -1.5 (K 4096), -0.8 .. -4.0 (K 2048); 768 to 1536, K 1024, -0.5 .. -1.7; 768 to 2048, K 4096, -0.4 at one row, 0.7 .. 1.3 at eight
+static bool mid_o_faster(int E, int K, int rows) {
+    const int spare = (E <= 2560 ? 10 : LG_MID_NIT) - (E >> 8);
+    if (spare == 0 || (E <= 2560 && spare == 1)) return rows <= 4 || K >= (E <= 2560 ? 2048 : 3072);
+    if (E > 2560) return spare <= 2 && rows <= (K >= 3072 ? 4 : 2);
+    return rows >= 4 && K >= (E >= 1280 ? 3072 : 4096);
+}
+// ffn_down with q/k/v: one and two rows have had the row work inside the q/k/v launch, so that there is one launch less to save.  One row: 768 to 2048 -0.4 .. -1.3,
+// 2304 to 3584 +-0.2, 3840 0.8; two: 768 and 1024 -0.1 .. -0.7, 1280 to 2048 0.8 .. 0, wider 1.0 .. 3.1; three and more (from 2304 on) 0.6 .. 7.2
+static bool mid_down_faster(int E, int rows) { return rows >= 3 || (rows == 2 && E >= 1280) || E > 3584; }
+// the per-layer projection with q/k/v, the same: one row 768 to 2048 -0.8 .. -1.6, wider -0.1 .. -0.3; two: up to 1280 -0.4 .. -0.8, wider 0.1 .. 1.1; three and more 0.2 .. 6.7
+static bool mid_proj_faster(int E, int rows) { return rows >= 3 || (rows == 2 && E >= 1536); }
 // shapes lg_k_attn_tail is instantiated for: pairs of blocks per chain, row blocks per unit
 static bool attn_tail_shape(int qd, int E, int *np, int *rbs) {
     if (qd % 512 || lg_segments(qd) != 8 || E % 256 || E > 4096) return false;
@@ -954,6 +973,9 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
     m->pin[32 + LG_REPORT_SEQ] = 0;
     HIP_TRY(hipDeviceSynchronize());
     m->wide_built = !m->target && m->wide_prefill;
+    for (int rows = 1; rows <= LG_HIP_MAX_ROWS; ++rows)
+        for (const Layer &y : m->L)
+            if ((y.wo_pc && mid_o_faster(E, y.qd, rows)) || (y.wqkv_pc && (m->ple ? mid_proj_faster(E, rows) : mid_down_faster(E, rows)))) m->mid_rows |= 1u << rows;
     m->committed = true;
     return 0;
 }
@@ -1398,7 +1420,7 @@ static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int t
 }
 // attn_output, row work and gate/up as one launch; not where one of the options does that row work elsewhere
 static bool use_mid_o(const lg_hip_model *m, const Layer &y, int rows) {
-    return m->mid && m->attn_out && m->mido && may_wait(m) && y.wo_pc && y.wgu && !(rows >= 4 && (m->rows_geglu || (m->xcd_ffn && y.xgu)));
+    return m->mid && (m->mid == 1 || mid_o_faster(m->E, y.qd, rows)) && m->attn_out && m->mido && may_wait(m) && y.wo_pc && y.wgu && !(rows >= 4 && (m->rows_geglu || (m->xcd_ffn && y.xgu)));
 }
 // ... and the merge of attention's partials: up to LG_MID_MERGE_ROWS rows (more: no gain, see lg_k_o_geglu) of up to LG_AOUT_TILES tiles, which a wavefront holds in
 // registers.  (Rows of up to 2560 values have lg_k_attn_out.)
@@ -1407,15 +1429,17 @@ static bool use_mid_merge(const lg_hip_model *m, const Layer &y, int rows, int t
 }
 // ffn_down, row work and the next layer's q/k/v projections as one launch (1 to 3 rows: with the whole rows in LDS)
 static bool use_mid_down(const lg_hip_model *m, const Layer &y, const Layer &next, int rows) {
-    if (!m->mid || !m->midd || !may_wait(m) || m->ple || !next.wqkv_pc) return false;
+    if (!m->mid || !(m->mid == 1 || mid_down_faster(m->E, rows)) || !m->midd || !may_wait(m) || m->ple || !next.wqkv_pc) return false;
     if (rows >= 4) return m->down_m == 1 && y.wdn_m && m->E > 2048 && lg_down_m_geo(m->E, y.nff).npairs <= LG_MID_NDP;
     return lg_downqkv_lds(rows, y.nff) <= 160 * 1024;
 }
 // ... with the per-layer projection of a float type in ffn_down's place
-static bool use_mid_proj(const lg_hip_model *m, const Layer &next) { return m->mid && m->midd && may_wait(m) && m->ple && next.wqkv_pc; }
+static bool use_mid_proj(const lg_hip_model *m, const Layer &next, int rows) {
+    return m->mid && (m->mid == 1 || mid_proj_faster(m->E, rows)) && m->midd && may_wait(m) && m->ple && next.wqkv_pc;
+}
 // Whether a step has launches whose workgroups wait for one another, if it may
 static bool step_waits(const lg_hip_model *m, int rows) {
-    return may_wait(m) && (use_narrow(m, rows) || (m->attn_out && m->aosync) || (m->mid && m->mido) || use_ple_tail(m, rows, true) || m->rows_geglu || m->xcd_attn_tail > 0 ||
+    return may_wait(m) && (use_narrow(m, rows) || (m->attn_out && m->aosync) || (m->mido && (m->mid == 1 || (m->mid && m->mid_rows >> rows & 1))) || use_ple_tail(m, rows, true) || m->rows_geglu || m->xcd_attn_tail > 0 ||
                            (rows >= 4 && ((m->down_m == 1 && m->dmsync) || m->xcd_ffn)));
 }
 // Held while a step of m is launched (or a round of `head` and m, its target); begin() finds out whether it may have such launches
@@ -1918,7 +1942,7 @@ static int enqueue_step(lg_hip_model *m, lg_hip_kv *kv, bool with_head, bool dry
             MmfArgs g{ y.winp_f, E, m->ple, m->x[cur], E, M, m->pgf, m->ple, m->pmp_raw + (size_t)L * m->ple, m->ple * nl };
             launch_mmf<M>(lx, KC_PLEGATE, g);
             }
-            if (pos_off == 0 && L + 1 < nl && use_mid_proj(m, m->L[L + 1])) {      // the projection, the row work behind it and the next layer's projections
+            if (pos_off == 0 && L + 1 < nl && use_mid_proj(m, m->L[L + 1], M)) {      // the projection, the row work behind it and the next layer's projections
                 DownQkvArgs f{};
                 f.d = DownHere{ (const uint8_t *)y.wproj_f, m->pgf, 0, E, nullptr, m->midd, m->wait_polls };
                 f.r = MidRowArgs{ m->x[cur], y.post_norm, y.out_scale, m->L[L + 1].attn_norm, m->x[cur ^ 1], nullptr, m->midrd, E, m->wait_polls, m->eps };
@@ -2177,7 +2201,7 @@ static GraphKey graph_key(const lg_hip_model *m, const lg_hip_kv *kv, int rows, 
     put(what, 2); put(rows, 4); put(m->store_logits != 0, 1); put(m->draft_chain, 1); put(m->fuse_rows, 1); put(m->attn_rows, 1); put(m->attn_rows_fq, 1);
     put(m->head_mfma, 1); put(m->down_kq, 1); put(m->xcd_ffn, 1); put(m->fork_ple, 1); put(m->rows_geglu, 1); put(m->tail_stamps != 0, 1);
     put(m->tail_spread == 1 ? 1 : m->tail_spread ? 2 : 0, 2); put(m->xcd_tail, 2); put(m->down_m, 2); put(m->xcd_attn_tail, 2); put(m->merge_o, 2);
-    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->tail_qkv, 1); put(m->attn_geglu, 1); put(m->mid, 1); put(m->wait_polls, 17); put(may_wait(m), 1);
+    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->tail_qkv, 1); put(m->attn_geglu, 1); put(m->mid, 2); put(m->wait_polls, 17); put(may_wait(m), 1);
     return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices, 0 };
 }
 
@@ -2241,7 +2265,7 @@ extern "C" int lg_hip_set_option(lg_hip_model *m, const char *name, int value) {
     else if (!strcmp(name, "rows_geglu")) m->rows_geglu = value != 0;
     else if (!strcmp(name, "narrow")) m->narrow = value != 0;
     else if (!strcmp(name, "attn_out")) m->attn_out = value != 0;
-    else if (!strcmp(name, "mid")) m->mid = value != 0;
+    else if (!strcmp(name, "mid")) m->mid = value == 1 ? 1 : value ? 2 : 0;
     else if (!strcmp(name, "tail_qkv")) m->tail_qkv = value != 0;
     else if (!strcmp(name, "attn_geglu")) m->attn_geglu = value != 0;
     else if (!strcmp(name, "down_kq")) m->down_kq = value != 0;
@@ -2589,7 +2613,7 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
     const bool narrow = use_narrow(m, rows);              // (everything but the attention and the first layer's projections)
     for (int L = 0; L < m->n_layer; ++L) {
         const Layer &y = m->L[L];
-        b[L && (narrow || (!y.winp_f && tail_does_qkv(m, rows, y) && use_ple_tail(m, rows, true))) ? KC_TAIL : L && !narrow && (use_mid_down(m, m->L[L - 1], y, rows) || (y.winp_f && use_mid_proj(m, y))) ? KC_ROWS : KC_QKV] += (double)m->E * y.qkv_m * q;
+        b[L && (narrow || (!y.winp_f && tail_does_qkv(m, rows, y) && use_ple_tail(m, rows, true))) ? KC_TAIL : L && !narrow && (use_mid_down(m, m->L[L - 1], y, rows) || (y.winp_f && use_mid_proj(m, y, rows))) ? KC_ROWS : KC_QKV] += (double)m->E * y.qkv_m * q;
         if (narrow) b[KC_TAIL] += ((double)y.qd * m->E + 3.0 * m->E * y.nff + 2.0 * m->E * m->ple) * q;
         else {
         {
@@ -2601,7 +2625,7 @@ static void class_bytes(const lg_hip_model *m, const lg_hip_kv *kv, int pos, int
         if (m->xffn_built && m->xcd_ffn && may_wait(m) && rows >= 4) b[KC_FFN] += 3.0 * m->E * y.nff * q;
         else { b[use_attn_out(m, y, rows, tiles) ? attn_out_geglu(m, y, rows, tiles) ? KC_ATAIL : KC_GATEUP : use_mid_o(m, y, rows) ? KC_O : KC_GATEUP] += 2.0 * m->E * y.nff * q; b[L + 1 < m->n_layer && use_mid_down(m, y, m->L[L + 1], rows) ? KC_ROWS : KC_DOWN] += (double)y.nff * m->E * q; }
         if (m->ple && !y.winp_f && use_ple_tail(m, rows, L + 1 < m->n_layer && tail_does_qkv(m, rows, m->L[L + 1]))) b[KC_TAIL] += 2.0 * m->E * m->ple * q;
-        else if (m->ple) { const double pq = y.winp_f ? 4.0 : q; b[KC_PLEGATE] += (double)m->E * m->ple * pq; b[L + 1 < m->n_layer && y.winp_f && use_mid_proj(m, m->L[L + 1]) ? KC_ROWS : KC_PLEPROJ] += (double)m->ple * m->E * pq; }
+        else if (m->ple) { const double pq = y.winp_f ? 4.0 : q; b[KC_PLEGATE] += (double)m->E * m->ple * pq; b[L + 1 < m->n_layer && y.winp_f && use_mid_proj(m, m->L[L + 1], rows) ? KC_ROWS : KC_PLEPROJ] += (double)m->ple * m->E * pq; }
         }
         const int window = (y.is_local && m->window > 0) ? m->window : 0;
         const int last = pos + rows - 1, start = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;

@@ -113,3 +113,44 @@ def test_merge_inside_the_launch(lg, gpu_required, model_path, over, pos0, cache
         assert all(np.array_equal(a, b) for a, b in zip(*got))
     finally:
         gpu.close()
+
+
+# (over, widths at which the launches are taken unless the option says otherwise: with gate/up, with q/k/v)
+@pytest.mark.parametrize("name,over,o,down", [
+    ("tiny", dict(n_embd=768, n_head=16, head_dim=64, n_ff=3072), (), ()),
+    ("tiny", dict(n_embd=768, n_head=20, head_dim=64, n_head_kv=4, n_ff=5120), (), (3,)),
+    ("tiny", dict(n_embd=1280, n_head=12, head_dim=256, n_ff=5632), range(4, 9), ()),
+    ("tiny", dict(n_embd=1536, n_head=20, head_dim=64, n_head_kv=4, n_ff=6144), (), (2, 3)),
+    ("tiny", dict(n_embd=2304, n_head=12, head_dim=256, n_ff=9216), ALL, range(2, 9)),
+    ("tiny", dict(n_embd=2560, n_head=16, head_dim=64, n_ff=10240), range(1, 5), range(2, 9)),
+    ("tiny", dict(n_embd=3072, n_head=16, head_dim=256, n_ff=8192), (), range(2, 9)),
+    ("tiny", dict(n_embd=3328, n_head=16, head_dim=128, n_ff=4608), (1, 2), ()),
+    ("tiny", dict(n_embd=3584, n_head=16, head_dim=256, n_ff=4608), range(1, 5), ()),
+    ("tiny", dict(n_embd=3840, n_head=16, head_dim=128, n_ff=4608), range(1, 5), ()),
+    ("tiny", dict(n_embd=3840, n_head=16, head_dim=256, n_head_kv=8, n_ff=5120), ALL, ALL),
+    ("tiny_full_bf16", dict(n_layer=4, n_embd=768), (), range(3, 9)),
+    ("tiny_full_bf16", dict(n_layer=4, n_embd=2560, head_dim_full=64), (), range(2, 9))])
+def test_taken_where_it_is_the_faster_form(lg, gpu_required, model_path, name, over, o, down):
+    """The default: the launches that join products where they were measured faster than the separate ones, by the widths of model and block; same bits as without."""
+    path, spec = model_path(name, **dict(dict(n_layer=3, n_vocab=2048, n_ff=512, sliding_window=64), **over))
+    toks = np.random.default_rng(spec["n_embd"]).integers(1, spec["n_vocab"], 40).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, 400, max_rows=8)
+    try:
+        got = []
+        for mid in (None, 0):
+            if mid is not None:
+                gpu.set_option("mid", mid)
+            gpu.new_cache()
+            res, pos = [], 0
+            for rows in ALL:
+                print(f"{name} {over}, {rows} rows, mid {mid}", flush=True)
+                n = {k["name"]: k["launches"] for k in gpu.profile_step(toks[:rows], 90, 1)}
+                assert (n.get("gate_up_geglu", 0) == 0) == (mid is None and rows in o), (rows, n)
+                assert n["qkv"] == (1 if mid is None and rows in down else spec["n_layer"]), (rows, n)
+                gpu.forward_spec(toks[pos:pos + rows], pos)
+                res.append(gpu.last_hidden(spec["n_embd"]).view(np.uint32))
+                pos += rows
+            got.append(res + [gpu.kv_read(0, w) for w in (0, 1)])
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
+    finally:
+        gpu.close()
