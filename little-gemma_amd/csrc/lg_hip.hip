@@ -697,6 +697,13 @@ static bool attn_out_shape(const lg_hip_model *m, const Layer &y) {
     return m->numbered && m->E > LG_NARROW_E && m->E <= LG_AOUT_E && m->E % 256 == 0 && y.qd == LG_AOUT_K && y.hd % 64 == 0 && y.wo;
 }
 
+// tiles of 32 positions that a block of `rows` rows of a sliding layer can touch, wherever it starts
+static int window_tiles(int window, int rows) { return (window + rows - 1 + 31) / 32 + 1; }
+// Layers that it serves at every width of the model's blocks: nothing then asks for attn_output in another launch's form
+static bool attn_out_always(const lg_hip_model *m, const Layer &y, int max_rows) {
+    return attn_out_shape(m, y) && y.is_local && m->window > 0 && window_tiles(m->window, max_rows) <= (max_rows > LG_AOUT_DOT_ROWS ? LG_AOUT_BATCH : LG_AOUT_TILES);
+}
+
 static const float *rope_table(lg_hip_model *m, int is_local, int hd, int *rc) {
     auto key = std::make_pair(is_local, hd);
     auto it = m->rope_tabs.find(key);
@@ -818,7 +825,7 @@ extern "C" int lg_hip_model_commit(lg_hip_model *m, int max_rows) {
         push_rows(rows, o, 0, E);
         if ((rc = upload_tiled(m, rows, y.qd, &y.wo, stage))) return rc;
         if ((rc = wide_form(m, y.wo, y.qd, E, false, &y.wo_w))) return rc;
-        if (mid_o_shape(m, y.qd, y.nff) && (rc = upload_pairs(m, rows, y.qd, &y.wo_pc, stage))) return rc;
+        if (mid_o_shape(m, y.qd, y.nff) && !attn_out_always(m, y, max_rows) && (rc = upload_pairs(m, rows, y.qd, &y.wo_pc, stage))) return rc;
         // (8 query heads: the K segments of this projection are the heads, and the merge can run their chains itself)
         if (!m->target && cu_count() == LG_XCDS * LG_XCD_WGS &&
             ((getenv("LG_HIP_XCD_ATTN_TAIL") && atoi(getenv("LG_HIP_XCD_ATTN_TAIL")) > 0 && attn_tail_shape(y.qd, E, nullptr, nullptr)) ||
@@ -1398,7 +1405,7 @@ static void launch_down_m(Launcher &lx, const DownMArgs &a) {
 static int step_tiles(const lg_hip_model *m, const lg_hip_kv *kv, const Layer &y, int rows, int pos_off) {
     const int window = (y.is_local && m->window > 0) ? m->window + pos_off : 0;
     if (window <= 0) return kv->tiles_max;
-    const int t = (window + rows - 1 + 31) / 32 + 1;
+    const int t = window_tiles(window, rows);
     return t < kv->tiles_max ? t : kv->tiles_max;
 }
 // (tiles: what one wavefront holds; more of them, a global layer in a cache of 1248 positions and more, are merged by more of the chip.  The row work

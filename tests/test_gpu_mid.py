@@ -1,6 +1,10 @@
 """A product, the row work behind it and the next product as one launch (lg_k_o_geglu, lg_k_down_qkv; option mid) against the separate kernels."""
+import ctypes as C
+
 import numpy as np
 import pytest
+
+from test_zz_no_alloc import loaded_hip_runtime
 
 pytestmark = pytest.mark.gpu
 
@@ -154,3 +158,25 @@ def test_taken_where_it_is_the_faster_form(lg, gpu_required, model_path, name, o
         assert all(np.array_equal(a, b) for a, b in zip(*got))
     finally:
         gpu.close()
+
+
+def test_no_copy_of_what_another_launch_always_serves(lg, gpu_required, model_path):
+    """attn_output as pairs of K segments is for layers that lg_k_attn_out cannot serve: sliding layers of a window that it holds at every width keep none, those of a wider one do."""
+    lg.load_hip()
+    hip, layers, used = C.CDLL(loaded_hip_runtime()), 24, []
+
+    def free():
+        free, total = C.c_size_t(0), C.c_size_t(0)
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+    for window in (512, 512, 1024):                            # (the first for what the process takes once)
+        path, spec = model_path("tiny", n_layer=layers, n_embd=2560, n_head=8, head_dim=256, n_ff=512, n_vocab=2048, sliding_window=window, local_period=100)
+        before = free()
+        gpu = lg.hiplib.HipBackend(path, 64, max_rows=8)
+        try:
+            gpu.forward_spec(np.ones(1, np.int32), 0)
+            used.append(before - free())
+        finally:
+            gpu.close()
+    copies = layers * 2560 * 2048 * 18 // 32
+    assert used[2] - used[1] > copies * 3 // 4, (used, copies)
