@@ -360,9 +360,9 @@ static int mark_alloc(lg_hip_model *m, T **p, size_t n = 1) {
     HIP_TRY(clear_now(m->stream, *p, 0, n * sizeof(T)));
     return 0;
 }
-// Called ahead of `steps` more steps of the model on its stream, never under capture.  A mark has 28 bits, so the numbers come round after 2^20 steps (half an hour
+// Called ahead of `steps` more steps of the model on its stream, never under capture.  Marks come round, a tag's 28 bits after 2^20 steps, those of a FarRows unit after 2^16 (two minutes
 // of steps of 1.7 ms), and what no launch has written since (the rows of a wider block, say) would then count as the present launch's.
-// Cleared every LG_MARK_STEPS it is never that old.
+// Cleared every LG_MARK_STEPS it is never that old.  (2 MB at most, a few microseconds.)
 static int count_steps(lg_hip_model *m, int steps) {
     if ((m->marked_steps += steps) <= LG_MARK_STEPS) return 0;
     m->marked_steps = steps;

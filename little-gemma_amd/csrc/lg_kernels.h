@@ -23,8 +23,9 @@ struct StepCtl {            // device-resident step state
                             // whenever it starts, also when another of them has given up its wait and left
 };
 #define LG_STEP_LAUNCHES 256 // more than the layers of a model that has such launches
-#define LG_MARK_STEPS (1 << 19)  // steps after which the marks of launches are cleared: they come round after 2^28 launch numbers
-static_assert((uint64_t)2 * LG_MARK_STEPS * LG_STEP_LAUNCHES <= (uint64_t)1 << 28, "marks older than half their range are cleared");
+#define LG_MARK_STEPS (1 << 15)  // steps after which the marks of launches are cleared: those of a FarRows unit come round after 2^16 steps, tags after 2^28 launch numbers
+static_assert(2 * LG_MARK_STEPS <= 1 << 16 && (uint64_t)2 * LG_MARK_STEPS * LG_STEP_LAUNCHES <= (uint64_t)1 << 28, "marks older than half their range are cleared");
+static_assert(LG_STEP_LAUNCHES == 256, "lg_far_marks takes the layer and the step from a number");
 
 // ---------------------------------------------------------------------------------------------
 // Row kernel: everything that happens to the M residual rows between two matmuls, one wavefront

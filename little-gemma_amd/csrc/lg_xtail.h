@@ -35,16 +35,16 @@
 #include "lg_fused.h"
 #include "lg_xcd.h"
 #include "lg_xffn.h"
+#include "lg_far.h"
 
 #define LG_XTAIL_UNITS 64           // most units of a launch (lane i of a wavefront polls flag i)
 struct XtailSync {
     uint32_t flags[2][LG_XTAIL_UNITS];      // lg_k_attn_tail: lg_tag of each unit's last arrival
 };
 
-// q8 rows that a launch hands from its one XCD to the workgroups on the other seven, in units of 16 bytes: three dwords and the launch's number exclusive-or'ed
-// with them (a lane's 16 bytes travel together; were they ever seen apart, the fourth dword would not fit).  Stored and loaded with an agent's scope: through the
-// writer's L2 to memory, and around the reader's.  A block of 32 values is three units, its 8 dwords and its scale.  On v_dot4 (lg_take_far_rows) the sum
-// of the values is added up by the reader; on the matrix cores weights are signed and none is needed.
+// q8 rows that a launch hands from its one XCD to the workgroups on the other seven, in units of 16 bytes, three dwords and the launch's marks (lg_far.h).  Stored and
+// loaded with an agent's scope: through the writer's L2 to memory, and around the reader's.  A block of 32 values is three units, its 8 dwords and its scale.  On v_dot4
+// (lg_take_far) the sum of the values is added up by the reader; on the matrix cores weights are signed and none is needed.
 struct FarRows {
     uint2 soon;                     // {-, tag}: the rows are on their way, from here on the waiting workgroups load them until they are there
     uint2 pad[15];
@@ -61,7 +61,7 @@ __device__ __forceinline__ void lg_put_far_q8(FarRows *f, int k, int j, int quad
     if (dw % 3) return;                                        // lanes 0, 3 and 6 store
     const uint32_t z = dw == 6 ? __float_as_uint(d) : c;
     const __amdgpu_buffer_rsrc_t r = lg_buffer_rsrc(f->u);
-    lg_x4u v; v.x = packed; v.y = b; v.z = z; v.w = tag ^ packed ^ b ^ z;
+    const lg_x4u v = lg_far_unit<lg_x4u>(packed, b, z, lg_far_marks(tag));
     __builtin_amdgcn_raw_buffer_store_b128(v, r, ((j * (k >> 5) + (quad >> 3)) * 3 + dw / 3) * 16, 0, 16);      // (16: the scope bit sc1)
 }
 // 64 values of row j (dims 64 u + lane) as q8 q, d their block's scale
@@ -70,7 +70,7 @@ __device__ __forceinline__ void lg_put_far_dims(FarRows *f, int k, int j, int u,
     const int l = lane < 6 ? lane : 5, b = l / 3, e = l - 3 * b, at = b * 32 + e * 12;          // lanes 0 .. 5 store a unit each
     const uint32_t x = __shfl(word, at), y = __shfl(word, at + 4), w = __shfl(word, e < 2 ? at + 8 : at), s = __float_as_uint(__shfl(d, at)), z = e < 2 ? w : s;
     const __amdgpu_buffer_rsrc_t r = lg_buffer_rsrc(f->u);
-    lg_x4u v; v.x = x; v.y = y; v.z = z; v.w = tag ^ x ^ y ^ z;
+    const lg_x4u v = lg_far_unit<lg_x4u>(x, y, z, lg_far_marks(tag));
     if (lane < 6) __builtin_amdgcn_raw_buffer_store_b128(v, r, ((j * (k >> 5) + 2 * u + b) * 3 + e) * 16, 0, 16);
 }
 // Wait until the rows are on their way (one load per wavefront and trip: workgroups that load the rows all the time keep the memory from the ones that make them)
@@ -85,6 +85,7 @@ __device__ __forceinline__ int lg_wait_soon(const FarRows *f, uint32_t tag, int 
 template <int N, typename A, typename P>
 __device__ __forceinline__ int lg_take_far(const FarRows *f, int total, int t, int nt, uint32_t tag, int spin_limit, A &&at, P &&put) {
     const __amdgpu_buffer_rsrc_t r = lg_buffer_rsrc(f->u);
+    const LgFarMarks marks = lg_far_marks(tag);
     lg_x4u v[N];
     int err = 0, o[N];
     #pragma unroll
@@ -94,13 +95,13 @@ __device__ __forceinline__ int lg_take_far(const FarRows *f, int total, int t, i
         #pragma unroll
         for (int i = 0; i < N; ++i) v[i] = __builtin_bit_cast(lg_x4u, __builtin_amdgcn_raw_buffer_load_b128(r, o[i], 0, 16));
         #pragma unroll
-        for (int i = 0; i < N; ++i) diff |= v[i].x ^ v[i].y ^ v[i].z ^ v[i].w ^ tag;
-        if (__all(diff == 0)) break;
+        for (int i = 0; i < N; ++i) diff |= lg_far_miss(v[i], marks);
+        if (__all(diff >> 16 == 0)) break;
         if (spins >= spin_limit) { err = LG_XFFN_ERR_WAIT; break; }
         asm volatile("" ::: "memory");
     }
     #pragma unroll
-    for (int i = 0; i < N; ++i) if (t + nt * i < total) put(t + nt * i, v[i]);
+    for (int i = 0; i < N; ++i) if (t + nt * i < total) { v[i].y = lg_far_y(v[i]); put(t + nt * i, v[i]); }
     return err;
 }
 // The rows in LDS for the matrix cores: a block of 32 values of all rows is LG_FAR_BLK bytes, 8 slots of 32 bytes (dwords in the order 0 1 4 5 2 3 6 7, the K halves
@@ -121,6 +122,7 @@ __device__ __forceinline__ int lg_take_far_segment(const FarRows *f, int k, int 
     const int st = e == 2 ? 1 : 8;                             // dwords from a slot to the next
     const __amdgpu_buffer_rsrc_t r = lg_buffer_rsrc(f->u);
     const int at = (wave * nit * 3 + w) * 16, row = nb * 48;
+    const LgFarMarks marks = lg_far_marks(tag);
     lg_x4u v[N];
     int err = 0;
     auto load = [&] {
@@ -135,8 +137,8 @@ __device__ __forceinline__ int lg_take_far_segment(const FarRows *f, int k, int 
     for (int spins = 0;; ++spins) {
         uint32_t diff = 0;
         #pragma unroll
-        for (int i = 0; i < N; ++i) diff |= v[i].x ^ v[i].y ^ v[i].z ^ v[i].w ^ tag;
-        if (__all(diff == 0)) break;
+        for (int i = 0; i < N; ++i) diff |= lg_far_miss(v[i], marks);
+        if (__all(diff >> 16 == 0)) break;
         if (spins >= spin_limit) { err = LG_XFFN_ERR_WAIT; break; }
         asm volatile("" ::: "memory");
         load();
@@ -144,7 +146,7 @@ __device__ __forceinline__ int lg_take_far_segment(const FarRows *f, int k, int 
     #pragma unroll
     for (int i = 0; i < N; ++i) {                              // (row H i + h: slot 4 h + i, or lg_far_slot(i))
         const int z = H == 2 ? i : lg_far_slot(i);
-        s0[z * 8] = v[i].x; s1[z * 8] = v[i].y; s2[z * st] = v[i].z;
+        s0[z * 8] = v[i].x; s1[z * 8] = lg_far_y(v[i]); s2[z * st] = v[i].z;
     }
     return err;
 }

@@ -216,3 +216,82 @@ def test_no_prompt_runs_beside_launches_that_wait(checks_prompts):
             twos += on.count("waiting") > 1
         assert not live, "a thread waits for ever"
     assert not twos and bool(together) is not checks_prompts
+
+
+SHIM = """
+#include "%s/lg_far.h"
+struct U { unsigned x, y, z, w; };
+extern "C" void put(const unsigned *xyz, unsigned tag, unsigned *u) { const U v = lg_far_unit<U>(xyz[0], xyz[1], xyz[2], lg_far_marks(tag)); u[0] = v.x; u[1] = v.y; u[2] = v.z; u[3] = v.w; }
+extern "C" int take(const unsigned *u, unsigned tag, unsigned *xyz) {
+    const U v = { u[0], u[1], u[2], u[3] };
+    xyz[0] = v.x; xyz[1] = lg_far_y(v); xyz[2] = v.z;
+    return lg_far_miss(v, lg_far_marks(tag)) >> 16 == 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def far(tmp_path_factory):
+    """put(three words, step, layer) -> a unit; take(unit, step, layer) -> its words, or None: the functions that the kernels call, built for the host."""
+    import ctypes as C
+    import os
+    import subprocess
+    d = tmp_path_factory.mktemp("far")
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "little-gemma_amd", "csrc")
+    (d / "far.cpp").write_text(SHIM % csrc)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", str(d / "far.so"), str(d / "far.cpp")], check=True)
+    L = C.CDLL(str(d / "far.so"))
+    U3, U4 = C.c_uint * 3, C.c_uint * 4
+
+    def tag(step, layer):
+        return (step * 256 + layer + 1) << 4 & 0xFFFFFFFF               # (lg_far_tag(lg_tag(launch + layer)))
+
+    def put(words, step, layer):
+        u = U4()
+        L.put(U3(*words), C.c_uint(tag(step, layer)), u)
+        return list(u)
+
+    def take(u, step, layer):
+        w = U3()
+        return list(w) if L.take(U4(*u), C.c_uint(tag(step, layer)), w) else None
+    return put, take
+
+
+def words(rng):
+    """What rows hold, and what hides a mix of two of them best: zeros and equal words."""
+    return rng.choice(([0, 0, 0], [w := rng.getrandbits(32), w, w], [rng.getrandbits(32) for _ in range(3)]))
+
+
+@pytest.mark.parametrize("layers", [(0, 1), (3, 7, 11, 254), tuple(range(42))])
+def test_a_unit_of_a_launch_is_whole_and_its_own(far, layers):
+    """A unit in memory, written by the launches of steps of any width (some leave it alone), seen with either half of the present and the other of the launch before it at
+    that place: taken only when both are the present launch's; nor is one of any earlier launch, or cleared memory, taken whole."""
+    import random
+    put, take = far
+    rng = random.Random(len(layers))
+    cell, step = [0, 0, 0, 0], rng.getrandbits(20)
+    for _ in range(300):
+        step = (step + rng.choice((1, 1, 2, 255, 256, 257, rng.randrange(1, 1 << 15)))) % (1 << 20)
+        for layer in layers:
+            w = words(rng)
+            new = put(w, step, layer)
+            assert take(cell, step, layer) is None
+            assert take([0, 0, 0, 0], step, layer) is None
+            assert take(new[:2] + cell[2:], step, layer) is None and take(cell[:2] + new[2:], step, layer) is None, (step, layer)
+            assert take(new, step, layer) == w
+            cell = new
+
+
+def test_a_unit_of_the_only_layer_with_such_launches(far):
+    """The same layer step after step: halves of steps up to 254 apart do not fit together, whole units up to 2^16 - 1 (they are cleared in half that)."""
+    import random
+    put, take = far
+    rng = random.Random(1)
+    for step in [rng.getrandbits(20) for _ in range(40)] + [255, 256, 65535, 65536, (1 << 20) - 1]:
+        w = words(rng)
+        new = put(w, step, 5)
+        for back in list(range(1, 255)) + [255, 256, 511, 512, 65280, 65535] + [rng.randrange(255, 1 << 16) for _ in range(50)]:
+            old = put(w, (step - back) % (1 << 20), 5)
+            assert take(old, step, 5) is None
+            if back < 255:
+                assert take(new[:2] + old[2:], step, 5) is None and take(old[:2] + new[2:], step, 5) is None
