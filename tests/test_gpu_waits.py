@@ -94,3 +94,51 @@ def test_steps_without_such_launches_leave_the_same_bits(lg, gpu_required, model
     finally:
         gpu.close()
     assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("name,over,rows", [("tiny", {"n_layer": 2, "n_ff": 5120, "n_embd": 3840, "n_head": 16, "head_dim": 256, "n_head_kv": 8, "n_vocab": 2048}, 2),
+                                            ("tiny", {"n_layer": 2, "n_ff": 5120, "n_embd": 3840, "n_head": 16, "head_dim": 256, "n_head_kv": 8, "n_vocab": 2048}, 5),
+                                            ("tiny", {"n_layer": 2, "n_ff": 8192, "n_embd": 2560, "n_vocab": 2048}, 3), ("tiny_full_bf16", {"n_embd": 768, "n_vocab": 2048}, 4)])
+def test_a_wait_given_up_in_a_launch_of_two_products(lg, ob, gpu_required, model_path, name, over, rows):
+    """The same of lg_k_o_geglu with the merge in it and without, of lg_k_down_qkv on v_dot4 and on the matrix cores, and with the per-layer projection of a float type in ffn_down's place."""
+    test_a_wait_given_up_is_reported_once(lg, ob, gpu_required, model_path, name, over, rows)
+
+
+WAITS = dict(narrow=1, attn_out=1, xcd_tail=1, down_m=1, mid=1)
+NONE = dict(narrow=0, attn_out=0, xcd_tail=0, down_m=2, mid=0)
+
+
+@pytest.mark.parametrize("name,over", [("tiny_full", {"n_embd": 2560, "n_head": 8, "head_dim": 256, "head_dim_full": 0, "n_ff": 8192, "n_vocab": 2048}), ("tiny_full", {}),
+                                       ("tiny", {"n_embd": 2560, "n_head": 8, "head_dim": 256, "n_ff": 8192, "n_vocab": 2048}), ("tiny_full_bf16", {"n_ff": 8192, "n_embd": 768}),
+                                       ("tiny", {"n_layer": 3, "n_embd": 3840, "n_head": 16, "head_dim": 256, "n_head_kv": 8, "n_ff": 5120, "n_vocab": 2048})])
+def test_every_launch_that_waits_against_none(lg, gpu_required, model_path, name, over):
+    """All launches whose workgroups wait for one another, those that join two products among them, against none at all: logits, hidden state and cache rows at every width;
+    and at every width the launches say that none was left (q/k/v, gate/up and ffn_down have one of their own in every layer)."""
+    path, spec = model_path(name, **over)
+    rng = np.random.default_rng(5)
+    V, nl, owners = spec["n_vocab"], spec["n_layer"], spec["n_layer"] - spec["shared_kv_layers"]
+    prompt, toks = rng.integers(1, V, 70).astype(np.int32), rng.integers(1, V, 40).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, 160, max_rows=8)
+    got = []
+    try:
+        gpu.set_option("store_logits", 1)
+        for opts in (WAITS, NONE):
+            for k, v in opts.items():
+                gpu.set_option(k, v)
+            gpu.new_cache()
+            gpu.prefill(prompt, 0)
+            pos, res, joined = 70, [], 0
+            for rows in range(1, 9):
+                print(f"{name} {over} {opts}: {rows} rows", flush=True)
+                adv, out = gpu.forward_spec(toks[pos - 70:pos - 70 + rows], pos)
+                res += [out, gpu.last_hidden(spec["n_embd"])] + [gpu.logits_row(j, V) for j in range(rows)]
+                pos += rows
+                n = {k["name"]: k["launches"] for k in gpu.profile_step(toks[:rows], 110, 1)}
+                if opts is NONE:
+                    assert not any(n.get(k, 0) for k in ("ple_tail", "attn_tail", "ffn_xcd")) and [n.get(k, 0) for k in ("qkv", "gate_up_geglu", "ffn_down")] == [nl] * 3, (rows, n)
+                joined += n["qkv"] < nl
+            assert (joined > 0) == (opts is WAITS)
+            got.append([np.ascontiguousarray(r).view(np.uint8) for r in res + [gpu.kv_read(L, w) for L in range(owners) for w in (0, 1)]])
+    finally:
+        gpu.close()
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
