@@ -85,7 +85,7 @@ __device__ __forceinline__ int lg_wait_soon(const FarRows *f, uint32_t tag, int 
 template <int N, typename A, typename P>
 __device__ __forceinline__ int lg_take_far(const FarRows *f, int total, int t, int nt, uint32_t tag, int spin_limit, A &&at, P &&put) {
     const __amdgpu_buffer_rsrc_t r = lg_buffer_rsrc(f->u);
-    const LgFarMarks marks = lg_far_marks(tag);
+    const uint32_t marks = lg_far_marks(tag);
     lg_x4u v[N];
     int err = 0, o[N];
     #pragma unroll
@@ -96,7 +96,7 @@ __device__ __forceinline__ int lg_take_far(const FarRows *f, int total, int t, i
         for (int i = 0; i < N; ++i) v[i] = __builtin_bit_cast(lg_x4u, __builtin_amdgcn_raw_buffer_load_b128(r, o[i], 0, 16));
         #pragma unroll
         for (int i = 0; i < N; ++i) diff |= lg_far_miss(v[i], marks);
-        if (__all(diff >> 16 == 0)) break;
+        if (__all(diff == 0)) break;
         if (spins >= spin_limit) { err = LG_XFFN_ERR_WAIT; break; }
         asm volatile("" ::: "memory");
     }
@@ -122,7 +122,7 @@ __device__ __forceinline__ int lg_take_far_segment(const FarRows *f, int k, int 
     const int st = e == 2 ? 1 : 8;                             // dwords from a slot to the next
     const __amdgpu_buffer_rsrc_t r = lg_buffer_rsrc(f->u);
     const int at = (wave * nit * 3 + w) * 16, row = nb * 48;
-    const LgFarMarks marks = lg_far_marks(tag);
+    const uint32_t marks = lg_far_marks(tag);
     lg_x4u v[N];
     int err = 0;
     auto load = [&] {
@@ -138,7 +138,7 @@ __device__ __forceinline__ int lg_take_far_segment(const FarRows *f, int k, int 
         uint32_t diff = 0;
         #pragma unroll
         for (int i = 0; i < N; ++i) diff |= lg_far_miss(v[i], marks);
-        if (__all(diff >> 16 == 0)) break;
+        if (__all(diff == 0)) break;
         if (spins >= spin_limit) { err = LG_XFFN_ERR_WAIT; break; }
         asm volatile("" ::: "memory");
         load();

@@ -142,3 +142,21 @@ def test_every_launch_that_waits_against_none(lg, gpu_required, model_path, name
     finally:
         gpu.close()
     assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
+def test_marks_are_cleared_while_steps_go_on(lg, gpu_required, model_path):
+    """2^15 steps and more in a row, across the clearing of what launches hand over: the last schedule's tokens are the first one's."""
+    path, spec = model_path("tiny_full", n_embd=768, n_layer=4, n_ff=512, n_vocab=2048, sliding_window=32, local_period=100)
+    toks = np.random.default_rng(7).integers(1, spec["n_vocab"], (4096, 1)).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, 4096, max_rows=2)
+    try:
+        got = []
+        for i in range(9):
+            gpu.schedule(toks, 0)
+            gpu.schedule_run(4096)
+            out, adv, pos = gpu.schedule_wait()
+            print(f"schedule {i}: {len(adv)} steps, position {pos}", flush=True)
+            got.append(out)
+        assert all(np.array_equal(g, got[0]) for g in got[1:])
+    finally:
+        gpu.close()

@@ -225,7 +225,7 @@ extern "C" void put(const unsigned *xyz, unsigned tag, unsigned *u) { const U v 
 extern "C" int take(const unsigned *u, unsigned tag, unsigned *xyz) {
     const U v = { u[0], u[1], u[2], u[3] };
     xyz[0] = v.x; xyz[1] = lg_far_y(v); xyz[2] = v.z;
-    return lg_far_miss(v, lg_far_marks(tag)) >> 16 == 0;
+    return lg_far_miss(v, lg_far_marks(tag)) == 0;
 }
 """
 
