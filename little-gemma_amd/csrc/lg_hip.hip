@@ -314,8 +314,10 @@ static int dev_alloc(lg_hip_model *m, T **p, size_t n) {
 // Launches whose workgroups wait for one another, of several models on a device.  Such a launch is sound when its workgroups are all resident
 // at some time: a waiting one keeps its CU, up to a whole one.  Two of them at a time, on the streams of two models, could each hold a part of an
 // XCD's 32 and wait for the rest until both give up.  So one model has them at a time: the one whose latest such step has not ended yet.  A step of another
-// model takes the kernels that wait for nobody (same bits) and overlaps with it as streams do.  Two models of 512 values, a step each at a time: 106 us
-// with separate kernels in both, 162 when the steps of one waited for the other's, 97 and 80 so; of 2560 values and 5 rows 156, 316, 165 and 155.  With one model at work this is an uncontended lock twice a step.
+// model takes the kernels that wait for nobody (same bits) and overlaps with it as streams do.  With one model at work this is an uncontended lock twice a
+// step.  Two models of 12 layers, a step each at a time, us a step (alone; so; with separate kernels in both): 512 values, one row, 203; 217 and 282; 313.  2560 values, five rows, 457; 534 and
+// 697; 630.  3840 values, five rows, 628; 778 and 1050; 915, one row 529; 670 and 853; 747.  3840 and 2560 values, five rows, 627 and 459; 722 and 869; 797 and 739: the more of the
+// chip the launches of one take, the longer the other's steps, about as many in all.  (Three layers of 512 and of 2560 values when steps waited for one another's: 162 for 106 with separate kernels, 316 for 156.)
 // A prompt's blocks wait for nobody, but their kernels run for milliseconds (of rows far into a long cache for tens of them), and their workgroups go on filling the CUs
 // that a waiting launch needs whole, up to all 256, while those of it that have a place hold theirs and poll, a bounded number of times: the
 // step would be refused.  So while a model has prompt blocks under way the others' steps take the separate kernels too, and the
@@ -1425,12 +1427,12 @@ static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int t
     const int slices = (m->E + 1023) / 1024;
     return tiles < 128 && m->H * rows <= 2 * LG_XCD_WGS && slices * rows <= LG_XCD_WGS && y.hd % 32 == 0 && y.hd <= 256;
 }
-// attn_output, row work and gate/up as one launch; not where one of the options does that row work elsewhere
+// attn_output, row work and gate/up as one launch; not where one of the options does that row work elsewhere, or has attn_output as a launch of its own (attn_out = 0)
 static bool use_mid_o(const lg_hip_model *m, const Layer &y, int rows) {
     return m->mid && (m->mid == 1 || mid_o_faster(m->E, y.qd, rows)) && m->attn_out && m->mido && may_wait(m) && y.wo_pc && y.wgu && !(rows >= 4 && (m->rows_geglu || (m->xcd_ffn && y.xgu)));
 }
 // ... and the merge of attention's partials: up to LG_MID_MERGE_ROWS rows (more: no gain, see lg_k_o_geglu) of up to LG_AOUT_TILES tiles, which a wavefront holds in
-// registers.  (Rows of up to 2560 values have lg_k_attn_out.)
+// registers.  (Rows of up to 2560 values have lg_k_attn_out where their layers have 2048 inputs; the others' merge was not tried in here.)
 static bool use_mid_merge(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
     return rows <= LG_MID_MERGE_ROWS && use_mid_o(m, y, rows) && m->E > 2560 && tiles <= LG_AOUT_TILES && y.hd % 64 == 0;
 }

@@ -7,9 +7,9 @@
 //   the last rows x E/1024 workgroups are the row units (lg_k_rows, a slice of a row each) and hand the q8 rows on (FarRows, lg_xtail.h);
 //   take a share of the second product, whose weights have been on their way to registers and LDS since the first one's had arrived.
 // Sums, their order and every rounding are those of the separate kernels.  Waits are bounded and reported as in lg_xtail.h.
-// Bound by memory once the first product's weights are there: 12B shape, 75 MB in lg_k_o_geglu and 51 in lg_k_down_qkv, which take 17.2 and 12.7 us at one row,
-// 19.9 and 16.0 at five, where the launches they replace took 4.3 + 4.3 + 11.4 and 6.5 + 7.5 (with the row work inside), 5.1 + 4.3 + 12.2 and 9.2 + 4.3 + 6.6 and their
-// gaps: a step 2480 -> 2365 us, 3333 -> 3042.  What it takes for that (12B decode and five rows, us a step): a wavefront's second product's weights requested
+// Bound by memory once the first product's weights are there: 12B shape, 75 MB in lg_k_o_geglu and 51 in lg_k_down_qkv, which take 18.8 and 14.0 us at one row in the
+// trace, 21.7 and 17.6 at five, where the launches they replace took 4.3 + 4.3 + 11.4 and 6.5 + 7.5 (with the row work inside), 5.1 + 4.3 + 12.2 and 9.2 + 4.3 + 6.6 and their
+// gaps: a step 2480 -> 2365 us, 3333 -> 3042.  Narrow models gain nothing or lose (mid_o_faster, mid_down_faster, mid_proj_faster).  What it takes for that (12B decode and five rows, us a step): a wavefront's second product's weights requested
 // behind the arrival of the first one's (2578, 3131 with them ahead); without a condition around loads in flight, where the compiler waits for all of them
 // (2436, 3111; 2390, 3078); three tiles at most ahead of attn_output's products, or the wavefront stands at the CU's address unit (2365, 3052); the
 // second column block's tiles in LDS, so that its products run while the first one's last tiles arrive.
@@ -394,7 +394,7 @@ struct OGegluArgs {
 static_assert((size_t)9 * 16 * LG_FAR_BLK >= 2 * 8 * 8 * 64 * 4, "the sums of two column blocks take the rows' place");
 // MG (up to LG_MID_MERGE_ROWS rows): the merge of attention's partials (lg_k_attn_merge) is part of the launch too, 64 dims of a row by a wavefront, a workgroup
 // each; the q8 is handed over as the rows are.  12B shape at 3001, one to five rows, us a step: 2322 -> 2245, 2495 -> 2413, 2635 -> 2565, 2715 -> 2704, 2855 -> 2855
-// (the launch 18.0 -> 20.4 at one row, the 4.3 of the merge and its gap gone; 20.6 -> 24.4 at five, where 256 workgroups pull 31 KB of q8 each and a merge takes 4.9).
+// (the launch 18.8 -> 21.4 at one row in the trace, the 4.3 of the merge and its gap gone; at five, by events, 20.6 -> 24.4, where 256 workgroups pull 31 KB of q8 each and a merge takes 4.9).
 // One row: gate/up's first tiles requested ahead of the q8 2276, `soon` put behind the q8 2255.
 template <int M, int NIT, bool MG>
 __global__ __launch_bounds__(512) void lg_k_o_geglu(StepCtl *ctl, LG_OGEGLU_FIELDS(LG_XP, _) int p_end_) {
