@@ -245,7 +245,7 @@ struct lg_hip_model {
     int last_rows = 0, last_adv = 0;
     float *lstage = nullptr;           // pinned: two rows of logits on their way to a caller (lg_hip_get_logits), row j in half j % 2
     int lread = -1, lcoming = -1;      // the row of the latest step read last, and the one whose copy has been started
-    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1, attn_out = 1, tail_qkv = 1, attn_geglu = 1, mid = 2;
+    int store_logits = 0, use_graph = 1, wide_prefill = 1, fuse_rows = 1, attn_rows = 1, attn_rows_fq = 1, head_mfma = 1, down_kq = 1, tail_spread = 1, rows_geglu = 0, narrow = 1, attn_out = 1, tail_qkv = 1, attn_geglu = 2, mid = 2;
     uint32_t mid_rows = 0;             // bit r: blocks of r rows have launches of lg_mid.h while mid is 2
     // the feed-forward half of a layer as one XCD-partitioned launch (lg_xffn.h): built when the shape and the chip fit
     int xcd_ffn = 0;                         // option: use it (verify blocks of 4..8 rows)
@@ -1418,9 +1418,13 @@ static bool use_attn_out(const lg_hip_model *m, const Layer &y, int rows, int ti
 }
 // ... on the matrix cores: 4 rows and more, and three of up to 20 tiles
 static bool attn_out_chains(const Layer &y, int rows, int tiles) { return rows > LG_AOUT_DOT_ROWS || (rows == LG_AOUT_DOT_ROWS && y.wo_ch && tiles <= LG_AOUT_BATCH); }
+// With gate/up the launch has 224 workgroups for blocks of 32 FFN columns, a launch of its own one for each of up to 256: in between, two blocks to some workgroups cost narrow models of
+// five rows and more what the join gives (12 layers, us a layer saved at four, five and eight rows: 768 values, FFN 7168 1.3, 0.6, 0.7; 7424 0.1, -0.3, -1.3; 9216 0.6, -0.3, -0.3;
+// 1280, 8192 0.3, -0.3, -0.7; 8960 1.3, 0.4, 0.2; 1536, 8192 0.7, -0.2, -0.5; 1792, 7424 0.8, 0.4, 0.1; 2304, 7424 1.4, 0.8, 0.9)
+static bool attn_geglu_faster(int E, int blocks, int rows) { return rows <= 4 || blocks <= LG_AOUT_GU_WGS || blocks > LG_XCDS * LG_XCD_WGS || E > 1536; }
 // ... with gate/up as part of the launch: two blocks of 32 FFN columns at most for a workgroup on the other seven XCDs; not beside the 13 wavefronts of lg_k_attn_out<3>
 static bool attn_out_geglu(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
-    return m->attn_geglu && m->aorows && y.wgu && y.nff / 32 <= 2 * LG_AOUT_GU_WGS && (rows < LG_AOUT_DOT_ROWS || attn_out_chains(y, rows, tiles));
+    return m->attn_geglu && (m->attn_geglu == 1 || attn_geglu_faster(m->E, y.nff / 32, rows)) && m->aorows && y.wgu && y.nff / 32 <= 2 * LG_AOUT_GU_WGS && (rows < LG_AOUT_DOT_ROWS || attn_out_chains(y, rows, tiles));
 }
 static bool use_attn_tail(const lg_hip_model *m, const Layer &y, int rows, int tiles) {
     if (!y.wo_ch || !m->tsync || !may_wait(m) || !attn_tail_shape(y.qd, m->E, nullptr, nullptr) || m->xcd_attn_tail <= 0 || (m->xcd_attn_tail == 1 && rows < 3)) return false;
@@ -2210,7 +2214,7 @@ static GraphKey graph_key(const lg_hip_model *m, const lg_hip_kv *kv, int rows, 
     put(what, 2); put(rows, 4); put(m->store_logits != 0, 1); put(m->draft_chain, 1); put(m->fuse_rows, 1); put(m->attn_rows, 1); put(m->attn_rows_fq, 1);
     put(m->head_mfma, 1); put(m->down_kq, 1); put(m->xcd_ffn, 1); put(m->fork_ple, 1); put(m->rows_geglu, 1); put(m->tail_stamps != 0, 1);
     put(m->tail_spread == 1 ? 1 : m->tail_spread ? 2 : 0, 2); put(m->xcd_tail, 2); put(m->down_m, 2); put(m->xcd_attn_tail, 2); put(m->merge_o, 2);
-    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->tail_qkv, 1); put(m->attn_geglu, 1); put(m->mid, 2); put(m->wait_polls, 17); put(may_wait(m), 1);
+    put(m->xffn_delay, 10); put(m->narrow, 1); put(m->attn_out, 1); put(m->tail_qkv, 1); put(m->attn_geglu, 2); put(m->mid, 2); put(m->wait_polls, 17); put(may_wait(m), 1);
     return { (uint64_t)kv->id, o, (uint64_t)m->merge_o_slices, 0 };
 }
 
@@ -2276,7 +2280,7 @@ extern "C" int lg_hip_set_option(lg_hip_model *m, const char *name, int value) {
     else if (!strcmp(name, "attn_out")) m->attn_out = value != 0;
     else if (!strcmp(name, "mid")) m->mid = value == 1 ? 1 : value ? 2 : 0;
     else if (!strcmp(name, "tail_qkv")) m->tail_qkv = value != 0;
-    else if (!strcmp(name, "attn_geglu")) m->attn_geglu = value != 0;
+    else if (!strcmp(name, "attn_geglu")) m->attn_geglu = value == 1 ? 1 : value ? 2 : 0;
     else if (!strcmp(name, "down_kq")) m->down_kq = value != 0;
     else if (!strcmp(name, "xcd_ffn")) m->xcd_ffn = value != 0 && m->xffn_built;
     else if (!strcmp(name, "fork_ple")) m->fork_ple = value != 0;

@@ -38,3 +38,27 @@ def test_one_launch_equals_two(lg, gpu_required, model_path, over, fused):
         assert all(np.array_equal(a, b) for a, b in zip(*got))
     finally:
         gpu.close()
+
+
+@pytest.mark.parametrize("over,fused", [
+    (dict(W8, n_embd=768, n_ff=7168), range(1, 9)), (dict(W8, n_embd=768, n_ff=7424), range(1, 5)), (dict(W8, n_embd=1536, n_ff=8192), range(1, 5)),
+    (dict(W8, n_embd=1536, n_ff=8448), range(1, 9)), (dict(W8, n_embd=1792, n_ff=7424), range(1, 9))])
+def test_taken_where_it_is_the_faster_form(lg, gpu_required, model_path, over, fused):
+    """The default: not at five rows and more of a narrow model whose blocks of FFN columns are two to some of 224 workgroups and one to a CU in a launch of their own."""
+    path, spec = model_path("tiny", **dict(dict(n_layer=2, n_vocab=2048, sliding_window=512), **over))
+    toks = np.random.default_rng(spec["n_ff"]).integers(1, spec["n_vocab"], 8).astype(np.int32)
+    gpu = lg.hiplib.HipBackend(path, 400, max_rows=8)
+    try:
+        for rows in range(1, 9):
+            got = []
+            for on in (None, 0):
+                if on is not None:
+                    gpu.set_option("attn_geglu", on)
+                n = {k["name"]: k["launches"] for k in gpu.profile_step(toks[:rows], 33, 1)}.get("gate_up_geglu", 0)
+                assert n == (0 if on is None and rows in fused else 2), (rows, on, n)
+                gpu.forward_spec(toks[:rows], 0)
+                got.append(gpu.last_hidden(spec["n_embd"]).view(np.uint32))
+            assert np.array_equal(*got), rows
+            gpu.set_option("attn_geglu", 2)
+    finally:
+        gpu.close()
